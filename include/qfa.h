@@ -50,7 +50,7 @@ const char *qfa_last_error(void);
  *     code[d] = clamp(roundf(x[d]/scale + zp))         -- all IEEE binary32, roundf = ties away
  *   x         [B,H,N,D] of x_dtype (QFA_F32 / QFA_F16 / QFA_BF16), strides sxb,sxh,sxn
  *   codes     [B,H,N,D] int8, strides scb,sch,scn (the reference uses the input's strides)
- *   scale_f32 [B*H*N] float: the unrounded scale the codes were computed with
+ *   scale_f32 [B*H*N] float: the unrounded scale the codes were computed with; may be NULL when scale_lp is given
  *   scale_lp  nullable; [B*H*N] copy of the scale rounded to scale_lp_dtype (QFA_F16/QFA_BF16)
  *             -- the fp16 scale tensor the reference returns (asymmetric_quant.py:93,128)
  *   zp        [B*H*N] int8

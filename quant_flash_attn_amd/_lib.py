@@ -1,6 +1,7 @@
-"""ctypes binding of libqfa.so (the C ABI declared in include/qfa.h).
+"""ctypes binding of libqfa.so (the C ABI declared in include/qfa.h), and the native host path on top of it.
 
-The library is loaded from the package directory (or from $QFA_LIB).  There is no
+The Python entry points go through host(): the module _qfa_host.so (csrc/qfa_torch.cpp), which checks arguments,
+allocates and calls the library's entry points at the addresses it is given here.  The library is loaded from the package directory (or from $QFA_LIB).  There is no
 fallback: if it is missing, or a call returns non-zero, a RuntimeError is raised.
 """
 from __future__ import annotations
@@ -18,6 +19,7 @@ DTYPE_CODE = {torch.float32: QFA_F32, torch.float16: QFA_F16, torch.bfloat16: QF
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 # argument lists mirror include/qfa.h one to one
 _P, _I, _L, _F = c_void_p, c_int, c_int64, c_float
@@ -67,6 +69,23 @@ def lib():
     return _lib
 
 
+def host():
+    """The native host path, bound to the loaded library."""
+    global _host
+    if _host is None:
+        handle = lib()
+        with _lock:
+            if _host is None:
+                try:
+                    from . import _qfa_host
+                except ImportError as e:
+                    raise RuntimeError(f"quant_flash_attn_amd: the host module cannot be loaded ({e}). Build it with "
+                                       "`python -m quant_flash_attn_amd.build` (there is no fallback path).") from e
+                _qfa_host.init({name: ctypes.cast(getattr(handle, name), c_void_p).value for name in _SIGNATURES})
+                _host = _qfa_host
+    return _host
+
+
 def check(code: int, what: str) -> None:
     if code != 0:
         msg = lib().qfa_last_error().decode("utf-8", "replace")
@@ -76,14 +95,3 @@ def check(code: int, what: str) -> None:
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on the tensor's device."""
     return torch.cuda.current_stream(t.device).cuda_stream
-
-
-def require_gpu(*tensors: torch.Tensor) -> None:
-    for t in tensors:
-        if not t.is_cuda:
-            raise RuntimeError("quant_flash_attn_amd runs on the GPU only: got a tensor on "
-                               f"'{t.device}'. There is no CPU implementation in this package.")
-    dev = tensors[0].device
-    for t in tensors[1:]:
-        if t.device != dev:
-            raise RuntimeError(f"all tensors must be on the same device, got {dev} and {t.device}")

@@ -1,8 +1,9 @@
-"""Builds quant_flash_attn_amd/libqfa.so from csrc/ with hipcc for gfx950.
+"""Builds quant_flash_attn_amd/libqfa.so from csrc/ with hipcc for gfx950, and the module of its host path.
 
     python -m quant_flash_attn_amd.build          # compile every translation unit, then link
 
-The library is built in-tree so that a source snapshot carries it along; nothing is
+libqfa.so holds the kernels behind the C ABI; _qfa_host.so (csrc/qfa_torch.cpp, host code only, against torch's headers)
+is what the Python entry points call.  Both are built in-tree so that a source snapshot carries it along; nothing is
 JIT-compiled at import time.  Compilation needs no GPU (hipcc cross-compiles).
 """
 from __future__ import annotations
@@ -10,11 +11,13 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libqfa.so")
+HOST_MODULE = os.path.join(HERE, "_qfa_host.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 # -packed-fp32-ops: keep hipcc from forming v_pk_*_f32 out of scalar float code.
@@ -46,15 +49,35 @@ def _compile(src: str, extra=()) -> str:
     return obj
 
 
+def _compile_host_module() -> str:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    tmp = HOST_MODULE + ".tmp"
+    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_qfa_host",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(x for i in inc for x in ("-isystem", i)),
+           os.path.join(CSRC, "qfa_torch.cpp"), "-o", tmp, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip",
+           "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for qfa_torch.cpp:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_MODULE)
+    return HOST_MODULE
+
+
 def build_library(extra_flags=(), jobs: int = 4) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host_module)
         objs = list(pool.map(lambda s: _compile(s, extra_flags), SOURCES))
     tmp = LIB + ".tmp"
     res = subprocess.run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs],
                          capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
+    host.result()
     os.replace(tmp, LIB)
     return LIB
 

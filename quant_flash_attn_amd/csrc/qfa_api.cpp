@@ -51,7 +51,8 @@ const char *qfa_last_error(void) { return g_err; }
 int qfa_quant_per_token(const void *x, int x_dtype, int8_t *codes, float *scale_f32, void *scale_lp,
                         int scale_lp_dtype, int8_t *zp, int32_t *rowsum, int64_t B, int64_t H, int64_t N, int D,
                         int64_t sxb, int64_t sxh, int64_t sxn, int64_t scb, int64_t sch, int64_t scn, void *stream) {
-  if (!x || !codes || !scale_f32 || !zp) return set_error(QFA_EINVAL, "quant: null x/codes/scale_f32/zp pointer");
+  if (!x || !codes || (!scale_f32 && !scale_lp) || !zp)
+    return set_error(QFA_EINVAL, "quant: null x/codes/scale_f32/zp pointer (scale_f32 may be null where scale_lp is given)");
   if (!is_float_dtype(x_dtype)) return set_error(QFA_EINVAL, "quant: x_dtype %d is not QFA_F32/F16/BF16", x_dtype);
   if (scale_lp && scale_lp_dtype != QFA_F16 && scale_lp_dtype != QFA_BF16)
     return set_error(QFA_EINVAL, "quant: scale_lp_dtype %d is not QFA_F16/BF16", scale_lp_dtype);

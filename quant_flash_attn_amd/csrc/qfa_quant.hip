@@ -190,7 +190,7 @@ __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) 
       *reinterpret_cast<u32x2 *>(cb + n * a.scn + sub * 8) = w;
       if (sub == 0) {
         const int64_t t = bh * a.N + n;
-        a.scale[t] = scale;
+        if (a.scale) a.scale[t] = scale;
         a.zp[t] = (int8_t)(int)zp;
         if (a.rowsum) a.rowsum[t] = sum;
         if (a.scale_lp) {
