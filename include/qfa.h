@@ -209,6 +209,30 @@ int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale
                            int64_t sdkh, int64_t sdkn, float sm_scale, void *stream);
 
 /*
+ * Attention forward of a SHORT query block on an INT8 cache of keys and values (decoding, a few queries at a time):
+ *     O = softmax(sm_scale * Q^ K^^T) V^,   Q^, K^, V^ = scale * (codes - zero_point) per token
+ * Q is quantized inside by the arithmetic of qfa_quant_per_token, the scores are those of qfa_attn_fwd on these codes,
+ * V enters as its exact codes; no LSE.  One pass over the cache (bound by reading it); every 16 queries read it again
+ * (from the L2), so long query blocks belong to qfa_attn_fwd.  No counterpart in the reference, whose operator has one
+ * tensor for K and V (quant_flash_attn.py:22-83).
+ *   q, o   [B,H,Nq,D] of q_dtype (QFA_F32 / QFA_F16 / QFA_BF16)
+ *   kc, vc int8 [B,H,Nk,D];  ks, vs [B*H*Nk] of scale_dtype (QFA_F32 / QFA_F16 / QFA_BF16);  kz, vz int8 [B*H*Nk]
+ *   D in {64, 128, 256}; causal, sm_scale, alignment and stride rules as in qfa_attn_fwd (codes as its kc, q and o as
+ *   its o).  Range, not checked: the probabilities are multiplied by V's scale before they are packed to binary16
+ *   (scales up to about 4e3).
+ *   workspace  nullable (never split then); else qfa_attn_fwd_cache_workspace_bytes(...) bytes, 16-byte aligned (0: no
+ *              split pays): the keys of a query block are split over several workgroups whose partial results a second
+ *              small kernel merges.
+ */
+int64_t qfa_attn_fwd_cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
+
+int qfa_attn_fwd_cache(const void *q, int q_dtype, const int8_t *kc, const void *ks, const int8_t *kz, const int8_t *vc,
+                       const void *vs, const int8_t *vz, int scale_dtype, void *o, int64_t B, int64_t H, int64_t Nq,
+                       int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh, int64_t skn,
+                       int64_t svb, int64_t svh, int64_t svn, int64_t sob, int64_t soh, int64_t son, float sm_scale,
+                       int causal, void *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * Measurement hook, same arguments as qfa_attn_fwd: runs the forward kernel with the exponentials
  * and the P.V product compiled out (same K/V/Q loads, INT8 QK^T MFMAs, zero-point correction, key
  * scaling and running row maximum).  O is left untouched; lse receives the scaled row maxima.

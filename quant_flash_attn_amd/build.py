@@ -23,9 +23,10 @@ OBJ_DIR = os.path.join(HERE, "build")
 # -packed-fp32-ops: keep hipcc from forming v_pk_*_f32 out of scalar float code.
 COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-# the quantizer must evaluate its expressions as single IEEE operations (bit-exact codes)
-PER_FILE = {"qfa_quant.hip": ["-ffp-contract=off", "-fno-fast-math"]}
-SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_bwd.hip", "qfa_skv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip"]
+# whatever quantizes must evaluate its expressions as single IEEE operations (bit-exact codes)
+PER_FILE = {f: ["-ffp-contract=off", "-fno-fast-math"] for f in ("qfa_quant.hip", "qfa_cache.hip")}
+SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_bwd.hip", "qfa_skv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
+           "qfa_cache.hip"]
 
 
 def _hipcc() -> str:

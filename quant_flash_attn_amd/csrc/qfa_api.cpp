@@ -266,6 +266,53 @@ int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale
   return one_pass ? launch_skv_bwd(a, (hipStream_t)stream) : launch_skv_bwd_long(a, (hipStream_t)stream);
 }
 
+int64_t qfa_attn_fwd_cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0 || (D != 64 && D != 128 && D != 256)) return 0;
+  return cache_workspace_bytes(B, H, Nq, Nk, D);
+}
+
+int qfa_attn_fwd_cache(const void *q, int q_dtype, const int8_t *kc, const void *ks, const int8_t *kz, const int8_t *vc,
+                       const void *vs, const int8_t *vz, int scale_dtype, void *o, int64_t B, int64_t H, int64_t Nq,
+                       int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh, int64_t skn,
+                       int64_t svb, int64_t svh, int64_t svn, int64_t sob, int64_t soh, int64_t son, float sm_scale,
+                       int causal, void *workspace, int64_t workspace_bytes, void *stream) {
+  const char *who = "attn_fwd_cache";
+  if (!q || !kc || !ks || !kz || !vc || !vs || !vz || !o) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
+  if (!is_float_dtype(q_dtype)) return set_error(QFA_EINVAL, "%s: q_dtype %d is not QFA_F32/F16/BF16", who, q_dtype);
+  if (!is_float_dtype(scale_dtype)) return set_error(QFA_EINVAL, "%s: scale_dtype %d is not QFA_F32/F16/BF16", who, scale_dtype);
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0) return set_error(QFA_EINVAL, "%s: B, H, Nq, Nk must be positive", who);
+  if (Nq > kMaxTokens || Nk > kMaxTokens)
+    return set_error(QFA_EUNSUPPORTED, "%s: sequences of more than 2^28 tokens are not supported", who);
+  if (D != 64 && D != 128 && D != 256) return set_error(QFA_EUNSUPPORTED, "%s: head_dim %d not in {64, 128, 256}", who, D);
+  if (!(sm_scale > 0.0f) || !(sm_scale < 3.0e38f)) return set_error(QFA_EINVAL, "%s: sm_scale must be a positive finite number", who);
+  if (causal && Nq > Nk)
+    return set_error(QFA_EUNSUPPORTED, "%s: causal needs Nq <= Nk (the mask is aligned to the last key)", who);
+  if (!aligned16(q) || !aligned16(kc) || !aligned16(vc) || !aligned16(o))
+    return set_error(QFA_EINVAL, "%s: q, kc, vc, o must be 16-byte aligned", who);
+  const int es = elem_size(q_dtype);
+  if (!strides_ok(sqb, sqh, sqn, D, es) || !strides_ok(skb, skh, skn, D, 1) || !strides_ok(svb, svh, svn, D, 1) ||
+      !strides_ok(sob, soh, son, D, es))
+    return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
+  // offsets inside a 32-key tile are formed in 31 bits
+  if (skn >= (1 << 23) || svn >= (1 << 23))
+    return set_error(QFA_EUNSUPPORTED, "%s: token strides of 2^23 elements or more are not supported", who);
+  CacheAttnArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = q; a.kc = kc; a.ks = ks; a.kz = kz; a.vc = vc; a.vs = vs; a.vz = vz; a.o = o;
+  a.B = B; a.H = H; a.Nq = Nq; a.Nk = Nk; a.D = D; a.q_dtype = q_dtype; a.scale_dtype = scale_dtype;
+  a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.skb = skb; a.skh = skh; a.skn = skn;
+  a.svb = svb; a.svh = svh; a.svn = svn; a.sob = sob; a.soh = soh; a.son = son;
+  a.sm_scale = sm_scale; a.causal = causal != 0;
+  if (workspace) {
+    const int64_t need = cache_workspace_bytes(B, H, Nq, Nk, D);
+    if (!aligned16(workspace) || workspace_bytes < need)
+      return set_error(QFA_EINVAL, "%s: workspace must be 16-byte aligned and hold %lld bytes "
+                       "(qfa_attn_fwd_cache_workspace_bytes), got %lld", who, (long long)need, (long long)workspace_bytes);
+    a.workspace = need > 0 ? workspace : nullptr;
+  }
+  return launch_cache_fwd(a, (hipStream_t)stream);
+}
+
 int qfa_bench_qk_stage(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
                        const float *sk, const int8_t *zk, const int32_t *rk, const void *v, void *o, float *lse,
                        int io_dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh,

@@ -73,4 +73,17 @@ int launch_dout_normalise(const void *dout, int dout_dtype, int64_t n, const voi
                           float *partials, void *out, float *back, hipStream_t st);
 int launch_skv_bwd_long(const SkvAttnArgs &a, hipStream_t st);   // io_dtype QFA_F16, any Nq: dQ kernel + dKV kernel
 
+// Attention of a short query block on an INT8 cache (K and V quantized separately, Q quantized inside), after validation.
+struct CacheAttnArgs {
+  const void *q; const int8_t *kc; const void *ks; const int8_t *kz; const int8_t *vc; const void *vs; const int8_t *vz;
+  void *o;
+  void *workspace;   // nullable: partial results when the keys are split
+  int64_t B, H, Nq, Nk;
+  int64_t sqb, sqh, sqn, skb, skh, skn, svb, svh, svn, sob, soh, son;
+  float sm_scale;
+  int causal, D, q_dtype, scale_dtype;
+};
+int launch_cache_fwd(const CacheAttnArgs &a, hipStream_t st);
+int64_t cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
+
 }  // namespace qfa

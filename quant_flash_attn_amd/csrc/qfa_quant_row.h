@@ -1,0 +1,142 @@
+// The quantizer's arithmetic on one token row, shared by the stand-alone quantizer and the kernels that quantize their
+// queries themselves.  Every step is one IEEE binary32 operation (see qfa_quant.hip): the file that includes this is
+// compiled with -ffp-contract=off.
+#pragma once
+#include "qfa_device.h"
+
+namespace qfa {
+
+// One reduction step = one instruction: the lane permute is the DPP modifier of the min / max itself.
+// (Written as asm: through the builtin the permuted value comes back as an integer, and the compiler
+// then spends a v_mov_b32_dpp and a canonicalising v_max on every step.  The s_nop covers the two wait
+// states a DPP read needs after a vector write of the same register, which the compiler does not
+// insert for instructions it cannot see.)
+#define QFA_DPP_STEP(OP, CTRL)                                                                           \
+  asm("s_nop 1\n\t" OP " %0, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(v))
+template <int LPT> __device__ __forceinline__ float group_min(float v) {
+  float r;
+  QFA_DPP_STEP("v_min_f32_dpp", "quad_perm:[1,0,3,2]"); v = r;
+  if (LPT >= 4) { QFA_DPP_STEP("v_min_f32_dpp", "quad_perm:[2,3,0,1]"); v = r; }
+  if (LPT >= 8) { QFA_DPP_STEP("v_min_f32_dpp", "row_half_mirror"); v = r; }
+  if (LPT >= 16) { QFA_DPP_STEP("v_min_f32_dpp", "row_mirror"); v = r; }
+  if (LPT >= 32) v = fminf(v, __shfl_xor(v, 16, 64));
+  return v;
+}
+template <int LPT> __device__ __forceinline__ float group_max(float v) {
+  float r;
+  QFA_DPP_STEP("v_max_f32_dpp", "quad_perm:[1,0,3,2]"); v = r;
+  if (LPT >= 4) { QFA_DPP_STEP("v_max_f32_dpp", "quad_perm:[2,3,0,1]"); v = r; }
+  if (LPT >= 8) { QFA_DPP_STEP("v_max_f32_dpp", "row_half_mirror"); v = r; }
+  if (LPT >= 16) { QFA_DPP_STEP("v_max_f32_dpp", "row_mirror"); v = r; }
+  if (LPT >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
+  return v;
+}
+#undef QFA_DPP_STEP
+// integer sum: `old` = 0, the identity of the addition (never used: every lane reads a valid lane),
+// lets the compiler fold the permute into v_add_u32_dpp
+template <int CTRL> __device__ __forceinline__ int dpp_zero(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false); }
+template <int LPT> __device__ __forceinline__ int group_sum(int v) {
+  v += dpp_zero<0xB1>(v);
+  if (LPT >= 4) v += dpp_zero<0x4E>(v);
+  if (LPT >= 8) v += dpp_zero<0x141>(v);
+  if (LPT >= 16) v += dpp_zero<0x140>(v);
+  if (LPT >= 32) v += __shfl_xor(v, 16, 64);
+  return v;
+}
+
+template <typename T> struct Load8;
+template <> struct Load8<float> {
+  static __device__ __forceinline__ void run(const void *p, float (&v)[8]) {
+    const f32x4 *q = reinterpret_cast<const f32x4 *>(p);
+    f32x4 a = __builtin_nontemporal_load(q), b = __builtin_nontemporal_load(q + 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
+  }
+};
+template <> struct Load8<__bf16> {
+  static __device__ __forceinline__ void run(const void *p, float (&v)[8]) {
+    u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {   // bf16 -> fp32 is a 16-bit shift
+      v[2 * e] = __builtin_bit_cast(float, w[e] << 16);
+      v[2 * e + 1] = __builtin_bit_cast(float, w[e] & 0xffff0000u);
+    }
+  }
+};
+template <> struct Load8<_Float16> {
+  static __device__ __forceinline__ void run(const void *p, float (&v)[8]) {
+    f16x8 w = __builtin_bit_cast(f16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p)));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)w[e];
+  }
+};
+
+// The row arithmetic: eight elements per lane, a token in LPT adjacent lanes.  Returns the lane's eight codes and, in
+// every lane of the token, its scale, zero point (an integer in [-128, 127]) and code sum.  `used`: false in the lanes
+// past the row's end (they hold a copy of elements of the row and add nothing to the sum).
+struct QuantRow {
+  u32x2 codes;
+  float scale, zp;
+  int sum;
+};
+template <int LPT> __device__ __forceinline__ QuantRow quant_row(const float (&v)[8], bool used) {
+#pragma clang fp contract(off)
+  float mn = v[0], mx = v[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) { mn = fminf(mn, v[e]); mx = fmaxf(mx, v[e]); }
+  mn = group_min<LPT>(mn);
+  mx = group_max<LPT>(mx);
+  float scale = (mx - mn) / 255.0f;
+  scale = (scale == 0.0f) ? 1.0f : scale;
+  // Division by the per-token scale.  In the common exponent range the quotient is formed with the
+  // same FMA refinement the hardware division sequence uses (reciprocal refined once, two residual
+  // corrections of the quotient), which gives the correctly rounded x/scale without the per-element
+  // operand scaling; outside that range (tiny scale, huge values, NaN) the IEEE `/` is used.
+  // Quotients below 2^-30 in magnitude may differ in their last bits, which cannot matter: they
+  // vanish in the addition of the zero point or round to zero.
+  const bool fast = (scale >= 0x1p-60f) && (fmaxf(fabsf(mn), fabsf(mx)) <= 0x1p60f);
+  float r = __builtin_amdgcn_rcpf(scale);
+  r = __builtin_fmaf(__builtin_fmaf(-scale, r, 1.0f), r, r);
+  auto fdiv = [&](float x) -> float {
+    float q = x * r;
+    q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
+    q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
+    return q;
+  };
+  // roundf (ties away from zero) in three instructions: add the largest float below one half with the
+  // sign of y, truncate.  Equal to roundf for every binary32 value (checked exhaustively on the CPU; the
+  // classic y + 0.5 fails at 0.49999997).
+  auto round_away = [](float y) -> float {
+    return __builtin_truncf(y + __builtin_copysignf(0x1.fffffep-2f, y));
+  };
+  float q[8], qmn;
+  if (fast) {
+    qmn = fdiv(mn);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = fdiv(v[e]);
+  } else {
+    qmn = mn / scale;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) q[e] = v[e] / scale;
+  }
+  const float zpf = -128.0f - qmn;
+  const float zp = fmaxf(-128.0f, fminf(127.0f, round_away(zpf)));
+  // codes leave as biased bytes: roundf(.) + 128 converted with unsigned saturation (= the clamp to
+  // [-128, 127]), flipped back to two's complement with one XOR per dword
+  u32x2 w = {0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float y = q[e] + zp;
+    const float c = round_away(y) + 128.0f;
+    w[e / 4] = __builtin_amdgcn_cvt_pk_u8_f32(c, e % 4, w[e / 4]);
+  }
+  int sum = (int)__builtin_amdgcn_sad_u8(w[0], 0u, 0u);
+  sum = (int)__builtin_amdgcn_sad_u8(w[1], 0u, (unsigned)sum) - 8 * 128;
+  if (!used) sum = 0;
+  w[0] ^= 0x80808080u;
+  w[1] ^= 0x80808080u;
+  sum = group_sum<LPT>(sum);
+  return {w, scale, zp, sum};
+}
+
+}  // namespace qfa

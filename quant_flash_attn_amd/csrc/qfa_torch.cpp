@@ -38,6 +38,8 @@ struct Api {
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
   QFA_ENTRY(qfa_attn_bwd_shared_kv);
+  QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
+  QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
   QFA_ENTRY(qfa_dout_normalise);
 #undef QFA_ENTRY
@@ -62,6 +64,8 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
   QFA_ENTRY(qfa_attn_bwd_shared_kv);
+  QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
+  QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
   QFA_ENTRY(qfa_dout_normalise);
 #undef QFA_ENTRY
@@ -428,6 +432,34 @@ CacheKept cache_forward(const Tensor &q_in, const Tensor &kc, const Tensor &ks, 
   r.o = to(r.o16, q.scalar_type());
   return r;
 }
+// Longest query block for qfa_attn_fwd_cache, which walks the cache once per 16 queries (about 40 us per 16 queries at B8
+// H32 Nk8192 D128 once the MFMAs are the bound: 64 queries 203 us, where the pass over V, the row sums of K and
+// qfa_attn_fwd take 470 up to 128 queries; at B1 H8 Nk1024 it is 11 against 34 us) and leaves nothing for a backward
+constexpr int64_t CACHE_MAX_Q = 128;
+Tensor cache_short(const Tensor &q_in, const Tensor &kc_in, const Tensor &ks_in, const Tensor &kz, const Tensor &vc_in,
+                   const Tensor &vs_in, const Tensor &vz, bool causal, double sm) {
+  const c10::DeviceGuard guard(q_in.device());
+  const Tensor q = check_input(q_in);
+  check_codes(kc_in, "k.codes");
+  check_codes(vc_in, "v.codes");
+  const Tensor kc = rows16(kc_in), vc = rows16(vc_in);
+  const int64_t B = q.size(0), H = q.size(1), Nq = q.size(2), D = q.size(3), Nk = kc.size(2), n = B * H * Nk;
+  const bool as_is = ks_in.scalar_type() == vs_in.scalar_type() && dtype_code(ks_in.scalar_type()) >= 0;
+  const at::ScalarType sdt = as_is ? ks_in.scalar_type() : at::kFloat;
+  const Tensor ks = flat(to(ks_in, sdt), sdt, n, "k.scale"), vs = flat(to(vs_in, sdt), sdt, n, "v.scale"),
+               kzf = flat(kz, at::kChar, n, "k.zero_point"), vzf = flat(vz, at::kChar, n, "v.zero_point");
+  Tensor o = empty({B, H, Nq, D}, q.scalar_type(), q), ws;
+  const int64_t ws_bytes = api.qfa_attn_fwd_cache_workspace_bytes(B, H, Nq, Nk, (int)D);
+  if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, q);
+  check(api.qfa_attn_fwd_cache(q.data_ptr(), dtype_code(q.scalar_type()), kc.data_ptr<int8_t>(), ks.data_ptr(),
+                               kzf.data_ptr<int8_t>(), vc.data_ptr<int8_t>(), vs.data_ptr(), vzf.data_ptr<int8_t>(),
+                               dtype_code(sdt), o.data_ptr(), B, H, Nq, Nk, (int)D, QFA_STRIDES(q), QFA_STRIDES(kc),
+                               QFA_STRIDES(vc), QFA_STRIDES(o), (float)sm, causal, ws_bytes > 0 ? ws.data_ptr() : nullptr,
+                               ws_bytes, stream_of(q)),
+        "qfa_attn_fwd_cache");
+  return o;
+}
+
 struct CacheFn : torch::autograd::Function<CacheFn> {
   static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc,
                         const Tensor &ks, const Tensor &kz, const Tensor &vc, const Tensor &vs, const Tensor &vz, bool causal,
@@ -463,6 +495,7 @@ Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const 
                         q.size(0) == kc.size(0) && q.size(1) == kc.size(1),
                     "shape mismatch: q ", q.sizes(), ", k codes ", kc.sizes(), ", v codes ", vc.sizes());
   if (wants_grad({&q, &k_fp16, &v_fp16})) return CacheFn::apply(q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz, causal, sm);
+  if (q.size(2) <= CACHE_MAX_Q) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
   return cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm).o;
 }
 
