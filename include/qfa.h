@@ -135,7 +135,7 @@ int qfa_attn_fwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
  *   q, o   [B,H,Nq,D] of io_dtype (QFA_F16 or QFA_BF16; bf16 queries enter the products rounded
  *          to binary16), strides sq?, so?;  lse float [B*H*Nq]
  *   codes  int8 [B,H,Nk,D], strides sc?;  zp int8 [B*H*Nk]
- *   scale  [B*H*Nk] of scale_dtype: QFA_F32, or the same 16-bit type as io_dtype
+ *   scale  [B*H*Nk] of scale_dtype: QFA_F32, QFA_F16 (what asymmetric_quant.py:128 stores), or the same type as io_dtype
  *   D in {64, 128, 256}.  q, codes, o 16-byte aligned, strides multiples of 16 bytes, scn < 2^23.
  *   The codes' binary16 offset (1152) is removed through the sum of a query's D elements: |sum| must
  *   stay below 2^21, and the scores carry an absolute error of a few fp32 ulp of 1152 * |sum| code

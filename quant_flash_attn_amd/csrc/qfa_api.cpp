@@ -171,8 +171,8 @@ static int check_shared_kv(const char *who, const SkvAttnArgs &a) {
   if (!a.q || !a.codes || !a.scale || !a.zp || !a.o || !a.lse) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
   if (a.io_dtype != QFA_BF16 && a.io_dtype != QFA_F16)
     return set_error(QFA_EINVAL, "%s: io_dtype must be QFA_BF16 or QFA_F16", who);
-  if (a.scale_dtype != QFA_F32 && a.scale_dtype != a.io_dtype)
-    return set_error(QFA_EINVAL, "%s: scale_dtype must be QFA_F32 or equal to io_dtype", who);
+  if (a.scale_dtype != QFA_F32 && a.scale_dtype != QFA_F16 && a.scale_dtype != a.io_dtype)
+    return set_error(QFA_EINVAL, "%s: scale_dtype must be QFA_F32, QFA_F16 or equal to io_dtype", who);
   if (a.B <= 0 || a.H <= 0 || a.Nq <= 0 || a.Nk <= 0) return set_error(QFA_EINVAL, "%s: B, H, Nq, Nk must be positive", who);
   // the kernels form byte offsets into the per-token vectors (4 bytes per token) in 31 bits
   if (a.Nq > kMaxTokens || a.Nk > kMaxTokens)

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "qfa_host.h"
+#include "qfa_merge.h"
 #include "qfa_quant_row.h"
 #include "qfa_skv_common.h"
 
@@ -38,27 +39,12 @@ struct CacheArgs {
   int Nq, Nk, BH, qblocks, splits, tiles_per_split, causal, q_dtype;
 };
 
-// row maximum of a wave or split that saw no key: finite, so that differences of two of them are zero and not NaN
-constexpr float CACHE_NO_KEY = -1e30f;
-
 // Workgroups per CU the registers are budgeted for: two tiles in registers (80 of them at head_dim 128, 148 at 256) beside
 // the accumulators.  With one tile per wave in flight that keeps 64 KB (48 at head_dim 64) per CU under way.
 constexpr int cache_wgs_per_cu(int D) { return D == 256 ? 1 : D == 128 ? 2 : 3; }
 
 __device__ __forceinline__ i32x4 mfma_i8_16(i32x4 a, i32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
-}
-
-// four consecutive outputs of a row, rounded to the queries' type
-__device__ __forceinline__ void store4(void *row, int q_dtype, int d, f32x4 x) {
-  if (q_dtype == QFA_F32) {
-    *reinterpret_cast<f32x4 *>(static_cast<float *>(row) + d) = x;
-  } else {
-    u32x2 w;
-    if (q_dtype == QFA_BF16) w = u32x2{pack2<__bf16>(x[0], x[1]), pack2<__bf16>(x[2], x[3])};
-    else w = u32x2{pack2<_Float16>(x[0], x[1]), pack2<_Float16>(x[2], x[3])};
-    *reinterpret_cast<u32x2 *>(static_cast<unsigned short *>(row) + d) = w;
-  }
 }
 
 template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(D)) void cache_fwd_kernel(CacheArgs a) {
@@ -179,7 +165,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
     // token constants: K (scale, zp as an integer), V (scale, the binary16 number 1152 + zp)
     {
       u32x2 w;
-      w[0] = std::is_same<S, float>::value ? t.sc : __builtin_bit_cast(unsigned, lo_to_f32<std::conditional_t<std::is_same<S, float>::value, _Float16, S>>(t.sc));
+      w[0] = __builtin_bit_cast(unsigned, scale_to_f32<S>(t.sc));
       w[1] = lane < 32 ? (unsigned)(int)(signed char)t.zp : (0x6400u | (t.zp ^ 0x80u));
       *reinterpret_cast<u32x2 *>(tc + 2 * lane) = w;
     }
@@ -282,14 +268,14 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
         *reinterpret_cast<f32x4 *>(dst + VB * (4 * G + v) + j) = x;
       }
     if (G == 0) {
-      ml[2 * (wave * 16 + q16)] = m_ref == -INFINITY ? CACHE_NO_KEY : a_i * m_ref;
+      ml[2 * (wave * 16 + q16)] = m_ref == -INFINITY ? NO_KEY : a_i * m_ref;
       ml[2 * (wave * 16 + q16) + 1] = l_tot;
     }
   }
   __syncthreads();
   for (int x = tid; x < nqv * (D / 4); x += 256) {
     const int q = x / (D / 4), d = 4 * (x % (D / 4));
-    float m = CACHE_NO_KEY, l = 0.f;
+    float m = NO_KEY, l = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; ++w) m = fmaxf(m, ml[2 * (16 * w + q)]);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -315,50 +301,6 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
   }
 }
 
-// O of one query from the partial results of its splits: one workgroup per query, D/4 lanes of four columns times
-// 1024/D groups of splits.  All loads of a thread are independent, so the kernel is one memory latency long.
-template <int D> __global__ __launch_bounds__(256) void cache_merge_kernel(CacheArgs a) {
-  constexpr int CL = D / 4, SG = 256 / CL;
-  __shared__ float red[SG][D + 4];
-  const int tid = threadIdx.x, d = 4 * (tid % CL), sg = tid / CL;
-  const int64_t row = blockIdx.x, slot = row * a.splits;
-  float m = CACHE_NO_KEY, l = 0.f;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = sg; s < a.splits; s += SG) {
-    const f32x2 ml = *reinterpret_cast<const f32x2 *>(a.pml + 2 * (slot + s));
-    const f32x4 y = *reinterpret_cast<const f32x4 *>(a.po + (slot + s) * D + d);
-    const float m_new = fmaxf(m, ml[0]), s0 = __builtin_amdgcn_exp2f(m - m_new), s1 = __builtin_amdgcn_exp2f(ml[0] - m_new);
-    m = m_new;
-    l = l * s0 + ml[1] * s1;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] = acc[e] * s0 + y[e] * s1;
-  }
-  *reinterpret_cast<f32x4 *>(&red[sg][d]) = acc;
-  if (tid % CL == 0) {
-    red[sg][D] = m;
-    red[sg][D + 1] = l;
-  }
-  __syncthreads();
-  if (sg > 0) return;
-  float ma = CACHE_NO_KEY, la = 0.f;
-#pragma unroll
-  for (int s = 0; s < SG; ++s) ma = fmaxf(ma, red[s][D]);
-  acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < SG; ++s) {
-    const float w = __builtin_amdgcn_exp2f(red[s][D] - ma);
-    la += red[s][D + 1] * w;
-    const f32x4 y = *reinterpret_cast<const f32x4 *>(&red[s][d]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] += y[e] * w;
-  }
-  const float inv = 1.0f / la;
-  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
-  store4(static_cast<char *>(a.o) + off * (a.q_dtype == QFA_F32 ? 4 : 2), a.q_dtype, d,
-         f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
-}
-
 // How the keys of a query block are split: as many workgroups as are resident at once (cache_wgs_per_cu;
 // a second, partly filled round would cost a whole one), at least 8 tiles per workgroup.
 static void cache_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
@@ -374,7 +316,7 @@ static void cache_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *spl
 int64_t cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
   int splits, tps;
   cache_split_plan(B * H, Nq, Nk, D, &splits, &tps);
-  return splits > 1 ? B * H * Nq * splits * (int64_t)(D + 2) * 4 : 0;
+  return splits > 1 ? split_partial_bytes(B * H * Nq, splits, D) : 0;
 }
 
 template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, hipStream_t st) {
@@ -400,8 +342,8 @@ template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, 
   cache_fwd_kernel<S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_cache")) return e;
   if (a.splits > 1) {
-    cache_merge_kernel<D><<<dim3((unsigned)(x.B * x.H * x.Nq)), dim3(256), 0, st>>>(a);
-    return check_launch("qfa_attn_fwd_cache (merge)");
+    const SplitMergeArgs m = {a.po, a.pml, a.o, nullptr, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, a.q_dtype};
+    return launch_split_merge<D>(m, x.B * x.H * x.Nq, "qfa_attn_fwd_cache (merge)", st);
   }
   return 0;
 }

@@ -1,0 +1,82 @@
+// Merge of the partial results of an attention whose keys are split over workgroups (shared-KV forward, cache decode).
+#pragma once
+#include "qfa_device.h"
+#include "qfa_host.h"
+
+namespace qfa {
+
+// row maximum of a wave or split that saw no key: finite, so that differences of two of them are zero and not NaN
+constexpr float NO_KEY = -1e30f;
+
+// four consecutive outputs of a row, rounded to the queries' type
+__device__ __forceinline__ void store4(void *row, int q_dtype, int d, f32x4 x) {
+  if (q_dtype == QFA_F32) {
+    *reinterpret_cast<f32x4 *>(static_cast<float *>(row) + d) = x;
+  } else {
+    u32x2 w;
+    if (q_dtype == QFA_BF16) w = u32x2{pack2<__bf16>(x[0], x[1]), pack2<__bf16>(x[2], x[3])};
+    else w = u32x2{pack2<_Float16>(x[0], x[1]), pack2<_Float16>(x[2], x[3])};
+    *reinterpret_cast<u32x2 *>(static_cast<unsigned short *>(row) + d) = w;
+  }
+}
+
+struct SplitMergeArgs {
+  const float *po, *pml;   // [B*H*Nq][splits][D] unnormalised O, and (m in log2 units, l)
+  void *o;
+  float *lse;              // nullable, [B*H*Nq]
+  int64_t H, sob, soh, son;
+  int Nq, splits, o_dtype;
+};
+
+// O of one query from the partial results of its splits: one workgroup per query, D/4 lanes of four columns times
+// 1024/D groups of splits.  All loads of a thread are independent, so the kernel is one memory latency long.
+template <int D> __global__ __launch_bounds__(256) void split_merge_kernel(SplitMergeArgs a) {
+  constexpr int CL = D / 4, SG = 256 / CL;
+  __shared__ float red[SG][D + 4];
+  const int tid = threadIdx.x, d = 4 * (tid % CL), sg = tid / CL;
+  const int64_t row = blockIdx.x, slot = row * a.splits;
+  float m = NO_KEY, l = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = sg; s < a.splits; s += SG) {
+    const f32x2 ml = *reinterpret_cast<const f32x2 *>(a.pml + 2 * (slot + s));
+    const f32x4 y = *reinterpret_cast<const f32x4 *>(a.po + (slot + s) * D + d);
+    const float m_new = fmaxf(m, ml[0]), s0 = __builtin_amdgcn_exp2f(m - m_new), s1 = __builtin_amdgcn_exp2f(ml[0] - m_new);
+    m = m_new;
+    l = l * s0 + ml[1] * s1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = acc[e] * s0 + y[e] * s1;
+  }
+  *reinterpret_cast<f32x4 *>(&red[sg][d]) = acc;
+  if (tid % CL == 0) {
+    red[sg][D] = m;
+    red[sg][D + 1] = l;
+  }
+  __syncthreads();
+  if (sg > 0) return;
+  float ma = NO_KEY, la = 0.f;
+#pragma unroll
+  for (int s = 0; s < SG; ++s) ma = fmaxf(ma, red[s][D]);
+  acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < SG; ++s) {
+    const float w = __builtin_amdgcn_exp2f(red[s][D] - ma);
+    la += red[s][D + 1] * w;
+    const f32x4 y = *reinterpret_cast<const f32x4 *>(&red[s][d]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += y[e] * w;
+  }
+  const float inv = 1.0f / la;
+  if (a.lse && d == 0) a.lse[row] = (ma + __log2f(la)) * kLn2;
+  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
+  store4(static_cast<char *>(a.o) + off * (a.o_dtype == QFA_F32 ? 4 : 2), a.o_dtype, d,
+         f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+}
+
+inline int64_t split_partial_bytes(int64_t rows, int splits, int D) { return rows * splits * (int64_t)(D + 2) * 4; }
+template <int D> int launch_split_merge(const SplitMergeArgs &a, int64_t rows, const char *who, hipStream_t st) {
+  split_merge_kernel<D><<<dim3((unsigned)rows), dim3(256), 0, st>>>(a);
+  return check_launch(who);
+}
+
+}  // namespace qfa

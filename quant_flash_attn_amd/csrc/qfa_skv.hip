@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "qfa_host.h"
+#include "qfa_merge.h"
 #include "qfa_skv_common.h"
 
 namespace qfa {
@@ -43,7 +44,7 @@ struct SkvArgs {
   int BH;        // batch * heads
   int splits;    // workgroups sharing the keys of one query block (1: the result goes straight to o / lse)
   int tiles_per_split;
-  float *partial;   // splits > 1: [BH][qblocks][splits][16*D + 32] floats (O^T unnormalised, m in log2 units, l)
+  float *po, *pml;   // splits > 1: partial results per query and split (qfa_merge.h)
 };
 
 // ring depth per wave: three tiles, two at D = 256 (8 KB tiles)
@@ -101,7 +102,7 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
     }
   };
   auto scale_of = [](unsigned w) -> float {
-    return std::is_same<S, float>::value ? __builtin_bit_cast(float, w) : lo_to_f32<T>(w);
+    return scale_to_f32<S>(w);
   };
 #pragma unroll
   for (int i = 0; i < SKV_NBUF - 1; ++i)
@@ -298,21 +299,22 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
       sw[w] = __builtin_amdgcn_exp2f(a_s * (mg[w * MG + 16 * D + q16] - m_all));   // -inf for a wave without tiles
       l_all += mg[w * MG + 16 * D + 16 + q16] * sw[w];
     }
-    if (a.splits > 1) {   // hand the unnormalised block result to the merge kernel
-      float *dst = a.partial + ((int64_t)(bh * a.qblocks + qb) * a.splits + split) * MG;
+    if (a.splits > 1) {   // hand the unnormalised result to the merge kernel
+      if (qi < a.Nq) {
+        const int64_t slot = (tq0 + qi) * a.splits + split;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db) {
+          f32x4 r;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int d = 16 * db + 4 * G + v;
-          float acc = (oacc[db][v] - w_tot) * s0;
+          for (int v = 0; v < 4; ++v) {
+            const int d = 16 * db + 4 * G + v;
+            r[v] = (oacc[db][v] - w_tot) * s0;
 #pragma unroll
-          for (int w = 0; w < 3; ++w) acc += mg[w * MG + d * 16 + q16] * sw[w];
-          dst[d * 16 + q16] = acc;
+            for (int w = 0; w < 3; ++w) r[v] += mg[w * MG + d * 16 + q16] * sw[w];
+          }
+          *reinterpret_cast<f32x4 *>(a.po + slot * D + 16 * db + 4 * G) = r;
         }
-      if (G == 0) {
-        dst[16 * D + q16] = a_s * m_all;
-        dst[16 * D + 16 + q16] = l_all;
+        if (G == 0) *reinterpret_cast<f32x2 *>(a.pml + 2 * slot) = f32x2{a_s * m_all, l_all};
       }
       return;
     }
@@ -340,39 +342,12 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
   }
 }
 
-// Sum of the `splits` partial results of every query block: O = sum_s O_s 2^(m_s - m) / sum_s l_s 2^(m_s - m).
-// One workgroup per (batch*head, query block); thread = (query tid%16, columns tid/16 + 16k).
-template <typename T, int D> __global__ __launch_bounds__(256) void skv_merge_kernel(SkvArgs a) {
-  constexpr int MG = 16 * D + 32;
-  const int bh = blockIdx.x / a.qblocks, qb = blockIdx.x % a.qblocks;
-  const int64_t b = bh / a.H, h = bh % a.H;
-  const int q16 = threadIdx.x % 16, dg = threadIdx.x / 16;
-  const int qi = 16 * qb + q16;
-  const float *src = a.partial + (int64_t)blockIdx.x * a.splits * MG;
-  float m = -INFINITY;
-  for (int s = 0; s < a.splits; ++s) m = fmaxf(m, src[s * MG + 16 * D + q16]);
-  float l = 0.f, acc[D / 16];
-#pragma unroll
-  for (int k = 0; k < D / 16; ++k) acc[k] = 0.f;
-  for (int s = 0; s < a.splits; ++s) {
-    const float w = __builtin_amdgcn_exp2f(src[s * MG + 16 * D + q16] - m);
-    l += src[s * MG + 16 * D + 16 + q16] * w;
-#pragma unroll
-    for (int k = 0; k < D / 16; ++k) acc[k] += src[s * MG + (dg + 16 * k) * 16 + q16] * w;
-  }
-  if (qi >= a.Nq) return;
-  const float inv = 1.0f / l;
-  T *orow = reinterpret_cast<T *>(a.o) + b * a.sob + h * a.soh + (int64_t)qi * a.son;
-#pragma unroll
-  for (int k = 0; k < D / 16; ++k) orow[dg + 16 * k] = (T)(acc[k] * inv);
-  if (dg == 0) a.lse[(int64_t)bh * a.Nq + qi] = (m + __log2f(l)) * kLn2;
-}
-
-// How the keys of one query block are split over workgroups: enough workgroups to fill the chip
-// (about four per CU), never fewer than 8 tiles per workgroup; 1 = no split.
-static void skv_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int *splits, int *tiles_per_split) {
+// How the keys of one query block are split over workgroups: as many as are resident at once (three per CU; a second,
+// partly filled round costs a whole one), at head_dim 256 about four per CU (two are resident); never fewer than 8 tiles
+// per workgroup; 1 = no split.
+static void skv_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
   const int64_t ntiles = (Nk + SKV_TILE - 1) / SKV_TILE, wgs = BH * ((Nq + 15) / 16);
-  int64_t want = wgs >= 512 ? 1 : (1024 + wgs - 1) / wgs;
+  int64_t want = D == 256 ? (wgs >= 512 ? 1 : (1024 + wgs - 1) / wgs) : 768 / wgs;
   if (want > ntiles / 8) want = ntiles / 8;
   if (want < 1) want = 1;
   const int64_t tps = (ntiles + want - 1) / want;
@@ -382,8 +357,8 @@ static void skv_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int *splits, int 
 
 int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
   int splits, tps;
-  skv_split_plan(B * H, Nq, Nk, &splits, &tps);
-  return splits > 1 ? B * H * ((Nq + 15) / 16) * splits * (int64_t)(16 * D + 32) * 4 : 0;
+  skv_split_plan(B * H, Nq, Nk, D, &splits, &tps);
+  return splits > 1 ? split_partial_bytes(B * H * Nq, splits, D) : 0;
 }
 
 template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const SkvAttnArgs &x, hipStream_t st) {
@@ -398,25 +373,29 @@ template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const Skv
   a.qblocks = (int)((x.Nq + 15) / 16);
   a.splits = 1;
   a.tiles_per_split = (int)((x.Nk + SKV_TILE - 1) / SKV_TILE);
-  a.partial = nullptr;
+  a.po = a.pml = nullptr;
   if (x.workspace) {   // validated: large enough for the plan below
-    skv_split_plan(x.B * x.H, x.Nq, x.Nk, &a.splits, &a.tiles_per_split);
-    a.partial = static_cast<float *>(x.workspace);
+    skv_split_plan(x.B * x.H, x.Nq, x.Nk, D, &a.splits, &a.tiles_per_split);
+    a.po = static_cast<float *>(x.workspace);
+    a.pml = a.po + x.B * x.H * x.Nq * a.splits * (int64_t)D;
   }
   const int64_t total = (int64_t)a.qblocks * a.splits * ((a.BH + 7) / 8) * 8;   // ids past batch*heads exit at once
-  if (total > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_fwd_shared_kv: too many query blocks for one launch");
+  if (total > 0x7fffffffLL || (a.splits > 1 && x.B * x.H * x.Nq > 0x7fffffffLL))
+    return set_error(QFA_EUNSUPPORTED, "attn_fwd_shared_kv: too many query blocks for one launch");
   skv_fwd_kernel<T, S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_shared_kv")) return e;
   if (a.splits > 1) {
-    skv_merge_kernel<T, D><<<dim3((unsigned)(a.BH * a.qblocks)), dim3(256), 0, st>>>(a);
-    return check_launch("qfa_attn_fwd_shared_kv (merge)");
+    const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, x.io_dtype};
+    return launch_split_merge<D>(m, x.B * x.H * x.Nq, "qfa_attn_fwd_shared_kv (merge)", st);
   }
   return 0;
 }
 
 template <typename T, int D> static int launch_skv_fwd_td(const SkvAttnArgs &x, hipStream_t st) {
   if (x.scale_dtype == QFA_F32) return launch_skv_fwd_tsd<T, float, D>(x, st);
-  return launch_skv_fwd_tsd<T, T, D>(x, st);   // validated: scale_dtype == io_dtype
+  // validated: the io type, or binary16
+  if (x.scale_dtype == QFA_F16) return launch_skv_fwd_tsd<T, _Float16, D>(x, st);
+  return launch_skv_fwd_tsd<T, T, D>(x, st);
 }
 
 // ---- scratch for callers that cannot allocate --------------------------------------------------------

@@ -120,7 +120,7 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     }
   };
   auto scale_of = [](unsigned w) -> float {
-    return std::is_same<S, float>::value ? __builtin_bit_cast(float, w) : lo_to_f32<_Float16>(w);
+    return scale_to_f32<S>(w);
   };
 #pragma unroll
   for (int i = 0; i < SKVB_NBUF; ++i)

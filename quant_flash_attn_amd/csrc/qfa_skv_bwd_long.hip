@@ -69,7 +69,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
     skv_issue_tile<S, D>(cp, smem + wave_off + slot_idx * SLOT, codes_bh, a.scale, a.zp, tk0, wave + 4 * i, a.Nk, a.scn, lane);
   };
   auto scale_of = [](unsigned w) -> float {
-    return std::is_same<S, float>::value ? __builtin_bit_cast(float, w) : lo_to_f32<_Float16>(w);
+    return scale_to_f32<S>(w);
   };
   const float osc = a.grad_scale ? *a.grad_scale : 1.0f;
   auto pack_out = [&](float x, float y) -> unsigned {
@@ -419,7 +419,7 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
     const unsigned *skp = reinterpret_cast<const unsigned *>(slot + SKV_TILE * D);
     const unsigned skw = skp[lr];
     zw = skp[SKV_TILE + lr];
-    sk = std::is_same<S, float>::value ? __builtin_bit_cast(float, skw) : lo_to_f32<_Float16>(skw);
+    sk = scale_to_f32<S>(skw);
   };
 
   f32x16 dkv[DBW];

@@ -55,6 +55,12 @@ __device__ __forceinline__ u32x2 offset_query_operand(float rs, bool big) {
   return u32x2{pack_h2(-(float)h0, -(float)h1), pack_h2(-(float)h2, 0.f)};
 }
 
+// a token's scale out of the dword its tile copy left (a 16-bit scale in the low half)
+template <typename S> __device__ __forceinline__ float scale_to_f32(unsigned w) {
+  if constexpr (sizeof(S) == 4) return __builtin_bit_cast(float, w);
+  else return lo_to_f32<S>(w);
+}
+
 // ds_read_b64_tr_b8, issued like lds_read_tr16_async: invisible to the compiler's wait bookkeeping
 // (which would make it wait for every direct-to-LDS load in flight); use the result only after
 // lds_wait_all() and through tie().

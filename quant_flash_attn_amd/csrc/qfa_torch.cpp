@@ -510,7 +510,8 @@ std::tuple<Tensor, Tensor> skv_fwd(const Tensor &q_in, const Tensor &codes_in, c
                     "shape mismatch: q ", q_in.sizes(), ", codes ", codes_in.sizes());
   const c10::DeviceGuard guard(q_in.device());
   const int64_t B = q_in.size(0), H = q_in.size(1), Nq = q_in.size(2), D = q_in.size(3), Nk = codes_in.size(2);
-  const bool as_is = scale_in.scalar_type() == at::kFloat || scale_in.scalar_type() == q_in.scalar_type();
+  const bool as_is = scale_in.scalar_type() == at::kFloat || scale_in.scalar_type() == at::kHalf ||
+                     scale_in.scalar_type() == q_in.scalar_type();
   const Tensor s = as_is ? scale_in : scale_in.to(at::kFloat);
   const Tensor scale = flat(s, s.scalar_type(), B * H * Nk, "scale"), zp = flat(zp_in, at::kChar, B * H * Nk, "zero_point");
   const Tensor q = rows16(q_in), codes = rows16(codes_in);
