@@ -1,0 +1,24 @@
+"""The backward kernels at the edges of their tiles: one row less, as many and one more than a step of 32 and a tile of 64
+streamed rows, the 64 (32) rows of a wave and the 256 (128) of a workgroup, with the first visible tile of a wave in any
+place.  Against the closed-form gradients of the CPU oracle; the bar is the backward's (see helpers.py)."""
+import math
+
+import pytest
+import torch
+
+from test_attn_bwd_gpu import _check_grads, _fwd_bwd, _oracle_bwd
+from quant_flash_attn_amd.synthetic import make_inputs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
+@pytest.mark.parametrize("Nq,Nk,causal", [(1, 1, False), (31, 33, True), (32, 64, False), (33, 127, True), (63, 129, False),
+                                          (64, 255, True), (65, 257, False), (96, 256, True), (257, 257, True), (161, 513, True)])
+def test_backward_at_tile_edges(qfa, Nq, Nk, causal, D, dtype):
+    q, k, v, do = make_inputs("offset", 1, 3, max(Nq, Nk), D, seed=Nq + 7 * Nk + D, dtype=dtype)
+    q, do = q[:, :, :Nq].contiguous(), do[:, :, :Nq].contiguous()
+    k, v = k[:, :, :Nk].contiguous(), v[:, :, :Nk].contiguous()
+    sm = 1.0 / math.sqrt(D)
+    qq, kq, o, _, dq, dk, dv = _fwd_bwd(qfa, q, k, v, do, causal, sm)
+    want, spreads = _oracle_bwd(qq, kq, v, do, o, causal, sm)
+    _check_grads("", (dq.cpu(), dk.cpu(), dv.cpu()), want, spreads)
