@@ -2,7 +2,7 @@
 // into AccVGPRs (and copies every score out again) or none, and as C++ values accumulators are copied around wherever
 // control flow joins, without the wait states that a copy behind an MFMA needs when the MFMA is inline assembly.  Here tile
 // i of a wave's accumulators (32x32, 16 registers) IS a[16i : 16i+15]: the statements below name the registers, and every
-// one of them clobbers all 256, so that no value of the compiler's can live in an AccVGPR across one.  The scores and the
+// one of them clobbers all that the kernel has tiles in, so that no value of the compiler's can live there across one.  The scores and the
 // other MFMA results that vector instructions read use the builtins (files that include this are compiled with
 // -amdgpu-mfma-vgpr-form: results in vector registers, wait states by the compiler).
 //
@@ -15,16 +15,18 @@
 
 namespace qfa {
 
-#define QFA_ACC_64 \
+#define QFA_ACC_32 \
   "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
-  "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
+  "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31"
+#define QFA_ACC_64 QFA_ACC_32, \
   "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", \
   "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63"
-#define QFA_ACC_256 QFA_ACC_64, \
+#define QFA_ACC_128 QFA_ACC_64, \
   "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", \
   "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", \
   "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", \
-  "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", \
+  "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127"
+#define QFA_ACC_256 QFA_ACC_128, \
   "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", \
   "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", \
   "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", \
@@ -34,15 +36,22 @@ namespace qfa {
   "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", \
   "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
 
-// tile I += A.B; TILES: the wave's tiles (4: only a0-a63 are taken, for kernels of two waves per SIMD)
+// tile I += A.B; TILES: the wave's tiles (2, 4, 8 or 16 of them take the first 32, 64, 128 or 256
+// AccVGPRs, the compiler has the others)
 template <typename T, int I, int TILES> __device__ __forceinline__ void acc_mfma(u32x4 a, u32x4 b) {
   static_assert(I >= 0 && I < TILES && TILES <= 16, "a wave has 256 AccVGPRs");
 #ifdef __HIP_DEVICE_COMPILE__
 #define QFA_M(TYPE, REGS) \
   asm volatile("v_mfma_f32_32x32x16_" TYPE " a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(16 * I), "n"(16 * I + 15) : REGS)
-  if constexpr (TILES <= 4) {
+  if constexpr (TILES <= 2) {
+    if constexpr (__is_same(T, __bf16)) QFA_M("bf16", QFA_ACC_32);
+    else QFA_M("f16", QFA_ACC_32);
+  } else if constexpr (TILES <= 4) {
     if constexpr (__is_same(T, __bf16)) QFA_M("bf16", QFA_ACC_64);
     else QFA_M("f16", QFA_ACC_64);
+  } else if constexpr (TILES <= 8) {
+    if constexpr (__is_same(T, __bf16)) QFA_M("bf16", QFA_ACC_128);
+    else QFA_M("f16", QFA_ACC_128);
   } else {
     if constexpr (__is_same(T, __bf16)) QFA_M("bf16", QFA_ACC_256);
     else QFA_M("f16", QFA_ACC_256);
@@ -60,7 +69,9 @@ template <int I, int TILES> __device__ __forceinline__ void acc_zero_tile() {
                "n"(16 * I + 4), "n"(16 * I + 5), "n"(16 * I + 6), "n"(16 * I + 7), "n"(16 * I + 8), "n"(16 * I + 9), \
                "n"(16 * I + 10), "n"(16 * I + 11), "n"(16 * I + 12), "n"(16 * I + 13), "n"(16 * I + 14), "n"(16 * I + 15) \
                : REGS)
-  if constexpr (TILES <= 4) QFA_Z16(QFA_ACC_64);
+  if constexpr (TILES <= 2) QFA_Z16(QFA_ACC_32);
+  else if constexpr (TILES <= 4) QFA_Z16(QFA_ACC_64);
+  else if constexpr (TILES <= 8) QFA_Z16(QFA_ACC_128);
   else QFA_Z16(QFA_ACC_256);
 #undef QFA_Z16
 #undef QFA_Z

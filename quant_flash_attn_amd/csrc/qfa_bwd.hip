@@ -1,27 +1,21 @@
-// Backward kernels for gfx950: two staging passes, then two MFMA kernels that recompute
-// P = exp(S - LSE) from the INT8 codes exactly as the forward does.
+// Backward for gfx950: the staging passes here, then two MFMA kernels that recompute P = exp(S - LSE) from the INT8 codes
+// exactly as the forward does.
 //
 //   prep_q       per 64-query tile: delta = rowsum(O o dO) in fp32; Qz^T = ((Qc - zq) * sq)^T as a
 //                16-bit tile [d][query] in the key order the MFMA layouts want; per-query constants
 //   prep_k       per 64-key tile: Kz^T = ((Kc - zk) * sk)^T likewise; per-key constants
 //                (both write into the caller's workspace; every tile is converted and transposed
 //                once instead of once per consuming workgroup)
-//   dq kernel    one workgroup = 128 queries (32 per wave), loops over 64-key tiles.
-//                S^T = Kc.Qc^T (INT8 MFMA), dP^T = V.dO^T, dS^T = P^T o (dP^T - delta),
-//                dQ^T += Kz^T.dS^T                with Kz = (Kc - zk) * sk, the dequantized K rounded to 16 bits
-//   dkdv kernel  one workgroup = 128 keys (32 per wave), loops over 64-query tiles.
-//                S = Qc.Kc^T (INT8 MFMA), dP = dO.V^T, dV^T += dO^T.P (dO^T read out of the dO tile by
-//                the transposing LDS reads),
-//                dK^T += Qz^T.dS                  with Qz = (Qc - zq) * sq, the dequantized Q rounded to 16 bits
+//   dK / dV      qfa_bwd_dkv.hip: a workgroup owns keys and streams query tiles
+//   dQ           qfa_bwd_dq.hip: a workgroup owns queries and streams key tiles
 // In both, the wave's own operand (queries resp. keys) stays in registers as the MFMA B operand
 // for the whole loop and the streamed operand comes from LDS as the A operand.  The 32x32
 // accumulator layout then leaves P / dS in registers exactly in the B-operand layout of the next
-// product; the transposed LDS tiles (Kz^T, Qz^T) are written in the matching permuted order.
+// product; the transposed tiles (Kz^T, Qz^T) are written in the matching permuted order.
 // dQ is produced by its own kernel instead of atomics, so results are deterministic.
 // The scales of the streamed operand are folded into its transposed 16-bit tile (Kz^T, Qz^T) by the staging
 // pass, so dS is used as it comes: the tiles then hold the dequantized K and Q rounded to the 16-bit type, the
-// operands an unquantized backward would use.  The dK/dV kernel is bound by LDS reads (48 KB per 32x32 block
-// and wave pair, 16 KB of it per-query constants), and the fold takes one constant vector out of its loop.
+// operands an unquantized backward would use.
 #include <type_traits>
 
 #include "qfa_bwd_common.h"
@@ -218,8 +212,8 @@ template <typename T, int D> __global__ __launch_bounds__(256) void bwd_prep_k_k
       sreg[r] = a.sk[tk0 + j];
     }
     // the dequantized K, rounded to the 16-bit type (what dQ = sm * dS K^ contracts with)
-    store_codes_transposed<T>(creg, zreg, sreg,
-                              [&](int e) { return blob + (dc * 8 + e) * (BWD_TILE * 2) + perm_pos4(r4) * 2; });
+    const int pos = perm_pos4(r4);
+    store_codes_transposed<T>(creg, zreg, sreg, [&](int e) { return blob + qt_offset<D>(dc * 8 + e, pos); });
   }
   if (tid < BWD_TILE) {
     const int j = min(j0 + tid, a.Nk - 1);
@@ -231,203 +225,6 @@ template <typename T, int D> __global__ __launch_bounds__(256) void bwd_prep_k_k
     reinterpret_cast<u32x2 *>(ck)[tid] = dg;
     reinterpret_cast<float *>(ck)[2 * BWD_TILE + tid] = a.sk[tk0 + j];
   }
-}
-
-// ------------------------------------------------------------------------------------------ dQ
-// Threads per workgroup (32 queries per wave) and waves per SIMD the registers are budgeted for.  D=128:
-// 8 waves = 256 queries, one workgroup per CU (two 41 KB tile buffers).  D=64: the loop fits 170 registers
-// and the buffers 42 KB, so three workgroups of 4 waves run per CU (3 waves per SIMD; backward of
-// B16 H16 N2048 D64 causal 0.90 -> 0.84 ms against 8-wave workgroups, 2-wave ones are slower again).
-// D=256: 4 waves, one per SIMD (128 accumulators, 96 operand registers), two 41 KB buffers of 32-key tiles.
-template <int D> struct DqShape {
-  static constexpr int THREADS = D == 128 ? 512 : 256;
-  static constexpr int WAVES_PER_SIMD = D == 64 ? 3 : D == 128 ? 2 : 1;
-  static constexpr int BLK = 32 * (THREADS / 64);
-};
-
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(DqShape<D>::THREADS, DqShape<D>::WAVES_PER_SIMD) void bwd_dq_kernel(BwdArgs a) {
-  constexpr int DQ_THREADS = DqShape<D>::THREADS, DQ_BLK = DqShape<D>::BLK;
-  typedef BwdWs<D> WS;
-  constexpr int BWD_TILE = WS::TILE, NBLK = BWD_TILE / 32;
-  typedef Swz<D> SK;            // K code rows
-  typedef Swz<2 * D> SV;        // V rows
-  typedef Swz<BWD_TILE * 2> ST; // transposed rows
-  constexpr int KS = D / 32, DB = D / 32, KD = D / 16;
-  constexpr int K_BYTES = BWD_TILE * D, V_BYTES = BWD_TILE * 2 * D, T_BYTES = WS::T_BYTES;
-  constexpr int OFF_V = K_BYTES, OFF_T = OFF_V + V_BYTES, OFF_C = OFF_T + T_BYTES, BUF = OFF_C + WS::CK_BYTES;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * BUF];
-
-  const int L = blockIdx.x;
-  const int vid = (L % 8) * a.blocks_per_xcd + (L / 8);
-  if (vid >= a.total_blocks) return;
-  int bh = vid / a.nblocks;
-  int mb = vid % a.nblocks;
-  if (CAUSAL) {
-    // longest rows first, 2^group_log2 heads at a time (ids cycle through the heads of a group): with one
-    // head after the other the last head's long blocks start while the chip is already draining
-    const int GL = a.group_log2;
-    const int pb = bh >> GL << GL;
-    if (pb + (1 << GL) <= a.total_blocks / a.nblocks) {
-      const int idx = (bh - pb) * a.nblocks + mb;
-      bh = pb + (idx & ((1 << GL) - 1));
-      mb = idx >> GL;
-    }
-    mb = a.nblocks - 1 - mb;
-  }
-  const int64_t b = bh / a.H, h = bh % a.H;
-  const int m0 = mb * DQ_BLK;
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, lr = lane % 32, g = lane / 32;
-
-  const int8_t *qc_bh = a.qc + b * a.sqb + h * a.sqh;
-  const unsigned char *kc_bh = reinterpret_cast<const unsigned char *>(a.kc + b * a.skb + h * a.skh);
-  const unsigned char *v_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh);
-  const T *do_bh = reinterpret_cast<const T *>(a.dout) + b * a.sdob + h * a.sdoh;
-  T *dq_bh = reinterpret_cast<T *>(a.dq) + b * a.sdqb + h * a.sdqh;
-  const unsigned char *wsk_bh = a.ws_k + (int64_t)bh * a.tiles_k * WS::K_BLOB;
-  const unsigned char *wsq_bh = a.ws_q + (int64_t)bh * a.tiles_q * WS::Q_BLOB;
-
-  const int qi = m0 + wave * 32 + lr;
-  const int qi_c = qi < a.Nq ? qi : a.Nq - 1;
-  i32x4 qf[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-    qf[ks] = *reinterpret_cast<const i32x4 *>(qc_bh + (int64_t)qi_c * a.sqn + ks * 32 + g * 16);
-  u32x4 dof[KD];
-#pragma unroll
-  for (int kd = 0; kd < KD; ++kd)
-    dof[kd] = *reinterpret_cast<const u32x4 *>(do_bh + (int64_t)qi_c * a.sdon + kd * 16 + g * 8);
-  // per-query constants prepared by prep_q: correction digits, a = sq*sm*log2e, -lse*log2e, -delta
-  const unsigned *cq = reinterpret_cast<const unsigned *>(wsq_bh + (int64_t)(qi_c / BWD_TILE) * WS::Q_BLOB + WS::T_BYTES);
-  const int ql = qi_c % BWD_TILE;
-  const u32x4 corr_q = {cq[2 * ql + g], 0u, 0u, 0u};
-  const float a_i = __builtin_bit_cast(float, cq[2 * BWD_TILE + ql]);
-  const float nlse2 = __builtin_bit_cast(float, cq[3 * BWD_TILE + ql]);
-  const float ndelta_i = __builtin_bit_cast(float, cq[4 * BWD_TILE + ql]);   // -delta
-  const int q_first = m0 + wave * 32, q_last = q_first + 31;
-
-  int kv_end = a.Nk;
-  const int coff = CAUSAL ? a.Nk - a.Nq : 0;   // causal: query i keeps keys j <= i + coff (mask aligned to the last key)
-  if (CAUSAL) kv_end = min(a.Nk, m0 + DQ_BLK + coff);
-  const int ntiles = (kv_end + BWD_TILE - 1) / BWD_TILE;
-
-  // full tiles: per-thread offsets computed once, one copy instruction per chunk afterwards
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  TileCopy<D, BWD_TILE, DQ_THREADS> cp_k;
-  TileCopy<2 * D, BWD_TILE, DQ_THREADS> cp_v;
-  TileCopy<BWD_TILE * 2, D, DQ_THREADS> cp_t;
-  TileCopy<WS::CK_BYTES, 1, DQ_THREADS, NoSwz<WS::CK_BYTES>> cp_c;
-  cp_k.init((unsigned)a.skn, tid);
-  cp_v.init((unsigned)a.svn * 2u, tid);
-  cp_t.init(BWD_TILE * 2, tid);
-  cp_c.init(0, tid);
-  // the copy of a tile goes out in two halves (one before each 32-key block of the tile in work), so
-  // that the memory pipe is not handed all of it in one burst
-  auto load_tile_a = [&](int t) {
-    unsigned char *base = smem + (t & 1) * BUF;
-    if ((t + 1) * BWD_TILE <= a.Nk) {
-      cp_k.issue(kc_bh + (int64_t)t * BWD_TILE * a.skn, base, wave_u, tid);
-      cp_v.issue(v_bh + (int64_t)t * BWD_TILE * a.svn * 2, base + OFF_V, wave_u, tid);
-    } else {
-      dma_rows<D, BWD_TILE, DQ_THREADS>(kc_bh, a.skn, t * BWD_TILE, a.Nk - 1, base, tid);
-      dma_rows<2 * D, BWD_TILE, DQ_THREADS>(v_bh, a.svn * 2, t * BWD_TILE, a.Nk - 1, base + OFF_V, tid);
-    }
-  };
-  auto load_tile_b = [&](int t) {
-    unsigned char *base = smem + (t & 1) * BUF;
-    const unsigned char *blob = wsk_bh + (int64_t)t * WS::K_BLOB;
-    cp_t.issue(blob, base + OFF_T, wave_u, tid);
-    cp_c.issue(blob + WS::T_BYTES, base + OFF_C, wave_u, tid);
-  };
-  auto load_tile = [&](int t) {
-    load_tile_a(t);
-    load_tile_b(t);
-  };
-
-  f32x16 dqacc[DB];
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) dqacc[db][v] = 0.f;
-
-  // one 32-key block of tile t
-  auto block = [&](int t, int nb, auto masked_tag) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
-    const unsigned char *base = smem + (t & 1) * BUF;
-    const unsigned *dgp = reinterpret_cast<const unsigned *>(base + OFF_C);
-    const float *skp = reinterpret_cast<const float *>(base + OFF_C) + 2 * BWD_TILE;
-    const int j0 = t * BWD_TILE;
-    i32x16 acc;
-    f32x16 dp;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) { acc[v] = 0; dp[v] = ndelta_i; }   // dp = dP^T - delta straight from the MFMAs
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const i32x4 kf = *reinterpret_cast<const i32x4 *>(base + SK::off(32 * nb + lr, 2 * ks + g));
-      acc = mfma_i8(kf, qf[ks], acc);
-    }
-#pragma unroll
-    for (int kd = 0; kd < KD; ++kd) {
-      const u32x4 vf = *reinterpret_cast<const u32x4 *>(base + OFF_V + SV::off(32 * nb + lr, 2 * kd + g));
-      dp = mfma_16b<T>(vf, dof[kd], dp);
-    }
-    f32x16 f;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) f[v] = (float)acc[v];
-    const u32x4 corr_k = {dgp[2 * (32 * nb + lr) + g], 0u, 0u, 0u};
-    f = mfma_16b<T>(corr_k, corr_q, f);
-    float ds[16];
-#pragma unroll
-    for (int aa = 0; aa < 4; ++aa) {
-      const int jl = 32 * nb + 8 * aa + 4 * g;
-      const f32x4 sk4 = *reinterpret_cast<const f32x4 *>(skp + jl);
-#pragma unroll
-      for (int bb = 0; bb < 4; ++bb) {
-        const int v = 4 * aa + bb;
-        float p = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[v] * sk4[bb], nlse2));
-        if (MASKED) {
-          const int j = j0 + jl + bb;
-          if ((CAUSAL && j > qi + coff) || j >= a.Nk) p = 0.f;
-        }
-        ds[v] = p * dp[v];
-      }
-    }
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      u32x4 dsf;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dsf[e] = pack2<T>(ds[8 * hh + 2 * e], ds[8 * hh + 2 * e + 1]);
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const u32x4 ktf = *reinterpret_cast<const u32x4 *>(base + OFF_T + ST::off(32 * db + lr, 4 * nb + 2 * hh + g));
-        dqacc[db] = mfma_16b<T>(ktf, dsf, dqacc[db]);
-      }
-    }
-  };
-
-  load_tile(0);
-  dma_wait();
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const int j0 = t * BWD_TILE;
-#pragma unroll
-    for (int nb = 0; nb < NBLK; ++nb) {
-      if (t + 1 < ntiles) {
-        if (nb == 0) load_tile_a(t + 1);
-        if (nb == NBLK - 1) load_tile_b(t + 1);
-      }
-      const int jb = j0 + 32 * nb;
-      if ((jb >= a.Nk) || (CAUSAL && jb > q_last + coff)) continue;        // wave-uniform
-      if ((CAUSAL && jb + 31 > q_first + coff) || (jb + 32 > a.Nk)) block(t, nb, std::true_type{});
-      else block(t, nb, std::false_type{});
-    }
-    dma_wait();
-    __syncthreads();
-  }
-
-  // dQ leaves as whole rows through LDS (the tile buffers are free after the last barrier)
-  static_assert((DQ_THREADS / 64) * 32 * 2 * D <= 2 * BUF, "output staging fits the tile buffers");
-  store_tile_rows<T, D>(dqacc, a.sm_scale, smem + (tid / 64) * (32 * 2 * D), dq_bh, a.sdqn, q_first, a.Nq, tid % 64);
 }
 
 template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStream_t st) {
@@ -457,25 +254,7 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
   if (int e = check_launch("qfa_attn_bwd (prep k)")) return e;
   // dK, dV
   if (int e = launch_dkv<T, D>(a, BH, x.causal, st)) return e;
-  // dQ
-  {
-    constexpr int DQ_THREADS = DqShape<D>::THREADS, DQ_BLK = DqShape<D>::BLK;
-    a.nblocks = (int)((x.Nq + DQ_BLK - 1) / DQ_BLK);
-    // per head the kernel streams Kc, V and Kz^T (5 bytes per key and d): two to eight heads together, within
-    // about 6 MB (pairs at N=4096, D=128, measured)
-    const int64_t head_bytes_k = x.Nk * (int64_t)D * 5;
-    a.group_log2 = 1;
-    while (a.group_log2 < 3 && (head_bytes_k << (a.group_log2 + 1)) <= (6 << 20)) ++a.group_log2;
-    const int64_t total = (int64_t)a.nblocks * BH;
-    if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many query blocks for one launch");
-    a.total_blocks = (int)total;
-    a.blocks_per_xcd = (a.total_blocks + 7) / 8;
-    const dim3 grid((unsigned)(a.blocks_per_xcd * 8));
-    if (x.causal) bwd_dq_kernel<T, D, true><<<grid, dim3(DQ_THREADS), 0, st>>>(a);
-    else bwd_dq_kernel<T, D, false><<<grid, dim3(DQ_THREADS), 0, st>>>(a);
-    if (int e = check_launch("qfa_attn_bwd (dq)")) return e;
-  }
-  return 0;
+  return launch_dq<T, D>(a, BH, x.causal, st);
 }
 
 int launch_bwd(const AttnArgs &x, hipStream_t st) {

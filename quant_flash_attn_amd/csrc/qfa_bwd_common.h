@@ -1,5 +1,5 @@
-// Workspace layout, arguments and small helpers shared by the backward kernels (qfa_bwd.hip: staging passes and the
-// kernels for head_dim 256; qfa_bwd_dkv.hip: dK / dV).
+// Workspace layout, arguments and small helpers shared by the backward kernels (qfa_bwd.hip: staging passes;
+// qfa_bwd_dkv.hip: dK / dV; qfa_bwd_dq.hip: dQ).
 #pragma once
 #include "qfa_device.h"
 #include "qfa_host.h"
