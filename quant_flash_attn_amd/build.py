@@ -25,9 +25,9 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # whatever quantizes must evaluate its expressions as single IEEE operations (bit-exact codes)
 PER_FILE = {f: ["-ffp-contract=off", "-fno-fast-math"] for f in ("qfa_quant.hip", "qfa_cache.hip")}
-for _f in ("qfa_bwd_dkv.hip", "qfa_bwd_dq.hip"):
+for _f in ("qfa_fwd_wide.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip"):
     PER_FILE[_f] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]   # MFMA results in vector registers (see qfa_acc.h)
-SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_bwd.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
+SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_fwd_wide.hip", "qfa_bwd.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
            "qfa_cache.hip"]
 
 

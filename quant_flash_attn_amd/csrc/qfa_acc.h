@@ -35,6 +35,10 @@ namespace qfa {
   "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223", \
   "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", \
   "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+// eight tiles and up to eight fragments behind them
+#define QFA_ACC_160 QFA_ACC_128, \
+  "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", \
+  "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159"
 
 // tile I += A.B; TILES: the wave's tiles (2, 4, 8 or 16 of them take the first 32, 64, 128 or 256
 // AccVGPRs, the compiler has the others)
@@ -56,6 +60,29 @@ template <typename T, int I, int TILES> __device__ __forceinline__ void acc_mfma
     if constexpr (__is_same(T, __bf16)) QFA_M("bf16", QFA_ACC_256);
     else QFA_M("f16", QFA_ACC_256);
   }
+#undef QFA_M
+#endif
+}
+// A fragments that stay in flight across a branch (an LDS read that the compiler does not know of may not have its register
+// copied or spilled before it arrives): fragment F of eight IS a[128 + 4F : 131 + 4F], behind eight tiles.
+// acc_request: the transposing read of 8 bytes at a0 + OFF and 8 at a1 + OFF + 256, to be waited for by count;
+// acc_mfma_frag: tile I += fragment F . B
+template <int F, int OFF> __device__ __forceinline__ void acc_request(unsigned a0, unsigned a1) {
+  static_assert(F >= 0 && F < 8, "eight fragments");
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("ds_read_b64_tr_b16 a[%2:%3], %0 offset:%6\n\tds_read_b64_tr_b16 a[%4:%5], %1 offset:%7"
+               ::"v"(a0), "v"(a1), "n"(128 + 4 * F), "n"(129 + 4 * F), "n"(130 + 4 * F), "n"(131 + 4 * F), "n"(OFF), "n"(OFF + 256)
+               : QFA_ACC_160, "memory");
+#endif
+}
+template <typename T, int I, int F> __device__ __forceinline__ void acc_mfma_frag(u32x4 b) {
+  static_assert(I >= 0 && I < 8 && F >= 0 && F < 8, "eight tiles, eight fragments");
+#ifdef __HIP_DEVICE_COMPILE__
+#define QFA_M(TYPE) \
+  asm volatile("v_mfma_f32_32x32x16_" TYPE " a[%1:%2], a[%3:%4], %0, a[%1:%2]" ::"v"(b), "n"(16 * I), "n"(16 * I + 15), \
+               "n"(128 + 4 * F), "n"(131 + 4 * F) : QFA_ACC_160)
+  if constexpr (__is_same(T, __bf16)) QFA_M("bf16");
+  else QFA_M("f16");
 #undef QFA_M
 #endif
 }
@@ -91,6 +118,18 @@ template <int R0, int... R> __device__ __forceinline__ f32x16 acc_read_regs(std:
   return f32x16{acc_read_reg<R0 + R>()...};
 }
 template <int I> __device__ __forceinline__ f32x16 acc_read() { return acc_read_regs<16 * I>(std::make_integer_sequence<int, 16>{}); }
+// tiles T0 .. T0 + N - 1 times x (a factor per column); acc_settle() in front of it and behind it
+template <int R> __device__ __forceinline__ void acc_write_reg(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("v_accvgpr_write_b32 a[%1], %0" ::"v"(x), "n"(R) : QFA_ACC_160);
+#endif
+}
+template <int R0, int... R> __device__ __forceinline__ void acc_scale_regs(float x, std::integer_sequence<int, R...>) {
+  (acc_write_reg<R0 + R>(acc_read_reg<R0 + R>() * x), ...);
+}
+template <int T0, int N> __device__ __forceinline__ void acc_scale(float x) {
+  acc_scale_regs<16 * T0>(x, std::make_integer_sequence<int, 16 * N>{});
+}
 __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
 // 32 rows of a row-major tensor from tiles T0 .. T0 + D/32 - 1, scaled and rounded (store_tile_rows)

@@ -293,6 +293,11 @@ template <int OFF> __device__ __forceinline__ u32x2 lds_read_b64_async(unsigned 
   asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
   return r;
 }
+__device__ __forceinline__ unsigned lds_read_b32_async(unsigned addr) {
+  unsigned r;
+  asm volatile("ds_read_b32 %0, %1" : "=v"(r) : "v"(addr));
+  return r;
+}
 // wait until at most N LDS operations of this wave are outstanding; the values named are tied behind the wait
 template <typename A> __device__ __forceinline__ void lds_tie(A &a) { asm volatile("" : "+v"(a)); }
 template <typename A, int K> __device__ __forceinline__ void lds_tie(A (&a)[K]) {

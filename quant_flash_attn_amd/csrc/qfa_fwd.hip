@@ -54,7 +54,8 @@
 // the window -- rows pinned at one end of the code range, e.g. all-positive rows -- runs the instance of the same
 // loop that converts explicitly (2 % slower).
 //
-// Head dimensions 64, 128 and 256 are instances of the same code: three, two and one workgroup per CU.
+// Head dimensions 64 and 128 are instances of this code (three and two workgroups per CU), and so is the stage measurement
+// at 256; the forward at head_dim 256, and long ones at 128, are qfa_fwd_wide.hip's (see launch_fwd_td).
 //
 // V lies in LDS as it does in memory ([key][d] rows, 64-byte quarters XOR-swizzled against bank
 // conflicts) and is transposed on the way out: ds_read_b64_tr_b16 hands lane (d, k-group) four
@@ -727,8 +728,20 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
     if (x.causal) fwd_kernel<T, D, true, true><<<grid, block, 0, st>>>(a);
     else fwd_kernel<T, D, false, true><<<grid, block, 0, st>>>(a);
   } else {
-    if (x.causal) fwd_kernel<T, D, true><<<grid, block, 0, st>>>(a);
-    else fwd_kernel<T, D, false><<<grid, block, 0, st>>>(a);
+    // One wave per SIMD: always at head_dim 256 (4096 causal, 64 heads: 640 -> 515 us; 1500 x 1500, 8 heads: 62 -> 43 us).
+    // At 128, where two waves of this kernel share a SIMD, only long sequences without a mask that fill whole rounds of 256
+    // workgroups with 15/16 of their rows: one workgroup per CU has nothing beside it while it starts and ends
+    // (16384 x 16384, 16 heads: 1740 -> 1645 us; 8192 x 8192, 8 heads: 231 -> 219; 2048 x 2048, 64 heads: the same; causal 4096,
+    // 128 heads: 475 -> 512; 2048 x 2048, 4 heads: 36 -> 51).
+    if constexpr (D == 256) return launch_fwd_wide<T, D>(a, x.B * x.H, x.causal, st);
+    if constexpr (D == 128) {
+      const int64_t BH = x.B * x.H, rounds = ((x.Nq + 255) / 256 * BH + 255) / 256;
+      if (!x.causal && x.Nk >= 4096 && x.Nq * BH * 16 >= rounds * (256 * 256 * 15)) return launch_fwd_wide<T, D>(a, BH, false, st);
+    }
+    if constexpr (D < 256) {
+      if (x.causal) fwd_kernel<T, D, true><<<grid, block, 0, st>>>(a);
+      else fwd_kernel<T, D, false><<<grid, block, 0, st>>>(a);
+    }
   }
   return check_launch("qfa_attn_fwd");
 }

@@ -19,6 +19,9 @@ struct FwdArgs {
   int group_log2;        // causal: log2 of the number of heads whose query blocks are dispatched together
 };
 
+// the kernel with one wave per SIMD (qfa_fwd_wide.hip); it fills in the launch's own fields
+template <typename T, int D> int launch_fwd_wide(FwdArgs a, int64_t BH, bool causal, hipStream_t st);
+
 #ifndef QFA_FWD_WAVES
 #define QFA_FWD_WAVES 4
 #endif
