@@ -133,7 +133,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
     if (a.q_dtype == QFA_F32) Load8<float>::run(static_cast<const float *>(a.q) + off, v);
     else if (a.q_dtype == QFA_BF16) Load8<__bf16>::run(static_cast<const __bf16 *>(a.q) + off, v);
     else Load8<_Float16>::run(static_cast<const _Float16 *>(a.q) + off, v);
-    const QuantRow r = quant_row<LPT>(v, true);
+    const QuantRow r = quant_row<LPT, false>(v, true);
     if (tok < 16) {
       *reinterpret_cast<u32x2 *>(smem + tok * D + sub * 8) = r.codes;
       if (sub == 0) {

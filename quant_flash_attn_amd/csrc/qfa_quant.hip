@@ -63,22 +63,34 @@ __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) 
     const int64_t nn = live[u] ? n : a.N - 1;   // tail lanes re-read the last token, never store
     Load8<T>::run(xb + nn * a.sxn + sub_ld * 8, v[u]);
   }
+  // the per-token results leave through LDS, one token per lane: stored by the lanes that hold them, every store
+  // instruction would carry four tokens (128 columns; 256 heads of 4096 x 128 binary16: 81 -> 76 us)
+  __shared__ float s_scale[TPP * U];
+  __shared__ int s_sum[TPP * U];
+  __shared__ int8_t s_zp[TPP * U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t n = n0 + (int64_t)u * TPP;
-    const QuantRow r = quant_row<LPT>(v[u], !PARTIAL || lane_used);
-    if (live[u] && lane_used) {
-      *reinterpret_cast<u32x2 *>(cb + n * a.scn + sub * 8) = r.codes;
-      if (sub == 0) {
-        const int64_t t = bh * a.N + n;
-        if (a.scale) a.scale[t] = r.scale;
-        a.zp[t] = (int8_t)(int)r.zp;
-        if (a.rowsum) a.rowsum[t] = r.sum;
-        if (a.scale_lp) {
-          if (a.scale_lp_dtype == QFA_F16) reinterpret_cast<_Float16 *>(a.scale_lp)[t] = (_Float16)r.scale;
-          else reinterpret_cast<__bf16 *>(a.scale_lp)[t] = (__bf16)r.scale;
-        }
-      }
+    const QuantRow r = quant_row<LPT, sizeof(T) == 2>(v[u], !PARTIAL || lane_used);
+    if (live[u] && lane_used) *reinterpret_cast<u32x2 *>(cb + n * a.scn + sub * 8) = r.codes;
+    if (sub == 0) {
+      s_scale[u * TPP + tid / LPT] = r.scale;
+      s_sum[u * TPP + tid / LPT] = r.sum;
+      s_zp[u * TPP + tid / LPT] = (int8_t)(int)r.zp;
+    }
+  }
+  __syncthreads();
+  static_assert(TPP * U <= 256, "one token per thread");
+  const int64_t n = chunk * (int64_t)(TPP * U) + tid;
+  if (tid < TPP * U && n < a.N) {
+    const int64_t t = bh * a.N + n;
+    const float scale = s_scale[tid];
+    if (a.scale) a.scale[t] = scale;
+    a.zp[t] = s_zp[tid];
+    if (a.rowsum) a.rowsum[t] = s_sum[tid];
+    if (a.scale_lp) {
+      if (a.scale_lp_dtype == QFA_F16) reinterpret_cast<_Float16 *>(a.scale_lp)[t] = (_Float16)scale;
+      else reinterpret_cast<__bf16 *>(a.scale_lp)[t] = (__bf16)scale;
     }
   }
 }

@@ -6,32 +6,26 @@
 
 namespace qfa {
 
-// One reduction step = one instruction: the lane permute is the DPP modifier of the min / max itself.
-// (Written as asm: through the builtin the permuted value comes back as an integer, and the compiler
-// then spends a v_mov_b32_dpp and a canonicalising v_max on every step.  The s_nop covers the two wait
-// states a DPP read needs after a vector write of the same register, which the compiler does not
-// insert for instructions it cannot see.)
-#define QFA_DPP_STEP(OP, CTRL)                                                                           \
-  asm("s_nop 1\n\t" OP " %0, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(v))
-template <int LPT> __device__ __forceinline__ float group_min(float v) {
-  float r;
-  QFA_DPP_STEP("v_min_f32_dpp", "quad_perm:[1,0,3,2]"); v = r;
-  if (LPT >= 4) { QFA_DPP_STEP("v_min_f32_dpp", "quad_perm:[2,3,0,1]"); v = r; }
-  if (LPT >= 8) { QFA_DPP_STEP("v_min_f32_dpp", "row_half_mirror"); v = r; }
-  if (LPT >= 16) { QFA_DPP_STEP("v_min_f32_dpp", "row_mirror"); v = r; }
-  if (LPT >= 32) v = fminf(v, __shfl_xor(v, 16, 64));
-  return v;
+// Minimum and maximum over the LPT lanes of a token.  One reduction step = one instruction: the lane permute is the DPP
+// modifier of the min / max itself.  (Written as asm: through the builtin the permuted value comes back as an integer, and
+// the compiler then spends a v_mov_b32_dpp and a canonicalising v_max on every step.  A DPP read needs two wait states after
+// a vector write of the same register, which the compiler does not insert for instructions it cannot see: the two chains
+// are each other's first one, an s_nop the second; all steps are one statement, so that nothing comes between.)
+template <int LPT> __device__ __forceinline__ void group_min_max(float &mn, float &mx) {
+#define QFA_STEP(CTRL) \
+  "v_min_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\tv_max_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t"
+#define QFA_QUADS "s_nop 1\n\t" QFA_STEP("quad_perm:[1,0,3,2]") "s_nop 0\n\t" QFA_STEP("quad_perm:[2,3,0,1]")
+  static_assert(LPT >= 4, "a token takes four lanes at least");
+  if constexpr (LPT == 4) asm(QFA_QUADS : "+v"(mn), "+v"(mx));
+  else if constexpr (LPT == 8) asm(QFA_QUADS "s_nop 0\n\t" QFA_STEP("row_half_mirror") : "+v"(mn), "+v"(mx));
+  else asm(QFA_QUADS "s_nop 0\n\t" QFA_STEP("row_half_mirror") "s_nop 0\n\t" QFA_STEP("row_mirror") : "+v"(mn), "+v"(mx));
+  if constexpr (LPT >= 32) {
+    mn = fminf(mn, __shfl_xor(mn, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  }
+#undef QFA_QUADS
+#undef QFA_STEP
 }
-template <int LPT> __device__ __forceinline__ float group_max(float v) {
-  float r;
-  QFA_DPP_STEP("v_max_f32_dpp", "quad_perm:[1,0,3,2]"); v = r;
-  if (LPT >= 4) { QFA_DPP_STEP("v_max_f32_dpp", "quad_perm:[2,3,0,1]"); v = r; }
-  if (LPT >= 8) { QFA_DPP_STEP("v_max_f32_dpp", "row_half_mirror"); v = r; }
-  if (LPT >= 16) { QFA_DPP_STEP("v_max_f32_dpp", "row_mirror"); v = r; }
-  if (LPT >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
-  return v;
-}
-#undef QFA_DPP_STEP
 // integer sum: `old` = 0, the identity of the addition (never used: every lane reads a valid lane),
 // lets the compiler fold the permute into v_add_u32_dpp
 template <int CTRL> __device__ __forceinline__ int dpp_zero(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false); }
@@ -79,13 +73,13 @@ struct QuantRow {
   float scale, zp;
   int sum;
 };
-template <int LPT> __device__ __forceinline__ QuantRow quant_row(const float (&v)[8], bool used) {
+// SHORT: the elements have at most 11 significant bits (16-bit tensors).
+template <int LPT, bool SHORT> __device__ __forceinline__ QuantRow quant_row(const float (&v)[8], bool used) {
 #pragma clang fp contract(off)
   float mn = v[0], mx = v[0];
 #pragma unroll
   for (int e = 1; e < 8; ++e) { mn = fminf(mn, v[e]); mx = fmaxf(mx, v[e]); }
-  mn = group_min<LPT>(mn);
-  mx = group_max<LPT>(mx);
+  group_min_max<LPT>(mn, mx);
   float scale = (mx - mn) / 255.0f;
   scale = (scale == 0.0f) ? 1.0f : scale;
   // Division by the per-token scale.  In the common exponent range the quotient is formed with the
@@ -93,14 +87,16 @@ template <int LPT> __device__ __forceinline__ QuantRow quant_row(const float (&v
   // corrections of the quotient), which gives the correctly rounded x/scale without the per-element
   // operand scaling; outside that range (tiny scale, huge values, NaN) the IEEE `/` is used.
   // Quotients below 2^-30 in magnitude may differ in their last bits, which cannot matter: they
-  // vanish in the addition of the zero point or round to zero.
+  // vanish in the addition of the zero point or round to zero.  Elements of at most 11 significant bits need one
+  // correction only: all 2^33 pairs of such a significand with a scale's were compared with `/` on the GPU, none differs
+  // (neither step depends on the exponents).
   const bool fast = (scale >= 0x1p-60f) && (fmaxf(fabsf(mn), fabsf(mx)) <= 0x1p60f);
   float r = __builtin_amdgcn_rcpf(scale);
   r = __builtin_fmaf(__builtin_fmaf(-scale, r, 1.0f), r, r);
   auto fdiv = [&](float x) -> float {
     float q = x * r;
     q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
-    q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
+    if (!SHORT) q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
     return q;
   };
   // roundf (ties away from zero) in three instructions: add the largest float below one half with the
