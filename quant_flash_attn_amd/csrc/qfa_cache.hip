@@ -133,9 +133,9 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
     if (a.q_dtype == QFA_F32) Load8<float>::run(static_cast<const float *>(a.q) + off, v);
     else if (a.q_dtype == QFA_BF16) Load8<__bf16>::run(static_cast<const __bf16 *>(a.q) + off, v);
     else Load8<_Float16>::run(static_cast<const _Float16 *>(a.q) + off, v);
-    const QuantRow r = quant_row<LPT, false>(v, true);
+    const QuantRow<8> r = quant_row<LPT, false, 8>(v, true);
     if (tok < 16) {
-      *reinterpret_cast<u32x2 *>(smem + tok * D + sub * 8) = r.codes;
+      *reinterpret_cast<u32x2 *>(smem + tok * D + sub * 8) = u32x2{r.codes[0], r.codes[1]};
       if (sub == 0) {
         st_a[tok] = r.scale * a.sm_scale_log2;
         st_z[tok] = (int)r.zp;

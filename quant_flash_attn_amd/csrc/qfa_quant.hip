@@ -7,16 +7,16 @@
 // correctly rounded division and nothing is fused or re-associated: codes and zero points
 // are bit-identical to a CPU evaluation of the same expressions.
 //
-// Mapping: a token of D elements is held by D/8 adjacent lanes, rounded up to a power of two (head dimensions
-// that are not one leave the group's last lanes idle: they hold a second copy of the token's first eight
-// elements, which changes no minimum or maximum, and neither add to the row sum nor store -- the reference
-// masks its tail lanes the same way, asymmetric_quant.py:72-75,97-99) (8 elements = one 16-byte
-// load per lane for 16-bit inputs, two for fp32), so one wave64 load instruction covers
-// 512/D tokens with fully coalesced 16-byte accesses.  The row is read once, kept in
-// registers, reduced with DPP lane permutes inside the lane group (no LDS), and the codes
-// leave as one 8-byte store per lane.  HBM-bound in principle (D*sizeof(in) + D + 9 bytes per token,
-// +2 with the 16-bit scale copy); in practice the exact arithmetic makes VALU issue the limiter, so
-// the per-element instruction count is kept low (see the division and packing notes below).
+// Mapping: a token of D elements is held by D/16 adjacent lanes, each with two pieces of 8 elements D/2 apart, so that a
+// load instruction covers half rows in 16-byte accesses next to each other (two for fp32).  Head dimensions up to 32 and
+// those that are not a power of two take D/8 lanes of one piece, rounded up to a power of two; the idle lanes hold a second
+// copy of the token's first eight elements, which changes no minimum or maximum, and neither add to the row sum nor store
+// (the reference masks its tail lanes the same way, asymmetric_quant.py:72-75,97-99).  The row is read once, kept in
+// registers, reduced with DPP lane permutes inside the lane group, and the codes leave as 8-byte stores.  HBM-bound in
+// principle (D*sizeof(in) + D + 9 bytes per token, +2 with the 16-bit scale copy); the exact arithmetic is about as long, so
+// the instruction count is kept low (see the division and packing notes in qfa_quant_row.h): what a row costs once, every
+// lane of its group computes, hence 16 elements per lane (256 heads of 4096 x 128 binary16: 76 us with 8, 71 us with 16,
+// 405 MB at 5.7 TB/s).
 #include "qfa_host.h"
 #include "qfa_quant_row.h"
 
@@ -37,11 +37,16 @@ struct QuantArgs {
   int D;              // head dimension (a multiple of 8, at most the kernel's DP)
 };
 
-// One block = 256 threads = U passes over 256/(DP/8) tokens of one (b,h) slice.  DP = the head dimension
+// A lane's elements: two pieces of eight where every lane of the group is full
+template <int DP, bool PARTIAL> constexpr int quant_e() { return DP >= 64 && !PARTIAL ? 16 : 8; }
+template <int E> constexpr int quant_u() { return 32 / E; }   // rows a lane holds at once
+
+// One block = 256 threads = U passes over 256/LPT tokens of one (b,h) slice.  DP = the head dimension
 // rounded up to a power of two; PARTIAL: the head dimension is smaller than DP.
-template <typename T, int DP, int U, bool PARTIAL>
+template <typename T, int DP, bool PARTIAL>
 __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) {
-  constexpr int LPT = DP / 8;         // lanes per token
+  constexpr int E = quant_e<DP, PARTIAL>(), U = quant_u<E>();
+  constexpr int LPT = DP / E;         // lanes per token
   constexpr int TPP = 256 / LPT;      // tokens per pass
   const int tid = threadIdx.x;
   const int sub = tid % LPT;
@@ -54,14 +59,20 @@ __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) 
   const T *xb = reinterpret_cast<const T *>(a.x) + b * a.sxb + h * a.sxh;
   int8_t *cb = a.codes + b * a.scb + h * a.sch;
 
-  float v[U][8];
+  float v[U][E];
   bool live[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t n = n0 + (int64_t)u * TPP;
     live[u] = n < a.N;
     const int64_t nn = live[u] ? n : a.N - 1;   // tail lanes re-read the last token, never store
-    Load8<T>::run(xb + nn * a.sxn + sub_ld * 8, v[u]);
+#pragma unroll
+    for (int p = 0; p < E / 8; ++p) {
+      float piece[8];
+      Load8<T>::run(xb + nn * a.sxn + p * (DP / 2) + sub_ld * 8, piece);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[u][8 * p + e] = piece[e];
+    }
   }
   // the per-token results leave through LDS, one token per lane: stored by the lanes that hold them, every store
   // instruction would carry four tokens (128 columns; 256 heads of 4096 x 128 binary16: 81 -> 76 us)
@@ -71,8 +82,12 @@ __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t n = n0 + (int64_t)u * TPP;
-    const QuantRow r = quant_row<LPT, sizeof(T) == 2>(v[u], !PARTIAL || lane_used);
-    if (live[u] && lane_used) *reinterpret_cast<u32x2 *>(cb + n * a.scn + sub * 8) = r.codes;
+    const QuantRow<E> r = quant_row<LPT, sizeof(T) == 2, E>(v[u], !PARTIAL || lane_used);
+    if (live[u] && lane_used) {
+#pragma unroll
+      for (int p = 0; p < E / 8; ++p)
+        *reinterpret_cast<u32x2 *>(cb + n * a.scn + p * (DP / 2) + sub * 8) = u32x2{r.codes[2 * p], r.codes[2 * p + 1]};
+    }
     if (sub == 0) {
       s_scale[u * TPP + tid / LPT] = r.scale;
       s_sum[u * TPP + tid / LPT] = r.sum;
@@ -80,7 +95,7 @@ __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) 
     }
   }
   __syncthreads();
-  static_assert(TPP * U <= 256, "one token per thread");
+  static_assert(TPP * U == 8192 / DP && TPP * U <= 256, "one token per thread, the launcher's count of them");
   const int64_t n = chunk * (int64_t)(TPP * U) + tid;
   if (tid < TPP * U && n < a.N) {
     const int64_t t = bh * a.N + n;
@@ -95,8 +110,8 @@ __device__ __forceinline__ void quant_block(const QuantArgs &a, unsigned block) 
   }
 }
 
-template <typename T, int DP, int U, bool PARTIAL> __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
-  quant_block<T, DP, U, PARTIAL>(a, blockIdx.x);
+template <typename T, int DP, bool PARTIAL> __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
+  quant_block<T, DP, PARTIAL>(a, blockIdx.x);
 }
 // Two tensors of one element type and head dimension in one launch (the queries and the keys of an attention call):
 // the first blocks0 workgroups take tensor 0, the others tensor 1.  One launch ramp and one tail instead of two.
@@ -104,21 +119,20 @@ struct QuantPairArgs {
   QuantArgs t[2];
   unsigned blocks0;
 };
-template <typename T, int DP, int U, bool PARTIAL> __global__ __launch_bounds__(256) void quant_pair_kernel(QuantPairArgs p) {
-  if (blockIdx.x < p.blocks0) quant_block<T, DP, U, PARTIAL>(p.t[0], blockIdx.x);
-  else quant_block<T, DP, U, PARTIAL>(p.t[1], blockIdx.x - p.blocks0);
+template <typename T, int DP, bool PARTIAL> __global__ __launch_bounds__(256) void quant_pair_kernel(QuantPairArgs p) {
+  if (blockIdx.x < p.blocks0) quant_block<T, DP, PARTIAL>(p.t[0], blockIdx.x);
+  else quant_block<T, DP, PARTIAL>(p.t[1], blockIdx.x - p.blocks0);
 }
 
 template <typename T, int DP> static int launch_quant_d(const QuantArgs &a0, int64_t BH, hipStream_t st) {
-  constexpr int U = 4;
-  constexpr int TOK = (256 / (DP / 8)) * U;
+  constexpr int TOK = 8192 / DP;   // tokens per workgroup, however they are held
   QuantArgs a = a0;
   const int64_t chunks = (a.N + TOK - 1) / TOK;
   if (chunks * BH > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "quant: too many tokens for one launch");
   a.chunks_per_bh = (int)chunks;
   const dim3 grid((unsigned)(chunks * BH)), block(256);
-  if (a.D == DP) quant_kernel<T, DP, U, false><<<grid, block, 0, st>>>(a);
-  else quant_kernel<T, DP, U, true><<<grid, block, 0, st>>>(a);
+  if (a.D == DP) quant_kernel<T, DP, false><<<grid, block, 0, st>>>(a);
+  else quant_kernel<T, DP, true><<<grid, block, 0, st>>>(a);
   return check_launch("qfa_quant_per_token");
 }
 // head dimension rounded up to a power of two (the lane groups the reductions run over), 32 at least
@@ -149,8 +163,7 @@ int launch_quant(const void *x, int x_dtype, int8_t *codes, float *scale, void *
 }
 
 template <typename T, int DP> static int launch_quant_pair_d(QuantPairArgs p, int64_t BH, hipStream_t st) {
-  constexpr int U = 4;
-  constexpr int TOK = (256 / (DP / 8)) * U;
+  constexpr int TOK = 8192 / DP;   // tokens per workgroup, however they are held
   int64_t blocks[2];
   for (int i = 0; i < 2; ++i) {
     const int64_t chunks = (p.t[i].N + TOK - 1) / TOK;
@@ -160,8 +173,8 @@ template <typename T, int DP> static int launch_quant_pair_d(QuantPairArgs p, in
   if (blocks[0] + blocks[1] > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "quant_pair: too many tokens for one launch");
   p.blocks0 = (unsigned)blocks[0];
   const dim3 grid((unsigned)(blocks[0] + blocks[1])), block(256);
-  if (p.t[0].D == DP) quant_pair_kernel<T, DP, U, false><<<grid, block, 0, st>>>(p);
-  else quant_pair_kernel<T, DP, U, true><<<grid, block, 0, st>>>(p);
+  if (p.t[0].D == DP) quant_pair_kernel<T, DP, false><<<grid, block, 0, st>>>(p);
+  else quant_pair_kernel<T, DP, true><<<grid, block, 0, st>>>(p);
   return check_launch("qfa_quant_per_token_pair");
 }
 template <typename T> static int launch_quant_pair_t(const QuantPairArgs &p, int64_t BH, hipStream_t st) {

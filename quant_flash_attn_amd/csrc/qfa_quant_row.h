@@ -65,20 +65,20 @@ template <> struct Load8<_Float16> {
   }
 };
 
-// The row arithmetic: eight elements per lane, a token in LPT adjacent lanes.  Returns the lane's eight codes and, in
+// The row arithmetic: E (8 or 16) elements per lane, a token in LPT adjacent lanes.  Returns the lane's codes and, in
 // every lane of the token, its scale, zero point (an integer in [-128, 127]) and code sum.  `used`: false in the lanes
 // past the row's end (they hold a copy of elements of the row and add nothing to the sum).
-struct QuantRow {
-  u32x2 codes;
+template <int E> struct QuantRow {
+  unsigned codes[E / 4];
   float scale, zp;
   int sum;
 };
 // SHORT: the elements have at most 11 significant bits (16-bit tensors).
-template <int LPT, bool SHORT> __device__ __forceinline__ QuantRow quant_row(const float (&v)[8], bool used) {
+template <int LPT, bool SHORT, int E> __device__ __forceinline__ QuantRow<E> quant_row(const float (&v)[E], bool used) {
 #pragma clang fp contract(off)
   float mn = v[0], mx = v[0];
 #pragma unroll
-  for (int e = 1; e < 8; ++e) { mn = fminf(mn, v[e]); mx = fmaxf(mx, v[e]); }
+  for (int e = 1; e < E; ++e) { mn = fminf(mn, v[e]); mx = fmaxf(mx, v[e]); }
   group_min_max<LPT>(mn, mx);
   float scale = (mx - mn) / 255.0f;
   scale = (scale == 0.0f) ? 1.0f : scale;
@@ -105,34 +105,37 @@ template <int LPT, bool SHORT> __device__ __forceinline__ QuantRow quant_row(con
   auto round_away = [](float y) -> float {
     return __builtin_truncf(y + __builtin_copysignf(0x1.fffffep-2f, y));
   };
-  float q[8], qmn;
+  float q[E], qmn;
   if (fast) {
     qmn = fdiv(mn);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) q[e] = fdiv(v[e]);
+    for (int e = 0; e < E; ++e) q[e] = fdiv(v[e]);
   } else {
     qmn = mn / scale;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) q[e] = v[e] / scale;
+    for (int e = 0; e < E; ++e) q[e] = v[e] / scale;
   }
   const float zpf = -128.0f - qmn;
   const float zp = fmaxf(-128.0f, fminf(127.0f, round_away(zpf)));
   // codes leave as biased bytes: roundf(.) + 128 converted with unsigned saturation (= the clamp to
   // [-128, 127]), flipped back to two's complement with one XOR per dword
-  u32x2 w = {0u, 0u};
+  QuantRow<E> row;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
+  for (int e = 0; e < E; ++e) {
     const float y = q[e] + zp;
     const float c = round_away(y) + 128.0f;
-    w[e / 4] = __builtin_amdgcn_cvt_pk_u8_f32(c, e % 4, w[e / 4]);
+    row.codes[e / 4] = __builtin_amdgcn_cvt_pk_u8_f32(c, e % 4, e % 4 == 0 ? 0u : row.codes[e / 4]);
   }
-  int sum = (int)__builtin_amdgcn_sad_u8(w[0], 0u, 0u);
-  sum = (int)__builtin_amdgcn_sad_u8(w[1], 0u, (unsigned)sum) - 8 * 128;
-  if (!used) sum = 0;
-  w[0] ^= 0x80808080u;
-  w[1] ^= 0x80808080u;
-  sum = group_sum<LPT>(sum);
-  return {w, scale, zp, sum};
+  unsigned sum = 0;
+#pragma unroll
+  for (int i = 0; i < E / 4; ++i) {
+    sum = __builtin_amdgcn_sad_u8(row.codes[i], 0u, sum);
+    row.codes[i] ^= 0x80808080u;
+  }
+  row.sum = group_sum<LPT>(used ? (int)sum - E * 128 : 0);
+  row.scale = scale;
+  row.zp = zp;
+  return row;
 }
 
 }  // namespace qfa
