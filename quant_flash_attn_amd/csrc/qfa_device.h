@@ -164,19 +164,6 @@ template <int ROW_BYTES> struct SwzQuad {
   static __device__ __forceinline__ int swz(int row) { return 4 * ((row / RPL) % QPR); }
 };
 
-// Layout for a [row][d] tile of 16-bit floats that is read BOTH ways: row-wise (16 lanes = 16 consecutive
-// rows at one logical chunk) and through the transposing reads (32 lanes = 4 consecutive rows x 64
-// contiguous bytes).  The row's low bits move the 64-byte quarter, bits 2-3 the chunk inside the quarter, so
-// either pattern lands on 16 different 16-byte slots of the 256-byte bank line.
-template <int ROW_BYTES> struct SwzDual {
-  static_assert(ROW_BYTES == 512 || ROW_BYTES == 256 || ROW_BYTES == 128, "rows of 256, 128 or 64 16-bit floats");
-  static constexpr int CPR = ROW_BYTES / 16;
-  // the part of the XOR that moves quarters (a function of the row's low bits only)
-  static __device__ __forceinline__ int quarter(int row) { return ROW_BYTES >= 256 ? (row & 3) : ((row >> 1) & 1); }
-  static __device__ __forceinline__ int swz(int row) { return (quarter(row) << 2) | ((row >> 2) & 3); }
-  static __device__ __forceinline__ int off(int r, int c) { return r * ROW_BYTES + ((c ^ swz(r)) << 4); }
-};
-
 // rows [row0, row0+ROWS) (clamped to row_max) of a row-major global array -> swizzled LDS tile; NT threads
 template <int ROW_BYTES, int ROWS, int NT, typename S = Swz<ROW_BYTES>>
 __device__ __forceinline__ void dma_rows(const unsigned char *g, int64_t gstride, int row0, int row_max,
@@ -248,23 +235,6 @@ template <int ROW_BYTES, int ROWS, int NT, typename S = Swz<ROW_BYTES>> struct T
     for (int i = 0; i < N; ++i) issue_one(rs, lds, wave_u, i);
   }
 };
-// dense swizzle-free layout for TileCopy (contiguous bytes)
-template <int ROW_BYTES> struct NoSwz {
-  static constexpr int CPR = ROW_BYTES / 16;
-  static __device__ __forceinline__ int swz(int) { return 0; }
-};
-
-// BYTES contiguous bytes, copied as they are
-template <int BYTES, int NT>
-__device__ __forceinline__ void dma_flat(const unsigned char *g, unsigned char *lds, int tid) {
-  constexpr int TOTAL = BYTES / 16;
-#pragma unroll
-  for (int i = 0; i < (TOTAL + NT - 1) / NT; ++i) {
-    const int p = tid + NT * i;
-    if (TOTAL % NT == 0 || p < TOTAL)
-      __builtin_amdgcn_global_load_lds((gptr_t)(g + p * 16), (lptr_t)(lds + ((tid & ~63) + NT * i) * 16), 16, 0, 0);
-  }
-}
 // all direct loads of this wave have landed (vmcnt(0)); follow with a barrier before other waves read
 __device__ __forceinline__ void dma_wait() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 // ds_read_b64_tr_b16: inside each group of 16 lanes, lane i receives element i%4 of the four 8-byte
@@ -282,15 +252,10 @@ template <int OFF> __device__ __forceinline__ u32x2 lds_read_tr16_async(unsigned
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
   return r;
 }
-// The same for plain 16-byte and 8-byte reads (a loop that times every LDS request itself issues all of them this way)
+// The same for plain 16-byte and 4-byte reads (a loop that times every LDS request itself issues all of them this way)
 template <int OFF> __device__ __forceinline__ u32x4 lds_read_b128_async(unsigned addr) {
   u32x4 r;
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
-  return r;
-}
-template <int OFF> __device__ __forceinline__ u32x2 lds_read_b64_async(unsigned addr) {
-  u32x2 r;
-  asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFF));
   return r;
 }
 __device__ __forceinline__ unsigned lds_read_b32_async(unsigned addr) {
