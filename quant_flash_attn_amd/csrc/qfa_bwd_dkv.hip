@@ -18,7 +18,7 @@
 // so that no product waits for the vector work it depends on.  What bounds it: the instructions one wave can issue (about
 // 5 cycles each, 16 + 2 MFMAs' worth of vector work per block against 29 MFMAs of 32 cycles), then power.
 // Measured, the whole backward before and after: 16384 x 16384, 16 heads of 128: 6.70 -> 5.81 ms (matrix pipe of this kernel
-// busy 42 -> 68 % of the time, at 1.83 GHz); 4096 causal, 128 heads of 128: 1.97 -> 1.79; 64 heads of 256: 2.74 -> 2.31;
+// busy 42 -> 72 % of the time, at 1.85 GHz); 4096 causal, 128 heads of 128: 1.97 -> 1.79; 64 heads of 256: 2.74 -> 2.31;
 // 2048 causal, 256 heads of 64: 0.737 -> 0.68 (there exponentials and vector work take longer than the products).
 //
 // LDS layout of a tile.  Rows of codes and of dO are cut into slabs of 32 bytes: slab s holds bytes 32s..32s+31 of every

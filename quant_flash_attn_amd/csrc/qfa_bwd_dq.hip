@@ -15,7 +15,7 @@
 // operands come out of LDS at 1 KB per MFMA: with one block the LDS reads take as long as the products.  At head_dim 256 the
 // operands and accumulators of one block fill the registers; at 64 two waves of one block share a SIMD, since its exponentials
 // take longer than its products.  Bound by the instructions a wave can issue (74 vector instructions beside 21 MFMAs of 32
-// cycles per 32 x 32 block; matrix pipe busy about 65 %), then by power.
+// cycles per 32 x 32 block; matrix pipe busy 72 % at 1.85 GHz on the long sequence below, 54 % on the causal one), then by power.
 // Measured, this kernel alone against the one before it (32 queries per wave, scheduled by the compiler, no bias trick):
 // 16384 x 16384, 16 heads of 128: 2890 -> 2200 us; 4096 causal, 128 heads of 128: 789 -> 650; 64 heads of 256: 1276 -> 789;
 // 2048 causal, 256 heads of 64: 251 -> 226.
@@ -188,15 +188,8 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
         f[qb][v] = __builtin_fmaf(a_i[qb], f[qb][v] * sk[aa % 2][2 * (x % 2)], nlse[qb]);
         f[qb][v + 1] = __builtin_fmaf(a_i[qb], f[qb][v + 1] * sk[aa % 2][2 * (x % 2) + 1], nlse[qb]);
       } else {
-        float x0 = __builtin_amdgcn_exp2f(f[qb][v]);
-        float x1 = __builtin_amdgcn_exp2f(f[qb][v + 1]);
-        if constexpr (MASKED) {
-          const int j = j0 + 8 * aa + 2 * (x % 2);
-          x0 = j <= k_hi[qb] ? x0 : 0.f;
-          x1 = j + 1 <= k_hi[qb] ? x1 : 0.f;
-        }
-        f[qb][v] = x0;
-        f[qb][v + 1] = x1;
+        f[qb][v] = __builtin_amdgcn_exp2f(f[qb][v]);
+        f[qb][v + 1] = __builtin_amdgcn_exp2f(f[qb][v + 1]);
       }
       // the scales of quad aa + 2 replace those of aa behind their last use
       constexpr int last0 = QB == 2 ? 10 : 2, last1 = QB == 2 ? 14 : 6;
@@ -205,7 +198,13 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
     };
     auto ds_dword = [&](auto k_tag) __attribute__((always_inline)) {
       constexpr int k = decltype(k_tag)::value, qb = k / 4 % QB, hh = k / (4 * QB), e = k % 4, v = 8 * hh + 2 * e;
-      ds_out[qb][hh][e] = pack2<T>(f[qb][v] * dp[qb][v], f[qb][v + 1] * dp[qb][v + 1]);
+      float x0 = f[qb][v] * dp[qb][v], x1 = f[qb][v + 1] * dp[qb][v + 1];
+      if constexpr (MASKED) {   // dS and not P: dP of a masked pair may be anything (V may be infinite there)
+        const int j = j0 + 8 * (v / 4) + v % 4;
+        x0 = j <= k_hi[qb] ? x0 : 0.f;
+        x1 = j + 1 <= k_hi[qb] ? x1 : 0.f;
+      }
+      ds_out[qb][hh][e] = pack2<T>(x0, x1);
     };
     // the copy's pieces are spread over the slots behind the turn of the tile
     TileDesc td;

@@ -22,3 +22,16 @@ def test_backward_at_tile_edges(qfa, Nq, Nk, causal, D, dtype):
     qq, kq, o, _, dq, dk, dv = _fwd_bwd(qfa, q, k, v, do, causal, sm)
     want, spreads = _oracle_bwd(qq, kq, v, do, o, causal, sm)
     _check_grads("", (dq.cpu(), dk.cpu(), dv.cpu()), want, spreads)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
+def test_infinite_value_row_stays_with_the_queries_that_see_it(qfa, D, dtype):
+    """The last key's V row is infinite: O and dQ of the query blocks of 32 that end before it stay finite (a block that
+    the diagonal cuts multiplies the masked probabilities with it)."""
+    N = 128
+    q, k, v, do = make_inputs("normal", 1, 2, N, D, seed=D, dtype=dtype)
+    v[:, :, -1] = float("inf")
+    _, _, o, _, dq, _, _ = _fwd_bwd(qfa, q, k, v, do, True, 1.0 / math.sqrt(D))
+    assert torch.isfinite(o[:, :, :96].float()).all() and torch.isfinite(dq[:, :, :96].float()).all()
+    assert not torch.isfinite(o[:, :, -1].float()).all()
