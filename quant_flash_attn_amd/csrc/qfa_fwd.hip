@@ -728,7 +728,7 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
     if (x.causal) fwd_kernel<T, D, true, true><<<grid, block, 0, st>>>(a);
     else fwd_kernel<T, D, false, true><<<grid, block, 0, st>>>(a);
   } else {
-    // One wave per SIMD: always at head_dim 256 (4096 causal, 64 heads: 640 -> 515 us; 1500 x 1500, 8 heads: 62 -> 43 us).
+    // One wave per SIMD: always at head_dim 256 (4096 causal, 64 heads: 645 -> 560 us; 1500 x 1500, 8 heads: 62 -> 43 us).
     // At 128, where two waves of this kernel share a SIMD, only long sequences without a mask that fill whole rounds of 256
     // workgroups with 15/16 of their rows: one workgroup per CU has nothing beside it while it starts and ends
     // (16384 x 16384, 16 heads: 1740 -> 1645 us; 8192 x 8192, 8 heads: 231 -> 219; 2048 x 2048, 64 heads: the same; causal 4096,
