@@ -218,8 +218,8 @@ int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale
  *   q, o   [B,H,Nq,D] of q_dtype (QFA_F32 / QFA_F16 / QFA_BF16)
  *   kc, vc int8 [B,H,Nk,D];  ks, vs [B*H*Nk] of scale_dtype (QFA_F32 / QFA_F16 / QFA_BF16);  kz, vz int8 [B*H*Nk]
  *   D in {64, 128, 256}; causal, sm_scale, alignment and stride rules as in qfa_attn_fwd (codes as its kc, q and o as
- *   its o).  Range, not checked: the probabilities are multiplied by V's scale before they are packed to binary16
- *   (scales up to about 4e3).
+ *   its o).  V may be of any size: the products of probability and scale are normalised per query before they are packed
+ *   to binary16.
  *   workspace  nullable (never split then); else qfa_attn_fwd_cache_workspace_bytes(...) bytes, 16-byte aligned (0: no
  *              split pays): the keys of a query block are split over several workgroups whose partial results a second
  *              small kernel merges.

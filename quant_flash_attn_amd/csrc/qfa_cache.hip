@@ -18,6 +18,10 @@
 //        and one byte permute plus one XOR turn a pair of keys at one d into two binary16 numbers 1152 + code exactly
 //        (qfa_skv_common.h); MFMA i of the D/16 takes byte i, so its row r is d = (D/16) * r + i.
 //   The offset 1152 + zero point is removed through sum_j (1152 + zp_j) p'_j, accumulated over the rounded p' = p * scale_j.
+//   p' enters the product as binary16, and the scales carry V's magnitude, so each query keeps a factor beta for p' beside
+//   its reference maximum for p: the largest p' * beta seen is at least 1 and at most 2^15, whatever V's size, and beta is
+//   taken out of O once at the end.  (Without it V of size 1e-3 put p' among binary16's subnormals: relative error of O
+//   1.8e-2, 1.7e-1 at 1e-4, where dequantizing V first leaves 3e-3 in bf16; and scales above 4e3 overflowed.)
 // Per-token scales and zero points pass through 512 bytes of LDS per wave, which turns one load per token into the
 // broadcast the accumulator layout wants.
 #include <type_traits>
@@ -42,6 +46,8 @@ struct CacheArgs {
 // Workgroups per CU the registers are budgeted for: two tiles in registers (80 of them at head_dim 128, 148 at 256) beside
 // the accumulators.  With one tile per wave in flight that keeps 64 KB (48 at head_dim 64) per CU under way.
 constexpr int cache_wgs_per_cu(int D) { return D == 256 ? 1 : D == 128 ? 2 : 3; }
+
+constexpr float CACHE_P_MAX = 0x1p15f;   // largest p * scale * beta (binary16 ends at 65504)
 
 __device__ __forceinline__ i32x4 mfma_i8_16(i32x4 a, i32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
@@ -156,6 +162,9 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
 #pragma unroll
   for (int i = 0; i < DB; ++i) oacc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_ref = -INFINITY, m_bound = -INFINITY, nm = 0.f, l_run = 0.f, w_run = 0.f;
+  // oacc and w_run hold sums of p * scale_j * beta; p * scale_j above ps_bound would leave binary16.  (Nothing summed yet: any
+  // beta will do, and the largest leaves only p * scale_j <= 2^-105 as it is.)
+  float beta = 0x1p120f, ps_bound = CACHE_P_MAX * 0x1p-120f;
   const float thr = SKV_RESCALE_THRESHOLD / a_i;
   unsigned *tc = reinterpret_cast<unsigned *>(smem + OFF_TC + wave * 512);   // [64] x (scale, zero point operand)
   const i32x4 ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
@@ -196,35 +205,58 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
       mt = fmaxf(mt, __shfl_xor(mt, 16, 64));   // the reference maximum is common to the four lanes of a query
       mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
       const float m_new = fmaxf(m_ref, mt);
-      const float alpha = m_new == m_ref ? 1.0f : __builtin_amdgcn_exp2f(a_i * (m_ref - m_new));
+      const float old = m_ref, alpha = m_new == old ? 1.0f : __builtin_amdgcn_exp2f(a_i * (old - m_new));
       m_ref = m_new;
       m_bound = m_new + thr;
       nm = m_new == -INFINITY ? 0.f : -a_i * m_new;   // a query that has seen no key yet
       l_run *= alpha;
-      w_run *= alpha;
-#pragma unroll
-      for (int j = 0; j < DB; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) oacc[j][v] *= alpha;
+      // oacc and w_run stay as they are: what shrinks is p, by alpha
+      const float grow = m_new == old ? 1.0f : __builtin_amdgcn_exp2f(fminf(a_i * (m_new - old), 120.0f));
+      beta = fminf(beta * grow, 0x1p120f);
+      ps_bound = CACHE_P_MAX * __builtin_amdgcn_rcpf(beta);
     }
-    // ---- p, p' = p * scale_j as binary16, row sum, offset term
-    u32x4 pf;
+    // ---- p and its row sum; p * scale_j and the largest of them
+    float ps[8], mx = 0.f;
+    unsigned zz[4];   // the binary16 numbers 1152 + zero point
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
-      const u32x4 c0 = *reinterpret_cast<const u32x4 *>(tc + 2 * (32 + 16 * rb + 4 * G)),
-                  c1 = *reinterpret_cast<const u32x4 *>(tc + 2 * (32 + 16 * rb + 4 * G) + 4);
+      const unsigned *c = tc + 2 * (32 + 16 * rb + 4 * G);
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const u32x4 c = e == 0 ? c0 : c1;
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[rb][2 * e], nm));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[rb][2 * e + 1], nm));
+      for (int v = 0; v < 4; v += 2) {
+        const u32x4 w = *reinterpret_cast<const u32x4 *>(c + 2 * v);
+        const unsigned s0 = w[0], z0 = w[1], s1 = w[2], z1 = w[3];   // (a bit cast of a vector's element takes element 0)
+        zz[2 * rb + v / 2] = z0 | (z1 << 16);
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[rb][v], nm));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[rb][v + 1], nm));
         l_run += p0 + p1;
-        const unsigned s0 = c[0], z0 = c[1], s1 = c[2], z1 = c[3];
-        const unsigned pp = pack_h2(p0 * __builtin_bit_cast(float, s0), p1 * __builtin_bit_cast(float, s1));
-        pf[2 * rb + e] = pp;
-        const unsigned zz = z0 | (z1 << 16);
-        w_run = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pp), __builtin_bit_cast(f16x2, zz), w_run, false);
+        ps[4 * rb + v] = p0 * __builtin_bit_cast(float, s0);
+        ps[4 * rb + v + 1] = p1 * __builtin_bit_cast(float, s1);
+        mx = fmaxf(mx, fmaxf(fabsf(ps[4 * rb + v]), fabsf(ps[4 * rb + v + 1])));
       }
+    }
+    if (__builtin_amdgcn_ballot_w64(mx > ps_bound) != 0) {
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));   // beta is common to the four lanes of a query
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      if (mx > ps_bound) {   // the power of two that brings mx to [1, 2)
+        const int e = (int)(__builtin_bit_cast(unsigned, mx) >> 23);
+        const float b_new = __builtin_bit_cast(float, (unsigned)min(max(254 - e, 7), 247) << 23);
+        const float gamma = b_new * __builtin_amdgcn_rcpf(beta);
+        beta = b_new;
+        ps_bound = CACHE_P_MAX * __builtin_amdgcn_rcpf(beta);
+        w_run *= gamma;
+#pragma unroll
+        for (int j = 0; j < DB; ++j)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) oacc[j][v] *= gamma;
+      }
+    }
+    // ---- p' = p * scale_j * beta as binary16, offset term
+    u32x4 pf;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const unsigned pp = pack_h2(ps[2 * x] * beta, ps[2 * x + 1] * beta);
+      pf[x] = pp;
+      w_run = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pp), __builtin_bit_cast(f16x2, zz[x]), w_run, false);
     }
     // ---- O^T += (1152 + codes)^T . P'^T
 #pragma unroll
@@ -254,6 +286,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
   float l_tot = l_run + __shfl_xor(l_run, 16, 64), w_tot = w_run + __shfl_xor(w_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
   w_tot += __shfl_xor(w_tot, 32, 64);
+  const float inv_beta = __builtin_amdgcn_rcpf(beta);
   __syncthreads();   // query codes and token constants are done with
   float *mg = reinterpret_cast<float *>(smem), *ml = mg + 4 * 16 * D;
   if (q16 < nqv) {
@@ -264,7 +297,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
       for (int j = 0; j < DB; j += 4) {
         f32x4 x;
 #pragma unroll
-        for (int y = 0; y < 4; ++y) x[y] = oacc[j + y][v] - w_tot;
+        for (int y = 0; y < 4; ++y) x[y] = (oacc[j + y][v] - w_tot) * inv_beta;
         *reinterpret_cast<f32x4 *>(dst + VB * (4 * G + v) + j) = x;
       }
     if (G == 0) {

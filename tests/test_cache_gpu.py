@@ -90,6 +90,62 @@ def test_growing_scores_and_one_sided_rows(qfa):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("dtype,sdtype,size", [
+    (torch.bfloat16, torch.float16, 1.0), (torch.bfloat16, torch.float16, 1e-2), (torch.bfloat16, torch.float16, 1e-4),
+    (torch.float16, torch.float16, 1e-3), (torch.float32, torch.float16, 1e-4), (torch.bfloat16, torch.float16, 1e6),
+    (torch.bfloat16, torch.float32, 1e-20), (torch.bfloat16, torch.bfloat16, 1e20), (torch.bfloat16, torch.float32, "ramp"),
+    (torch.bfloat16, torch.float32, "masked out"), (torch.float32, torch.float32, "rising scores")])
+def test_size_of_the_values(qfa, D, dtype, sdtype, size):
+    """V of any size, alike for all keys or not: values that grow by 2^40 along the keys, large values at keys that hardly
+    any query attends to, and scores that rise (by hundreds) while the values fall.
+
+    Bound: as above, but every term is weighted with the probabilities (the scales differ by key), and binary16's smallest
+    step, 2^-24, is one of the largest p_j scale_j of the row, once per key, times |code - zero point| <= 255."""
+    B, H, Nq, Nk = 1, 3, 5, 2100
+    q, k, v, _ = make_inputs("normal", B, H, Nk, D, seed=D, dtype=torch.float32)
+    q, sm = q[:, :, :Nq].to(dtype), 1.0 / math.sqrt(D)
+    ramp = torch.arange(Nk).view(1, 1, -1, 1) / Nk
+    if size == "ramp":
+        v = v * 2.0 ** (40 * ramp - 20)
+    elif size == "masked out":     # scores near -40 at the keys with large values, in the first tile and later
+        q = (q.float().abs() + 0.5).to(dtype)
+        far = (ramp < 0.01) | ((ramp > 0.5) & (ramp < 0.52))
+        k = torch.where(far, -40 * sm * torch.ones_like(k), k * 0.1)
+        v = torch.where(far, v * 1e5, v)
+    elif size == "rising scores":
+        q = (q.float().abs() + 0.5).to(dtype)
+        k, v = k * 0.1 + 40 * ramp, v * 2.0 ** (-60 * ramp)
+    else:
+        v = v * size
+    kq = tuple(t.to(DEV) for t in oracle.quantize_per_token_c(k)[:3])
+    vc, vs, vz, _ = oracle.quantize_per_token_c(v)
+    kq = (kq[0], kq[1].to(sdtype), kq[2])
+    vq = (vc.to(DEV), vs.to(sdtype).to(DEV), vz.to(DEV))
+    none = torch.empty(0, dtype=dtype, device=DEV)
+    with torch.no_grad():
+        o = qfa.quant_flash_attn_quantized_kv(q.to(DEV), none, none, kq, vq, True, sm).cpu()
+    f64 = lambda c, s, z: oracle.dequantize_per_token(c.cpu(), s.cpu(), z.cpu(), torch.float64)   # noqa: E731
+    qh, kh, vh = f64(*oracle.quantize_per_token_c(q)[:3]), f64(*kq), f64(*vq)
+    want, lse = oracle.attn_fwd(qh, kh, vh, True, sm)
+    s = (qh @ kh.transpose(-1, -2)) * sm
+    seen = torch.arange(Nk) <= torch.arange(Nq).view(-1, 1) + Nk - Nq
+    p = torch.where(seen, torch.exp(s - lse[..., None]), torch.zeros(()).double())
+    ps = p * vq[1].cpu().double().reshape(B, H, 1, Nk)
+    size_of = p @ vh.abs()
+    # (fp32 scores: a rounding of the largest |score| in the exponent, twice)
+    bound = (OUT_ULP[dtype] * want.abs() + (2.0 ** -10 + 2.0 ** -22 * float(s.abs().max())) * size_of
+             + ((32 + Nk / 32) * 2.0 ** -24 * (1152 + 255) * ps.sum(-1, keepdim=True))
+             + Nk * 255 * 2.0 ** -25 * ps.max(-1, keepdim=True).values)
+    if dtype == torch.float16:
+        bound = bound + 2.0 ** -25
+    excess = (o.double() - want).abs() - bound
+    assert torch.isfinite(o.float()).all() and excess.max() <= 0, (
+        f"over the bound by {(excess / bound).max().item():.2f} times it; relative error "
+        f"{float((o.double() - want).norm() / want.norm()):.2e}")
+
+
+@pytest.mark.gpu
 def test_graph_capture_and_replay(qfa):
     q, k, v, _ = (t.to(DEV) for t in make_inputs("offset", 1, 4, 4096, 128, seed=3))
     q = q[:, :, :1].contiguous()
