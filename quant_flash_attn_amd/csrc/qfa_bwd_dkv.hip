@@ -179,6 +179,12 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     const int rowb = buf + row_l + mbk * 1024;
     const int cb = cq_a(buf, mbk);
     const int i0 = TILE * t + 32 * mbk + 4 * g;
+    // dO^T is zero for the key blocks that none of the step's queries sees (the first tile of a wave may hold such steps): P
+    // is zero there, and dO may be infinite
+    constexpr bool UNSEEN = MASKED && CAUSAL && (NSTEP > 1 || KB > 1);
+    unsigned dv_mask[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) dv_mask[kb] = TILE * t + 32 * mbk + 31 >= k_first + 32 * kb - coff ? ~0u : 0u;
 
     // ---- the vector work of P, in 16 KB half items dealt to the MFMA slots: scaling of a pair of scores and packing of the
     // pair before it (even), exponentials (odd).  Pairs in an order that lets two quads' constants serve all key blocks:
@@ -283,7 +289,12 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     constexpr int DSW = 8 * KB;   // dwords of dS
     auto ds_dword = [&](auto k_tag) __attribute__((always_inline)) {
       constexpr int k = decltype(k_tag)::value, kb = k / 8, hh = k / 4 % 2, e = k % 4, v = 8 * hh + 2 * e;
-      ds[kb][hh][e] = pack2<T>(f[kb][v] * dp[kb][v], f[kb][v + 1] * dp[kb][v + 1]);
+      float x0 = f[kb][v] * dp[kb][v], x1 = f[kb][v + 1] * dp[kb][v + 1];
+      if constexpr (MASKED) {   // a masked pair has P = 0, but its dP may be anything: dO may be infinite there
+        x0 = f[kb][v] == 0.f ? 0.f : x0;
+        x1 = f[kb][v + 1] == 0.f ? 0.f : x1;
+      }
+      ds[kb][hh][e] = pack2<T>(x0, x1);
     };
     // S comes before the last dV fragment, whose MFMAs cover the time its results take
     constexpr int NV = 2 * DB, V1 = NV - 1;
@@ -297,9 +308,14 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
       if constexpr (n + 2 < NV) lds_wait_for<4>(w);
       else if constexpr (n + 1 < NV) lds_wait_for<2>(w);
       else lds_wait_for<0>(w);
-      const u32x4 g4 = {w[0][0], w[0][1], w[1][0], w[1][1]};
+      u32x4 g4 = {w[0][0], w[0][1], w[1][0], w[1][1]};
       static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
         constexpr int kb = decltype(kb_tag)::value, m = KB * n + kb;
+        if constexpr (UNSEEN) {   // (a later key block is seen by fewer queries)
+          g4 &= dv_mask[kb];
+          QFA_FENCE();
+          asm volatile("s_nop 1");
+        }
         QFA_FENCE();
         acc_mfma<T, DV0 + kb * DB + n % DB, ACC>(g4, pf[kb][n / DB]);
         QFA_FENCE();

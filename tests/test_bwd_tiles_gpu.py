@@ -35,3 +35,24 @@ def test_infinite_value_row_stays_with_the_queries_that_see_it(qfa, D, dtype):
     _, _, o, _, dq, _, _ = _fwd_bwd(qfa, q, k, v, do, True, 1.0 / math.sqrt(D))
     assert torch.isfinite(o[:, :, :96].float()).all() and torch.isfinite(dq[:, :, :96].float()).all()
     assert not torch.isfinite(o[:, :, -1].float()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
+@pytest.mark.parametrize("H,Nq,Nk", [(2, 128, 128), (256, 256, 256), (256, 193, 300)])
+@pytest.mark.parametrize("row", [0, 37, 70, 127])
+def test_infinite_output_gradient_stays_with_the_keys_that_its_query_sees(qfa, D, dtype, H, Nq, Nk, row):
+    """One dO row is infinite: dQ of the other queries stays finite, and so does dK of every key that the query does not see;
+    dV of the key blocks of 32 that its block of 32 queries does not see at all (a block that the diagonal cuts multiplies
+    the masked probabilities with it).  256 heads: 64 keys per wave at head_dim 128."""
+    q, k, v, do = make_inputs("normal", 1, H, Nk, D, seed=D + row, dtype=dtype)
+    q, do = q[:, :, :Nq].contiguous(), do[:, :, :Nq].contiguous()
+    do[:, :, row] = float("inf")
+    _, _, _, _, dq, dk, dv = _fwd_bwd(qfa, q, k, v, do, True, 1.0 / math.sqrt(D))
+    off = Nk - Nq
+    block = (row // 32 * 32 + 31 + off) // 32 * 32 + 32   # first key block behind what the query's block sees
+    others = [i for i in range(Nq) if i != row]
+    assert torch.isfinite(dq[:, :, others].float()).all()
+    assert torch.isfinite(dk[:, :, row + off + 1:].float()).all()
+    assert torch.isfinite(dv[:, :, block:].float()).all()
+    assert not torch.isfinite(dv[:, :, :row + off + 1].float()).all()
