@@ -462,7 +462,10 @@ template <typename S> __device__ __forceinline__ float max_abs_chunk(const u32x4
     return max_abs8<S>(w, m);
   } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(__builtin_bit_cast(float, w[e])));
+    for (int e = 0; e < 4; ++e) {
+      const unsigned x = w[e];   // (this compiler's bit cast of a vector's element takes element 0)
+      m = fmaxf(m, fabsf(__builtin_bit_cast(float, x)));
+    }
     return m;
   }
 }

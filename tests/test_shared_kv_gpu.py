@@ -214,6 +214,17 @@ def test_dout_normalisation_through_the_c_abi(qfa, dtype, sdtype, do_scale, kv_s
         assert top <= 2.0 ** 14 and (top * float(smax) > 4.0 * (1 - 1e-6) or top > 2.0 ** 13)
 
 
+@pytest.mark.parametrize("sdtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("at", list(range(8)) + [1003, 1004])
+def test_dout_normalisation_finds_the_largest_scale_at_any_position(qfa, sdtype, at):
+    from quant_flash_attn_amd.quant_flash_attn import _normalised_dout
+    do = torch.ones(1, 1, 4, 64, dtype=torch.float16, device=DEV)
+    sc = torch.full((1, 1, 1005, 1), 2.0 ** -5, dtype=sdtype, device=DEV)
+    sc[0, 0, at] = 2.0
+    do16, back = _normalised_dout(do, sc)
+    assert float(back.cpu()) == 2.0 ** -2 and float(do16[0, 0, 0, 0].cpu()) == 4.0   # 1 * 2^2 * 2 = 8
+
+
 def test_shared_kv_entry_point_long_query_block(qfa):
     """97 queries (a reference test shape, test_accuracy.py:44): the forward splits them over workgroups
     of 16, the backward runs its dQ and dKV kernels."""
