@@ -8,7 +8,9 @@
 // Nothing is kept between calls.
 #include <ATen/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
+#include <torch/library.h>
 
 #include <array>
 #include <string>
@@ -348,6 +350,22 @@ bool wants_grad(std::initializer_list<const Tensor *> ts) {
   return false;
 }
 
+// The operators have no forward-mode derivative: a tangent is refused, with or without a backward gradient beside it (an
+// input that needs none does not reach the autograd node, which would refuse it).
+void refuse_tangents(std::initializer_list<const Tensor *> ts) {
+  for (const Tensor *t : ts)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->_fw_grad(0).defined(),
+                                "quant_flash_attn_amd: forward-mode differentiation (jvp) is not implemented for this operator");
+}
+// A call that is being traced goes through the dispatcher, which records the operator as one node of the graph (what the
+// function below does by itself is invisible there but for its allocations); others save themselves that round trip.
+template <typename F> struct Traced;
+template <typename... A> struct Traced<Tensor(A...)> {
+  static Tensor call(const char *name, A... args) {
+    return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Tensor(A...)>().call(args...);
+  }
+};
+
 // forward results that the backward needs: the pair buffer (codes, scales, zero points, row sums, LSE), v and o in 16 bit
 struct Kept {
   Tensor buf, v16, o16, o;
@@ -394,13 +412,18 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
             to(g[2], (at::ScalarType)(dt >> 16)), Tensor(), Tensor()};
   }
 };
-Tensor qkv(const Tensor &q, const Tensor &k, const Tensor &v, bool causal, double sm) {
+Tensor qkv_op(const Tensor &q, const Tensor &k, const Tensor &v, bool causal, double sm) {
+  refuse_tangents({&q, &k, &v});
   require_gpu(q, k, v);
   TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q, k, v must be 4-D (Batch, Heads, Seq, Head_Dim)");
   TORCH_CHECK_VALUE(q.size(3) == k.size(3) && k.sizes() == v.sizes() && q.size(0) == k.size(0) && q.size(1) == k.size(1),
                     "shape mismatch: q ", q.sizes(), ", k ", k.sizes(), ", v ", v.sizes());
   if (wants_grad({&q, &k, &v})) return QkvFn::apply(q, k, v, causal, sm);
   return qkv_forward(q, k, v, causal, sm).o;
+}
+Tensor qkv(const Tensor &q, const Tensor &k, const Tensor &v, bool causal, double sm) {
+  if (torch::jit::tracer::isTracing()) return Traced<decltype(qkv_op)>::call("quant_flash_attn_amd::qkv", q, k, v, causal, sm);
+  return qkv_op(q, k, v, causal, sm);
 }
 
 // ---- q and an INT8 cache of keys and values
@@ -488,8 +511,9 @@ struct CacheFn : torch::autograd::Function<CacheFn> {
     return out;
   }
 };
-Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc, const Tensor &ks,
-             const Tensor &kz, const Tensor &vc, const Tensor &vs, const Tensor &vz, bool causal, double sm) {
+Tensor cache_op(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc, const Tensor &ks,
+                const Tensor &kz, const Tensor &vc, const Tensor &vs, const Tensor &vz, bool causal, double sm) {
+  refuse_tangents({&q, &k_fp16, &v_fp16});
   require_gpu(q, kc, ks, kz, vc, vs, vz);
   TORCH_CHECK_VALUE(q.dim() == 4 && kc.dim() == 4 && kc.sizes() == vc.sizes() && q.size(3) == kc.size(3) &&
                         q.size(0) == kc.size(0) && q.size(1) == kc.size(1),
@@ -497,6 +521,13 @@ Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const 
   if (wants_grad({&q, &k_fp16, &v_fp16})) return CacheFn::apply(q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz, causal, sm);
   if (q.size(2) <= CACHE_MAX_Q) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
   return cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm).o;
+}
+Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc, const Tensor &ks,
+             const Tensor &kz, const Tensor &vc, const Tensor &vs, const Tensor &vz, bool causal, double sm) {
+  if (torch::jit::tracer::isTracing())
+    return Traced<decltype(cache_op)>::call("quant_flash_attn_amd::quantized_kv", q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz,
+                                            causal, sm);
+  return cache_op(q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz, causal, sm);
 }
 
 // ------------------------------------------------------------------------------------------- shared K = V
@@ -638,8 +669,9 @@ struct SharedLongFn : torch::autograd::Function<SharedLongFn> {
   }
 };
 // max_q: longest query block for the shared-KV kernels at this head dimension
-Tensor shared(const Tensor &q, const Tensor &kv_fp16, const Tensor &codes, const Tensor &scale, const Tensor &zp, double sm,
-              int64_t max_q) {
+Tensor shared_op(const Tensor &q, const Tensor &kv_fp16, const Tensor &codes, const Tensor &scale, const Tensor &zp, double sm,
+                 int64_t max_q) {
+  refuse_tangents({&q, &kv_fp16});
   require_gpu(q, codes, scale, zp);
   TORCH_CHECK_VALUE(q.dim() == 4 && codes.sizes() == kv_fp16.sizes() && codes.dim() == 4 && q.size(3) == codes.size(3),
                     "shape mismatch: q ", q.sizes(), ", kv ", kv_fp16.sizes(), ", codes ", codes.sizes());
@@ -648,8 +680,23 @@ Tensor shared(const Tensor &q, const Tensor &kv_fp16, const Tensor &codes, const
   return grad ? SharedLongFn::apply(q, kv_fp16, codes, scale, zp, sm)
               : cache_forward(q, codes, scale, zp, codes, scale, zp, false, sm).o;
 }
+Tensor shared(const Tensor &q, const Tensor &kv_fp16, const Tensor &codes, const Tensor &scale, const Tensor &zp, double sm,
+              int64_t max_q) {
+  if (torch::jit::tracer::isTracing())
+    return Traced<decltype(shared_op)>::call("quant_flash_attn_amd::shared_kv", q, kv_fp16, codes, scale, zp, sm, max_q);
+  return shared_op(q, kv_fp16, codes, scale, zp, sm, max_q);
+}
 
 }  // namespace
+
+// (no backend key: the operators attach their autograd nodes themselves)
+TORCH_LIBRARY(quant_flash_attn_amd, m) {
+  m.def("qkv(Tensor q, Tensor k, Tensor v, bool causal, float sm_scale) -> Tensor", &qkv_op);
+  m.def("quantized_kv(Tensor q, Tensor k_fp16, Tensor v_fp16, Tensor k_codes, Tensor k_scale, Tensor k_zero_point, "
+        "Tensor v_codes, Tensor v_scale, Tensor v_zero_point, bool causal, float sm_scale) -> Tensor", &cache_op);
+  m.def("shared_kv(Tensor q, Tensor kv_fp16, Tensor codes, Tensor scale, Tensor zero_point, float sm_scale, int max_q) -> Tensor",
+        &shared_op);
+}
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   typedef py::call_guard<py::gil_scoped_release> nogil;
