@@ -12,7 +12,10 @@ import os
 import subprocess
 import sys
 import sysconfig
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
+
+from . import acc_check
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -25,8 +28,10 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # whatever quantizes must evaluate its expressions as single IEEE operations (bit-exact codes)
 PER_FILE = {f: ["-ffp-contract=off", "-fno-fast-math"] for f in ("qfa_quant.hip", "qfa_cache.hip")}
-for _f in ("qfa_fwd_wide.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip"):
-    PER_FILE[_f] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]   # MFMA results in vector registers (see qfa_acc.h)
+# accumulators in AccVGPRs by hand (see qfa_acc.h): other MFMA results in vector registers, and the assembly is checked
+BY_HAND = ("qfa_fwd_wide.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip")
+for _f in BY_HAND:
+    PER_FILE[_f] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_fwd_wide.hip", "qfa_bwd.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
            "qfa_cache.hip"]
 
@@ -41,6 +46,31 @@ def _hipcc() -> str:
 def _compile(src: str, extra=()) -> str:
     obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
     cmd = [_hipcc(), *COMMON, *PER_FILE.get(src, []), *extra, "-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj]
+    if src in BY_HAND:
+        return _compile_checked(src, cmd, obj)
+    _run(src, cmd)
+    return obj
+
+
+def assembly_path(src: str) -> str:
+    """The device assembly that the build keeps of a file in BY_HAND."""
+    return os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".s")
+
+
+def _compile_checked(src: str, cmd, obj: str) -> str:
+    with tempfile.TemporaryDirectory(dir=OBJ_DIR) as tmp:
+        made = os.path.join(tmp, os.path.basename(obj))
+        _run(src, [*cmd[:-1], made, "--save-temps=obj"])
+        asm, = (f for f in os.listdir(tmp) if f.endswith("gfx950.s"))
+        os.replace(os.path.join(tmp, asm), assembly_path(src))
+        found = acc_check.check(assembly_path(src))
+        if found:
+            raise RuntimeError(f"{src}: the compiler's output breaks the rules of qfa_acc.h:\n" + "\n".join(found))
+        os.replace(made, obj)
+    return obj
+
+
+def _run(src: str, cmd) -> None:
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{res.stdout}\n{res.stderr}")
@@ -49,7 +79,6 @@ def _compile(src: str, extra=()) -> str:
     for line in res.stderr.splitlines():
         if line.strip() and not any(n in line for n in noise):
             print(line, file=sys.stderr)
-    return obj
 
 
 def _compile_host_module() -> str:

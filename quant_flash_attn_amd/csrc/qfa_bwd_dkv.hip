@@ -316,6 +316,8 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
           QFA_FENCE();
           asm volatile("s_nop 1");
         }
+        // (at head_dim 64 the last pair of P is packed in the slot before the first product that reads it)
+        if constexpr (m == 2 && n / DB == 1 && !UNSEEN) asm volatile("s_nop 1");
         QFA_FENCE();
         acc_mfma<T, DV0 + kb * DB + n % DB, ACC>(g4, pf[kb][n / DB]);
         QFA_FENCE();
