@@ -1,10 +1,14 @@
 """Checks the assembly of the kernels that keep accumulators in AccVGPRs by hand (csrc/qfa_acc.h), as the compiler wrote it.
 
-The compiler does not see the hazards of their inline MFMAs.  So the build looks at what it made of them:
+Their inline MFMAs name AccVGPRs that the compiler does not know to hold anything between two statements, and it does not
+see these MFMAs' hazards.  So the build looks at what it made of them:
 
-  1. a vector instruction that writes A or B of an inline MFMA is followed by at least two wait states before it, and one that
+  1. no instruction of the compiler's touches a register that inline assembly uses as an AccVGPR, between the statements
+     or anywhere else in the kernel (it may use the others);
+  2. a vector instruction that writes A or B of an inline MFMA is followed by at least two wait states before it, and one that
      writes an accumulator likewise;
-  2. an accumulator is read, or written by a vector instruction, no earlier than 20 wait states behind an MFMA that writes it.
+  3. an accumulator is read, or written by a vector instruction, no earlier than 20 wait states behind an MFMA that writes it;
+  4. these kernels spill nothing: an LDS request that the compiler does not know of may not have its registers moved.
 
     python -m quant_flash_attn_amd.acc_check FILE.s
 """
@@ -55,7 +59,7 @@ def _parse_instr(line: int, text: str, inline: bool) -> Instr:
 
 
 def _kernels(path: str):
-    """(name, instructions, label -> index) of every kernel in an assembly file."""
+    """(name, instructions, label -> index, bytes of scratch) of every kernel in an assembly file."""
     name, instrs, labels, inline = None, [], {}, False
     with open(path) as f:
         for n, raw in enumerate(f, 1):
@@ -72,7 +76,7 @@ def _kernels(path: str):
                 for part in text.split("\n"):
                     instrs.append(_parse_instr(n, part.strip().replace("\t", " "), inline))
             elif name and text.startswith(".amdhsa_private_segment_fixed_size"):
-                yield name, instrs, labels
+                yield name, instrs, labels, int(text.split()[1])
                 name = None
 
 
@@ -83,11 +87,13 @@ def _wait_states(i: Instr) -> int:
 def check(path: str) -> List[str]:
     """What is wrong, one line each; empty: nothing."""
     bad: List[str] = []
-    for name, ins, labels in _kernels(path):
+    for name, ins, labels, scratch in _kernels(path):
         acc = {r for i in ins if i.inline for r in i.reads | i.writes if r[0] == "a"}
         if not acc:
             continue
         tell = lambda i, what: bad.append(f"{path}:{i.line}: {name}: {what}: {i.text}")   # noqa: E731
+        if scratch:
+            bad.append(f"{path}: {name}: {scratch} bytes of scratch")
         before: Dict[int, List[int]] = {}
         for k, i in enumerate(ins):
             if k + 1 < len(ins) and i.op not in ("s_branch", "s_endpgm", "s_setpc_b64"):
@@ -112,6 +118,8 @@ def check(path: str) -> List[str]:
         valu = lambda i: i.op.startswith("v_") and not mfma(i)              # noqa: E731
         for k, i in enumerate(ins):
             used = i.reads | i.writes
+            if not i.inline and used & acc:
+                tell(i, "the compiler uses an accumulator's register")
             if i.inline and mfma(i):
                 if written_within(k, i.reads | i.writes, VALU_TO_MFMA, valu):
                     tell(i, f"an operand is written less than {VALU_TO_MFMA} wait states earlier")

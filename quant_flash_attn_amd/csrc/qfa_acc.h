@@ -2,9 +2,12 @@
 // into AccVGPRs (and copies every score out again) or none, and as C++ values accumulators are copied around wherever
 // control flow joins, without the wait states that a copy behind an MFMA needs when the MFMA is inline assembly.  Here tile
 // i of a wave's accumulators (32x32, 16 registers) IS a[16i : 16i+15]: the statements below name the registers, and every
-// one of them clobbers all that the kernel has tiles in, so that no value of the compiler's can live there across one.  The scores and the
-// other MFMA results that vector instructions read use the builtins (files that include this are compiled with
-// -amdgpu-mfma-vgpr-form: results in vector registers, wait states by the compiler).
+// one of them clobbers all that the kernel has tiles in.  That keeps the compiler's values out of them ACROSS a statement; it
+// does not keep it from using one of them between two statements, and there are stretches of a hundred instructions without
+// one.  What does is the build: it reads the assembly of these files and fails if an instruction of the compiler's names a
+// register that a statement uses, anywhere in the kernel, if one of the two rules below is broken, or if anything was
+// spilled (acc_check.py).  The scores and the other MFMA results that vector instructions read use the builtins (files that
+// include this are compiled with -amdgpu-mfma-vgpr-form: results in vector registers, wait states by the compiler).
 //
 // The caller keeps two rules: A and B of acc_mfma were written at least two instructions earlier, and acc_settle() stands
 // between the last acc_mfma and the first acc_read.

@@ -47,6 +47,21 @@ def test_accumulator_used_before_its_mfma_is_done(tmp_path, use, wait, ok):
     assert (not _kernel(tmp_path, "!" + MFMA, *wait, "!" + use)) == ok
 
 
+@pytest.mark.parametrize("line,ok", [("v_accvgpr_write_b32 a15, v9", False), ("v_accvgpr_read_b32 v9, a0", False),
+                                     ("global_load_dwordx4 a[12:15], v[8:9], off", False), ("v_mov_b32_e32 v9, v8", True),
+                                     ("v_accvgpr_write_b32 a16, v9", True), ("ds_write_b128 v9, a[16:19]", True)])
+@pytest.mark.parametrize("place", [0, 2])
+def test_the_compiler_in_an_accumulator(tmp_path, line, ok, place):
+    lines = ["!" + MFMA, "s_nop 15", "s_nop 15", "!" + MFMA]
+    lines.insert(place, line)
+    assert (not _kernel(tmp_path, *lines)) == ok
+
+
+def test_scratch(tmp_path):
+    assert _kernel(tmp_path, "!" + MFMA, scratch=16)
+    assert not _kernel(tmp_path, "v_mov_b32_e32 v9, v8", scratch=16)   # no accumulators by hand: not its business
+
+
 @pytest.mark.parametrize("src", build.BY_HAND)
 def test_the_library_as_built(src):
     asm = build.assembly_path(src)
