@@ -18,10 +18,10 @@
 //        and one byte permute plus one XOR turn a pair of keys at one d into two binary16 numbers 1152 + code exactly
 //        (qfa_skv_common.h); MFMA i of the D/16 takes byte i, so its row r is d = (D/16) * r + i.
 //   The offset 1152 + zero point is removed through sum_j (1152 + zp_j) p'_j, accumulated over the rounded p' = p * scale_j.
-//   p' enters the product as binary16, and the scales carry V's magnitude, so each query keeps a factor beta for p' beside
-//   its reference maximum for p: the largest p' * beta seen is at least 1 and at most 2^15, whatever V's size, and beta is
-//   taken out of O once at the end.  (Without it V of size 1e-3 put p' among binary16's subnormals: relative error of O
-//   1.8e-2, 1.7e-1 at 1e-4, where dequantizing V first leaves 3e-3 in bf16; and scales above 4e3 overflowed.)
+//   p' enters the product as binary16, and the scales carry V's magnitude: the reference that p is taken against follows the
+//   largest p', not the largest p, so that p' stays at 2^15 or below with the largest one seen at 2^7 or above, whatever V's
+//   size.  (p <= 1 put p' among binary16's subnormals for small V: relative error of O 1.8e-2 at size 1e-3, 1.7e-1 at 1e-4,
+//   where dequantizing V first leaves 3e-3 in bf16; and scales above 4e3 overflowed.)
 // Per-token scales and zero points pass through 512 bytes of LDS per wave, which turns one load per token into the
 // broadcast the accumulator layout wants.
 #include <type_traits>
@@ -43,17 +43,18 @@ struct CacheArgs {
   int Nq, Nk, BH, qblocks, splits, tiles_per_split, causal, q_dtype;
 };
 
-// Workgroups per CU the registers are budgeted for: two tiles in registers (80 of them at head_dim 128, 148 at 256) beside
-// the accumulators.  With one tile per wave in flight that keeps 64 KB (48 at head_dim 64) per CU under way.
+// Workgroups per CU that a launch counts on: two tiles in registers (80 of them at head_dim 128, 148 at 256) beside the
+// accumulators.  With one tile per wave in flight that keeps 64 KB (48 at head_dim 64) per CU under way.
 constexpr int cache_wgs_per_cu(int D) { return D == 256 ? 1 : D == 128 ? 2 : 3; }
 
-constexpr float CACHE_P_MAX = 0x1p15f;   // largest p * scale * beta (binary16 ends at 65504)
+constexpr float CACHE_P_MAX = 0x1p15f;   // largest p' (binary16 ends at 65504)
+constexpr float CACHE_P_REF = 7.0f;      // log2 of the largest p' at a new reference
 
 __device__ __forceinline__ i32x4 mfma_i8_16(i32x4 a, i32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
-template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(D)) void cache_fwd_kernel(CacheArgs a) {
+template <typename S, int D> __global__ __launch_bounds__(256, D == 64 ? 4 : cache_wgs_per_cu(D)) void cache_fwd_kernel(CacheArgs a) {
   constexpr int KM = D / 64;    // 64-wide k-steps of the score product
   constexpr int DB = D / 16;    // 16-row blocks of O^T
   constexpr int VB = D / 16;    // bytes of a V row per lane
@@ -61,7 +62,8 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
   constexpr int LPT = D / 8, TPP = 256 / LPT;   // quantizer: lanes per token, tokens per pass
   // LDS: query codes and constants, per-wave token constants; the merge of the four waves overlays them
   constexpr int OFF_ST = 16 * D, OFF_TC = OFF_ST + 3 * 16 * 4, MERGE = 4 * 16 * (D + 2) * 4;
-  constexpr int TOTAL = MERGE > OFF_TC + 4 * 512 ? MERGE : OFF_TC + 4 * 512;
+  constexpr int TC = 512 + 128;   // per wave: [64] x (scale, zero point operand), log2 of the 32 values' scales
+  constexpr int TOTAL = MERGE > OFF_TC + 4 * TC ? MERGE : OFF_TC + 4 * TC;
   __shared__ __attribute__((aligned(16))) unsigned char smem[TOTAL];
 
   const int per_bh = a.qblocks * a.splits;
@@ -161,12 +163,9 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
   f32x4 oacc[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) oacc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_ref = -INFINITY, m_bound = -INFINITY, nm = 0.f, l_run = 0.f, w_run = 0.f;
-  // oacc and w_run hold sums of p * scale_j * beta; p * scale_j above ps_bound would leave binary16.  (Nothing summed yet: any
-  // beta will do, and the largest leaves only p * scale_j <= 2^-105 as it is.)
-  float beta = 0x1p120f, ps_bound = CACHE_P_MAX * 0x1p-120f;
-  const float thr = SKV_RESCALE_THRESHOLD / a_i;
-  unsigned *tc = reinterpret_cast<unsigned *>(smem + OFF_TC + wave * 512);   // [64] x (scale, zero point operand)
+  // p = 2^(a_i * u - ref); a query that sees no key of the wave's first tile sees none later either
+  float ref = NO_KEY, l_run = 0.f, w_run = 0.f;
+  unsigned *tc = reinterpret_cast<unsigned *>(smem + OFF_TC + wave * TC);
   const i32x4 ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 
   auto tile = [&](const Tile &t, int i, auto masked_tag) __attribute__((always_inline)) {
@@ -180,7 +179,6 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
     }
     // ---- scores of keys 16rb + 4G + v
     f32x4 f[2];
-    float mt = -INFINITY;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       i32x4 s = {0, 0, 0, 0}, rk = {0, 0, 0, 0};
@@ -198,63 +196,73 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
         float u = (float)x * __builtin_bit_cast(float, scw);
         if (MASKED && (t0 + wave + 4 * i) * SKV_TILE + 16 * rb + 4 * G + v > lim) u = -INFINITY;
         f[rb][v] = u;
-        mt = fmaxf(mt, u);
       }
     }
-    if (__builtin_amdgcn_ballot_w64(mt > m_bound) != 0) {
-      mt = fmaxf(mt, __shfl_xor(mt, 16, 64));   // the reference maximum is common to the four lanes of a query
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-      const float m_new = fmaxf(m_ref, mt);
-      const float old = m_ref, alpha = m_new == old ? 1.0f : __builtin_amdgcn_exp2f(a_i * (old - m_new));
-      m_ref = m_new;
-      m_bound = m_new + thr;
-      nm = m_new == -INFINITY ? 0.f : -a_i * m_new;   // a query that has seen no key yet
-      l_run *= alpha;
-      // oacc and w_run stay as they are: what shrinks is p, by alpha
-      const float grow = m_new == old ? 1.0f : __builtin_amdgcn_exp2f(fminf(a_i * (m_new - old), 120.0f));
-      beta = fminf(beta * grow, 0x1p120f);
-      ps_bound = CACHE_P_MAX * __builtin_amdgcn_rcpf(beta);
-    }
-    // ---- p and its row sum; p * scale_j and the largest of them
-    float ps[8], mx = 0.f;
+    // ---- p and its row sum, p' = p * scale_j and the largest of them
+    float ps[8], mx = 0.f, l_new = 0.f;
     unsigned zz[4];   // the binary16 numbers 1152 + zero point
+    u32x4 cv[4];      // keys 16(x/2) + 4G + 2(x%2) + {0, 1}: scale, 1152 + zero point, and again
+    auto load_cv = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const unsigned *c = tc + 2 * (32 + 16 * rb + 4 * G);
+      for (int x = 0; x < 4; ++x) cv[x] = *reinterpret_cast<const u32x4 *>(tc + 2 * (32 + 16 * (x / 2) + 4 * G + 2 * (x % 2)));
+    };
+    if constexpr (D > 64) load_cv();   // (at 64 the registers of a fourth workgroup per CU are worth more)
+    auto probs = [&]() __attribute__((always_inline)) {
+      mx = 0.f;
+      l_new = l_run;
+      if constexpr (D == 64) load_cv();
 #pragma unroll
-      for (int v = 0; v < 4; v += 2) {
-        const u32x4 w = *reinterpret_cast<const u32x4 *>(c + 2 * v);
-        const unsigned s0 = w[0], z0 = w[1], s1 = w[2], z1 = w[3];   // (a bit cast of a vector's element takes element 0)
-        zz[2 * rb + v / 2] = z0 | (z1 << 16);
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[rb][v], nm));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[rb][v + 1], nm));
-        l_run += p0 + p1;
-        ps[4 * rb + v] = p0 * __builtin_bit_cast(float, s0);
-        ps[4 * rb + v + 1] = p1 * __builtin_bit_cast(float, s1);
-        mx = fmaxf(mx, fmaxf(fabsf(ps[4 * rb + v]), fabsf(ps[4 * rb + v + 1])));
+      for (int x = 0; x < 4; ++x) {
+        const unsigned s0 = cv[x][0], z0 = cv[x][1], s1 = cv[x][2], z1 = cv[x][3];   // (a bit cast of a vector's element takes element 0)
+        zz[x] = z0 | (z1 << 16);
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[x / 2][2 * (x % 2)], -ref));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(a_i, f[x / 2][2 * (x % 2) + 1], -ref));
+        l_new += p0 + p1;
+        ps[2 * x] = p0 * __builtin_bit_cast(float, s0);
+        ps[2 * x + 1] = p1 * __builtin_bit_cast(float, s1);
+        mx = fmaxf(mx, fmaxf(fabsf(ps[2 * x]), fabsf(ps[2 * x + 1])));
       }
-    }
-    if (__builtin_amdgcn_ballot_w64(mx > ps_bound) != 0) {
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));   // beta is common to the four lanes of a query
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      if (mx > ps_bound) {   // the power of two that brings mx to [1, 2)
-        const int e = (int)(__builtin_bit_cast(unsigned, mx) >> 23);
-        const float b_new = __builtin_bit_cast(float, (unsigned)min(max(254 - e, 7), 247) << 23);
-        const float gamma = b_new * __builtin_amdgcn_rcpf(beta);
-        beta = b_new;
-        ps_bound = CACHE_P_MAX * __builtin_amdgcn_rcpf(beta);
-        w_run *= gamma;
+    };
+    // a new reference, common to the four lanes of a query: log2 of the tile's largest p' (and p itself within fp32)
+    auto move = [&]() __attribute__((always_inline)) -> float {
+      float *tl = reinterpret_cast<float *>(tc + 128);
+      if (lane >= 32) tl[lane - 32] = __builtin_amdgcn_logf(fabsf((*reinterpret_cast<const f32x2 *>(tc + 2 * lane))[0]));
+      float t = -INFINITY, u = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < DB; ++j)
+      for (int rb = 0; rb < 2; ++rb) {
+        const f32x4 ls = *reinterpret_cast<const f32x4 *>(tl + 16 * rb + 4 * G);
 #pragma unroll
-          for (int v = 0; v < 4; ++v) oacc[j][v] *= gamma;
+        for (int v = 0; v < 4; ++v) {
+          t = fmaxf(t, __builtin_fmaf(a_i, f[rb][v], ls[v]));
+          u = fmaxf(u, f[rb][v]);
+        }
       }
+      t = fmaxf(t - CACHE_P_REF, __builtin_fmaf(a_i, u, -100.0f));
+      t = fmaxf(t, __shfl_xor(t, 16, 64));
+      t = fmaxf(t, __shfl_xor(t, 32, 64));
+      t = fmaxf(t, ref);
+      const float alpha = __builtin_amdgcn_exp2f(ref - t);
+      ref = t;
+      return alpha;
+    };
+    if (i == 0) move();   // (nothing summed yet)
+    probs();
+    if (i != 0 && __builtin_amdgcn_ballot_w64(mx > CACHE_P_MAX || !(l_new <= 0x1p100f)) != 0) {
+      const float alpha = move();
+      l_run *= alpha;
+      w_run *= alpha;
+#pragma unroll
+      for (int j = 0; j < DB; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) oacc[j][v] *= alpha;
+      probs();
     }
-    // ---- p' = p * scale_j * beta as binary16, offset term
+    l_run = l_new;
+    // ---- p' as binary16, offset term
     u32x4 pf;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-      const unsigned pp = pack_h2(ps[2 * x] * beta, ps[2 * x + 1] * beta);
+      const unsigned pp = pack_h2(ps[2 * x], ps[2 * x + 1]);
       pf[x] = pp;
       w_run = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pp), __builtin_bit_cast(f16x2, zz[x]), w_run, false);
     }
@@ -286,7 +294,6 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
   float l_tot = l_run + __shfl_xor(l_run, 16, 64), w_tot = w_run + __shfl_xor(w_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
   w_tot += __shfl_xor(w_tot, 32, 64);
-  const float inv_beta = __builtin_amdgcn_rcpf(beta);
   __syncthreads();   // query codes and token constants are done with
   float *mg = reinterpret_cast<float *>(smem), *ml = mg + 4 * 16 * D;
   if (q16 < nqv) {
@@ -297,11 +304,11 @@ template <typename S, int D> __global__ __launch_bounds__(256, cache_wgs_per_cu(
       for (int j = 0; j < DB; j += 4) {
         f32x4 x;
 #pragma unroll
-        for (int y = 0; y < 4; ++y) x[y] = (oacc[j + y][v] - w_tot) * inv_beta;
+        for (int y = 0; y < 4; ++y) x[y] = oacc[j + y][v] - w_tot;
         *reinterpret_cast<f32x4 *>(dst + VB * (4 * G + v) + j) = x;
       }
     if (G == 0) {
-      ml[2 * (wave * 16 + q16)] = m_ref == -INFINITY ? NO_KEY : a_i * m_ref;
+      ml[2 * (wave * 16 + q16)] = ref;
       ml[2 * (wave * 16 + q16) + 1] = l_tot;
     }
   }
