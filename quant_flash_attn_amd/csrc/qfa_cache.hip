@@ -341,16 +341,11 @@ template <typename S, int D> __global__ __launch_bounds__(256, D == 64 ? 4 : cac
   }
 }
 
-// How the keys of a query block are split: as many workgroups as are resident at once (cache_wgs_per_cu;
-// a second, partly filled round would cost a whole one), at least 8 tiles per workgroup.
+// How the keys of a query block are split: as many workgroups as are resident at once (cache_wgs_per_cu; a second, partly
+// filled round would cost a whole one), or what split_plan finds better
 static void cache_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
-  const int64_t ntiles = (Nk + SKV_TILE - 1) / SKV_TILE, wgs = BH * ((Nq + 15) / 16), slots = 256 * cache_wgs_per_cu(D);
-  int64_t want = slots / wgs;
-  if (want > ntiles / 8) want = ntiles / 8;
-  if (want < 1) want = 1;
-  const int64_t tps = (ntiles + want - 1) / want;
-  *tiles_per_split = (int)tps;
-  *splits = (int)((ntiles + tps - 1) / tps);
+  const int64_t wgs = BH * ((Nq + 15) / 16);
+  split_plan(wgs, BH * Nq, (Nk + SKV_TILE - 1) / SKV_TILE, D, 256 * cache_wgs_per_cu(D) / wgs, splits, tiles_per_split);
 }
 
 int64_t cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {

@@ -343,16 +343,12 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
 }
 
 // How the keys of one query block are split over workgroups: as many as are resident at once (three per CU; a second,
-// partly filled round costs a whole one), at head_dim 256 about four per CU (two are resident); never fewer than 8 tiles
-// per workgroup; 1 = no split.
+// partly filled round costs a whole one), at head_dim 256 about four per CU (two are resident), or what split_plan finds
+// better
 static void skv_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
-  const int64_t ntiles = (Nk + SKV_TILE - 1) / SKV_TILE, wgs = BH * ((Nq + 15) / 16);
-  int64_t want = D == 256 ? (wgs >= 512 ? 1 : (1024 + wgs - 1) / wgs) : 768 / wgs;
-  if (want > ntiles / 8) want = ntiles / 8;
-  if (want < 1) want = 1;
-  const int64_t tps = (ntiles + want - 1) / want;
-  *tiles_per_split = (int)tps;
-  *splits = (int)((ntiles + tps - 1) / tps);
+  const int64_t wgs = BH * ((Nq + 15) / 16);
+  const int64_t fill = D == 256 ? (wgs >= 512 ? 1 : (1024 + wgs - 1) / wgs) : 768 / wgs;
+  split_plan(wgs, BH * Nq, (Nk + SKV_TILE - 1) / SKV_TILE, D, fill, splits, tiles_per_split);
 }
 
 int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {

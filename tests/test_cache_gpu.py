@@ -55,7 +55,10 @@ def test_shapes(qfa, D, Nq, Nk, causal):
 # keys split over workgroups (few heads, long cache), ragged splits, and no split (many heads)
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,Nq,Nk,D", [(1, 1, 1, 8192, 128), (1, 3, 1, 5001, 64), (1, 2, 5, 3333, 256), (2, 5, 40, 2047, 128),
-                                         (9, 64, 1, 70, 128), (9, 61, 2, 300, 64)])
+                                         (9, 64, 1, 70, 128), (9, 61, 2, 300, 64),
+                                         # more splits than fill the slots once (5, 3 for none), none where 2 or 3 would
+                                         (1, 300, 1, 8192, 128), (2, 170, 1, 4099, 256), (1, 150, 16, 700, 128),
+                                         (1, 256, 16, 777, 64)])
 def test_splits(qfa, B, H, Nq, Nk, D):
     _check(qfa, B, H, Nq, Nk, D, True, torch.bfloat16, torch.float16, seed=1)
 

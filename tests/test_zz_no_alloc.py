@@ -74,3 +74,13 @@ def test_static_scratch_rejects_what_does_not_fit(qfa):
     assert rc == -2 and b"scratch" in L.qfa_last_error()
     rc = L.qfa_attn_fwd_shared_kv_static(None, p, p, 0, p, p, p, 1, B, H, Nq, Nk, D, *sq, *sc, *sq, 0.1, None)
     assert rc == -1 and b"null" in L.qfa_last_error()
+
+
+def test_every_plan_up_to_head_dim_128_fits_the_built_in_scratch(qfa):
+    import random
+    from quant_flash_attn_amd import _lib
+    L, rng = _lib.lib(), random.Random(1)
+    for _ in range(20000):
+        need = L.qfa_attn_fwd_shared_kv_workspace_bytes(1, rng.randint(1, 3000), rng.choice((1, 2, 15, 16, 17, 33, 512)),
+                                                        rng.randint(1, 40000), rng.choice((64, 128)))
+        assert 0 <= need <= (16 << 20)
