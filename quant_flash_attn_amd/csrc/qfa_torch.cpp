@@ -455,10 +455,20 @@ CacheKept cache_forward(const Tensor &q_in, const Tensor &kc, const Tensor &ks, 
   r.o = to(r.o16, q.scalar_type());
   return r;
 }
-// Longest query block for qfa_attn_fwd_cache, which walks the cache once per 16 queries (about 40 us per 16 queries at B8
-// H32 Nk8192 D128 once the MFMAs are the bound: 64 queries 203 us, where the pass over V, the row sums of K and
-// qfa_attn_fwd take 470 up to 128 queries; at B1 H8 Nk1024 it is 11 against 34 us) and leaves nothing for a backward
-constexpr int64_t CACHE_MAX_Q = 128;
+// Longest query block for qfa_attn_fwd_cache, which reads the cache once per 16 queries and leaves nothing for a backward;
+// what it saves is a pass over V, the row sums of K and the casts, so the line depends on the keys per head_dim.  Measured
+// against these passes and qfa_attn_fwd with the chip full (256 to 1024 heads), the queries at which both take as long:
+//     keys / head_dim      1     2        4        8          16
+//     head_dim 64                         100      115        130
+//     head_dim 128               78       88       100-128    130
+//     head_dim 256         49    66       95       118        135
+// (at the old line of 128: 256 heads, 256 keys of 256: 95 against 51 us).  While one round of workgroups covers the call it
+// wins up to 128 queries at any of these sizes (64 heads, 1024 keys of 256, 128 queries: 44 against 59 us; 32 heads: 25
+// against 57).
+int64_t cache_max_q(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
+  if (BH * ((Nq + 15) / 16) <= 512 || Nk >= 16 * D) return 128;
+  return Nk >= 8 * D ? 112 : Nk >= 4 * D ? 80 : Nk >= 2 * D ? 64 : 48;
+}
 Tensor cache_short(const Tensor &q_in, const Tensor &kc_in, const Tensor &ks_in, const Tensor &kz, const Tensor &vc_in,
                    const Tensor &vs_in, const Tensor &vz, bool causal, double sm) {
   const c10::DeviceGuard guard(q_in.device());
@@ -519,7 +529,7 @@ Tensor cache_op(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, con
                         q.size(0) == kc.size(0) && q.size(1) == kc.size(1),
                     "shape mismatch: q ", q.sizes(), ", k codes ", kc.sizes(), ", v codes ", vc.sizes());
   if (wants_grad({&q, &k_fp16, &v_fp16})) return CacheFn::apply(q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz, causal, sm);
-  if (q.size(2) <= CACHE_MAX_Q) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
+  if (q.size(2) <= cache_max_q(q.size(0) * q.size(1), q.size(2), kc.size(2), q.size(3))) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
   return cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm).o;
 }
 Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc, const Tensor &ks,

@@ -72,6 +72,15 @@ def test_types_and_layouts(qfa, dtype, sdtype, layout):
         _check(qfa, 2, 3, 5, 700, D, True, dtype, sdtype, dist="uniform", seed=2, layout=layout)
 
 
+# either side of the lines between this kernel and the long-query path (keys / head_dim, and one round of workgroups)
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,H,Nk,edges", [(64, 200, 120, (48, 49)), (64, 200, 128, (64, 65)), (128, 160, 512, (80, 81)),
+                                          (64, 120, 512, (112, 113)), (128, 2, 300, (128, 129))])
+def test_longest_query_block(qfa, D, H, Nk, edges):
+    for Nq in edges:
+        _check(qfa, 1, H, Nq, Nk, D, True, torch.float16, torch.float16, dist="normal", seed=Nq)
+
+
 @pytest.mark.gpu
 def test_growing_scores_and_one_sided_rows(qfa):
     """Scores that grow along the keys move the running maximum in every tile; all-positive rows pin the zero points."""
