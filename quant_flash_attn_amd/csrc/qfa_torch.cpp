@@ -469,6 +469,9 @@ int64_t cache_max_q(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
   if (BH * ((Nq + 15) / 16) <= 512 || Nk >= 16 * D) return 128;
   return Nk >= 8 * D ? 112 : Nk >= 4 * D ? 80 : Nk >= 2 * D ? 64 : 48;
 }
+bool cache_takes_short(const Tensor &q, const Tensor &kc) {
+  return q.size(2) <= cache_max_q(q.size(0) * q.size(1), q.size(2), kc.size(2), q.size(3));
+}
 Tensor cache_short(const Tensor &q_in, const Tensor &kc_in, const Tensor &ks_in, const Tensor &kz, const Tensor &vc_in,
                    const Tensor &vs_in, const Tensor &vz, bool causal, double sm) {
   const c10::DeviceGuard guard(q_in.device());
@@ -499,6 +502,9 @@ struct CacheFn : torch::autograd::Function<CacheFn> {
                         double sm) {
     const at::AutoDispatchBelowADInplaceOrView below;
     CacheKept r = cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm);
+    // what a call without a gradient returns, bit for bit (a forward that is computed again for its gradient, as activation
+    // checkpointing does); the backward takes O, LSE and V of the path above
+    if (cache_takes_short(q, kc)) r.o = cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
     ctx->save_for_backward({r.buf, r.v16, r.o16, r.kc, r.ks, r.kz, r.kr});
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["sm"] = sm;
@@ -529,7 +535,7 @@ Tensor cache_op(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, con
                         q.size(0) == kc.size(0) && q.size(1) == kc.size(1),
                     "shape mismatch: q ", q.sizes(), ", k codes ", kc.sizes(), ", v codes ", vc.sizes());
   if (wants_grad({&q, &k_fp16, &v_fp16})) return CacheFn::apply(q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz, causal, sm);
-  if (q.size(2) <= cache_max_q(q.size(0) * q.size(1), q.size(2), kc.size(2), q.size(3))) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
+  if (cache_takes_short(q, kc)) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
   return cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm).o;
 }
 Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc, const Tensor &ks,

@@ -82,6 +82,21 @@ def test_longest_query_block(qfa, D, H, Nk, edges):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Nq", [1, 64, 200])
+def test_with_and_without_a_gradient(qfa, Nq, dtype):
+    q, k, v, _ = (t.to(DEV) for t in make_inputs("offset", 1, 2, 512, 128, seed=Nq, dtype=dtype))
+    q = q[:, :, :Nq].contiguous()
+    kq, vq = qfa.asymmetric_quant_per_token(k), qfa.asymmetric_quant_per_token(v)
+    with torch.no_grad():
+        first = qfa.quant_flash_attn_quantized_kv(q, k, v, kq, vq, True, 0.1)
+    again = qfa.quant_flash_attn_quantized_kv(q.requires_grad_(True), k.requires_grad_(True), v, kq, vq, True, 0.1)
+    assert torch.equal(again.detach(), first)
+    again.sum().backward()
+    assert torch.isfinite(q.grad).all() and torch.isfinite(k.grad).all()
+
+
+@pytest.mark.gpu
 def test_growing_scores_and_one_sided_rows(qfa):
     """Scores that grow along the keys move the running maximum in every tile; all-positive rows pin the zero points."""
     for D in (64, 128, 256):
