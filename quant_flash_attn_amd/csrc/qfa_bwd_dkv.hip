@@ -179,9 +179,9 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     const int rowb = buf + row_l + mbk * 1024;
     const int cb = cq_a(buf, mbk);
     const int i0 = TILE * t + 32 * mbk + 4 * g;
-    // dO^T is zero for the key blocks that none of the step's queries sees (the first tile of a wave may hold such steps): P
-    // is zero there, and dO may be infinite
-    constexpr bool UNSEEN = MASKED && CAUSAL && (NSTEP > 1 || KB > 1);
+    // dO^T is zero for the key blocks that none of the step's queries sees (a wave's first step may hold such blocks): P is
+    // zero there, and dO may be infinite
+    constexpr bool UNSEEN = MASKED && CAUSAL && KB > 1;
     unsigned dv_mask[KB];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) dv_mask[kb] = TILE * t + 32 * mbk + 31 >= k_first + 32 * kb - coff ? ~0u : 0u;
@@ -289,11 +289,9 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     constexpr int DSW = 8 * KB;   // dwords of dS
     auto ds_dword = [&](auto k_tag) __attribute__((always_inline)) {
       constexpr int k = decltype(k_tag)::value, kb = k / 8, hh = k / 4 % 2, e = k % 4, v = 8 * hh + 2 * e;
-      float x0 = f[kb][v] * dp[kb][v], x1 = f[kb][v + 1] * dp[kb][v + 1];
-      if constexpr (MASKED) {   // a masked pair has P = 0, but its dP may be anything: dO may be infinite there
-        x0 = f[kb][v] == 0.f ? 0.f : x0;
-        x1 = f[kb][v + 1] == 0.f ? 0.f : x1;
-      }
+      // (a masked pair has P = 0, but its dP may be anything: dO may be infinite there)
+      const float x0 = MASKED ? mul_zero_wins(f[kb][v], dp[kb][v]) : f[kb][v] * dp[kb][v];
+      const float x1 = MASKED ? mul_zero_wins(f[kb][v + 1], dp[kb][v + 1]) : f[kb][v + 1] * dp[kb][v + 1];
       ds[kb][hh][e] = pack2<T>(x0, x1);
     };
     // S comes before the last dV fragment, whose MFMAs cover the time its results take
@@ -311,8 +309,8 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
       u32x4 g4 = {w[0][0], w[0][1], w[1][0], w[1][1]};
       static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
         constexpr int kb = decltype(kb_tag)::value, m = KB * n + kb;
-        if constexpr (UNSEEN) {   // (a later key block is seen by fewer queries)
-          g4 &= dv_mask[kb];
+        if constexpr (UNSEEN && kb == 0 && mbk == 0) {   // (a tile's second step sees it)
+          g4 &= dv_mask[0];
           QFA_FENCE();
           asm volatile("s_nop 1");
         }
@@ -321,6 +319,11 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
         QFA_FENCE();
         acc_mfma<T, DV0 + kb * DB + n % DB, ACC>(g4, pf[kb][n / DB]);
         QFA_FENCE();
+        if constexpr (UNSEEN && kb == 0) {   // (fewer queries see the second block)
+          g4 &= dv_mask[KB - 1];
+          QFA_FENCE();
+          if constexpr (m >= S1) asm volatile("s_nop 1");
+        }
         if constexpr (m < S1) {
           if constexpr (m < 2) work(ic<SLOTS + m>{});
           if constexpr (m == 1) pack_pair(ic<8 * KB - 1>{});
@@ -353,8 +356,10 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     QFA_FENCE();
   };
 
-  // ---- first tile this wave sees (its first step may lie before the first visible one: all masked, adds nothing)
+  // ---- first tile this wave sees; with one key block per wave it begins with the first step that the wave sees, so that
+  // every block of a step is seen by some query (with two the second block's masks do that)
   int ft = it0;
+  const bool late = CAUSAL && KB == 1 && NSTEP == 2 && max(k_first - coff, 0) / 32 % 2 == 1;
   if (CAUSAL) ft = max(ft, max(k_first - coff, 0) / TILE);
   if (k_first >= a.Nk) ft = ntiles;
   dma_wait();
@@ -371,17 +376,21 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     for (int kb = 0; kb < KB; ++kb) {
       i32x16 si = bias;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) si = mfma_i8(__builtin_bit_cast(i32x4, ld(buf + row_l + SM::OFF_Q + ks * SLAB)), kf[kb][ks], si);
+      for (int ks = 0; ks < KS; ++ks)
+        si = mfma_i8(__builtin_bit_cast(i32x4, ld(buf + row_l + (late ? 1024 : 0) + SM::OFF_Q + ks * SLAB)), kf[kb][ks], si);
       f[kb] = __builtin_bit_cast(f32x16, si);
     }
     int qt_prev = buf + SM::OFF_QT + row_l;     // (dS is zero: the product adds nothing)
-    request_head(buf, 0, qt_prev);
+    request_head(buf, late ? 1 : 0, qt_prev);
     const int k_last = k_first + KEYS - 1;
     // masked tiles (diagonal), full ones, masked ones (ragged end)
     auto tiles = [&](int t_end, auto masked_tag) __attribute__((always_inline)) {
       for (; t < t_end; ++t) {
         static_for<NSTEP>([&](auto mbk_tag) __attribute__((always_inline)) {
           constexpr int mbk = decltype(mbk_tag)::value;
+          if constexpr (decltype(masked_tag)::value && CAUSAL && KB == 1 && NSTEP == 2 && mbk == 0) {
+            if (late && t == ft) return;
+          }
           body(t, buf, mbk == NSTEP - 1 ? nbuf : buf, qt_prev, mbk_tag, masked_tag);
           qt_prev = buf + SM::OFF_QT + row_l + mbk * (2 * DB * 1024);
         });

@@ -52,6 +52,16 @@ template <typename T> __device__ __forceinline__ float hi_to_f32(unsigned w) {
   return (float)q[1];
 }
 
+// a * b, but 0 where a or b is 0, whatever the other is (v_mul_legacy_f32; clang has no builtin for the intrinsic)
+extern "C" __device__ __attribute__((const)) float qfa_mul_legacy(float, float) __asm("llvm.amdgcn.fmul.legacy");
+__device__ __forceinline__ float mul_zero_wins(float a, float b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return qfa_mul_legacy(a, b);
+#else
+  return a == 0.f || b == 0.f ? 0.f : a * b;
+#endif
+}
+
 // c + lo(w) + hi(w) for a packed pair of 16-bit floats (v_dot2 with a pair of ones), fp32 accumulate
 template <typename T> __device__ __forceinline__ float dot2_ones(unsigned w, float c);
 template <> __device__ __forceinline__ float dot2_ones<__bf16>(unsigned w, float c) {
