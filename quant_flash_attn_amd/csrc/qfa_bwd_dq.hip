@@ -364,12 +364,16 @@ template <typename T, int D, int QB> static int launch_dq_qb(BwdArgs a, int64_t 
 }
 
 // Cost of a launch of workgroups of 128 * qb queries on 256 CUs, one per CU, in steps of 32 keys: whole rounds when all are
-// equally long; causal, the mean load and half of the longest.  `step`: cost of a step; starting and finishing a workgroup
-// costs about two.
+// equally long; causal, the mean load and half of the longest, or the longest where all run at once (a tenth more, since the
+// mean of shorter ones fills in better than that).  `step`: cost of a step; starting and finishing a workgroup costs about
+// two.  Both kernels' variants timed for 16 to 1024 heads of 64 to 2048 tokens: the choice is within 5 % of the best but
+// for 128 heads of 768 (6 %); 256 heads of 200 and 256 causal tokens, the whole backward: 70 -> 66 and 74 -> 69 us with one
+// round of 256-row workgroups.
 static float dq_cost(const BwdArgs &a, int64_t BH, bool causal, int qb, float step) {
   const int64_t nb = (a.Nq + 128 * qb - 1) / (128 * qb);
   const float steps = (float)((a.Nk + 31) / 32) * step, fix = 2.0f;
   if (!causal) return (float)((nb * BH + 255) / 256) * (steps + fix);
+  if (nb * BH <= 256) return 1.1f * (steps + fix);
   const float f = (float)a.Nq / (float)a.Nk;   // a head's triangle (trapezoid: few queries) of steps
   const float sum = (float)(nb * BH) * (steps * (1.0f - 0.5f * f) + 2.0f * (float)qb * step + fix);
   return sum / 256.0f + 0.5f * steps;

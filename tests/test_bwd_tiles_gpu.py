@@ -31,7 +31,8 @@ def test_backward_at_tile_edges(qfa, Nq, Nk, causal, D, dtype):
 @pytest.mark.parametrize("Nq,Nk,causal", [(63, 129, False),     # dK / dV
                                           (128, 256, True),     # dK / dV
                                           (161, 513, True), (511, 515, True),   # dQ
-                                          (193, 300, False), (257, 257, False), (512, 512, False), (449, 449, True),
+                                          (193, 300, False), (257, 257, False), (512, 512, False), (200, 200, True),
+                                          (256, 256, True), (449, 449, True),
                                           (512, 512, True), (420, 512, True)])
 def test_64_rows_per_wave(qfa, Nq, Nk, causal, dtype, layout):
     B, H, D = 2, 128, 128
