@@ -73,7 +73,27 @@ template <int E> struct QuantRow {
   float scale, zp;
   int sum;
 };
-// SHORT: the elements have at most 11 significant bits (16-bit tensors).
+// Division by the per-token scale.  In the common exponent range the quotient is formed with the same FMA refinement the
+// hardware division sequence uses (reciprocal refined once, two residual corrections of the quotient), which gives the
+// correctly rounded x/scale without the per-element operand scaling.  Quotients below 2^-30 in magnitude may differ in their
+// last bits, which cannot matter: they vanish in the addition of the zero point or round to zero.  SHORT: elements of at most
+// 11 significant bits (16-bit tensors) need one correction only: no pair of such a significand with a scale's 24-bit one
+// gives another quotient than `/` (tests/test_quant_division_gpu.py compares all 2^33; the steps do not depend on the
+// exponents).
+__device__ __forceinline__ float quant_reciprocal(float scale) {
+#pragma clang fp contract(off)
+  const float r = __builtin_amdgcn_rcpf(scale);
+  return __builtin_fmaf(__builtin_fmaf(-scale, r, 1.0f), r, r);
+}
+template <bool SHORT> __device__ __forceinline__ float quant_quotient(float x, float scale, float r) {
+#pragma clang fp contract(off)
+  float q = x * r;
+  q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
+  if (!SHORT) q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
+  return q;
+}
+
+// SHORT: as above.
 template <int LPT, bool SHORT, int E> __device__ __forceinline__ QuantRow<E> quant_row(const float (&v)[E], bool used) {
 #pragma clang fp contract(off)
   float mn = v[0], mx = v[0];
@@ -82,23 +102,10 @@ template <int LPT, bool SHORT, int E> __device__ __forceinline__ QuantRow<E> qua
   group_min_max<LPT>(mn, mx);
   float scale = (mx - mn) / 255.0f;
   scale = (scale == 0.0f) ? 1.0f : scale;
-  // Division by the per-token scale.  In the common exponent range the quotient is formed with the
-  // same FMA refinement the hardware division sequence uses (reciprocal refined once, two residual
-  // corrections of the quotient), which gives the correctly rounded x/scale without the per-element
-  // operand scaling; outside that range (tiny scale, huge values, NaN) the IEEE `/` is used.
-  // Quotients below 2^-30 in magnitude may differ in their last bits, which cannot matter: they
-  // vanish in the addition of the zero point or round to zero.  Elements of at most 11 significant bits need one
-  // correction only: all 2^33 pairs of such a significand with a scale's were compared with `/` on the GPU, none differs
-  // (neither step depends on the exponents).
+  // the shared reciprocal's range: a tiny scale, huge values and NaN take the IEEE `/`
   const bool fast = (scale >= 0x1p-60f) && (fmaxf(fabsf(mn), fabsf(mx)) <= 0x1p60f);
-  float r = __builtin_amdgcn_rcpf(scale);
-  r = __builtin_fmaf(__builtin_fmaf(-scale, r, 1.0f), r, r);
-  auto fdiv = [&](float x) -> float {
-    float q = x * r;
-    q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
-    if (!SHORT) q = __builtin_fmaf(__builtin_fmaf(-scale, q, x), r, q);
-    return q;
-  };
+  const float r = quant_reciprocal(scale);
+  auto fdiv = [&](float x) -> float { return quant_quotient<SHORT>(x, scale, r); };
   // roundf (ties away from zero) in three instructions: add the largest float below one half with the
   // sign of y, truncate.  Equal to roundf for every binary32 value (checked exhaustively on the CPU; the
   // classic y + 0.5 fails at 0.49999997).
