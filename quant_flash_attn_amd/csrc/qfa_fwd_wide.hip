@@ -412,8 +412,13 @@ template <typename T, int D, int QB> static int launch_wide(FwdArgs a, int64_t B
   a.total_blocks = (int)total;
   a.blocks_per_xcd = (a.total_blocks + 7) / 8;
   const dim3 grid((unsigned)(a.blocks_per_xcd * 8));
-  if (causal) fwd_wide_kernel<T, D, QB, true><<<grid, dim3(256), 0, st>>>(a);
-  else fwd_wide_kernel<T, D, QB, false><<<grid, dim3(256), 0, st>>>(a);
+  if constexpr (D == 256) {
+    if (causal) fwd_wide_kernel<T, D, QB, true><<<grid, dim3(256), 0, st>>>(a);
+    else fwd_wide_kernel<T, D, QB, false><<<grid, dim3(256), 0, st>>>(a);
+  } else {
+    if (causal) return set_error(QFA_EUNSUPPORTED, "attn_fwd: no wide kernel for a mask at this head_dim");
+    fwd_wide_kernel<T, D, QB, false><<<grid, dim3(256), 0, st>>>(a);
+  }
   return check_launch("qfa_attn_fwd");
 }
 

@@ -371,12 +371,12 @@ struct Kept {
   Tensor buf, v16, o16, o;
 };
 // backward from them
-Grads bwd_from(AutogradContext *ctx, const variable_list &saved, const Tensor &grad, const Quantized *k_given = nullptr) {
+Grads bwd_from(AutogradContext *ctx, const variable_list &saved, const Tensor &grad) {
   const Tensor &buf = saved[0], &v16 = saved[1], &o16 = saved[2];
   const int64_t Nk = v16.size(2);
   const PairBuffer pb(o16.size(0), o16.size(1), o16.size(2), Nk, o16.size(3));
   const c10::DeviceGuard guard(v16.device());
-  return bwd_of(pb.view(buf, 0), k_given ? *k_given : pb.view(buf, 1), v16, o16, grad, pb.lse_of(buf),
+  return bwd_of(pb.view(buf, 0), pb.view(buf, 1), v16, o16, grad, pb.lse_of(buf),
                 ctx->saved_data["causal"].toBool(), ctx->saved_data["sm"].toDouble());
 }
 
