@@ -6,11 +6,12 @@
 // Bound by reading the cache once (2 D + 6 bytes per key).  Through the kernels for long query blocks the same call
 // dequantizes V to 16 bits first (2 D more bytes written and read), sums K's codes in a pass of its own and then walks
 // each (batch, head) with one workgroup of 128 query rows, nearly all of them padding: B8 H32 Nq1 Nk8192 D128 took 459 us
-// that way (dequantize 175, row sums 100, attention 200 with the casts); this kernel and its merge take 99 us (5.5 TB/s of cache; 35 -> 17.5 for B1).
+// that way (dequantize 175, row sums 100, attention 200 with the casts); this kernel and its merge take 96 us (5.7 TB/s of
+// cache; 35 -> 17.5 for B1).
 //
-// Work split.  A workgroup = 4 waves = 16 queries of one (batch, head) and a share of its keys (split over as many
-// workgroups as fill the chip once); its 32-key tiles are dealt to the waves, each with its own online softmax.  The tile
-// lives in registers, double-buffered: nothing of it is used twice inside a workgroup, so LDS would only add a trip.
+// Work split.  A workgroup = 4 waves = 16 queries of one (batch, head) and a share of its keys (split_plan, qfa_merge.h);
+// its 32-key tiles are dealt to the waves, each with its own online softmax.  The tile lives in registers, double-buffered:
+// nothing of it is used twice inside a workgroup, so LDS would only add a trip.
 //   K    is the A operand of v_mfma_i32_16x16x64_i8 as it lies in memory (lane = key row, 16 bytes of it per k-group); a
 //        second product with a column of ones gives the row sums the zero-point term needs.
 //   V^T  is the A operand of the P.V product (rows = d, contracted over keys).  A lane loads the D/16 bytes at
@@ -19,9 +20,9 @@
 //        (qfa_skv_common.h); MFMA i of the D/16 takes byte i, so its row r is d = (D/16) * r + i.
 //   The offset 1152 + zero point is removed through sum_j (1152 + zp_j) p'_j, accumulated over the rounded p' = p * scale_j.
 //   p' enters the product as binary16, and the scales carry V's magnitude: the reference that p is taken against follows the
-//   largest p', not the largest p, so that p' stays at 2^15 or below with the largest one seen at 2^7 or above, whatever V's
-//   size.  (p <= 1 put p' among binary16's subnormals for small V: relative error of O 1.8e-2 at size 1e-3, 1.7e-1 at 1e-4,
-//   where dequantizing V first leaves 3e-3 in bf16; and scales above 4e3 overflowed.)
+//   largest p', not the largest p, so that the largest one seen lies between 2^7 and 2^10, whatever V's size.  (p <= 1 put p'
+//   among binary16's subnormals for small V: relative error of O 1.8e-2 at size 1e-3, 1.7e-1 at 1e-4, where dequantizing V
+//   first leaves 3e-3 in bf16; and scales above 4e3 overflowed.)
 // Per-token scales and zero points pass through 512 bytes of LDS per wave, which turns one load per token into the
 // broadcast the accumulator layout wants.
 #include <type_traits>
@@ -47,8 +48,12 @@ struct CacheArgs {
 // accumulators.  With one tile per wave in flight that keeps 64 KB (48 at head_dim 64) per CU under way.
 constexpr int cache_wgs_per_cu(int D) { return D == 256 ? 1 : D == 128 ? 2 : 3; }
 
-constexpr float CACHE_P_MAX = 0x1p15f;   // largest p' (binary16 ends at 65504)
-constexpr float CACHE_P_REF = 7.0f;      // log2 of the largest p' at a new reference
+// log2 of the largest p' at a new reference, and the p' past which the reference moves.  The key at the reference has an exact
+// p' (see `move`), so moving it sooner is more exact: against a reference that moves where p passes 2^4, as in the other
+// kernels, the error of fp32 results is 0.85 to 1.0 times as large over head_dim 64, 128 and 256 and all value
+// distributions (1.0e-4 to 2.1e-4); moved at 2^15 it is up to 1.38 times as large, moved at 2^9 0.73 to 1.0, for 1 to 3 %
+// more time at head_dim 64.
+constexpr float CACHE_P_REF = 7.0f, CACHE_P_MAX = 0x1p10f;
 
 __device__ __forceinline__ i32x4 mfma_i8_16(i32x4 a, i32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
@@ -62,7 +67,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, D == 64 ? 4 : cac
   constexpr int LPT = D / 8, TPP = 256 / LPT;   // quantizer: lanes per token, tokens per pass
   // LDS: query codes and constants, per-wave token constants; the merge of the four waves overlays them
   constexpr int OFF_ST = 16 * D, OFF_TC = OFF_ST + 3 * 16 * 4, MERGE = 4 * 16 * (D + 2) * 4;
-  constexpr int TC = 512 + 128;   // per wave: [64] x (scale, zero point operand), log2 of the 32 values' scales
+  constexpr int TC = 512 + 128;   // per wave: [64] x (scale, zero point operand), exponents of the 32 values' scales
   constexpr int TOTAL = MERGE > OFF_TC + 4 * TC ? MERGE : OFF_TC + 4 * TC;
   __shared__ __attribute__((aligned(16))) unsigned char smem[TOTAL];
 
@@ -223,10 +228,11 @@ template <typename S, int D> __global__ __launch_bounds__(256, D == 64 ? 4 : cac
         mx = fmaxf(mx, fmaxf(fabsf(ps[2 * x]), fabsf(ps[2 * x + 1])));
       }
     };
-    // a new reference, common to the four lanes of a query: log2 of the tile's largest p' (and p itself within fp32)
+    // a new reference, common to the four lanes of a query: log2 of the tile's largest p' (and p itself within fp32), but for the
+    // scale's mantissa: that key's p is a power of two, and its p' the scale itself, which a binary16 scale is exactly
     auto move = [&]() __attribute__((always_inline)) -> float {
       float *tl = reinterpret_cast<float *>(tc + 128);
-      if (lane >= 32) tl[lane - 32] = __builtin_amdgcn_logf(fabsf((*reinterpret_cast<const f32x2 *>(tc + 2 * lane))[0]));
+      if (lane >= 32) tl[lane - 32] = __builtin_floorf(__builtin_amdgcn_logf(fabsf((*reinterpret_cast<const f32x2 *>(tc + 2 * lane))[0])));
       float t = -INFINITY, u = -INFINITY;
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {

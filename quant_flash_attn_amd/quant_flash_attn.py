@@ -100,11 +100,12 @@ class QuantFlashAttnQuantizedKV:
     scale and zero point, a 16-bit placeholder leaf receives the gradient) with K and V as two separately quantized
     tensors instead of one shared tensor, and a causal flag.  k_quant and v_quant are (codes, scale, zero_point)
     tuples as asymmetric_quant_per_token returns them; k_fp16 and v_fp16 are only placeholders.
-    Short query blocks without a gradient (decoding) run in one pass over the cache (qfa_attn_fwd_cache).  Otherwise the K
-    codes are used as they are (INT8 scores) and V is dequantized once per call by the HIP dequantizer into a
-    16-bit tensor that the P.V product streams: converting int8 V inside the attention kernel would add about 110
-    vector instructions per 32x32 block to a loop that is bound by its vector instructions, the separate pass adds
-    a read of the codes and one 16-bit write and read (8 % of the forward at B4 H32 N4096 D128)."""
+    Short query blocks (decoding) run in one pass over the cache (qfa_attn_fwd_cache), with V as its exact codes.  In longer
+    ones the K codes are used as they are (INT8 scores) and V is dequantized once per call by the HIP dequantizer into a
+    16-bit tensor that the P.V product streams: converting int8 V inside that kernel would add about 56 vector
+    instructions per 32x32 block to a loop that issues 83 and is bound by them, the separate pass adds
+    a read of the codes and one 16-bit write and read (8 % of the forward at B4 H32 N4096 D128).  With and without a
+    gradient the result is the same, bit for bit."""
 
     @staticmethod
     def apply(q, k_fp16, v_fp16, k_quant, v_quant, causal, sm_scale):
