@@ -1,7 +1,7 @@
 // Host path of the Python entry points: argument checks, output allocation, autograd and the calls into libqfa.so, as
 // one CPython module (_qfa_host).  A call costs a few microseconds here against 60 to 250 when the same steps run as
 // Python (a dozen torch.empty, three torch.autograd.Function round trips through the interpreter, ctypes calls of up to
-// 45 arguments): at B1 H4 N256 D64 the kernels of a training step take about 60 us, so the host was the bound.
+// 45 arguments): at B1 H4 N256 D64 the kernels of a training step take about 50 us, so the host was the bound.
 //
 // The module does not link against libqfa.so: the binding that loads the library hands over the addresses of its entry
 // points (init), so there is one place that decides which library file is used, and none of this works without it.
