@@ -10,7 +10,7 @@ if ROOT not in sys.path:
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
 def pytest_collection_modifyitems(config, items):
@@ -34,7 +34,7 @@ def _oracle_lib():
 
 @pytest.fixture(scope="session")
 def qfa():
-    """The product package; on a GPU box a missing libqfa.so is an error, never a skip."""
+    """The product package; where a GPU is present a missing libqfa.so is an error, never a skip."""
     import quant_flash_attn_amd
     from quant_flash_attn_amd import _lib
     _lib.lib()
