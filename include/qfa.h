@@ -209,6 +209,22 @@ int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale
                            int64_t sdkh, int64_t sdkn, float sm_scale, void *stream);
 
 /*
+ * The same with a caller-owned scratch (16-byte aligned, qfa_attn_bwd_shared_kv_workspace_bytes(...) bytes; the function
+ * returns 0 when no split pays; NULL: never split).  With few (batch, head) pairs the keys are split over several workgroups,
+ * each with its own part of dKV; their partial dQ meet in the scratch and a small kernel adds them in a fixed order.
+ */
+int64_t qfa_attn_bwd_shared_kv_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
+
+int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
+                                 const void *o, const void *dout, const float *lse, void *dq, void *dkv, int io_dtype,
+                                 int grad_dtype, const float *grad_scale,
+                                 int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                                 int64_t scb, int64_t sch, int64_t scn, int64_t sob, int64_t soh, int64_t son, int64_t sdob,
+                                 int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
+                                 int64_t sdkh, int64_t sdkn, float sm_scale, void *workspace, int64_t workspace_bytes,
+                                 void *stream);
+
+/*
  * Attention forward of a SHORT query block on an INT8 cache of keys and values (decoding, a few queries at a time):
  *     O = softmax(sm_scale * Q^ K^^T) V^,   Q^, K^, V^ = scale * (codes - zero_point) per token
  * Q is quantized inside by the arithmetic of qfa_quant_per_token, the scores are those of qfa_attn_fwd on these codes,

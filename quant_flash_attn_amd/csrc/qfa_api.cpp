@@ -238,6 +238,24 @@ int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale
                            int64_t scb, int64_t sch, int64_t scn, int64_t sob, int64_t soh, int64_t son, int64_t sdob,
                            int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
                            int64_t sdkh, int64_t sdkn, float sm_scale, void *stream) {
+  return qfa_attn_bwd_shared_kv_split(q, codes, scale, scale_dtype, zp, o, dout, lse, dq, dkv, io_dtype, grad_dtype, grad_scale, B,
+                                      H, Nq, Nk, D, sqb, sqh, sqn, scb, sch, scn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh,
+                                      sdqn, sdkb, sdkh, sdkn, sm_scale, nullptr, 0, stream);
+}
+
+int64_t qfa_attn_bwd_shared_kv_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0 || (D != 64 && D != 128 && D != 256)) return 0;
+  return skv_bwd_workspace_bytes(B, H, Nq, Nk, D);
+}
+
+int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
+                           const void *o, const void *dout, const float *lse, void *dq, void *dkv, int io_dtype,
+                           int grad_dtype, const float *grad_scale,
+                           int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                           int64_t scb, int64_t sch, int64_t scn, int64_t sob, int64_t soh, int64_t son, int64_t sdob,
+                           int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
+                           int64_t sdkh, int64_t sdkn, float sm_scale, void *workspace, int64_t workspace_bytes,
+                                 void *stream) {
   const char *who = "attn_bwd_shared_kv";
   SkvAttnArgs a;
   memset(&a, 0, sizeof(a));
@@ -260,10 +278,14 @@ int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale
   // the row copies of the two-kernel path form offsets inside a 32-row block in 31 bits
   if (sqn >= (1 << 23) || son >= (1 << 23) || sdon >= (1 << 23))
     return set_error(QFA_EUNSUPPORTED, "%s: token strides of 2^23 elements or more are not supported", who);
-  // one fused pass keeps a (batch, head)'s dQ in registers: at most 32 queries, head_dim up to 128
-  // one fused pass while the per-wave accumulators fit: 32 queries up to head_dim 128, 16 at 256
-  const bool one_pass = (Nq <= 32 && D <= 128) || (Nq <= 16 && D == 256);
-  return one_pass ? launch_skv_bwd(a, (hipStream_t)stream) : launch_skv_bwd_long(a, (hipStream_t)stream);
+  if (workspace) {
+    const int64_t need = skv_bwd_workspace_bytes(B, H, Nq, Nk, D);
+    if (!aligned16(workspace) || workspace_bytes < need)
+      return set_error(QFA_EINVAL, "%s: workspace must be 16-byte aligned and hold %lld bytes "
+                       "(qfa_attn_bwd_shared_kv_workspace_bytes), got %lld", who, (long long)need, (long long)workspace_bytes);
+    a.workspace = need > 0 ? workspace : nullptr;
+  }
+  return skv_bwd_one_pass(Nq, D) ? launch_skv_bwd(a, (hipStream_t)stream) : launch_skv_bwd_long(a, (hipStream_t)stream);
 }
 
 int64_t qfa_attn_fwd_cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {

@@ -72,9 +72,9 @@ template <typename S, int D> __global__ __launch_bounds__(256, D == 64 ? 4 : cac
   __shared__ __attribute__((aligned(16))) unsigned char smem[TOTAL];
 
   const int per_bh = a.qblocks * a.splits;
-  const int bh = (int)(blockIdx.x / (8 * per_bh)) * 8 + (int)(blockIdx.x % 8);   // blocks of one (batch, head): one XCD
-  const int qb = (int)(blockIdx.x / 8) % per_bh % a.qblocks, split = (int)(blockIdx.x / 8) % per_bh / a.qblocks;
-  if (bh >= a.BH) return;
+  const XcdBlock id(a.BH, per_bh);
+  if (!id.live) return;
+  const int bh = id.bh, qb = id.sub % a.qblocks, split = id.sub / a.qblocks;
   const int64_t b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x, lane = tid % 64, q16 = lane % 16, G = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -377,7 +377,7 @@ template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, 
     a.po = static_cast<float *>(x.workspace);
     a.pml = a.po + x.B * x.H * x.Nq * a.splits * (int64_t)D;
   }
-  const int64_t total = (int64_t)a.qblocks * a.splits * ((a.BH + 7) / 8) * 8;   // ids past batch*heads exit at once
+  const int64_t total = xcd_grid(a.BH, (int64_t)a.qblocks * a.splits);
   if (x.B * x.H > 0x7fffffffLL || total > 0x7fffffffLL || x.B * x.H * x.Nq > 0x7fffffffLL)
     return set_error(QFA_EUNSUPPORTED, "attn_fwd_cache: too many query blocks for one launch");
   cache_fwd_kernel<S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);

@@ -48,12 +48,18 @@ int launch_bwd(const AttnArgs &a, hipStream_t st);
 int launch_sum16(const void *a, const void *b, void *out, int dtype, int64_t n, hipStream_t st);   // out = a + b, n % 8 == 0
 int64_t bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
 
+// grid of a kernel that maps ids with XcdBlock (qfa_skv_common.h): per_bh workgroups for each of BH heads
+__host__ __device__ inline bool xcd_whole_heads(int64_t BH) { return BH >= 64 || BH % 8 == 0; }
+inline int64_t xcd_grid(int64_t BH, int64_t per_bh) {
+  return xcd_whole_heads(BH) ? (BH + 7) / 8 * 8 * per_bh : (BH * per_bh + 7) / 8 * 8;
+}
+
 // Shared-KV attention (K = V = one quantized tensor, Q in 16-bit float), after validation.
 struct SkvAttnArgs {
   const void *q; const int8_t *codes; const void *scale; const int8_t *zp;
   void *o; float *lse;
   const void *dout; void *dq; void *dkv;   // backward only
-  void *workspace;                         // forward only, nullable: partial results when the keys are split
+  void *workspace;                         // nullable: partial results when the keys are split
   int64_t B, H, Nq, Nk;
   int64_t sqb, sqh, sqn, scb, sch, scn, sob, soh, son;
   int64_t sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn;
@@ -71,6 +77,22 @@ int launch_skv_bwd(const SkvAttnArgs &a, hipStream_t st);        // io_dtype QFA
 int64_t dout_normalise_workspace_bytes();
 int launch_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *scale, int scale_dtype, int64_t ns,
                           float *partials, void *out, float *back, hipStream_t st);
+// Query blocks of more than 16: forward and dQ on tiles of 64 keys that a workgroup expands once.  qw: waves side by side on
+// the queries (0: not this kernel), splits: workgroups that share the keys, tiles of 64 keys each
+struct SkvTilePlan { int qw, splits, tiles; };
+void skv_fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split);   // 16 queries per workgroup
+SkvTilePlan skv_tile_fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D);
+SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D);
+int launch_skv_tile_fwd(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t st);
+int launch_skv_tile_dq(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t st);
+int launch_skv_dkv(const SkvAttnArgs &a, hipStream_t st);
+// dQ = the sum of its partial results [B*H*Nq][splits][D] in a.workspace, times *grad_scale, rounded
+int launch_split_sum(const SkvAttnArgs &a, int splits, hipStream_t st);
+// one fused backward pass while the per-wave accumulators of dQ fit: 32 queries up to head_dim 128, 16 at 256
+inline bool skv_bwd_one_pass(int64_t Nq, int D) { return D == 256 ? Nq <= 16 : Nq <= 32; }
+// workgroups that share the keys of a (batch, head) in that pass, given a workspace
+int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D);
+int64_t skv_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
 int launch_skv_bwd_long(const SkvAttnArgs &a, hipStream_t st);   // io_dtype QFA_F16, any Nq: dQ kernel + dKV kernel
 
 // Attention of a short query block on an INT8 cache (K and V quantized separately, Q quantized inside), after validation.

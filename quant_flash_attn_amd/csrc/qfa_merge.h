@@ -73,6 +73,33 @@ template <int D> __global__ __launch_bounds__(256) void split_merge_kernel(Split
          f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
 }
 
+// The same for few splits: D/4 lanes per query, 1024/D queries per workgroup.  A workgroup per query is as many workgroups
+// as rows, most of whose lanes have nothing to do where there are fewer splits than groups (64 heads, 200 queries, two
+// splits: the whole forward 32 -> 24 us).
+template <int D> __global__ __launch_bounds__(256) void split_merge_few_kernel(SplitMergeArgs a, int64_t rows) {
+  constexpr int CL = D / 4, RPW = 256 / CL;
+  const int d = 4 * (threadIdx.x % CL);
+  const int64_t row = (int64_t)blockIdx.x * RPW + threadIdx.x / CL, slot = row * a.splits;
+  if (row >= rows) return;
+  float m = NO_KEY, l = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s) {
+    const f32x2 ml = *reinterpret_cast<const f32x2 *>(a.pml + 2 * (slot + s));
+    const f32x4 y = *reinterpret_cast<const f32x4 *>(a.po + (slot + s) * D + d);
+    const float m_new = fmaxf(m, ml[0]), s0 = __builtin_amdgcn_exp2f(m - m_new), s1 = __builtin_amdgcn_exp2f(ml[0] - m_new);
+    m = m_new;
+    l = l * s0 + ml[1] * s1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = acc[e] * s0 + y[e] * s1;
+  }
+  const float inv = 1.0f / l;
+  if (a.lse && d == 0) a.lse[row] = (m + __log2f(l)) * kLn2;
+  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
+  store4(static_cast<char *>(a.o) + off * (a.o_dtype == QFA_F32 ? 4 : 2), a.o_dtype, d,
+         f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+}
+
 inline int64_t split_partial_bytes(int64_t rows, int64_t splits, int D) { return rows * splits * (int64_t)(D + 2) * 4; }
 
 // How `ntiles` tiles of keys are dealt: `wgs` workgroups of up to 16 of `rows` queries per split, at least 8 tiles each.
@@ -106,7 +133,9 @@ inline void split_plan(int64_t wgs, int64_t rows, int64_t ntiles, int D, int64_t
   *splits = (int)((ntiles + tps - 1) / tps);
 }
 template <int D> int launch_split_merge(const SplitMergeArgs &a, int64_t rows, const char *who, hipStream_t st) {
-  split_merge_kernel<D><<<dim3((unsigned)rows), dim3(256), 0, st>>>(a);
+  constexpr int RPW = 1024 / D;
+  if (a.splits <= 16 && rows >= 1024) split_merge_few_kernel<D><<<dim3((unsigned)((rows + RPW - 1) / RPW)), dim3(256), 0, st>>>(a, rows);
+  else split_merge_kernel<D><<<dim3((unsigned)rows), dim3(256), 0, st>>>(a);
   return check_launch(who);
 }
 

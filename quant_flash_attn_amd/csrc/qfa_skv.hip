@@ -9,7 +9,8 @@
 // tiles of the sequence are dealt round-robin to the waves, every wave runs its own online softmax
 // over its tiles from a private ring of LDS buffers filled by direct global->LDS loads (no
 // workgroup barrier in the loop), and the four partial results are merged at the end.  Longer query
-// blocks are split into several workgroups that run on the same XCD and share its L2 copy of the codes.
+// blocks are split into several workgroups that run on the same XCD and share its L2 copy of the codes, as long as
+// there is little to do: with more work the tiles of qfa_skv_tile.hip take over (skv_tile_fwd_plan).
 //
 // Codes as MFMA operands.  A code byte c (two's complement) with its top bit flipped is the
 // unsigned byte c + 128; OR-ed under the constant 0x6400 it is the binary16 number 1152 + c
@@ -61,13 +62,9 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
   static_assert(3 * MG * 4 <= 4 * WAVE, "the merge area overlays the rings");
   __shared__ __attribute__((aligned(16))) unsigned char smem[4 * WAVE];
 
-  // block id -> (batch*head, query block): the query blocks of one (batch, head) get ids that differ
-  // by 8, i.e. run on the same XCD close in time, and share its L2 copy of the codes
-  const int per_bh = a.qblocks * a.splits;
-  const int bh = (int)(blockIdx.x / (8 * per_bh)) * 8 + (int)(blockIdx.x % 8);
-  const int qb = (int)(blockIdx.x / 8) % a.qblocks;
-  const int split = ((int)(blockIdx.x / 8) % per_bh) / a.qblocks;
-  if (bh >= a.BH) return;
+  const XcdBlock id(a.BH, a.qblocks * a.splits);
+  if (!id.live) return;
+  const int bh = id.bh, qb = id.sub % a.qblocks, split = id.sub / a.qblocks;
   const int64_t b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x, lane = tid % 64, q16 = lane % 16, G = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -342,18 +339,11 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
   }
 }
 
-// How the keys of one query block are split over workgroups: as many as are resident at once (three per CU; a second,
-// partly filled round costs a whole one), at head_dim 256 about four per CU (two are resident), or what split_plan finds
-// better
-static void skv_split_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
-  const int64_t wgs = BH * ((Nq + 15) / 16);
-  const int64_t fill = D == 256 ? (wgs >= 512 ? 1 : (1024 + wgs - 1) / wgs) : 768 / wgs;
-  split_plan(wgs, BH * Nq, (Nk + SKV_TILE - 1) / SKV_TILE, D, fill, splits, tiles_per_split);
-}
-
 int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
   int splits, tps;
-  skv_split_plan(B * H, Nq, Nk, D, &splits, &tps);
+  if (const SkvTilePlan p = skv_tile_fwd_plan(B * H, Nq, Nk, D); p.qw)
+    return p.splits > 1 ? split_partial_bytes(B * H * Nq, p.splits, D) : 0;
+  skv_fwd16_plan(B * H, Nq, Nk, D, &splits, &tps);
   return splits > 1 ? split_partial_bytes(B * H * Nq, splits, D) : 0;
 }
 
@@ -371,11 +361,11 @@ template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const Skv
   a.tiles_per_split = (int)((x.Nk + SKV_TILE - 1) / SKV_TILE);
   a.po = a.pml = nullptr;
   if (x.workspace) {   // validated: large enough for the plan below
-    skv_split_plan(x.B * x.H, x.Nq, x.Nk, D, &a.splits, &a.tiles_per_split);
+    skv_fwd16_plan(x.B * x.H, x.Nq, x.Nk, D, &a.splits, &a.tiles_per_split);
     a.po = static_cast<float *>(x.workspace);
     a.pml = a.po + x.B * x.H * x.Nq * a.splits * (int64_t)D;
   }
-  const int64_t total = (int64_t)a.qblocks * a.splits * ((a.BH + 7) / 8) * 8;   // ids past batch*heads exit at once
+  const int64_t total = xcd_grid(a.BH, (int64_t)a.qblocks * a.splits);
   if (total > 0x7fffffffLL || (a.splits > 1 && x.B * x.H * x.Nq > 0x7fffffffLL))
     return set_error(QFA_EUNSUPPORTED, "attn_fwd_shared_kv: too many query blocks for one launch");
   skv_fwd_kernel<T, S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
@@ -441,6 +431,8 @@ int launch_skv_fwd_static(const SkvAttnArgs &x, hipStream_t st) {
 }
 
 int launch_skv_fwd(const SkvAttnArgs &x, hipStream_t st) {
+  if (const SkvTilePlan p = skv_tile_fwd_plan(x.B * x.H, x.Nq, x.Nk, x.D); p.qw && (p.splits == 1 || x.workspace))
+    return launch_skv_tile_fwd(x, p, st);
   if (x.io_dtype == QFA_F16) {
     if (x.D == 256) return launch_skv_fwd_td<_Float16, 256>(x, st);
     if (x.D == 128) return launch_skv_fwd_td<_Float16, 128>(x, st);

@@ -5,7 +5,9 @@
 // with KV = scale * (codes - zero_point) per token and delta = rowsum(O o dO) (:97-99).
 // Everything is computed in binary16 products with fp32 accumulation, like the reference.
 //
-// One workgroup = 4 waves = one (batch, head).  The 32-key tiles are dealt round-robin to the
+// One workgroup = 4 waves = one (batch, head), or a share of its keys: with few heads (and a workspace) the keys are split over
+// workgroups, each writes its own rows of dKV, and split_sum_kernel adds the partial dQ in a fixed order (5 heads, 16 queries,
+// 8000 keys of 128: 171 -> 19 us).  The 32-key tiles are dealt round-robin to the
 // waves; a wave streams its tiles through two private LDS slots (direct global->LDS loads, no
 // workgroup barrier in the loop), writes the dKV rows of a tile as soon as they are complete and
 // keeps a partial dQ in registers; the four partial dQ are summed at the end.  The last step of a
@@ -26,6 +28,7 @@
 #include <type_traits>
 
 #include "qfa_host.h"
+#include "qfa_merge.h"
 #include "qfa_skv_common.h"
 
 namespace qfa {
@@ -38,7 +41,9 @@ struct SkvBwdArgs {
   const float *grad_scale;     // nullable device scalar: dq and dkv are multiplied by it before rounding
   int grad_bf16;
   int64_t H;
-  int Nq, Nk;
+  int Nq, Nk, BH;
+  int splits, tiles_per_split;   // workgroups that share the keys of a (batch, head)
+  float *po;                     // splits > 1: partial dQ per query and split
   int64_t sqb, sqh, sqn, scb, sch, scn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn;
   float sm_scale, sm_scale_log2;
 };
@@ -82,7 +87,9 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
   constexpr int OPS = Copy::N + 2;
   __shared__ __attribute__((aligned(256))) unsigned char smem[SM::TOTAL];
 
-  const int bh = blockIdx.x;
+  const XcdBlock id(a.BH, a.splits);
+  if (!id.live) return;
+  const int bh = id.bh, split = id.sub;
   const int64_t b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -95,14 +102,14 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
 
   const unsigned char *codes_bh = reinterpret_cast<const unsigned char *>(a.codes + b * a.scb + h * a.sch);
   const int64_t tk0 = (int64_t)bh * a.Nk, tq0 = (int64_t)bh * a.Nq;
-  const int ntiles = (a.Nk + SKV_TILE - 1) / SKV_TILE;
+  const int t0 = split * a.tiles_per_split, ntiles = min(a.tiles_per_split, (a.Nk + SKV_TILE - 1) / SKV_TILE - t0);
   const int my_tiles = ntiles > wave ? (ntiles - wave + 3) / 4 : 0;
 
   // ---- tile copies (as in the forward)
   Copy cp;
   cp.init((unsigned)a.scn, lane);
   auto issue = [&](int i) {
-    const int t = wave + 4 * i;
+    const int t = t0 + wave + 4 * i;
     unsigned char *slot = smem + wave_off + (i % SKVB_NBUF) * SM::SLOT;
     const int rows = min(SKV_TILE, a.Nk - t * SKV_TILE);
     const rsrc_t rs_k = make_rsrc(codes_bh + (int64_t)t * SKV_TILE * a.scn, (unsigned)((rows - 1) * (int)a.scn + D));
@@ -236,7 +243,7 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     const unsigned char *slot = smem + slot_off;
     const unsigned *skp = reinterpret_cast<const unsigned *>(slot + SM::K_BYTES);
     const unsigned *zpp = skp + SKV_TILE;
-    const int j0 = (wave + 4 * i) * SKV_TILE;
+    const int j0 = (t0 + wave + 4 * i) * SKV_TILE;
     const bool key_ok = j0 + lr < a.Nk;
     const float sk = scale_of(skp[lr]);
     const unsigned zmine = zpp[lr];
@@ -323,7 +330,7 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
   };
   auto tile_dkv = [&](int i) {
     // ---- 4. dKV^T = dO^T P + Q^T dS for one block of 32 d at a time; column = this lane's key
-    const int j0 = (wave + 4 * i) * SKV_TILE;
+    const int j0 = (t0 + wave + 4 * i) * SKV_TILE;
     unsigned char *stage = smem + wave_off + SKVB_NBUF * SM::SLOT;
     // two blocks (64 columns, 128 bytes a row) are staged in LDS and leave as whole 128-byte lines:
     // 16-byte pair p of row j sits at position p ^ (j % 8)
@@ -394,7 +401,21 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
       for (int v = 0; v < 16; ++v) dst[(32 * db + 8 * (v / 4) + 4 * g + v % 4) * 32 + lr] = dq[db][v] - w_tot;
   }
   __syncthreads();
-  if (wave == 0 && lr < a.Nq) {
+  if (wave == 0 && lr < a.Nq && a.splits > 1) {
+    float *prow = a.po + ((tq0 + lr) * a.splits + split) * D;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int aa = 0; aa < 4; ++aa) {
+        f32x4 r;
+#pragma unroll
+        for (int bb = 0; bb < 4; ++bb) {
+          const int d = 32 * db + 8 * aa + 4 * g + bb;
+          r[bb] = dq[db][4 * aa + bb] - w_tot + mg[d * 32 + lr] + mg[MG + d * 32 + lr] + mg[2 * MG + d * 32 + lr];
+        }
+        *reinterpret_cast<f32x4 *>(prow + 32 * db + 8 * aa + 4 * g) = r;
+      }
+  } else if (wave == 0 && lr < a.Nq) {
     _Float16 *qrow = a.dq + b * a.sdqb + h * a.sdqh + (int64_t)lr * a.sdqn;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -427,12 +448,54 @@ template <typename S, int D> static int launch_skv_bwd_sd(const SkvAttnArgs &x, 
   a.sdqb = x.sdqb; a.sdqh = x.sdqh; a.sdqn = x.sdqn; a.sdkb = x.sdkb; a.sdkh = x.sdkh; a.sdkn = x.sdkn;
   a.sm_scale = x.sm_scale;
   a.sm_scale_log2 = x.sm_scale * kLog2e;
-  const int64_t total = x.B * x.H;
+  a.BH = (int)(x.B * x.H);
+  const int ntiles = (int)((x.Nk + SKV_TILE - 1) / SKV_TILE);
+  a.splits = 1;
+  a.tiles_per_split = ntiles;
+  a.po = static_cast<float *>(x.workspace);
+  if (x.workspace) {
+    a.splits = skv_bwd_splits(x.B * x.H, x.Nq, x.Nk, D);
+    a.tiles_per_split = (ntiles + a.splits - 1) / a.splits;   // (the plan's splits are those that this leaves non-empty)
+  }
+  const int64_t total = xcd_grid(x.B * x.H, a.splits);
   if (total > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many (batch, head) pairs for one launch");
   if (x.Nq <= 16) skv_bwd_kernel<S, D, true><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   else if constexpr (D <= 128) skv_bwd_kernel<S, D, false><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   else return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: the one-pass kernel takes at most 16 queries at head_dim 256");
-  return check_launch("qfa_attn_bwd_shared_kv");
+  if (int e = check_launch("qfa_attn_bwd_shared_kv")) return e;
+  return a.splits > 1 ? launch_split_sum(x, a.splits, st) : 0;
+}
+
+struct SplitSumArgs {
+  const float *po;
+  void *dq;
+  const float *grad_scale;
+  int64_t H, rows, sdqb, sdqh, sdqn;
+  int Nq, splits, dtype;
+};
+// D/4 lanes per query, all loads of a thread independent
+template <int D> __global__ __launch_bounds__(256) void split_sum_kernel(SplitSumArgs a) {
+  constexpr int CL = D / 4, RPW = 256 / CL;
+  const int d = 4 * (threadIdx.x % CL);
+  const int64_t row = (int64_t)blockIdx.x * RPW + threadIdx.x / CL;
+  if (row >= a.rows) return;
+  const float *p = a.po + row * a.splits * D + d;
+  const float osc = a.grad_scale ? *a.grad_scale : 1.0f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int s = 0; s < a.splits; ++s) acc += *reinterpret_cast<const f32x4 *>(p + (int64_t)s * D);
+  const int64_t bh = row / a.Nq, off = bh / a.H * a.sdqb + bh % a.H * a.sdqh + row % a.Nq * a.sdqn;
+  store4(static_cast<unsigned short *>(a.dq) + off, a.dtype, d, f32x4{acc[0] * osc, acc[1] * osc, acc[2] * osc, acc[3] * osc});
+}
+int launch_split_sum(const SkvAttnArgs &x, int splits, hipStream_t st) {
+  const SplitSumArgs a = {static_cast<const float *>(x.workspace), x.dq, x.grad_scale, x.H, x.B * x.H * x.Nq, x.sdqb, x.sdqh, x.sdqn,
+                          (int)x.Nq, splits, x.grad_dtype};
+  const int64_t rpw = 1024 / x.D, blocks = (a.rows + rpw - 1) / rpw;
+  if (blocks > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many queries for one launch");
+  if (x.D == 256) split_sum_kernel<256><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
+  else if (x.D == 128) split_sum_kernel<128><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
+  else split_sum_kernel<64><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(a);
+  return check_launch("qfa_attn_bwd_shared_kv (sum of dQ)");
 }
 
 int launch_skv_bwd(const SkvAttnArgs &x, hipStream_t st) {

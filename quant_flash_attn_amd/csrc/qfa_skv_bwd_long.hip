@@ -1,22 +1,18 @@
-// Backward of the shared-KV attention for query blocks of any length, in two kernels (the fused
-// one-pass kernel of qfa_skv_bwd.hip keeps a (batch, head)'s whole dQ in registers and is limited to
-// 32 queries).  Same mathematics (quant_flash_attn.py:104-166):
+// Backward of the shared-KV attention for query blocks that the fused one-pass kernel (qfa_skv_bwd.hip) does not take, as a dQ
+// kernel and a dKV kernel.  Same mathematics (quant_flash_attn.py:104-166):
 //     P = exp(sm_scale * Q KV^T - LSE),   dP = dO KV^T,   dS = sm_scale * P o (dP - delta),
 //     dQ = dS KV,   dKV = P^T dO + dS^T Q,   delta = rowsum(O o dO)
 //
-// skv_dq_kernel   one workgroup per block of 16 queries, built like the forward: the 32-key tiles are
-//                 dealt to the four waves, streamed through private LDS rings, S^T and dP^T share the
-//                 expanded code operands, dS * scale_j is the operand of dQ^T += C^T (dS*scale)^T, the
-//                 four partial dQ are summed at the end.  LSE is known, so there is no running maximum.
-// skv_dkv_kernel  one workgroup per 128 keys of a (batch, head): every wave owns ONE 32-key tile for the
-//                 whole kernel (its code operands expanded once into registers, its dKV^T accumulators in
-//                 registers) and the workgroup walks over the query blocks of 32, whose Q / dO / O rows
-//                 arrive in a double-buffered LDS area by direct global->LDS loads.  Every (tile, query
-//                 block) pair is visited once; each dKV row is written once, as whole 128-byte lines.
-//                 At D = 256 the accumulators of a tile do not fit one wave: two waves share a tile, each
-//                 keeping 128 of the 256 columns (both compute S and dP), a workgroup covers 64 keys and
-//                 the row area is single-buffered.
-// Both recompute delta from O and dO (no workspace), S and dP are computed in both kernels.
+// dQ    skv_dq_kernel here where there is little to do: one workgroup per block of 16 queries, built like the forward of
+//       qfa_skv.hip (the 32-key tiles are dealt to the four waves, streamed through private LDS rings, S^T and dP^T share the
+//       expanded code operands, dS * scale_j is the operand of dQ^T += C^T (dS*scale)^T, the four partial dQ are summed at the
+//       end).  Its tiles start at once; with more work skv_tile_dq_kernel (qfa_skv_tile.hip) takes over (skv_tile_dq_plan).
+// dKV   skv_dkv_kernel (qfa_skv_dkv.hip) up to head_dim 128.  At 256 the accumulators of a tile do not fit one of two waves per
+//       SIMD: in skv_dkv256_kernel two waves share a tile of 32 keys, each keeping 128 of the 256 columns (both compute S and
+//       dP), a workgroup covers 64 keys and walks over the query blocks of 32, whose Q / dO rows arrive in LDS by direct loads.
+//       (skv_dkv_kernel with one wave per SIMD takes 1.25 instead of 1.07 ms for the backward of 1584 heads, 97 queries, 689
+//       keys.)
+// All of them compute delta from O and dO; S and dP are computed for dQ and for dKV.
 #include <type_traits>
 
 #include "qfa_host.h"
@@ -49,10 +45,9 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
   static_assert(3 * MG * 4 <= 4 * WAVE, "the merge area overlays the rings");
   __shared__ __attribute__((aligned(16))) unsigned char smem[4 * WAVE];
 
-  // query blocks of one (batch, head) get ids that differ by 8: same XCD, shared L2 copy of the codes
-  const int bh = (int)(blockIdx.x / (8 * a.qblocks)) * 8 + (int)(blockIdx.x % 8);
-  const int qb = (int)(blockIdx.x / 8) % a.qblocks;
-  if (bh >= a.BH) return;
+  const XcdBlock id(a.BH, a.qblocks);
+  if (!id.live) return;
+  const int bh = id.bh, qb = id.sub;
   const int64_t b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x, lane = tid % 64, q16 = lane % 16, G = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -267,37 +262,29 @@ template <int D> struct RowSwz {
   static __device__ __forceinline__ int swz(int i) { return (2 * (i % 4) + (i / 4) % 2 + 8 * ((i / 8) % 2)) % CPR; }
 };
 
-template <int D> struct SkvDkvSmem {
-  static constexpr int DS = D == 256 ? 2 : 1;                    // waves sharing one tile (each keeps D / DS columns of dKV)
-  static constexpr int NRB = D == 256 ? 1 : 2;                   // row buffers
-  static constexpr bool O_IN_LDS = NRB == 2;                     // one buffer: O (needed for delta only) is read from memory
-  static constexpr int SLOT = SKV_TILE * D + 2 * SKV_TILE * 4;   // one tile copy per wave, used in the prologue only
+struct SkvDkvSmem {
+  static constexpr int D = 256, DS = 2;                          // waves sharing one tile (each keeps D / DS columns of dKV)
+  static constexpr int SLOT = SKV_TILE * D + 2 * SKV_TILE * 4;   // one tile copy per wave
   static constexpr int ROWS = 32 * D * 2;                        // one block of 32 binary16 rows
-  static constexpr int BUF = (O_IN_LDS ? 3 : 2) * ROWS;          // Q, dO (, O) of one query block
-  static constexpr int OFF_SLOT = NRB * BUF;                     // tile copies behind the row buffers: both are
-  static constexpr int OFF_STAT = OFF_SLOT + 4 * SLOT;           //   copied at once in the prologue
+  static constexpr int BUF = 2 * ROWS;                           // Q, dO of one query block
+  static constexpr int OFF_SLOT = BUF;                           // tile copies behind the rows: both are copied at once in the prologue
+  static constexpr int OFF_STAT = OFF_SLOT + 4 * SLOT;
   static constexpr int STAGE = 32 * 128;                         // per wave: 64 columns of its tile's dKV rows on their way out
-  // where the stages live while the rows stay resident: in the O rows (not needed after the statistics) when
-  // two stages fit one block of them, else in the tile slot when a stage fits it, else in an area of their own
-  static constexpr int STAGE_MODE = O_IN_LDS && 2 * STAGE <= ROWS ? 0 : (!O_IN_LDS && STAGE <= SLOT ? 2 : 1);
-  static constexpr int OFF_STAGE = OFF_STAT + NRB * 4 * 32 * 4;  // per buffer: lse (log2), delta, rowsum(Q), rowsum(dO)
-  static constexpr int TOTAL = OFF_STAGE + (STAGE_MODE == 1 ? 4 * STAGE : 0);
-  static_assert(4 * STAGE <= NRB * BUF, "the output stage overlays the row buffers");
+  static constexpr int TOTAL = OFF_STAT + 4 * 32 * 4;            // statistics: lse (log2), delta, rowsum(Q), rowsum(dO)
+  static_assert(4 * STAGE <= BUF && STAGE <= SLOT, "the output stage overlays the rows or the slot");
   static_assert(ROWS % 256 == 0, "row offsets are XOR-ed with block offsets");
   static_assert(2 * TOTAL <= 160 * 1024, "two workgroups per CU");
 };
 
-// KEEP: all query blocks fit the row buffers (Nq <= 32 * NRB).  They are copied once, their statistics are
-// computed once, and the workgroup then walks over `cpw` consecutive 128-key chunks of its (batch, head)
-// with no barrier at all: each wave waits for its own tile copy, expands it into registers, puts the copy
-// of its next tile into the same slot, and computes.  Otherwise (longer query blocks) one workgroup per
-// chunk, the row blocks cycling through the buffers with two barriers a block.
-template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_dkv_kernel(SkvBwdLongArgs a) {
-  typedef SkvDkvSmem<D> SM;
+// KEEP: at most 32 queries.  They are copied once, their statistics are computed once, and the workgroup then walks over `cpw`
+// consecutive 64-key chunks of its (batch, head) with no barrier at all.  Otherwise one workgroup per chunk, two barriers per
+// block of rows.
+template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_dkv256_kernel(SkvBwdLongArgs a) {
+  typedef SkvDkvSmem SM;
+  constexpr int D = SM::D, DS = SM::DS;
   typedef Swz<D> KSW;
   typedef TileCopy<D, SKV_TILE, 64, KSW> Copy;
   typedef TileCopy<D * 2, 32, 256, RowSwz<D>> RowCopy;
-  constexpr int DS = SM::DS, NRB = SM::NRB;
   constexpr int DB = D / 32, DBW = DB / DS, CPR = D / 8, KD = D / 16;
   __shared__ __attribute__((aligned(256))) unsigned char smem[SM::TOTAL];
 
@@ -319,31 +306,28 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
     return a.grad_bf16 ? pack2<__bf16>(x * osc, y * osc) : pack2<_Float16>(x * osc, y * osc);
   };
 
-  // ---- row copies of a query block: Q, dO (, O) -> buffer (direct loads)
-  RowCopy cq, cd, co;
+  // ---- row copies of a query block: Q, dO (direct loads)
+  RowCopy cq, cd;
   cq.init((unsigned)(a.sqn * 2), tid);
   cd.init((unsigned)(a.sdon * 2), tid);
-  co.init((unsigned)(a.son * 2), tid);
   const _Float16 *q_bh = a.q + b * a.sqb + h * a.sqh, *d_bh = a.dout + b * a.sdob + h * a.sdoh, *o_bh = a.o + b * a.sob + h * a.soh;
   auto issue_rows = [&](int qb) {
-    unsigned char *buf = smem + (qb % NRB) * SM::BUF;
+    unsigned char *buf = smem;
     const int rows = min(32, a.Nq - 32 * qb);
     // rows past Nq read as zeros (exact bounds)
     const rsrc_t rq = make_rsrc(q_bh + (int64_t)32 * qb * a.sqn, (unsigned)(((rows - 1) * (int)a.sqn + D) * 2));
     const rsrc_t rd = make_rsrc(d_bh + (int64_t)32 * qb * a.sdon, (unsigned)(((rows - 1) * (int)a.sdon + D) * 2));
-    const rsrc_t ro = make_rsrc(o_bh + (int64_t)32 * qb * a.son, (unsigned)(((rows - 1) * (int)a.son + D) * 2));
 #pragma unroll
     for (int c = 0; c < RowCopy::N; ++c) {
       cq.issue_one(rq, buf, wave, tid, c);
       cd.issue_one(rd, buf + SM::ROWS, wave, tid, c);
-      if (SM::O_IN_LDS) co.issue_one(ro, buf + 2 * SM::ROWS, wave, tid, c);
     }
   };
-  // delta, row sums, LSE of block qb from its buffer (thread = row tid/8, chunks tid%8 + 8k).  One buffer:
-  // O does not pass through LDS, `og` holds this thread's chunks of it.
+  // delta, row sums, LSE of block qb from its rows (thread = row tid/8, chunks tid%8 + 8k); `og` holds this thread's chunks
+  // of O, which does not pass through LDS
   auto block_stats = [&](int qb, const u32x4 *og) {
-    const unsigned char *buf = smem + (qb % NRB) * SM::BUF;
-    float *stat = reinterpret_cast<float *>(smem + SM::OFF_STAT) + (qb % NRB) * 128;
+    const unsigned char *buf = smem;
+    float *stat = reinterpret_cast<float *>(smem + SM::OFF_STAT);
     const int pi = tid / 8, part = tid % 8;
     float dsum = 0.f, rq = 0.f, rd = 0.f;
 #pragma unroll
@@ -351,7 +335,7 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
       const int off = pi * (D * 2) + ((c ^ RowSwz<D>::swz(pi)) << 4);
       const u32x4 qv = *reinterpret_cast<const u32x4 *>(buf + off);
       const u32x4 dv = *reinterpret_cast<const u32x4 *>(buf + SM::ROWS + off);
-      const u32x4 ov = SM::O_IN_LDS ? *reinterpret_cast<const u32x4 *>(buf + 2 * SM::ROWS + off) : og[c / 8];
+      const u32x4 ov = og[c / 8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const unsigned qw = qv[e], dw = dv[e], ow = ov[e];
@@ -375,7 +359,7 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
       stat[96 + pi] = rd;
     }
   };
-  auto load_o = [&](int qb, u32x4 *og) {   // one buffer: this thread's chunks of O straight from memory
+  auto load_o = [&](int qb, u32x4 *og) {
     const int pi = tid / 8, part = tid % 8;
     const bool live = 32 * qb + pi < a.Nq;
 #pragma unroll
@@ -425,8 +409,8 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
   f32x16 dkv[DBW];
   // dKV^T of this wave's tile += contributions of query block qb (its rows and statistics are in LDS)
   auto add_block = [&](int qb, bool key_ok) {
-    const unsigned char *buf = smem + (qb % NRB) * SM::BUF;
-    const float *stat = reinterpret_cast<const float *>(smem + SM::OFF_STAT) + (qb % NRB) * 128;
+    const unsigned char *buf = smem;
+    const float *stat = reinterpret_cast<const float *>(smem + SM::OFF_STAT);
     const float a_sk = key_ok ? a.sm_scale_log2 * sk : 0.f;
     const float sm_k = key_ok ? a.sm_scale : 0.f;
     // operands of the rank-1 offset removal: one scaling for the whole query block
@@ -457,22 +441,17 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
     }
     sacc = mfma_h(corr_q, corr_k, sacc);
     pacc = mfma_h(corr_do, corr_k, pacc);
-    // The transposed rows are requested a block of 32 columns ahead of its products, the first under p and ds (99 x 53 heads,
-    // 97 queries, 689 keys: 1055 -> 1028 us); at head_dim 256 the registers are full and they are requested when needed.
-    constexpr bool AHEAD = D < 256;
-    const unsigned bufa = lds0 + (qb % NRB) * SM::BUF;
-    u32x2 fr[2][2][2];   // [matrix: dO, Q][hh][r]
+    u32x2 fr[2][2][2];   // [matrix: dO, Q][hh][r], requested when needed: the registers are full
     auto request = [&](int db) __attribute__((always_inline)) {
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-          const unsigned ad = bufa + (qt_off[hh][r] ^ ((4 * (db0 + db)) << 4));
+          const unsigned ad = lds0 + (qt_off[hh][r] ^ ((4 * (db0 + db)) << 4));
           fr[0][hh][r] = lds_read_tr16_async<SM::ROWS>(ad);
           fr[1][hh][r] = lds_read_tr16_async<0>(ad);
         }
     };
-    if (AHEAD) request(0);
     // p and ds for this lane's key; registers run over the queries 8aa + 4g + bb
     u32x4 pf[2], df[2];
 #pragma unroll
@@ -495,12 +474,11 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
     // dKV^T += dO^T P + Q^T dS
 #pragma unroll
     for (int db = 0; db < DBW; ++db) {
-      if (!AHEAD) request(db);
+      request(db);
       lds_wait_all();
       u32x2 now[2][2][2];
 #pragma unroll
       for (int x = 0; x < 8; ++x) now[x / 4][x / 2 % 2][x % 2] = tie(fr[x / 4][x / 2 % 2][x % 2]);
-      if (AHEAD && db + 1 < DBW) request(db + 1);
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         const u32x2(&d)[2] = now[0][hh], (&q)[2] = now[1][hh];
@@ -540,41 +518,29 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
       for (int v = 0; v < 16; ++v) dkv[db][v] = 0.f;
   };
 
+  u32x4 og[(CPR + 7) / 8];
   if (KEEP) {
-    // ---- rows of every query block and the first tile, copied together; statistics once
+    // ---- the rows and the first tile, copied together; statistics once
     if (tile_of(c_begin) < ntiles) issue_tile(tile_of(c_begin));
-    for (int qb = 0; qb < nqb; ++qb) issue_rows(qb);
-    u32x4 og[SM::O_IN_LDS ? 1 : (CPR + 7) / 8];
-    if (!SM::O_IN_LDS) load_o(0, og);
+    issue_rows(0);
+    load_o(0, og);
     dma_wait();
     __syncthreads();
-    for (int qb = 0; qb < nqb; ++qb) block_stats(qb, og);
+    block_stats(0, og);
     __syncthreads();
-    // stage: in the O rows (waves 0,1 use buffer 0's, waves 2,3 buffer 1's), in an area of its own, or in the
-    // wave's tile slot once its operands are in registers
-    unsigned char *stage = SM::STAGE_MODE == 0 ? smem + (wave / 2) * SM::BUF + 2 * SM::ROWS + (wave % 2) * SM::STAGE
-                           : SM::STAGE_MODE == 1 ? smem + SM::OFF_STAGE + wave * SM::STAGE : slot;
-    // The dKV stores share the memory counter with the tile copies, so the wait for the next tile sits
-    // BEFORE the stores of the current one: by then the copy, issued a whole compute phase earlier, is the
-    // only thing that can still be in flight.  (Stage in the slot: the copy can only be issued after the
-    // stores, and the wait at the top of the next round also covers them.)
+    // The output stage is the wave's tile slot once its operands are in registers, so the next tile's copy goes out after the
+    // stores, and the wait at the top of the next round covers both.
     for (int c = c_begin; c < c_end; ++c) {
       const int t = tile_of(c);
       if (t >= ntiles) break;   // (tiles of a wave grow with c)
-      if (SM::STAGE_MODE == 2) dma_wait();
+      dma_wait();
       expand_tile();
       const int tn = tile_of(c + 1);
-      const bool more = c + 1 < c_end && tn < ntiles;
-      if (SM::STAGE_MODE != 2 && more) {   // the slot is free once its contents are in registers
-        lds_wait_all();
-        issue_tile(tn);
-      }
       clear_dkv();
       const int j0 = t * SKV_TILE;
-      for (int qb = 0; qb < nqb; ++qb) add_block(qb, j0 + lr < a.Nk);
-      if (SM::STAGE_MODE != 2) dma_wait();
-      write_out(stage, j0);
-      if (SM::STAGE_MODE == 2 && more) {   // the stage was the slot: refill it only now
+      add_block(0, j0 + lr < a.Nk);
+      write_out(slot, j0);
+      if (c + 1 < c_end && tn < ntiles) {
         lds_wait_all();
         issue_tile(tn);
       }
@@ -582,7 +548,7 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
     return;
   }
 
-  // ---- one chunk per workgroup, the row blocks cycle through the buffers
+  // ---- one chunk per workgroup
   const int t = tile_of(c_begin);
   const bool t_ok = t < ntiles;                   // (a wave without a tile still takes part in copies and barriers)
   const int j0 = t * SKV_TILE;
@@ -592,20 +558,18 @@ template <typename S, int D, bool KEEP> __global__ __launch_bounds__(256, 2) voi
   if (t_ok) expand_tile();
   clear_dkv();
   for (int qb = 0; qb < nqb; ++qb) {
-    if (NRB == 1 && qb > 0) {
+    if (qb > 0) {
       __syncthreads();   // everybody is done with block qb-1
       issue_rows(qb);
     }
-    u32x4 og[SM::O_IN_LDS ? 1 : (CPR + 7) / 8];
-    if (!SM::O_IN_LDS) load_o(qb, og);
+    load_o(qb, og);
     dma_wait();          // this thread's share of block qb has landed ...
-    __syncthreads();     // ... and everybody's; (two buffers:) everybody is also done with block qb-1
+    __syncthreads();     // ... and everybody's
     block_stats(qb, og);
-    if (NRB == 2 && qb + 1 < nqb) issue_rows(qb + 1);   // the other buffer: nobody reads it any more
     __syncthreads();
     if (t_ok) add_block(qb, j0 + lr < a.Nk);
   }
-  __syncthreads();   // the row buffers are done with: the stages overlay them
+  __syncthreads();   // the rows are done with: the stages overlay them
   if (t_ok) write_out(smem + wave * SM::STAGE, j0);
 }
 
@@ -625,25 +589,34 @@ template <typename S, int D> static int launch_skv_bwd_long_sd(const SkvAttnArgs
   if (x.B * x.H > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many (batch, head) pairs");
   a.BH = (int)(x.B * x.H);
   a.qblocks = (int)((x.Nq + 15) / 16);
-  const int keys_per_wg = 4 * SKV_TILE / SkvDkvSmem<D>::DS;
-  a.kchunks = (int)((x.Nk + keys_per_wg - 1) / keys_per_wg);
-  // query blocks that fit the row buffers stay resident and a workgroup walks over several chunks: as many
-  // as leave about 2048 workgroups (four rounds of two per CU)
-  const bool keep = x.Nq <= 32 * SkvDkvSmem<D>::NRB;
-  a.cpw = 1;
-  if (keep) {
-    const int64_t want = ((int64_t)a.kchunks * a.BH + 2047) / 2048;
-    a.cpw = (int)(want < 1 ? 1 : want > a.kchunks ? a.kchunks : want);
+  const int64_t total_q = xcd_grid(a.BH, a.qblocks);
+  if (total_q > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many blocks for one launch");
+  const SkvTilePlan p = skv_tile_dq_plan(x.B * x.H, x.Nq, x.Nk, D);
+  if (p.qw && (p.splits == 1 || x.workspace)) {
+    if (int e = launch_skv_tile_dq(x, p, st)) return e;
+  } else {
+    skv_dq_kernel<S, D><<<dim3((unsigned)total_q), dim3(256), 0, st>>>(a);
+    if (int e = check_launch("qfa_attn_bwd_shared_kv (dQ)")) return e;
   }
-  const int64_t total_q = (int64_t)a.qblocks * ((a.BH + 7) / 8) * 8;
-  const int64_t total_k = (int64_t)((a.kchunks + a.cpw - 1) / a.cpw) * a.BH;
-  if (total_q > 0x7fffffffLL || total_k > 0x7fffffffLL)
-    return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many blocks for one launch");
-  skv_dq_kernel<S, D><<<dim3((unsigned)total_q), dim3(256), 0, st>>>(a);
-  if (int e = check_launch("qfa_attn_bwd_shared_kv (dQ)")) return e;
-  if (keep) skv_dkv_kernel<S, D, true><<<dim3((unsigned)total_k), dim3(256), 0, st>>>(a);
-  else skv_dkv_kernel<S, D, false><<<dim3((unsigned)total_k), dim3(256), 0, st>>>(a);
-  return check_launch("qfa_attn_bwd_shared_kv (dKV)");
+  if constexpr (D < 256) {
+    return launch_skv_dkv(x, st);
+  } else {
+    const int keys_per_wg = 4 * SKV_TILE / SkvDkvSmem::DS;
+    a.kchunks = (int)((x.Nk + keys_per_wg - 1) / keys_per_wg);
+    // a query block that stays resident: a workgroup walks over as many chunks as leave about 2048 workgroups (four rounds of
+    // two per CU)
+    const bool keep = x.Nq <= 32;
+    a.cpw = 1;
+    if (keep) {
+      const int64_t want = ((int64_t)a.kchunks * a.BH + 2047) / 2048;
+      a.cpw = (int)(want < 1 ? 1 : want > a.kchunks ? a.kchunks : want);
+    }
+    const int64_t total_k = (int64_t)((a.kchunks + a.cpw - 1) / a.cpw) * a.BH;
+    if (total_k > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many blocks for one launch");
+    if (keep) skv_dkv256_kernel<S, true><<<dim3((unsigned)total_k), dim3(256), 0, st>>>(a);
+    else skv_dkv256_kernel<S, false><<<dim3((unsigned)total_k), dim3(256), 0, st>>>(a);
+    return check_launch("qfa_attn_bwd_shared_kv (dKV)");
+  }
 }
 
 int launch_skv_bwd_long(const SkvAttnArgs &x, hipStream_t st) {

@@ -8,6 +8,7 @@
 // the codes are contracted over d, a v_dot2 accumulation where they are contracted over tokens).
 #pragma once
 #include "qfa_device.h"
+#include "qfa_host.h"
 
 namespace qfa {
 
@@ -109,6 +110,24 @@ __device__ __forceinline__ void skv_issue_tile(const Copy &cp, unsigned char *sl
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_z, (lptr_t)(slot + SKV_TILE * D + SKV_TILE * 4), 1, lane, 0, 0, 0);
   }
 }
+
+// Workgroup -> (batch*head, workgroup of it).  Consecutive ids go round the 8 XCDs.  The workgroups of a (batch, head) run on
+// one XCD close in time and share its L2 copy of the codes: whole heads are dealt to the XCDs in turn, which keeps all of
+// them in the same region of memory (a cache of 256 heads, 8192 keys: 97 us, 100 with a contiguous eighth of the heads each).
+// Few heads that 8 does not divide would leave XCDs idle (two heads ran on two of them): there every XCD takes a contiguous
+// eighth of all pairs.  Ids past the last pair are not live.
+struct XcdBlock {
+  int bh, sub;
+  bool live;
+  __device__ __forceinline__ XcdBlock(int BH, int per_bh) {
+    const unsigned xcd = blockIdx.x % 8, at = blockIdx.x / 8;
+    const bool whole = xcd_whole_heads(BH);
+    const unsigned id = whole ? at : xcd * (gridDim.x / 8) + at, head = id / (unsigned)per_bh;
+    bh = (int)(whole ? head * 8 + xcd : head);
+    sub = (int)(id - head * (unsigned)per_bh);
+    live = bh < BH;
+  }
+};
 
 // wait for every LDS operation of this wave; `tie` keeps the users of an asynchronously loaded
 // register pair behind the wait that precedes it in program order

@@ -39,7 +39,8 @@ struct Api {
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
-  QFA_ENTRY(qfa_attn_bwd_shared_kv);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_workspace_bytes);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_split);
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
@@ -65,7 +66,8 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
-  QFA_ENTRY(qfa_attn_bwd_shared_kv);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_workspace_bytes);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_split);
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
@@ -577,7 +579,7 @@ std::tuple<Tensor, Tensor> skv_fwd(const Tensor &q_in, const Tensor &codes_in, c
 
 std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, const Tensor &scale_in, const Tensor &zp_in,
                                    const Tensor &o_in, const Tensor &do_in, const Tensor &lse_in, double sm,
-                                   at::ScalarType grad_dtype, const std::optional<Tensor> &grad_scale_in) {
+                                   at::ScalarType grad_dtype, const std::optional<Tensor> &grad_scale_in, bool split) {
   TORCH_CHECK_TYPE(q_in.scalar_type() == at::kHalf && o_in.scalar_type() == at::kHalf,
                    "the shared-KV backward kernel computes in float16: q and o must be float16");
   TORCH_CHECK_TYPE(is_io(grad_dtype), "grad_dtype must be float16 or bfloat16, got ", grad_dtype);
@@ -599,13 +601,17 @@ std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, c
                lse = flat(lse_in, at::kFloat, B * H * Nq, "lse");
   const Tensor q = rows16(q_in), codes = rows16(codes_in), o = rows16(o_in), dout = rows16(to(do_in, at::kHalf));
   Tensor dq = empty({B, H, Nq, D}, grad_dtype, q), dkv = empty({B, H, Nk, D}, grad_dtype, q);
-  check(api.qfa_attn_bwd_shared_kv(q.data_ptr(), codes.data_ptr<int8_t>(), scale.data_ptr(), dtype_code(scale.scalar_type()),
+  // scratch for the split over keys where B*H alone cannot fill the GPU (0: no split)
+  const int64_t ws_bytes = split ? api.qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) : 0;
+  Tensor ws;
+  if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, q);
+  check(api.qfa_attn_bwd_shared_kv_split(q.data_ptr(), codes.data_ptr<int8_t>(), scale.data_ptr(), dtype_code(scale.scalar_type()),
                                    zp.data_ptr<int8_t>(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
                                    dq.data_ptr(), dkv.data_ptr(), QFA_F16, dtype_code(grad_dtype),
                                    grad_scale.defined() ? grad_scale.data_ptr<float>() : nullptr, B, H, Nq, Nk, (int)D,
                                    QFA_STRIDES(q), QFA_STRIDES(codes), QFA_STRIDES(o), QFA_STRIDES(dout), QFA_STRIDES(dq),
-                                   QFA_STRIDES(dkv), (float)sm, stream_of(q)),
-        "qfa_attn_bwd_shared_kv");
+                                   QFA_STRIDES(dkv), (float)sm, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q)),
+        "qfa_attn_bwd_shared_kv_split");
   return {dq, dkv};
 }
 
@@ -651,7 +657,7 @@ struct SharedFn : torch::autograd::Function<SharedFn> {
     // while they round them.  q and o convert exactly from bf16 (more mantissa, values of order one).
     auto [do16, back] = normalised_dout(grads[0], s[2]);
     auto [dq, dkv] = skv_bwd(to(q, at::kHalf), s[1], s[2], s[3], to(o, at::kHalf), do16, s[5],
-                             ctx->saved_data["sm"].toDouble(), q.scalar_type(), back);
+                             ctx->saved_data["sm"].toDouble(), q.scalar_type(), back, true);
     return {dq, to(dkv, (at::ScalarType)ctx->saved_data["kv_dtype"].toInt()), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -727,7 +733,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv", &qkv, nogil());
   m.def("cache", &cache, nogil());
   m.def("skv_fwd", &skv_fwd, nogil());
-  m.def("skv_bwd", &skv_bwd, nogil());
+  // (what qfa_attn_bwd_shared_kv returns, bit for bit: not split)
+  m.def("skv_bwd", [](const Tensor &q, const Tensor &codes, const Tensor &scale, const Tensor &zp, const Tensor &o, const Tensor &dout,
+                      const Tensor &lse, double sm, at::ScalarType grad_dtype, const std::optional<Tensor> &grad_scale) {
+    return skv_bwd(q, codes, scale, zp, o, dout, lse, sm, grad_dtype, grad_scale, false);
+  }, nogil());
   m.def("normalised_dout", &normalised_dout, nogil());
   m.def("shared", &shared, nogil());
 }

@@ -41,10 +41,10 @@ def attn_bwd_quantized(qq: QuantizedTokens, kq: QuantizedTokens, v: torch.Tensor
     return tuple(_lib.host().attn_bwd(qq, kq, v, o, do, lse, bool(causal), float(sm_scale)))
 
 
-# Longest query block the shared-KV kernels are used for.  They stream the codes once per 16 queries
-# (from L2 after the first block), which wins while Nq is small against Nk -- the reference's test and
-# benchmark shapes; measured crossover with the INT8-score kernels at Nk=4096, D=128: between 512 and
-# 1024 queries (fwd 1.16 vs 1.51 ms at 512, 1.14 vs 1.01 ms at 1024).
+# Longest query block the shared-KV kernels are used for: they keep Q in 16 bits, and beat the INT8-score kernels while Nq is
+# small against Nk -- the reference's test and benchmark shapes; crossover at Nk=4096, D=128 when the line was drawn: between
+# 512 and 1024 queries (fwd 1.16 vs 1.51 ms at 512, 1.14 vs 1.01 ms at 1024; the tiled kernels have made the shared-KV side
+# 1.8 times faster since, and the line stays because the two sides round differently).
 SHARED_KV_MAX_Q = 512
 # head_dim 256 (compute_flops.py:94): the INT8-score kernels run one wave per SIMD there and the crossover moves up
 # (Nk=4096: fwd+bwd 5.9 vs 4.5 ms at 512 queries, 9.0 vs 8.9 at 1024; Nq=Nk=2048: 3.9 vs 4.9 ms, INT8-score first).
@@ -73,7 +73,8 @@ def attn_bwd_shared_kv(q: torch.Tensor, codes: torch.Tensor, scale: torch.Tensor
     [B,H,Nq,D] (the kernels compute in binary16); lse as returned by the forward.  dQ and dKV come back
     in `grad_dtype` (fp16 by default, or bf16), multiplied by the one-element device tensor `grad_scale`
     if given.  Up to 32 queries (16 at head_dim 256) run in one fused pass over the codes, longer blocks
-    in a dQ kernel plus a dKV kernel."""
+    in a dQ kernel plus a dKV kernel.  The keys are not split over workgroups here (`quant_flash_attn`'s backward does where
+    there are few heads)."""
     return _lib.host().skv_bwd(q, codes, scale, zero_point, o, do, lse, float(sm_scale), grad_dtype or torch.float16,
                                grad_scale)
 

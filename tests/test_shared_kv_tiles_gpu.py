@@ -1,0 +1,109 @@
+"""The shared-KV kernels that expand a tile of keys once per workgroup (forward, dQ), the dKV kernel with resident rows, and
+the backward with its keys split over workgroups, at the sizes where they can go wrong: one key, tiles and blocks of 32, 64
+and 128 with one more or one less, two and four waves side by side, one wave without queries, and few heads (splits).
+Many heads make the dispatch take these kernels at small sizes; the first, a middle and the last head are compared with the
+oracle, with the tolerances of helpers.py."""
+import math
+import random
+
+import pytest
+import torch
+
+from helpers import COS_TOL, assert_close, max_abs
+from oracle import oracle
+
+DEV = "cuda:0"
+
+CASES = [
+    # heads, Nq, Nk, dtype, scale dtype
+    (512, 33, 1, torch.float16, torch.float16),      # one key
+    (512, 65, 31, torch.float16, torch.float32),     # three blocks on four waves, one key less than a block
+    (300, 200, 33, torch.bfloat16, torch.float16),   # two workgroups per head, four and three blocks
+    (256, 97, 65, torch.float16, torch.float16),     # one key more than a tile; resident rows, the last block one query
+    (256, 128, 129, torch.float16, torch.float16),   # all resident rows, one key more than four waves' tiles
+    (256, 129, 128, torch.bfloat16, torch.float32),  # one query more than the resident rows
+    (64, 512, 97, torch.float16, torch.float16),
+    (600, 64, 70, torch.float16, torch.bfloat16),
+    (600, 32, 70, torch.float16, torch.float16),     # one-pass backward, not split
+    (3, 16, 3001, torch.float16, torch.float16),     # one-pass backward, split
+    (2, 31, 2500, torch.bfloat16, torch.float32),
+    (1, 200, 9001, torch.float16, torch.float16),    # forward and dQ split
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("BH,Nq,Nk,dtype,sdtype", CASES)
+def test_tiles_vs_oracle(qfa, BH, Nq, Nk, dtype, sdtype, D):
+    g = torch.Generator().manual_seed(BH + Nq + Nk + D)
+    kv = (torch.randn((1, BH, Nk, D), generator=g) + 0.3 * torch.randn((1, BH, Nk, 1), generator=g)).to(dtype)
+    q, do = (torch.randn((1, BH, Nq, D), generator=g).to(dtype) for _ in range(2))
+    sm = 1.0 / math.sqrt(D)
+    qd, kvd = q.to(DEV).requires_grad_(True), kv.to(DEV).requires_grad_(True)
+    codes, scale, zp = qfa.asymmetric_quant_per_token(kvd.detach(), scale_dtype=sdtype)
+    o = qfa.quant_flash_attn(qd, kvd, (codes, scale, zp), sm)
+    dq, dkv = torch.autograd.grad(o, [qd, kvd], do.to(DEV))
+    o2, lse = qfa.attn_fwd_shared_kv(qd.detach(), codes, scale, zp, sm)
+    torch.cuda.synchronize()
+    assert torch.equal(o, o2)
+    pick = sorted({0, BH // 2, BH - 1})
+    q, do, codes, scale, zp, o, lse, dq, dkv = (t.detach()[:, pick].cpu() for t in (q, do, codes, scale, zp, o, lse, dq, dkv))
+    o_ref, lse_ref = oracle.legacy_fwd(q, codes, scale, zp, sm)
+    assert_close("O", o, o_ref, scaled=True)
+    assert max_abs(lse, lse_ref) < 2.0 ** -8
+    (dq_ref, dkv_ref), (nq, nkv) = oracle.legacy_bwd(q, codes, scale, zp, do, sm, o=o, spread=True)
+    assert_close("dQ", dq, dq_ref, scaled=True, spread=nq, cos_tol=COS_TOL if Nk > 1 else -1.0)   # one key: dQ is zero
+    assert_close("dKV", dkv, dkv_ref, scaled=True, spread=nkv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_infinite_rows_stay_with_their_queries(qfa, D):
+    """An infinite query or dO row reaches O and dQ of its own query only.  The others may be taken against another reference
+    maximum (a wave moves its queries' references together), which rounds their probabilities differently: 2^-11 each, so
+    2^-9 of the largest value bounds what two roundings of a weighted sum and of the result can move."""
+    BH, Nq, Nk = 512, 65, 70
+    g = torch.Generator().manual_seed(D)
+    kv, q, do = (torch.randn(s, generator=g).to(torch.float16).to(DEV) for s in ((1, BH, Nk, D), (1, BH, Nq, D), (1, BH, Nq, D)))
+    codes, scale, zp = qfa.asymmetric_quant_per_token(kv)
+    sm = 1.0 / math.sqrt(D)
+
+    def run(q, do):
+        o, lse = qfa.attn_fwd_shared_kv(q, codes, scale, zp, sm)
+        return o, qfa.attn_bwd_shared_kv(q, codes, scale, zp, o, do, lse, sm)[0]
+    want = run(q, do)
+    q2, do2 = q.clone(), do.clone()
+    q2[:, :, 40, 3] = float("inf")
+    do2[:, :, 7] = float("inf")
+    got = run(q2, do2)
+    keep = [i for i in range(Nq) if i not in (7, 40)]
+    for a, b in zip(got, want):
+        a, b = a[:, :, keep].float(), b[:, :, keep].float()
+        assert torch.isfinite(a).all()
+        assert float((a - b).abs().max()) <= 2.0 ** -9 * float(b.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sm", [1e-25, 1e-3, 30.0])
+def test_softmax_scales(qfa, sm):
+    """The forward multiplies the key scales by sm_scale: O and LSE at scales far from 1/sqrt(D)."""
+    BH, Nq, Nk, D = 512, 65, 130, 128
+    g = torch.Generator().manual_seed(3)
+    kv, q = (torch.randn(s, generator=g).to(torch.float16) for s in ((1, BH, Nk, D), (1, BH, Nq, D)))
+    codes, scale, zp = qfa.asymmetric_quant_per_token(kv.to(DEV))
+    o, lse = (t[:, :2].cpu() for t in qfa.attn_fwd_shared_kv(q.to(DEV), codes, scale, zp, sm))
+    o_ref, lse_ref = oracle.legacy_fwd(q[:, :2], *(t[:, :2].cpu() for t in (codes, scale, zp)), sm)
+    assert_close("O", o, o_ref, scaled=True)
+    # scores reach 30 * 60: binary32 of the exponent in log2 units loses 2^-24 of that per operation
+    assert max_abs(lse, lse_ref) < 2.0 ** -8 * max(1.0, float(lse_ref.abs().max()) * 2.0 ** -8)
+
+
+def test_backward_workspace_is_bounded(qfa):
+    """Partial results of a split stay within 64 MiB, and a chip that is full is not split (head_dim up to 128)."""
+    from quant_flash_attn_amd import _lib
+    L, rng = _lib.lib(), random.Random(2)
+    for _ in range(20000):
+        B, H, Nq, Nk = rng.randint(1, 64), rng.randint(1, 64), rng.choice((1, 16, 17, 32, 33, 512, 2000)), rng.randint(1, 40000)
+        for D in (64, 128, 256):
+            assert 0 <= L.qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) <= (64 << 20)
+    assert L.qfa_attn_bwd_shared_kv_workspace_bytes(512, 16, 16, 3000, 128) == 0
