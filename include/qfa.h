@@ -81,6 +81,16 @@ int qfa_quant_per_token_pair(const void *x0, const void *x1, int x_dtype, int8_t
                              int64_t sc0n, int64_t sc1b, int64_t sc1h, int64_t sc1n, void *stream);
 
 /*
+ * qfa_quant_per_token_pair for fp32 queries and keys (D in {64, 128, 256}), with the values of the same attention call converted
+ * to bf16 in the same launch: v fp32 [B,H,N1,D] with strides sv?, v_bf16 dense.
+ */
+int qfa_quant_qkv_f32(const float *q, const float *k, const float *v, int8_t *codes0, int8_t *codes1, float *scale0, float *scale1,
+                      int8_t *zp0, int8_t *zp1, int32_t *rowsum0, int32_t *rowsum1, void *v_bf16, int64_t B, int64_t H, int64_t N0,
+                      int64_t N1, int D, int64_t sx0b, int64_t sx0h, int64_t sx0n, int64_t sx1b, int64_t sx1h, int64_t sx1n,
+                      int64_t svb, int64_t svh, int64_t svn, int64_t sc0b, int64_t sc0h, int64_t sc0n, int64_t sc1b, int64_t sc1h,
+                      int64_t sc1n, void *stream);
+
+/*
  * out = (codes - zp) * scale, per token (asymmetric_quant.py:158-160, and the in-kernel
  * dequantization quant_flash_attn.py:65).  scale_dtype is the element type of `scale`
  * (QFA_F32 / QFA_F16 / QFA_BF16); out has out_dtype and strides sob,soh,son.
@@ -118,6 +128,15 @@ int qfa_code_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, 
  */
 int qfa_attn_fwd(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
                  const float *sk, const int8_t *zk, const int32_t *rk, const void *v, void *o, float *lse,
+                 int io_dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh,
+                 int64_t sqn, int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn,
+                 int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *stream);
+
+/*
+ * The same with O in fp32 as well: o32 [B,H,Nq,D] dense, unrounded; o (the 16-bit one that a backward takes) may be NULL.
+ */
+int qfa_attn_fwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, float *o32, void *o, float *lse,
                  int io_dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh,
                  int64_t sqn, int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn,
                  int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *stream);
@@ -314,6 +333,22 @@ int qfa_attn_bwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
                  const float *sk, const int8_t *zk, const int32_t *rk, const void *v, const void *o,
                  const void *dout, const float *lse, void *workspace, int64_t workspace_bytes, void *dq, void *dk,
                  void *dv, int io_dtype,
+                 int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                 int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, int64_t sob,
+                 int64_t soh, int64_t son, int64_t sdob, int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh,
+                 int64_t sdqn, int64_t sdkb, int64_t sdkh, int64_t sdkn, int64_t sdvb, int64_t sdvh,
+                 int64_t sdvn, float sm_scale, int causal, void *stream);
+
+/*
+ * The same with fp32 dout, dq, dk and dv (strides in elements of those, multiples of 16 bytes): the staging pass rounds dout to
+ * io_dtype on its way, and the gradients leave unrounded.  The workspace holds the rounded dout too.
+ */
+int64_t qfa_attn_bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
+
+int qfa_attn_bwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, const void *o,
+                 const float *dout, const float *lse, void *workspace, int64_t workspace_bytes, float *dq, float *dk,
+                 float *dv, int io_dtype,
                  int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
                  int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, int64_t sob,
                  int64_t soh, int64_t son, int64_t sdob, int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh,

@@ -28,9 +28,11 @@ _SIGNATURES = {
     "qfa_last_error": (ctypes.c_char_p, []),
     "qfa_quant_per_token": (c_int, [_P, _I, _P, _P, _P, _I, _P, _P, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_quant_per_token_pair": (c_int, [_P, _P, _I] + [_P] * 8 + [_L, _L, _L, _L, _I] + [_L] * 12 + [_P]),
+    "qfa_quant_qkv_f32": (c_int, [_P] * 12 + [_L, _L, _L, _L, _I] + [_L] * 15 + [_P]),
     "qfa_dequant_per_token": (c_int, [_P, _P, _I, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_code_rowsum": (c_int, [_P, _P, _L, _L, _L, _I, _L, _L, _L, _P]),
     "qfa_attn_fwd": (c_int, [_P] * 11 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P]),
+    "qfa_attn_fwd_f32": (c_int, [_P] * 12 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P]),
     "qfa_attn_fwd_shared_kv_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
     "qfa_attn_fwd_shared_kv": (c_int, [_P, _P, _P, _I, _P, _P, _P, _I, _L, _L, _L, _L, _I] + [_L] * 9 + [_F, _P, _L, _P]),
     "qfa_attn_fwd_shared_kv_static": (c_int, [_P, _P, _P, _I, _P, _P, _P, _I, _L, _L, _L, _L, _I] + [_L] * 9 + [_F, _P]),
@@ -47,6 +49,8 @@ _SIGNATURES = {
     "qfa_dout_normalise": (c_int, [_P, _I, _L, _P, _I, _L, _P, _P, _P, _P]),
     "qfa_bwd_delta": (c_int, [_P, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_attn_bwd_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
+    "qfa_attn_bwd_f32_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
+    "qfa_attn_bwd_f32": (c_int, [_P] * 13 + [_L] + [_P] * 3 + [_I, _L, _L, _L, _L, _I] + [_L] * 24 + [_F, _I, _P]),
     "qfa_attn_bwd": (c_int, [_P] * 13 + [_L] + [_P] * 3 + [_I, _L, _L, _L, _L, _I] + [_L] * 24 + [_F, _I, _P]),
 }
 

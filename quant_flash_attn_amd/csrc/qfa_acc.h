@@ -143,6 +143,16 @@ __device__ __forceinline__ void acc_store_rows_seq(std::integer_sequence<int, DB
   store_tile_rows<T, D>(acc, scale, stage, rows, stride, row0, nrows, lane);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the stage may be written again
 }
+template <int D, int T0, int... DB>
+__device__ __forceinline__ void acc_store_rows_f32_seq(std::integer_sequence<int, DB...>, float scale, float *rows, int64_t stride,
+                                                       int row0, int nrows, int lane) {
+  const f32x16 acc[sizeof...(DB)] = {acc_read<T0 + DB>()...};
+  store_tile_rows_f32<D>(acc, scale, rows, stride, row0, nrows, lane);
+}
+template <int D, int T0>
+__device__ __forceinline__ void acc_store_rows_f32(float scale, float *rows, int64_t stride, int row0, int nrows, int lane) {
+  acc_store_rows_f32_seq<D, T0>(std::make_integer_sequence<int, D / 32>{}, scale, rows, stride, row0, nrows, lane);
+}
 template <typename T, int D, int T0>
 __device__ __forceinline__ void acc_store_rows(float scale, unsigned char *stage, T *rows, int64_t stride, int row0, int nrows,
                                                int lane) {

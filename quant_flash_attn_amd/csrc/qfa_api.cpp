@@ -95,6 +95,34 @@ int qfa_quant_per_token_pair(const void *x0, const void *x1, int x_dtype, int8_t
   return launch_quant_pair(x, x_dtype, codes, scale, zp, rowsum, B, H, N, D, sx, sc, (hipStream_t)stream);
 }
 
+int qfa_quant_qkv_f32(const float *q, const float *k, const float *v, int8_t *codes0, int8_t *codes1, float *scale0, float *scale1,
+                      int8_t *zp0, int8_t *zp1, int32_t *rowsum0, int32_t *rowsum1, void *v_bf16, int64_t B, int64_t H, int64_t N0,
+                      int64_t N1, int D, int64_t sx0b, int64_t sx0h, int64_t sx0n, int64_t sx1b, int64_t sx1h, int64_t sx1n,
+                      int64_t svb, int64_t svh, int64_t svn, int64_t sc0b, int64_t sc0h, int64_t sc0n, int64_t sc1b, int64_t sc1h,
+                      int64_t sc1n, void *stream) {
+  const float *const x[2] = {q, k};
+  int8_t *const codes[2] = {codes0, codes1};
+  float *const scale[2] = {scale0, scale1};
+  int8_t *const zp[2] = {zp0, zp1};
+  int32_t *const rowsum[2] = {rowsum0, rowsum1};
+  const int64_t N[2] = {N0, N1}, sv[3] = {svb, svh, svn};
+  const int64_t sx[2][3] = {{sx0b, sx0h, sx0n}, {sx1b, sx1h, sx1n}}, sc[2][3] = {{sc0b, sc0h, sc0n}, {sc1b, sc1h, sc1n}};
+  if (B <= 0 || H <= 0 || N0 <= 0 || N1 <= 0) return set_error(QFA_EINVAL, "quant_qkv: B, H, N0, N1 must be positive");
+  if (D != 64 && D != 128 && D != 256) return set_error(QFA_EUNSUPPORTED, "quant_qkv: head_dim %d not in {64, 128, 256}", D);
+  if (!v || !v_bf16) return set_error(QFA_EINVAL, "quant_qkv: null pointer argument");
+  if (!aligned16(v) || !aligned16(v_bf16) || !strides_ok(svb, svh, svn, D, 4))
+    return set_error(QFA_EINVAL, "quant_qkv: v must be 16-byte aligned, its strides positive multiples of 16 bytes, token stride >= D");
+  for (int i = 0; i < 2; ++i) {
+    if (!x[i] || !codes[i] || !scale[i] || !zp[i]) return set_error(QFA_EINVAL, "quant_qkv: null pointer argument");
+    if (!aligned16(x[i]) || !aligned8(codes[i])) return set_error(QFA_EINVAL, "quant_qkv: q and k must be 16-byte, codes 8-byte aligned");
+    if (!strides_ok(sx[i][0], sx[i][1], sx[i][2], D, 4))
+      return set_error(QFA_EINVAL, "quant_qkv: strides must be positive multiples of 16 bytes, token stride >= D");
+    if (sc[i][0] <= 0 || sc[i][1] <= 0 || sc[i][2] < D || sc[i][0] % 8 != 0 || sc[i][1] % 8 != 0 || sc[i][2] % 8 != 0)
+      return set_error(QFA_EINVAL, "quant_qkv: codes strides must be positive multiples of 8 bytes, token stride >= D");
+  }
+  return launch_quant_qkv(x, codes, scale, zp, rowsum, v, v_bf16, B, H, N, D, sx, sc, sv, (hipStream_t)stream);
+}
+
 int qfa_dequant_per_token(const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp, void *out,
                           int out_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t scb, int64_t sch,
                           int64_t scn, int64_t sob, int64_t soh, int64_t son, void *stream) {
@@ -125,7 +153,7 @@ int qfa_code_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, 
 }
 
 static int check_attn_common(const char *who, const AttnArgs &a) {
-  if (!a.qc || !a.sq || !a.zq || !a.rq || !a.kc || !a.sk || !a.zk || !a.rk || !a.v || !a.o || !a.lse)
+  if (!a.qc || !a.sq || !a.zq || !a.rq || !a.kc || !a.sk || !a.zk || !a.rk || !a.v || (!a.o && !a.o32) || !a.lse)
     return set_error(QFA_EINVAL, "%s: null pointer argument", who);
   if (a.io_dtype != QFA_BF16 && a.io_dtype != QFA_F16)
     return set_error(QFA_EINVAL, "%s: io_dtype must be QFA_BF16 or QFA_F16", who);
@@ -139,10 +167,10 @@ static int check_attn_common(const char *who, const AttnArgs &a) {
     return set_error(QFA_EINVAL, "%s: sm_scale must be a positive finite number", who);
   if (a.causal && a.Nq > a.Nk)
     return set_error(QFA_EUNSUPPORTED, "%s: causal needs Nq <= Nk (the mask is aligned to the last key)", who);
-  if (!aligned16(a.qc) || !aligned16(a.kc) || !aligned16(a.v) || !aligned16(a.o))
+  if (!aligned16(a.qc) || !aligned16(a.kc) || !aligned16(a.v) || !aligned16(a.o) || !aligned16(a.o32))
     return set_error(QFA_EINVAL, "%s: qc, kc, v, o must be 16-byte aligned", who);
   if (!strides_ok(a.sqb, a.sqh, a.sqn, a.D, 1) || !strides_ok(a.skb, a.skh, a.skn, a.D, 1) ||
-      !strides_ok(a.svb, a.svh, a.svn, a.D, 2) || !strides_ok(a.sob, a.soh, a.son, a.D, 2))
+      !strides_ok(a.svb, a.svh, a.svn, a.D, 2) || (a.o && !strides_ok(a.sob, a.soh, a.son, a.D, 2)))
     return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
   // offsets inside a 64-token tile are formed in 31 bits
   if (a.skn >= (1 << 23) || a.svn >= (1 << 23) || a.sqn >= (1 << 23))
@@ -164,6 +192,24 @@ int qfa_attn_fwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
   a.svb = svb; a.svh = svh; a.svn = svn; a.sob = sob; a.soh = soh; a.son = son;
   a.sm_scale = sm_scale; a.causal = causal;
   if (int e = check_attn_common("attn_fwd", a)) return e;
+  return launch_fwd(a, (hipStream_t)stream);
+}
+
+int qfa_attn_fwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, float *o32, void *o, float *lse,
+                 int io_dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh,
+                 int64_t sqn, int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn,
+                 int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *stream) {
+  AttnArgs a;
+  memset(&a, 0, sizeof(a));
+  a.qc = qc; a.sq = sq; a.zq = zq; a.rq = rq; a.kc = kc; a.sk = sk; a.zk = zk; a.rk = rk;
+  a.v = v; a.o = o; a.o32 = o32; a.lse = lse; a.io_dtype = io_dtype;
+  a.B = B; a.H = H; a.Nq = Nq; a.Nk = Nk; a.D = D;
+  a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.skb = skb; a.skh = skh; a.skn = skn;
+  a.svb = svb; a.svh = svh; a.svn = svn; a.sob = sob; a.soh = soh; a.son = son;
+  a.sm_scale = sm_scale; a.causal = causal;
+  if (!o32) return set_error(QFA_EINVAL, "attn_fwd_f32: null pointer argument");
+  if (int e = check_attn_common("attn_fwd_f32", a)) return e;
   return launch_fwd(a, (hipStream_t)stream);
 }
 
@@ -393,7 +439,7 @@ int64_t qfa_attn_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t N
   return bwd_workspace_bytes(B, H, Nq, Nk, D);
 }
 
-int qfa_attn_bwd(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+static int attn_bwd(const char *who, int f32, const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
                  const float *sk, const int8_t *zk, const int32_t *rk, const void *v, const void *o,
                  const void *dout, const float *lse, void *workspace, int64_t workspace_bytes, void *dq, void *dk,
                  void *dv, int io_dtype,
@@ -412,19 +458,53 @@ int qfa_attn_bwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
   a.svb = svb; a.svh = svh; a.svn = svn; a.sob = sob; a.soh = soh; a.son = son;
   a.sdob = sdob; a.sdoh = sdoh; a.sdon = sdon; a.sdqb = sdqb; a.sdqh = sdqh; a.sdqn = sdqn;
   a.sdkb = sdkb; a.sdkh = sdkh; a.sdkn = sdkn; a.sdvb = sdvb; a.sdvh = sdvh; a.sdvn = sdvn;
-  a.sm_scale = sm_scale; a.causal = causal;
-  if (int e = check_attn_common("attn_bwd", a)) return e;
-  if (!dout || !workspace || !dq || !dk || !dv) return set_error(QFA_EINVAL, "attn_bwd: null pointer argument");
+  a.sm_scale = sm_scale; a.causal = causal; a.f32 = f32;
+  if (int e = check_attn_common(who, a)) return e;
+  if (!dout || !workspace || !dq || !dk || !dv) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
   if (!aligned16(dout) || !aligned16(dq) || !aligned16(dk) || !aligned16(dv) || !aligned16(workspace))
-    return set_error(QFA_EINVAL, "attn_bwd: dout, dq, dk, dv, workspace must be 16-byte aligned");
-  const int64_t need = bwd_workspace_bytes(B, H, Nq, Nk, D);
+    return set_error(QFA_EINVAL, "%s: dout, dq, dk, dv, workspace must be 16-byte aligned", who);
+  const int64_t need = f32 ? bwd_f32_workspace_bytes(B, H, Nq, Nk, D) : bwd_workspace_bytes(B, H, Nq, Nk, D);
+  const int es = f32 ? 4 : 2;
   if (workspace_bytes < need)
-    return set_error(QFA_EINVAL, "attn_bwd: workspace of %lld bytes is too small, need %lld (qfa_attn_bwd_workspace_bytes)",
-                     (long long)workspace_bytes, (long long)need);
-  if (!strides_ok(sdob, sdoh, sdon, D, 2) || !strides_ok(sdqb, sdqh, sdqn, D, 2) ||
-      !strides_ok(sdkb, sdkh, sdkn, D, 2) || !strides_ok(sdvb, sdvh, sdvn, D, 2))
-    return set_error(QFA_EINVAL, "attn_bwd: strides must be positive multiples of 16 bytes, token stride >= D");
+    return set_error(QFA_EINVAL, "%s: workspace of %lld bytes is too small, need %lld (qfa_attn_bwd%s_workspace_bytes)", who,
+                     (long long)workspace_bytes, (long long)need, f32 ? "_f32" : "");
+  if (!strides_ok(sdob, sdoh, sdon, D, es) || !strides_ok(sdqb, sdqh, sdqn, D, es) ||
+      !strides_ok(sdkb, sdkh, sdkn, D, es) || !strides_ok(sdvb, sdvh, sdvn, D, es))
+    return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
   return launch_bwd(a, (hipStream_t)stream);
+}
+
+int qfa_attn_bwd(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, const void *o,
+                 const void *dout, const float *lse, void *workspace, int64_t workspace_bytes, void *dq, void *dk,
+                 void *dv, int io_dtype,
+                 int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                 int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, int64_t sob,
+                 int64_t soh, int64_t son, int64_t sdob, int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh,
+                 int64_t sdqn, int64_t sdkb, int64_t sdkh, int64_t sdkn, int64_t sdvb, int64_t sdvh,
+                 int64_t sdvn, float sm_scale, int causal, void *stream) {
+  return attn_bwd("attn_bwd", 0, qc, sq, zq, rq, kc, sk, zk, rk, v, o, dout, lse, workspace, workspace_bytes, dq, dk, dv, io_dtype, B, H, Nq, Nk, D, sqb, sqh, sqn,
+                  skb, skh, skn, svb, svh, svn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn, sdvb, sdvh, sdvn,
+                  sm_scale, causal, stream);
+}
+
+int64_t qfa_attn_bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0 || (D != 64 && D != 128 && D != 256)) return 0;
+  return bwd_f32_workspace_bytes(B, H, Nq, Nk, D);
+}
+
+int qfa_attn_bwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, const void *o,
+                 const float *dout, const float *lse, void *workspace, int64_t workspace_bytes, float *dq, float *dk,
+                 float *dv, int io_dtype,
+                 int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                 int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, int64_t sob,
+                 int64_t soh, int64_t son, int64_t sdob, int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh,
+                 int64_t sdqn, int64_t sdkb, int64_t sdkh, int64_t sdkn, int64_t sdvb, int64_t sdvh,
+                 int64_t sdvn, float sm_scale, int causal, void *stream) {
+  return attn_bwd("attn_bwd_f32", 1, qc, sq, zq, rq, kc, sk, zk, rk, v, o, dout, lse, workspace, workspace_bytes, dq, dk, dv, io_dtype, B, H, Nq, Nk, D, sqb, sqh, sqn,
+                  skb, skh, skn, svb, svh, svn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn, sdvb, sdvh, sdvn,
+                  sm_scale, causal, stream);
 }
 
 }  // extern "C"

@@ -167,7 +167,15 @@ template <typename T, int D> __device__ __forceinline__ void prep_q(const BwdArg
     for (int r = 0; r < 4; ++r) {
       const int i = min(i0 + 4 * r4 + r, a.Nq - 1);
       creg[r] = *reinterpret_cast<const u32x2 *>(qc_bh + (int64_t)i * a.sqn + dc * 8);
-      const u32x4 gw = *reinterpret_cast<const u32x4 *>(do_bh + (int64_t)i * a.sdon + dc * 8);
+      u32x4 gw;
+      if (a.dout32) {
+        const f32x4 *g32 = reinterpret_cast<const f32x4 *>(a.dout32 + b * a.sd32b + h * a.sd32h + (int64_t)i * a.sd32n + dc * 8);
+        const f32x4 x = g32[0], y = g32[1];
+        gw = u32x4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
+        if (i0 + 4 * r4 + r < a.Nq) *reinterpret_cast<u32x4 *>(reinterpret_cast<T *>(a.do16) + (tq0 + i) * D + dc * 8) = gw;
+      } else {
+        gw = *reinterpret_cast<const u32x4 *>(do_bh + (int64_t)i * a.sdon + dc * 8);
+      }
       const u32x4 ow = *reinterpret_cast<const u32x4 *>(o_bh + (int64_t)i * a.son + dc * 8);
       zreg[r] = (float)a.zq[tq0 + i];
       sreg[r] = a.sq[tq0 + i];
@@ -268,6 +276,14 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
   a.sm_scale = x.sm_scale; a.sm_scale_log2 = x.sm_scale * kLog2e;
   a.nblocks = 0; a.total_blocks = 0; a.blocks_per_xcd = 0; a.group_log2 = 0;
   const int64_t BH = x.B * x.H;
+  a.dout32 = nullptr; a.do16 = nullptr; a.sd32b = a.sd32h = a.sd32n = 0;
+  a.grad_f32 = x.f32;
+  if (x.f32) {   // dO and the gradients in fp32: the 16-bit dO lies behind the staged tiles
+    a.dout32 = static_cast<const float *>(x.dout);
+    a.sd32b = x.sdob; a.sd32h = x.sdoh; a.sd32n = x.sdon;
+    a.dout = a.do16 = a.ws_k + BH * (int64_t)a.tiles_k * WS::K_BLOB;
+    a.sdob = x.H * x.Nq * D; a.sdoh = x.Nq * D; a.sdon = D;
+  }
   if (BH * (a.tiles_q + a.tiles_k) > 0x7fffffffLL)
     return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many tiles for one launch");
   bwd_prep_kernel<T, D><<<dim3((unsigned)(BH * (a.tiles_q + a.tiles_k))), dim3(256), 0, st>>>(a, (int)(BH * a.tiles_q));

@@ -34,6 +34,10 @@ struct BwdArgs {
   float sm_scale, sm_scale_log2;
   int nblocks;          // query blocks (dq) or key blocks (dkdv) per (b,h)
   int total_blocks, blocks_per_xcd;
+  const float *dout32;  // nullable: dO in fp32; the staging pass then writes the 16-bit one to do16, which is `dout`
+  void *do16;
+  int64_t sd32b, sd32h, sd32n;
+  int grad_f32;         // dQ, dK, dV are fp32
   int group_log2;       // causal: log2 of the number of heads whose blocks are dispatched together (set per launch)
 };
 

@@ -413,8 +413,17 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
   __syncthreads();   // the tile buffers are done with: the output stages overlay them
   static_assert(4 * 32 * 2 * D <= 3 * SM::BUF, "output staging fits the tile buffers");
   unsigned char *stage = smem + wave * (32 * 2 * D);
-  T *dk_bh = reinterpret_cast<T *>(a.dk) + b * a.sdkb + h * a.sdkh;
-  T *dv_bh = reinterpret_cast<T *>(a.dv) + b * a.sdvb + h * a.sdvh;
+  const int64_t dk_at = b * a.sdkb + h * a.sdkh, dv_at = b * a.sdvb + h * a.sdvh;
+  if (a.grad_f32) {
+    float *dk_bh = reinterpret_cast<float *>(a.dk) + dk_at, *dv_bh = reinterpret_cast<float *>(a.dv) + dv_at;
+    static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
+      constexpr int kb = decltype(kb_tag)::value;
+      acc_store_rows_f32<D, kb * DB>(a.sm_scale, dk_bh, a.sdkn, k_first + 32 * kb, a.Nk, lane);
+      acc_store_rows_f32<D, DV0 + kb * DB>(1.0f, dv_bh, a.sdvn, k_first + 32 * kb, a.Nk, lane);
+    });
+    return;
+  }
+  T *dk_bh = reinterpret_cast<T *>(a.dk) + dk_at, *dv_bh = reinterpret_cast<T *>(a.dv) + dv_at;
   static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
     constexpr int kb = decltype(kb_tag)::value;
     acc_store_rows<T, D, kb * DB>(a.sm_scale, stage, dk_bh, a.sdkn, k_first + 32 * kb, a.Nk, lane);

@@ -338,6 +338,14 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   __syncthreads();   // the tile buffers are done with: the output stages overlay them
   static_assert(4 * 32 * 2 * D <= 3 * SM::BUF, "output staging fits the tile buffers");
   unsigned char *stage = smem + wave * (32 * 2 * D);
+  if (a.grad_f32) {
+    float *dq_bh = reinterpret_cast<float *>(a.dq) + b * a.sdqb + h * a.sdqh;
+    static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
+      constexpr int qb = decltype(qb_tag)::value;
+      acc_store_rows_f32<D, qb * DB>(a.sm_scale, dq_bh, a.sdqn, q_first + 32 * qb, a.Nq, lane);
+    });
+    return;
+  }
   T *dq_bh = reinterpret_cast<T *>(a.dq) + b * a.sdqb + h * a.sdqh;
   static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
     constexpr int qb = decltype(qb_tag)::value;

@@ -329,6 +329,22 @@ __device__ __forceinline__ void store_tile_rows(const f32x16 (&acc)[D / 32], flo
   }
 }
 
+// The same tile to fp32 rows, straight from the registers: 16 bytes per lane
+template <int D>
+__device__ __forceinline__ void store_tile_rows_f32(const f32x16 (&acc)[D / 32], float scale, float *base, int64_t row_stride,
+                                                    int row0, int nrows, int lane) {
+  asm volatile("" : "+v"(lane));
+  const int lr = lane % 32, g = lane / 32;
+  if (row0 + lr >= nrows) return;
+  float *row = base + (int64_t)(row0 + lr) * row_stride + 4 * g;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int aa = 0; aa < 4; ++aa)
+      *reinterpret_cast<f32x4 *>(row + 32 * db + 8 * aa) =
+          f32x4{acc[db][4 * aa] * scale, acc[db][4 * aa + 1] * scale, acc[db][4 * aa + 2] * scale, acc[db][4 * aa + 3] * scale};
+}
+
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every outstanding
 // global access, including direct-to-LDS loads issued for a LATER tile, which would serialise the
 // prefetch; this one leaves them in flight (pair it with dma_wait() where a tile must have landed).

@@ -699,7 +699,8 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   // O leaves as whole rows through LDS (all tile buffers are free after the last barrier; every wave takes 32 * 2D
   // bytes at the start of the K area)
   static_assert(SM::OFF_K + FWD_WAVES * 32 * 2 * D <= SM::TOTAL, "output staging fits the tile buffers");
-  store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), o_bh, a.son, m0 + wave * 32, a.Nq, lane);
+  if (a.o32) store_tile_rows_f32<D>(oacc, inv, a.o32 + tq0 * D, D, m0 + wave * 32, a.Nq, lane);
+  if (a.o) store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), o_bh, a.son, m0 + wave * 32, a.Nq, lane);
   if (qi < a.Nq && g == 0) a.lse[tq0 + qi] = (a_i * m_ref + __log2f(l_tot)) * kLn2;
 }
 
@@ -707,7 +708,7 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
   FwdArgs a;
   a.qc = x.qc; a.sq = x.sq; a.zq = x.zq; a.rq = x.rq;
   a.kc = x.kc; a.sk = x.sk; a.zk = x.zk; a.rk = x.rk;
-  a.v = x.v; a.o = x.o; a.lse = x.lse;
+  a.v = x.v; a.o = x.o; a.lse = x.lse; a.o32 = x.o32;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk;
   a.sqb = x.sqb; a.sqh = x.sqh; a.sqn = x.sqn; a.skb = x.skb; a.skh = x.skh; a.skn = x.skn;
   a.svb = x.svb; a.svh = x.svh; a.svn = x.svn; a.sob = x.sob; a.soh = x.soh; a.son = x.son;

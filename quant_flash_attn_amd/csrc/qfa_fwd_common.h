@@ -9,6 +9,7 @@ struct FwdArgs {
   const int8_t *qc; const float *sq; const int8_t *zq; const int32_t *rq;
   const int8_t *kc; const float *sk; const int8_t *zk; const int32_t *rk;
   const void *v; void *o; float *lse;
+  float *o32;            // nullable: O in fp32, dense; then o is nullable too
   int64_t H;
   int Nq, Nk;
   int64_t sqb, sqh, sqn, skb, skh, skn, svb, svh, svn, sob, soh, son;

@@ -398,7 +398,8 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
     constexpr int qb = decltype(qb_tag)::value;
     const float l_tot = l_run[qb] + swap32_f(l_run[qb]);
-    acc_store_rows<T, D, qb * DB>(1.0f / l_tot, stage, o_bh, a.son, q_first + 32 * qb, a.Nq, lane);
+    if (a.o32) acc_store_rows_f32<D, qb * DB>(1.0f / l_tot, a.o32 + tq0 * D, D, q_first + 32 * qb, a.Nq, lane);
+    if (a.o) acc_store_rows<T, D, qb * DB>(1.0f / l_tot, stage, o_bh, a.son, q_first + 32 * qb, a.Nq, lane);
     const int qi = q_first + 32 * qb + lr;
     if (qi < a.Nq && g == 0) a.lse[tq0 + qi] = (a_i[qb] * m_ref[qb] + __log2f(l_tot)) * kLn2;
   });

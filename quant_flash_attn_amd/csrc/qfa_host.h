@@ -20,6 +20,10 @@ int launch_quant(const void *x, int x_dtype, int8_t *codes, float *scale, void *
 int launch_quant_pair(const void *const x[2], int x_dtype, int8_t *const codes[2], float *const scale[2],
                       int8_t *const zp[2], int32_t *const rowsum[2], int64_t B, int64_t H, const int64_t N[2], int D,
                       const int64_t sx[2][3], const int64_t sc[2][3], hipStream_t st);
+// fp32 queries and keys quantized, fp32 values converted to bf16 (dense), in one launch; head_dim 64, 128 or 256
+int launch_quant_qkv(const float *const x[2], int8_t *const codes[2], float *const scale[2], int8_t *const zp[2],
+                     int32_t *const rowsum[2], const float *v, void *v16, int64_t B, int64_t H, const int64_t N[2], int D,
+                     const int64_t sx[2][3], const int64_t sc[2][3], const int64_t sv[3], hipStream_t st);
 int launch_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, int64_t N, int D, int64_t scb,
                   int64_t sch, int64_t scn, hipStream_t st);
 int launch_dequant(const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp, void *out,
@@ -39,6 +43,8 @@ struct AttnArgs {
   int causal;
   int D;
   int io_dtype;
+  float *o32;   // forward: nullable, O in fp32 (dense); o is nullable then
+  int f32;      // backward: dO and the gradients are fp32, the workspace holds bwd_f32_workspace_bytes
 };
 
 int launch_fwd(const AttnArgs &a, hipStream_t st, bool qk_only = false);
@@ -47,6 +53,9 @@ int launch_delta(const void *o, const void *dout, float *delta, int io_dtype, in
 int launch_bwd(const AttnArgs &a, hipStream_t st);
 int launch_sum16(const void *a, const void *b, void *out, int dtype, int64_t n, hipStream_t st);   // out = a + b, n % 8 == 0
 int64_t bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
+inline int64_t bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
+  return bwd_workspace_bytes(B, H, Nq, Nk, D) + B * H * Nq * D * 2;
+}
 
 // grid of a kernel that maps ids with XcdBlock (qfa_skv_common.h): per_bh workgroups for each of BH heads
 __host__ __device__ inline bool xcd_whole_heads(int64_t BH) { return BH >= 64 || BH % 8 == 0; }

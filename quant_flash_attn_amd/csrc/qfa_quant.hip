@@ -124,6 +124,41 @@ template <typename T, int DP, bool PARTIAL> __global__ __launch_bounds__(256) vo
   else quant_block<T, DP, PARTIAL>(p.t[1], blockIdx.x - p.blocks0);
 }
 
+// The same for fp32 queries and keys with the conversion of the values to bf16 behind them: what an fp32 attention call needs,
+// in one launch.  A block takes as many tokens of the values as of the others.
+struct QuantQkvArgs {
+  QuantPairArgs p;
+  unsigned blocks1;     // of the pair
+  const float *v;
+  __bf16 *v16;          // dense
+  int64_t svb, svh, svn;
+};
+template <int D> __global__ __launch_bounds__(256) void quant_qkv_kernel(QuantQkvArgs a) {
+  if (blockIdx.x < a.p.blocks0) {
+    quant_block<float, D, false>(a.p.t[0], blockIdx.x);
+  } else if (blockIdx.x < a.blocks1) {
+    quant_block<float, D, false>(a.p.t[1], blockIdx.x - a.p.blocks0);
+  } else {
+    constexpr int TOK = 8192 / D;
+    const QuantArgs &k = a.p.t[1];   // (the values have the keys' sizes)
+    const unsigned block = blockIdx.x - a.blocks1;
+    const int64_t bh = block / k.chunks_per_bh, n0 = (int64_t)(block % k.chunks_per_bh) * TOK;
+    const float *v = a.v + bh / k.H * a.svb + bh % k.H * a.svh;
+    __bf16 *out = a.v16 + bh * k.N * D;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = (threadIdx.x + 256 * i) * 8;
+      const int64_t n = n0 + at / D;
+      if (n < k.N) {
+        const f32x4 *src = reinterpret_cast<const f32x4 *>(v + n * a.svn + at % D);
+        const f32x4 x = src[0], y = src[1];
+        *reinterpret_cast<u32x4 *>(out + n * D + at % D) =
+            u32x4{pack2<__bf16>(x[0], x[1]), pack2<__bf16>(x[2], x[3]), pack2<__bf16>(y[0], y[1]), pack2<__bf16>(y[2], y[3])};
+      }
+    }
+  }
+}
+
 template <typename T, int DP> static int launch_quant_d(const QuantArgs &a0, int64_t BH, hipStream_t st) {
   constexpr int TOK = 8192 / DP;   // tokens per workgroup, however they are held
   QuantArgs a = a0;
@@ -204,6 +239,40 @@ int launch_quant_pair(const void *const x[2], int x_dtype, int8_t *const codes[2
     case QFA_BF16: return launch_quant_pair_t<__bf16>(p, B * H, st);
   }
   return set_error(QFA_EINVAL, "quant_pair: bad x_dtype");
+}
+
+template <int D> static int launch_quant_qkv_d(QuantQkvArgs a, int64_t BH, hipStream_t st) {
+  constexpr int TOK = 8192 / D;
+  int64_t blocks[2];
+  for (int i = 0; i < 2; ++i) {
+    const int64_t chunks = (a.p.t[i].N + TOK - 1) / TOK;
+    a.p.t[i].chunks_per_bh = (int)chunks;
+    blocks[i] = chunks * BH;
+  }
+  const int64_t total = blocks[0] + 2 * blocks[1];
+  if (total > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "quant_qkv: too many tokens for one launch");
+  a.p.blocks0 = (unsigned)blocks[0];
+  a.blocks1 = (unsigned)(blocks[0] + blocks[1]);
+  quant_qkv_kernel<D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
+  return check_launch("qfa_quant_qkv_f32");
+}
+int launch_quant_qkv(const float *const x[2], int8_t *const codes[2], float *const scale[2], int8_t *const zp[2],
+                     int32_t *const rowsum[2], const float *v, void *v16, int64_t B, int64_t H, const int64_t N[2], int D,
+                     const int64_t sx[2][3], const int64_t sc[2][3], const int64_t sv[3], hipStream_t st) {
+  QuantQkvArgs q;
+  for (int i = 0; i < 2; ++i) {
+    QuantArgs &a = q.p.t[i];
+    a.x = x[i]; a.codes = codes[i]; a.scale = scale[i]; a.scale_lp = nullptr; a.zp = zp[i]; a.rowsum = rowsum[i];
+    a.N = N[i]; a.H = H; a.sxb = sx[i][0]; a.sxh = sx[i][1]; a.sxn = sx[i][2];
+    a.scb = sc[i][0]; a.sch = sc[i][1]; a.scn = sc[i][2];
+    a.chunks_per_bh = 0; a.scale_lp_dtype = 0; a.D = D;
+  }
+  q.p.blocks0 = q.blocks1 = 0;
+  q.v = v; q.v16 = static_cast<__bf16 *>(v16);
+  q.svb = sv[0]; q.svh = sv[1]; q.svn = sv[2];
+  if (D == 256) return launch_quant_qkv_d<256>(q, B * H, st);
+  if (D == 128) return launch_quant_qkv_d<128>(q, B * H, st);
+  return launch_quant_qkv_d<64>(q, B * H, st);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -30,12 +30,16 @@ struct Api {
   QFA_ENTRY(qfa_last_error);
   QFA_ENTRY(qfa_quant_per_token);
   QFA_ENTRY(qfa_quant_per_token_pair);
+  QFA_ENTRY(qfa_quant_qkv_f32);
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
   QFA_ENTRY(qfa_attn_fwd);
+  QFA_ENTRY(qfa_attn_fwd_f32);
   QFA_ENTRY(qfa_bench_qk_stage);
   QFA_ENTRY(qfa_attn_bwd_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd);
+  QFA_ENTRY(qfa_attn_bwd_f32_workspace_bytes);
+  QFA_ENTRY(qfa_attn_bwd_f32);
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
@@ -57,12 +61,16 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_last_error);
   QFA_ENTRY(qfa_quant_per_token);
   QFA_ENTRY(qfa_quant_per_token_pair);
+  QFA_ENTRY(qfa_quant_qkv_f32);
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
   QFA_ENTRY(qfa_attn_fwd);
+  QFA_ENTRY(qfa_attn_fwd_f32);
   QFA_ENTRY(qfa_bench_qk_stage);
   QFA_ENTRY(qfa_attn_bwd_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd);
+  QFA_ENTRY(qfa_attn_bwd_f32_workspace_bytes);
+  QFA_ENTRY(qfa_attn_bwd_f32);
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
@@ -283,14 +291,24 @@ void fwd_into(const Quantized &q, const Quantized &k, const Tensor &v, const Ten
 }
 
 using Grads = std::array<Tensor, 3>;
+// f32: dO comes and the gradients leave in fp32
 Grads bwd_of(const Quantized &q, const Quantized &k, const Tensor &v_in, const Tensor &o_in, const Tensor &do_in,
-             const float *lse, bool causal, double sm) {
-  const Tensor v = rows16(v_in), o = rows16(o_in), dout = rows16(to(do_in, v_in.scalar_type()));
-  const int64_t ws_bytes = api.qfa_attn_bwd_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D);
+             const float *lse, bool causal, double sm, bool f32 = false) {
+  const at::ScalarType gt = f32 ? at::kFloat : v_in.scalar_type();
+  const Tensor v = rows16(v_in), o = rows16(o_in), dout = rows16(to(do_in, gt));
+  const int64_t ws_bytes = (f32 ? api.qfa_attn_bwd_f32_workspace_bytes : api.qfa_attn_bwd_workspace_bytes)(q.B, q.H, q.N, k.N, (int)q.D);
   TORCH_CHECK_VALUE(ws_bytes > 0, "unsupported backward shape B=", q.B, " H=", q.H, " Nq=", q.N, " Nk=", k.N, " D=", q.D);
   const Tensor ws = empty({ws_bytes}, at::kByte, v);
-  Tensor dq = empty({q.B, q.H, q.N, q.D}, v.scalar_type(), v), dk = empty({q.B, q.H, k.N, q.D}, v.scalar_type(), v),
-         dv = empty({q.B, q.H, k.N, q.D}, v.scalar_type(), v);
+  Tensor dq = empty({q.B, q.H, q.N, q.D}, gt, v), dk = empty({q.B, q.H, k.N, q.D}, gt, v), dv = empty({q.B, q.H, k.N, q.D}, gt, v);
+  if (f32) {
+    check(api.qfa_attn_bwd_f32(q.codes, q.scale, q.zp, q.rowsum, k.codes, k.scale, k.zp, k.rowsum, v.data_ptr(), o.data_ptr(),
+                               dout.data_ptr<float>(), lse, ws.data_ptr(), ws_bytes, dq.data_ptr<float>(), dk.data_ptr<float>(),
+                               dv.data_ptr<float>(), dtype_code(v.scalar_type()), q.B, q.H, q.N, k.N, (int)q.D, q.sb, q.sh, q.sn,
+                               k.sb, k.sh, k.sn, QFA_STRIDES(v), QFA_STRIDES(o), QFA_STRIDES(dout), QFA_STRIDES(dq),
+                               QFA_STRIDES(dk), QFA_STRIDES(dv), (float)sm, causal, stream_of(v)),
+          "qfa_attn_bwd_f32");
+    return {dq, dk, dv};
+  }
   check(api.qfa_attn_bwd(q.codes, q.scale, q.zp, q.rowsum, k.codes, k.scale, k.zp, k.rowsum, v.data_ptr(), o.data_ptr(),
                          dout.data_ptr(), lse, ws.data_ptr(), ws_bytes, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                          dtype_code(v.scalar_type()), q.B, q.H, q.N, k.N, (int)q.D, q.sb, q.sh, q.sn, k.sb, k.sh, k.sn,
@@ -373,22 +391,48 @@ struct Kept {
   Tensor buf, v16, o16, o;
 };
 // backward from them
-Grads bwd_from(AutogradContext *ctx, const variable_list &saved, const Tensor &grad) {
+Grads bwd_from(AutogradContext *ctx, const variable_list &saved, const Tensor &grad, bool f32) {
   const Tensor &buf = saved[0], &v16 = saved[1], &o16 = saved[2];
   const int64_t Nk = v16.size(2);
   const PairBuffer pb(o16.size(0), o16.size(1), o16.size(2), Nk, o16.size(3));
   const c10::DeviceGuard guard(v16.device());
   return bwd_of(pb.view(buf, 0), pb.view(buf, 1), v16, o16, grad, pb.lse_of(buf),
-                ctx->saved_data["causal"].toBool(), ctx->saved_data["sm"].toDouble());
+                ctx->saved_data["causal"].toBool(), ctx->saved_data["sm"].toDouble(), f32);
 }
 
 // ---- q, k, v
-Kept qkv_forward(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, bool causal, double sm) {
+bool all_f32(const Tensor &q, const Tensor &k, const Tensor &v) {
+  return q.scalar_type() == at::kFloat && k.scalar_type() == at::kFloat && v.scalar_type() == at::kFloat;
+}
+// keep: what a backward takes is made too
+Kept qkv_forward(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, bool causal, double sm, bool keep) {
   const c10::DeviceGuard guard(q_in.device());
   const Tensor q = check_input(q_in), k = check_input(k_in);
   const PairBuffer pb(q.size(0), q.size(1), q.size(2), k.size(2), q.size(3));
   Kept r;
   r.buf = empty({pb.bytes}, at::kByte, q);
+  if (all_f32(q, k, v_in) && (pb.D == 64 || pb.D == 128 || pb.D == 256)) {
+    // fp32 in and out without launches of their own for the conversions: the quantizer's launch takes V along, the forward
+    // writes O in both types, the staging pass rounds dO, and the gradients leave in fp32 (B1 H4 N256 D64, forward and backward:
+    // 5 launches instead of 11, 105 -> 45 us)
+    const Tensor v = rows16(v_in);
+    const Quantized a = pb.view(r.buf, 0), b = pb.view(r.buf, 1);
+    auto w = [](auto *p) { return const_cast<std::remove_const_t<std::remove_pointer_t<decltype(p)>> *>(p); };
+    r.v16 = empty({pb.B, pb.H, pb.N[1], pb.D}, at::kBFloat16, q);
+    check(api.qfa_quant_qkv_f32(q.data_ptr<float>(), k.data_ptr<float>(), v.data_ptr<float>(), w(a.codes), w(b.codes), w(a.scale),
+                                w(b.scale), w(a.zp), w(b.zp), w(a.rowsum), w(b.rowsum), r.v16.data_ptr(), a.B, a.H, a.N, b.N,
+                                (int)a.D, QFA_STRIDES(q), QFA_STRIDES(k), QFA_STRIDES(v), a.sb, a.sh, a.sn, b.sb, b.sh, b.sn,
+                                stream_of(q)),
+          "qfa_quant_qkv_f32");
+    r.o = empty({pb.B, pb.H, pb.N[0], pb.D}, at::kFloat, q);
+    if (keep) r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, at::kBFloat16, q);
+    check(api.qfa_attn_fwd_f32(a.codes, a.scale, a.zp, a.rowsum, b.codes, b.scale, b.zp, b.rowsum, r.v16.data_ptr(),
+                               r.o.data_ptr<float>(), keep ? r.o16.data_ptr() : nullptr, pb.lse_of(r.buf), QFA_BF16, a.B, a.H, a.N,
+                               b.N, (int)a.D, a.sb, a.sh, a.sn, b.sb, b.sh, b.sn, QFA_STRIDES(r.v16), QFA_STRIDES(r.o), (float)sm,
+                               causal, stream_of(q)),
+          "qfa_attn_fwd_f32");
+    return r;
+  }
   quantize_pair_into(q, k, pb.view(r.buf, 0), pb.view(r.buf, 1));
   r.v16 = rows16(to(v_in, io_dtype(v_in)));
   r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, r.v16.scalar_type(), q);
@@ -399,7 +443,7 @@ Kept qkv_forward(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, boo
 struct QkvFn : torch::autograd::Function<QkvFn> {
   static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, bool causal, double sm) {
     const at::AutoDispatchBelowADInplaceOrView below;
-    Kept r = qkv_forward(q, k, v, causal, sm);
+    Kept r = qkv_forward(q, k, v, causal, sm, true);
     ctx->save_for_backward({r.buf, r.v16, r.o16});
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["sm"] = sm;
@@ -408,8 +452,9 @@ struct QkvFn : torch::autograd::Function<QkvFn> {
   }
   static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
     const at::AutoDispatchBelowADInplaceOrView below;
-    const Grads g = bwd_from(ctx, ctx->get_saved_variables(), grads[0]);
     const int64_t dt = ctx->saved_data["dt"].toInt();
+    const int64_t f = (int64_t)at::kFloat, all = f | f << 8 | f << 16;
+    const Grads g = bwd_from(ctx, ctx->get_saved_variables(), grads[0], dt == all);
     return {to(g[0], (at::ScalarType)(dt & 255)), to(g[1], (at::ScalarType)(dt >> 8 & 255)),
             to(g[2], (at::ScalarType)(dt >> 16)), Tensor(), Tensor()};
   }
@@ -421,7 +466,7 @@ Tensor qkv_op(const Tensor &q, const Tensor &k, const Tensor &v, bool causal, do
   TORCH_CHECK_VALUE(q.size(3) == k.size(3) && k.sizes() == v.sizes() && q.size(0) == k.size(0) && q.size(1) == k.size(1),
                     "shape mismatch: q ", q.sizes(), ", k ", k.sizes(), ", v ", v.sizes());
   if (wants_grad({&q, &k, &v})) return QkvFn::apply(q, k, v, causal, sm);
-  return qkv_forward(q, k, v, causal, sm).o;
+  return qkv_forward(q, k, v, causal, sm, false).o;
 }
 Tensor qkv(const Tensor &q, const Tensor &k, const Tensor &v, bool causal, double sm) {
   if (torch::jit::tracer::isTracing()) return Traced<decltype(qkv_op)>::call("quant_flash_attn_amd::qkv", q, k, v, causal, sm);

@@ -82,7 +82,8 @@ def attn_bwd_shared_kv(q: torch.Tensor, codes: torch.Tensor, scale: torch.Tensor
 class QuantFlashAttnQKV:
     """apply(q, k, v, causal, sm_scale) -> o   (argument order of flash_attn_triton.py:441); backward -> (dq, dk, dv).
 
-    q, k, v: [B,H,N,D] bf16 / fp16 (fp32 is accepted: V and O then pass through bf16).
+    q, k, v: [B,H,N,D] bf16 / fp16 / fp32 (fp32: V, dO and the O that the backward takes are rounded to bf16; where all three are
+    fp32, O and the gradients are not).
     causal keeps key j for query i when j <= i (flash_attn_triton.py:50); with fewer queries than keys the mask is
     aligned to the last key (j <= i + Nk - Nq)."""
 
