@@ -133,13 +133,19 @@ int qfa_attn_fwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
                  int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *stream);
 
 /*
- * The same with O in fp32 as well: o32 [B,H,Nq,D] dense, unrounded; o (the 16-bit one that a backward takes) may be NULL.
+ * The same with two additions.  o32 (nullable): O in fp32, [B,H,Nq,D] dense, unrounded; o, the 16-bit one that a backward takes,
+ * may be NULL then.  workspace (nullable): with few queries in all, most of the chip is idle; given a caller-owned scratch of
+ * qfa_attn_fwd_split_workspace_bytes(...) bytes (16-byte aligned; 0 when no split pays) the keys are split over workgroups and
+ * a second small kernel merges their partial (O, m, l).
  */
-int qfa_attn_fwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
-                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, float *o32, void *o, float *lse,
+int64_t qfa_attn_fwd_split_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal);
+
+int qfa_attn_fwd_split(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, void *o, float *o32, float *lse,
                  int io_dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh,
                  int64_t sqn, int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn,
-                 int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *stream);
+                 int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *workspace,
+                 int64_t workspace_bytes, void *stream);
 
 /*
  * Attention forward of the reference's own operator, for short query blocks:

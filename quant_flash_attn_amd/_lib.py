@@ -32,7 +32,8 @@ _SIGNATURES = {
     "qfa_dequant_per_token": (c_int, [_P, _P, _I, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_code_rowsum": (c_int, [_P, _P, _L, _L, _L, _I, _L, _L, _L, _P]),
     "qfa_attn_fwd": (c_int, [_P] * 11 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P]),
-    "qfa_attn_fwd_f32": (c_int, [_P] * 12 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P]),
+    "qfa_attn_fwd_split_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I, _I]),
+    "qfa_attn_fwd_split": (c_int, [_P] * 12 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P, _L, _P]),
     "qfa_attn_fwd_shared_kv_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
     "qfa_attn_fwd_shared_kv": (c_int, [_P, _P, _P, _I, _P, _P, _P, _I, _L, _L, _L, _L, _I] + [_L] * 9 + [_F, _P, _L, _P]),
     "qfa_attn_fwd_shared_kv_static": (c_int, [_P, _P, _P, _I, _P, _P, _P, _I, _L, _L, _L, _L, _I] + [_L] * 9 + [_F, _P]),

@@ -195,11 +195,17 @@ int qfa_attn_fwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
   return launch_fwd(a, (hipStream_t)stream);
 }
 
-int qfa_attn_fwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
-                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, float *o32, void *o, float *lse,
+int64_t qfa_attn_fwd_split_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal) {
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0 || (D != 64 && D != 128 && D != 256)) return 0;
+  return fwd_workspace_bytes(B, H, Nq, Nk, D, causal);
+}
+
+int qfa_attn_fwd_split(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
+                 const float *sk, const int8_t *zk, const int32_t *rk, const void *v, void *o, float *o32, float *lse,
                  int io_dtype, int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh,
                  int64_t sqn, int64_t skb, int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn,
-                 int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *stream) {
+                 int64_t sob, int64_t soh, int64_t son, float sm_scale, int causal, void *workspace,
+                 int64_t workspace_bytes, void *stream) {
   AttnArgs a;
   memset(&a, 0, sizeof(a));
   a.qc = qc; a.sq = sq; a.zq = zq; a.rq = rq; a.kc = kc; a.sk = sk; a.zk = zk; a.rk = rk;
@@ -208,8 +214,14 @@ int qfa_attn_fwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const 
   a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.skb = skb; a.skh = skh; a.skn = skn;
   a.svb = svb; a.svh = svh; a.svn = svn; a.sob = sob; a.soh = soh; a.son = son;
   a.sm_scale = sm_scale; a.causal = causal;
-  if (!o32) return set_error(QFA_EINVAL, "attn_fwd_f32: null pointer argument");
-  if (int e = check_attn_common("attn_fwd_f32", a)) return e;
+  if (int e = check_attn_common("attn_fwd_split", a)) return e;
+  if (workspace) {
+    const int64_t need = fwd_workspace_bytes(B, H, Nq, Nk, D, causal);
+    if (!aligned16(workspace) || workspace_bytes < need)
+      return set_error(QFA_EINVAL, "attn_fwd_split: workspace must be 16-byte aligned and hold %lld bytes "
+                       "(qfa_attn_fwd_split_workspace_bytes), got %lld", (long long)need, (long long)workspace_bytes);
+    a.workspace = need > 0 ? workspace : nullptr;
+  }
   return launch_fwd(a, (hipStream_t)stream);
 }
 

@@ -383,7 +383,7 @@ template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, 
   cache_fwd_kernel<S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_cache")) return e;
   if (a.splits > 1) {
-    const SplitMergeArgs m = {a.po, a.pml, a.o, nullptr, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, a.q_dtype};
+    const SplitMergeArgs m = {a.po, a.pml, a.o, nullptr, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, a.q_dtype, nullptr};
     return launch_split_merge<D>(m, x.B * x.H * x.Nq, "qfa_attn_fwd_cache (merge)", st);
   }
   return 0;

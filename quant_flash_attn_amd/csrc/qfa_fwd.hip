@@ -65,6 +65,7 @@
 #include <type_traits>
 
 #include "qfa_fwd_common.h"
+#include "qfa_merge.h"
 
 namespace qfa {
 
@@ -76,7 +77,9 @@ template <int V> using ic = std::integral_constant<int, V>;
 // correction, scaling and a maximum over the scores, with the V copies, the exponentials and the P.V product compiled
 // out (it writes the scaled row maximum where the LSE would go and leaves O untouched).  It exists to
 // time the QK^T stage by itself against the INT8 MFMA peak.
-template <typename T, int D, bool CAUSAL, bool QK_ONLY = false, int NW = FWD_WAVES>
+// SPLIT: the keys are shared by a.splits workgroups; one takes keys key0 .. key0 + Nk - 1, as a sequence of its own whose mask is
+// shifted, and leaves its unnormalised result for the merge.
+template <typename T, int D, bool CAUSAL, bool QK_ONLY = false, bool SPLIT = false, int NW = FWD_WAVES>
 __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(FwdArgs a) {
   constexpr int NT = 64 * NW;        // threads per workgroup
   constexpr int FWD_BM = 32 * NW;    // queries per workgroup
@@ -95,7 +98,14 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   if (vid >= a.total_blocks) return;
   int bh = vid / a.mblocks;
   int mb = vid % a.mblocks;
-  if (CAUSAL) {
+  int split = 0, key0 = 0;
+  if (SPLIT) {   // (all of them are resident at once: any order will do)
+    split = bh % a.splits;
+    bh /= a.splits;
+    key0 = split * a.keys_per_split;
+  }
+  const int Nk = SPLIT ? min(a.keys_per_split, a.Nk - key0) : a.Nk;
+  if (CAUSAL && !SPLIT) {
     // Longest rows first, and a group of heads at a time: ids run over the query blocks of 2^group_log2
     // heads, cycling through them from the longest block down.  With one head after the other the last
     // head's long blocks start when the chip is already draining (10 % longer makespan in a list-scheduling
@@ -120,11 +130,10 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   const int g = lane / 32;    // k-group
 
   const int8_t *qc_bh = a.qc + b * a.sqb + h * a.sqh;
-  const int8_t *kc_bh = a.kc + b * a.skb + h * a.skh;
-  const T *v_bh = reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh;
-  T *o_bh = reinterpret_cast<T *>(a.o) + b * a.sob + h * a.soh;
+  const int8_t *kc_bh = a.kc + b * a.skb + h * a.skh + key0 * a.skn;
+  const T *v_bh = reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh + key0 * a.svn;
   const int64_t tq0 = (int64_t)bh * a.Nq;
-  const int64_t tk0 = (int64_t)bh * a.Nk;
+  const int64_t tk0 = (int64_t)bh * a.Nk + key0;
 
   // ---- this lane's query
   const int qi = m0 + wave * 32 + lr;
@@ -173,12 +182,12 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   }
 
   // ---- tile range
-  int kv_end = a.Nk;
+  int kv_end = Nk;
   // causal: query i keeps keys j <= i + coff, the mask aligned to the last key (coff = Nk - Nq >= 0; the rule
   // row >= col when Nq == Nk)
-  const int coff = CAUSAL ? a.Nk - a.Nq : 0;
-  if (CAUSAL) kv_end = min(a.Nk, m0 + FWD_BM + coff);
-  const int ntiles = (kv_end + FWD_BN - 1) / FWD_BN;
+  const int coff = CAUSAL ? a.Nk - a.Nq - key0 : 0;
+  if (CAUSAL) kv_end = min(Nk, m0 + FWD_BM + coff);
+  const int ntiles = SPLIT && kv_end <= 0 ? 0 : (kv_end + FWD_BN - 1) / FWD_BN;
 
   // ---- tile copies: K and V by direct loads, the per-key constants through registers
   typedef Swz<D> KSW;
@@ -197,9 +206,9 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   // arithmetic), so a copy costs one instruction per 16-byte chunk and thread; the per-key constant
   // vectors are read the same way, with exact bounds (keys past the end read as zero and are masked).
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const rsrc_t rs_sk = make_rsrc(a.sk + tk0, (unsigned)a.Nk * 4u);
-  const rsrc_t rs_rk = make_rsrc(a.rk + tk0, (unsigned)a.Nk * 4u);
-  const rsrc_t rs_zk = make_rsrc(a.zk + tk0, (unsigned)a.Nk);
+  const rsrc_t rs_sk = make_rsrc(a.sk + tk0, (unsigned)Nk * 4u);
+  const rsrc_t rs_rk = make_rsrc(a.rk + tk0, (unsigned)Nk * 4u);
+  const rsrc_t rs_zk = make_rsrc(a.zk + tk0, (unsigned)Nk);
   auto load_kc = [&](int t) {   // per-key constants of tile t -> registers
     if (tid < FWD_BN) {
       c_sk = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_sk, tid * 4, t * FWD_BN * 4, 0));
@@ -210,10 +219,10 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   auto load_k = [&](int t, int buf) {
     const int j0 = t * FWD_BN;
     unsigned char *dst = smem + SM::OFF_K + buf * SM::K_BYTES;
-    if (j0 + FWD_BN <= a.Nk)
+    if (j0 + FWD_BN <= Nk)
       cp_k.issue(reinterpret_cast<const unsigned char *>(kc_bh) + (int64_t)j0 * a.skn, dst, wave_u);
     else
-      dma_rows<D, FWD_BN, NT, KSW>(reinterpret_cast<const unsigned char *>(kc_bh), a.skn, j0, a.Nk - 1, dst, tid);
+      dma_rows<D, FWD_BN, NT, KSW>(reinterpret_cast<const unsigned char *>(kc_bh), a.skn, j0, Nk - 1, dst, tid);
     load_kc(t);
   };
   auto store_k = [&](int buf) {
@@ -233,10 +242,10 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     const int j0 = t * FWD_BN;
     unsigned char *dst = smem + SM::OFF_V + buf * SM::V_BYTES;
     const int64_t vstride = a.svn * (int64_t)sizeof(T);
-    if (j0 + FWD_BN <= a.Nk)
+    if (j0 + FWD_BN <= Nk)
       cp_v.issue(reinterpret_cast<const unsigned char *>(v_bh) + (int64_t)j0 * vstride, dst, wave_u);
     else
-      dma_rows<2 * D, FWD_BN, NT, VSW>(reinterpret_cast<const unsigned char *>(v_bh), vstride, j0, a.Nk - 1, dst, tid);
+      dma_rows<2 * D, FWD_BN, NT, VSW>(reinterpret_cast<const unsigned char *>(v_bh), vstride, j0, Nk - 1, dst, tid);
   };
   // this lane's read offsets inside a tile (the swizzle terms only depend on the lane)
   const int k_swz = KSW::swz(lr);                                        // rows 32*nb + lr
@@ -299,7 +308,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
         float uu = f[4 * aa + bb] * sk4[bb];
         if (MASKED) {
           const int j = j0 + jl + bb;
-          if ((CAUSAL && j > qi + coff) || j >= a.Nk) uu = -INFINITY;
+          if ((CAUSAL && j > qi + coff) || j >= Nk) uu = -INFINITY;
         }
         u[4 * aa + bb] = uu;
         mt = fmaxf(mt, uu);
@@ -313,10 +322,11 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   auto move_ref = [&](float mt) __attribute__((always_inline)) {
     {
       const float m_new = fmaxf(m_ref, mt);
-      const float alpha = __builtin_amdgcn_exp2f(a_i * (m_ref - m_new));
+      float alpha = __builtin_amdgcn_exp2f(a_i * (m_ref - m_new));
+      if (SPLIT && m_ref == m_new) alpha = 1.0f;   // also of a row that has seen no key of the split: -inf both
       m_ref = m_new;
       m_bound = m_new + thr_i;
-      nm = -a_i * m_new;
+      nm = SPLIT && m_new == -INFINITY ? 0.f : -a_i * m_new;   // and then p = exp2(-inf + 0) = 0
       l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -364,9 +374,11 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   };
 
   // ---- prologue: K(0), K(1) (with their constants) and V(0) resident
-  load_k(0, 0);
-  load_v(0, 0);
-  store_k(0);
+  if (!SPLIT || ntiles > 0) {
+    load_k(0, 0);
+    load_v(0, 0);
+    store_k(0);
+  }
   if (ntiles > 1) {
     load_k(1, 1);
     store_k(1);
@@ -375,7 +387,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   __syncthreads();
 
   // tiles [0, t_hot) contain no masked score for this wave (wave-uniform)
-  int t_hot = a.Nk / FWD_BN;
+  int t_hot = Nk / FWD_BN;
   if (CAUSAL) t_hot = min(t_hot, (q_first + coff + 1) / FWD_BN);
   t_hot = min(t_hot, ntiles);
 
@@ -596,7 +608,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     };
     {
       // tiles [0, t_steady) are unmasked for this wave, and their copies (two tiles ahead) are full tiles
-      const int t_steady = min(t_hot, min(ntiles - 2, a.Nk / FWD_BN - 2));
+      const int t_steady = min(t_hot, min(ntiles - 2, Nk / FWD_BN - 2));
       if constexpr (D <= 128 && !QK_ONLY) {
         // three tiles per trip with constant buffer indices
         for (; t + 3 <= t_steady; t += 3) {
@@ -632,7 +644,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     // block then only needs the mask, the maximum and the P.V step: no score product is formed twice and the visible
     // block keeps the pipelined pace (the generic loop below took 2 900 cycles per block where this takes 1 600).
     if (!QK_ONLY && CAUSAL && D <= 128 && t < ntiles && coff % 32 == 0 && t == (q_first + coff + 1) / FWD_BN &&
-        (t + 1) * FWD_BN <= a.Nk) {
+        (t + 1) * FWD_BN <= Nk) {
       if (t + 2 < ntiles) load_k(t + 2, kb_free);
       if (t + 1 < ntiles) load_v(t + 1, kb_nxt);
       const int j0 = t * FWD_BN;
@@ -676,7 +688,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
       const int jb = j0 + 32 * nb;
-      if ((CAUSAL && jb > q_last + coff) || jb >= a.Nk) continue;   // wave-uniform: nothing to keep
+      if ((CAUSAL && jb > q_last + coff) || jb >= Nk) continue;   // wave-uniform: nothing to keep
       i32x16 s;
       float u[16];
       qk_block(kb_cur, nb, s);
@@ -695,13 +707,31 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     return;
   }
   const float l_tot = l_run + swap32_f(l_run);
+  // What only the epilogue needs is read from the kernel arguments here: held in scalar registers through the loop it
+  // would push others out to memory.
+  typedef __attribute__((address_space(4))) const FwdArgs KernArgs;
+  KernArgs *ep = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ep));
+  if (SPLIT) {
+    if (qi < a.Nq) {
+      const int64_t at = (tq0 + qi) * a.splits + split;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int aa = 0; aa < 4; ++aa)
+          *reinterpret_cast<f32x4 *>(ep->po + at * D + 32 * db + 8 * aa + 4 * g) =
+              f32x4{oacc[db][4 * aa], oacc[db][4 * aa + 1], oacc[db][4 * aa + 2], oacc[db][4 * aa + 3]};
+      if (g == 0) *reinterpret_cast<f32x2 *>(ep->pml + 2 * at) = f32x2{a_i * m_ref, l_tot};
+    }
+    return;
+  }
   const float inv = 1.0f / l_tot;
   // O leaves as whole rows through LDS (all tile buffers are free after the last barrier; every wave takes 32 * 2D
   // bytes at the start of the K area)
   static_assert(SM::OFF_K + FWD_WAVES * 32 * 2 * D <= SM::TOTAL, "output staging fits the tile buffers");
-  if (a.o32) store_tile_rows_f32<D>(oacc, inv, a.o32 + tq0 * D, D, m0 + wave * 32, a.Nq, lane);
-  if (a.o) store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), o_bh, a.son, m0 + wave * 32, a.Nq, lane);
-  if (qi < a.Nq && g == 0) a.lse[tq0 + qi] = (a_i * m_ref + __log2f(l_tot)) * kLn2;
+  if (ep->o32) store_tile_rows_f32<D>(oacc, inv, ep->o32 + tq0 * D, D, m0 + wave * 32, a.Nq, lane);
+  if (ep->o) store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), reinterpret_cast<T *>(ep->o) + b * ep->sob + h * ep->soh, ep->son, m0 + wave * 32, a.Nq, lane);
+  if (qi < a.Nq && g == 0) ep->lse[tq0 + qi] = (a_i * m_ref + __log2f(l_tot)) * kLn2;
 }
 
 template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStream_t st, bool qk_only) {
@@ -715,7 +745,15 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
   a.sm_scale_log2 = x.sm_scale * kLog2e;
   constexpr int FWD_BM = 32 * FWD_WAVES;
   a.mblocks = (int)((x.Nq + FWD_BM - 1) / FWD_BM);
-  const int64_t total = (int64_t)a.mblocks * x.B * x.H;
+  a.splits = 1;
+  a.keys_per_split = 0;
+  a.po = a.pml = nullptr;
+  if (x.workspace && !qk_only) {   // validated: large enough for the plan
+    fwd_plan(x.B * x.H, x.Nq, x.Nk, D, x.causal, &a.splits, &a.keys_per_split);
+    a.po = static_cast<float *>(x.workspace);
+    a.pml = a.po + x.B * x.H * x.Nq * a.splits * (int64_t)D;
+  }
+  const int64_t total = (int64_t)a.mblocks * x.B * x.H * a.splits;
   if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_fwd: too many query blocks for one launch");
   a.total_blocks = (int)total;
   a.blocks_per_xcd = (a.total_blocks + 7) / 8;
@@ -729,6 +767,17 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
     if (x.causal) fwd_kernel<T, D, true, true><<<grid, block, 0, st>>>(a);
     else fwd_kernel<T, D, false, true><<<grid, block, 0, st>>>(a);
   } else {
+    if (a.splits > 1) {
+      if constexpr (D == 256) {
+        if (int e = launch_fwd_wide<T, D>(a, x.B * x.H, x.causal, st)) return e;
+      } else {
+        if (x.causal) fwd_kernel<T, D, true, false, true><<<grid, block, 0, st>>>(a);
+        else fwd_kernel<T, D, false, false, true><<<grid, block, 0, st>>>(a);
+        if (int e = check_launch("qfa_attn_fwd")) return e;
+      }
+      const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, x.io_dtype, a.o32};
+      return launch_split_merge<D>(m, x.B * x.H * x.Nq, "qfa_attn_fwd (merge)", st);
+    }
     // One wave per SIMD: always at head_dim 256 (4096 causal, 64 heads: 645 -> 560 us; 1500 x 1500, 8 heads: 62 -> 43 us).
     // At 128, where two waves of this kernel share a SIMD, only long sequences without a mask that fill whole rounds of 256
     // workgroups with 15/16 of their rows: one workgroup per CU has nothing beside it while it starts and ends

@@ -17,6 +17,8 @@ struct FwdArgs {
   int mblocks;           // query blocks of one workgroup each per (batch, head)
   int total_blocks;      // mblocks * B * H
   int blocks_per_xcd;    // ceil(total_blocks / 8)
+  int splits, keys_per_split;   // workgroups that share the keys of a query block (a multiple of 64 each)
+  float *po, *pml;       // splits > 1: partial results per query and split (qfa_merge.h)
   int group_log2;        // causal: log2 of the number of heads whose query blocks are dispatched together
 };
 

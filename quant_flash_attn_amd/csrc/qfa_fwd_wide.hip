@@ -32,7 +32,7 @@ template <int D> struct FwdWideSmem {
   static_assert(BUF % 256 == 0 && 3 * BUF <= 160 * 1024, "three tile buffers");
 };
 
-template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(FwdArgs a) {
+template <typename T, int D, int QB, bool CAUSAL, bool SPLIT> __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(FwdArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__   // (with the body in view the host pass of this compiler emits no launch stub)
   typedef FwdWideSmem<D> SM;
   constexpr int TILE = SM::TILE, NSTEP = TILE / 32, SLAB = SM::SLAB;
@@ -46,7 +46,14 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   if (vid >= a.total_blocks) return;
   int bh = vid / a.mblocks;
   int mb = vid % a.mblocks;
-  if (CAUSAL) {
+  int split = 0, key0 = 0;
+  if (SPLIT) {   // the keys of a query block in a.splits parts, as in qfa_fwd.hip
+    split = bh % a.splits;
+    bh /= a.splits;
+    key0 = split * a.keys_per_split;
+  }
+  const int Nk = SPLIT ? min(a.keys_per_split, a.Nk - key0) : a.Nk;
+  if (CAUSAL && !SPLIT) {
     const int gsz = 1 << a.group_log2;
     const int pb = bh >> a.group_log2 << a.group_log2;
     if (pb + gsz <= a.total_blocks / a.mblocks) {
@@ -63,13 +70,13 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   const int q_first = m0 + wave * QUERIES;
 
   const int8_t *qc_bh = a.qc + b * a.sqb + h * a.sqh;
-  const unsigned char *kc_bh = reinterpret_cast<const unsigned char *>(a.kc + b * a.skb + h * a.skh);
-  const unsigned char *v_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh);
-  const int64_t tq0 = (int64_t)bh * a.Nq, tk0 = (int64_t)bh * a.Nk;
+  const unsigned char *kc_bh = reinterpret_cast<const unsigned char *>(a.kc + b * a.skb + h * a.skh + key0 * a.skn);
+  const unsigned char *v_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh + key0 * a.svn);
+  const int64_t tq0 = (int64_t)bh * a.Nq, tk0 = (int64_t)bh * a.Nk + key0;
 
-  const int coff = CAUSAL ? a.Nk - a.Nq : 0;   // causal: query i keeps keys j <= i + coff (mask aligned to the last key)
-  const int ntiles = ((CAUSAL ? min(a.Nk, m0 + 4 * QUERIES + coff) : a.Nk) + TILE - 1) / TILE;
-  const int wtiles = q_first >= a.Nq ? 0 : ((CAUSAL ? min(a.Nk, q_first + QUERIES + coff) : a.Nk) + TILE - 1) / TILE;
+  const int coff = CAUSAL ? a.Nk - a.Nq - key0 : 0;   // causal: query i keeps keys j <= i + coff (mask aligned to the last key)
+  const int ntiles = ((CAUSAL ? min(Nk, m0 + 4 * QUERIES + coff) : Nk) + TILE - 1) / TILE;
+  const int wtiles = q_first >= a.Nq ? 0 : ((CAUSAL ? min(Nk, q_first + QUERIES + coff) : Nk) + TILE - 1) / TILE;
 
   // ---- tile copies (direct to LDS); the per-key constants through registers, key = lane, the same in every wave
   typedef SlabCopy<TILE, KS> CopyK;
@@ -77,12 +84,12 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   const CopyK cp_k(lane, (unsigned)a.skn);
   const CopyV cp_v(lane, (unsigned)a.svn * 2u);
   constexpr int PIECES = CopyK::N + CopyV::N;
-  const rsrc_t rs_sk = make_rsrc(a.sk + tk0, (unsigned)a.Nk * 4u);
-  const rsrc_t rs_rk = make_rsrc(a.rk + tk0, (unsigned)a.Nk * 4u);
-  const rsrc_t rs_zk = make_rsrc(a.zk + tk0, (unsigned)a.Nk);
+  const rsrc_t rs_sk = make_rsrc(a.sk + tk0, (unsigned)Nk * 4u);
+  const rsrc_t rs_rk = make_rsrc(a.rk + tk0, (unsigned)Nk * 4u);
+  const rsrc_t rs_zk = make_rsrc(a.zk + tk0, (unsigned)Nk);
   struct TileDesc { rsrc_t k, v; unsigned char *dst; };
   auto tile_desc = [&](int t) __attribute__((always_inline)) -> TileDesc {
-    const int rows = t < ntiles ? min(TILE, a.Nk - TILE * t) : 0;
+    const int rows = t < ntiles ? min(TILE, Nk - TILE * t) : 0;
     return {cp_k.desc(kc_bh + (int64_t)t * TILE * a.skn, rows), cp_v.desc(v_bh + (int64_t)t * TILE * a.svn * 2, rows),
             smem + t % 3 * SM::BUF};
   };
@@ -119,7 +126,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const int qi = q_first + 32 * qb + lr, qc = min(qi, a.Nq - 1);
-    k_hi[qb] = CAUSAL ? min(qc + coff, a.Nk - 1) : a.Nk - 1;
+    k_hi[qb] = CAUSAL ? min(qc + coff, Nk - 1) : Nk - 1;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[qb][ks] = *reinterpret_cast<const i32x4 *>(qc_bh + (int64_t)qc * a.sqn + ks * 32 + g * 16);
@@ -319,9 +326,10 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
         float u[16];
         float mt = fmaxf(scores(qb, t, buf, mbk, u), m_ref[qb] + __log2f(fmaxf(l_run[qb], 1.0f)) / a_i[qb]);
         const float m_new = fmaxf(m_ref[qb], max_across_halves(mt));
-        const float alpha = __builtin_amdgcn_exp2f(a_i[qb] * (m_ref[qb] - m_new));
+        float alpha = __builtin_amdgcn_exp2f(a_i[qb] * (m_ref[qb] - m_new));
+        if (SPLIT && m_ref[qb] == m_new) alpha = 1.0f;   // also of a row without keys: -inf both
         m_ref[qb] = m_new;
-        nm[qb] = -a_i[qb] * m_new;
+        nm[qb] = SPLIT && m_new == -INFINITY ? 0.f : -a_i[qb] * m_new;
         l[qb] = l_run[qb] * alpha;
         acc_scale<qb * DB, DB>(alpha);
 #pragma unroll
@@ -342,12 +350,12 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   __syncthreads();
   int t = 0, buf = 0, nbuf = SM::BUF;
   if (wtiles > 0) {
-    // the first step: reference maximum (every query sees key 0), raw scores, constants and first fragments
+    // the first step: reference maximum (every query sees key 0, or no key of its split), raw scores, constants and first fragments
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       float u[16];
       m_ref[qb] = max_across_halves(scores(qb, 0, 0, 0, u));
-      nm[qb] = -a_i[qb] * m_ref[qb];
+      nm[qb] = SPLIT && m_ref[qb] == -INFINITY ? 0.f : -a_i[qb] * m_ref[qb];
       si[qb] = bias;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) si[qb] = mfma_i8(__builtin_bit_cast(i32x4, ld(row_l + SM::OFF_K + ks * SLAB)), qf[qb][ks], si[qb]);
@@ -369,7 +377,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
         nbuf = b2;
       }
     };
-    tiles(min(wtiles, min(a.Nk / TILE, CAUSAL ? (q_first + coff + 1) / TILE : wtiles)), std::false_type{});
+    tiles(min(wtiles, min(Nk / TILE, CAUSAL ? (q_first + coff + 1) / TILE : wtiles)), std::false_type{});
     tiles(wtiles, std::true_type{});
     // P.V of the last step (fragments 0 .. AHEAD-1 are under way)
     const int j_last = TILE * wtiles - 32;
@@ -398,9 +406,15 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
     constexpr int qb = decltype(qb_tag)::value;
     const float l_tot = l_run[qb] + swap32_f(l_run[qb]);
+    const int qi = q_first + 32 * qb + lr;
+    if constexpr (SPLIT) {
+      const int64_t at = tq0 * a.splits + split;
+      acc_store_rows_f32<D, qb * DB>(1.0f, a.po + at * D, (int64_t)a.splits * D, q_first + 32 * qb, a.Nq, lane);
+      if (qi < a.Nq && g == 0) *reinterpret_cast<f32x2 *>(a.pml + 2 * (at + (int64_t)qi * a.splits)) = f32x2{a_i[qb] * m_ref[qb], l_tot};
+      return;
+    }
     if (a.o32) acc_store_rows_f32<D, qb * DB>(1.0f / l_tot, a.o32 + tq0 * D, D, q_first + 32 * qb, a.Nq, lane);
     if (a.o) acc_store_rows<T, D, qb * DB>(1.0f / l_tot, stage, o_bh, a.son, q_first + 32 * qb, a.Nq, lane);
-    const int qi = q_first + 32 * qb + lr;
     if (qi < a.Nq && g == 0) a.lse[tq0 + qi] = (a_i[qb] * m_ref[qb] + __log2f(l_tot)) * kLn2;
   });
 #endif
@@ -408,17 +422,22 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
 
 template <typename T, int D, int QB> static int launch_wide(FwdArgs a, int64_t BH, bool causal, hipStream_t st) {
   a.mblocks = (a.Nq + 128 * QB - 1) / (128 * QB);
-  const int64_t total = (int64_t)a.mblocks * BH;
+  const int64_t total = (int64_t)a.mblocks * BH * a.splits;
   if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_fwd: too many query blocks for one launch");
   a.total_blocks = (int)total;
   a.blocks_per_xcd = (a.total_blocks + 7) / 8;
   const dim3 grid((unsigned)(a.blocks_per_xcd * 8));
   if constexpr (D == 256) {
-    if (causal) fwd_wide_kernel<T, D, QB, true><<<grid, dim3(256), 0, st>>>(a);
-    else fwd_wide_kernel<T, D, QB, false><<<grid, dim3(256), 0, st>>>(a);
+    if (a.splits > 1) {
+      if (causal) fwd_wide_kernel<T, D, QB, true, true><<<grid, dim3(256), 0, st>>>(a);
+      else fwd_wide_kernel<T, D, QB, false, true><<<grid, dim3(256), 0, st>>>(a);
+      return check_launch("qfa_attn_fwd");
+    }
+    if (causal) fwd_wide_kernel<T, D, QB, true, false><<<grid, dim3(256), 0, st>>>(a);
+    else fwd_wide_kernel<T, D, QB, false, false><<<grid, dim3(256), 0, st>>>(a);
   } else {
     if (causal) return set_error(QFA_EUNSUPPORTED, "attn_fwd: no wide kernel for a mask at this head_dim");
-    fwd_wide_kernel<T, D, QB, false><<<grid, dim3(256), 0, st>>>(a);
+    fwd_wide_kernel<T, D, QB, false, false><<<grid, dim3(256), 0, st>>>(a);
   }
   return check_launch("qfa_attn_fwd");
 }

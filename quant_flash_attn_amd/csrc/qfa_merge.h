@@ -1,11 +1,14 @@
-// Merge of the partial results of an attention whose keys are split over workgroups (shared-KV forward, cache decode).
+// Merge of the partial results of an attention whose keys are split over workgroups (shared-KV and INT8-score forward, cache decode).
 #pragma once
+#include <cfloat>
+
 #include "qfa_device.h"
 #include "qfa_host.h"
 
 namespace qfa {
 
-// row maximum of a wave or split that saw no key: finite, so that differences of two of them are zero and not NaN
+// row maximum of a wave or split that saw no key: finite, so that differences of two of them are zero and not NaN (a
+// split may also leave -inf: the merges start from the lowest finite value)
 constexpr float NO_KEY = -1e30f;
 
 // four consecutive outputs of a row, rounded to the queries' type
@@ -26,7 +29,19 @@ struct SplitMergeArgs {
   float *lse;              // nullable, [B*H*Nq]
   int64_t H, sob, soh, son;
   int Nq, splits, o_dtype;
+  float *o32;   // nullable: O in fp32, dense; then o is nullable too
 };
+
+// one row's columns d .. d + 3, normalised, to where they go
+__device__ __forceinline__ void merge_store(const SplitMergeArgs &a, int64_t row, int D, int d, const f32x4 &acc, float m, float l) {
+  const float inv = 1.0f / l;
+  const f32x4 x = {acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+  if (a.lse && d == 0) a.lse[row] = (m + __log2f(l)) * kLn2;
+  if (a.o32) *reinterpret_cast<f32x4 *>(a.o32 + row * D + d) = x;
+  if (!a.o) return;
+  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
+  store4(static_cast<char *>(a.o) + off * (a.o_dtype == QFA_F32 ? 4 : 2), a.o_dtype, d, x);
+}
 
 // O of one query from the partial results of its splits: one workgroup per query, D/4 lanes of four columns times
 // 1024/D groups of splits.  All loads of a thread are independent, so the kernel is one memory latency long.
@@ -35,7 +50,7 @@ template <int D> __global__ __launch_bounds__(256) void split_merge_kernel(Split
   __shared__ float red[SG][D + 4];
   const int tid = threadIdx.x, d = 4 * (tid % CL), sg = tid / CL;
   const int64_t row = blockIdx.x, slot = row * a.splits;
-  float m = NO_KEY, l = 0.f;
+  float m = -FLT_MAX, l = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = sg; s < a.splits; s += SG) {
@@ -54,7 +69,7 @@ template <int D> __global__ __launch_bounds__(256) void split_merge_kernel(Split
   }
   __syncthreads();
   if (sg > 0) return;
-  float ma = NO_KEY, la = 0.f;
+  float ma = -FLT_MAX, la = 0.f;
 #pragma unroll
   for (int s = 0; s < SG; ++s) ma = fmaxf(ma, red[s][D]);
   acc = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -66,11 +81,7 @@ template <int D> __global__ __launch_bounds__(256) void split_merge_kernel(Split
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] += y[e] * w;
   }
-  const float inv = 1.0f / la;
-  if (a.lse && d == 0) a.lse[row] = (ma + __log2f(la)) * kLn2;
-  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
-  store4(static_cast<char *>(a.o) + off * (a.o_dtype == QFA_F32 ? 4 : 2), a.o_dtype, d,
-         f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+  merge_store(a, row, D, d, acc, ma, la);
 }
 
 // The same for few splits: D/4 lanes per query, 1024/D queries per workgroup.  A workgroup per query is as many workgroups
@@ -81,7 +92,7 @@ template <int D> __global__ __launch_bounds__(256) void split_merge_few_kernel(S
   const int d = 4 * (threadIdx.x % CL);
   const int64_t row = (int64_t)blockIdx.x * RPW + threadIdx.x / CL, slot = row * a.splits;
   if (row >= rows) return;
-  float m = NO_KEY, l = 0.f;
+  float m = -FLT_MAX, l = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = 0; s < a.splits; ++s) {
@@ -93,11 +104,7 @@ template <int D> __global__ __launch_bounds__(256) void split_merge_few_kernel(S
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = acc[e] * s0 + y[e] * s1;
   }
-  const float inv = 1.0f / l;
-  if (a.lse && d == 0) a.lse[row] = (m + __log2f(l)) * kLn2;
-  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
-  store4(static_cast<char *>(a.o) + off * (a.o_dtype == QFA_F32 ? 4 : 2), a.o_dtype, d,
-         f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+  merge_store(a, row, D, d, acc, m, l);
 }
 
 inline int64_t split_partial_bytes(int64_t rows, int64_t splits, int D) { return rows * splits * (int64_t)(D + 2) * 4; }

@@ -371,7 +371,7 @@ template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const Skv
   skv_fwd_kernel<T, S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_shared_kv")) return e;
   if (a.splits > 1) {
-    const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, x.io_dtype};
+    const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, x.io_dtype, nullptr};
     return launch_split_merge<D>(m, x.B * x.H * x.Nq, "qfa_attn_fwd_shared_kv (merge)", st);
   }
   return 0;

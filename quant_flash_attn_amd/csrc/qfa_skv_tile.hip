@@ -577,7 +577,7 @@ template <int D> static int launch_fwd_d(const SkvAttnArgs &x, const SkvTilePlan
   else skv_tile_fwd_kernel<D, 2><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_shared_kv")) return e;
   if (a.splits > 1) {
-    const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, x.io_dtype};
+    const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, x.io_dtype, nullptr};
     return launch_split_merge<D>(m, rows, "qfa_attn_fwd_shared_kv (merge)", st);
   }
   return 0;

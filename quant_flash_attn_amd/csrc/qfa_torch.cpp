@@ -34,7 +34,8 @@ struct Api {
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
   QFA_ENTRY(qfa_attn_fwd);
-  QFA_ENTRY(qfa_attn_fwd_f32);
+  QFA_ENTRY(qfa_attn_fwd_split_workspace_bytes);
+  QFA_ENTRY(qfa_attn_fwd_split);
   QFA_ENTRY(qfa_bench_qk_stage);
   QFA_ENTRY(qfa_attn_bwd_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd);
@@ -65,7 +66,8 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
   QFA_ENTRY(qfa_attn_fwd);
-  QFA_ENTRY(qfa_attn_fwd_f32);
+  QFA_ENTRY(qfa_attn_fwd_split_workspace_bytes);
+  QFA_ENTRY(qfa_attn_fwd_split);
   QFA_ENTRY(qfa_bench_qk_stage);
   QFA_ENTRY(qfa_attn_bwd_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd);
@@ -290,6 +292,21 @@ void fwd_into(const Quantized &q, const Quantized &k, const Tensor &v, const Ten
         qk_only ? "qfa_bench_qk_stage" : "qfa_attn_fwd");
 }
 
+// the same with the keys split over workgroups where there are few queries; o32 dense, o or o32 may be undefined
+void fwd_split_into(const Quantized &q, const Quantized &k, const Tensor &v, const Tensor &o, const Tensor &o32, float *lse,
+                    bool causal, double sm) {
+  const int64_t ws_bytes = api.qfa_attn_fwd_split_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D, causal);
+  Tensor ws;
+  if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, v);
+  const Tensor &like = o.defined() ? o : o32;
+  check(api.qfa_attn_fwd_split(q.codes, q.scale, q.zp, q.rowsum, k.codes, k.scale, k.zp, k.rowsum, v.data_ptr(),
+                               o.defined() ? o.data_ptr() : nullptr, o32.defined() ? o32.data_ptr<float>() : nullptr, lse,
+                               dtype_code(v.scalar_type()), q.B, q.H, q.N, k.N, (int)q.D, q.sb, q.sh, q.sn, k.sb, k.sh, k.sn,
+                               QFA_STRIDES(v), QFA_STRIDES(like), (float)sm, causal, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
+                               stream_of(v)),
+        "qfa_attn_fwd_split");
+}
+
 using Grads = std::array<Tensor, 3>;
 // f32: dO comes and the gradients leave in fp32
 Grads bwd_of(const Quantized &q, const Quantized &k, const Tensor &v_in, const Tensor &o_in, const Tensor &do_in,
@@ -426,17 +443,13 @@ Kept qkv_forward(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, boo
           "qfa_quant_qkv_f32");
     r.o = empty({pb.B, pb.H, pb.N[0], pb.D}, at::kFloat, q);
     if (keep) r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, at::kBFloat16, q);
-    check(api.qfa_attn_fwd_f32(a.codes, a.scale, a.zp, a.rowsum, b.codes, b.scale, b.zp, b.rowsum, r.v16.data_ptr(),
-                               r.o.data_ptr<float>(), keep ? r.o16.data_ptr() : nullptr, pb.lse_of(r.buf), QFA_BF16, a.B, a.H, a.N,
-                               b.N, (int)a.D, a.sb, a.sh, a.sn, b.sb, b.sh, b.sn, QFA_STRIDES(r.v16), QFA_STRIDES(r.o), (float)sm,
-                               causal, stream_of(q)),
-          "qfa_attn_fwd_f32");
+    fwd_split_into(a, b, r.v16, r.o16, r.o, pb.lse_of(r.buf), causal, sm);
     return r;
   }
   quantize_pair_into(q, k, pb.view(r.buf, 0), pb.view(r.buf, 1));
   r.v16 = rows16(to(v_in, io_dtype(v_in)));
   r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, r.v16.scalar_type(), q);
-  fwd_into(pb.view(r.buf, 0), pb.view(r.buf, 1), r.v16, r.o16, pb.lse_of(r.buf), causal, sm);
+  fwd_split_into(pb.view(r.buf, 0), pb.view(r.buf, 1), r.v16, r.o16, Tensor(), pb.lse_of(r.buf), causal, sm);
   r.o = to(r.o16, q.scalar_type());
   return r;
 }
@@ -498,7 +511,7 @@ CacheKept cache_forward(const Tensor &q_in, const Tensor &kc, const Tensor &ks, 
   r.kr = rowsum(r.kc);
   r.v16 = dequant(vc, vs, vz, io_dtype(q));
   r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, r.v16.scalar_type(), q);
-  fwd_into(pb.view(r.buf, 0), keys_of(r.kc, r.ks, r.kz, r.kr), r.v16, r.o16, pb.lse_of(r.buf), causal, sm);
+  fwd_split_into(pb.view(r.buf, 0), keys_of(r.kc, r.ks, r.kz, r.kr), r.v16, r.o16, Tensor(), pb.lse_of(r.buf), causal, sm);
   r.o = to(r.o16, q.scalar_type());
   return r;
 }
