@@ -361,6 +361,13 @@ int qfa_attn_bwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const 
                  int64_t sdqn, int64_t sdkb, int64_t sdkh, int64_t sdkn, int64_t sdvb, int64_t sdvh,
                  int64_t sdvn, float sm_scale, int causal, void *stream);
 
+/*
+ * The workspace with which qfa_attn_bwd (f32: qfa_attn_bwd_f32) may split its work further where B*H and the sequence alone
+ * leave CUs idle: the queries of dK and dV, and the keys of dQ, are dealt to several workgroups, whose fp32 parts lie behind
+ * what the plain call needs and are added by a third small kernel.  The same number where no split pays.
+ */
+int64_t qfa_attn_bwd_split_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal, int f32);
+
 #ifdef __cplusplus
 }
 #endif

@@ -50,6 +50,7 @@ _SIGNATURES = {
     "qfa_dout_normalise": (c_int, [_P, _I, _L, _P, _I, _L, _P, _P, _P, _P]),
     "qfa_bwd_delta": (c_int, [_P, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_attn_bwd_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
+    "qfa_attn_bwd_split_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I, _I, _I]),
     "qfa_attn_bwd_f32_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
     "qfa_attn_bwd_f32": (c_int, [_P] * 13 + [_L] + [_P] * 3 + [_I, _L, _L, _L, _L, _I] + [_L] * 24 + [_F, _I, _P]),
     "qfa_attn_bwd": (c_int, [_P] * 13 + [_L] + [_P] * 3 + [_I, _L, _L, _L, _L, _I] + [_L] * 24 + [_F, _I, _P]),

@@ -33,7 +33,7 @@ BY_HAND = ("qfa_fwd_wide.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip")
 PER_FILE["qfa_skv_tile.hip"] = PER_FILE["qfa_skv_dkv.hip"] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]   # head_dim 256: 26 registers spilled instead of 177
 for _f in BY_HAND:
     PER_FILE[_f] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_fwd_wide.hip", "qfa_fwd_plan.cpp", "qfa_bwd.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv_plan.cpp", "qfa_skv.hip", "qfa_skv_tile.hip", "qfa_skv_dkv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
+SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_fwd_wide.hip", "qfa_split_plan.cpp", "qfa_bwd.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv_plan.cpp", "qfa_skv.hip", "qfa_skv_tile.hip", "qfa_skv_dkv.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
            "qfa_cache.hip"]
 
 

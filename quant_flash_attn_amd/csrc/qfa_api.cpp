@@ -483,6 +483,8 @@ static int attn_bwd(const char *who, int f32, const int8_t *qc, const float *sq,
   if (!strides_ok(sdob, sdoh, sdon, D, es) || !strides_ok(sdqb, sdqh, sdqn, D, es) ||
       !strides_ok(sdkb, sdkh, sdkn, D, es) || !strides_ok(sdvb, sdvh, sdvn, D, es))
     return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
+  const int64_t parts = bwd_split_bytes(B, H, Nq, Nk, D, causal);
+  a.may_split = parts > 0 && workspace_bytes - need >= parts;
   return launch_bwd(a, (hipStream_t)stream);
 }
 
@@ -498,6 +500,11 @@ int qfa_attn_bwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
   return attn_bwd("attn_bwd", 0, qc, sq, zq, rq, kc, sk, zk, rk, v, o, dout, lse, workspace, workspace_bytes, dq, dk, dv, io_dtype, B, H, Nq, Nk, D, sqb, sqh, sqn,
                   skb, skh, skn, svb, svh, svn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn, sdvb, sdvh, sdvn,
                   sm_scale, causal, stream);
+}
+
+int64_t qfa_attn_bwd_split_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal, int f32) {
+  const int64_t need = f32 ? qfa_attn_bwd_f32_workspace_bytes(B, H, Nq, Nk, D) : qfa_attn_bwd_workspace_bytes(B, H, Nq, Nk, D);
+  return need > 0 ? need + bwd_split_bytes(B, H, Nq, Nk, D, causal) : 0;
 }
 
 int64_t qfa_attn_bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {

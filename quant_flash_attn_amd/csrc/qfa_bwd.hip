@@ -35,7 +35,7 @@ template <typename T, int D> __global__ __launch_bounds__(256) void delta_kernel
   constexpr int TPP = 256 / LPT;
   const int tid = threadIdx.x, sub = tid % LPT;
   const int64_t bh = blockIdx.x / a.chunks_per_bh, chunk = blockIdx.x % a.chunks_per_bh;
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int64_t n = chunk * (int64_t)TPP + tid / LPT;
   const int64_t nn = n < a.N ? n : a.N - 1;
   const u32x4 ow = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const T *>(a.o) + b * a.sob + h * a.soh +
@@ -152,7 +152,7 @@ template <typename T, int D> __device__ __forceinline__ void prep_q(const BwdArg
   constexpr int BWD_TILE = WS::TILE;
   const int tid = threadIdx.x;
   const int bh = blk / a.tiles_q, tile = blk % a.tiles_q;
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int i0 = tile * BWD_TILE;
   const int64_t tq0 = (int64_t)bh * a.Nq;
   unsigned char *blob = a.ws_q + ((int64_t)bh * a.tiles_q + tile) * WS::Q_BLOB;
@@ -162,20 +162,27 @@ template <typename T, int D> __device__ __forceinline__ void prep_q(const BwdArg
     const T *do_bh = reinterpret_cast<const T *>(a.dout) + b * a.sdob + h * a.sdoh;
     const T *o_bh = reinterpret_cast<const T *>(a.o) + b * a.sob + h * a.soh;
     u32x2 creg[4];
+    u32x4 greg[4];
     float zreg[4], sreg[4];
+    if (a.dout32) {   // (outside the loop below, whose loads go out together)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = min(i0 + 4 * r4 + r, a.Nq - 1);
+        const f32x4 *g32 = reinterpret_cast<const f32x4 *>(a.dout32 + b * a.sd32b + h * a.sd32h + (int64_t)i * a.sd32n + dc * 8);
+        const f32x4 x = g32[0], y = g32[1];
+        greg[r] = u32x4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
+        if (i0 + 4 * r4 + r < a.Nq) *reinterpret_cast<u32x4 *>(reinterpret_cast<T *>(a.do16) + (tq0 + i) * D + dc * 8) = greg[r];
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        greg[r] = *reinterpret_cast<const u32x4 *>(do_bh + (int64_t)min(i0 + 4 * r4 + r, a.Nq - 1) * a.sdon + dc * 8);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = min(i0 + 4 * r4 + r, a.Nq - 1);
       creg[r] = *reinterpret_cast<const u32x2 *>(qc_bh + (int64_t)i * a.sqn + dc * 8);
-      u32x4 gw;
-      if (a.dout32) {
-        const f32x4 *g32 = reinterpret_cast<const f32x4 *>(a.dout32 + b * a.sd32b + h * a.sd32h + (int64_t)i * a.sd32n + dc * 8);
-        const f32x4 x = g32[0], y = g32[1];
-        gw = u32x4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3])};
-        if (i0 + 4 * r4 + r < a.Nq) *reinterpret_cast<u32x4 *>(reinterpret_cast<T *>(a.do16) + (tq0 + i) * D + dc * 8) = gw;
-      } else {
-        gw = *reinterpret_cast<const u32x4 *>(do_bh + (int64_t)i * a.sdon + dc * 8);
-      }
+      const u32x4 gw = greg[r];
       const u32x4 ow = *reinterpret_cast<const u32x4 *>(o_bh + (int64_t)i * a.son + dc * 8);
       zreg[r] = (float)a.zq[tq0 + i];
       sreg[r] = a.sq[tq0 + i];
@@ -217,7 +224,7 @@ template <typename T, int D> __device__ __forceinline__ void prep_k(const BwdArg
   constexpr int BWD_TILE = WS::TILE;
   const int tid = threadIdx.x;
   const int bh = blk / a.tiles_k, tile = blk % a.tiles_k;
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int j0 = tile * BWD_TILE;
   const int64_t tk0 = (int64_t)bh * a.Nk;
   unsigned char *blob = a.ws_k + ((int64_t)bh * a.tiles_k + tile) * WS::K_BLOB;
@@ -259,6 +266,36 @@ template <typename T, int D> __global__ __launch_bounds__(256) void bwd_prep_ker
   else prep_k<T, D>(a, blk - blocks_q, sm);
 }
 
+// ------------------------------------------------------------------------------------------ sum of parts
+// Gradients whose streamed rows were split: up to three tensors, each [B*H][splits][N][D] in fp32, added in the order of the
+// parts and rounded once.  Bound by memory.
+struct BwdSumArgs {
+  struct One { const float *part; void *out; int64_t sb, sh, sn, rows; int N, splits, first_block; } t[3];
+  int64_t H;
+  int count, out_f32;
+};
+template <typename T, int D> __global__ __launch_bounds__(256) void bwd_sum_kernel(BwdSumArgs a) {
+  constexpr int CL = D / 4, RPW = 256 / CL;   // four columns of a row per thread
+  int i = 0;
+  while (i + 1 < a.count && (int)blockIdx.x >= a.t[i + 1].first_block) ++i;
+  const BwdSumArgs::One &x = a.t[i];
+  const int64_t row = (int64_t)((int)blockIdx.x - x.first_block) * RPW + threadIdx.x / CL;   // of B*H*N
+  const int d = 4 * (threadIdx.x % CL);
+  if (row >= x.rows) return;
+  const int64_t bh = index_div(row, x.N), n = row - bh * x.N, step = (int64_t)x.N * D, b = index_div(bh, a.H), h = bh - b * a.H;
+  const float *p = x.part + bh * x.splits * step + n * D + d;
+  f32x4 acc = *reinterpret_cast<const f32x4 *>(p);
+#pragma unroll 4
+  for (int s = 1; s < x.splits; ++s) {
+    const f32x4 y = *reinterpret_cast<const f32x4 *>(p + s * step);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += y[e];
+  }
+  const int64_t at = b * x.sb + h * x.sh + n * x.sn + d;
+  if (a.out_f32) *reinterpret_cast<f32x4 *>(static_cast<float *>(x.out) + at) = acc;
+  else *reinterpret_cast<u32x2 *>(static_cast<T *>(x.out) + at) = u32x2{pack2<T>(acc[0], acc[1]), pack2<T>(acc[2], acc[3])};
+}
+
 template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStream_t st) {
   typedef BwdWs<D> WS;
   BwdArgs a;
@@ -288,9 +325,44 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
     return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many tiles for one launch");
   bwd_prep_kernel<T, D><<<dim3((unsigned)(BH * (a.tiles_q + a.tiles_k))), dim3(256), 0, st>>>(a, (int)(BH * a.tiles_q));
   if (int e = check_launch("qfa_attn_bwd (staging)")) return e;
-  // dK, dV
-  if (int e = launch_dkv<T, D>(a, BH, x.causal, st)) return e;
-  return launch_dq<T, D>(a, BH, x.causal, st);
+  const BwdPlan plan = bwd_plan(BH, x.Nq, x.Nk, D, x.causal, x.may_split);
+  float *part = reinterpret_cast<float *>(a.ws_q + (x.f32 ? bwd_f32_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)
+                                                         : bwd_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)));
+  BwdSumArgs sum;
+  sum.count = 0; sum.H = x.H; sum.out_f32 = x.f32;
+  int64_t blocks = 0;
+  // the split gradient of N rows: where its parts go, and what adds them
+  auto split = [&](void *&out, int64_t &sb, int64_t &sh, int64_t &sn, int64_t N, int splits) {
+    sum.t[sum.count++] = {part, out, sb, sh, sn, BH * N, (int)N, splits, (int)blocks};
+    blocks += (BH * N + 1024 / D - 1) / (1024 / D);
+    out = part;
+    sn = D; sh = splits * N * D; sb = x.H * sh;
+    part += BH * splits * N * D;
+  };
+  BwdArgs k = a;   // dK, dV
+  k.per_split = plan.queries_per_split;
+  k.last_part = (plan.splits_dkv - 1) * plan.queries_per_split;
+  k.split_stride = 0;
+  if (plan.splits_dkv > 1) {
+    split(k.dk, k.sdkb, k.sdkh, k.sdkn, x.Nk, plan.splits_dkv);
+    split(k.dv, k.sdvb, k.sdvh, k.sdvn, x.Nk, plan.splits_dkv);
+    k.split_stride = x.Nk * D;
+    k.grad_f32 = 1;
+  }
+  if (int e = launch_dkv<T, D>(k, BH, x.causal, plan.blocks_dkv, plan.splits_dkv, st)) return e;
+  BwdArgs q = a;
+  q.per_split = plan.keys_per_split;
+  q.last_part = (plan.splits_dq - 1) * plan.keys_per_split;
+  q.split_stride = 0;
+  if (plan.splits_dq > 1) {
+    split(q.dq, q.sdqb, q.sdqh, q.sdqn, x.Nq, plan.splits_dq);
+    q.split_stride = x.Nq * D;
+    q.grad_f32 = 1;
+  }
+  if (int e = launch_dq<T, D>(q, BH, x.causal, plan.blocks_dq, plan.splits_dq, st)) return e;
+  if (sum.count == 0) return 0;
+  bwd_sum_kernel<T, D><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sum);
+  return check_launch("qfa_attn_bwd (sum)");
 }
 
 int launch_bwd(const AttnArgs &x, hipStream_t st) {

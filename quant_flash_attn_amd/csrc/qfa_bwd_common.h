@@ -38,6 +38,9 @@ struct BwdArgs {
   void *do16;
   int64_t sd32b, sd32h, sd32n;
   int grad_f32;         // dQ, dK, dV are fp32
+  int per_split;        // streamed rows per part (a multiple of 64), part blockIdx.y; all of them in one where not split
+  int last_part;        // first row of the last part
+  int64_t split_stride; // fp32 elements from one part's gradients to the next's
   int group_log2;       // causal: log2 of the number of heads whose blocks are dispatched together (set per launch)
 };
 
@@ -97,7 +100,8 @@ template <int T_BYTES, int C_COPY> struct BlobCopy {
   }
 };
 
-template <typename T, int D> int launch_dkv(BwdArgs a, int64_t BH, bool causal, hipStream_t st);
-template <typename T, int D> int launch_dq(BwdArgs a, int64_t BH, bool causal, hipStream_t st);
+// blocks: 32-row blocks per wave (2 only at head_dim 128); splits: parts of the streamed rows (grid.y)
+template <typename T, int D> int launch_dkv(BwdArgs a, int64_t BH, bool causal, int blocks, int splits, hipStream_t st);
+template <typename T, int D> int launch_dq(BwdArgs a, int64_t BH, bool causal, int blocks, int splits, hipStream_t st);
 
 }  // namespace qfa

@@ -67,22 +67,25 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
       nbk = idx >> GL;
     }
   }
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
+  // this workgroup's queries: q0 .. q0 + Nq - 1, a sequence of its own whose mask is shifted (late ones first: causal, they see
+  // the most keys)
+  const int q0 = a.last_part - (int)blockIdx.y * a.per_split, Nq = min(a.per_split, a.Nq - q0);
   const int n0 = nbk * 4 * KEYS;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int k_first = n0 + wave * KEYS;
 
-  const unsigned char *qc_bh = reinterpret_cast<const unsigned char *>(a.qc + b * a.sqb + h * a.sqh);
+  const unsigned char *qc_bh = reinterpret_cast<const unsigned char *>(a.qc + b * a.sqb + h * a.sqh + q0 * a.sqn);
   const int8_t *kc_bh = a.kc + b * a.skb + h * a.skh;
   const T *v_bh = reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh;
-  const unsigned char *do_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.dout) + b * a.sdob + h * a.sdoh);
+  const unsigned char *do_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.dout) + b * a.sdob + h * a.sdoh + q0 * a.sdon);
   const unsigned char *wsk_bh = a.ws_k + (int64_t)bh * a.tiles_k * WS::K_BLOB;
-  const unsigned char *wsq_bh = a.ws_q + (int64_t)bh * a.tiles_q * WS::Q_BLOB;
+  const unsigned char *wsq_bh = a.ws_q + ((int64_t)bh * a.tiles_q + q0 / TILE) * WS::Q_BLOB;
 
-  const int coff = CAUSAL ? a.Nk - a.Nq : 0;   // causal: key j is seen by the queries i >= j - coff
+  const int coff = CAUSAL ? a.Nk - a.Nq + q0 : 0;   // causal: key j is seen by the queries i >= j - coff
   const int it0 = CAUSAL ? max(n0 - coff, 0) / TILE : 0;
-  const int ntiles = a.tiles_q;
+  const int ntiles = (Nq + TILE - 1) / TILE;
 
   // ---- tile copies (direct to LDS)
   typedef SlabCopy<TILE, KS> CopyQ;
@@ -93,7 +96,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
   constexpr int PIECES = CopyQ::N + CopyDo::N + CopyB::N;
   struct TileDesc { rsrc_t q, g, b; unsigned char *dst; };
   auto tile_desc = [&](int t) __attribute__((always_inline)) -> TileDesc {
-    const int rows = min(TILE, a.Nq - TILE * t);
+    const int rows = min(TILE, Nq - TILE * t);
     return {cp_q.desc(qc_bh + (int64_t)t * TILE * a.sqn, rows), cp_do.desc(do_bh + (int64_t)t * TILE * a.sdon * 2, rows),
             make_rsrc(wsq_bh + (int64_t)t * WS::Q_BLOB, rows > 0 ? (unsigned)WS::Q_BLOB : 0u), smem + (t - it0) % 3 * SM::BUF};
   };
@@ -119,7 +122,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
     const int kj = k_first + 32 * kb + lr, kc = min(kj, a.Nk - 1);
-    q_lo[kb] = kj >= a.Nk ? 0x7fffffff : CAUSAL ? kj - (a.Nk - a.Nq) : 0;
+    q_lo[kb] = kj >= a.Nk ? 0x7fffffff : CAUSAL ? kj - coff : 0;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       kf[kb][ks] = *reinterpret_cast<const i32x4 *>(kc_bh + (int64_t)kc * a.skn + ks * 32 + g * 16);
@@ -206,8 +209,8 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
         x1 = __builtin_amdgcn_exp2f(x1);
         if constexpr (MASKED) {   // (no short circuit: a branch per element would end the block)
           const int q = i0 + 8 * aa + 2 * (x % 2);
-          x0 = ((q >= q_lo[kb]) & (q < a.Nq)) ? x0 : 0.f;
-          x1 = ((q + 1 >= q_lo[kb]) & (q + 1 < a.Nq)) ? x1 : 0.f;
+          x0 = ((q >= q_lo[kb]) & (q < Nq)) ? x0 : 0.f;
+          x1 = ((q + 1 >= q_lo[kb]) & (q + 1 < Nq)) ? x1 : 0.f;
         }
         f[kb][v] = x0;
         f[kb][v + 1] = x1;
@@ -362,6 +365,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
   const bool late = CAUSAL && KB == 1 && NSTEP == 2 && max(k_first - coff, 0) / 32 % 2 == 1;
   if (CAUSAL) ft = max(ft, max(k_first - coff, 0) / TILE);
   if (k_first >= a.Nk) ft = ntiles;
+  ft = min(ft, ntiles);   // (a part of the queries may hold none that sees the wave's keys)
   dma_wait();
   __syncthreads();
   int t = it0;
@@ -401,7 +405,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     };
     const int full0 = k_last >= a.Nk ? ntiles : CAUSAL ? max(k_last - coff + TILE - 1, 0) / TILE : 0;
     tiles(min(full0, ntiles), std::true_type{});
-    tiles(a.Nq / TILE, std::false_type{});
+    tiles(Nq / TILE, std::false_type{});
     tiles(ntiles, std::true_type{});
     static_for<2 * DB>([&](auto n_tag) __attribute__((always_inline)) {
       constexpr int n = decltype(n_tag)::value;
@@ -409,30 +413,42 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
       static_for<KB>([&](auto kb) __attribute__((always_inline)) { acc_mfma<T, decltype(kb)::value * DB + n % DB, ACC>(tq, ds[kb][n / DB]); });
     });
   }
+  // what only the epilogue needs is read and formed here: held in scalar registers through the loop it would push others out,
+  // and behind the barrier its latency would be seen
+  typedef __attribute__((address_space(4))) const BwdArgs KernArgs;
+  KernArgs *ep = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  int bh_ = bh;
+  asm volatile("" : "+s"(ep), "+s"(bh_));
+  const int64_t eb = index_div(bh_, ep->H), eh = bh_ - eb * ep->H;
+  void *dk = ep->dk, *dv = ep->dv;
+  int64_t dk_at = eb * ep->sdkb + eh * ep->sdkh + blockIdx.y * ep->split_stride,
+          dv_at = eb * ep->sdvb + eh * ep->sdvh + blockIdx.y * ep->split_stride, sdkn = ep->sdkn, sdvn = ep->sdvn;
+  float sm = ep->sm_scale;
+  int f32 = ep->grad_f32;
+  asm volatile("" : "+s"(dk), "+s"(dv), "+s"(dk_at), "+s"(dv_at), "+s"(sdkn), "+s"(sdvn), "+s"(sm), "+s"(f32));
   acc_settle();
   __syncthreads();   // the tile buffers are done with: the output stages overlay them
   static_assert(4 * 32 * 2 * D <= 3 * SM::BUF, "output staging fits the tile buffers");
   unsigned char *stage = smem + wave * (32 * 2 * D);
-  const int64_t dk_at = b * a.sdkb + h * a.sdkh, dv_at = b * a.sdvb + h * a.sdvh;
-  if (a.grad_f32) {
-    float *dk_bh = reinterpret_cast<float *>(a.dk) + dk_at, *dv_bh = reinterpret_cast<float *>(a.dv) + dv_at;
+  if (f32) {
+    float *dk_bh = reinterpret_cast<float *>(dk) + dk_at, *dv_bh = reinterpret_cast<float *>(dv) + dv_at;
     static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
       constexpr int kb = decltype(kb_tag)::value;
-      acc_store_rows_f32<D, kb * DB>(a.sm_scale, dk_bh, a.sdkn, k_first + 32 * kb, a.Nk, lane);
-      acc_store_rows_f32<D, DV0 + kb * DB>(1.0f, dv_bh, a.sdvn, k_first + 32 * kb, a.Nk, lane);
+      acc_store_rows_f32<D, kb * DB>(sm, dk_bh, sdkn, k_first + 32 * kb, a.Nk, lane);
+      acc_store_rows_f32<D, DV0 + kb * DB>(1.0f, dv_bh, sdvn, k_first + 32 * kb, a.Nk, lane);
     });
     return;
   }
-  T *dk_bh = reinterpret_cast<T *>(a.dk) + dk_at, *dv_bh = reinterpret_cast<T *>(a.dv) + dv_at;
+  T *dk_bh = reinterpret_cast<T *>(dk) + dk_at, *dv_bh = reinterpret_cast<T *>(dv) + dv_at;
   static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
     constexpr int kb = decltype(kb_tag)::value;
-    acc_store_rows<T, D, kb * DB>(a.sm_scale, stage, dk_bh, a.sdkn, k_first + 32 * kb, a.Nk, lane);
-    acc_store_rows<T, D, DV0 + kb * DB>(1.0f, stage, dv_bh, a.sdvn, k_first + 32 * kb, a.Nk, lane);
+    acc_store_rows<T, D, kb * DB>(sm, stage, dk_bh, sdkn, k_first + 32 * kb, a.Nk, lane);
+    acc_store_rows<T, D, DV0 + kb * DB>(1.0f, stage, dv_bh, sdvn, k_first + 32 * kb, a.Nk, lane);
   });
 #endif
 }
 
-template <typename T, int D, int KB> static int launch_dkv_kb(BwdArgs a, int64_t BH, bool causal, hipStream_t st) {
+template <typename T, int D, int KB> static int launch_dkv_kb(BwdArgs a, int64_t BH, bool causal, int splits, hipStream_t st) {
   a.nblocks = (a.Nk + 128 * KB - 1) / (128 * KB);
   // per head the kernel streams Qc, dO and Qz^T (5 bytes per query and d): group heads while that stays
   // within about 6 MB (pairs at N=4096, D=128: 5.2 MB against the XCD's 4 MB L2, measured 1 % better than
@@ -444,43 +460,25 @@ template <typename T, int D, int KB> static int launch_dkv_kb(BwdArgs a, int64_t
   if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many key blocks for one launch");
   a.total_blocks = (int)total;
   a.blocks_per_xcd = (a.total_blocks + 7) / 8;
-  const dim3 grid((unsigned)(a.blocks_per_xcd * 8));
+  const dim3 grid((unsigned)(a.blocks_per_xcd * 8), (unsigned)splits);
   if (causal) bwd_dkv_kernel<T, D, KB, true><<<grid, dim3(256), 0, st>>>(a);
   else bwd_dkv_kernel<T, D, KB, false><<<grid, dim3(256), 0, st>>>(a);
   return check_launch("qfa_attn_bwd (dk, dv)");
 }
 
-// Cost of a launch of workgroups of 128 * kb keys on 256 CUs, one per CU, in steps of 32 queries: whole rounds when all are
-// equally long; causal, the mean load and half of the longest, or the longest where all run at once (a tenth more, since the
-// mean of shorter ones fills in better than that).  `step`: cost of a step; starting and finishing a workgroup costs about
-// two.  Both kernels' variants timed for 16 to 1024 heads of 64 to 2048 tokens: the choice is within 5 % of the best but
-// for 128 heads of 768 (6 %); 256 heads of 200 and 256 causal tokens, the whole backward: 70 -> 66 and 74 -> 69 us with one
-// round of 256-row workgroups.
-static float dkv_cost(const BwdArgs &a, int64_t BH, bool causal, int kb, float step) {
-  const int64_t nb = (a.Nk + 128 * kb - 1) / (128 * kb);
-  const float steps = (float)((a.Nq + 31) / 32) * step, fix = 2.0f;
-  if (!causal) return (float)((nb * BH + 255) / 256) * (steps + fix);
-  if (nb * BH <= 256) return 1.1f * (steps + fix);
-  const float f = (float)a.Nq / (float)a.Nk;   // a head's triangle (trapezoid: few queries) of steps
-  const float sum = (float)(nb * BH) * (steps * (1.0f - 0.5f * f) + 2.0f * (float)kb * step + fix);
-  return sum / 256.0f + 0.5f * steps;
-}
-
-template <typename T, int D> int launch_dkv(BwdArgs a, int64_t BH, bool causal, hipStream_t st) {
+template <typename T, int D> int launch_dkv(BwdArgs a, int64_t BH, bool causal, int blocks, int splits, hipStream_t st) {
   if constexpr (D == 128) {
-    // 64 keys per wave need fewer LDS reads per key (a step of 32 costs 0.62 of one of 64 keys, measured); 32 keys fill the
-    // chip with twice the workgroups and waste less of the last one
-    if (dkv_cost(a, BH, causal, 1, 0.62f) >= dkv_cost(a, BH, causal, 2, 1.0f)) return launch_dkv_kb<T, D, 2>(a, BH, causal, st);
+    if (blocks == 2) return launch_dkv_kb<T, D, 2>(a, BH, causal, splits, st);
   }
   // (head_dim 256: the registers hold the operands and accumulators of 32 keys; head_dim 64: of 32 keys in two waves per
   // SIMD, which share the issue slots better than one wave of 64 keys: 3 - 10 % faster, 20 % when the chip is not full)
-  return launch_dkv_kb<T, D, 1>(a, BH, causal, st);
+  return launch_dkv_kb<T, D, 1>(a, BH, causal, splits, st);
 }
-template int launch_dkv<__bf16, 64>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dkv<__bf16, 128>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dkv<__bf16, 256>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dkv<_Float16, 64>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dkv<_Float16, 128>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dkv<_Float16, 256>(BwdArgs, int64_t, bool, hipStream_t);
+template int launch_dkv<__bf16, 64>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dkv<__bf16, 128>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dkv<__bf16, 256>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dkv<_Float16, 64>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dkv<_Float16, 128>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dkv<_Float16, 256>(BwdArgs, int64_t, bool, int, int, hipStream_t);
 
 }  // namespace qfa

@@ -61,22 +61,24 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
     }
     mb = a.nblocks - 1 - mb;
   }
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
+  // this workgroup's keys: key0 .. key0 + Nk - 1, a sequence of its own whose mask is shifted
+  const int key0 = blockIdx.y * a.per_split, Nk = min(a.per_split, a.Nk - key0);
   const int m0 = mb * 4 * QUERIES;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int q_first = m0 + wave * QUERIES;
 
   const int8_t *qc_bh = a.qc + b * a.sqb + h * a.sqh;
-  const unsigned char *kc_bh = reinterpret_cast<const unsigned char *>(a.kc + b * a.skb + h * a.skh);
-  const unsigned char *v_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh);
+  const unsigned char *kc_bh = reinterpret_cast<const unsigned char *>(a.kc + b * a.skb + h * a.skh + key0 * a.skn);
+  const unsigned char *v_bh = reinterpret_cast<const unsigned char *>(reinterpret_cast<const T *>(a.v) + b * a.svb + h * a.svh + key0 * a.svn);
   const T *do_bh = reinterpret_cast<const T *>(a.dout) + b * a.sdob + h * a.sdoh;
-  const unsigned char *wsk_bh = a.ws_k + (int64_t)bh * a.tiles_k * WS::K_BLOB;
+  const unsigned char *wsk_bh = a.ws_k + ((int64_t)bh * a.tiles_k + key0 / TILE) * WS::K_BLOB;
   const unsigned char *wsq_bh = a.ws_q + (int64_t)bh * a.tiles_q * WS::Q_BLOB;
 
-  const int coff = CAUSAL ? a.Nk - a.Nq : 0;   // causal: query i keeps keys j <= i + coff (mask aligned to the last key)
-  const int ntiles = ((CAUSAL ? min(a.Nk, m0 + 4 * QUERIES + coff) : a.Nk) + TILE - 1) / TILE;
-  const int wtiles = q_first >= a.Nq ? 0 : ((CAUSAL ? min(a.Nk, q_first + QUERIES + coff) : a.Nk) + TILE - 1) / TILE;
+  const int coff = CAUSAL ? a.Nk - a.Nq - key0 : 0;   // causal: query i keeps keys j <= i + coff (mask aligned to the last key)
+  const int ntiles = ((CAUSAL ? min(Nk, m0 + 4 * QUERIES + coff) : Nk) + TILE - 1) / TILE;
+  const int wtiles = q_first >= a.Nq ? 0 : ((CAUSAL ? min(Nk, q_first + QUERIES + coff) : Nk) + TILE - 1) / TILE;
 
   // ---- tile copies (direct to LDS)
   typedef SlabCopy<TILE, KS> CopyK;
@@ -87,7 +89,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   constexpr int PIECES = CopyK::N + CopyV::N + CopyB::N;
   struct TileDesc { rsrc_t k, v, b; unsigned char *dst; };
   auto tile_desc = [&](int t) __attribute__((always_inline)) -> TileDesc {
-    const int rows = t < ntiles ? min(TILE, a.Nk - TILE * t) : 0;
+    const int rows = t < ntiles ? min(TILE, Nk - TILE * t) : 0;
     return {cp_k.desc(kc_bh + (int64_t)t * TILE * a.skn, rows), cp_v.desc(v_bh + (int64_t)t * TILE * a.svn * 2, rows),
             make_rsrc(wsk_bh + (int64_t)t * WS::K_BLOB, rows > 0 ? (unsigned)WS::K_BLOB : 0u), smem + t % 3 * SM::BUF};
   };
@@ -114,7 +116,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const int qi = q_first + 32 * qb + lr, qc = min(qi, a.Nq - 1);
-    k_hi[qb] = CAUSAL ? min(qc + coff, a.Nk - 1) : a.Nk - 1;
+    k_hi[qb] = CAUSAL ? min(qc + coff, Nk - 1) : Nk - 1;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[qb][ks] = *reinterpret_cast<const i32x4 *>(qc_bh + (int64_t)qc * a.sqn + ks * 32 + g * 16);
@@ -321,7 +323,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
         nbuf = b2;
       }
     };
-    tiles(min(wtiles, min(a.Nk / TILE, CAUSAL ? (q_first + coff + 1) / TILE : wtiles)), std::false_type{});
+    tiles(min(wtiles, min(Nk / TILE, CAUSAL ? (q_first + coff + 1) / TILE : wtiles)), std::false_type{});
     tiles(wtiles, std::true_type{});
     static_for<NX>([&](auto n_tag) __attribute__((always_inline)) {
       constexpr int n = decltype(n_tag)::value;
@@ -334,27 +336,39 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
     lds_barrier();
     copy_tile(t + 2);
   }
+  // what only the epilogue needs is read and formed here: held in scalar registers through the loop it would push others out,
+  // and behind the barrier its latency would be seen
+  typedef __attribute__((address_space(4))) const BwdArgs KernArgs;
+  KernArgs *ep = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  int bh_ = bh;
+  asm volatile("" : "+s"(ep), "+s"(bh_));
+  const int64_t eb = index_div(bh_, ep->H), eh = bh_ - eb * ep->H;
+  void *dq = ep->dq;
+  int64_t dq_at = eb * ep->sdqb + eh * ep->sdqh + blockIdx.y * ep->split_stride, sdqn = ep->sdqn;
+  float sm = ep->sm_scale;
+  int f32 = ep->grad_f32;
+  asm volatile("" : "+s"(dq), "+s"(dq_at), "+s"(sdqn), "+s"(sm), "+s"(f32));
   acc_settle();
   __syncthreads();   // the tile buffers are done with: the output stages overlay them
   static_assert(4 * 32 * 2 * D <= 3 * SM::BUF, "output staging fits the tile buffers");
   unsigned char *stage = smem + wave * (32 * 2 * D);
-  if (a.grad_f32) {
-    float *dq_bh = reinterpret_cast<float *>(a.dq) + b * a.sdqb + h * a.sdqh;
+  if (f32) {
+    float *dq_bh = reinterpret_cast<float *>(dq) + dq_at;
     static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
       constexpr int qb = decltype(qb_tag)::value;
-      acc_store_rows_f32<D, qb * DB>(a.sm_scale, dq_bh, a.sdqn, q_first + 32 * qb, a.Nq, lane);
+      acc_store_rows_f32<D, qb * DB>(sm, dq_bh, sdqn, q_first + 32 * qb, a.Nq, lane);
     });
     return;
   }
-  T *dq_bh = reinterpret_cast<T *>(a.dq) + b * a.sdqb + h * a.sdqh;
+  T *dq_bh = reinterpret_cast<T *>(dq) + dq_at;
   static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
     constexpr int qb = decltype(qb_tag)::value;
-    acc_store_rows<T, D, qb * DB>(a.sm_scale, stage, dq_bh, a.sdqn, q_first + 32 * qb, a.Nq, lane);
+    acc_store_rows<T, D, qb * DB>(sm, stage, dq_bh, sdqn, q_first + 32 * qb, a.Nq, lane);
   });
 #endif
 }
 
-template <typename T, int D, int QB> static int launch_dq_qb(BwdArgs a, int64_t BH, bool causal, hipStream_t st) {
+template <typename T, int D, int QB> static int launch_dq_qb(BwdArgs a, int64_t BH, bool causal, int splits, hipStream_t st) {
   a.nblocks = (a.Nq + 128 * QB - 1) / (128 * QB);
   // per head the kernel streams Kc, V and Kz^T (5 bytes per key and d): two to eight heads together, within
   // about 6 MB (pairs at N=4096, D=128, measured)
@@ -365,42 +379,23 @@ template <typename T, int D, int QB> static int launch_dq_qb(BwdArgs a, int64_t 
   if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many query blocks for one launch");
   a.total_blocks = (int)total;
   a.blocks_per_xcd = (a.total_blocks + 7) / 8;
-  const dim3 grid((unsigned)(a.blocks_per_xcd * 8));
+  const dim3 grid((unsigned)(a.blocks_per_xcd * 8), (unsigned)splits);
   if (causal) bwd_dq_kernel<T, D, QB, true><<<grid, dim3(256), 0, st>>>(a);
   else bwd_dq_kernel<T, D, QB, false><<<grid, dim3(256), 0, st>>>(a);
   return check_launch("qfa_attn_bwd (dq)");
 }
 
-// Cost of a launch of workgroups of 128 * qb queries on 256 CUs, one per CU, in steps of 32 keys: whole rounds when all are
-// equally long; causal, the mean load and half of the longest, or the longest where all run at once (a tenth more, since the
-// mean of shorter ones fills in better than that).  `step`: cost of a step; starting and finishing a workgroup costs about
-// two.  Both kernels' variants timed for 16 to 1024 heads of 64 to 2048 tokens: the choice is within 5 % of the best but
-// for 128 heads of 768 (6 %); 256 heads of 200 and 256 causal tokens, the whole backward: 70 -> 66 and 74 -> 69 us with one
-// round of 256-row workgroups.
-static float dq_cost(const BwdArgs &a, int64_t BH, bool causal, int qb, float step) {
-  const int64_t nb = (a.Nq + 128 * qb - 1) / (128 * qb);
-  const float steps = (float)((a.Nk + 31) / 32) * step, fix = 2.0f;
-  if (!causal) return (float)((nb * BH + 255) / 256) * (steps + fix);
-  if (nb * BH <= 256) return 1.1f * (steps + fix);
-  const float f = (float)a.Nq / (float)a.Nk;   // a head's triangle (trapezoid: few queries) of steps
-  const float sum = (float)(nb * BH) * (steps * (1.0f - 0.5f * f) + 2.0f * (float)qb * step + fix);
-  return sum / 256.0f + 0.5f * steps;
-}
-
-template <typename T, int D> int launch_dq(BwdArgs a, int64_t BH, bool causal, hipStream_t st) {
+template <typename T, int D> int launch_dq(BwdArgs a, int64_t BH, bool causal, int blocks, int splits, hipStream_t st) {
   if constexpr (D == 128) {
-    // 64 queries per wave need fewer LDS reads per query (the ratio of the steps is that of the dK / dV kernel, which reads
-    // the same operands); 32 fill the chip with twice the workgroups: 1024 x 1024, 16 heads: 44 -> 22 us, 2048 x 2048, 4
-    // heads: 81 -> 36 us against 256-query workgroups
-    if (dq_cost(a, BH, causal, 1, 0.62f) >= dq_cost(a, BH, causal, 2, 1.0f)) return launch_dq_qb<T, D, 2>(a, BH, causal, st);
+    if (blocks == 2) return launch_dq_qb<T, D, 2>(a, BH, causal, splits, st);
   }
-  return launch_dq_qb<T, D, 1>(a, BH, causal, st);
+  return launch_dq_qb<T, D, 1>(a, BH, causal, splits, st);
 }
-template int launch_dq<__bf16, 64>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dq<__bf16, 128>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dq<__bf16, 256>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dq<_Float16, 64>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dq<_Float16, 128>(BwdArgs, int64_t, bool, hipStream_t);
-template int launch_dq<_Float16, 256>(BwdArgs, int64_t, bool, hipStream_t);
+template int launch_dq<__bf16, 64>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dq<__bf16, 128>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dq<__bf16, 256>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dq<_Float16, 64>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dq<_Float16, 128>(BwdArgs, int64_t, bool, int, int, hipStream_t);
+template int launch_dq<_Float16, 256>(BwdArgs, int64_t, bool, int, int, hipStream_t);
 
 }  // namespace qfa

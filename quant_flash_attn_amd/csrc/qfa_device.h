@@ -350,4 +350,7 @@ __device__ __forceinline__ void store_tile_rows_f32(const f32x16 (&acc)[D / 32],
 // prefetch; this one leaves them in flight (pair it with dma_wait() where a tile must have landed).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// x / y of a workgroup's or a row's index, which every launch keeps below 2^31: a 64-bit division is a hundred instructions
+__device__ __forceinline__ int64_t index_div(int64_t x, int64_t y) { return (unsigned)x / (unsigned)y; }
+
 }  // namespace qfa

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     }
     mb = a.mblocks - 1 - mb;
   }
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int m0 = mb * FWD_BM;
 
   const int tid = threadIdx.x;
@@ -680,6 +680,17 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
       pipelined(std::false_type{});
     }
   }
+  // What only the epilogue needs is read from the kernel arguments here: held in scalar registers through the loop it
+  // would push others out to memory, and behind the last tile its latency would be seen.
+  typedef __attribute__((address_space(4))) const FwdArgs KernArgs;
+  KernArgs *ep = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  int bh_ = bh;
+  asm volatile("" : "+s"(ep), "+s"(bh_));
+  const int64_t eb = index_div(bh_, ep->H), eh = bh_ - eb * ep->H;
+  int64_t o_at = eb * ep->sob + eh * ep->soh, son = ep->son;
+  void *out = SPLIT ? (void *)ep->po : ep->o;
+  float *out32 = SPLIT ? ep->pml : ep->o32, *lse = ep->lse;
+  asm volatile("" : "+s"(o_at), "+s"(son), "+s"(out), "+s"(out32), "+s"(lse));
   // ---- masked tiles (diagonal, ragged end): one block at a time, nothing carried between blocks
   for (; t < ntiles; ++t) {
     if (t + 2 < ntiles) load_k(t + 2, kb_free);
@@ -703,15 +714,10 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
 
   // ---- epilogue: normalise, store O (as whole rows, through LDS) and LSE
   if (QK_ONLY) {
-    if (qi < a.Nq && g == 0) a.lse[tq0 + qi] = a_i * fmaxf(m_ref, l_run);
+    if (qi < a.Nq && g == 0) lse[tq0 + qi] = a_i * fmaxf(m_ref, l_run);
     return;
   }
   const float l_tot = l_run + swap32_f(l_run);
-  // What only the epilogue needs is read from the kernel arguments here: held in scalar registers through the loop it
-  // would push others out to memory.
-  typedef __attribute__((address_space(4))) const FwdArgs KernArgs;
-  KernArgs *ep = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(ep));
   if (SPLIT) {
     if (qi < a.Nq) {
       const int64_t at = (tq0 + qi) * a.splits + split;
@@ -719,9 +725,9 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
       for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int aa = 0; aa < 4; ++aa)
-          *reinterpret_cast<f32x4 *>(ep->po + at * D + 32 * db + 8 * aa + 4 * g) =
+          *reinterpret_cast<f32x4 *>(static_cast<float *>(out) + at * D + 32 * db + 8 * aa + 4 * g) =
               f32x4{oacc[db][4 * aa], oacc[db][4 * aa + 1], oacc[db][4 * aa + 2], oacc[db][4 * aa + 3]};
-      if (g == 0) *reinterpret_cast<f32x2 *>(ep->pml + 2 * at) = f32x2{a_i * m_ref, l_tot};
+      if (g == 0) *reinterpret_cast<f32x2 *>(out32 + 2 * at) = f32x2{a_i * m_ref, l_tot};
     }
     return;
   }
@@ -729,9 +735,11 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   // O leaves as whole rows through LDS (all tile buffers are free after the last barrier; every wave takes 32 * 2D
   // bytes at the start of the K area)
   static_assert(SM::OFF_K + FWD_WAVES * 32 * 2 * D <= SM::TOTAL, "output staging fits the tile buffers");
-  if (ep->o32) store_tile_rows_f32<D>(oacc, inv, ep->o32 + tq0 * D, D, m0 + wave * 32, a.Nq, lane);
-  if (ep->o) store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), reinterpret_cast<T *>(ep->o) + b * ep->sob + h * ep->soh, ep->son, m0 + wave * 32, a.Nq, lane);
-  if (qi < a.Nq && g == 0) ep->lse[tq0 + qi] = (a_i * m_ref + __log2f(l_tot)) * kLn2;
+  if (out32) store_tile_rows_f32<D>(oacc, inv, out32 + tq0 * D, D, m0 + wave * 32, a.Nq, lane);
+  if (out)
+    store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), static_cast<T *>(out) + o_at, son, m0 + wave * 32, a.Nq,
+                          lane);
+  if (qi < a.Nq && g == 0) lse[tq0 + qi] = (a_i * m_ref + __log2f(l_tot)) * kLn2;
 }
 
 template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStream_t st, bool qk_only) {

@@ -63,7 +63,7 @@ template <typename T, int D, int QB, bool CAUSAL, bool SPLIT> __global__ __launc
     }
     mb = a.mblocks - 1 - mb;
   }
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int m0 = mb * 4 * QUERIES;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);

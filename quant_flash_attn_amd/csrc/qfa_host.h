@@ -45,6 +45,7 @@ struct AttnArgs {
   int io_dtype;
   float *o32;   // forward: nullable, O in fp32 (dense); o is nullable then
   int f32;      // backward: dO and the gradients are fp32, the workspace holds bwd_f32_workspace_bytes
+  int may_split;   // backward: and bwd_split_bytes behind them
 };
 
 int launch_fwd(const AttnArgs &a, hipStream_t st, bool qk_only = false);   // workspace: nullable, the keys are split with one
@@ -59,6 +60,11 @@ int64_t bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D)
 inline int64_t bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
   return bwd_workspace_bytes(B, H, Nq, Nk, D) + B * H * Nq * D * 2;
 }
+
+// How the backward's two MFMA kernels are launched: 32-row blocks per wave, and the parts of the streamed rows
+struct BwdPlan { int blocks_dkv, splits_dkv, queries_per_split, blocks_dq, splits_dq, keys_per_split; };
+BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_split);
+int64_t bwd_split_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal);
 
 // grid of a kernel that maps ids with XcdBlock (qfa_skv_common.h): per_bh workgroups for each of BH heads
 __host__ __device__ inline bool xcd_whole_heads(int64_t BH) { return BH >= 64 || BH % 8 == 0; }

@@ -1,0 +1,172 @@
+// Into how many parts the streamed rows of the INT8-score kernels are dealt: the keys of the forward (qfa_fwd.hip,
+// qfa_fwd_wide.hip) and of dQ (qfa_bwd_dq.hip), the queries of dK and dV (qfa_bwd_dkv.hip).
+//
+// A workgroup is a chain of tiles whose pace hardly depends on what the rest of the chip does, so few rows against many take the
+// time of one chain while the other CUs idle (forward, 4 heads, 333 queries, 30000 keys of 128: 12 workgroups, 458 us; their
+// keys in 20 parts 40 us, with the merge).  A second workgroup on a CU is only worth a third to a half of one more CU, and each
+// part writes its fp32 results for another kernel to add.  The model below is that and no more.  Its constants are fitted to
+// 2600 (forward) and 1000 (backward) shapes of 1 to 512 heads, 17 to 16384 queries, 64 to 30000 keys, causal or not, each timed
+// with every division.  Over these shapes the forward takes 1.01 times the best division's time in the geometric mean where the
+// undivided one takes 1.9 times, dK / dV 1.01 against 1.045, dQ 1.004 against 1.11 (both of the whole backward).  Small gains
+// are left, being within the model's error: no shape got slower by more than 4 %.
+#include <algorithm>
+#include <cmath>
+
+#include "qfa_host.h"
+
+namespace qfa {
+
+struct SplitCost {
+  double tile[3];      // us per tile with one, two, three workgroups on a CU
+  int resident;        // workgroups on a CU
+  double start, tail;  // of a workgroup, in tiles; share of the last workgroup that runs alone
+  double merge, mb;    // us: the merge or sum, and per MB that it moves
+  double base;
+};
+
+constexpr int64_t MAX_WGS = 1700, MAX_WGS_BWD = 1100;   // of a divided launch: as far as was measured, and bounds the parts' memory
+
+// `blocks` workgroups of `rows` rows each for each of `heads` heads, the streamed rows in tiles of `tile` (64 or 32), s parts of
+// `each` rows; ends: block i sees streamed rows up to (i + 1) * rows + coff, otherwise from i * rows - coff on
+struct SplitWork {
+  int64_t heads, blocks, rows, streamed, tile, coff;
+  bool causal, ends;
+  double total = 0, longest = 0;   // tiles of a head, of its longest block
+  int64_t seen(int64_t i) const {
+    if (!causal) return streamed;
+    return ends ? std::min(streamed, (i + 1) * rows + coff) : streamed - std::max<int64_t>(i * rows - coff, 0);
+  }
+  void count() {   // (only for launches that may be divided: few blocks)
+    if (!causal) {
+      longest = (double)((streamed + tile - 1) / tile);
+      total = longest * (double)blocks;
+      return;
+    }
+    for (int64_t i = 0; i < blocks; ++i) {
+      const double n = (double)((seen(i) + tile - 1) / tile);
+      total += n;
+      longest = std::max(longest, n);
+    }
+  }
+  double time(const SplitCost &c, int64_t s, int64_t each, double mbytes) const {
+    const double per = (double)(each / tile);
+    double wgs = (double)(blocks * s);
+    if (causal) wgs = std::min(wgs, total / per + 0.5 * (double)blocks);   // the others have nothing to do
+    const double n = wgs * (double)heads, slots = 256.0 * c.resident, last = std::min(longest, per) + c.start;
+    const double body = n <= slots ? last * c.tile[std::min(c.resident, (int)std::ceil(n / 256.0)) - 1]
+                                   : ((total * (double)heads + n * c.start) / slots + c.tail * last) * c.tile[c.resident - 1];
+    return c.base + body + (s > 1 ? c.merge + c.mb * mbytes : 0.0);
+  }
+};
+
+// the parts of `streamed` rows that cost least, at most `most`: f(s, rows of a part) in us, if below `best`
+template <typename F> static void best_division(int64_t streamed, int64_t most, double best, int64_t *splits, int64_t *each, F f) {
+  const int64_t tiles = (streamed + 63) / 64;
+  for (int64_t s = 2; s <= std::min(tiles, most); ++s) {
+    const int64_t e = (tiles + s - 1) / s;
+    if ((tiles + e - 1) / e != s) continue;
+    const double t = f(s, e * 64);
+    if (t < best) {
+      best = t;
+      *splits = s;
+      *each = e * 64;
+    }
+  }
+}
+
+void fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int *splits, int *keys_per_split) {
+  static const SplitCost c64 = {{0.85, 1.00, 1.34}, 3, 1.85, 0.28, 2.1, 0.275, 4.3}, c128 = {{1.13, 1.45, 0}, 2, 1.14, 0.48, 2.6, 0.265, 4.5},
+                         c256 = {{1.58, 0, 0}, 1, 1.08, 0.53, 4.1, 0.26, 5.2};
+  const SplitCost &c = D == 64 ? c64 : D == 128 ? c128 : c256;
+  const int64_t blocks = (Nq + 127) / 128;
+  int64_t s = 1, each = (Nk + 63) / 64 * 64;
+  if (BH <= MAX_WGS && blocks <= MAX_WGS && 2 * BH * blocks <= MAX_WGS) {
+    SplitWork w = {BH, blocks, 128, Nk, 64, Nk - Nq, causal != 0, true};
+    w.count();
+    best_division(Nk, std::min<int64_t>(64, MAX_WGS / (BH * blocks)), 0.92 * w.time(c, 1, each, 0), &s, &each,
+                  [&](int64_t n, int64_t e) { return w.time(c, n, e, 8e-6 * (double)(BH * Nq * n * (D + 2))); });
+  }
+  *splits = (int)s;
+  *keys_per_split = (int)each;
+}
+
+int64_t fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal) {
+  int splits, keys;
+  fwd_plan(B * H, Nq, Nk, D, causal, &splits, &keys);
+  return splits > 1 ? B * H * Nq * splits * (int64_t)(D + 2) * 4 : 0;
+}
+
+// ---- backward
+// Blocks of 32 rows per wave.  Two at head_dim 128: a step of 64 rows per wave costs 1 / 0.62 of one of 32, which need more LDS
+// reads per row, but fill the chip with twice the workgroups and waste less of the last one (1024 x 1024, 16 heads: dQ 44 -> 22
+// us; 2048 x 2048, 4 heads: 81 -> 36 us against 64 rows).  The cost of a launch on 256 CUs, one workgroup per CU, in steps of 32
+// streamed rows: whole rounds when all are equally long; causal, the mean load and half of the longest, or the longest where
+// all run at once (a tenth more, since the mean of shorter ones fills in better than that); starting and finishing a workgroup
+// costs about two.  Both kernels' variants timed for 16 to 1024 heads of 64 to 2048 tokens: the choice is within 5 % of the
+// best but for 128 heads of 768 (6 %); 256 heads of 200 and 256 causal tokens, the whole backward: 70 -> 66 and 74 -> 69 us with
+// one round of 256-row workgroups.
+static float undivided_cost(int64_t BH, int64_t rows, int64_t streamed, bool causal, float f, int rb, float step) {
+  const int64_t nb = (rows + 128 * rb - 1) / (128 * rb);
+  const float steps = (float)((streamed + 31) / 32) * step, fix = 2.0f;
+  if (!causal) return (float)((nb * BH + 255) / 256) * (steps + fix);
+  if (nb * BH <= 256) return 1.1f * (steps + fix);
+  const float sum = (float)(nb * BH) * (steps * (1.0f - 0.5f * f) + 2.0f * (float)rb * step + fix);   // f: a head's triangle (trapezoid)
+  return sum / 256.0f + 0.5f * steps;
+}
+
+// one of the two kernels: `tensors` fp32 results per row
+static void bwd_part(int64_t BH, int64_t rows, int64_t streamed, int D, bool causal, bool ends, int64_t coff, float f, bool may_split,
+                     const SplitCost (&c)[2], int tensors, int *blocks, int *splits, int *per_split) {
+  int rb = 1;
+  if (D == 128 && undivided_cost(BH, rows, streamed, causal, f, 1, 0.62f) >= undivided_cost(BH, rows, streamed, causal, f, 2, 1.0f)) rb = 2;
+  int64_t s = 1, each = (streamed + 63) / 64 * 64;
+  *blocks = rb;
+  if (may_split && BH <= MAX_WGS_BWD && rows <= 128 * MAX_WGS_BWD) {
+    SplitWork w[2];
+    for (int r = 1; r <= (D == 128 ? 2 : 1); ++r) {
+      w[r - 1] = {BH, (rows + 128 * r - 1) / (128 * r), 128 * r, streamed, 32, coff, causal, ends};
+      if (2 * BH * w[r - 1].blocks <= MAX_WGS_BWD || r == rb) w[r - 1].count();
+    }
+    double best = 0.93 * w[rb - 1].time(c[rb - 1], 1, each, 0);
+    for (int r = 1; r <= (D == 128 ? 2 : 1); ++r) {
+      const SplitWork &x = w[r - 1];
+      const int64_t was = s;
+      s = 1;
+      best_division(streamed, std::min<int64_t>(32, MAX_WGS_BWD / (BH * x.blocks)), best, &s, &each, [&](int64_t n, int64_t e) {
+        return x.time(c[r - 1], n, e, 8e-6 * (double)(BH * rows * n) * D * tensors);
+      });
+      if (s > 1) {
+        best = x.time(c[r - 1], s, each, 8e-6 * (double)(BH * rows * s) * D * tensors);
+        *blocks = r;
+      } else {
+        s = was;
+      }
+    }
+  }
+  *splits = (int)s;
+  *per_split = (int)each;
+}
+
+BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_split) {
+  // [head_dim][32-row blocks per wave], in tiles of 32 rows
+  static const SplitCost dkv64[2] = {{{0.522, 0.590, 0}, 2, 0.462, 0.662, 2.96, 0.186, 0}, {}},
+                         dkv128[2] = {{{0.642, 0, 0}, 1, 0.373, 0.541, 3.96, 0.174, 0}, {{0.756, 0, 0}, 1, 0.373, 0.541, 3.96, 0.174, 0}},
+                         dkv256[2] = {{{1.137, 0, 0}, 1, 3.005, 0.686, 7.39, 0.143, 0}, {}},
+                         dq64[2] = {{{0.337, 0.473, 0}, 2, 0.255, 0.515, 2.74, 0.254, 0}, {}},
+                         dq128[2] = {{{0.448, 0, 0}, 1, 0.577, 0.585, 3.62, 0.245, 0}, {{0.668, 0, 0}, 1, 0.577, 0.585, 3.62, 0.245, 0}},
+                         dq256[2] = {{{0.852, 0, 0}, 1, 3.596, 0.833, 4.97, 0.147, 0}, {}};
+  const float f = (float)Nq / (float)Nk;
+  BwdPlan p;
+  bwd_part(BH, Nk, Nq, D, causal, false, Nk - Nq, f, may_split, D == 64 ? dkv64 : D == 128 ? dkv128 : dkv256, 2, &p.blocks_dkv,
+           &p.splits_dkv, &p.queries_per_split);
+  bwd_part(BH, Nq, Nk, D, causal, true, Nk - Nq, f, may_split, D == 64 ? dq64 : D == 128 ? dq128 : dq256, 1, &p.blocks_dq, &p.splits_dq,
+           &p.keys_per_split);
+  return p;
+}
+
+int64_t bwd_split_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal) {
+  const BwdPlan p = bwd_plan(B * H, Nq, Nk, D, causal, 1);
+  return B * H * D * 4 * ((p.splits_dkv > 1 ? 2 * Nk * p.splits_dkv : 0) + (p.splits_dq > 1 ? Nq * p.splits_dq : 0));
+}
+
+}  // namespace qfa

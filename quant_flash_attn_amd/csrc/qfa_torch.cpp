@@ -39,7 +39,7 @@ struct Api {
   QFA_ENTRY(qfa_bench_qk_stage);
   QFA_ENTRY(qfa_attn_bwd_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd);
-  QFA_ENTRY(qfa_attn_bwd_f32_workspace_bytes);
+  QFA_ENTRY(qfa_attn_bwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd_f32);
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
@@ -71,7 +71,7 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_bench_qk_stage);
   QFA_ENTRY(qfa_attn_bwd_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd);
-  QFA_ENTRY(qfa_attn_bwd_f32_workspace_bytes);
+  QFA_ENTRY(qfa_attn_bwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd_f32);
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
@@ -308,12 +308,14 @@ void fwd_split_into(const Quantized &q, const Quantized &k, const Tensor &v, con
 }
 
 using Grads = std::array<Tensor, 3>;
+// split: the streamed rows may be dealt to several workgroups (autograd; the public call's bits do not depend on the batch);
 // f32: dO comes and the gradients leave in fp32
 Grads bwd_of(const Quantized &q, const Quantized &k, const Tensor &v_in, const Tensor &o_in, const Tensor &do_in,
-             const float *lse, bool causal, double sm, bool f32 = false) {
+             const float *lse, bool causal, double sm, bool split, bool f32 = false) {
   const at::ScalarType gt = f32 ? at::kFloat : v_in.scalar_type();
   const Tensor v = rows16(v_in), o = rows16(o_in), dout = rows16(to(do_in, gt));
-  const int64_t ws_bytes = (f32 ? api.qfa_attn_bwd_f32_workspace_bytes : api.qfa_attn_bwd_workspace_bytes)(q.B, q.H, q.N, k.N, (int)q.D);
+  const int64_t ws_bytes = split || f32 ? api.qfa_attn_bwd_split_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D, causal, f32)
+                                        : api.qfa_attn_bwd_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D);
   TORCH_CHECK_VALUE(ws_bytes > 0, "unsupported backward shape B=", q.B, " H=", q.H, " Nq=", q.N, " Nk=", k.N, " D=", q.D);
   const Tensor ws = empty({ws_bytes}, at::kByte, v);
   Tensor dq = empty({q.B, q.H, q.N, q.D}, gt, v), dk = empty({q.B, q.H, k.N, q.D}, gt, v), dv = empty({q.B, q.H, k.N, q.D}, gt, v);
@@ -376,7 +378,8 @@ Grads attn_bwd(const QuantTensors &qq, const QuantTensors &kq, const Tensor &v, 
   TORCH_CHECK_TYPE(o.scalar_type() == v.scalar_type(), "o and v must have the same dtype");
   require_gpu(q.hold[0], k.hold[0], v, o, dout, lse);
   const c10::DeviceGuard guard(v.device());
-  return bwd_of(q, k, v, o, dout, flat(lse, at::kFloat, q.B * q.H * q.N, "lse").data_ptr<float>(), causal, sm);
+  return bwd_of(q, k, v, o, dout, flat(lse, at::kFloat, q.B * q.H * q.N, "lse").data_ptr<float>(), causal, sm,
+                false);
 }
 
 at::ScalarType io_dtype(const Tensor &t) { return is_io(t.scalar_type()) ? t.scalar_type() : at::kBFloat16; }
@@ -414,7 +417,7 @@ Grads bwd_from(AutogradContext *ctx, const variable_list &saved, const Tensor &g
   const PairBuffer pb(o16.size(0), o16.size(1), o16.size(2), Nk, o16.size(3));
   const c10::DeviceGuard guard(v16.device());
   return bwd_of(pb.view(buf, 0), pb.view(buf, 1), v16, o16, grad, pb.lse_of(buf),
-                ctx->saved_data["causal"].toBool(), ctx->saved_data["sm"].toDouble(), f32);
+                ctx->saved_data["causal"].toBool(), ctx->saved_data["sm"].toDouble(), true, f32);
 }
 
 // ---- q, k, v
@@ -580,7 +583,7 @@ struct CacheFn : torch::autograd::Function<CacheFn> {
     const PairBuffer pb(o16.size(0), o16.size(1), o16.size(2), 0, o16.size(3));
     const c10::DeviceGuard guard(v16.device());
     const Grads g = bwd_of(pb.view(buf, 0), k, v16, o16, grads[0], pb.lse_of(buf), ctx->saved_data["causal"].toBool(),
-                           ctx->saved_data["sm"].toDouble());
+                           ctx->saved_data["sm"].toDouble(), true);
     const int64_t dt = ctx->saved_data["dt"].toInt();
     variable_list out(11);
     for (int i = 0; i < 3; ++i) out[i] = to(g[i], (at::ScalarType)(dt >> (8 * i) & 255));
@@ -739,7 +742,7 @@ struct SharedLongFn : torch::autograd::Function<SharedLongFn> {
     const PairBuffer pb(o16.size(0), o16.size(1), o16.size(2), 0, o16.size(3));
     const c10::DeviceGuard guard(v16.device());
     const Grads g = bwd_of(pb.view(buf, 0), keys_of(s[3], s[4], s[5], s[6]), v16, o16, grads[0], pb.lse_of(buf), false,
-                           ctx->saved_data["sm"].toDouble());
+                           ctx->saved_data["sm"].toDouble(), true);
     // quant_flash_attn.py:161 (dk already carries sm_scale): one pass, added in fp32 and rounded once
     check(api.qfa_sum_grads(g[1].data_ptr(), g[2].data_ptr(), g[1].data_ptr(), dtype_code(g[1].scalar_type()), g[1].numel(),
                             stream_of(g[1])),
