@@ -100,6 +100,15 @@ int qfa_dequant_per_token(const int8_t *codes, const void *scale, int scale_dtyp
                           int64_t scn, int64_t sob, int64_t soh, int64_t son, void *stream);
 
 /*
+ * What qfa_attn_fwd needs of an INT8 K / V cache, in one launch: rowsum [B*H*N] = the row sums of kc, ks32 (nullable) [B*H*N] = ks
+ * (QFA_F16 or QFA_BF16) in fp32, v [B,H,N,D] dense of v_dtype (QFA_F16 or QFA_BF16) = (vc - vz) * vs with vs of QFA_F32, QFA_F16
+ * or QFA_BF16.  kc, vc [B,H,N,D] with strides; D 64, 128 or 256; the scales and zero points dense.
+ */
+int qfa_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
+                    int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb,
+                    int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, void *stream);
+
+/*
  * rowsum[b,h,n] = sum_d codes[b,h,n,d] (int32, dense [B*H*N]): the side output of qfa_quant_per_token, for
  * codes that arrive already quantized.  qfa_attn_fwd / qfa_attn_bwd need it for the exact zero-point term of the
  * INT8 score product; the reference has no counterpart (its kernels dequantize K before the product,

@@ -140,6 +140,23 @@ int qfa_dequant_per_token(const int8_t *codes, const void *scale, int scale_dtyp
                         (hipStream_t)stream);
 }
 
+int qfa_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
+                    int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb,
+                    int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, void *stream) {
+  const char *who = "cache_stage";
+  if (!kc || !rowsum || !vc || !vs || !vz || !v || (ks32 && !ks)) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
+  if (B <= 0 || H <= 0 || N <= 0) return set_error(QFA_EINVAL, "%s: B, H, N must be positive", who);
+  if (D != 64 && D != 128 && D != 256) return set_error(QFA_EUNSUPPORTED, "%s: head_dim %d not in {64, 128, 256}", who, D);
+  if (ks32 && ks_dtype != QFA_F16 && ks_dtype != QFA_BF16) return set_error(QFA_EINVAL, "%s: ks_dtype must be QFA_F16 or QFA_BF16", who);
+  if (!is_float_dtype(vs_dtype)) return set_error(QFA_EINVAL, "%s: vs_dtype %d is not QFA_F32/F16/BF16", who, vs_dtype);
+  if (v_dtype != QFA_F16 && v_dtype != QFA_BF16) return set_error(QFA_EINVAL, "%s: v_dtype must be QFA_F16 or QFA_BF16", who);
+  if (!aligned16(kc) || !aligned16(vc) || !aligned16(v)) return set_error(QFA_EINVAL, "%s: kc, vc, v must be 16-byte aligned", who);
+  if (!strides_ok(skb, skh, skn, D, 1) || !strides_ok(svb, svh, svn, D, 1))
+    return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
+  const int64_t sk[3] = {skb, skh, skn}, sv[3] = {svb, svh, svn};
+  return launch_cache_stage(kc, ks, ks_dtype, ks32, rowsum, vc, vs, vs_dtype, vz, v, v_dtype, B, H, N, D, sk, sv, (hipStream_t)stream);
+}
+
 int qfa_code_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, int64_t N, int D, int64_t scb,
                     int64_t sch, int64_t scn, void *stream) {
   if (!codes || !rowsum) return set_error(QFA_EINVAL, "code_rowsum: null pointer");

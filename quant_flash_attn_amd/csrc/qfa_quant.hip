@@ -420,4 +420,99 @@ int launch_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, in
   return check_launch("qfa_code_rowsum");
 }
 
+// ---------------------------------------------------------------------------------------------
+// What the INT8-score forward needs of an INT8 K / V cache, in one launch: the row sums of K and its scales in fp32, V
+// dequantized.  Bound by memory (5 bytes per element of both; 64 heads of 7001 x 128: 229 MB).  Four tokens per lane group, all
+// loads before any result, as in rowsum_kernel.
+struct CacheStageArgs {
+  const int8_t *kc, *vc;
+  const void *ks, *vs;
+  const int8_t *vz;
+  float *ks32;         // nullable
+  int32_t *rowsum;
+  void *v;             // dense
+  int64_t N, H;
+  int64_t skb, skh, skn, svb, svh, svn;
+  int chunks_per_bh, blocks_k, ks_dtype, vs_dtype;
+};
+template <typename TO, int D> __global__ __launch_bounds__(256) void cache_stage_kernel(CacheStageArgs a) {
+  constexpr int LPT = D / 8, TPP = 256 / LPT, U = 4;
+  const int tid = threadIdx.x, sub = tid % LPT;
+  const bool is_k = (int)blockIdx.x < a.blocks_k;
+  const unsigned blk = is_k ? blockIdx.x : blockIdx.x - a.blocks_k;
+  const unsigned bh = blk / (unsigned)a.chunks_per_bh, chunk = blk - bh * a.chunks_per_bh;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
+  const int64_t n0 = (int64_t)chunk * (TPP * U) + tid / LPT, t0 = (int64_t)bh * a.N;
+  const int8_t *c = (is_k ? a.kc + b * a.skb + h * a.skh : a.vc + b * a.svb + h * a.svh) + sub * 8;
+  const int64_t sn = is_k ? a.skn : a.svn;
+  u32x2 w[U];
+  int64_t n[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    n[u] = n0 + u * TPP < a.N ? n0 + u * TPP : a.N - 1;   // every lane takes part in the reduction
+    w[u] = *reinterpret_cast<const u32x2 *>(c + n[u] * sn);
+  }
+  if (is_k) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int sum = (int)__builtin_amdgcn_sad_u8(w[u][0] ^ 0x80808080u, 0u, 0u);   // biased bytes: code + 128
+      sum = (int)__builtin_amdgcn_sad_u8(w[u][1] ^ 0x80808080u, 0u, (unsigned)sum) - 8 * 128;
+      sum = group_sum<LPT>(sum);
+      if (n0 + u * TPP >= a.N || sub != 0) continue;
+      a.rowsum[t0 + n[u]] = sum;
+      if (a.ks32)
+        a.ks32[t0 + n[u]] = a.ks_dtype == QFA_F16 ? (float)static_cast<const _Float16 *>(a.ks)[t0 + n[u]]
+                                                  : (float)static_cast<const __bf16 *>(a.ks)[t0 + n[u]];
+    }
+    return;
+  }
+  float scale[U], zp[U];
+  if (a.vs_dtype == QFA_F32) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) scale[u] = static_cast<const float *>(a.vs)[t0 + n[u]];
+  } else if (a.vs_dtype == QFA_F16) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) scale[u] = (float)static_cast<const _Float16 *>(a.vs)[t0 + n[u]];
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) scale[u] = (float)static_cast<const __bf16 *>(a.vs)[t0 + n[u]];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) zp[u] = (float)a.vz[t0 + n[u]];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (n0 + u * TPP >= a.N) break;
+    u32x4 p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned x = w[u][e / 2] >> (16 * (e % 2));
+      p[e] = pack2<TO>(((float)(int)(int8_t)(x & 0xff) - zp[u]) * scale[u], ((float)(int)(int8_t)(x >> 8 & 0xff) - zp[u]) * scale[u]);
+    }
+    *reinterpret_cast<u32x4 *>(static_cast<TO *>(a.v) + (t0 + n[u]) * D + sub * 8) = p;
+  }
+}
+template <typename TO, int D> static int launch_cache_stage_td(CacheStageArgs a, int64_t BH, hipStream_t st) {
+  constexpr int TOK = 8192 / D;   // tokens per workgroup
+  const int64_t chunks = (a.N + TOK - 1) / TOK;
+  if (2 * chunks * BH > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "cache_stage: too many tokens for one launch");
+  a.chunks_per_bh = (int)chunks;
+  a.blocks_k = (int)(chunks * BH);
+  cache_stage_kernel<TO, D><<<dim3((unsigned)(2 * chunks * BH)), dim3(256), 0, st>>>(a);
+  return check_launch("qfa_cache_stage");
+}
+int launch_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
+                       int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D,
+                       const int64_t sk[3], const int64_t sv[3], hipStream_t st) {
+  CacheStageArgs a = {kc, vc, ks, vs, vz, ks32, rowsum, v, N, H, sk[0], sk[1], sk[2], sv[0], sv[1], sv[2], 0, 0, ks_dtype, vs_dtype};
+  const int64_t BH = B * H;
+  if (v_dtype == QFA_BF16) {
+    if (D == 64) return launch_cache_stage_td<__bf16, 64>(a, BH, st);
+    if (D == 128) return launch_cache_stage_td<__bf16, 128>(a, BH, st);
+    return launch_cache_stage_td<__bf16, 256>(a, BH, st);
+  }
+  if (D == 64) return launch_cache_stage_td<_Float16, 64>(a, BH, st);
+  if (D == 128) return launch_cache_stage_td<_Float16, 128>(a, BH, st);
+  return launch_cache_stage_td<_Float16, 256>(a, BH, st);
+}
+
 }  // namespace qfa

@@ -33,6 +33,7 @@ struct Api {
   QFA_ENTRY(qfa_quant_qkv_f32);
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
+  QFA_ENTRY(qfa_cache_stage);
   QFA_ENTRY(qfa_attn_fwd);
   QFA_ENTRY(qfa_attn_fwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_split);
@@ -65,6 +66,7 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_quant_qkv_f32);
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
+  QFA_ENTRY(qfa_cache_stage);
   QFA_ENTRY(qfa_attn_fwd);
   QFA_ENTRY(qfa_attn_fwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_split);
@@ -509,10 +511,23 @@ CacheKept cache_forward(const Tensor &q_in, const Tensor &kc, const Tensor &ks, 
   r.buf = empty({pb.bytes}, at::kByte, q);
   quantize_into(q, pb.view(r.buf, 0));
   r.kc = rows16(kc);
-  r.ks = flat(to(ks, at::kFloat), at::kFloat, nk, "k.scale");
   r.kz = flat(kz, at::kChar, nk, "k.zero_point");
-  r.kr = rowsum(r.kc);
-  r.v16 = dequant(vc, vs, vz, io_dtype(q));
+  require_gpu(q, kc, ks, kz, vc, vs, vz);
+  check_codes(vc, "v.codes");
+  // K's row sums and fp32 scales and V dequantized, in one launch
+  const Tensor v = rows16(vc), vzf = flat(vz, at::kChar, nk, "v.zero_point");
+  TORCH_CHECK_TYPE(dtype_code(vs.scalar_type()) >= 0, "dtype and scale.dtype must be float16, bfloat16 or float32");
+  const Tensor vsf = flat(vs, vs.scalar_type(), nk, "v.scale");
+  const bool widen = is_io(ks.scalar_type());
+  const Tensor ksf = widen ? flat(ks, ks.scalar_type(), nk, "k.scale") : flat(to(ks, at::kFloat), at::kFloat, nk, "k.scale");
+  r.ks = widen ? empty({nk}, at::kFloat, q) : ksf;
+  r.kr = empty({nk}, at::kInt, q);
+  r.v16 = empty({kc.size(0), kc.size(1), kc.size(2), kc.size(3)}, io_dtype(q), q);
+  check(api.qfa_cache_stage(r.kc.data_ptr<int8_t>(), ksf.data_ptr(), dtype_code(ksf.scalar_type()),
+                            widen ? r.ks.data_ptr<float>() : nullptr, r.kr.data_ptr<int32_t>(), v.data_ptr<int8_t>(), vsf.data_ptr(),
+                            dtype_code(vsf.scalar_type()), vzf.data_ptr<int8_t>(), r.v16.data_ptr(), dtype_code(r.v16.scalar_type()),
+                            pb.B, pb.H, kc.size(2), (int)pb.D, QFA_STRIDES(r.kc), QFA_STRIDES(v), stream_of(q)),
+        "qfa_cache_stage");
   r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, r.v16.scalar_type(), q);
   fwd_split_into(pb.view(r.buf, 0), keys_of(r.kc, r.ks, r.kz, r.kr), r.v16, r.o16, Tensor(), pb.lse_of(r.buf), causal, sm);
   r.o = to(r.o16, q.scalar_type());
