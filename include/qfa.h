@@ -309,6 +309,10 @@ int qfa_bench_qk_stage(const int8_t *qc, const float *sq, const int8_t *zq, cons
 int64_t qfa_dout_normalise_workspace_bytes(void);
 int qfa_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *kv_scale, int scale_dtype, int64_t n_scale,
                        void *workspace, void *out, float *back, void *stream);
+/* ... and y0 = x0, y1 = x1 (nullable) as binary16, of two bf16 tensors of the same n elements, dense and 16-byte aligned */
+int qfa_dout_normalise_cast(const void *dout, int dout_dtype, int64_t n, const void *kv_scale, int scale_dtype, int64_t n_scale,
+                       void *workspace, void *out, float *back, const void *x0, void *y0, const void *x1,
+                            void *y1, void *stream);
 
 /*
  * out[i] = a[i] + b[i] for two dense 16-bit tensors of n elements (n a multiple of 8, pointers 16-byte aligned;

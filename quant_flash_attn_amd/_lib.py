@@ -49,6 +49,7 @@ _SIGNATURES = {
     "qfa_sum_grads": (c_int, [_P, _P, _P, _I, _L, _P]),
     "qfa_dout_normalise_workspace_bytes": (c_int64, []),
     "qfa_dout_normalise": (c_int, [_P, _I, _L, _P, _I, _L, _P, _P, _P, _P]),
+    "qfa_dout_normalise_cast": (c_int, [_P, _I, _L, _P, _I, _L, _P, _P, _P, _P, _P, _P, _P, _P]),
     "qfa_bwd_delta": (c_int, [_P, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_attn_bwd_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
     "qfa_attn_bwd_split_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I, _I, _I]),

@@ -450,8 +450,8 @@ int qfa_sum_grads(const void *a, const void *b, void *out, int dtype, int64_t n,
 
 int64_t qfa_dout_normalise_workspace_bytes(void) { return dout_normalise_workspace_bytes(); }
 
-int qfa_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *kv_scale, int scale_dtype, int64_t n_scale,
-                       void *workspace, void *out, float *back, void *stream) {
+int qfa_dout_normalise_cast(const void *dout, int dout_dtype, int64_t n, const void *kv_scale, int scale_dtype, int64_t n_scale,
+                       void *workspace, void *out, float *back, const void *x0, void *y0, const void *x1, void *y1, void *stream) {
   if (!dout || !kv_scale || !workspace || !out || !back) return set_error(QFA_EINVAL, "dout_normalise: null pointer argument");
   if (dout_dtype != QFA_BF16 && dout_dtype != QFA_F16) return set_error(QFA_EINVAL, "dout_normalise: dout_dtype must be QFA_BF16 or QFA_F16");
   if (scale_dtype != QFA_F32 && scale_dtype != QFA_F16) return set_error(QFA_EINVAL, "dout_normalise: scale_dtype must be QFA_F32 or QFA_F16");
@@ -459,8 +459,16 @@ int qfa_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *
   if (n_scale <= 0) return set_error(QFA_EINVAL, "dout_normalise: n_scale must be positive");
   if (!aligned16(dout) || !aligned16(out) || !aligned16(kv_scale))
     return set_error(QFA_EINVAL, "dout_normalise: dout, kv_scale and out must be 16-byte aligned");
-  return launch_dout_normalise(dout, dout_dtype, n, kv_scale, scale_dtype, n_scale, static_cast<float *>(workspace), out, back,
+  if (!x0 != !y0 || !x1 != !y1 || (x1 && !x0)) return set_error(QFA_EINVAL, "dout_normalise: every x needs its y, and x1 an x0");
+  if (!aligned16(x0) || !aligned16(y0) || !aligned16(x1) || !aligned16(y1))
+    return set_error(QFA_EINVAL, "dout_normalise: x0, y0, x1, y1 must be 16-byte aligned");
+  return launch_dout_normalise(dout, dout_dtype, n, kv_scale, scale_dtype, n_scale, static_cast<float *>(workspace), out, back, x0, y0, x1, y1,
                                (hipStream_t)stream);
+}
+
+int qfa_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *kv_scale, int scale_dtype, int64_t n_scale,
+                       void *workspace, void *out, float *back, void *stream) {
+  return qfa_dout_normalise_cast(dout, dout_dtype, n, kv_scale, scale_dtype, n_scale, workspace, out, back, nullptr, nullptr, nullptr, nullptr, stream);
 }
 
 int64_t qfa_attn_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {

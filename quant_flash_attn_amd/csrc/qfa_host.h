@@ -97,7 +97,8 @@ int launch_skv_bwd(const SkvAttnArgs &a, hipStream_t st);        // io_dtype QFA
 // partials: dout_normalise_workspace_bytes() of scratch
 int64_t dout_normalise_workspace_bytes();
 int launch_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *scale, int scale_dtype, int64_t ns,
-                          float *partials, void *out, float *back, hipStream_t st);
+                          float *partials, void *out, float *back, const void *x0, void *y0, const void *x1,
+                          void *y1, hipStream_t st);
 // Query blocks of more than 16: forward and dQ on tiles of 64 keys that a workgroup expands once.  qw: waves side by side on
 // the queries (0: not this kernel), splits: workgroups that share the keys, tiles of 64 keys each
 struct SkvTilePlan { int qw, splits, tiles; };

@@ -39,7 +39,7 @@ __device__ __forceinline__ void merge_store(const SplitMergeArgs &a, int64_t row
   if (a.lse && d == 0) a.lse[row] = (m + __log2f(l)) * kLn2;
   if (a.o32) *reinterpret_cast<f32x4 *>(a.o32 + row * D + d) = x;
   if (!a.o) return;
-  const int64_t bh = row / a.Nq, b = bh / a.H, h = bh % a.H, off = b * a.sob + h * a.soh + (row % a.Nq) * a.son;
+  const int64_t bh = index_div(row, a.Nq), b = index_div(bh, a.H), h = bh - b * a.H, off = b * a.sob + h * a.soh + (row - bh * a.Nq) * a.son;
   store4(static_cast<char *>(a.o) + off * (a.o_dtype == QFA_F32 ? 4 : 2), a.o_dtype, d, x);
 }
 

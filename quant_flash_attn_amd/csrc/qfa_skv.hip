@@ -65,7 +65,7 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
   const XcdBlock id(a.BH, a.qblocks * a.splits);
   if (!id.live) return;
   const int bh = id.bh, qb = id.sub % a.qblocks, split = id.sub / a.qblocks;
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid % 64, q16 = lane % 16, G = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wave_off = wave * WAVE;

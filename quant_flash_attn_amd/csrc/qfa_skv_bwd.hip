@@ -564,10 +564,23 @@ __global__ __launch_bounds__(256) void dout_max_kernel(const T *dout, int64_t n8
   }
 }
 
+// Workgroups of blockIdx.y > 0 cast one of two more bf16 tensors of the same size (Q and O of a bf16 call, which the kernels take
+// in binary16 too): two launches less.
+struct DoutCast { const __bf16 *x[2]; _Float16 *y[2]; };
 template <typename T>
 __global__ __launch_bounds__(256) void dout_scale_kernel(const T *dout, int64_t n8, const float *partials, _Float16 *out,
-                                                         float *back) {
+                                                         float *back, DoutCast cast) {
   __shared__ float red[4];
+  if (blockIdx.y > 0) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const u32x4 w = reinterpret_cast<const u32x4 *>(cast.x[blockIdx.y - 1])[i];
+    u32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = pack2<_Float16>(lo_to_f32<__bf16>(w[e]), hi_to_f32<__bf16>(w[e]));
+    reinterpret_cast<u32x4 *>(cast.y[blockIdx.y - 1])[i] = r;
+    return;
+  }
   float m = 0.f, ms = 0.f;
   for (int i = threadIdx.x; i < NORM_BLOCKS; i += 256) {
     m = fmaxf(m, partials[2 * i]);
@@ -590,24 +603,26 @@ __global__ __launch_bounds__(256) void dout_scale_kernel(const T *dout, int64_t 
 
 template <typename T, typename S>
 static int launch_dout_normalise_ts(const void *dout, int64_t n, const void *scale, int64_t ns, float *partials,
-                                    void *out, float *back, hipStream_t st) {
+                                    void *out, float *back, const DoutCast &cast, hipStream_t st) {
   const int64_t n8 = n / 8, blocks = (n8 + 255) / 256;
   if (blocks > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "dout_normalise: too many elements for one launch");
   dout_max_kernel<T, S><<<dim3(NORM_BLOCKS), dim3(256), 0, st>>>((const T *)dout, n8, (const S *)scale, ns, partials);
-  dout_scale_kernel<T><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const T *)dout, n8, partials, (_Float16 *)out, back);
+  const unsigned tensors = cast.x[1] ? 3 : cast.x[0] ? 2 : 1;
+  dout_scale_kernel<T><<<dim3((unsigned)blocks, tensors), dim3(256), 0, st>>>((const T *)dout, n8, partials, (_Float16 *)out, back, cast);
   return check_launch("qfa_dout_normalise");
 }
 
 int64_t dout_normalise_workspace_bytes() { return (int64_t)NORM_BLOCKS * 2 * sizeof(float); }
 
 int launch_dout_normalise(const void *dout, int dout_dtype, int64_t n, const void *scale, int scale_dtype, int64_t ns,
-                          float *partials, void *out, float *back, hipStream_t st) {
+                          float *partials, void *out, float *back, const void *x0, void *y0, const void *x1, void *y1, hipStream_t st) {
+  const DoutCast cast = {{static_cast<const __bf16 *>(x0), static_cast<const __bf16 *>(x1)}, {static_cast<_Float16 *>(y0), static_cast<_Float16 *>(y1)}};
   const bool s32 = scale_dtype == QFA_F32;
   if (dout_dtype == QFA_BF16)
-    return s32 ? launch_dout_normalise_ts<__bf16, float>(dout, n, scale, ns, partials, out, back, st)
-               : launch_dout_normalise_ts<__bf16, _Float16>(dout, n, scale, ns, partials, out, back, st);
-  return s32 ? launch_dout_normalise_ts<_Float16, float>(dout, n, scale, ns, partials, out, back, st)
-             : launch_dout_normalise_ts<_Float16, _Float16>(dout, n, scale, ns, partials, out, back, st);
+    return s32 ? launch_dout_normalise_ts<__bf16, float>(dout, n, scale, ns, partials, out, back, cast, st)
+               : launch_dout_normalise_ts<__bf16, _Float16>(dout, n, scale, ns, partials, out, back, cast, st);
+  return s32 ? launch_dout_normalise_ts<_Float16, float>(dout, n, scale, ns, partials, out, back, cast, st)
+             : launch_dout_normalise_ts<_Float16, _Float16>(dout, n, scale, ns, partials, out, back, cast, st);
 }
 
 }  // namespace qfa

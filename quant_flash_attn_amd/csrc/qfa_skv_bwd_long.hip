@@ -48,7 +48,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
   const XcdBlock id(a.BH, a.qblocks);
   if (!id.live) return;
   const int bh = id.bh, qb = id.sub;
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid % 64, q16 = lane % 16, G = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wave_off = wave * WAVE;
@@ -291,7 +291,7 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   const int wgs_per_bh = (a.kchunks + a.cpw - 1) / a.cpw;
   const int bh = blockIdx.x / wgs_per_bh;
   const int c_begin = (blockIdx.x % wgs_per_bh) * a.cpw, c_end = min(a.kchunks, c_begin + a.cpw);
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int ntiles = (a.Nk + SKV_TILE - 1) / SKV_TILE;

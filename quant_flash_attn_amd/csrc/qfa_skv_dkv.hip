@@ -46,7 +46,7 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
   const XcdBlock id(a.BH, a.wgs_per_bh);
   if (!id.live) return;
   const int bh = id.bh, part = id.sub;
-  const int64_t b = bh / a.H, h = bh % a.H;
+  const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int nqb = (a.Nq + 31) / 32, ntiles = (a.Nk + 31) / 32;

@@ -184,7 +184,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
 
   const XcdBlock id(a.BH, a.qwgs * a.splits);
   if (!id.live) return;
-  const int64_t b = id.bh / a.H, h = id.bh % a.H;
+  const int64_t b = index_div(id.bh, a.H), h = id.bh - b * a.H;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int split = id.sub / a.qwgs;
@@ -404,7 +404,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
 
   const XcdBlock id(a.BH, a.qwgs * a.splits);
   if (!id.live) return;
-  const int64_t b = id.bh / a.H, h = id.bh % a.H;
+  const int64_t b = index_div(id.bh, a.H), h = id.bh - b * a.H;
   const int tid = threadIdx.x, lane = tid % 64, lr = lane % 32, g = lane / 32;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int split = id.sub / a.qwgs;

@@ -50,7 +50,7 @@ struct Api {
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
-  QFA_ENTRY(qfa_dout_normalise);
+  QFA_ENTRY(qfa_dout_normalise_cast);
 #undef QFA_ENTRY
 };
 Api api;
@@ -83,7 +83,7 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
-  QFA_ENTRY(qfa_dout_normalise);
+  QFA_ENTRY(qfa_dout_normalise_cast);
 #undef QFA_ENTRY
 }
 
@@ -693,7 +693,9 @@ std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, c
 
 // (dO * 2^k as float16, 2^-k as a one-element float32 tensor) for the binary16 backward kernels: two launches, nothing
 // synchronises
-std::tuple<Tensor, Tensor> normalised_dout(const Tensor &grad_in, const Tensor &scale_in) {
+// and q and o (undefined or) in float16: bf16 ones are cast by the second of these launches, which takes dense tensors
+struct Normalised { Tensor dout, back, q, o; };
+Normalised normalise(const Tensor &grad_in, const Tensor &scale_in, const Tensor &q, const Tensor &o) {
   require_gpu(grad_in, scale_in);
   const c10::DeviceGuard guard(grad_in.device());
   // (a gradient that is not 16-bit is not what autograd hands over for a 16-bit output; bf16 keeps the range)
@@ -703,11 +705,29 @@ std::tuple<Tensor, Tensor> normalised_dout(const Tensor &grad_in, const Tensor &
   if (reinterpret_cast<uintptr_t>(scale.data_ptr()) % 16) scale = scale.clone();   // a view that starts inside an allocation
   Tensor do16 = empty(grad.sizes(), at::kHalf, grad), back = empty({1}, at::kFloat, grad);
   const Tensor ws = empty({api.qfa_dout_normalise_workspace_bytes()}, at::kByte, grad);
-  check(api.qfa_dout_normalise(grad.data_ptr(), dtype_code(grad.scalar_type()), grad.numel(), scale.data_ptr(),
-                               dtype_code(scale.scalar_type()), scale.numel(), ws.data_ptr(), do16.data_ptr(),
-                               back.data_ptr<float>(), stream_of(grad)),
+  const void *x[2] = {nullptr, nullptr};
+  void *y[2] = {nullptr, nullptr};
+  int casts = 0;
+  auto half = [&](const Tensor &t) -> Tensor {
+    if (!t.defined()) return t;
+    if (t.scalar_type() != at::kBFloat16 || !t.is_contiguous() || t.numel() != grad.numel() || t.device() != grad.device() ||
+        reinterpret_cast<uintptr_t>(t.data_ptr()) % 16)
+      return to(t, at::kHalf);
+    const Tensor h = empty(t.sizes(), at::kHalf, t);
+    x[casts] = t.data_ptr();
+    y[casts++] = h.data_ptr();
+    return h;
+  };
+  const Tensor q16 = half(q), o16 = half(o);
+  check(api.qfa_dout_normalise_cast(grad.data_ptr(), dtype_code(grad.scalar_type()), grad.numel(), scale.data_ptr(),
+                                    dtype_code(scale.scalar_type()), scale.numel(), ws.data_ptr(), do16.data_ptr(),
+                                    back.data_ptr<float>(), x[0], y[0], x[1], y[1], stream_of(grad)),
         "qfa_dout_normalise");
-  return {do16, back};
+  return {do16, back, q16, o16};
+}
+std::tuple<Tensor, Tensor> normalised_dout(const Tensor &grad, const Tensor &scale) {
+  const Normalised n = normalise(grad, scale, Tensor(), Tensor());
+  return {n.dout, n.back};
 }
 
 // The reference's operator with the shared-KV kernels (short query blocks, Q as it comes)
@@ -731,9 +751,8 @@ struct SharedFn : torch::autograd::Function<SharedFn> {
     // so dO is handed over scaled by a power of two chosen on the device (no synchronisation) from
     // its largest magnitude and from the largest key scale, and the kernels scale dQ and dKV back
     // while they round them.  q and o convert exactly from bf16 (more mantissa, values of order one).
-    auto [do16, back] = normalised_dout(grads[0], s[2]);
-    auto [dq, dkv] = skv_bwd(to(q, at::kHalf), s[1], s[2], s[3], to(o, at::kHalf), do16, s[5],
-                             ctx->saved_data["sm"].toDouble(), q.scalar_type(), back, true);
+    const Normalised n = normalise(grads[0], s[2], q, o);
+    auto [dq, dkv] = skv_bwd(n.q, s[1], s[2], s[3], n.o, n.dout, s[5], ctx->saved_data["sm"].toDouble(), q.scalar_type(), n.back, true);
     return {dq, to(dkv, (at::ScalarType)ctx->saved_data["kv_dtype"].toInt()), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
