@@ -6,6 +6,8 @@
 // The module does not link against libqfa.so: the binding that loads the library hands over the addresses of its entry
 // points (init), so there is one place that decides which library file is used, and none of this works without it.
 // Nothing is kept between calls.
+#include <algorithm>
+#include <cmath>
 #include <ATen/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -547,8 +549,29 @@ int64_t cache_max_q(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
   if (BH * ((Nq + 15) / 16) <= 512 || Nk >= 16 * D) return 128;
   return Nk >= 8 * D ? 112 : Nk >= 4 * D ? 80 : Nk >= 2 * D ? 64 : 48;
 }
+// Beyond that line the few launches of qfa_attn_fwd_cache still win where the work is small or the other path fills the chip badly
+// (4 heads, 200 queries, 1000 keys of 64: 9 against 20 us).  Both paths' times in us as fitted to 6500 calls of 2 to 1024 heads, 8
+// to 512 queries, 300 to 20000 keys (within 8 % in the mean): the short one takes what its memory or its blocks of 16 queries
+// take, and loses by a last round of workgroups that is not full; the other one the pass over the cache and blocks of 128
+// queries.  Calls are taken from the other path where that should gain 12 %: over all shapes the choice costs 0.4 - 1 % against
+// the better path each time, where the line alone cost 3 - 6 %; the moved calls gain 1.4 times in the mean, the worst lost 15 %.
+bool cache_short_cheaper(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
+  struct Cost { double s0, s_byte, s_block, s_start, s_fill, l0, l_byte, l_block, l_idle, l_query; };
+  static const Cost c64 = {9.8, 0.48, 11.4, 2.0, 0.37, 18.6, 0.84, 33.7, 0.1, 0.69}, c128 = {11.6, 0.56, 22.4, 6.1, 0.22, 20.4, 0.88, 51.9, 0.095, 0.42},
+                    c256 = {15.3, 0.59, 41.9, 30.8, 0.22, 23.0, 0.88, 127.0, 0.0, 0.6};
+  const Cost &c = D == 64 ? c64 : D == 128 ? c128 : c256;
+  const int64_t nb = (Nq + 15) / 16, mb = (Nq + 127) / 128, wgs = BH * nb;
+  const double n = (double)BH * (double)Nk * 1e-6, fill = wgs <= 512 ? (double)(wgs * (512 / wgs)) / 512.0 : (double)wgs / (double)((wgs + 511) / 512 * 512);
+  const double blocks = (double)nb / std::pow(fill, c.s_fill), work = c.s_block * n * blocks + c.s_start * (double)BH * blocks * 1e-3;
+  const double s = c.s0 + std::pow(std::pow(c.s_byte * n * (double)D, 4.0) + std::pow(work, 4.0), 0.25);
+  const double idle = std::max(0.0, 1.0 - (double)(BH * mb) / 256.0);
+  const double l = c.l0 + c.l_byte * n * (double)D + c.l_block * n * (double)mb * (1.0 + c.l_idle * idle) + c.l_query * (double)(BH * Nq * D) * 1e-6;
+  return s < 0.88 * l;
+}
 bool cache_takes_short(const Tensor &q, const Tensor &kc) {
-  return q.size(2) <= cache_max_q(q.size(0) * q.size(1), q.size(2), kc.size(2), q.size(3));
+  const int64_t BH = q.size(0) * q.size(1), Nq = q.size(2), Nk = kc.size(2), D = q.size(3);
+  if (Nq <= cache_max_q(BH, Nq, Nk, D)) return true;
+  return Nq <= 512 && BH > 0 && Nk > 0 && cache_short_cheaper(BH, Nq, Nk, D);   // (as far as was measured)
 }
 Tensor cache_short(const Tensor &q_in, const Tensor &kc_in, const Tensor &ks_in, const Tensor &kz, const Tensor &vc_in,
                    const Tensor &vs_in, const Tensor &vz, bool causal, double sm) {
