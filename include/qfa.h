@@ -259,6 +259,22 @@ int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void 
                                  void *stream);
 
 /*
+ * The same on q and o of io_dtype (QFA_F16 or QFA_BF16) and dout of dout_dtype as a caller has them: the casts and the scaling
+ * of dO by a power of two (qfa_dout_normalise) happen inside, per workgroup.  For the query blocks that one pass takes, where
+ * qfa_attn_bwd_shared_kv_is_direct(Nq, D) is 1 (up to 32 queries, 16 at head_dim 256); others are QFA_EUNSUPPORTED.
+ */
+int qfa_attn_bwd_shared_kv_is_direct(int64_t Nq, int D);
+
+int qfa_attn_bwd_shared_kv_direct(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
+                                 const void *o, const void *dout, const float *lse, void *dq, void *dkv, int io_dtype,
+                                 int dout_dtype, int grad_dtype,
+                                 int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                                 int64_t scb, int64_t sch, int64_t scn, int64_t sob, int64_t soh, int64_t son, int64_t sdob,
+                                 int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
+                                 int64_t sdkh, int64_t sdkn, float sm_scale, void *workspace, int64_t workspace_bytes,
+                                 void *stream);
+
+/*
  * Attention forward of a SHORT query block on an INT8 cache of keys and values (decoding, a few queries at a time):
  *     O = softmax(sm_scale * Q^ K^^T) V^,   Q^, K^, V^ = scale * (codes - zero_point) per token
  * Q is quantized inside by the arithmetic of qfa_quant_per_token, the scores are those of qfa_attn_fwd on these codes,

@@ -306,6 +306,50 @@ int qfa_attn_fwd_shared_kv_static(const void *q, const int8_t *codes, const void
   return launch_skv_fwd_static(a, (hipStream_t)stream);
 }
 
+static int skv_bwd_entry(const char *who, int direct, int dout_dtype, const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
+                           const void *o, const void *dout, const float *lse, void *dq, void *dkv, int io_dtype,
+                           int grad_dtype, const float *grad_scale,
+                           int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                           int64_t scb, int64_t sch, int64_t scn, int64_t sob, int64_t soh, int64_t son, int64_t sdob,
+                           int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
+                           int64_t sdkh, int64_t sdkn, float sm_scale, void *workspace, int64_t workspace_bytes,
+                                 void *stream) {
+  SkvAttnArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = q; a.codes = codes; a.scale = scale; a.zp = zp; a.o = const_cast<void *>(o); a.lse = const_cast<float *>(lse);
+  a.dout = dout; a.dq = dq; a.dkv = dkv; a.grad_dtype = grad_dtype; a.grad_scale = grad_scale;
+  a.B = B; a.H = H; a.Nq = Nq; a.Nk = Nk; a.D = D; a.io_dtype = io_dtype; a.scale_dtype = scale_dtype;
+  a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.scb = scb; a.sch = sch; a.scn = scn; a.sob = sob; a.soh = soh; a.son = son;
+  a.sdob = sdob; a.sdoh = sdoh; a.sdon = sdon; a.sdqb = sdqb; a.sdqh = sdqh; a.sdqn = sdqn;
+  a.sdkb = sdkb; a.sdkh = sdkh; a.sdkn = sdkn;
+  a.sm_scale = sm_scale; a.direct = direct; a.dout_dtype = dout_dtype;
+  if (int e = check_shared_kv(who, a)) return e;
+  if (!dout || !dq || !dkv) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
+  if (direct) {
+    if (!skv_bwd_one_pass(Nq, D))
+      return set_error(QFA_EUNSUPPORTED, "%s: %lld queries of head_dim %d take the scaled form", who, (long long)Nq, D);
+    if (dout_dtype != QFA_F16 && dout_dtype != QFA_BF16) return set_error(QFA_EINVAL, "%s: dout_dtype must be QFA_F16 or QFA_BF16", who);
+  }
+  if (!direct && io_dtype != QFA_F16) return set_error(QFA_EUNSUPPORTED, "%s: io_dtype (q, o, dout) must be QFA_F16", who);
+  if (grad_dtype != QFA_F16 && grad_dtype != QFA_BF16)
+    return set_error(QFA_EINVAL, "%s: grad_dtype (dq, dkv) must be QFA_F16 or QFA_BF16", who);
+  if (!aligned16(dout) || !aligned16(dq) || !aligned16(dkv))
+    return set_error(QFA_EINVAL, "%s: dout, dq, dkv must be 16-byte aligned", who);
+  if (!strides_ok(sdob, sdoh, sdon, D, 2) || !strides_ok(sdqb, sdqh, sdqn, D, 2) || !strides_ok(sdkb, sdkh, sdkn, D, 2))
+    return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
+  // the row copies of the two-kernel path form offsets inside a 32-row block in 31 bits
+  if (sqn >= (1 << 23) || son >= (1 << 23) || sdon >= (1 << 23))
+    return set_error(QFA_EUNSUPPORTED, "%s: token strides of 2^23 elements or more are not supported", who);
+  if (workspace) {
+    const int64_t need = skv_bwd_workspace_bytes(B, H, Nq, Nk, D);
+    if (!aligned16(workspace) || workspace_bytes < need)
+      return set_error(QFA_EINVAL, "%s: workspace must be 16-byte aligned and hold %lld bytes "
+                       "(qfa_attn_bwd_shared_kv_workspace_bytes), got %lld", who, (long long)need, (long long)workspace_bytes);
+    a.workspace = need > 0 ? workspace : nullptr;
+  }
+  return skv_bwd_one_pass(Nq, D) ? launch_skv_bwd(a, (hipStream_t)stream) : launch_skv_bwd_long(a, (hipStream_t)stream);
+}
+
 int qfa_attn_bwd_shared_kv(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
                            const void *o, const void *dout, const float *lse, void *dq, void *dkv, int io_dtype,
                            int grad_dtype, const float *grad_scale,
@@ -331,36 +375,26 @@ int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void 
                            int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
                            int64_t sdkh, int64_t sdkn, float sm_scale, void *workspace, int64_t workspace_bytes,
                                  void *stream) {
-  const char *who = "attn_bwd_shared_kv";
-  SkvAttnArgs a;
-  memset(&a, 0, sizeof(a));
-  a.q = q; a.codes = codes; a.scale = scale; a.zp = zp; a.o = const_cast<void *>(o); a.lse = const_cast<float *>(lse);
-  a.dout = dout; a.dq = dq; a.dkv = dkv; a.grad_dtype = grad_dtype; a.grad_scale = grad_scale;
-  a.B = B; a.H = H; a.Nq = Nq; a.Nk = Nk; a.D = D; a.io_dtype = io_dtype; a.scale_dtype = scale_dtype;
-  a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.scb = scb; a.sch = sch; a.scn = scn; a.sob = sob; a.soh = soh; a.son = son;
-  a.sdob = sdob; a.sdoh = sdoh; a.sdon = sdon; a.sdqb = sdqb; a.sdqh = sdqh; a.sdqn = sdqn;
-  a.sdkb = sdkb; a.sdkh = sdkh; a.sdkn = sdkn;
-  a.sm_scale = sm_scale;
-  if (int e = check_shared_kv(who, a)) return e;
-  if (!dout || !dq || !dkv) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
-  if (io_dtype != QFA_F16) return set_error(QFA_EUNSUPPORTED, "%s: io_dtype (q, o, dout) must be QFA_F16", who);
-  if (grad_dtype != QFA_F16 && grad_dtype != QFA_BF16)
-    return set_error(QFA_EINVAL, "%s: grad_dtype (dq, dkv) must be QFA_F16 or QFA_BF16", who);
-  if (!aligned16(dout) || !aligned16(dq) || !aligned16(dkv))
-    return set_error(QFA_EINVAL, "%s: dout, dq, dkv must be 16-byte aligned", who);
-  if (!strides_ok(sdob, sdoh, sdon, D, 2) || !strides_ok(sdqb, sdqh, sdqn, D, 2) || !strides_ok(sdkb, sdkh, sdkn, D, 2))
-    return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
-  // the row copies of the two-kernel path form offsets inside a 32-row block in 31 bits
-  if (sqn >= (1 << 23) || son >= (1 << 23) || sdon >= (1 << 23))
-    return set_error(QFA_EUNSUPPORTED, "%s: token strides of 2^23 elements or more are not supported", who);
-  if (workspace) {
-    const int64_t need = skv_bwd_workspace_bytes(B, H, Nq, Nk, D);
-    if (!aligned16(workspace) || workspace_bytes < need)
-      return set_error(QFA_EINVAL, "%s: workspace must be 16-byte aligned and hold %lld bytes "
-                       "(qfa_attn_bwd_shared_kv_workspace_bytes), got %lld", who, (long long)need, (long long)workspace_bytes);
-    a.workspace = need > 0 ? workspace : nullptr;
-  }
-  return skv_bwd_one_pass(Nq, D) ? launch_skv_bwd(a, (hipStream_t)stream) : launch_skv_bwd_long(a, (hipStream_t)stream);
+  return skv_bwd_entry("attn_bwd_shared_kv", 0, QFA_F16, q, codes, scale, scale_dtype, zp, o, dout, lse, dq, dkv, io_dtype, grad_dtype, grad_scale, B, H, Nq, Nk, D, sqb, sqh, sqn,
+                       scb, sch, scn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn, sm_scale, workspace,
+                       workspace_bytes, stream);
+}
+
+int qfa_attn_bwd_shared_kv_is_direct(int64_t Nq, int D) {
+  return Nq > 0 && (D == 64 || D == 128 || D == 256) && skv_bwd_one_pass(Nq, D);
+}
+
+int qfa_attn_bwd_shared_kv_direct(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
+                           const void *o, const void *dout, const float *lse, void *dq, void *dkv, int io_dtype,
+                           int dout_dtype, int grad_dtype,
+                           int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn,
+                           int64_t scb, int64_t sch, int64_t scn, int64_t sob, int64_t soh, int64_t son, int64_t sdob,
+                           int64_t sdoh, int64_t sdon, int64_t sdqb, int64_t sdqh, int64_t sdqn, int64_t sdkb,
+                           int64_t sdkh, int64_t sdkn, float sm_scale, void *workspace, int64_t workspace_bytes,
+                                 void *stream) {
+  return skv_bwd_entry("attn_bwd_shared_kv_direct", 1, dout_dtype, q, codes, scale, scale_dtype, zp, o, dout, lse, dq, dkv, io_dtype, grad_dtype, nullptr, B, H, Nq, Nk, D, sqb, sqh, sqn,
+                       scb, sch, scn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn, sm_scale, workspace,
+                       workspace_bytes, stream);
 }
 
 int64_t qfa_attn_fwd_cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {

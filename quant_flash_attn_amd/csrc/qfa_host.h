@@ -87,6 +87,7 @@ struct SkvAttnArgs {
   float sm_scale;
   int D, io_dtype, scale_dtype;
   int grad_dtype; const float *grad_scale;   // backward only: type of dq / dkv, optional device scalar multiplying them
+  int direct, dout_dtype;   // backward in one pass only: q and o of io_dtype, dO of dout_dtype, scaled inside
 };
 int launch_skv_fwd(const SkvAttnArgs &a, hipStream_t st);
 int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);

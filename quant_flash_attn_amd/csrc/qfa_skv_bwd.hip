@@ -33,6 +33,46 @@
 
 namespace qfa {
 
+// ---- the power of two by which dO is scaled (see dout_max_kernel)
+template <typename T> __device__ __forceinline__ float max_abs8(const u32x4 w, float m) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(lo_to_f32<T>(w[e])), fabsf(hi_to_f32<T>(w[e]))));
+  return m;
+}
+// largest magnitude of the 16 bytes of scales a thread loads at a time
+template <typename S> __device__ __forceinline__ float max_abs_chunk(const u32x4 w, float m) {
+  if constexpr (sizeof(S) == 2) {
+    return max_abs8<S>(w, m);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned x = w[e];   // (this compiler's bit cast of a vector's element takes element 0)
+      m = fmaxf(m, fabsf(__builtin_bit_cast(float, x)));
+    }
+    return m;
+  }
+}
+__device__ __forceinline__ float block_max_256(float m, float *red) {
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = m;
+  __syncthreads();
+  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+// floor(log2(c / y)) for c = 2^ce and a positive normal y, exactly (no logarithm): y = m * 2^e with m in [1, 2)
+__device__ __forceinline__ int floor_log2_quot(int ce, float y) {
+  const unsigned b = __builtin_bit_cast(unsigned, y);
+  const int e = (int)((b >> 23) & 0xff) - 127;
+  return ce - e - ((b & 0x7fffffu) != 0 ? 1 : 0);
+}
+
+// k of the largest magnitudes of dO and of the key scales
+__device__ __forceinline__ int dout_exponent(float m, float ms) {
+  m = fmaxf(m, 1e-30f);     // inf stays inf: k = -100 below
+  ms = fmaxf(ms, 1e-30f);
+  return max(-100, min(100, min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m))));
+}
+
 struct SkvBwdArgs {
   const _Float16 *q, *o, *dout;
   const int8_t *codes; const void *scale; const int8_t *zp;
@@ -40,6 +80,7 @@ struct SkvBwdArgs {
   _Float16 *dq, *dkv;          // 16-bit outputs: binary16, or bfloat16 when grad_bf16 is set
   const float *grad_scale;     // nullable device scalar: dq and dkv are multiplied by it before rounding
   int grad_bf16;
+  int direct, q_bf16, do_bf16;   // direct: q, o and dO as the caller has them, dO scaled here (grad_scale is not used)
   int64_t H;
   int Nq, Nk, BH;
   int splits, tiles_per_split;   // workgroups that share the keys of a (batch, head)
@@ -95,7 +136,7 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wave_off = wave * SM::WAVE;
   float *stat = reinterpret_cast<float *>(smem + SM::OFF_STAT);
-  const float osc = a.grad_scale ? *a.grad_scale : 1.0f;
+  float osc = a.grad_scale ? *a.grad_scale : 1.0f;
   auto pack_out = [&](float x, float y) -> unsigned {
     return a.grad_bf16 ? pack2<__bf16>(x * osc, y * osc) : pack2<_Float16>(x * osc, y * osc);
   };
@@ -142,24 +183,67 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     const _Float16 *orow = a.o + b * a.sob + h * a.soh + (int64_t)pi_c * a.son;
     const _Float16 *drow = a.dout + b * a.sdob + h * a.sdoh + (int64_t)pi_c * a.sdon;
     float dsum = 0.f, rq = 0.f, rd = 0.f;
+    constexpr int CPT = CPR / 8;   // chunks per thread
+    u32x4 qv[CPT], dv[CPT], ov[CPT];
 #pragma unroll
-    for (int c = part; c < CPR; c += 8) {
-      u32x4 qv = {0u, 0u, 0u, 0u}, dv = qv, ov = qv;
+    for (int i = 0; i < CPT; ++i) {
+      qv[i] = dv[i] = ov[i] = u32x4{0u, 0u, 0u, 0u};
       if (valid) {
-        qv = *reinterpret_cast<const u32x4 *>(qrow + c * 8);
-        dv = *reinterpret_cast<const u32x4 *>(drow + c * 8);
-        ov = *reinterpret_cast<const u32x4 *>(orow + c * 8);
+        const int c = part + 8 * i;
+        qv[i] = *reinterpret_cast<const u32x4 *>(qrow + c * 8);
+        dv[i] = *reinterpret_cast<const u32x4 *>(drow + c * 8);
+        ov[i] = *reinterpret_cast<const u32x4 *>(orow + c * 8);
       }
+    }
+    if (a.direct) {
+      // What otherwise takes two to four launches in front of this one: bf16 q and o cast, dO scaled by a power of two that is
+      // this workgroup's own (its queries and its keys decide it)
+      float m = 0.f, ms = 0.f;
+      const int64_t k0 = tk0 + (int64_t)t0 * SKV_TILE;
+      const int nk = min(ntiles * SKV_TILE, a.Nk - t0 * SKV_TILE);
+#pragma unroll 8
+      for (int j = tid; j < nk; j += 256) ms = fmaxf(ms, fabsf((float)reinterpret_cast<const S *>(a.scale)[k0 + j]));
+      auto as_half = [](u32x4 w) -> u32x4 {
+        u32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = pack2<_Float16>(lo_to_f32<__bf16>(w[e]), hi_to_f32<__bf16>(w[e]));
+        return r;
+      };
+      auto scaled = [&](u32x4 w, float f) -> u32x4 {
+        u32x4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          r[e] = a.do_bf16 ? pack2<_Float16>(lo_to_f32<__bf16>(w[e]) * f, hi_to_f32<__bf16>(w[e]) * f)
+                           : pack2<_Float16>(lo_to_f32<_Float16>(w[e]) * f, hi_to_f32<_Float16>(w[e]) * f);
+        return r;
+      };
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) m = a.do_bf16 ? max_abs8<__bf16>(dv[i], m) : max_abs8<_Float16>(dv[i], m);
+      m = block_max_256(m, stat);
+      const int k = __builtin_amdgcn_readfirstlane(dout_exponent(m, block_max_256(ms, stat + 4)));
+      const float f = __builtin_ldexpf(1.0f, k);
+      osc = __builtin_ldexpf(1.0f, -k);
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) {
+        dv[i] = scaled(dv[i], f);
+        if (a.q_bf16) qv[i] = as_half(qv[i]), ov[i] = as_half(ov[i]);
+      }
+      __syncthreads();   // the maxima are read: `stat` is written below
+    }
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int c = part + 8 * i;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float d0 = lo_to_f32<_Float16>(dv[e]), d1 = hi_to_f32<_Float16>(dv[e]);
-        rq += lo_to_f32<_Float16>(qv[e]) + hi_to_f32<_Float16>(qv[e]);
+        const unsigned dw = dv[i][e], qw = qv[i][e], ow = ov[i][e];
+        const float d0 = lo_to_f32<_Float16>(dw), d1 = hi_to_f32<_Float16>(dw);
+        rq += lo_to_f32<_Float16>(qw) + hi_to_f32<_Float16>(qw);
         rd += d0 + d1;
-        dsum += lo_to_f32<_Float16>(ov[e]) * d0 + hi_to_f32<_Float16>(ov[e]) * d1;
+        dsum += lo_to_f32<_Float16>(ow) * d0 + hi_to_f32<_Float16>(ow) * d1;
       }
       const int off = pi * (D * 2) + ((c ^ row_swizzle<CPR>(pi)) << 4);
-      *reinterpret_cast<u32x4 *>(smem + SM::OFF_Q + off) = qv;
-      *reinterpret_cast<u32x4 *>(smem + SM::OFF_DO + off) = dv;
+      *reinterpret_cast<u32x4 *>(smem + SM::OFF_Q + off) = qv[i];
+      *reinterpret_cast<u32x4 *>(smem + SM::OFF_DO + off) = dv[i];
     }
 #pragma unroll
     for (int m = 1; m < 8; m *= 2) {
@@ -413,6 +497,7 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
           const int d = 32 * db + 8 * aa + 4 * g + bb;
           r[bb] = dq[db][4 * aa + bb] - w_tot + mg[d * 32 + lr] + mg[MG + d * 32 + lr] + mg[2 * MG + d * 32 + lr];
         }
+        if (a.direct) r = f32x4{r[0] * osc, r[1] * osc, r[2] * osc, r[3] * osc};
         *reinterpret_cast<f32x4 *>(prow + 32 * db + 8 * aa + 4 * g) = r;
       }
   } else if (wave == 0 && lr < a.Nq) {
@@ -442,6 +527,7 @@ template <typename S, int D> static int launch_skv_bwd_sd(const SkvAttnArgs &x, 
   a.codes = x.codes; a.scale = x.scale; a.zp = x.zp; a.lse = x.lse;
   a.dq = static_cast<_Float16 *>(x.dq); a.dkv = static_cast<_Float16 *>(x.dkv);
   a.grad_scale = x.grad_scale; a.grad_bf16 = x.grad_dtype == QFA_BF16;
+  a.direct = x.direct; a.q_bf16 = x.io_dtype == QFA_BF16; a.do_bf16 = x.dout_dtype == QFA_BF16;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk;
   a.sqb = x.sqb; a.sqh = x.sqh; a.sqn = x.sqn; a.scb = x.scb; a.sch = x.sch; a.scn = x.scn;
   a.sob = x.sob; a.soh = x.soh; a.son = x.son; a.sdob = x.sdob; a.sdoh = x.sdoh; a.sdon = x.sdon;
@@ -514,38 +600,6 @@ int launch_skv_bwd(const SkvAttnArgs &x, hipStream_t st) {
 // every block of the second reduces all of them again (a few KB out of the L2) before it scales its share.
 constexpr int NORM_BLOCKS = 2048;   // blocks of the first launch = pairs of floats in the partials buffer
 
-template <typename T> __device__ __forceinline__ float max_abs8(const u32x4 w, float m) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(lo_to_f32<T>(w[e])), fabsf(hi_to_f32<T>(w[e]))));
-  return m;
-}
-// largest magnitude of the 16 bytes of scales a thread loads at a time
-template <typename S> __device__ __forceinline__ float max_abs_chunk(const u32x4 w, float m) {
-  if constexpr (sizeof(S) == 2) {
-    return max_abs8<S>(w, m);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const unsigned x = w[e];   // (this compiler's bit cast of a vector's element takes element 0)
-      m = fmaxf(m, fabsf(__builtin_bit_cast(float, x)));
-    }
-    return m;
-  }
-}
-__device__ __forceinline__ float block_max_256(float m, float *red) {
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  __syncthreads();
-  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = m;
-  __syncthreads();
-  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-// floor(log2(c / y)) for c = 2^ce and a positive normal y, exactly (no logarithm): y = m * 2^e with m in [1, 2)
-__device__ __forceinline__ int floor_log2_quot(int ce, float y) {
-  const unsigned b = __builtin_bit_cast(unsigned, y);
-  const int e = (int)((b >> 23) & 0xff) - 127;
-  return ce - e - ((b & 0x7fffffu) != 0 ? 1 : 0);
-}
-
 // 16 bytes per thread and trip for both vectors (the scales' last ns % (16 / sizeof(S)) elements one by one)
 template <typename T, typename S>
 __global__ __launch_bounds__(256) void dout_max_kernel(const T *dout, int64_t n8, const S *scale, int64_t ns, float *partials) {
@@ -586,10 +640,8 @@ __global__ __launch_bounds__(256) void dout_scale_kernel(const T *dout, int64_t 
     m = fmaxf(m, partials[2 * i]);
     ms = fmaxf(ms, partials[2 * i + 1]);
   }
-  m = fmaxf(block_max_256(m, red), 1e-30f);     // inf stays inf: k = -100 below
-  ms = fmaxf(block_max_256(ms, red), 1e-30f);
-  int k = min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m));
-  k = max(-100, min(100, k));
+  m = block_max_256(m, red);
+  const int k = dout_exponent(m, block_max_256(ms, red));
   const float f = __builtin_ldexpf(1.0f, k);
   if (blockIdx.x == 0 && threadIdx.x == 0) back[0] = __builtin_ldexpf(1.0f, -k);
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;

@@ -49,6 +49,8 @@ struct Api {
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
   QFA_ENTRY(qfa_attn_bwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd_shared_kv_split);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_is_direct);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_direct);
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
@@ -82,6 +84,8 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
   QFA_ENTRY(qfa_attn_bwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd_shared_kv_split);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_is_direct);
+  QFA_ENTRY(qfa_attn_bwd_shared_kv_direct);
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_cache);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
@@ -678,8 +682,9 @@ std::tuple<Tensor, Tensor> skv_fwd(const Tensor &q_in, const Tensor &codes_in, c
 
 std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, const Tensor &scale_in, const Tensor &zp_in,
                                    const Tensor &o_in, const Tensor &do_in, const Tensor &lse_in, double sm,
-                                   at::ScalarType grad_dtype, const std::optional<Tensor> &grad_scale_in, bool split) {
-  TORCH_CHECK_TYPE(q_in.scalar_type() == at::kHalf && o_in.scalar_type() == at::kHalf,
+                                   at::ScalarType grad_dtype, const std::optional<Tensor> &grad_scale_in, bool split,
+                                   bool direct = false) {
+  TORCH_CHECK_TYPE(direct || (q_in.scalar_type() == at::kHalf && o_in.scalar_type() == at::kHalf),
                    "the shared-KV backward kernel computes in float16: q and o must be float16");
   TORCH_CHECK_TYPE(is_io(grad_dtype), "grad_dtype must be float16 or bfloat16, got ", grad_dtype);
   check_codes(codes_in, "codes");
@@ -698,12 +703,23 @@ std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, c
   const Tensor s = as_is ? scale_in : scale_in.to(at::kFloat);
   const Tensor scale = flat(s, s.scalar_type(), B * H * Nk, "scale"), zp = flat(zp_in, at::kChar, B * H * Nk, "zero_point"),
                lse = flat(lse_in, at::kFloat, B * H * Nq, "lse");
-  const Tensor q = rows16(q_in), codes = rows16(codes_in), o = rows16(o_in), dout = rows16(to(do_in, at::kHalf));
+  const Tensor q = rows16(q_in), codes = rows16(codes_in), o = rows16(o_in), dout = rows16(to(do_in, direct ? io_dtype(do_in) : at::kHalf));
   Tensor dq = empty({B, H, Nq, D}, grad_dtype, q), dkv = empty({B, H, Nk, D}, grad_dtype, q);
   // scratch for the split over keys where B*H alone cannot fill the GPU (0: no split)
   const int64_t ws_bytes = split ? api.qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) : 0;
   Tensor ws;
   if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, q);
+  if (direct) {
+    check(api.qfa_attn_bwd_shared_kv_direct(q.data_ptr(), codes.data_ptr<int8_t>(), scale.data_ptr(), dtype_code(scale.scalar_type()),
+                                            zp.data_ptr<int8_t>(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
+                                            dq.data_ptr(), dkv.data_ptr(), dtype_code(q.scalar_type()),
+                                            dtype_code(dout.scalar_type()), dtype_code(grad_dtype), B, H, Nq, Nk, (int)D,
+                                            QFA_STRIDES(q), QFA_STRIDES(codes), QFA_STRIDES(o), QFA_STRIDES(dout),
+                                            QFA_STRIDES(dq), QFA_STRIDES(dkv), (float)sm, ws_bytes > 0 ? ws.data_ptr() : nullptr,
+                                            ws_bytes, stream_of(q)),
+          "qfa_attn_bwd_shared_kv_direct");
+    return {dq, dkv};
+  }
   check(api.qfa_attn_bwd_shared_kv_split(q.data_ptr(), codes.data_ptr<int8_t>(), scale.data_ptr(), dtype_code(scale.scalar_type()),
                                    zp.data_ptr<int8_t>(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
                                    dq.data_ptr(), dkv.data_ptr(), QFA_F16, dtype_code(grad_dtype),
@@ -774,8 +790,15 @@ struct SharedFn : torch::autograd::Function<SharedFn> {
     // so dO is handed over scaled by a power of two chosen on the device (no synchronisation) from
     // its largest magnitude and from the largest key scale, and the kernels scale dQ and dKV back
     // while they round them.  q and o convert exactly from bf16 (more mantissa, values of order one).
-    const Normalised n = normalise(grads[0], s[2], q, o);
-    auto [dq, dkv] = skv_bwd(n.q, s[1], s[2], s[3], n.o, n.dout, s[5], ctx->saved_data["sm"].toDouble(), q.scalar_type(), n.back, true);
+    // Where one pass takes all queries it does that itself.
+    const double sm = ctx->saved_data["sm"].toDouble();
+    Tensor dq, dkv;
+    if (is_io(o.scalar_type()) && o.scalar_type() == q.scalar_type() && api.qfa_attn_bwd_shared_kv_is_direct(q.size(2), (int)q.size(3))) {
+      std::tie(dq, dkv) = skv_bwd(q, s[1], s[2], s[3], o, grads[0], s[5], sm, q.scalar_type(), std::nullopt, true, true);
+    } else {
+      const Normalised n = normalise(grads[0], s[2], q, o);
+      std::tie(dq, dkv) = skv_bwd(n.q, s[1], s[2], s[3], n.o, n.dout, s[5], sm, q.scalar_type(), n.back, true);
+    }
     return {dq, to(dkv, (at::ScalarType)ctx->saved_data["kv_dtype"].toInt()), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };

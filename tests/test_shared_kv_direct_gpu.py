@@ -1,0 +1,80 @@
+"""Up to 32 queries, shared-KV backward: q, o and dO as the caller has them, cast and scaled inside, against the launches that cast
+and scale first, and with gradients of very different size in different heads."""
+import pytest
+import torch
+
+from quant_flash_attn_amd import _lib
+from quant_flash_attn_amd.quant_flash_attn import _normalised_dout
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+
+
+def _tensors(B, H, Nq, Nk, D, dtype, sdtype):
+    g = torch.Generator().manual_seed(Nq + Nk + D)
+    r = lambda n: torch.randn((B, H, n, D), generator=g)
+    q, o, do = (r(Nq).to(dtype).to(DEV) for _ in range(3))
+    codes = torch.randint(-128, 128, (B, H, Nk, D), dtype=torch.int8, generator=g).to(DEV)
+    scale = (torch.rand((B, H, Nk, 1), generator=g) * 0.02 + 0.001).to(sdtype).to(DEV)
+    zp = torch.randint(-20, 20, (B, H, Nk, 1), dtype=torch.int8, generator=g).to(DEV)
+    lse = (torch.rand((B, H, Nq), generator=g) * 2 + 6).to(DEV)
+    return q, o, do, codes, scale, zp, lse
+
+
+def _direct(q, o, do, codes, scale, zp, lse, sm, split):
+    L = _lib.lib()
+    B, H, Nq, D = q.shape
+    Nk = codes.shape[2]
+    dq, dkv = torch.empty_like(q), torch.empty((B, H, Nk, D), dtype=q.dtype, device=DEV)
+    n = L.qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) if split else 0
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device=DEV)
+    st = lambda t: t.stride()[:3]
+    rc = L.qfa_attn_bwd_shared_kv_direct(q.data_ptr(), codes.data_ptr(), scale.data_ptr(), CODE[scale.dtype], zp.data_ptr(),
+                                         o.data_ptr(), do.data_ptr(), lse.data_ptr(), dq.data_ptr(), dkv.data_ptr(), CODE[q.dtype],
+                                         CODE[do.dtype], CODE[q.dtype], B, H, Nq, Nk, D, *st(q), *st(codes), *st(o), *st(do), *st(dq),
+                                         *st(dkv), sm, ws.data_ptr() if n else None, n, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.qfa_last_error()
+    return dq, dkv, n
+
+
+def _scaled_first(q, o, do, codes, scale, zp, lse, sm):
+    do16, back = _normalised_dout(do, scale)
+    return _lib.host().skv_bwd(q.half(), codes, scale, zp, o.half(), do16, lse, sm, q.dtype, back)
+
+
+@pytest.mark.parametrize("dtype,sdtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("B,H,Nq,Nk,D", [(1, 1, 1, 33, 64), (1, 3, 16, 700, 128), (2, 3, 17, 257, 64), (1, 2, 32, 4000, 128),
+                                         (1, 2, 5, 100, 256), (1, 4, 16, 3001, 256), (300, 2, 3, 31, 64)])
+def test_direct_against_scaled_first(qfa, B, H, Nq, Nk, D, dtype, sdtype):
+    t = _tensors(B, H, Nq, Nk, D, dtype, sdtype)
+    t[2].mul_(1e-4)
+    want = _scaled_first(*t, 0.09)
+    for split in (False, True):
+        got = _direct(*t, 0.09, split)
+        for a, b in zip(got[:2], want):
+            # another power of two per workgroup: the same products but for what binary16 loses below 2^-14 of the largest (2^-10
+            # of such a value), and with a split another order of fp32 sums, rounded to 8 bits once
+            assert (a.double() - b.double()).norm() <= 2.0 ** -8 * b.double().norm()
+    assert _lib.lib().qfa_attn_bwd_shared_kv_is_direct(33, 64) == 0 and _lib.lib().qfa_attn_bwd_shared_kv_is_direct(17, 256) == 0
+
+
+def test_heads_do_not_share_the_scaling(qfa):
+    """Gradients 2^40 apart in two heads: each head's are as good as alone (one scaling for both loses the small ones)."""
+    q, o, do, codes, scale, zp, lse = _tensors(1, 2, 16, 500, 128, torch.bfloat16, torch.float16)
+    do[:, 0] *= 2.0 ** -40
+    dq, dkv, _ = _direct(q, o, do, codes, scale, zp, lse, 0.09, False)
+    for h in (0, 1):
+        one = [x[:, h:h + 1].contiguous() for x in (q, o, do, codes, scale, zp, lse)]
+        for a, b in zip((dq, dkv), _scaled_first(*one, 0.09)):
+            assert b.abs().max() > 0 and torch.equal(a[:, h:h + 1], b)
+
+
+def test_infinite_and_zero_gradients(qfa):
+    q, o, do, codes, scale, zp, lse = _tensors(1, 3, 7, 100, 64, torch.float16, torch.float16)
+    do[:, 0] = 0
+    do[0, 1, 3, 5] = float("inf")
+    dq, dkv, _ = _direct(q, o, do, codes, scale, zp, lse, 0.09, False)
+    assert (dq[:, 0] == 0).all() and (dkv[:, 0] == 0).all()
+    assert not torch.isfinite(dkv[:, 1]).all()
+    assert torch.isfinite(dq[:, 2]).all() and torch.isfinite(dkv[:, 2]).all()
