@@ -260,8 +260,8 @@ int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void 
 
 /*
  * The same on q and o of io_dtype (QFA_F16 or QFA_BF16) and dout of dout_dtype as a caller has them: the casts and the scaling
- * of dO by a power of two (qfa_dout_normalise) happen inside, per workgroup.  For the query blocks that one pass takes, where
- * qfa_attn_bwd_shared_kv_is_direct(Nq, D) is 1 (up to 32 queries, 16 at head_dim 256); others are QFA_EUNSUPPORTED.
+ * of dO by a power of two (qfa_dout_normalise) happen inside, per workgroup.  For query blocks whose rows a workgroup holds, where
+ * qfa_attn_bwd_shared_kv_is_direct(Nq, D) is 1 (up to 128 queries, 16 at head_dim 256); others are QFA_EUNSUPPORTED.
  */
 int qfa_attn_bwd_shared_kv_is_direct(int64_t Nq, int D);
 

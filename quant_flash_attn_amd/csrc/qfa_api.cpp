@@ -326,7 +326,7 @@ static int skv_bwd_entry(const char *who, int direct, int dout_dtype, const void
   if (int e = check_shared_kv(who, a)) return e;
   if (!dout || !dq || !dkv) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
   if (direct) {
-    if (!skv_bwd_one_pass(Nq, D))
+    if (!skv_bwd_direct(Nq, D))
       return set_error(QFA_EUNSUPPORTED, "%s: %lld queries of head_dim %d take the scaled form", who, (long long)Nq, D);
     if (dout_dtype != QFA_F16 && dout_dtype != QFA_BF16) return set_error(QFA_EINVAL, "%s: dout_dtype must be QFA_F16 or QFA_BF16", who);
   }
@@ -381,7 +381,7 @@ int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void 
 }
 
 int qfa_attn_bwd_shared_kv_is_direct(int64_t Nq, int D) {
-  return Nq > 0 && (D == 64 || D == 128 || D == 256) && skv_bwd_one_pass(Nq, D);
+  return Nq > 0 && (D == 64 || D == 128 || D == 256) && skv_bwd_direct(Nq, D);
 }
 
 int qfa_attn_bwd_shared_kv_direct(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,

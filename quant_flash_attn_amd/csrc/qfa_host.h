@@ -87,7 +87,7 @@ struct SkvAttnArgs {
   float sm_scale;
   int D, io_dtype, scale_dtype;
   int grad_dtype; const float *grad_scale;   // backward only: type of dq / dkv, optional device scalar multiplying them
-  int direct, dout_dtype;   // backward in one pass only: q and o of io_dtype, dO of dout_dtype, scaled inside
+  int direct, dout_dtype;   // backward: q and o of io_dtype, dO of dout_dtype, cast and scaled inside (where skv_bwd_direct)
 };
 int launch_skv_fwd(const SkvAttnArgs &a, hipStream_t st);
 int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
@@ -113,6 +113,8 @@ int launch_skv_dkv(const SkvAttnArgs &a, hipStream_t st);
 int launch_split_sum(const SkvAttnArgs &a, int splits, hipStream_t st);
 // one fused backward pass while the per-wave accumulators of dQ fit: 32 queries up to head_dim 128, 16 at 256
 inline bool skv_bwd_one_pass(int64_t Nq, int D) { return D == 256 ? Nq <= 16 : Nq <= 32; }
+// whether the backward's kernels cast and scale their rows themselves: that pass, and the two kernels while dKV's rows stay in LDS
+inline bool skv_bwd_direct(int64_t Nq, int D) { return skv_bwd_one_pass(Nq, D) || (D <= 128 && Nq <= 128); }
 // workgroups that share the keys of a (batch, head) in that pass, given a workspace
 int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D);
 int64_t skv_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);

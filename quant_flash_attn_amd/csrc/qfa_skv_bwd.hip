@@ -33,46 +33,6 @@
 
 namespace qfa {
 
-// ---- the power of two by which dO is scaled (see dout_max_kernel)
-template <typename T> __device__ __forceinline__ float max_abs8(const u32x4 w, float m) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(lo_to_f32<T>(w[e])), fabsf(hi_to_f32<T>(w[e]))));
-  return m;
-}
-// largest magnitude of the 16 bytes of scales a thread loads at a time
-template <typename S> __device__ __forceinline__ float max_abs_chunk(const u32x4 w, float m) {
-  if constexpr (sizeof(S) == 2) {
-    return max_abs8<S>(w, m);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const unsigned x = w[e];   // (this compiler's bit cast of a vector's element takes element 0)
-      m = fmaxf(m, fabsf(__builtin_bit_cast(float, x)));
-    }
-    return m;
-  }
-}
-__device__ __forceinline__ float block_max_256(float m, float *red) {
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  __syncthreads();
-  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = m;
-  __syncthreads();
-  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-// floor(log2(c / y)) for c = 2^ce and a positive normal y, exactly (no logarithm): y = m * 2^e with m in [1, 2)
-__device__ __forceinline__ int floor_log2_quot(int ce, float y) {
-  const unsigned b = __builtin_bit_cast(unsigned, y);
-  const int e = (int)((b >> 23) & 0xff) - 127;
-  return ce - e - ((b & 0x7fffffu) != 0 ? 1 : 0);
-}
-
-// k of the largest magnitudes of dO and of the key scales
-__device__ __forceinline__ int dout_exponent(float m, float ms) {
-  m = fmaxf(m, 1e-30f);     // inf stays inf: k = -100 below
-  ms = fmaxf(ms, 1e-30f);
-  return max(-100, min(100, min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m))));
-}
-
 struct SkvBwdArgs {
   const _Float16 *q, *o, *dout;
   const int8_t *codes; const void *scale; const int8_t *zp;
@@ -185,6 +145,8 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     float dsum = 0.f, rq = 0.f, rd = 0.f;
     constexpr int CPT = CPR / 8;   // chunks per thread
     u32x4 qv[CPT], dv[CPT], ov[CPT];
+    const KeyScaleMax scales(a.scale, sizeof(S) == 4 ? QFA_F32 : QFA_F16, tk0 + (int64_t)t0 * SKV_TILE,
+                             a.direct ? min(ntiles * SKV_TILE, a.Nk - t0 * SKV_TILE) : 1, tid);
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       qv[i] = dv[i] = ov[i] = u32x4{0u, 0u, 0u, 0u};
@@ -198,35 +160,16 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     if (a.direct) {
       // What otherwise takes two to four launches in front of this one: bf16 q and o cast, dO scaled by a power of two that is
       // this workgroup's own (its queries and its keys decide it)
-      float m = 0.f, ms = 0.f;
-      const int64_t k0 = tk0 + (int64_t)t0 * SKV_TILE;
-      const int nk = min(ntiles * SKV_TILE, a.Nk - t0 * SKV_TILE);
-#pragma unroll 8
-      for (int j = tid; j < nk; j += 256) ms = fmaxf(ms, fabsf((float)reinterpret_cast<const S *>(a.scale)[k0 + j]));
-      auto as_half = [](u32x4 w) -> u32x4 {
-        u32x4 r;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = pack2<_Float16>(lo_to_f32<__bf16>(w[e]), hi_to_f32<__bf16>(w[e]));
-        return r;
-      };
-      auto scaled = [&](u32x4 w, float f) -> u32x4 {
-        u32x4 r;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          r[e] = a.do_bf16 ? pack2<_Float16>(lo_to_f32<__bf16>(w[e]) * f, hi_to_f32<__bf16>(w[e]) * f)
-                           : pack2<_Float16>(lo_to_f32<_Float16>(w[e]) * f, hi_to_f32<_Float16>(w[e]) * f);
-        return r;
-      };
+      float m = 0.f;
 #pragma unroll
       for (int i = 0; i < CPT; ++i) m = a.do_bf16 ? max_abs8<__bf16>(dv[i], m) : max_abs8<_Float16>(dv[i], m);
-      m = block_max_256(m, stat);
-      const int k = __builtin_amdgcn_readfirstlane(dout_exponent(m, block_max_256(ms, stat + 4)));
+      const int k = block_dout_exponent(m, scales.get(), stat);
       const float f = __builtin_ldexpf(1.0f, k);
       osc = __builtin_ldexpf(1.0f, -k);
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
-        dv[i] = scaled(dv[i], f);
-        if (a.q_bf16) qv[i] = as_half(qv[i]), ov[i] = as_half(ov[i]);
+        dv[i] = scaled_dout(dv[i], a.do_bf16, f);
+        if (a.q_bf16) qv[i] = half_of_bf16(qv[i]), ov[i] = half_of_bf16(ov[i]);
       }
       __syncthreads();   // the maxima are read: `stat` is written below
     }

@@ -27,6 +27,7 @@ struct SkvBwdLongArgs {
   _Float16 *dq, *dkv;          // 16-bit outputs: binary16, or bfloat16 when grad_bf16 is set
   const float *grad_scale;     // nullable device scalar: dq and dkv are multiplied by it before rounding
   int grad_bf16;
+  int direct, q_bf16, do_bf16;   // dQ, up to head_dim 128: q, o and dO as the caller has them, dO scaled here (no grad_scale)
   int64_t H;
   int Nq, Nk, BH, qblocks, kchunks, cpw;   // cpw: key chunks per workgroup of the dKV kernel
   int64_t sqb, sqh, sqn, scb, sch, scn, sob, soh, son, sdob, sdoh, sdon, sdqb, sdqh, sdqn, sdkb, sdkh, sdkn;
@@ -66,7 +67,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
   auto scale_of = [](unsigned w) -> float {
     return scale_to_f32<S>(w);
   };
-  const float osc = a.grad_scale ? *a.grad_scale : 1.0f;
+  float osc = a.grad_scale ? *a.grad_scale : 1.0f;
   auto pack_out = [&](float x, float y) -> unsigned {
     return a.grad_bf16 ? pack2<__bf16>(x * osc, y * osc) : pack2<_Float16>(x * osc, y * osc);
   };
@@ -82,17 +83,35 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
   const _Float16 *qrow = a.q + b * a.sqb + h * a.sqh + (int64_t)qi_c * a.sqn;
   const _Float16 *orow = a.o + b * a.sob + h * a.soh + (int64_t)qi_c * a.son;
   const _Float16 *drow = a.dout + b * a.sdob + h * a.sdoh + (int64_t)qi_c * a.sdon;
-  u32x4 qf[KS], dof[KS];
+  u32x4 qf[KS], dof[KS], of[KS];
+  const KeyScaleMax scales(a.scale, sizeof(S) == 4 ? QFA_F32 : QFA_F16, tk0, a.direct ? a.Nk : 1, tid);
   float rq = 0.f, rd = 0.f, delta = 0.f;
 #pragma unroll
   for (int m = 0; m < KS; ++m) {
     const int d0 = 64 * (m / 2) + 16 * G + 8 * (m % 2);
     qf[m] = *reinterpret_cast<const u32x4 *>(qrow + d0);
     dof[m] = *reinterpret_cast<const u32x4 *>(drow + d0);
-    const u32x4 ov = *reinterpret_cast<const u32x4 *>(orow + d0);
+    of[m] = *reinterpret_cast<const u32x4 *>(orow + d0);
+  }
+  if (D <= 128 && a.direct) {   // a power of two of the workgroup's own queries and of its head's keys
+    __shared__ float red[8];
+    float mx = 0.f;
+#pragma unroll
+    for (int m = 0; m < KS; ++m) mx = a.do_bf16 ? max_abs8<__bf16>(dof[m], mx) : max_abs8<_Float16>(dof[m], mx);
+    const int k = block_dout_exponent(mx, scales.get(), red);
+    const float f = __builtin_ldexpf(1.0f, k);
+    osc = __builtin_ldexpf(1.0f, -k);
+#pragma unroll
+    for (int m = 0; m < KS; ++m) {
+      dof[m] = scaled_dout(dof[m], a.do_bf16, f);
+      if (a.q_bf16) qf[m] = half_of_bf16(qf[m]), of[m] = half_of_bf16(of[m]);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < KS; ++m) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const unsigned qw = qf[m][e], dw = dof[m][e], ow = ov[e];
+      const unsigned qw = qf[m][e], dw = dof[m][e], ow = of[m][e];
       const float d0f = lo_to_f32<_Float16>(dw), d1f = hi_to_f32<_Float16>(dw);
       rq += lo_to_f32<_Float16>(qw) + hi_to_f32<_Float16>(qw);
       rd += d0f + d1f;
@@ -580,6 +599,7 @@ template <typename S, int D> static int launch_skv_bwd_long_sd(const SkvAttnArgs
   a.codes = x.codes; a.scale = x.scale; a.zp = x.zp; a.lse = x.lse;
   a.dq = static_cast<_Float16 *>(x.dq); a.dkv = static_cast<_Float16 *>(x.dkv);
   a.grad_scale = x.grad_scale; a.grad_bf16 = x.grad_dtype == QFA_BF16;
+  a.direct = x.direct; a.q_bf16 = x.io_dtype == QFA_BF16; a.do_bf16 = x.dout_dtype == QFA_BF16;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk;
   a.sqb = x.sqb; a.sqh = x.sqh; a.sqn = x.sqn; a.scb = x.scb; a.sch = x.sch; a.scn = x.scn;
   a.sob = x.sob; a.soh = x.soh; a.son = x.son; a.sdob = x.sdob; a.sdoh = x.sdoh; a.sdon = x.sdon;

@@ -137,4 +137,103 @@ __device__ __forceinline__ u32x2 tie(u32x2 w) {
   return w;
 }
 
+// ---- the power of two by which dO is scaled (see dout_max_kernel, qfa_skv_bwd.hip)
+template <typename T> __device__ __forceinline__ float max_abs8(const u32x4 w, float m) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(lo_to_f32<T>(w[e])), fabsf(hi_to_f32<T>(w[e]))));
+  return m;
+}
+// largest magnitude of the 16 bytes of scales a thread loads at a time
+template <typename S> __device__ __forceinline__ float max_abs_chunk(const u32x4 w, float m) {
+  if constexpr (sizeof(S) == 2) {
+    return max_abs8<S>(w, m);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned x = w[e];   // (this compiler's bit cast of a vector's element takes element 0)
+      m = fmaxf(m, fabsf(__builtin_bit_cast(float, x)));
+    }
+    return m;
+  }
+}
+__device__ __forceinline__ float block_max_256(float m, float *red) {
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = m;
+  __syncthreads();
+  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+// floor(log2(c / y)) for c = 2^ce and a positive normal y, exactly (no logarithm): y = m * 2^e with m in [1, 2)
+__device__ __forceinline__ int floor_log2_quot(int ce, float y) {
+  const unsigned b = __builtin_bit_cast(unsigned, y);
+  const int e = (int)((b >> 23) & 0xff) - 127;
+  return ce - e - ((b & 0x7fffffu) != 0 ? 1 : 0);
+}
+
+// k of the largest magnitudes of dO and of the key scales
+__device__ __forceinline__ int dout_exponent(float m, float ms) {
+  m = fmaxf(m, 1e-30f);     // inf stays inf: k = -100 below
+  ms = fmaxf(ms, 1e-30f);
+  return max(-100, min(100, min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m))));
+}
+// eight bf16 values as binary16; eight of dO (bf16 or binary16) times f, as binary16
+__device__ __forceinline__ u32x4 half_of_bf16(u32x4 w) {
+  u32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = pack2<_Float16>(lo_to_f32<__bf16>(w[e]), hi_to_f32<__bf16>(w[e]));
+  return r;
+}
+__device__ __forceinline__ u32x4 scaled_dout(u32x4 w, int bf16, float f) {
+  u32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    r[e] = bf16 ? pack2<_Float16>(lo_to_f32<__bf16>(w[e]) * f, hi_to_f32<__bf16>(w[e]) * f)
+                : pack2<_Float16>(lo_to_f32<_Float16>(w[e]) * f, hi_to_f32<_Float16>(w[e]) * f);
+  return r;
+}
+// The largest of n key scales (fp32 or fp16) from k0 on, as one of 256 threads finds it: the first thousand are requested here
+// and looked at with the others later, so that the rows that the caller loads in between hide them.
+struct KeyScaleMax {
+  const void *p;
+  int n, tid;
+  bool f32;
+  float first[4];
+  __device__ __forceinline__ float at(int j) const {
+    return f32 ? static_cast<const float *>(p)[j] : (float)static_cast<const _Float16 *>(p)[j];
+  }
+  __device__ __forceinline__ KeyScaleMax(const void *scale, int dtype, int64_t k0, int n_, int tid_) : n(n_), tid(tid_), f32(dtype == QFA_F32) {
+    p = f32 ? static_cast<const void *>(static_cast<const float *>(scale) + k0)
+            : static_cast<const void *>(static_cast<const _Float16 *>(scale) + k0);
+    if (f32) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) first[i] = static_cast<const float *>(p)[min(tid + 256 * i, n - 1)];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) first[i] = (float)static_cast<const _Float16 *>(p)[min(tid + 256 * i, n - 1)];
+    }
+  }
+  __device__ __forceinline__ float get() const {
+    float ms = fmaxf(fmaxf(fabsf(first[0]), fabsf(first[1])), fmaxf(fabsf(first[2]), fabsf(first[3])));
+#pragma unroll 8
+    for (int j = tid + 1024; j < n; j += 256) ms = fmaxf(ms, fabsf(at(j)));
+    return ms;
+  }
+};
+// dout_exponent of 256 threads' m and ms; red: 8 floats of LDS that nobody uses
+__device__ __forceinline__ int block_dout_exponent(float m, float ms, float *red) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    m = fmaxf(m, __shfl_xor(m, off, 64));
+    ms = fmaxf(ms, __shfl_xor(ms, off, 64));
+  }
+  if (threadIdx.x % 64 == 0) {
+    red[threadIdx.x / 64] = m;
+    red[4 + threadIdx.x / 64] = ms;
+  }
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  ms = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
+  return __builtin_amdgcn_readfirstlane(dout_exponent(m, ms));
+}
+
 }  // namespace qfa

@@ -26,6 +26,7 @@ struct SkvDkvArgs {
   const float *grad_scale;     // nullable device scalar: dkv is multiplied by it before rounding
   int64_t H;
   int Nq, Nk, BH, grad_bf16, scale_dtype;
+  int direct, q_bf16, do_bf16;   // resident rows only: q, o and dO as the caller has them, dO scaled here (no grad_scale)
   int wgs_per_bh, tiles_per_wg;
   int64_t sqb, sqh, sqn, scb, sch, scn, sob, soh, son, sdob, sdoh, sdon, sdkb, sdkh, sdkn;
   float sm_scale, sm_scale_log2;
@@ -209,7 +210,7 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
       }
     }
   };
-  const float osc = a.grad_scale ? *a.grad_scale : 1.0f;
+  float osc = a.grad_scale ? *a.grad_scale : 1.0f;
   // the tile's rows leave through 2 KB of LDS as whole 128-byte lines: 64 columns of 16 rows at a time
   auto write_tile = [&](int t, unsigned char *stage) __attribute__((always_inline)) {
     unsigned short *out = static_cast<unsigned short *>(a.dkv) + b * a.sdkb + h * a.sdkh + (int64_t)32 * t * a.sdkn;
@@ -244,12 +245,45 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
   if (KEEP) {
     int t = part * a.tiles_per_wg + wave;
     const int t_end = min(ntiles, (part + 1) * a.tiles_per_wg);
+    const int key0 = part * a.tiles_per_wg * 32;
+    const KeyScaleMax scales(a.scale, a.scale_dtype, tk0 + key0, a.direct ? min(a.tiles_per_wg * 32, a.Nk - key0) : 1, tid);
     if (t < t_end) load_tile(t);
     for (int qb = 0; qb < nqb; ++qb) copy_rows(qb, qb);
     u32x4 of[OC];
     load_o(0, of);
     dma_wait();
     __syncthreads();
+    if (a.direct) {   // cast and scaled in place: a thread has 16 bytes of every slab
+      const bool live = tid < 64 * nqb;
+      unsigned char *mine = smem + tid * 16;
+      float *red = reinterpret_cast<float *>(smem + GM::OFF_STAGE);
+      u32x4 w[CPR];
+      float m = 0.f;
+#pragma unroll
+      for (int s = 0; s < CPR; ++s) {
+        w[s] = live ? *reinterpret_cast<const u32x4 *>(mine + GM::MAT + s * SLAB) : u32x4{0u, 0u, 0u, 0u};
+        m = a.do_bf16 ? max_abs8<__bf16>(w[s], m) : max_abs8<_Float16>(w[s], m);
+      }
+      const int k = block_dout_exponent(m, scales.get(), red);
+      const float f = __builtin_ldexpf(1.0f, k);
+      osc = __builtin_ldexpf(1.0f, -k);
+      if (live) {
+#pragma unroll
+        for (int s = 0; s < CPR; ++s) *reinterpret_cast<u32x4 *>(mine + GM::MAT + s * SLAB) = scaled_dout(w[s], a.do_bf16, f);
+        if (a.q_bf16) {
+#pragma unroll
+          for (int s = 0; s < CPR; ++s) {
+            u32x4 *q = reinterpret_cast<u32x4 *>(mine + s * SLAB);
+            *q = half_of_bf16(*q);
+          }
+        }
+      }
+      if (a.q_bf16) {
+#pragma unroll
+        for (int i = 0; i < OC; ++i) of[i] = half_of_bf16(of[i]);
+      }
+      __syncthreads();
+    }
     stats(0, 0, of);
     __syncthreads();
     for (; t < t_end; t += 4) {
@@ -297,6 +331,7 @@ template <int D> static int launch_d(const SkvAttnArgs &x, hipStream_t st) {
   a.dout = static_cast<const _Float16 *>(x.dout);
   a.codes = x.codes; a.scale = x.scale; a.zp = x.zp; a.lse = x.lse; a.dkv = x.dkv;
   a.grad_scale = x.grad_scale; a.grad_bf16 = x.grad_dtype == QFA_BF16; a.scale_dtype = x.scale_dtype;
+  a.direct = x.direct; a.q_bf16 = x.io_dtype == QFA_BF16; a.do_bf16 = x.dout_dtype == QFA_BF16;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk;
   a.sqb = x.sqb; a.sqh = x.sqh; a.sqn = x.sqn; a.scb = x.scb; a.sch = x.sch; a.scn = x.scn;
   a.sob = x.sob; a.soh = x.soh; a.son = x.son; a.sdob = x.sdob; a.sdoh = x.sdoh; a.sdon = x.sdon;

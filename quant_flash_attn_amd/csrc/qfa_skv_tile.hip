@@ -32,6 +32,7 @@ struct SkvTileArgs {
   const void *q; const int8_t *codes; const void *scale; const int8_t *zp;
   void *o; float *lse;
   const _Float16 *dout; void *dq; const float *grad_scale;   // dQ only
+  int direct, do_bf16;   // dQ: q, o (io_bf16) and dO as the caller has them, dO scaled here (grad_scale is not used)
   int64_t H;
   int Nq, Nk, BH;
   int io_bf16, scale_dtype, grad_bf16;
@@ -426,12 +427,28 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
 
   const int qi = 32 * qb + lr, qi_c = min(qi, a.Nq - 1);
   u32x4 qf[KD], dof[KD];
-  skv_load_row<D>(a.q, b * a.sqb + h * a.sqh + (int64_t)qi_c * a.sqn, 0, g, qf);
+  const KeyScaleMax scales(a.scale, a.scale_dtype, tk0 + (int64_t)t0 * TK, a.direct ? min(nt * TK, a.Nk - t0 * TK) : 1, tid);
+  skv_load_row<D>(a.q, b * a.sqb + h * a.sqh + (int64_t)qi_c * a.sqn, a.io_bf16, g, qf);
+  float osc = a.grad_scale ? *a.grad_scale : 1.0f;
   skv_load_row<D>(a.dout, b * a.sdob + h * a.sdoh + (int64_t)qi_c * a.sdon, 0, g, dof);
   float delta = 0.f;
   {
     u32x4 of[KD];
-    skv_load_row<D>(a.o, b * a.sob + h * a.soh + (int64_t)qi_c * a.son, 0, g, of);
+    skv_load_row<D>(a.o, b * a.sob + h * a.soh + (int64_t)qi_c * a.son, a.io_bf16, g, of);
+    // A power of two of the workgroup's own queries and keys.  The reduction in front of the first tile costs this kernel more
+    // than it saves in bytes (99 x 53 heads, 97 x 689, fp16: 439 -> 497 us, dKV 662 -> 684), but two launches of 91 us less, of
+    // 320 in bf16: the call 1447 -> 1431 and 1655 -> 1424 us; 14 heads, 100 x 1872 (bound by launches): 64 -> 54.
+    if (a.direct) {
+      __shared__ float red[8];
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < KD; ++i) m = a.do_bf16 ? max_abs8<__bf16>(dof[i], m) : max_abs8<_Float16>(dof[i], m);
+      const int k = block_dout_exponent(m, scales.get(), red);
+      const float f = __builtin_ldexpf(1.0f, k);
+      osc = __builtin_ldexpf(1.0f, -k);
+#pragma unroll
+      for (int i = 0; i < KD; ++i) dof[i] = scaled_dout(dof[i], a.do_bf16, f);
+    }
 #pragma unroll
     for (int m = 0; m < KD; ++m)
 #pragma unroll
@@ -523,6 +540,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
       for (int v = 0; v < 16; ++v) acc[db][v] += src[(16 * db + v) * 64];
   }
   if (a.splits > 1) {   // partial result for the sum
+    const float part = a.direct ? osc : 1.0f;   // (the sum applies grad_scale)
     if (qi < a.Nq) {
       const int64_t at = (tq0 + qi) * a.splits + split;
 #pragma unroll
@@ -530,11 +548,10 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
 #pragma unroll
         for (int aa = 0; aa < 4; ++aa)
           *reinterpret_cast<f32x4 *>(a.po + at * D + 32 * db + 8 * aa + 4 * g) =
-              f32x4{acc[db][4 * aa], acc[db][4 * aa + 1], acc[db][4 * aa + 2], acc[db][4 * aa + 3]};
+              f32x4{acc[db][4 * aa] * part, acc[db][4 * aa + 1] * part, acc[db][4 * aa + 2] * part, acc[db][4 * aa + 3] * part};
     }
     return;
   }
-  const float osc = a.grad_scale ? *a.grad_scale : 1.0f;
   unsigned char *stage = smem + (KW > 1 ? slot * GM::MERGE : wave * 64 * D);
   unsigned short *dq = static_cast<unsigned short *>(a.dq) + b * a.sdqb + h * a.sdqh;
   if (a.grad_bf16) store_tile_rows<__bf16, D>(acc, osc, stage, reinterpret_cast<__bf16 *>(dq), a.sdqn, 32 * qb, a.Nq, lane);
@@ -546,6 +563,7 @@ static SkvTileArgs skv_tile_args(const SkvAttnArgs &x, int qw) {
   SkvTileArgs a;
   a.q = x.q; a.codes = x.codes; a.scale = x.scale; a.zp = x.zp; a.o = x.o; a.lse = x.lse;
   a.dout = static_cast<const _Float16 *>(x.dout); a.dq = x.dq; a.grad_scale = x.grad_scale;
+  a.direct = x.direct; a.do_bf16 = x.dout_dtype == QFA_BF16;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk; a.BH = (int)(x.B * x.H);
   a.io_bf16 = x.io_dtype == QFA_BF16; a.scale_dtype = x.scale_dtype; a.grad_bf16 = x.grad_dtype == QFA_BF16;
   a.sqb = x.sqb; a.sqh = x.sqh; a.sqn = x.sqn; a.scb = x.scb; a.sch = x.sch; a.scn = x.scn;

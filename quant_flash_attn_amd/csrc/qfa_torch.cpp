@@ -790,7 +790,7 @@ struct SharedFn : torch::autograd::Function<SharedFn> {
     // so dO is handed over scaled by a power of two chosen on the device (no synchronisation) from
     // its largest magnitude and from the largest key scale, and the kernels scale dQ and dKV back
     // while they round them.  q and o convert exactly from bf16 (more mantissa, values of order one).
-    // Where one pass takes all queries it does that itself.
+    // Kernels whose workgroups hold all rows that they need do that themselves.
     const double sm = ctx->saved_data["sm"].toDouble();
     Tensor dq, dkv;
     if (is_io(o.scalar_type()) && o.scalar_type() == q.scalar_type() && api.qfa_attn_bwd_shared_kv_is_direct(q.size(2), (int)q.size(3))) {

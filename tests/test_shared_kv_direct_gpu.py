@@ -1,4 +1,4 @@
-"""Up to 32 queries, shared-KV backward: q, o and dO as the caller has them, cast and scaled inside, against the launches that cast
+"""Shared-KV backward of query blocks that a workgroup holds: q, o and dO as the caller has them, cast and scaled inside, against the launches that cast
 and scale first, and with gradients of very different size in different heads."""
 import pytest
 import torch
@@ -45,7 +45,10 @@ def _scaled_first(q, o, do, codes, scale, zp, lse, sm):
 
 @pytest.mark.parametrize("dtype,sdtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float16), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("B,H,Nq,Nk,D", [(1, 1, 1, 33, 64), (1, 3, 16, 700, 128), (2, 3, 17, 257, 64), (1, 2, 32, 4000, 128),
-                                         (1, 2, 5, 100, 256), (1, 4, 16, 3001, 256), (300, 2, 3, 31, 64)])
+                                         (1, 2, 5, 100, 256), (1, 4, 16, 3001, 256), (300, 2, 3, 31, 64),
+                                         # two kernels: 16 or 32 queries per wave in dQ, keys split or not
+                                         (1, 4, 33, 700, 128), (20, 53, 97, 300, 128), (1, 2, 128, 4097, 64), (3, 64, 65, 1000, 64),
+                                         (1, 1, 128, 31, 128)])
 def test_direct_against_scaled_first(qfa, B, H, Nq, Nk, D, dtype, sdtype):
     t = _tensors(B, H, Nq, Nk, D, dtype, sdtype)
     t[2].mul_(1e-4)
@@ -56,22 +59,29 @@ def test_direct_against_scaled_first(qfa, B, H, Nq, Nk, D, dtype, sdtype):
             # another power of two per workgroup: the same products but for what binary16 loses below 2^-14 of the largest (2^-10
             # of such a value), and with a split another order of fp32 sums, rounded to 8 bits once
             assert (a.double() - b.double()).norm() <= 2.0 ** -8 * b.double().norm()
-    assert _lib.lib().qfa_attn_bwd_shared_kv_is_direct(33, 64) == 0 and _lib.lib().qfa_attn_bwd_shared_kv_is_direct(17, 256) == 0
+    assert _lib.lib().qfa_attn_bwd_shared_kv_is_direct(129, 64) == 0 and _lib.lib().qfa_attn_bwd_shared_kv_is_direct(17, 256) == 0
 
 
 def test_heads_do_not_share_the_scaling(qfa):
     """Gradients 2^40 apart in two heads: each head's are as good as alone (one scaling for both loses the small ones)."""
-    q, o, do, codes, scale, zp, lse = _tensors(1, 2, 16, 500, 128, torch.bfloat16, torch.float16)
+    for Nq in (16, 100):
+        _scaling_of_heads(Nq)
+
+
+def _scaling_of_heads(Nq):
+    q, o, do, codes, scale, zp, lse = _tensors(1, 2, Nq, 500, 128, torch.bfloat16, torch.float16)
     do[:, 0] *= 2.0 ** -40
     dq, dkv, _ = _direct(q, o, do, codes, scale, zp, lse, 0.09, False)
     for h in (0, 1):
         one = [x[:, h:h + 1].contiguous() for x in (q, o, do, codes, scale, zp, lse)]
         for a, b in zip((dq, dkv), _scaled_first(*one, 0.09)):
-            assert b.abs().max() > 0 and torch.equal(a[:, h:h + 1], b)
+            # (up to 32 queries the same kernel and the same power of two)
+            assert b.abs().max() > 0 and (a[:, h:h + 1].double() - b.double()).norm() <= (0 if Nq <= 32 else 2.0 ** -8) * b.double().norm()
 
 
-def test_infinite_and_zero_gradients(qfa):
-    q, o, do, codes, scale, zp, lse = _tensors(1, 3, 7, 100, 64, torch.float16, torch.float16)
+@pytest.mark.parametrize("Nq", [7, 40, 100])
+def test_infinite_and_zero_gradients(qfa, Nq):
+    q, o, do, codes, scale, zp, lse = _tensors(1, 3, Nq, 100, 64, torch.float16, torch.float16)
     do[:, 0] = 0
     do[0, 1, 3, 5] = float("inf")
     dq, dkv, _ = _direct(q, o, do, codes, scale, zp, lse, 0.09, False)
