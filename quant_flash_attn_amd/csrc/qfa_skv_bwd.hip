@@ -160,16 +160,12 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     if (a.direct) {
       // What otherwise takes two to four launches in front of this one: bf16 q and o cast, dO scaled by a power of two that is
       // this workgroup's own (its queries and its keys decide it)
-      float m = 0.f;
+      const int k = block_dout_exponent(max_abs_dout(dv, a.do_bf16), scales.get(), stat);
+      osc = exp2_neg(k);
+      scale_dout(dv, a.do_bf16, k);
+      if (a.q_bf16) {
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) m = a.do_bf16 ? max_abs8<__bf16>(dv[i], m) : max_abs8<_Float16>(dv[i], m);
-      const int k = block_dout_exponent(m, scales.get(), stat);
-      const float f = __builtin_ldexpf(1.0f, k);
-      osc = __builtin_ldexpf(1.0f, -k);
-#pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        dv[i] = scaled_dout(dv[i], a.do_bf16, f);
-        if (a.q_bf16) qv[i] = half_of_bf16(qv[i]), ov[i] = half_of_bf16(ov[i]);
+        for (int i = 0; i < CPT; ++i) qv[i] = half_of_bf16(qv[i]), ov[i] = half_of_bf16(ov[i]);
       }
       __syncthreads();   // the maxima are read: `stat` is written below
     }

@@ -176,20 +176,54 @@ __device__ __forceinline__ int dout_exponent(float m, float ms) {
   ms = fmaxf(ms, 1e-30f);
   return max(-100, min(100, min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m))));
 }
-// eight bf16 values as binary16; eight of dO (bf16 or binary16) times f, as binary16
+// eight bf16 values as binary16
 __device__ __forceinline__ u32x4 half_of_bf16(u32x4 w) {
   u32x4 r;
 #pragma unroll
   for (int e = 0; e < 4; ++e) r[e] = pack2<_Float16>(lo_to_f32<__bf16>(w[e]), hi_to_f32<__bf16>(w[e]));
   return r;
 }
-__device__ __forceinline__ u32x4 scaled_dout(u32x4 w, int bf16, float f) {
-  u32x4 r;
+// largest magnitude of N x 8 values of dO; the same times 2^k, as binary16.  (One branch on the type around all of them: selected
+// value by value, dQ of 99 x 53 heads, 97 x 689 takes 5 us of 490 more.)
+template <int N> __device__ __forceinline__ float max_abs_dout(const u32x4 (&w)[N], int bf16) {
+  float m = 0.f;
+  if (bf16) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    r[e] = bf16 ? pack2<_Float16>(lo_to_f32<__bf16>(w[e]) * f, hi_to_f32<__bf16>(w[e]) * f)
-                : pack2<_Float16>(lo_to_f32<_Float16>(w[e]) * f, hi_to_f32<_Float16>(w[e]) * f);
-  return r;
+    for (int i = 0; i < N; ++i) m = max_abs8<__bf16>(w[i], m);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) m = max_abs8<_Float16>(w[i], m);
+  }
+  return m;
+}
+template <int N> __device__ __forceinline__ void scale_dout(u32x4 (&w)[N], int bf16, int k) {
+  const float f = __builtin_ldexpf(1.0f, k);
+  if (bf16) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned x = w[i][e];
+        w[i][e] = pack2<_Float16>(lo_to_f32<__bf16>(x) * f, hi_to_f32<__bf16>(x) * f);
+      }
+  } else if (k >= -14 && k <= 15) {   // 2^k is a normal binary16 number: one rounding too
+    const f16x2 f2 = {(_Float16)f, (_Float16)f};
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned x = w[i][e];
+        w[i][e] = __builtin_bit_cast(unsigned, __builtin_bit_cast(f16x2, x) * f2);
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned x = w[i][e];
+        w[i][e] = pack2<_Float16>(lo_to_f32<_Float16>(x) * f, hi_to_f32<_Float16>(x) * f);
+      }
+  }
 }
 // The largest of n key scales (fp32 or fp16) from k0 on, as one of 256 threads finds it: the first thousand are requested here
 // and looked at with the others later, so that the rows that the caller loads in between hide them.
@@ -219,6 +253,15 @@ struct KeyScaleMax {
     return ms;
   }
 };
+// Every load so far has arrived.  For the end of a prologue whose branches leave loads that one side never reads (KeyScaleMax): the
+// compiler then guards their registers wherever the main loop first writes them, and that wait is for the next tile's loads as well
+// (dQ of 99 x 53 heads, 97 x 689: 485 us with such waits in the loop, 452 with this one in front of it).
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }   // vmcnt(0), the other counters at their maximum
+// 2^-k, in a scalar register
+__device__ __forceinline__ float exp2_neg(int k) {
+  const int bits = (127 - k) << 23;   // |k| <= 100
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(bits));
+}
 // dout_exponent of 256 threads' m and ms; red: 8 floats of LDS that nobody uses
 __device__ __forceinline__ int block_dout_exponent(float m, float ms, float *red) {
 #pragma unroll

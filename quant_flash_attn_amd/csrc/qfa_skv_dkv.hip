@@ -72,14 +72,15 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
     }
   };
   // delta and LSE of RPT-row groups: 256 / TPR rows from row r0 of the sequence on, in rows a0.. of the row area; O comes
-  // from memory (`of`, loaded before), dO from the row area
+  // and the LSE from memory (`of`, `lse`, loaded before), dO from the row area
   constexpr int TPR = KEEP ? 2 : 4, OC = D / 8 / TPR;   // threads per row, 8-element chunks per thread
-  auto load_o = [&](int r0, u32x4 (&of)[OC]) __attribute__((always_inline)) {
+  auto load_o = [&](int r0, u32x4 (&of)[OC], float &lse) __attribute__((always_inline)) {
     const int row = min(r0 + tid / TPR, a.Nq - 1);
+    lse = a.lse[tq0 + row];
 #pragma unroll
     for (int k = 0; k < OC; ++k) of[k] = *reinterpret_cast<const u32x4 *>(o_bh + (int64_t)row * a.son + 8 * (tid % TPR + TPR * k));
   };
-  auto stats = [&](int r0, int a0, const u32x4 (&of)[OC]) __attribute__((always_inline)) {
+  auto stats = [&](int r0, int a0, const u32x4 (&of)[OC], float lse) __attribute__((always_inline)) {
     const int rr = tid / TPR, ra = a0 + rr;
     const bool live = r0 + rr < a.Nq;
     float sum = 0.f;
@@ -96,7 +97,7 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
 #pragma unroll
     for (int m = 1; m < TPR; m *= 2) sum += __shfl_xor(sum, m, 64);
     if (tid % TPR == 0) {
-      stat[ra] = live ? -a.lse[tq0 + r0 + rr] * kLog2e : -INFINITY;   // padding rows: p = 0
+      stat[ra] = live ? -lse * kLog2e : -INFINITY;   // padding rows: p = 0
       stat[GM::ROWS + ra] = live ? -a.sm_scale * sum : 0.f;
     }
   };
@@ -250,7 +251,8 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
     if (t < t_end) load_tile(t);
     for (int qb = 0; qb < nqb; ++qb) copy_rows(qb, qb);
     u32x4 of[OC];
-    load_o(0, of);
+    float lse;
+    load_o(0, of, lse);
     dma_wait();
     __syncthreads();
     if (a.direct) {   // cast and scaled in place: a thread has 16 bytes of every slab
@@ -258,18 +260,14 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
       unsigned char *mine = smem + tid * 16;
       float *red = reinterpret_cast<float *>(smem + GM::OFF_STAGE);
       u32x4 w[CPR];
-      float m = 0.f;
 #pragma unroll
-      for (int s = 0; s < CPR; ++s) {
-        w[s] = live ? *reinterpret_cast<const u32x4 *>(mine + GM::MAT + s * SLAB) : u32x4{0u, 0u, 0u, 0u};
-        m = a.do_bf16 ? max_abs8<__bf16>(w[s], m) : max_abs8<_Float16>(w[s], m);
-      }
-      const int k = block_dout_exponent(m, scales.get(), red);
-      const float f = __builtin_ldexpf(1.0f, k);
-      osc = __builtin_ldexpf(1.0f, -k);
+      for (int s = 0; s < CPR; ++s) w[s] = live ? *reinterpret_cast<const u32x4 *>(mine + GM::MAT + s * SLAB) : u32x4{0u, 0u, 0u, 0u};
+      const int k = block_dout_exponent(max_abs_dout(w, a.do_bf16), scales.get(), red);
+      scale_dout(w, a.do_bf16, k);
+      osc = exp2_neg(k);
       if (live) {
 #pragma unroll
-        for (int s = 0; s < CPR; ++s) *reinterpret_cast<u32x4 *>(mine + GM::MAT + s * SLAB) = scaled_dout(w[s], a.do_bf16, f);
+        for (int s = 0; s < CPR; ++s) *reinterpret_cast<u32x4 *>(mine + GM::MAT + s * SLAB) = w[s];
         if (a.q_bf16) {
 #pragma unroll
           for (int s = 0; s < CPR; ++s) {
@@ -284,7 +282,7 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
       }
       __syncthreads();
     }
-    stats(0, 0, of);
+    stats(0, 0, of, lse);
     __syncthreads();
     for (; t < t_end; t += 4) {
       expand_tile();
@@ -302,11 +300,12 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
   const bool t_ok = t < ntiles;   // (a wave without a tile still takes part in copies and barriers)
   const int ngroups = (nqb + HB - 1) / HB;
   u32x4 of[OC];
+  float lse;
   auto fetch = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < HB; ++i)
       if (HB * grp + i < nqb) copy_rows(HB * grp + i, HB * (grp & 1) + i);
-    load_o(32 * HB * grp, of);
+    load_o(32 * HB * grp, of, lse);
   };
   if (t_ok) load_tile(t);
   fetch(0);
@@ -315,7 +314,7 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
   for (int grp = 0; grp < ngroups; ++grp) {
     dma_wait();
     __syncthreads();   // the group's rows have landed
-    stats(32 * HB * grp, 32 * HB * (grp & 1), of);
+    stats(32 * HB * grp, 32 * HB * (grp & 1), of, lse);
     __syncthreads();   // its statistics are there, and everybody is done with the group before it
     if (grp + 1 < ngroups) fetch(grp + 1);
     if (t_ok)

@@ -429,25 +429,20 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   u32x4 qf[KD], dof[KD];
   const KeyScaleMax scales(a.scale, a.scale_dtype, tk0 + (int64_t)t0 * TK, a.direct ? min(nt * TK, a.Nk - t0 * TK) : 1, tid);
   skv_load_row<D>(a.q, b * a.sqb + h * a.sqh + (int64_t)qi_c * a.sqn, a.io_bf16, g, qf);
-  float osc = a.grad_scale ? *a.grad_scale : 1.0f;
+  int dout_k = 0;   // direct: dO is scaled by 2^dout_k
   skv_load_row<D>(a.dout, b * a.sdob + h * a.sdoh + (int64_t)qi_c * a.sdon, 0, g, dof);
+  const float lse = a.lse[tq0 + qi_c];
   float delta = 0.f;
   {
     u32x4 of[KD];
     skv_load_row<D>(a.o, b * a.sob + h * a.soh + (int64_t)qi_c * a.son, a.io_bf16, g, of);
-    // A power of two of the workgroup's own queries and keys.  The reduction in front of the first tile costs this kernel more
-    // than it saves in bytes (99 x 53 heads, 97 x 689, fp16: 439 -> 497 us, dKV 662 -> 684), but two launches of 91 us less, of
-    // 320 in bf16: the call 1447 -> 1431 and 1655 -> 1424 us; 14 heads, 100 x 1872 (bound by launches): 64 -> 54.
+    // A power of two of the workgroup's own queries and keys.  The reduction in front of the first tile costs this kernel a
+    // little (99 x 53 heads, 97 x 689, fp16: 442 -> 456 us, dKV 670 -> 690), but it takes the place of two launches, more in bf16:
+    // the call 1480 -> 1417 and 1519 -> 1426 us; 14 heads, 100 x 1872 (bound by launches): 84 -> 54 to 76.
     if (a.direct) {
       __shared__ float red[8];
-      float m = 0.f;
-#pragma unroll
-      for (int i = 0; i < KD; ++i) m = a.do_bf16 ? max_abs8<__bf16>(dof[i], m) : max_abs8<_Float16>(dof[i], m);
-      const int k = block_dout_exponent(m, scales.get(), red);
-      const float f = __builtin_ldexpf(1.0f, k);
-      osc = __builtin_ldexpf(1.0f, -k);
-#pragma unroll
-      for (int i = 0; i < KD; ++i) dof[i] = scaled_dout(dof[i], a.do_bf16, f);
+      dout_k = block_dout_exponent(max_abs_dout(dof, a.do_bf16), scales.get(), red);
+      scale_dout(dof, a.do_bf16, dout_k);
     }
 #pragma unroll
     for (int m = 0; m < KD; ++m)
@@ -459,7 +454,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
     delta += swap32_f(delta);
   }
   const float a_s = a.sm_scale_log2, sm = a.sm_scale;
-  const float nlse2 = qi < a.Nq ? -a.lse[tq0 + qi] * kLog2e : -INFINITY;   // padding rows: p = 0
+  const float nlse2 = qi < a.Nq ? -lse * kLog2e : -INFINITY;   // padding rows: p = 0
   const SkvTileReads<GM::SLAB> rd(lane);
 
   f32x16 acc[DB];
@@ -502,6 +497,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   };
 
   st.commit(smem, a.scale_dtype, 1.0f);
+  wait_loads();
   __syncthreads();
   for (int t = 0; t < nt; ++t) {
     unsigned char *buf = smem + (t & 1) * GM::BUF;
@@ -540,7 +536,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
       for (int v = 0; v < 16; ++v) acc[db][v] += src[(16 * db + v) * 64];
   }
   if (a.splits > 1) {   // partial result for the sum
-    const float part = a.direct ? osc : 1.0f;   // (the sum applies grad_scale)
+    const float part = exp2_neg(dout_k);   // (the sum applies grad_scale)
     if (qi < a.Nq) {
       const int64_t at = (tq0 + qi) * a.splits + split;
 #pragma unroll
@@ -552,6 +548,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
     }
     return;
   }
+  const float osc = a.grad_scale ? *a.grad_scale : exp2_neg(dout_k);
   unsigned char *stage = smem + (KW > 1 ? slot * GM::MERGE : wave * 64 * D);
   unsigned short *dq = static_cast<unsigned short *>(a.dq) + b * a.sdqb + h * a.sdqh;
   if (a.grad_bf16) store_tile_rows<__bf16, D>(acc, osc, stage, reinterpret_cast<__bf16 *>(dq), a.sdqn, 32 * qb, a.Nq, lane);
