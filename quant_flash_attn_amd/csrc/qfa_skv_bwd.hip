@@ -159,14 +159,21 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     }
     if (a.direct) {
       // What otherwise takes two to four launches in front of this one: bf16 q and o cast, dO scaled by a power of two that is
-      // this workgroup's own (its queries and its keys decide it)
-      const int k = block_dout_exponent(max_abs_dout(dv, a.do_bf16), scales.get(), stat);
-      osc = exp2_neg(k);
-      scale_dout(dv, a.do_bf16, k);
+      // this workgroup's own (its queries, their delta and its keys decide it)
       if (a.q_bf16) {
 #pragma unroll
         for (int i = 0; i < CPT; ++i) qv[i] = half_of_bf16(qv[i]), ov[i] = half_of_bf16(ov[i]);
       }
+      float md = 0.f;
+      if (a.splits > 1) {   // O comes from all keys of the head, the scales from a part of them
+        md = dot_dout(ov, dv, a.do_bf16);
+#pragma unroll
+        for (int m = 1; m < 8; m *= 2) md += __shfl_xor(md, m, 64);
+        md = finite_abs(a.sm_scale * md);
+      }
+      const int k = block_dout_exponent(max_abs_dout(dv, a.do_bf16), scales.get(), md, stat);
+      osc = exp2_neg(k);
+      scale_dout(dv, a.do_bf16, k);
       __syncthreads();   // the maxima are read: `stat` is written below
     }
 #pragma unroll

@@ -46,7 +46,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
   static_assert(3 * MG * 4 <= 4 * WAVE, "the merge area overlays the rings");
   // (One array: with the maxima of a direct call in a second one, the compiler waits for all LDS loads in
   // front of a tile's scales: 48 heads, 33 x 12000, 82 us against 75.)
-  __shared__ __attribute__((aligned(16))) unsigned char smem[4 * WAVE + (D <= 128 ? 32 : 0)];
+  __shared__ __attribute__((aligned(16))) unsigned char smem[4 * WAVE + (D <= 128 ? 48 : 0)];
 
   const XcdBlock id(a.BH, a.qblocks);
   if (!id.live) return;
@@ -95,8 +95,8 @@ template <typename S, int D> __global__ __launch_bounds__(256, 2) void skv_dq_ke
     dof[m] = *reinterpret_cast<const u32x4 *>(drow + d0);
     of[m] = *reinterpret_cast<const u32x4 *>(orow + d0);
   }
-  if (D <= 128 && a.direct) {   // a power of two of the workgroup's own queries and of its head's keys
-    const int k = block_dout_exponent(max_abs_dout(dof, a.do_bf16), scales.get(), reinterpret_cast<float *>(smem + 4 * WAVE));
+  if (D <= 128 && a.direct) {   // a power of two of the workgroup's own queries and of all its head's keys, which bound delta
+    const int k = block_dout_exponent(max_abs_dout(dof, a.do_bf16), scales.get(), 0.f, reinterpret_cast<float *>(smem + 4 * WAVE));
     osc = exp2_neg(k);
     scale_dout(dof, a.do_bf16, k);
     if (a.q_bf16) {

@@ -170,12 +170,35 @@ __device__ __forceinline__ int floor_log2_quot(int ce, float y) {
   return ce - e - ((b & 0x7fffffu) != 0 ? 1 : 0);
 }
 
-// k of the largest magnitudes of dO and of the key scales
-__device__ __forceinline__ int dout_exponent(float m, float ms) {
+// k of the largest magnitudes of dO (m), of the key scales (ms) and of sm_scale * delta (md).  What the kernels round to binary16
+// is dS = p * (sm_scale * dP - sm_scale * delta) and that times its key's scale.  m * 2^k * ms <= 8 bounds the first term by
+// 8 * 255 * head_dim * sm_scale (32640 at most for 1 / sqrt(head_dim)).  It bounds the second term too where ms is the largest scale
+// of all keys that O is made of; a workgroup that looks at the scales of a part of them passes md, which is kept below 2^15.
+__device__ __forceinline__ int dout_exponent(float m, float ms, float md = 0.f) {
   m = fmaxf(m, 1e-30f);     // inf stays inf: k = -100 below
   ms = fmaxf(ms, 1e-30f);
-  return max(-100, min(100, min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m))));
+  md = fmaxf(md * fmaxf(ms, 1.0f), 1e-30f);
+  return max(-100, min(100, min(min(floor_log2_quot(3, m * ms), floor_log2_quot(14, m)), floor_log2_quot(15, md))));
 }
+// sum of O * dO over N x 8 values, O in binary16
+template <int N> __device__ __forceinline__ float dot_dout(const u32x4 (&o)[N], const u32x4 (&w)[N], int bf16) {
+  float sum = 0.f;
+  auto add = [&](auto type) __attribute__((always_inline)) {
+    typedef decltype(type) T;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned ow = o[i][e], dw = w[i][e];
+        sum += lo_to_f32<_Float16>(ow) * lo_to_f32<T>(dw) + hi_to_f32<_Float16>(ow) * hi_to_f32<T>(dw);
+      }
+  };
+  if (bf16) add(__bf16{});
+  else add(_Float16{});
+  return sum;
+}
+// |sm_scale * delta| for dout_exponent: a row that is not finite has no say in how the others are scaled
+__device__ __forceinline__ float finite_abs(float x) { return fabsf(x) <= 3.4e38f ? fabsf(x) : 0.f; }
 // eight bf16 values as binary16
 __device__ __forceinline__ u32x4 half_of_bf16(u32x4 w) {
   u32x4 r;
@@ -262,21 +285,24 @@ __device__ __forceinline__ float exp2_neg(int k) {
   const int bits = (127 - k) << 23;   // |k| <= 100
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(bits));
 }
-// dout_exponent of 256 threads' m and ms; red: 8 floats of LDS that nobody uses
-__device__ __forceinline__ int block_dout_exponent(float m, float ms, float *red) {
+// dout_exponent of 256 threads' m, ms and md; red: 12 floats of LDS that nobody uses
+__device__ __forceinline__ int block_dout_exponent(float m, float ms, float md, float *red) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     m = fmaxf(m, __shfl_xor(m, off, 64));
     ms = fmaxf(ms, __shfl_xor(ms, off, 64));
+    md = fmaxf(md, __shfl_xor(md, off, 64));
   }
   if (threadIdx.x % 64 == 0) {
     red[threadIdx.x / 64] = m;
     red[4 + threadIdx.x / 64] = ms;
+    red[8 + threadIdx.x / 64] = md;
   }
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   ms = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
-  return __builtin_amdgcn_readfirstlane(dout_exponent(m, ms));
+  md = fmaxf(fmaxf(red[8], red[9]), fmaxf(red[10], red[11]));
+  return __builtin_amdgcn_readfirstlane(dout_exponent(m, ms, md));
 }
 
 }  // namespace qfa

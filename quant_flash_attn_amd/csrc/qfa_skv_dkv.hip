@@ -80,14 +80,17 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
 #pragma unroll
     for (int k = 0; k < OC; ++k) of[k] = *reinterpret_cast<const u32x4 *>(o_bh + (int64_t)row * a.son + 8 * (tid % TPR + TPR * k));
   };
+  auto dout_of = [&](int ra, int k) __attribute__((always_inline)) -> u32x4 {   // chunk k of a thread's row
+    const int c = tid % TPR + TPR * k;
+    return *reinterpret_cast<const u32x4 *>(smem + GM::MAT + c / 2 * SLAB + ra * 32 + (((c % 2) ^ (ra >> 3 & 1)) << 4));
+  };
   auto stats = [&](int r0, int a0, const u32x4 (&of)[OC], float lse) __attribute__((always_inline)) {
     const int rr = tid / TPR, ra = a0 + rr;
     const bool live = r0 + rr < a.Nq;
     float sum = 0.f;
 #pragma unroll
     for (int k = 0; k < OC; ++k) {
-      const int c = tid % TPR + TPR * k;
-      const u32x4 dv = *reinterpret_cast<const u32x4 *>(smem + GM::MAT + c / 2 * SLAB + ra * 32 + (((c % 2) ^ (ra >> 3 & 1)) << 4));
+      const u32x4 dv = dout_of(ra, k);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const unsigned dw = dv[e], ow = of[k][e];
@@ -262,7 +265,21 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
       u32x4 w[CPR];
 #pragma unroll
       for (int s = 0; s < CPR; ++s) w[s] = live ? *reinterpret_cast<const u32x4 *>(mine + GM::MAT + s * SLAB) : u32x4{0u, 0u, 0u, 0u};
-      const int k = block_dout_exponent(max_abs_dout(w, a.do_bf16), scales.get(), red);
+      if (a.q_bf16) {
+#pragma unroll
+        for (int i = 0; i < OC; ++i) of[i] = half_of_bf16(of[i]);
+      }
+      float md = 0.f;
+      if (a.wgs_per_bh > 1) {   // O comes from all keys of the head, the scales from a part of them
+        u32x4 dr[OC];
+#pragma unroll
+        for (int i = 0; i < OC; ++i) dr[i] = dout_of(tid / TPR, i);
+        md = dot_dout(of, dr, a.do_bf16);
+#pragma unroll
+        for (int m = 1; m < TPR; m *= 2) md += __shfl_xor(md, m, 64);
+        md = tid / TPR < a.Nq ? finite_abs(a.sm_scale * md) : 0.f;
+      }
+      const int k = block_dout_exponent(max_abs_dout(w, a.do_bf16), scales.get(), md, red);
       scale_dout(w, a.do_bf16, k);
       osc = exp2_neg(k);
       if (live) {
@@ -275,10 +292,6 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
             *q = half_of_bf16(*q);
           }
         }
-      }
-      if (a.q_bf16) {
-#pragma unroll
-        for (int i = 0; i < OC; ++i) of[i] = half_of_bf16(of[i]);
       }
       __syncthreads();
     }

@@ -436,12 +436,17 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   {
     u32x4 of[KD];
     skv_load_row<D>(a.o, b * a.sob + h * a.soh + (int64_t)qi_c * a.son, a.io_bf16, g, of);
-    // A power of two of the workgroup's own queries and keys.  The reduction in front of the first tile costs this kernel a
+    // A power of two of the workgroup's own queries, their delta and its keys.  The reduction in front of the first tile costs this kernel a
     // little (99 x 53 heads, 97 x 689, fp16: 442 -> 456 us, dKV 670 -> 690), but it takes the place of two launches, more in bf16:
     // the call 1480 -> 1417 and 1519 -> 1426 us; 14 heads, 100 x 1872 (bound by launches): 84 -> 54 to 76.
     if (a.direct) {
-      __shared__ float red[8];
-      dout_k = block_dout_exponent(max_abs_dout(dof, a.do_bf16), scales.get(), red);
+      __shared__ float red[12];
+      float md = 0.f;
+      if (a.splits > 1) {   // O comes from all keys of the head, the scales from a part of them
+        md = dot_dout(of, dof, a.do_bf16);
+        md = finite_abs(a.sm_scale * (md + swap32_f(md)));
+      }
+      dout_k = block_dout_exponent(max_abs_dout(dof, a.do_bf16), scales.get(), md, red);
       scale_dout(dof, a.do_bf16, dout_k);
     }
 #pragma unroll

@@ -1,8 +1,12 @@
 """Shared-KV backward of query blocks that a workgroup holds: q, o and dO as the caller has them, cast and scaled inside, against the launches that cast
 and scale first, and with gradients of very different size in different heads."""
+import math
+
 import pytest
 import torch
 
+from helpers import assert_close
+from oracle import oracle
 from quant_flash_attn_amd import _lib
 from quant_flash_attn_amd.quant_flash_attn import _normalised_dout
 
@@ -88,3 +92,26 @@ def test_infinite_and_zero_gradients(qfa, Nq):
     assert (dq[:, 0] == 0).all() and (dkv[:, 0] == 0).all()
     assert not torch.isfinite(dkv[:, 1]).all()
     assert torch.isfinite(dq[:, 2]).all() and torch.isfinite(dkv[:, 2]).all()
+
+
+@pytest.mark.parametrize("dtype,sdtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("last", [False, True])
+@pytest.mark.parametrize("Nq,Nk,D", [(16, 2048, 128), (32, 2048, 64), (16, 2048, 256),   # one pass, the keys split
+                                     (64, 256, 128), (128, 2048, 128), (100, 3000, 64)])   # dKV by chunks of keys, dQ split or not
+def test_small_keys_beside_large_ones(qfa, Nq, Nk, D, last, dtype, sdtype):
+    """delta = rowsum(O o dO) holds every key of the head, a workgroup's own key scales do not: where its keys are 2^-6 beside
+    others of 2^8 in the same head, dS = sm * p * (dP - delta) must stay within binary16 all the same."""
+    g = torch.Generator().manual_seed(Nq + D)
+    kv = torch.randn((1, 1, Nk, D), generator=g) * 2.0 ** -6
+    half = slice(Nk // 2, None) if last else slice(0, Nk // 2)
+    kv[:, :, half] = 256.0 * (1.0 + 64.0 * kv[:, :, half])
+    q = (torch.randn((1, 1, Nq, D), generator=g) / 256.0).to(dtype)
+    kv, do, sm = kv.to(dtype), torch.full((1, 1, Nq, D), 2.0 ** -6, dtype=dtype), 1.0 / math.sqrt(D)
+    qd, kvd = q.to(DEV).requires_grad_(True), kv.to(DEV).requires_grad_(True)
+    quant = qfa.asymmetric_quant_per_token(kvd.detach(), scale_dtype=sdtype)
+    o = qfa.quant_flash_attn(qd, kvd, quant, sm)
+    dq, dkv = torch.autograd.grad(o, [qd, kvd], do.to(DEV))
+    (dq_ref, dkv_ref), (nq, nkv) = oracle.legacy_bwd(q, *(t.cpu() for t in quant), do, sm, o=o.detach().cpu(), spread=True)
+    assert_close("dQ", dq.cpu(), dq_ref, scaled=True, spread=nq)
+    for part in (slice(0, Nk // 2), slice(Nk // 2, None)):
+        assert_close("dKV", dkv[:, :, part].cpu(), dkv_ref[:, :, part], scaled=True, spread=nkv[:, :, part])
