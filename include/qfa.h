@@ -225,7 +225,7 @@ int qfa_attn_fwd_shared_kv_static(const void *q, const int8_t *codes, const void
  *   grad_scale  nullable DEVICE pointer to one float that multiplies dq and dkv before they are rounded.
  *               dQ and dKV are linear in dO: a caller whose dO does not fit binary16 (bf16 training) hands
  *               over dO * 2^k and *grad_scale = 2^-k without a host synchronisation;
- *   codes, scale, scale_dtype, zp, lse as in the forward.  D in {64, 128, 256} (256: one pass up to 16 queries).
+ *   codes, scale, zp, lse as in the forward, scale_dtype QFA_F32 or QFA_F16.  D in {64, 128, 256} (256: one pass up to 16 queries).
  *   The sums of a query's and of a dO row's D elements must stay inside binary16 range.
  *   Range of dout: the kernels do not multiply by dO itself but by  ds = sm_scale * p * (dP - delta)  and by
  *   ds * scale_j,  both packed to binary16 (the reference rounds ds to fp16 as well, quant_flash_attn.py:159).
@@ -259,9 +259,10 @@ int qfa_attn_bwd_shared_kv_split(const void *q, const int8_t *codes, const void 
                                  void *stream);
 
 /*
- * The same on q and o of io_dtype (QFA_F16 or QFA_BF16) and dout of dout_dtype as a caller has them: the casts and the scaling
- * of dO by a power of two (qfa_dout_normalise) happen inside, per workgroup.  For query blocks whose rows a workgroup holds, where
- * qfa_attn_bwd_shared_kv_is_direct(Nq, D) is 1 (up to 128 queries, 16 at head_dim 256); others are QFA_EUNSUPPORTED.
+ * The same on q and o of io_dtype (QFA_F16 or QFA_BF16; the scales stay QFA_F32 or QFA_F16) and dout of dout_dtype as a caller has
+ * them: the casts and the scaling of dO by a power of two (qfa_dout_normalise) happen inside, per workgroup.  For query blocks
+ * whose rows a workgroup holds, where qfa_attn_bwd_shared_kv_is_direct(Nq, D) is 1 (up to 128 queries, 16 at head_dim 256); others
+ * are QFA_EUNSUPPORTED.
  */
 int qfa_attn_bwd_shared_kv_is_direct(int64_t Nq, int D);
 

@@ -331,6 +331,8 @@ static int skv_bwd_entry(const char *who, int direct, int dout_dtype, const void
     if (dout_dtype != QFA_F16 && dout_dtype != QFA_BF16) return set_error(QFA_EINVAL, "%s: dout_dtype must be QFA_F16 or QFA_BF16", who);
   }
   if (!direct && io_dtype != QFA_F16) return set_error(QFA_EUNSUPPORTED, "%s: io_dtype (q, o, dout) must be QFA_F16", who);
+  // (the forward takes bf16 scales too)
+  if (scale_dtype != QFA_F32 && scale_dtype != QFA_F16) return set_error(QFA_EINVAL, "%s: scale_dtype must be QFA_F32 or QFA_F16", who);
   if (grad_dtype != QFA_F16 && grad_dtype != QFA_BF16)
     return set_error(QFA_EINVAL, "%s: grad_dtype (dq, dkv) must be QFA_F16 or QFA_BF16", who);
   if (!aligned16(dout) || !aligned16(dq) || !aligned16(dkv))

@@ -121,6 +121,17 @@ def test_argument_errors_need_no_gpu(qfa):
     assert L.qfa_dout_normalise(ok_ptr, 1, 64, ok_ptr + 2, 1, 5, ok_ptr, ok_ptr, ok_ptr, None) == -1 and b"aligned" in L.qfa_last_error()
 
 
+@pytest.mark.parametrize("Nq,D", [(16, 128), (64, 128), (100, 64), (16, 256)])
+def test_shared_kv_backward_refuses_bf16_scales(qfa, Nq, D):
+    """Its kernels read scales of 32 bits or binary16, whatever type q has."""
+    from quant_flash_attn_amd import _lib
+    L, p, Nk = _lib.lib(), 0x1000, 300
+    sq, sc = (Nq * D, Nq * D, D), (Nk * D, Nk * D, D)
+    rc = L.qfa_attn_bwd_shared_kv_direct(p, p, p, 2, p, p, p, p, p, p, 2, 2, 2, 1, 1, Nq, Nk, D, *sq, *sc, *sq, *sq, *sq, *sc, 0.1,
+                                         None, 0, None)
+    assert rc == -1 and b"scale_dtype" in L.qfa_last_error()
+
+
 def test_cpu_tensors_are_refused_not_emulated(qfa):
     x = torch.randn(1, 2, 16, 64)
     with pytest.raises(RuntimeError, match="GPU only"):
