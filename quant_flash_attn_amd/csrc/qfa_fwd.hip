@@ -286,7 +286,8 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   float m_ref = -INFINITY;   // reference maximum of u = score / a_i used in the exponent
   float m_bound = -INFINITY;                        // m_ref + threshold / a_i
   const float thr_i = FWD_RESCALE_THRESHOLD / a_i;
-  float nm = INFINITY;       // -a_i * m_ref
+  // -a_i * m_ref; 0 while a row has seen no key of its split, as in move_ref, which never comes where all the wave sees is NaN
+  float nm = SPLIT ? 0.f : INFINITY;
   float l_run = 0.f;         // this lane's share of the row sum
 
   // raw int32 block -> u = sk * (S + zero-point correction); returns the block maximum of the row

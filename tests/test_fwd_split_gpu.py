@@ -98,3 +98,25 @@ def test_split_forward_replayed_from_a_graph(qfa):
             q.neg_()
             want = qfa.quant_flash_attn_qkv(q, k, v, True, 0.09)
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_nan_keys_stay_with_the_queries_that_see_them(qfa, D):
+    """A part of the keys in which some queries of a wave see NaN keys only and the others none: those others keep their rows."""
+    B, H, Nq, Nk, sm = 1, 2, 1090, 1100, 1.0 / math.sqrt(D)   # query i sees keys up to i + 10: parts begin inside a wave's triangle
+    rows = B * H * Nq * (D + 2) * 4
+    splits = _workspace(B, H, Nq, Nk, D, True) // rows
+    assert splits > 1, "the plan splits this shape"
+    part = -(-((Nk + 63) // 64) // splits) * 64
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn((B, H, n, D), generator=g).bfloat16().to(DEV) for n in (Nq, Nk, Nk))
+    (kc, ks, kz), vq, none = qfa.asymmetric_quant_per_token(k), qfa.asymmetric_quant_per_token(v), torch.empty(0, device=DEV)
+    with torch.no_grad():
+        want = qfa.quant_flash_attn_quantized_kv(q, none, none, (kc, ks, kz), vq, True, sm)
+        ks = ks.clone()
+        ks[:, :, part:] = float("nan")
+        got = qfa.quant_flash_attn_quantized_kv(q, none, none, (kc, ks, kz), vq, True, sm)
+    first = part - (Nk - Nq)   # the first query that sees a NaN key
+    assert torch.isnan(got[:, :, first:]).all()
+    # (a wave's references may move at other tiles: the probabilities are rounded against another one)
+    assert_close("O", got[:, :, :first].cpu(), want[:, :, :first].double().cpu(), scaled=True, rel=2.0 ** -7)
