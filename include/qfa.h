@@ -279,7 +279,7 @@ int qfa_attn_bwd_shared_kv_direct(const void *q, const int8_t *codes, const void
  * Attention forward of a SHORT query block on an INT8 cache of keys and values (decoding, a few queries at a time):
  *     O = softmax(sm_scale * Q^ K^^T) V^,   Q^, K^, V^ = scale * (codes - zero_point) per token
  * Q is quantized inside by the arithmetic of qfa_quant_per_token, the scores are those of qfa_attn_fwd on these codes,
- * V enters as its exact codes; no LSE.  One pass over the cache (bound by reading it); every 16 queries read it again
+ * V enters as its exact codes; no LSE (see below).  One pass over the cache (bound by reading it); every 16 queries read it again
  * (from the L2), so long query blocks belong to qfa_attn_fwd.  No counterpart in the reference, whose operator has one
  * tensor for K and V (quant_flash_attn.py:22-83).
  *   q, o   [B,H,Nq,D] of q_dtype (QFA_F32 / QFA_F16 / QFA_BF16)
@@ -298,6 +298,13 @@ int qfa_attn_fwd_cache(const void *q, int q_dtype, const int8_t *kc, const void 
                        int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh, int64_t skn,
                        int64_t svb, int64_t svh, int64_t svn, int64_t sob, int64_t soh, int64_t son, float sm_scale,
                        int causal, void *workspace, int64_t workspace_bytes, void *stream);
+
+/* ... with the LSE (nullable) that qfa_attn_fwd writes, [B*H*Nq]: a backward takes it beside this O */
+int qfa_attn_fwd_cache_lse(const void *q, int q_dtype, const int8_t *kc, const void *ks, const int8_t *kz, const int8_t *vc,
+                           const void *vs, const int8_t *vz, int scale_dtype, void *o, float *lse, int64_t B, int64_t H,
+                           int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh,
+                           int64_t skn, int64_t svb, int64_t svh, int64_t svn, int64_t sob, int64_t soh, int64_t son,
+                           float sm_scale, int causal, void *workspace, int64_t workspace_bytes, void *stream);
 
 /*
  * Measurement hook, same arguments as qfa_attn_fwd: runs the forward kernel with the exponentials

@@ -48,6 +48,7 @@ _SIGNATURES = {
                                      + [_F, _P, _L, _P]),
     "qfa_attn_fwd_cache_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I]),
     "qfa_attn_fwd_cache": (c_int, [_P, _I] + [_P] * 6 + [_I, _P, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P, _L, _P]),
+    "qfa_attn_fwd_cache_lse": (c_int, [_P, _I] + [_P] * 6 + [_I, _P, _P, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P, _L, _P]),
     "qfa_bench_qk_stage": (c_int, [_P] * 11 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P]),
     "qfa_sum_grads": (c_int, [_P, _P, _P, _I, _L, _P]),
     "qfa_dout_normalise_workspace_bytes": (c_int64, []),

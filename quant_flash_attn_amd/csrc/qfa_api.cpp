@@ -409,6 +409,15 @@ int qfa_attn_fwd_cache(const void *q, int q_dtype, const int8_t *kc, const void 
                        int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh, int64_t skn,
                        int64_t svb, int64_t svh, int64_t svn, int64_t sob, int64_t soh, int64_t son, float sm_scale,
                        int causal, void *workspace, int64_t workspace_bytes, void *stream) {
+  return qfa_attn_fwd_cache_lse(q, q_dtype, kc, ks, kz, vc, vs, vz, scale_dtype, o, nullptr, B, H, Nq, Nk, D, sqb, sqh, sqn, skb, skh,
+                                skn, svb, svh, svn, sob, soh, son, sm_scale, causal, workspace, workspace_bytes, stream);
+}
+
+int qfa_attn_fwd_cache_lse(const void *q, int q_dtype, const int8_t *kc, const void *ks, const int8_t *kz, const int8_t *vc,
+                           const void *vs, const int8_t *vz, int scale_dtype, void *o, float *lse, int64_t B, int64_t H,
+                           int64_t Nq, int64_t Nk, int D, int64_t sqb, int64_t sqh, int64_t sqn, int64_t skb, int64_t skh,
+                           int64_t skn, int64_t svb, int64_t svh, int64_t svn, int64_t sob, int64_t soh, int64_t son,
+                           float sm_scale, int causal, void *workspace, int64_t workspace_bytes, void *stream) {
   const char *who = "attn_fwd_cache";
   if (!q || !kc || !ks || !kz || !vc || !vs || !vz || !o) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
   if (!is_float_dtype(q_dtype)) return set_error(QFA_EINVAL, "%s: q_dtype %d is not QFA_F32/F16/BF16", who, q_dtype);
@@ -432,6 +441,7 @@ int qfa_attn_fwd_cache(const void *q, int q_dtype, const int8_t *kc, const void 
   CacheAttnArgs a;
   memset(&a, 0, sizeof(a));
   a.q = q; a.kc = kc; a.ks = ks; a.kz = kz; a.vc = vc; a.vs = vs; a.vz = vz; a.o = o;
+  a.lse = lse;
   a.B = B; a.H = H; a.Nq = Nq; a.Nk = Nk; a.D = D; a.q_dtype = q_dtype; a.scale_dtype = scale_dtype;
   a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.skb = skb; a.skh = skh; a.skn = skn;
   a.svb = svb; a.svh = svh; a.svn = svn; a.sob = sob; a.soh = soh; a.son = son;

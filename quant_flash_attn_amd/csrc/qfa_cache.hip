@@ -37,6 +37,7 @@ namespace qfa {
 struct CacheArgs {
   const void *q; const int8_t *kc; const void *ks; const int8_t *kz; const int8_t *vc; const void *vs; const int8_t *vz;
   void *o;
+  float *lse;          // nullable
   float *po, *pml;     // splits > 1: unnormalised partial results [B*H*Nq][splits][D], and (m in log2 units, l)
   int64_t H;
   int64_t sqb, sqh, sqn, skb, skh, skn, svb, svh, svn, sob, soh, son;
@@ -340,6 +341,7 @@ template <typename S, int D> __global__ __launch_bounds__(256, D == 64 ? 4 : cac
       if (d == 0) *reinterpret_cast<f32x2 *>(a.pml + 2 * slot) = f32x2{m, l};
     } else {
       const float inv = 1.0f / l;
+      if (a.lse && d == 0) a.lse[(int64_t)bh * a.Nq + qg] = (m + __log2f(l)) * kLn2;
       const int64_t off = b * a.sob + h * a.soh + (int64_t)qg * a.son;
       store4(static_cast<char *>(a.o) + off * (a.q_dtype == QFA_F32 ? 4 : 2), a.q_dtype, d,
              f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
@@ -362,7 +364,7 @@ int64_t cache_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int 
 
 template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, hipStream_t st) {
   CacheArgs a;
-  a.q = x.q; a.kc = x.kc; a.ks = x.ks; a.kz = x.kz; a.vc = x.vc; a.vs = x.vs; a.vz = x.vz; a.o = x.o;
+  a.q = x.q; a.kc = x.kc; a.ks = x.ks; a.kz = x.kz; a.vc = x.vc; a.vs = x.vs; a.vz = x.vz; a.o = x.o; a.lse = x.lse;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk; a.BH = (int)(x.B * x.H);
   a.sqb = x.sqb; a.sqh = x.sqh; a.sqn = x.sqn; a.skb = x.skb; a.skh = x.skh; a.skn = x.skn;
   a.svb = x.svb; a.svh = x.svh; a.svn = x.svn; a.sob = x.sob; a.soh = x.soh; a.son = x.son;
@@ -383,7 +385,7 @@ template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, 
   cache_fwd_kernel<S, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_cache")) return e;
   if (a.splits > 1) {
-    const SplitMergeArgs m = {a.po, a.pml, a.o, nullptr, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, a.q_dtype, nullptr};
+    const SplitMergeArgs m = {a.po, a.pml, a.o, a.lse, a.H, a.sob, a.soh, a.son, a.Nq, a.splits, a.q_dtype, nullptr};
     return launch_split_merge<D>(m, x.B * x.H * x.Nq, "qfa_attn_fwd_cache (merge)", st);
   }
   return 0;

@@ -124,6 +124,7 @@ int launch_skv_bwd_long(const SkvAttnArgs &a, hipStream_t st);   // io_dtype QFA
 struct CacheAttnArgs {
   const void *q; const int8_t *kc; const void *ks; const int8_t *kz; const int8_t *vc; const void *vs; const int8_t *vz;
   void *o;
+  float *lse;        // nullable
   void *workspace;   // nullable: partial results when the keys are split
   int64_t B, H, Nq, Nk;
   int64_t sqb, sqh, sqn, skb, skh, skn, svb, svh, svn, sob, soh, son;

@@ -52,7 +52,7 @@ struct Api {
   QFA_ENTRY(qfa_attn_bwd_shared_kv_is_direct);
   QFA_ENTRY(qfa_attn_bwd_shared_kv_direct);
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
-  QFA_ENTRY(qfa_attn_fwd_cache);
+  QFA_ENTRY(qfa_attn_fwd_cache_lse);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
   QFA_ENTRY(qfa_dout_normalise_cast);
 #undef QFA_ENTRY
@@ -87,7 +87,7 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_attn_bwd_shared_kv_is_direct);
   QFA_ENTRY(qfa_attn_bwd_shared_kv_direct);
   QFA_ENTRY(qfa_attn_fwd_cache_workspace_bytes);
-  QFA_ENTRY(qfa_attn_fwd_cache);
+  QFA_ENTRY(qfa_attn_fwd_cache_lse);
   QFA_ENTRY(qfa_dout_normalise_workspace_bytes);
   QFA_ENTRY(qfa_dout_normalise_cast);
 #undef QFA_ENTRY
@@ -504,8 +504,9 @@ struct CacheKept : Kept {
 Quantized keys_of(const Tensor &kc, const Tensor &ks, const Tensor &kz, const Tensor &kr) {
   return view_of({kc, ks, kz, kr});
 }
-CacheKept cache_forward(const Tensor &q_in, const Tensor &kc, const Tensor &ks, const Tensor &kz, const Tensor &vc,
-                        const Tensor &vs, const Tensor &vz, bool causal, double sm) {
+// what the long-query kernels take of q and the cache: everything but O and the LSE
+CacheKept cache_stage(const Tensor &q_in, const Tensor &kc, const Tensor &ks, const Tensor &kz, const Tensor &vc,
+                      const Tensor &vs, const Tensor &vz) {
   const c10::DeviceGuard guard(q_in.device());
   const Tensor q = check_input(q_in);
   check_codes(kc, "k.codes");
@@ -534,6 +535,13 @@ CacheKept cache_forward(const Tensor &q_in, const Tensor &kc, const Tensor &ks, 
                             dtype_code(vsf.scalar_type()), vzf.data_ptr<int8_t>(), r.v16.data_ptr(), dtype_code(r.v16.scalar_type()),
                             pb.B, pb.H, kc.size(2), (int)pb.D, QFA_STRIDES(r.kc), QFA_STRIDES(v), stream_of(q)),
         "qfa_cache_stage");
+  return r;
+}
+CacheKept cache_forward(const Tensor &q, const Tensor &kc, const Tensor &ks, const Tensor &kz, const Tensor &vc, const Tensor &vs,
+                        const Tensor &vz, bool causal, double sm) {
+  CacheKept r = cache_stage(q, kc, ks, kz, vc, vs, vz);
+  const c10::DeviceGuard guard(q.device());
+  const PairBuffer pb(q.size(0), q.size(1), q.size(2), 0, q.size(3));
   r.o16 = empty({pb.B, pb.H, pb.N[0], pb.D}, r.v16.scalar_type(), q);
   fwd_split_into(pb.view(r.buf, 0), keys_of(r.kc, r.ks, r.kz, r.kr), r.v16, r.o16, Tensor(), pb.lse_of(r.buf), causal, sm);
   r.o = to(r.o16, q.scalar_type());
@@ -558,7 +566,8 @@ int64_t cache_max_q(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
 // to 512 queries, 300 to 20000 keys (within 8 % in the mean): the short one takes what its memory or its blocks of 16 queries
 // take, and loses by a last round of workgroups that is not full; the other one the pass over the cache and blocks of 128
 // queries.  Calls are taken from the other path where that should gain 12 %: over all shapes the choice costs 0.4 - 1 % against
-// the better path each time, where the line alone cost 3 - 6 %; the moved calls gain 1.4 times in the mean, the worst lost 15 %.
+// the better path each time, where the line alone cost 3 - 6 %; the moved calls gain 1.4 times in the mean.  920 of them timed on both once more: 1.6 times, three
+// lost more than 3 % (7 heads, 149 queries, 19668 keys of 256: 4.6 %).
 bool cache_short_cheaper(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
   struct Cost { double s0, s_byte, s_block, s_start, s_fill, l0, l_byte, l_block, l_idle, l_query; };
   static const Cost c64 = {9.8, 0.48, 11.4, 2.0, 0.37, 18.6, 0.84, 33.7, 0.1, 0.69}, c128 = {11.6, 0.56, 22.4, 6.1, 0.22, 20.4, 0.88, 51.9, 0.095, 0.42},
@@ -572,13 +581,15 @@ bool cache_short_cheaper(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
   const double l = c.l0 + c.l_byte * n * (double)D + c.l_block * n * (double)mb * (1.0 + c.l_idle * idle) + c.l_query * (double)(BH * Nq * D) * 1e-6;
   return s < 0.88 * l;
 }
-bool cache_takes_short(const Tensor &q, const Tensor &kc) {
+enum class CachePath { Short, ShortBeyondLine, Long };
+CachePath cache_path(const Tensor &q, const Tensor &kc) {
   const int64_t BH = q.size(0) * q.size(1), Nq = q.size(2), Nk = kc.size(2), D = q.size(3);
-  if (Nq <= cache_max_q(BH, Nq, Nk, D)) return true;
-  return Nq <= 512 && BH > 0 && Nk > 0 && cache_short_cheaper(BH, Nq, Nk, D);   // (as far as was measured)
+  if (Nq <= cache_max_q(BH, Nq, Nk, D)) return CachePath::Short;
+  const bool cheaper = Nq <= 512 && BH > 0 && Nk > 0 && cache_short_cheaper(BH, Nq, Nk, D);   // (as far as was measured)
+  return cheaper ? CachePath::ShortBeyondLine : CachePath::Long;
 }
 Tensor cache_short(const Tensor &q_in, const Tensor &kc_in, const Tensor &ks_in, const Tensor &kz, const Tensor &vc_in,
-                   const Tensor &vs_in, const Tensor &vz, bool causal, double sm) {
+                   const Tensor &vs_in, const Tensor &vz, bool causal, double sm, float *lse = nullptr) {
   const c10::DeviceGuard guard(q_in.device());
   const Tensor q = check_input(q_in);
   check_codes(kc_in, "k.codes");
@@ -592,11 +603,11 @@ Tensor cache_short(const Tensor &q_in, const Tensor &kc_in, const Tensor &ks_in,
   Tensor o = empty({B, H, Nq, D}, q.scalar_type(), q), ws;
   const int64_t ws_bytes = api.qfa_attn_fwd_cache_workspace_bytes(B, H, Nq, Nk, (int)D);
   if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, q);
-  check(api.qfa_attn_fwd_cache(q.data_ptr(), dtype_code(q.scalar_type()), kc.data_ptr<int8_t>(), ks.data_ptr(),
-                               kzf.data_ptr<int8_t>(), vc.data_ptr<int8_t>(), vs.data_ptr(), vzf.data_ptr<int8_t>(),
-                               dtype_code(sdt), o.data_ptr(), B, H, Nq, Nk, (int)D, QFA_STRIDES(q), QFA_STRIDES(kc),
-                               QFA_STRIDES(vc), QFA_STRIDES(o), (float)sm, causal, ws_bytes > 0 ? ws.data_ptr() : nullptr,
-                               ws_bytes, stream_of(q)),
+  check(api.qfa_attn_fwd_cache_lse(q.data_ptr(), dtype_code(q.scalar_type()), kc.data_ptr<int8_t>(), ks.data_ptr(),
+                                   kzf.data_ptr<int8_t>(), vc.data_ptr<int8_t>(), vs.data_ptr(), vzf.data_ptr<int8_t>(),
+                                   dtype_code(sdt), o.data_ptr(), lse, B, H, Nq, Nk, (int)D, QFA_STRIDES(q), QFA_STRIDES(kc),
+                                   QFA_STRIDES(vc), QFA_STRIDES(o), (float)sm, causal, ws_bytes > 0 ? ws.data_ptr() : nullptr,
+                                   ws_bytes, stream_of(q)),
         "qfa_attn_fwd_cache");
   return o;
 }
@@ -606,10 +617,21 @@ struct CacheFn : torch::autograd::Function<CacheFn> {
                         const Tensor &ks, const Tensor &kz, const Tensor &vc, const Tensor &vs, const Tensor &vz, bool causal,
                         double sm) {
     const at::AutoDispatchBelowADInplaceOrView below;
-    CacheKept r = cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm);
     // what a call without a gradient returns, bit for bit (a forward that is computed again for its gradient, as activation
-    // checkpointing does); the backward takes O, LSE and V of the path above
-    if (cache_takes_short(q, kc)) r.o = cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
+    // checkpointing does)
+    const CachePath path = cache_path(q, kc);
+    CacheKept r;
+    if (path == CachePath::ShortBeyondLine) {
+      // O and the LSE of the short kernel serve the backward too, which wants the staged keys and values beside them
+      r = cache_stage(q, kc, ks, kz, vc, vs, vz);
+      const PairBuffer pb(q.size(0), q.size(1), q.size(2), 0, q.size(3));
+      r.o = cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm, pb.lse_of(r.buf));
+      r.o16 = to(r.o, io_dtype(q));
+    } else {
+      r = cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm);
+      // (the backward takes O, LSE and V of the long-query path here)
+      if (path == CachePath::Short) r.o = cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
+    }
     ctx->save_for_backward({r.buf, r.v16, r.o16, r.kc, r.ks, r.kz, r.kr});
     ctx->saved_data["causal"] = causal;
     ctx->saved_data["sm"] = sm;
@@ -640,7 +662,7 @@ Tensor cache_op(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, con
                         q.size(0) == kc.size(0) && q.size(1) == kc.size(1),
                     "shape mismatch: q ", q.sizes(), ", k codes ", kc.sizes(), ", v codes ", vc.sizes());
   if (wants_grad({&q, &k_fp16, &v_fp16})) return CacheFn::apply(q, k_fp16, v_fp16, kc, ks, kz, vc, vs, vz, causal, sm);
-  if (cache_takes_short(q, kc)) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
+  if (cache_path(q, kc) != CachePath::Long) return cache_short(q, kc, ks, kz, vc, vs, vz, causal, sm);
   return cache_forward(q, kc, ks, kz, vc, vs, vz, causal, sm).o;
 }
 Tensor cache(const Tensor &q, const Tensor &k_fp16, const Tensor &v_fp16, const Tensor &kc, const Tensor &ks,
