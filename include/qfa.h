@@ -144,9 +144,10 @@ int qfa_attn_fwd(const int8_t *qc, const float *sq, const int8_t *zq, const int3
 /*
  * The same with two additions.  o32 (nullable): O in fp32, [B,H,Nq,D] dense, unrounded; o, the 16-bit one that a backward takes,
  * may be NULL then.  workspace (nullable): with few queries in all, most of the chip is idle; given a caller-owned scratch of
- * qfa_attn_fwd_split_workspace_bytes(...) bytes (16-byte aligned; 0 when no split pays) the keys are split over workgroups and
- * a second small kernel merges their partial (O, m, l).
+ * qfa_attn_fwd_split_workspace_bytes(...) bytes (16-byte aligned; 0 when no split pays, at most QFA_SPLIT_PART_BYTES) the keys
+ * are split over workgroups and a second small kernel merges their partial (O, m, l).
  */
+#define QFA_SPLIT_PART_BYTES (224 << 20)
 int64_t qfa_attn_fwd_split_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal);
 
 int qfa_attn_fwd_split(const int8_t *qc, const float *sq, const int8_t *zq, const int32_t *rq, const int8_t *kc,
@@ -400,8 +401,9 @@ int qfa_attn_bwd_f32(const int8_t *qc, const float *sq, const int8_t *zq, const 
 
 /*
  * The workspace with which qfa_attn_bwd (f32: qfa_attn_bwd_f32) may split its work further where B*H and the sequence alone
- * leave CUs idle: the queries of dK and dV, and the keys of dQ, are dealt to several workgroups, whose fp32 parts lie behind
- * what the plain call needs and are added by a third small kernel.  The same number where no split pays.
+ * leave CUs idle: the queries of dK and dV, and the keys of dQ, are dealt to several workgroups, whose fp32 parts (at
+ * most QFA_SPLIT_PART_BYTES) lie behind what the plain call needs and are added by a third small kernel.  The same number where
+ * no split pays.
  */
 int64_t qfa_attn_bwd_split_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal, int f32);
 

@@ -326,8 +326,9 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
   bwd_prep_kernel<T, D><<<dim3((unsigned)(BH * (a.tiles_q + a.tiles_k))), dim3(256), 0, st>>>(a, (int)(BH * a.tiles_q));
   if (int e = check_launch("qfa_attn_bwd (staging)")) return e;
   const BwdPlan plan = bwd_plan(BH, x.Nq, x.Nk, D, x.causal, x.may_split);
-  float *part = reinterpret_cast<float *>(a.ws_q + (x.f32 ? bwd_f32_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)
+  float *const parts = reinterpret_cast<float *>(a.ws_q + (x.f32 ? bwd_f32_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)
                                                          : bwd_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)));
+  float *part = parts;
   BwdSumArgs sum;
   sum.count = 0; sum.H = x.H; sum.out_f32 = x.f32;
   int64_t blocks = 0;
@@ -350,6 +351,17 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
     k.grad_f32 = 1;
   }
   if (int e = launch_dkv<T, D>(k, BH, x.causal, plan.blocks_dkv, plan.splits_dkv, st)) return e;
+  auto add_parts = [&]() -> int {
+    if (sum.count == 0) return 0;
+    bwd_sum_kernel<T, D><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sum);
+    return check_launch("qfa_attn_bwd (sum)");
+  };
+  if (plan.sum_between) {   // dQ's parts take the place of these
+    if (int e = add_parts()) return e;
+    part = parts;
+    sum.count = 0;
+    blocks = 0;
+  }
   BwdArgs q = a;
   q.per_split = plan.keys_per_split;
   q.last_part = (plan.splits_dq - 1) * plan.keys_per_split;
@@ -360,9 +372,7 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
     q.grad_f32 = 1;
   }
   if (int e = launch_dq<T, D>(q, BH, x.causal, plan.blocks_dq, plan.splits_dq, st)) return e;
-  if (sum.count == 0) return 0;
-  bwd_sum_kernel<T, D><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sum);
-  return check_launch("qfa_attn_bwd (sum)");
+  return add_parts();
 }
 
 int launch_bwd(const AttnArgs &x, hipStream_t st) {

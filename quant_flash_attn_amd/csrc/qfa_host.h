@@ -64,8 +64,9 @@ inline int64_t bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t
   return bwd_workspace_bytes(B, H, Nq, Nk, D) + B * H * Nq * D * 2;
 }
 
-// How the backward's two MFMA kernels are launched: 32-row blocks per wave, and the parts of the streamed rows
-struct BwdPlan { int blocks_dkv, splits_dkv, queries_per_split, blocks_dq, splits_dq, keys_per_split; };
+// How the backward's two MFMA kernels are launched: 32-row blocks per wave, and the parts of the streamed rows; the memory of the
+// parts, and whether those of dQ take the place of the others
+struct BwdPlan { int blocks_dkv, splits_dkv, queries_per_split, blocks_dq, splits_dq, keys_per_split, sum_between; int64_t part_bytes; };
 BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_split);
 int64_t bwd_split_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal);
 

@@ -24,7 +24,11 @@ struct SplitCost {
   double base;
 };
 
-constexpr int64_t MAX_WGS = 1700, MAX_WGS_BWD = 1100;   // of a divided launch: as far as was measured, and bounds the parts' memory
+constexpr int64_t MAX_WGS = 1700, MAX_WGS_BWD = 1100;   // of a divided launch: as far as was measured
+// Of the parts of one launch: what MAX_WGS leaves of the forward (214 MiB, long sequences of few wide heads; 192 MiB cost 3 heads,
+// 22757 x 22757 of 256, causal, 1019 -> 1474 us), and less than dK and dV could fill (275 MiB).  Between 1.03 times faster and slower where it bites there
+// (5 heads of 17926 of 128, forward and backward: 3168 -> 3077 us; 5 of 24880, causal: 3680 -> 3765).
+constexpr int64_t MAX_PART_FLOATS = QFA_SPLIT_PART_BYTES / 4;
 
 // `blocks` workgroups of `rows` rows each for each of `heads` heads, the streamed rows in tiles of `tile` (64 or 32), s parts of
 // `each` rows; ends: block i sees streamed rows up to (i + 1) * rows + coff, otherwise from i * rows - coff on
@@ -83,7 +87,7 @@ void fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int *splits
   if (BH <= MAX_WGS && blocks <= MAX_WGS && 2 * BH * blocks <= MAX_WGS) {
     SplitWork w = {BH, blocks, 128, Nk, 64, Nk - Nq, causal != 0, true};
     w.count();
-    best_division(Nk, std::min<int64_t>(64, MAX_WGS / (BH * blocks)), 0.92 * w.time(c, 1, each, 0), &s, &each,
+    best_division(Nk, std::min<int64_t>({64, MAX_WGS / (BH * blocks), MAX_PART_FLOATS / (BH * Nq * (D + 2))}), 0.92 * w.time(c, 1, each, 0), &s, &each,
                   [&](int64_t n, int64_t e) { return w.time(c, n, e, 8e-6 * (double)(BH * Nq * n * (D + 2))); });
   }
   *splits = (int)s;
@@ -132,7 +136,7 @@ static void bwd_part(int64_t BH, int64_t rows, int64_t streamed, int D, bool cau
       const SplitWork &x = w[r - 1];
       const int64_t was = s;
       s = 1;
-      best_division(streamed, std::min<int64_t>(32, MAX_WGS_BWD / (BH * x.blocks)), best, &s, &each, [&](int64_t n, int64_t e) {
+      best_division(streamed, std::min<int64_t>({32, MAX_WGS_BWD / (BH * x.blocks), MAX_PART_FLOATS / (BH * rows * D * tensors)}), best, &s, &each, [&](int64_t n, int64_t e) {
         return x.time(c[r - 1], n, e, 8e-6 * (double)(BH * rows * n) * D * tensors);
       });
       if (s > 1) {
@@ -161,12 +165,17 @@ BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_
            &p.splits_dkv, &p.queries_per_split);
   bwd_part(BH, Nq, Nk, D, causal, true, Nk - Nq, f, may_split, D == 64 ? dq64 : D == 128 ? dq128 : dq256, 1, &p.blocks_dq, &p.splits_dq,
            &p.keys_per_split);
+  const int64_t kv = p.splits_dkv > 1 ? BH * D * 8 * Nk * p.splits_dkv : 0, q = p.splits_dq > 1 ? BH * D * 4 * Nq * p.splits_dq : 0;
+  // large parts of both: dK and dV are added before dQ starts, whose parts take their place.  One launch more, of a call of
+  // milliseconds (2 heads, 16384 x 16384 of 256, causal, forward and backward: 1939 -> 1908 us); smaller ones lose by it (4 heads of
+  // 2300: 188 -> 191)
+  p.sum_between = kv > 0 && q > 0 && kv + q > (128 << 20);
+  p.part_bytes = p.sum_between ? std::max(kv, q) : kv + q;
   return p;
 }
 
 int64_t bwd_split_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal) {
-  const BwdPlan p = bwd_plan(B * H, Nq, Nk, D, causal, 1);
-  return B * H * D * 4 * ((p.splits_dkv > 1 ? 2 * Nk * p.splits_dkv : 0) + (p.splits_dq > 1 ? Nq * p.splits_dq : 0));
+  return bwd_plan(B * H, Nq, Nk, D, causal, 1).part_bytes;
 }
 
 }  // namespace qfa

@@ -44,6 +44,7 @@ struct Api {
   QFA_ENTRY(qfa_attn_bwd);
   QFA_ENTRY(qfa_attn_bwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd_f32);
+  QFA_ENTRY(qfa_attn_bwd_f32_workspace_bytes);
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
@@ -79,6 +80,7 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_attn_bwd);
   QFA_ENTRY(qfa_attn_bwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_bwd_f32);
+  QFA_ENTRY(qfa_attn_bwd_f32_workspace_bytes);
   QFA_ENTRY(qfa_sum_grads);
   QFA_ENTRY(qfa_attn_fwd_shared_kv_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_shared_kv);
@@ -300,18 +302,28 @@ void fwd_into(const Quantized &q, const Quantized &k, const Tensor &v, const Ten
         qk_only ? "qfa_bench_qk_stage" : "qfa_attn_fwd");
 }
 
+// Scratch that a call can do without: undefined for none, and where the memory is not there (the call is not split then, and runs
+// wherever it runs without a scratch)
+Tensor optional_scratch(int64_t bytes, const Tensor &like) {
+  if (bytes <= 0) return Tensor();
+  try {
+    return empty({bytes}, at::kByte, like);
+  } catch (const c10::OutOfMemoryError &) {
+    return Tensor();
+  }
+}
+void *data_of(const Tensor &scratch) { return scratch.defined() ? scratch.data_ptr() : nullptr; }
+int64_t bytes_of(const Tensor &scratch) { return scratch.defined() ? scratch.numel() : 0; }
+
 // the same with the keys split over workgroups where there are few queries; o32 dense, o or o32 may be undefined
 void fwd_split_into(const Quantized &q, const Quantized &k, const Tensor &v, const Tensor &o, const Tensor &o32, float *lse,
                     bool causal, double sm) {
-  const int64_t ws_bytes = api.qfa_attn_fwd_split_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D, causal);
-  Tensor ws;
-  if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, v);
+  const Tensor ws = optional_scratch(api.qfa_attn_fwd_split_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D, causal), v);
   const Tensor &like = o.defined() ? o : o32;
   check(api.qfa_attn_fwd_split(q.codes, q.scale, q.zp, q.rowsum, k.codes, k.scale, k.zp, k.rowsum, v.data_ptr(),
                                o.defined() ? o.data_ptr() : nullptr, o32.defined() ? o32.data_ptr<float>() : nullptr, lse,
                                dtype_code(v.scalar_type()), q.B, q.H, q.N, k.N, (int)q.D, q.sb, q.sh, q.sn, k.sb, k.sh, k.sn,
-                               QFA_STRIDES(v), QFA_STRIDES(like), (float)sm, causal, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
-                               stream_of(v)),
+                               QFA_STRIDES(v), QFA_STRIDES(like), (float)sm, causal, data_of(ws), bytes_of(ws), stream_of(v)),
         "qfa_attn_fwd_split");
 }
 
@@ -322,11 +334,15 @@ Grads bwd_of(const Quantized &q, const Quantized &k, const Tensor &v_in, const T
              const float *lse, bool causal, double sm, bool split, bool f32 = false) {
   const at::ScalarType gt = f32 ? at::kFloat : v_in.scalar_type();
   const Tensor v = rows16(v_in), o = rows16(o_in), dout = rows16(to(do_in, gt));
-  const int64_t ws_bytes = split || f32 ? api.qfa_attn_bwd_split_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D, causal, f32)
-                                        : api.qfa_attn_bwd_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D);
-  TORCH_CHECK_VALUE(ws_bytes > 0, "unsupported backward shape B=", q.B, " H=", q.H, " Nq=", q.N, " Nk=", k.N, " D=", q.D);
-  const Tensor ws = empty({ws_bytes}, at::kByte, v);
+  const int64_t plain = f32 ? api.qfa_attn_bwd_f32_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D)
+                            : api.qfa_attn_bwd_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D),
+                most = split || f32 ? api.qfa_attn_bwd_split_workspace_bytes(q.B, q.H, q.N, k.N, (int)q.D, causal, f32) : plain;
+  TORCH_CHECK_VALUE(plain > 0, "unsupported backward shape B=", q.B, " H=", q.H, " Nq=", q.N, " Nk=", k.N, " D=", q.D);
   Tensor dq = empty({q.B, q.H, q.N, q.D}, gt, v), dk = empty({q.B, q.H, k.N, q.D}, gt, v), dv = empty({q.B, q.H, k.N, q.D}, gt, v);
+  Tensor ws;   // (last: what is left is for the parts)
+  if (most > plain) ws = optional_scratch(most, v);
+  if (!ws.defined()) ws = empty({plain}, at::kByte, v);
+  const int64_t ws_bytes = ws.numel();
   if (f32) {
     check(api.qfa_attn_bwd_f32(q.codes, q.scale, q.zp, q.rowsum, k.codes, k.scale, k.zp, k.rowsum, v.data_ptr(), o.data_ptr(),
                                dout.data_ptr<float>(), lse, ws.data_ptr(), ws_bytes, dq.data_ptr<float>(), dk.data_ptr<float>(),
@@ -728,17 +744,15 @@ std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, c
   const Tensor q = rows16(q_in), codes = rows16(codes_in), o = rows16(o_in), dout = rows16(to(do_in, direct ? io_dtype(do_in) : at::kHalf));
   Tensor dq = empty({B, H, Nq, D}, grad_dtype, q), dkv = empty({B, H, Nk, D}, grad_dtype, q);
   // scratch for the split over keys where B*H alone cannot fill the GPU (0: no split)
-  const int64_t ws_bytes = split ? api.qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) : 0;
-  Tensor ws;
-  if (ws_bytes > 0) ws = empty({ws_bytes}, at::kByte, q);
+  const Tensor ws = optional_scratch(split ? api.qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) : 0, q);
   if (direct) {
     check(api.qfa_attn_bwd_shared_kv_direct(q.data_ptr(), codes.data_ptr<int8_t>(), scale.data_ptr(), dtype_code(scale.scalar_type()),
                                             zp.data_ptr<int8_t>(), o.data_ptr(), dout.data_ptr(), lse.data_ptr<float>(),
                                             dq.data_ptr(), dkv.data_ptr(), dtype_code(q.scalar_type()),
                                             dtype_code(dout.scalar_type()), dtype_code(grad_dtype), B, H, Nq, Nk, (int)D,
                                             QFA_STRIDES(q), QFA_STRIDES(codes), QFA_STRIDES(o), QFA_STRIDES(dout),
-                                            QFA_STRIDES(dq), QFA_STRIDES(dkv), (float)sm, ws_bytes > 0 ? ws.data_ptr() : nullptr,
-                                            ws_bytes, stream_of(q)),
+                                            QFA_STRIDES(dq), QFA_STRIDES(dkv), (float)sm, data_of(ws), bytes_of(ws),
+                                            stream_of(q)),
           "qfa_attn_bwd_shared_kv_direct");
     return {dq, dkv};
   }
@@ -747,7 +761,7 @@ std::tuple<Tensor, Tensor> skv_bwd(const Tensor &q_in, const Tensor &codes_in, c
                                    dq.data_ptr(), dkv.data_ptr(), QFA_F16, dtype_code(grad_dtype),
                                    grad_scale.defined() ? grad_scale.data_ptr<float>() : nullptr, B, H, Nq, Nk, (int)D,
                                    QFA_STRIDES(q), QFA_STRIDES(codes), QFA_STRIDES(o), QFA_STRIDES(dout), QFA_STRIDES(dq),
-                                   QFA_STRIDES(dkv), (float)sm, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q)),
+                                   QFA_STRIDES(dkv), (float)sm, data_of(ws), bytes_of(ws), stream_of(q)),
         "qfa_attn_bwd_shared_kv_split");
   return {dq, dkv};
 }

@@ -1,0 +1,34 @@
+"""What the library's planning functions (C++, pure functions of the sizes) decide, so that a test can say which kernels a case is
+to reach (not collected by pytest)."""
+import ctypes
+
+from quant_flash_attn_amd import _lib
+
+_L, _I = ctypes.c_int64, ctypes.c_int
+
+
+class BwdPlan(ctypes.Structure):
+    _fields_ = [(n, _I) for n in ("blocks_dkv", "splits_dkv", "queries_per_split", "blocks_dq", "splits_dq", "keys_per_split",
+                                  "sum_between")] + [("part_bytes", _L)]
+
+
+class SkvTilePlan(ctypes.Structure):
+    _fields_ = [(n, _I) for n in ("waves", "splits", "tiles")]   # waves side by side; 0: the 16-query kernel
+
+
+def _plan(name, result, args):
+    f = getattr(_lib.lib(), name)
+    f.restype, f.argtypes = result, args
+    return f
+
+
+def bwd_plan(BH, Nq, Nk, D, causal, may_split=1):
+    return _plan("_ZN3qfa8bwd_planEllliii", BwdPlan, [_L, _L, _L, _I, _I, _I])(BH, Nq, Nk, D, int(causal), may_split)
+
+
+def skv_tile_fwd_plan(BH, Nq, Nk, D):
+    return _plan("_ZN3qfa17skv_tile_fwd_planEllli", SkvTilePlan, [_L, _L, _L, _I])(BH, Nq, Nk, D)
+
+
+def skv_tile_dq_plan(BH, Nq, Nk, D):
+    return _plan("_ZN3qfa16skv_tile_dq_planEllli", SkvTilePlan, [_L, _L, _L, _I])(BH, Nq, Nk, D)
