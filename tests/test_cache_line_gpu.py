@@ -15,11 +15,38 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
+CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+_ptr = lambda *ts: [t.data_ptr() for t in ts]
+_dense = lambda H, n, D: (H * n * D, n * D, D)
+
+
+def _short_kernel(q, kq, vq, causal, sm):
+    """O and LSE of qfa_attn_fwd_cache_lse, dense tensors"""
+    L = _lib.lib()
+    B, H, Nq, D = q.shape
+    Nk = kq[0].shape[2]
+    o, lse = torch.empty_like(q), torch.empty((B, H, Nq), device=DEV)
+    ws = torch.empty(L.qfa_attn_fwd_cache_workspace_bytes(B, H, Nq, Nk, D), dtype=torch.uint8, device=DEV)
+    strides = [s for n in (Nq, Nk, Nk, Nq) for s in _dense(H, n, D)]
+    assert L.qfa_attn_fwd_cache_lse(q.data_ptr(), CODE[q.dtype], *_ptr(*kq, *vq), CODE[kq[1].dtype], *_ptr(o, lse), B, H, Nq, Nk, D,
+                                    *strides, sm, int(causal), ws.data_ptr() if ws.numel() else None, ws.numel(),
+                                    torch.cuda.current_stream().cuda_stream) == 0, L.qfa_last_error()
+    return o, lse
+
+
 @pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("B,H,Nq,Nk,D", [(1, 4, 129, 1000, 64), (1, 3, 200, 777, 128), (2, 1, 257, 600, 256), (1, 40, 144, 300, 128),
-                                         (1, 2, 512, 513, 64), (1, 2, 513, 514, 64)])
-def test_long_blocks_on_the_short_kernel(qfa, B, H, Nq, Nk, D, causal):
+@pytest.mark.parametrize("B,H,Nq,Nk,D,short", [(1, 4, 129, 1000, 64, True), (1, 3, 200, 777, 128, True), (2, 1, 257, 600, 256, True),
+                                               (1, 40, 144, 300, 128, True), (1, 2, 512, 513, 64, True), (1, 2, 513, 514, 64, False),
+                                               (8, 8, 333, 1500, 128, False)])
+def test_long_blocks_on_the_short_kernel(qfa, B, H, Nq, Nk, D, short, causal):
     _check(qfa, B, H, Nq, Nk, D, causal, torch.float16, torch.float16, seed=Nq)
+    # which of the two took the call: the other one rounds V, and its probabilities, in other places
+    sm = 1.0 / math.sqrt(D)
+    q, k, v, _ = (t.to(DEV) for t in make_inputs("offset", B, H, Nk, D, seed=Nq, dtype=torch.float16))
+    q, kq, vq = q[:, :, :Nq].contiguous(), qfa.asymmetric_quant_per_token(k), qfa.asymmetric_quant_per_token(v)
+    none = torch.empty(0, dtype=torch.float16, device=DEV)
+    o = qfa.quant_flash_attn_quantized_kv(q, none, none, kq, vq, causal, sm)
+    assert torch.equal(o, _short_kernel(q, kq, vq, causal, sm)[0]) == short
 
 
 @pytest.mark.parametrize("B,H,Nq,Nk,D", [(1, 4, 129, 1000, 64), (1, 3, 200, 777, 128), (2, 1, 257, 600, 256), (1, 2, 512, 9001, 64)])
@@ -33,16 +60,10 @@ def test_gradient_of_the_short_kernels_output(qfa, B, H, Nq, Nk, D, dtype):
     leaves = [t.requires_grad_(True) for t in (q, k, v)]
     o = qfa.quant_flash_attn_quantized_kv(*leaves, kq, vq, True, sm)
     grads = torch.autograd.grad(o, leaves, do)
-    q, o, code = q.detach(), o.detach(), {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
-    st = torch.cuda.current_stream().cuda_stream
-    dense = lambda n: (H * n * D, n * D, D)
-    ptr = lambda *ts: [t.data_ptr() for t in ts]
+    q, o = q.detach(), o.detach()
+    dense, ptr = lambda n: _dense(H, n, D), _ptr
 
-    o2, lse = torch.empty_like(q), torch.empty((B, H, Nq), device=DEV)
-    ws = torch.empty(L.qfa_attn_fwd_cache_workspace_bytes(B, H, Nq, Nk, D), dtype=torch.uint8, device=DEV)
-    assert L.qfa_attn_fwd_cache_lse(q.data_ptr(), code[dtype], *ptr(*kq, *vq), code[kq[1].dtype], *ptr(o2, lse), B, H, Nq, Nk, D,
-                                    *dense(Nq), *dense(Nk), *dense(Nk), *dense(Nq), sm, 1, ws.data_ptr() if ws.numel() else None,
-                                    ws.numel(), st) == 0, L.qfa_last_error()
+    o2, lse = _short_kernel(q, kq, vq, True, sm)
     assert torch.equal(o, o2)
     qq = qfa.quantize_for_attention(q)
     qh, kh = (oracle.dequantize_per_token(*(x.cpu() for x in t[:3]), torch.float64) for t in (qq, kq))
@@ -55,7 +76,8 @@ def test_gradient_of_the_short_kernels_output(qfa, B, H, Nq, Nk, D, dtype):
     ws = torch.empty(L.qfa_attn_bwd_split_workspace_bytes(B, H, Nq, Nk, D, 1, 0), dtype=torch.uint8, device=DEV)
     want = torch.empty_like(do16), torch.empty_like(v16), torch.empty_like(v16)
     assert L.qfa_attn_bwd(*ptr(qq.codes, qq.scale, qq.zero_point, qq.rowsum, kq[0], kq[1].float(), kq[2], kr, v16, o16, do16, lse, ws),
-                          ws.numel(), *ptr(*want), code[io], B, H, Nq, Nk, D, *dense(Nq), *dense(Nk), *dense(Nk), *dense(Nq),
-                          *dense(Nq), *dense(Nq), *dense(Nk), *dense(Nk), sm, 1, st) == 0, L.qfa_last_error()
+                          ws.numel(), *ptr(*want), CODE[io], B, H, Nq, Nk, D, *dense(Nq), *dense(Nk), *dense(Nk), *dense(Nq),
+                          *dense(Nq), *dense(Nq), *dense(Nk), *dense(Nk), sm, 1,
+                          torch.cuda.current_stream().cuda_stream) == 0, L.qfa_last_error()
     for a, b in zip(grads, want):
         assert torch.equal(a, b.to(dtype))

@@ -30,8 +30,12 @@ def test_cast_beside_the_scaling(qfa, B, H, Nq, D):
     assert L.qfa_dout_normalise_cast(*args(b, 1), x0.data_ptr(), None, None, None, st) == -1
 
 
-def test_strided_queries_give_the_same_gradients(qfa):
-    B, H, Nq, Nk, D, sm = 2, 3, 20, 300, 128, 0.09
+@pytest.mark.parametrize("Nq,D,direct", [(20, 128, 1), (128, 128, 1), (129, 128, 0), (150, 64, 0), (17, 256, 0), (100, 256, 0)])
+def test_strided_queries_give_the_same_gradients(qfa, Nq, D, direct):
+    """Blocks whose rows a workgroup does not hold are cast in front of the backward: contiguous ones by the launch that scales dO,
+    strided ones by a copy of their own.  Shorter ones are cast inside the kernels (direct), from whatever strides."""
+    assert _lib.lib().qfa_attn_bwd_shared_kv_is_direct(Nq, D) == direct
+    B, H, Nk, sm = 2, 3, 300, 0.09
     g = torch.Generator().manual_seed(2)
     q0 = torch.randn((B, Nq, H, D), generator=g).bfloat16().to(DEV).transpose(1, 2)
     kv = torch.randn((B, H, Nk, D), generator=g).bfloat16().to(DEV)
@@ -40,5 +44,6 @@ def test_strided_queries_give_the_same_gradients(qfa):
     res = []
     for q in (q0, q0.contiguous()):
         leaves = [q.detach().requires_grad_(True), kv.detach().requires_grad_(True)]
+        assert leaves[0].is_contiguous() == (q is not q0)
         res.append(torch.autograd.grad(qfa.quant_flash_attn(leaves[0], leaves[1], quant, sm), leaves, do))
     assert all(torch.equal(a, b) for a, b in zip(*res))

@@ -11,29 +11,48 @@ import torch
 
 from helpers import COS_TOL, assert_close, max_abs
 from oracle import oracle
+from plans import skv_tile_dq_plan, skv_tile_fwd_plan
+from quant_flash_attn_amd import _lib
 
 DEV = "cuda:0"
 
+# the kernels that forward and backward (dQ) of a case are to reach, at head_dim 64, 128 and 256
+TILES = ["tiles, tiles"] * 3
 CASES = [
-    # heads, Nq, Nk, dtype, scale dtype
-    (512, 33, 1, torch.float16, torch.float16),      # one key
-    (512, 65, 31, torch.float16, torch.float32),     # three blocks on four waves, one key less than a block
-    (300, 200, 33, torch.bfloat16, torch.float16),   # two workgroups per head, four and three blocks
-    (256, 97, 65, torch.float16, torch.float16),     # one key more than a tile; resident rows, the last block one query
-    (256, 128, 129, torch.float16, torch.float16),   # all resident rows, one key more than four waves' tiles
-    (256, 129, 128, torch.bfloat16, torch.float32),  # one query more than the resident rows
-    (64, 512, 97, torch.float16, torch.float16),
-    (600, 64, 70, torch.float16, torch.bfloat16),
-    (600, 32, 70, torch.float16, torch.float16),     # one-pass backward, not split
-    (3, 16, 3001, torch.float16, torch.float16),     # one-pass backward, split
-    (2, 31, 2500, torch.bfloat16, torch.float32),
-    (1, 200, 9001, torch.float16, torch.float16),    # forward and dQ split
+    # heads, Nq, Nk, dtype, scale dtype, kernels
+    (512, 33, 1, torch.float16, torch.float16, ["tiles, tiles", "tiles, 16 queries", "tiles, 16 queries"]),   # one key
+    (512, 65, 31, torch.float16, torch.float32, TILES),     # three blocks on four waves, one key less than a block
+    (300, 200, 33, torch.bfloat16, torch.float16, TILES),   # two workgroups per head, four and three blocks
+    (256, 97, 65, torch.float16, torch.float16, TILES),     # one key more than a tile; resident rows, the last block one query
+    (256, 128, 129, torch.float16, torch.float16, TILES),   # all resident rows, one key more than four waves' tiles
+    (256, 129, 128, torch.bfloat16, torch.float32, TILES),  # one query more than the resident rows
+    (64, 512, 97, torch.float16, torch.float16, TILES),
+    (600, 64, 70, torch.float16, torch.bfloat16, TILES),
+    (24, 200, 2001, torch.float16, torch.float16, ["tiles split, 16 queries"] * 3),
+    (32, 65, 3001, torch.bfloat16, torch.float16, ["tiles split, tiles split", "tiles split, 16 queries", "16 queries split, 16 queries"]),
+    (600, 32, 70, torch.float16, torch.float16, ["16 queries, one pass"] * 2 + ["16 queries, 16 queries"]),
+    (3, 16, 3001, torch.float16, torch.float16, ["16 queries split, one pass split"] * 3),
+    (2, 31, 2500, torch.bfloat16, torch.float32, ["16 queries split, one pass split"] * 2 + ["16 queries split, tiles split"]),
+    (1, 200, 9001, torch.float16, torch.float16, ["16 queries split, tiles split"] * 3),
 ]
+
+
+def _kernels(BH, Nq, Nk, D):
+    L, fwd, dq = _lib.lib(), skv_tile_fwd_plan(BH, Nq, Nk, D), skv_tile_dq_plan(BH, Nq, Nk, D)
+    parts = [f(1, BH, Nq, Nk, D) for f in (L.qfa_attn_fwd_shared_kv_workspace_bytes, L.qfa_attn_bwd_shared_kv_workspace_bytes)]
+    names = ["tiles" if fwd.waves else "16 queries",
+             "one pass" if Nq <= (16 if D == 256 else 32) else "tiles" if dq.waves else "16 queries"]
+    return ", ".join(n + (" split" if p else "") for n, p in zip(names, parts))
+
+
+def test_cases_reach_the_kernels_they_name(qfa):
+    for BH, Nq, Nk, _, _, kernels in CASES:
+        assert [_kernels(BH, Nq, Nk, D) for D in (64, 128, 256)] == kernels, (BH, Nq, Nk)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128, 256])
-@pytest.mark.parametrize("BH,Nq,Nk,dtype,sdtype", CASES)
+@pytest.mark.parametrize("BH,Nq,Nk,dtype,sdtype", [c[:5] for c in CASES])
 def test_tiles_vs_oracle(qfa, BH, Nq, Nk, dtype, sdtype, D):
     g = torch.Generator().manual_seed(BH + Nq + Nk + D)
     kv = (torch.randn((1, BH, Nk, D), generator=g) + 0.3 * torch.randn((1, BH, Nk, 1), generator=g)).to(dtype)
@@ -100,7 +119,6 @@ def test_softmax_scales(qfa, sm):
 
 def test_backward_workspace_is_bounded(qfa):
     """Partial results of a split stay within 64 MiB, and a chip that is full is not split (head_dim up to 128)."""
-    from quant_flash_attn_amd import _lib
     L, rng = _lib.lib(), random.Random(2)
     for _ in range(20000):
         B, H, Nq, Nk = rng.randint(1, 64), rng.randint(1, 64), rng.choice((1, 16, 17, 32, 33, 512, 2000)), rng.randint(1, 40000)
