@@ -20,16 +20,17 @@ DEV = "cuda:0"
 TILES = ["tiles, tiles"] * 3
 CASES = [
     # heads, Nq, Nk, dtype, scale dtype, kernels
-    (512, 33, 1, torch.float16, torch.float16, ["tiles, tiles", "tiles, 16 queries", "tiles, 16 queries"]),   # one key
+    (512, 33, 1, torch.float16, torch.float16, ["16 queries, tiles", "tiles, 16 queries", "16 queries, 16 queries"]),   # one key
+    (512, 65, 1, torch.float16, torch.float16, TILES),
     (512, 65, 31, torch.float16, torch.float32, TILES),     # three blocks on four waves, one key less than a block
     (300, 200, 33, torch.bfloat16, torch.float16, TILES),   # two workgroups per head, four and three blocks
     (256, 97, 65, torch.float16, torch.float16, TILES),     # one key more than a tile; resident rows, the last block one query
     (256, 128, 129, torch.float16, torch.float16, TILES),   # all resident rows, one key more than four waves' tiles
     (256, 129, 128, torch.bfloat16, torch.float32, TILES),  # one query more than the resident rows
     (64, 512, 97, torch.float16, torch.float16, TILES),
-    (600, 64, 70, torch.float16, torch.bfloat16, TILES),
-    (24, 200, 2001, torch.float16, torch.float16, ["tiles split, 16 queries"] * 3),
-    (32, 65, 3001, torch.bfloat16, torch.float16, ["tiles split, tiles split", "tiles split, 16 queries", "16 queries split, 16 queries"]),
+    (600, 64, 70, torch.float16, torch.bfloat16, TILES[:2] + ["16 queries, 16 queries"]),
+    (40, 100, 2001, torch.float16, torch.float16, ["tiles split, 16 queries"] * 3),
+    (40, 65, 5001, torch.bfloat16, torch.float16, ["tiles split, tiles split"] * 2 + ["tiles split, 16 queries"]),
     (600, 32, 70, torch.float16, torch.float16, ["16 queries, one pass"] * 2 + ["16 queries, 16 queries"]),
     (3, 16, 3001, torch.float16, torch.float16, ["16 queries split, one pass split"] * 3),
     (2, 31, 2500, torch.bfloat16, torch.float32, ["16 queries split, one pass split"] * 2 + ["16 queries split, tiles split"]),

@@ -1,0 +1,32 @@
+"""Which shared-KV kernel the plan takes where the workgroups of whole heads do not fill the XCDs evenly, or where a workgroup has
+few tiles: launches measured with every kernel (us on an MI355X; 16 queries per workgroup, two and four waves side by side on
+tiles).  The choice may not cost more than a twentieth over the 16-query kernel."""
+import pytest
+
+from plans import skv_tile_dq_plan, skv_tile_fwd_plan
+
+FORWARD = [
+    # heads, Nq, Nk, D, {kernel: us}
+    (81, 173, 513, 256, {0: 32.0, 2: 45.9, 4: 31.2}),    # 33 workgroups on one XCD of 32 CUs with two waves
+    (85, 155, 2474, 256, {0: 91.1, 2: 135.7}),
+    (1820, 34, 345, 256, {0: 109.2, 2: 139.2}),
+    (1207, 137, 612, 256, {0: 318.4, 2: 353.5, 4: 333.3}),
+    (430, 42, 1109, 256, {0: 70.1, 2: 77.0}),
+    (18, 465, 132, 128, {0: 8.2, 2: 9.8, 4: 10.1}),
+    (555, 48, 380, 128, {0: 21.7, 2: 24.7}),
+    (1552, 32, 80, 128, {0: 23.6, 2: 27.5}),
+    (57, 188, 178, 128, {0: 9.1, 2: 10.2, 4: 10.0}),
+    (265, 47, 96, 64, {0: 6.0, 2: 7.7}),
+    (158, 65, 257, 64, {0: 8.7, 2: 11.2, 4: 9.7}),
+    (330, 35, 134, 64, {0: 7.0, 2: 8.9}),
+    (88, 150, 708, 64, {0: 13.2, 2: 16.2, 4: 16.3}),
+    (317, 39, 685, 64, {0: 13.1, 2: 16.0}),
+    (161, 85, 1550, 64, {0: 25.1, 2: 30.0, 4: 28.9}),
+]
+DQ = [(84, 347, 546, 256, {0: 175.0, 4: 195.6})]   # (the whole backward)
+
+
+@pytest.mark.parametrize("plan,BH,Nq,Nk,D,us", [(skv_tile_fwd_plan, *c) for c in FORWARD] + [(skv_tile_dq_plan, *c) for c in DQ])
+def test_choice_is_not_slower(qfa, plan, BH, Nq, Nk, D, us):
+    p = plan(BH, Nq, Nk, D)
+    assert p.splits == 1 and us.get(p.waves, float("inf")) <= 1.05 * us[0], (p.waves, p.splits)
