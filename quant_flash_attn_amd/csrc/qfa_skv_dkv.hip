@@ -84,9 +84,14 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
     const int c = tid % TPR + TPR * k;
     return *reinterpret_cast<const u32x4 *>(smem + GM::MAT + c / 2 * SLAB + ra * 32 + (((c % 2) ^ (ra >> 3 & 1)) << 4));
   };
+  auto set_stat = [&](int r0, int ra, float delta, float lse) __attribute__((always_inline)) {
+    if (tid % TPR != 0) return;
+    const bool live = r0 + tid / TPR < a.Nq;
+    stat[ra] = live ? -lse * kLog2e : -INFINITY;   // padding rows: p = 0
+    stat[GM::ROWS + ra] = live ? -a.sm_scale * delta : 0.f;
+  };
   auto stats = [&](int r0, int a0, const u32x4 (&of)[OC], float lse) __attribute__((always_inline)) {
-    const int rr = tid / TPR, ra = a0 + rr;
-    const bool live = r0 + rr < a.Nq;
+    const int ra = a0 + tid / TPR;
     float sum = 0.f;
 #pragma unroll
     for (int k = 0; k < OC; ++k) {
@@ -99,10 +104,7 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
     }
 #pragma unroll
     for (int m = 1; m < TPR; m *= 2) sum += __shfl_xor(sum, m, 64);
-    if (tid % TPR == 0) {
-      stat[ra] = live ? -lse * kLog2e : -INFINITY;   // padding rows: p = 0
-      stat[GM::ROWS + ra] = live ? -a.sm_scale * sum : 0.f;
-    }
+    set_stat(r0, ra, sum, lse);
   };
 
   // ---- a tile of 32 keys: codes on their way (raw), then as B operands (column = key lr; k-steps 2j, 2j + 1 and k-group g
@@ -269,17 +271,17 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
 #pragma unroll
         for (int i = 0; i < OC; ++i) of[i] = half_of_bf16(of[i]);
       }
-      float md = 0.f;
-      if (a.wgs_per_bh > 1) {   // O comes from all keys of the head, the scales from a part of them
-        u32x4 dr[OC];
+      // delta of the rows as they came: times 2^k it is that of the scaled ones, and what bounds k where O comes from all keys
+      // of the head and the scales from a part of them
+      u32x4 dr[OC];
 #pragma unroll
-        for (int i = 0; i < OC; ++i) dr[i] = dout_of(tid / TPR, i);
-        md = dot_dout(of, dr, a.do_bf16);
+      for (int i = 0; i < OC; ++i) dr[i] = dout_of(tid / TPR, i);
+      float delta = dot_dout(of, dr, a.do_bf16);
 #pragma unroll
-        for (int m = 1; m < TPR; m *= 2) md += __shfl_xor(md, m, 64);
-        md = tid / TPR < a.Nq ? finite_abs(a.sm_scale * md) : 0.f;
-      }
+      for (int m = 1; m < TPR; m *= 2) delta += __shfl_xor(delta, m, 64);
+      const float md = a.wgs_per_bh > 1 && tid / TPR < a.Nq ? finite_abs(a.sm_scale * delta) : 0.f;
       const int k = block_dout_exponent(max_abs_dout(w, a.do_bf16), scales.get(), md, red);
+      set_stat(0, tid / TPR, delta * exp2_neg(-k), lse);
       scale_dout(w, a.do_bf16, k);
       osc = exp2_neg(k);
       if (live) {
@@ -293,9 +295,9 @@ template <int D, bool KEEP> __global__ __launch_bounds__(256, D == 256 ? 1 : D =
           }
         }
       }
-      __syncthreads();
+    } else {
+      stats(0, 0, of, lse);
     }
-    stats(0, 0, of, lse);
     __syncthreads();
     for (; t < t_end; t += 4) {
       expand_tile();
