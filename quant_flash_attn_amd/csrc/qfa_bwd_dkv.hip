@@ -450,12 +450,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
 
 template <typename T, int D, int KB> static int launch_dkv_kb(BwdArgs a, int64_t BH, bool causal, int splits, hipStream_t st) {
   a.nblocks = (a.Nk + 128 * KB - 1) / (128 * KB);
-  // per head the kernel streams Qc, dO and Qz^T (5 bytes per query and d): group heads while that stays
-  // within about 6 MB (pairs at N=4096, D=128: 5.2 MB against the XCD's 4 MB L2, measured 1 % better than
-  // single heads; four heads are not)
-  const int64_t head_bytes = (int64_t)a.Nq * D * 5;
-  a.group_log2 = 0;
-  while (a.group_log2 < 2 && (head_bytes << (a.group_log2 + 1)) <= (6 << 20)) ++a.group_log2;
+  a.group_log2 = bwd_group_log2(a.Nq, D, false);   // per head the kernel streams Qc, dO and Qz^T: 5 bytes per query and d
   const int64_t total = (int64_t)a.nblocks * BH;
   if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many key blocks for one launch");
   a.total_blocks = (int)total;

@@ -370,11 +370,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
 
 template <typename T, int D, int QB> static int launch_dq_qb(BwdArgs a, int64_t BH, bool causal, int splits, hipStream_t st) {
   a.nblocks = (a.Nq + 128 * QB - 1) / (128 * QB);
-  // per head the kernel streams Kc, V and Kz^T (5 bytes per key and d): two to eight heads together, within
-  // about 6 MB (pairs at N=4096, D=128, measured)
-  const int64_t head_bytes = (int64_t)a.Nk * D * 5;
-  a.group_log2 = 1;
-  while (a.group_log2 < 3 && (head_bytes << (a.group_log2 + 1)) <= (6 << 20)) ++a.group_log2;
+  a.group_log2 = bwd_group_log2(a.Nk, D, true);   // per head the kernel streams Kc, V and Kz^T: 5 bytes per key and d
   const int64_t total = (int64_t)a.nblocks * BH;
   if (total > 0x3fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many query blocks for one launch");
   a.total_blocks = (int)total;

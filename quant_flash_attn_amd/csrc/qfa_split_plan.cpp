@@ -8,7 +8,8 @@
 // 2600 (forward) and 1000 (backward) shapes of 1 to 512 heads, 17 to 16384 queries, 64 to 30000 keys, causal or not, each timed
 // with every division.  Over these shapes the forward takes 1.01 times the best division's time in the geometric mean where the
 // undivided one takes 1.9 times, dK / dV 1.01 against 1.045, dQ 1.004 against 1.11 (both of the whole backward).  Small gains
-// are left, being within the model's error: no shape got slower by more than 4 %.
+// are left, being within the model's error: of 1500 more backwards that are divided (0.63 times the undivided time in the geometric
+// mean) three take more than 1.06 times, 1.12 at most; forwards up to 1.04.
 #include <algorithm>
 #include <cmath>
 
@@ -31,10 +32,15 @@ constexpr int64_t MAX_WGS = 1700, MAX_WGS_BWD = 1100;   // of a divided launch: 
 constexpr int64_t MAX_PART_FLOATS = QFA_SPLIT_PART_BYTES / 4;
 
 // `blocks` workgroups of `rows` rows each for each of `heads` heads, the streamed rows in tiles of `tile` (64 or 32), s parts of
-// `each` rows; ends: block i sees streamed rows up to (i + 1) * rows + coff, otherwise from i * rows - coff on
+// `each` rows; ends: block i sees streamed rows up to (i + 1) * rows + coff, otherwise from i * rows - coff on.
+// group_log2: how the backward's launches deal their blocks (-1: the forward's): every XCD takes an eighth of the blocks in a row
+// with all their parts, causal those of 2^group_log2 heads in turn from the longest block on.  The first XCD then has most to
+// do, and 255 workgroups of 85 blocks are 33 on its 32 CUs (5 heads, 4270 x 4270 of 128: counted evenly they were one round, and
+// 259 us took the place of 218).
 struct SplitWork {
   int64_t heads, blocks, rows, streamed, tile, coff;
   bool causal, ends;
+  int group_log2 = -1;
   double total = 0, longest = 0;   // tiles of a head, of its longest block
   int64_t seen(int64_t i) const {
     if (!causal) return streamed;
@@ -52,13 +58,41 @@ struct SplitWork {
       longest = std::max(longest, n);
     }
   }
+  // workgroups of the first XCD that have something to do, and their tiles
+  void first_xcd(int64_t s, int64_t each, double *live, double *tiles) const {
+    const int64_t ids = (heads * blocks + 7) / 8;
+    if (!causal) {
+      *live = (double)(ids * s);
+      *tiles = (double)ids * longest;
+      return;
+    }
+    const int64_t group = std::min<int64_t>(heads, (int64_t)1 << group_log2);
+    int64_t n = 0, t = 0;
+    for (int64_t at = 0; at < ids;) {
+      const int64_t i = at / group % blocks, seen_rows = seen(ends ? blocks - 1 - i : i), many = std::min(group, ids - at);
+      n += many * std::min<int64_t>(s, (int)(seen_rows + each - 1) / (int)each);
+      t += many * ((seen_rows + tile - 1) / tile);
+      at += many;
+    }
+    *live = (double)n;
+    *tiles = (double)t;
+  }
   double time(const SplitCost &c, int64_t s, int64_t each, double mbytes) const {
     const double per = (double)(each / tile);
-    double wgs = (double)(blocks * s);
-    if (causal) wgs = std::min(wgs, total / per + 0.5 * (double)blocks);   // the others have nothing to do
-    const double n = wgs * (double)heads, slots = 256.0 * c.resident, last = std::min(longest, per) + c.start;
+    double n, all;   // workgroups with something to do and their tiles, of the chip
+    if (group_log2 < 0) {
+      n = (double)(blocks * s);
+      if (causal) n = std::min(n, total / per + 0.5 * (double)blocks);   // the others have nothing to do
+      n *= (double)heads;
+      all = total * (double)heads;
+    } else {
+      first_xcd(s, each, &n, &all);
+      n *= 8.0;
+      all *= 8.0;
+    }
+    const double slots = 256.0 * c.resident, last = std::min(longest, per) + c.start;
     const double body = n <= slots ? last * c.tile[std::min(c.resident, (int)std::ceil(n / 256.0)) - 1]
-                                   : ((total * (double)heads + n * c.start) / slots + c.tail * last) * c.tile[c.resident - 1];
+                                   : ((all + n * c.start) / slots + c.tail * last) * c.tile[c.resident - 1];
     return c.base + body + (s > 1 ? c.merge + c.mb * mbytes : 0.0);
   }
 };
@@ -125,16 +159,20 @@ static void bwd_part(int64_t BH, int64_t rows, int64_t streamed, int D, bool cau
   if (D == 128 && undivided_cost(BH, rows, streamed, causal, f, 1, 0.62f) >= undivided_cost(BH, rows, streamed, causal, f, 2, 1.0f)) rb = 2;
   int64_t s = 1, each = (streamed + 63) / 64 * 64;
   *blocks = rb;
+  const int group_log2 = bwd_group_log2(streamed, D, ends);
   if (may_split && BH <= MAX_WGS_BWD && rows <= 128 * MAX_WGS_BWD) {
     SplitWork w[2];
     for (int r = 1; r <= (D == 128 ? 2 : 1); ++r) {
-      w[r - 1] = {BH, (rows + 128 * r - 1) / (128 * r), 128 * r, streamed, 32, coff, causal, ends};
+      w[r - 1] = {BH, (rows + 128 * r - 1) / (128 * r), 128 * r, streamed, 32, coff, causal, ends, group_log2};
       if (2 * BH * w[r - 1].blocks <= MAX_WGS_BWD || r == rb) w[r - 1].count();
     }
-    double best = 0.93 * w[rb - 1].time(c[rb - 1], 1, each, 0);
+    const double undivided = w[rb - 1].time(c[rb - 1], 1, each, 0);
+    double best = 0;
     for (int r = 1; r <= (D == 128 ? 2 : 1); ++r) {
       const SplitWork &x = w[r - 1];
       const int64_t was = s;
+      // (with another number of rows per wave a division has to promise more: 12 heads of 4037, causal, promised 0.915, took 1.11)
+      if (was == 1) best = (r == rb ? 0.93 : 0.9) * undivided;
       s = 1;
       best_division(streamed, std::min<int64_t>({32, MAX_WGS_BWD / (BH * x.blocks), MAX_PART_FLOATS / (BH * rows * D * tensors)}), best, &s, &each, [&](int64_t n, int64_t e) {
         return x.time(c[r - 1], n, e, 8e-6 * (double)(BH * rows * n) * D * tensors);
