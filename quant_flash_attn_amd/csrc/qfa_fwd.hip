@@ -99,7 +99,10 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   int bh = vid / a.mblocks;
   int mb = vid % a.mblocks;
   int split = 0, key0 = 0;
-  if (SPLIT) {   // (all of them are resident at once: any order will do)
+  // The parts are nearly equally long, so ids run over them as they come, also where a launch is more than one round (up to 1700
+  // workgroups; 768, 512, 256 are resident at head_dim 64, 128, 256).  From the longest query block down, causal: 12 heads
+  // of 6000 x 64 112 -> 100 us, but 4 of 12000 x 128 191 -> 217, 3 of 16000 x 256 537 -> 627 and nine others -2 to +20 %.
+  if (SPLIT) {
     split = bh % a.splits;
     bh /= a.splits;
     key0 = split * a.keys_per_split;

@@ -10,9 +10,12 @@
 //   cycle   longer query blocks: a workgroup takes 128 keys, blocks of 64 queries alternate between the halves of the row
 //           area, two barriers per 64 queries.
 // The kernel before it copied and summed the rows once per 128 keys, met at two barriers per 32 queries (52 % of its time was
-// waiting) and removed the codes' offset by two more MFMAs per block.  5247 heads, 97 queries, 689 keys of 128: 966 -> 640 us;
-// 512 heads, 512 queries, 4096 keys of 128: 1567 -> 1200.  Matrix pipe busy 44 % at 1.9 GHz; the S and dP of the next block
-// beside the vector work of this one (32 registers more) changed neither.
+// waiting) and removed the codes' offset by two more MFMAs per block.  Measured, that one -> this (us, one GPU): 5247 heads, 97 x 689
+// 941 -> 668 at head_dim 128, 497 -> 327 at 64; 512 heads, 512 x 4096 1565 -> 1180 and 842 -> 599.  Up to 64 queries it had its rows
+// resident too and was 7 to 9 % faster at 128 (1470 heads, 47 x 2737: 532 against 572).
+// What bounds it: at 512 queries the matrix pipe is busy 45 % at 1.89 GHz, issue stalls 37 %; the S and dP of the next block
+// beside the vector work of this one (32 registers more) changed nothing.  At 97 x 689 it is busy 33 % with 41 % waits: 16 KB
+// of rows and 16 KB transposed out of LDS for 32 products, and the last block of 32 queries holds one.
 #include "qfa_host.h"
 #include "qfa_skv_common.h"
 

@@ -13,13 +13,16 @@
 // two (64 queries) share the keys of a tile with the other two and their partial results meet in LDS.  With few workgroups the
 // keys are split over several of them (qfa_skv_plan.cpp).  The codes of the tile after the next are on their way in registers
 // while a tile is worked on.  The forward makes the scores of the next block beside the probabilities of this one (three
-// tiles in LDS); the same pipeline in dQ costs 35 KB more LDS and gained nothing (head_dim 128: 384 against 421 us).
+// tiles in LDS); the same pipeline in dQ costs 35 KB more LDS and gained nothing (head_dim 128, before the scaling moved in: 384
+// against 421 us).
 //
-// What bounds them: the forward's matrix pipe is busy 50 % and its vector pipe 57 % of the time at 1.76 GHz, 44 % of the LDS
-// cycles are used, and one workgroup per CU already reaches nine tenths of what two do: power and issue, not latency.
-// Measured, 16-query kernels -> these (us): 5247 heads, 97 queries, 689 keys: forward 561 -> 330, dQ 700 -> 384 at head_dim
-// 128, forward 335 -> 189 at 64; 512 heads, 512 queries, 4096 keys: 1054 -> 575 (128), 667 -> 350 (64); 256 heads of 256:
-// 982 -> 745.
+// What bounds them.  Long blocks (512 heads, 512 queries, 4096 keys of 128): the forward's matrix pipe is busy 47 % and its vector
+// pipe 54 % of the time at 1.86 GHz, 42 % of the LDS cycles are used, dQ 47, 49 and 28 %; one workgroup per CU already reaches
+// nine tenths of what two do: power and issue, not latency.  Short ones (5247 heads, 97 queries, 689 keys): matrix pipe 39 and 38 %,
+// waits 27 and 36 %: eleven tiles between a workgroup's start and end, and the fourth block of 32 queries holds one.
+// Measured, 16-query kernels -> these (us, one GPU): 5247 heads, 97 x 689: forward 538 -> 298, dQ with the scaling of dO 679 -> 439
+// at head_dim 128, 333 -> 186 and 420 -> 248 at 64; 512 heads, 512 x 4096: 1069 -> 566 and 1141 -> 831 (128), 670 -> 349 and 732 ->
+// 476 (64); 256 heads of 256: forward 997 -> 771 (dQ stays with the 16-query kernel).
 #include <type_traits>
 
 #include "qfa_host.h"
@@ -436,9 +439,9 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   {
     u32x4 of[KD];
     skv_load_row<D>(a.o, b * a.sob + h * a.soh + (int64_t)qi_c * a.son, a.io_bf16, g, of);
-    // A power of two of the workgroup's own queries, their delta and its keys.  The reduction in front of the first tile costs this kernel a
-    // little (99 x 53 heads, 97 x 689, fp16: 442 -> 456 us, dKV 670 -> 690), but it takes the place of two launches, more in bf16:
-    // the call 1480 -> 1417 and 1519 -> 1426 us; 14 heads, 100 x 1872 (bound by launches): 84 -> 54 to 76.
+    // A power of two of the workgroup's own queries, their delta and its keys.  The reduction in front of the first tile costs this
+    // kernel a little (99 x 53 heads, 97 x 689, fp16, when it moved in: 442 -> 456 us), but it takes the place of two launches, more
+    // in bf16: the call 1480 -> 1417 and 1519 -> 1426 us; 14 heads, 100 x 1872 (bound by launches): 84 -> 54 to 76.
     if (a.direct) {
       __shared__ float red[12];
       float md = 0.f;

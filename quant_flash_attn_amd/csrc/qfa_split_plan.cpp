@@ -27,8 +27,8 @@ struct SplitCost {
 
 constexpr int64_t MAX_WGS = 1700, MAX_WGS_BWD = 1100;   // of a divided launch: as far as was measured
 // Of the parts of one launch: what MAX_WGS leaves of the forward (214 MiB, long sequences of few wide heads; 192 MiB cost 3 heads,
-// 22757 x 22757 of 256, causal, 1019 -> 1474 us), and less than dK and dV could fill (275 MiB).  Between 1.03 times faster and slower where it bites there
-// (5 heads of 17926 of 128, forward and backward: 3168 -> 3077 us; 5 of 24880, causal: 3680 -> 3765).
+// 22757 x 22757 of 256, causal, 1019 -> 1474 us), and less than dK and dV could fill (275 MiB).  Between 1.03 times faster and slower
+// where it bites there (5 heads of 17926 of 128, forward and backward: 3168 -> 3077 us; 5 of 24880, causal: 3680 -> 3765).
 constexpr int64_t MAX_PART_FLOATS = QFA_SPLIT_PART_BYTES / 4;
 
 // `blocks` workgroups of `rows` rows each for each of `heads` heads, the streamed rows in tiles of `tile` (64 or 32), s parts of
@@ -174,7 +174,8 @@ static void bwd_part(int64_t BH, int64_t rows, int64_t streamed, int D, bool cau
       // (with another number of rows per wave a division has to promise more: 12 heads of 4037, causal, promised 0.915, took 1.11)
       if (was == 1) best = (r == rb ? 0.93 : 0.9) * undivided;
       s = 1;
-      best_division(streamed, std::min<int64_t>({32, MAX_WGS_BWD / (BH * x.blocks), MAX_PART_FLOATS / (BH * rows * D * tensors)}), best, &s, &each, [&](int64_t n, int64_t e) {
+      const int64_t most = std::min<int64_t>({32, MAX_WGS_BWD / (BH * x.blocks), MAX_PART_FLOATS / (BH * rows * D * tensors)});
+      best_division(streamed, most, best, &s, &each, [&](int64_t n, int64_t e) {
         return x.time(c[r - 1], n, e, 8e-6 * (double)(BH * rows * n) * D * tensors);
       });
       if (s > 1) {

@@ -458,7 +458,7 @@ Kept qkv_forward(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, boo
   if (all_f32(q, k, v_in) && (pb.D == 64 || pb.D == 128 || pb.D == 256)) {
     // fp32 in and out without launches of their own for the conversions: the quantizer's launch takes V along, the forward
     // writes O in both types, the staging pass rounds dO, and the gradients leave in fp32 (B1 H4 N256 D64, forward and backward:
-    // 5 launches instead of 11, 105 -> 45 us)
+    // 5 launches instead of 11, 103 -> 75 us, of which the kernels are 37)
     const Tensor v = rows16(v_in);
     const Quantized a = pb.view(r.buf, 0), b = pb.view(r.buf, 1);
     auto w = [](auto *p) { return const_cast<std::remove_const_t<std::remove_pointer_t<decltype(p)>> *>(p); };
@@ -582,8 +582,8 @@ int64_t cache_max_q(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
 // to 512 queries, 300 to 20000 keys (within 8 % in the mean): the short one takes what its memory or its blocks of 16 queries
 // take, and loses by a last round of workgroups that is not full; the other one the pass over the cache and blocks of 128
 // queries.  Calls are taken from the other path where that should gain 12 %: over all shapes the choice costs 0.4 - 1 % against
-// the better path each time, where the line alone cost 3 - 6 %; the moved calls gain 1.4 times in the mean.  920 of them timed on both once more: 1.6 times, three
-// lost more than 3 % (7 heads, 149 queries, 19668 keys of 256: 4.6 %).
+// the better path each time, where the line alone cost 3 - 6 %; the moved calls gain 1.4 times in the mean.  920 of them timed on
+// both once more: 1.6 times, three lost more than 3 % (7 heads, 149 queries, 19668 keys of 256: 4.6 %).
 bool cache_short_cheaper(int64_t BH, int64_t Nq, int64_t Nk, int64_t D) {
   struct Cost { double s0, s_byte, s_block, s_start, s_fill, l0, l_byte, l_block, l_idle, l_query; };
   static const Cost c64 = {9.8, 0.48, 11.4, 2.0, 0.37, 18.6, 0.84, 33.7, 0.1, 0.69}, c128 = {11.6, 0.56, 22.4, 6.1, 0.22, 20.4, 0.88, 51.9, 0.095, 0.42},
