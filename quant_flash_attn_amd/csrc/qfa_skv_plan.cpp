@@ -96,7 +96,15 @@ void skv_fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int 
   // 256 about four per CU (two are resident), or what split_plan finds better
   const int64_t wgs = BH * ((Nq + 15) / 16);
   const int64_t fill = D == 256 ? (wgs >= 512 ? 1 : (1024 + wgs - 1) / wgs) : 768 / wgs;
-  split_plan(wgs, BH * Nq, (Nk + 31) / 32, D, fill, splits, tiles_per_split);
+  const int64_t ntiles = (Nk + 31) / 32, rows = BH * Nq;
+  split_plan(wgs, rows, ntiles, D, fill, splits, tiles_per_split);
+  // Blocks of more than 16 queries that the tile kernels could take keep within the built-in scratch, as those do: which of the two
+  // is chosen does not decide whether a call without a workspace of its own is accepted
+  if (Nq > 16 && split_partial_bytes(rows, *splits, D) > QFA_STATIC_SCRATCH_BYTES) {
+    const int64_t most = std::max<int64_t>(1, QFA_STATIC_SCRATCH_BYTES / split_partial_bytes(rows, 1, D));
+    *tiles_per_split = (int)((ntiles + most - 1) / most);
+    *splits = (int)((ntiles + *tiles_per_split - 1) / *tiles_per_split);
+  }
 }
 
 SkvTilePlan skv_tile_fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {

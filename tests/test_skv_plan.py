@@ -1,9 +1,13 @@
 """Which shared-KV kernel the plan takes where the workgroups of whole heads do not fill the XCDs evenly, or where a workgroup has
 few tiles: launches measured with every kernel (us on an MI355X; 16 queries per workgroup, two and four waves side by side on
 tiles).  The choice may not cost more than a twentieth over the 16-query kernel."""
+import math
+import random
+
 import pytest
 
 from plans import skv_tile_dq_plan, skv_tile_fwd_plan
+from quant_flash_attn_amd import _lib
 
 FORWARD = [
     # heads, Nq, Nk, D, {kernel: us}
@@ -30,3 +34,13 @@ DQ = [(84, 347, 546, 256, {0: 175.0, 4: 195.6})]   # (the whole backward)
 def test_choice_is_not_slower(qfa, plan, BH, Nq, Nk, D, us):
     p = plan(BH, Nq, Nk, D)
     assert p.splits == 1 and us.get(p.waves, float("inf")) <= 1.05 * us[0], (p.waves, p.splits)
+
+
+def test_more_than_16_queries_fit_the_built_in_scratch(qfa):
+    """qfa_attn_fwd_shared_kv_static accepts every block of more than 16 queries, whichever kernel the plan takes."""
+    L, rng = _lib.lib(), random.Random(4)
+    log = lambda lo, hi: int(math.exp(rng.uniform(math.log(lo), math.log(hi))))
+    shapes = [(5, 537, 40160, 256), (83, 50, 10756, 256), (8, 144, 15338, 256)]   # (16 and 18 MB for the 16-query kernel's splits)
+    shapes += [(log(1, 1500), log(17, 1100), log(30, 60000), rng.choice((64, 128, 256))) for _ in range(40000)]
+    for BH, Nq, Nk, D in shapes:
+        assert 0 <= L.qfa_attn_fwd_shared_kv_workspace_bytes(1, BH, Nq, Nk, D) <= 16 << 20, (BH, Nq, Nk, D)
