@@ -85,7 +85,9 @@ class QuantFlashAttnQKV:
     q, k, v: [B,H,N,D] bf16 / fp16 / fp32 (fp32: V, dO and the O that the backward takes are rounded to bf16; where all three are
     fp32, O and the gradients are not).
     causal keeps key j for query i when j <= i (flash_attn_triton.py:50); with fewer queries than keys the mask is
-    aligned to the last key (j <= i + Nk - Nq)."""
+    aligned to the last key (j <= i + Nk - Nq).
+    With few (batch, head) pairs a head's keys (backward: streamed rows) are split over workgroups and their parts added in
+    fp32: the last bits of a head's results depend on B * H, not on the other heads' values, and repeat from call to call."""
 
     @staticmethod
     def apply(q, k, v, causal, sm_scale):
@@ -107,7 +109,7 @@ class QuantFlashAttnQuantizedKV:
     16-bit tensor that the P.V product streams: converting int8 V inside that kernel would add about 56 vector
     instructions per 32x32 block to a loop that issues 83 and is bound by them, the separate pass adds
     a read of the codes and one 16-bit write and read (8 % of the forward at B4 H32 N4096 D128).  With and without a
-    gradient the result is the same, bit for bit."""
+    gradient the result is the same, bit for bit; the keys are split as in QuantFlashAttnQKV."""
 
     @staticmethod
     def apply(q, k_fp16, v_fp16, k_quant, v_quant, causal, sm_scale):
@@ -124,7 +126,8 @@ class QuantFlashAttention:
 
     Positional contract of the reference (quant_flash_attn.py:178-237): kv_quant is the
     (codes, scale, zero_point) tuple returned by asymmetric_quant_per_token, kv_fp16 is only a
-    placeholder leaf that receives dkv, attention is non-causal, K == V == dequant(kv_quant)."""
+    placeholder leaf that receives dkv, attention is non-causal, K == V == dequant(kv_quant).  The keys are split as in
+    QuantFlashAttnQKV."""
 
     @staticmethod
     def apply(q, kv_fp16, kv_quant, sm_scale):
