@@ -43,7 +43,7 @@ def test_parts_are_bounded():
 @pytest.mark.parametrize("B,H,Nq,Nk,D,causal,dtype", [(1, 2, 8319, 8319, 256, True, torch.bfloat16), (1, 2, 8448, 8448, 256, False, torch.float32),
                                                       (2, 3, 6803, 6803, 128, True, torch.float16)])
 def test_parts_of_dq_in_the_place_of_the_others(qfa, B, H, Nq, Nk, D, causal, dtype):
-    """Parts of both beyond 64 MiB together: the gradients of the undivided call, and again on buffers that hold what the first
+    """Parts of both beyond 128 MiB together: the gradients of the undivided call, and again on buffers that hold what the first
     pass left."""
     plan = bwd_plan(B * H, Nq, Nk, D, causal)
     assert plan.sum_between and plan.splits_dkv > 1 and plan.splits_dq > 1 and plan.part_bytes == _parts(B, H, Nq, Nk, D, causal)
