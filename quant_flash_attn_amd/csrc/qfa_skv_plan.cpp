@@ -100,10 +100,11 @@ void skv_fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int 
   split_plan(wgs, rows, ntiles, D, fill, splits, tiles_per_split);
   // Blocks of more than 16 queries that the tile kernels could take keep within the built-in scratch, as those do: which of the two
   // is chosen does not decide whether a call without a workspace of its own is accepted
-  if (Nq > 16 && split_partial_bytes(rows, *splits, D) > QFA_STATIC_SCRATCH_BYTES) {
+  if (Nq > 16 && *splits > 1 && split_partial_bytes(rows, *splits, D) > QFA_STATIC_SCRATCH_BYTES) {
     const int64_t most = std::max<int64_t>(1, QFA_STATIC_SCRATCH_BYTES / split_partial_bytes(rows, 1, D));
-    *tiles_per_split = (int)((ntiles + most - 1) / most);
-    *splits = (int)((ntiles + *tiles_per_split - 1) / *tiles_per_split);
+    const int64_t each = (ntiles + most - 1) / most;
+    *tiles_per_split = (int)each;
+    *splits = (int)((ntiles + each - 1) / each);
   }
 }
 

@@ -44,3 +44,10 @@ def test_more_than_16_queries_fit_the_built_in_scratch(qfa):
     shapes += [(log(1, 1500), log(17, 1100), log(30, 60000), rng.choice((64, 128, 256))) for _ in range(40000)]
     for BH, Nq, Nk, D in shapes:
         assert 0 <= L.qfa_attn_fwd_shared_kv_workspace_bytes(1, BH, Nq, Nk, D) <= 16 << 20, (BH, Nq, Nk, D)
+
+
+@pytest.mark.parametrize("BH,Nq", [(1, 1 << 40), (5, 537), (1, 17), (1, 16)])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_sizes_beyond_any_memory_are_answered(qfa, BH, Nq, D):
+    """The size of a scratch can be asked for with any sizes: 2^40 keys are 2^35 tiles, a number that is 0 in 32 bits."""
+    assert 0 <= _lib.lib().qfa_attn_fwd_shared_kv_workspace_bytes(1, BH, Nq, 1 << 40, D)
