@@ -267,7 +267,7 @@ static int check_shared_kv(const char *who, const SkvAttnArgs &a) {
 
 int64_t qfa_attn_fwd_shared_kv_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
   if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0 || (D != 64 && D != 128 && D != 256)) return 0;
-  return skv_fwd_workspace_bytes(B, H, Nq, Nk, D);
+  return skv_fwd_plan(B * H, Nq, Nk, D).part_bytes;
 }
 
 int qfa_attn_fwd_shared_kv(const void *q, const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp,
@@ -282,14 +282,15 @@ int qfa_attn_fwd_shared_kv(const void *q, const int8_t *codes, const void *scale
   a.sqb = sqb; a.sqh = sqh; a.sqn = sqn; a.scb = scb; a.sch = sch; a.scn = scn; a.sob = sob; a.soh = soh; a.son = son;
   a.sm_scale = sm_scale;
   if (int e = check_shared_kv("attn_fwd_shared_kv", a)) return e;
+  const SkvFwdPlan plan = skv_fwd_plan(B * H, Nq, Nk, D);
   if (workspace) {
-    const int64_t need = skv_fwd_workspace_bytes(B, H, Nq, Nk, D);
+    const int64_t need = plan.part_bytes;
     if (!aligned16(workspace) || workspace_bytes < need)
       return set_error(QFA_EINVAL, "attn_fwd_shared_kv: workspace must be 16-byte aligned and hold %lld bytes "
                        "(qfa_attn_fwd_shared_kv_workspace_bytes), got %lld", (long long)need, (long long)workspace_bytes);
     a.workspace = need > 0 ? workspace : nullptr;
   }
-  return launch_skv_fwd(a, (hipStream_t)stream);
+  return launch_skv_fwd(a, plan, (hipStream_t)stream);
 }
 
 int qfa_attn_fwd_shared_kv_static(const void *q, const int8_t *codes, const void *scale, int scale_dtype,

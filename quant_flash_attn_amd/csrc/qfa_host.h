@@ -98,10 +98,6 @@ struct SkvAttnArgs {
   int grad_dtype; const float *grad_scale;   // backward only: type of dq / dkv, optional device scalar multiplying them
   int direct, dout_dtype;   // backward: q and o of io_dtype, dO of dout_dtype, cast and scaled inside (where skv_bwd_direct)
 };
-int launch_skv_fwd(const SkvAttnArgs &a, hipStream_t st);
-int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D);
-// the same with the partial results of a split in the library's own static device array (a.workspace is ignored)
-int launch_skv_fwd_static(const SkvAttnArgs &a, hipStream_t st);
 int launch_skv_bwd(const SkvAttnArgs &a, hipStream_t st);        // io_dtype QFA_F16, Nq <= 32: one fused pass
 // dO * 2^k as binary16 plus 2^-k for the binary16 backward kernels (k from max|dO| and the largest key scale);
 // partials: dout_normalise_workspace_bytes() of scratch
@@ -112,8 +108,13 @@ int launch_dout_normalise(const void *dout, int dout_dtype, int64_t n, const voi
 // Query blocks of more than 16: forward and dQ on tiles of 64 keys that a workgroup expands once.  qw: waves side by side on
 // the queries (0: not this kernel), splits: workgroups that share the keys, tiles of 64 keys each
 struct SkvTilePlan { int qw, splits, tiles; };
-void skv_fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split);   // 16 queries per workgroup
-SkvTilePlan skv_tile_fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D);
+// The forward: on tiles where tile.qw is not 0, otherwise 16 queries per workgroup and that many splits of 32-key tiles; the bytes
+// of the partial results.  An entry makes it once (up to 0.4 us, which calls of two small launches, 10 us in all, notice)
+struct SkvFwdPlan { SkvTilePlan tile; int splits, tiles_per_split; int64_t part_bytes; };
+SkvFwdPlan skv_fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D);
+int launch_skv_fwd(const SkvAttnArgs &a, const SkvFwdPlan &p, hipStream_t st);
+// the same with the partial results of a split in the library's own static device array (a.workspace is ignored)
+int launch_skv_fwd_static(const SkvAttnArgs &a, hipStream_t st);
 SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D);
 int launch_skv_tile_fwd(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t st);
 int launch_skv_tile_dq(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t st);

@@ -10,7 +10,7 @@
 // over its tiles from a private ring of LDS buffers filled by direct global->LDS loads (no
 // workgroup barrier in the loop), and the four partial results are merged at the end.  Longer query
 // blocks are split into several workgroups that run on the same XCD and share its L2 copy of the codes, as long as
-// there is little to do: with more work the tiles of qfa_skv_tile.hip take over (skv_tile_fwd_plan).
+// there is little to do: with more work the tiles of qfa_skv_tile.hip take over (skv_fwd_plan).
 //
 // Codes as MFMA operands.  A code byte c (two's complement) with its top bit flipped is the
 // unsigned byte c + 128; OR-ed under the constant 0x6400 it is the binary16 number 1152 + c
@@ -339,15 +339,7 @@ template <typename T, typename S, int D> __global__ __launch_bounds__(256, 2) vo
   }
 }
 
-int64_t skv_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
-  int splits, tps;
-  if (const SkvTilePlan p = skv_tile_fwd_plan(B * H, Nq, Nk, D); p.qw)
-    return p.splits > 1 ? split_partial_bytes(B * H * Nq, p.splits, D) : 0;
-  skv_fwd16_plan(B * H, Nq, Nk, D, &splits, &tps);
-  return splits > 1 ? split_partial_bytes(B * H * Nq, splits, D) : 0;
-}
-
-template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const SkvAttnArgs &x, hipStream_t st) {
+template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const SkvAttnArgs &x, const SkvFwdPlan &p, hipStream_t st) {
   SkvArgs a;
   a.q = x.q; a.codes = x.codes; a.scale = x.scale; a.zp = x.zp; a.o = x.o; a.lse = x.lse;
   a.H = x.H; a.Nq = (int)x.Nq; a.Nk = (int)x.Nk;
@@ -360,8 +352,9 @@ template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const Skv
   a.splits = 1;
   a.tiles_per_split = (int)((x.Nk + SKV_TILE - 1) / SKV_TILE);
   a.po = a.pml = nullptr;
-  if (x.workspace) {   // validated: large enough for the plan below
-    skv_fwd16_plan(x.B * x.H, x.Nq, x.Nk, D, &a.splits, &a.tiles_per_split);
+  if (x.workspace) {   // validated: large enough for the plan
+    a.splits = p.splits;
+    a.tiles_per_split = p.tiles_per_split;
     a.po = static_cast<float *>(x.workspace);
     a.pml = a.po + x.B * x.H * x.Nq * a.splits * (int64_t)D;
   }
@@ -377,11 +370,11 @@ template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const Skv
   return 0;
 }
 
-template <typename T, int D> static int launch_skv_fwd_td(const SkvAttnArgs &x, hipStream_t st) {
-  if (x.scale_dtype == QFA_F32) return launch_skv_fwd_tsd<T, float, D>(x, st);
+template <typename T, int D> static int launch_skv_fwd_td(const SkvAttnArgs &x, const SkvFwdPlan &p, hipStream_t st) {
+  if (x.scale_dtype == QFA_F32) return launch_skv_fwd_tsd<T, float, D>(x, p, st);
   // validated: the io type, or binary16
-  if (x.scale_dtype == QFA_F16) return launch_skv_fwd_tsd<T, _Float16, D>(x, st);
-  return launch_skv_fwd_tsd<T, T, D>(x, st);
+  if (x.scale_dtype == QFA_F16) return launch_skv_fwd_tsd<T, _Float16, D>(x, p, st);
+  return launch_skv_fwd_tsd<T, T, D>(x, p, st);
 }
 
 // ---- scratch for callers that cannot allocate --------------------------------------------------------
@@ -416,7 +409,8 @@ static int static_scratch(void **out) {
 }
 
 int launch_skv_fwd_static(const SkvAttnArgs &x, hipStream_t st) {
-  const int64_t need = skv_fwd_workspace_bytes(x.B, x.H, x.Nq, x.Nk, x.D);
+  const SkvFwdPlan plan = skv_fwd_plan(x.B * x.H, x.Nq, x.Nk, x.D);
+  const int64_t need = plan.part_bytes;
   if (need > (int64_t)QFA_STATIC_SCRATCH_BYTES)
     return set_error(QFA_EUNSUPPORTED,
                      "attn_fwd_shared_kv_static: this shape splits its keys into partial results of %lld bytes, more "
@@ -427,20 +421,19 @@ int launch_skv_fwd_static(const SkvAttnArgs &x, hipStream_t st) {
   if (need > 0) {   // every partial result is written by the first kernel before the merge reads it: nothing to clear
     if (int e = static_scratch(&y.workspace)) return e;
   }
-  return launch_skv_fwd(y, st);
+  return launch_skv_fwd(y, plan, st);
 }
 
-int launch_skv_fwd(const SkvAttnArgs &x, hipStream_t st) {
-  if (const SkvTilePlan p = skv_tile_fwd_plan(x.B * x.H, x.Nq, x.Nk, x.D); p.qw && (p.splits == 1 || x.workspace))
-    return launch_skv_tile_fwd(x, p, st);
+int launch_skv_fwd(const SkvAttnArgs &x, const SkvFwdPlan &p, hipStream_t st) {
+  if (p.tile.qw && (p.tile.splits == 1 || x.workspace)) return launch_skv_tile_fwd(x, p.tile, st);
   if (x.io_dtype == QFA_F16) {
-    if (x.D == 256) return launch_skv_fwd_td<_Float16, 256>(x, st);
-    if (x.D == 128) return launch_skv_fwd_td<_Float16, 128>(x, st);
-    if (x.D == 64) return launch_skv_fwd_td<_Float16, 64>(x, st);
+    if (x.D == 256) return launch_skv_fwd_td<_Float16, 256>(x, p, st);
+    if (x.D == 128) return launch_skv_fwd_td<_Float16, 128>(x, p, st);
+    if (x.D == 64) return launch_skv_fwd_td<_Float16, 64>(x, p, st);
   } else {
-    if (x.D == 256) return launch_skv_fwd_td<__bf16, 256>(x, st);
-    if (x.D == 128) return launch_skv_fwd_td<__bf16, 128>(x, st);
-    if (x.D == 64) return launch_skv_fwd_td<__bf16, 64>(x, st);
+    if (x.D == 256) return launch_skv_fwd_td<__bf16, 256>(x, p, st);
+    if (x.D == 128) return launch_skv_fwd_td<__bf16, 128>(x, p, st);
+    if (x.D == 64) return launch_skv_fwd_td<__bf16, 64>(x, p, st);
   }
   return set_error(QFA_EUNSUPPORTED, "attn_fwd_shared_kv: head_dim must be 64, 128 or 256");
 }

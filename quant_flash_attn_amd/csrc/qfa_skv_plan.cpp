@@ -54,13 +54,16 @@ const Cost kDqTile[2][3] = {
 
 const int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
 
-// the best split of `tiles` tiles for per_bh workgroups of each head; at least two tiles each, partial results of at most `room` floats
+// The best split of `tiles` tiles for per_bh workgroups of each head; at least two tiles each, partial results of at most `room` floats.
+// Only a cost below `limit` matters to the caller: no split is looked at where the merge and two tiles already take that long (most
+// small calls, whose 10 us this function is part of)
 void best_split(const Cost &c, Count how, int64_t BH, int64_t per_bh, int64_t rows, int64_t tiles, float per, int64_t row_floats,
-                int64_t room, int *splits, int64_t *tiles_each, float *cost) {
+                int64_t room, float limit, int *splits, int64_t *tiles_each, float *cost) {
   *splits = 1;
   *cost = 3e38f;
   for (const int s : kSplits) {
     if (s > 1 && (2 * s > tiles || BH * per_bh * s > 1600 || rows * s * row_floats > room)) break;
+    if (s > 1 && c.base + (c.alone * (per * 2.0f) + c.start) + c.merge >= limit) break;
     const int64_t each = (tiles + s - 1) / s, used = (tiles + each - 1) / each;
     const float t = c.of(count(how, BH, per_bh * used), per * (float)each, used, rows * used * row_floats);
     if (t < (s > 1 && *splits == 1 ? 0.9f : 1.0f) * *cost) {   // (a split has to promise a tenth)
@@ -71,7 +74,8 @@ void best_split(const Cost &c, Count how, int64_t BH, int64_t per_bh, int64_t ro
   }
 }
 // two or four waves side by side on the queries, the keys split
-SkvTilePlan best_tile(const Cost (*c)[3], Count how, int64_t BH, int64_t Nq, int64_t Nk, int D, int64_t row_floats, int64_t room, float *cost) {
+SkvTilePlan best_tile(const Cost (*c)[3], Count how, int64_t BH, int64_t Nq, int64_t Nk, int D, int64_t row_floats, int64_t room, float limit,
+                      float *cost) {
   const int64_t blocks = (Nq + 31) / 32, tiles = (Nk + 63) / 64;
   SkvTilePlan p = {2, 1, (int)tiles};
   *cost = 3e38f;
@@ -80,7 +84,7 @@ SkvTilePlan best_tile(const Cost (*c)[3], Count how, int64_t BH, int64_t Nq, int
     int splits = 1;
     int64_t each = tiles;
     float t;
-    best_split(c[i][by_dim(D)], how, BH, (blocks + qw - 1) / qw, BH * Nq, tiles, 1.0f, row_floats, room, &splits, &each, &t);
+    best_split(c[i][by_dim(D)], how, BH, (blocks + qw - 1) / qw, BH * Nq, tiles, 1.0f, row_floats, room, std::min(limit, *cost), &splits, &each, &t);
     if (t < *cost) {
       *cost = t;
       p = {qw, splits, (int)each};
@@ -89,9 +93,8 @@ SkvTilePlan best_tile(const Cost (*c)[3], Count how, int64_t BH, int64_t Nq, int
   return p;
 }
 
-}  // namespace
-
-void skv_fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
+// the 16-query kernel
+void fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int *tiles_per_split) {
   // as many workgroups as are resident at once (three per CU; a second, partly filled round costs a whole one), at head_dim
   // 256 about four per CU (two are resident), or what split_plan finds better
   const int64_t wgs = BH * ((Nq + 15) / 16);
@@ -108,34 +111,42 @@ void skv_fwd16_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int *splits, int 
   }
 }
 
-SkvTilePlan skv_tile_fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {
-  const SkvTilePlan none = {0, 1, 0};
-  if (Nq <= 16) return none;
-  // (partial results within the built-in scratch at every head_dim)
-  float t;
-  const SkvTilePlan p = best_tile(kFwdTile, Count::Xcd, BH, Nq, Nk, D, D + 2, QFA_STATIC_SCRATCH_BYTES / 4, &t);
-  int splits, each;
-  skv_fwd16_plan(BH, Nq, Nk, D, &splits, &each);
-  const float t16 = kFwd16[by_dim(D)].of(count(Count::Xcd, BH, (Nq + 15) / 16 * splits), 0.25f * (float)each, splits, BH * Nq * splits * (D + 2));
-  // (with 32 queries or fewer half of the waves have none)
-  return t < (Nq <= 32 ? 0.85f : 0.93f) * t16 ? p : none;
+}  // namespace
+
+SkvFwdPlan skv_fwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {
+  SkvFwdPlan f = {{0, 1, 0}, 1, 0, 0};
+  fwd16_plan(BH, Nq, Nk, D, &f.splits, &f.tiles_per_split);
+  if (Nq > 16) {
+    const float t16 = kFwd16[by_dim(D)].of(count(Count::Xcd, BH, (Nq + 15) / 16 * f.splits), 0.25f * (float)f.tiles_per_split, f.splits,
+                                           BH * Nq * f.splits * (D + 2));
+    // (with 32 queries or fewer half of the waves have none)
+    const float limit = (Nq <= 32 ? 0.85f : 0.93f) * t16;
+    // (partial results within the built-in scratch at every head_dim)
+    float t;
+    const SkvTilePlan p = best_tile(kFwdTile, Count::Xcd, BH, Nq, Nk, D, D + 2, QFA_STATIC_SCRATCH_BYTES / 4, limit, &t);
+    if (t < limit) f.tile = p;
+  }
+  const int parts = f.tile.qw ? f.tile.splits : f.splits;
+  f.part_bytes = parts > 1 ? split_partial_bytes(BH * Nq, parts, D) : 0;
+  return f;
 }
 
 SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   const Count how = D == 256 ? Count::Xcd : Count::Even;
-  float t;
-  const SkvTilePlan p = best_tile(kDqTile, how, BH, Nq, Nk, D, D, 16 << 20, &t);
   const float t16 = kDq16[by_dim(D)].of(count(how, BH, (Nq + 15) / 16), 0.25f * (float)((Nk + 31) / 32), 1, 0);
   // (33 to 48 queries leave a quarter of two waves' work to padding: 1024 heads, 48 queries, 3000 keys of 128 take 178 us with
   // the one kernel and 208 with the other)
-  return t < (Nq > 48 ? 0.93f : D == 256 ? 0.85f : 0.75f) * t16 ? p : SkvTilePlan{0, 1, 0};
+  const float limit = (Nq > 48 ? 0.93f : D == 256 ? 0.85f : 0.75f) * t16;
+  float t;
+  const SkvTilePlan p = best_tile(kDqTile, how, BH, Nq, Nk, D, D, 16 << 20, limit, &t);
+  return t < limit ? p : SkvTilePlan{0, 1, 0};
 }
 
 int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   int splits = 1;
   int64_t each;
   float t;
-  best_split(kPass[Nq <= 16 ? 0 : 1][by_dim(D)], Count::Even, BH, 1, BH * Nq, (Nk + 31) / 32, 0.25f, D, 16 << 20, &splits, &each, &t);
+  best_split(kPass[Nq <= 16 ? 0 : 1][by_dim(D)], Count::Even, BH, 1, BH * Nq, (Nk + 31) / 32, 0.25f, D, 16 << 20, 3e38f, &splits, &each, &t);
   return splits;
 }
 

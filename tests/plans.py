@@ -16,6 +16,10 @@ class SkvTilePlan(ctypes.Structure):
     _fields_ = [(n, _I) for n in ("waves", "splits", "tiles")]   # waves side by side; 0: the 16-query kernel
 
 
+class SkvFwdPlan(ctypes.Structure):
+    _fields_ = [("tile", SkvTilePlan), ("splits", _I), ("tiles_per_split", _I), ("part_bytes", _L)]
+
+
 def _plan(name, result, args):
     f = getattr(_lib.lib(), name)
     f.restype, f.argtypes = result, args
@@ -27,7 +31,7 @@ def bwd_plan(BH, Nq, Nk, D, causal, may_split=1):
 
 
 def skv_tile_fwd_plan(BH, Nq, Nk, D):
-    return _plan("_ZN3qfa17skv_tile_fwd_planEllli", SkvTilePlan, [_L, _L, _L, _I])(BH, Nq, Nk, D)
+    return _plan("_ZN3qfa12skv_fwd_planEllli", SkvFwdPlan, [_L, _L, _L, _I])(BH, Nq, Nk, D).tile
 
 
 def skv_tile_dq_plan(BH, Nq, Nk, D):
