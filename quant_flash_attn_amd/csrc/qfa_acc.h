@@ -89,6 +89,23 @@ template <typename T, int I, int F> __device__ __forceinline__ void acc_mfma_fra
 #undef QFA_M
 #endif
 }
+// Any registers: a[C : C+15] = (FIRST ? 0 : itself) + a[A : A+3] . b, A a constant operand that acc_request_const has put there
+template <int C, int A, bool FIRST> __device__ __forceinline__ void acc_mfma_const(u32x4 b) {
+  static_assert(C % 4 == 0 && A % 4 == 0 && C + 16 <= 256 && A + 4 <= 256 && (A + 4 <= C || A >= C + 16), "a wave has 256 AccVGPRs");
+#ifdef __HIP_DEVICE_COMPILE__
+  if constexpr (FIRST)
+    asm volatile("v_mfma_f32_32x32x16_f16 a[%1:%2], a[%3:%4], %0, 0" ::"v"(b), "n"(C), "n"(C + 15), "n"(A), "n"(A + 3) : QFA_ACC_256);
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 a[%1:%2], a[%3:%4], %0, a[%1:%2]" ::"v"(b), "n"(C), "n"(C + 15), "n"(A), "n"(A + 3) : QFA_ACC_256);
+#endif
+}
+// the transposing read of 8 bytes at a0 + OFF and 8 at a1 + OFF + 256 into a[A : A+3], which are there behind lds_wait_for<0>()
+template <int A, int OFF> __device__ __forceinline__ void acc_request_const(unsigned a0, unsigned a1) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("ds_read_b64_tr_b16 a[%2:%3], %0 offset:%6\n\tds_read_b64_tr_b16 a[%4:%5], %1 offset:%7"
+               ::"v"(a0), "v"(a1), "n"(A), "n"(A + 1), "n"(A + 2), "n"(A + 3), "n"(OFF), "n"(OFF + 256) : QFA_ACC_256, "memory");
+#endif
+}
 // tile I = 0 (one statement for the tile: between statements that clobber the same registers the compiler puts wait states)
 template <int I, int TILES> __device__ __forceinline__ void acc_zero_tile() {
 #ifdef __HIP_DEVICE_COMPILE__

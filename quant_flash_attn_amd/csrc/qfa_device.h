@@ -137,6 +137,11 @@ __device__ __forceinline__ float max_across_halves(float x) {
   return fmaxf(lo, hi);
 }
 
+// a's upper half of the wave and b's lower half change places
+__device__ __forceinline__ void swap_halves(unsigned &a, unsigned &b) {
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+
 // ---- direct global -> LDS tile copies -------------------------------------------------------------
 // global_load_lds_dwordx4 writes lane l's 16 bytes to LDS[wave-uniform base + 16*l], so a tile lands
 // in LDS as dense rows without padding.  Bank conflicts are avoided by an XOR swizzle applied on the

@@ -119,6 +119,9 @@ SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D);
 int launch_skv_tile_fwd(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t st);
 int launch_skv_tile_dq(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t st);
 int launch_skv_dkv(const SkvAttnArgs &a, hipStream_t st);
+// dQ and dKV of 33 to 128 queries in one pass (head_dim 64 and 128): a workgroup per head, where there are enough of them
+bool skv_pass_takes(int64_t BH, int64_t Nq, int64_t Nk, int D);
+int launch_skv_pass(const SkvAttnArgs &a, hipStream_t st);
 // dQ = the sum of its partial results [B*H*Nq][splits][D] in a.workspace, times *grad_scale, rounded
 int launch_split_sum(const SkvAttnArgs &a, int splits, hipStream_t st);
 // one fused backward pass while the per-wave accumulators of dQ fit: 32 queries up to head_dim 128, 16 at 256

@@ -1,4 +1,4 @@
-// dKV of the shared-KV attention for query blocks of any length:
+// dKV of the shared-KV attention for query blocks of any length (33 to 128 queries of many heads: qfa_skv_pass.hip):
 //     P = exp(sm_scale * Q KV^T - LSE),  dS = sm_scale * P o (dO KV^T - delta),  dKV = P^T dO + dS^T Q,  delta = rowsum(O o dO)
 // (quant_flash_attn.py:104-166).
 //

@@ -142,6 +142,18 @@ SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   return t < limit ? p : SkvTilePlan{0, 1, 0};
 }
 
+// One workgroup per (batch, head) does the whole backward, one on a CU at head_dim 128 and two at 64.  Timed beside the two kernels
+// with their splits in 2200 calls of 8 to 3000 heads, 33 to 128 queries and 64 to 16000 keys, time over theirs: head_dim 128 from 128
+// heads on 0.71 to 0.89 in the mean, at most 1.00, but 1.02 to 1.05 where a few heads more than the CUs leave a second round nearly
+// empty (257 to 280 heads) and where thousands of heads have one or two tiles each (its start weighs more than theirs); 64 to
+// 128 heads 0.98 to 1.01, up to 1.6 for long sequences, whose keys the others split.  head_dim 64 from 320 heads on 0.75 to 0.86, below
+// 0.97 to 1.3.
+bool skv_pass_takes(int64_t BH, int64_t Nq, int64_t Nk, int D) {
+  if (Nq <= 32 || Nq > 128 || BH > 0x7fffffffLL) return false;
+  if (D == 64) return BH >= 320;
+  return D == 128 && BH >= 128 && (BH <= 256 || BH >= 288) && (Nk > 128 || BH <= 1024);
+}
+
 int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   int splits = 1;
   int64_t each;
@@ -151,6 +163,7 @@ int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D) {
 }
 
 int64_t skv_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
+  if (skv_pass_takes(B * H, Nq, Nk, D)) return 0;
   const int s = skv_bwd_one_pass(Nq, D) ? skv_bwd_splits(B * H, Nq, Nk, D) : skv_tile_dq_plan(B * H, Nq, Nk, D).splits;
   return s > 1 ? B * H * Nq * s * (int64_t)D * 4 : 0;
 }

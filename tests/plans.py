@@ -36,3 +36,7 @@ def skv_tile_fwd_plan(BH, Nq, Nk, D):
 
 def skv_tile_dq_plan(BH, Nq, Nk, D):
     return _plan("_ZN3qfa16skv_tile_dq_planEllli", SkvTilePlan, [_L, _L, _L, _I])(BH, Nq, Nk, D)
+
+
+def skv_pass_takes(BH, Nq, Nk, D):
+    return _plan("_ZN3qfa14skv_pass_takesEllli", ctypes.c_bool, [_L, _L, _L, _I])(BH, Nq, Nk, D)

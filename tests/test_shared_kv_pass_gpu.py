@@ -1,0 +1,92 @@
+"""The shared-KV backward in one pass of 33 to 128 queries (one workgroup per head, where there are enough heads), at the sizes where
+it can go wrong: one key, blocks of 32 and tiles of 64 keys with one more or one less, odd and even numbers of tiles, one to five of
+them (its rings of tiles hold four and five), blocks of 32 queries that hold one or none, a partly filled second half of the queries'
+waves, strides."""
+import math
+
+import pytest
+import torch
+
+from helpers import COS_TOL, assert_close
+from oracle import oracle
+from plans import skv_pass_takes
+from quant_flash_attn_amd import _lib
+
+DEV = "cuda:0"
+NQ = [33, 61, 64, 65, 96, 97, 128]
+NK = [1, 31, 63, 64, 65, 97, 128, 129, 191, 256, 300, 389]
+HEADS = {64: 320, 128: 128}   # the fewest
+
+
+def test_line(qfa):
+    """Which calls take it, and that they need no scratch."""
+    for D, least in HEADS.items():
+        for Nq in (32, 33, 128, 129):
+            for BH in (least - 1, least, 5000):
+                takes = 33 <= Nq <= 128 and BH >= least
+                assert bool(skv_pass_takes(BH, Nq, 500, D)) == takes
+                if takes:
+                    assert _lib.lib().qfa_attn_bwd_shared_kv_workspace_bytes(1, BH, Nq, 500, D) == 0
+    assert not skv_pass_takes(5000, 64, 500, 256)
+    assert not skv_pass_takes(270, 64, 500, 128) and not skv_pass_takes(5000, 64, 128, 128)
+
+
+def _case(BH, Nq, Nk, D, dtype, sdtype, layout):
+    g = torch.Generator().manual_seed(1000 * Nq + Nk + D)
+    r = lambda n: torch.randn((1, BH, n, D), generator=g)
+    kv = (r(Nk) + 0.3 * torch.randn((1, BH, Nk, 1), generator=g)).to(dtype)
+    q, do = r(Nq).to(dtype), r(Nq).to(dtype)
+    dev = lambda t: t.to(DEV) if layout == "heads" else t.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)   # tokens outside, heads inside
+    return q, kv, do, dev(q), dev(kv), dev(do)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq", NQ)
+def test_against_the_oracle(qfa, Nq, D):
+    """dQ and dKV of three heads, for every number of keys; types and layouts by turns."""
+    BH, sm = HEADS[D], 1.0 / math.sqrt(D)
+    for i, Nk in enumerate(NK):
+        dtype, sdtype = (torch.float16, torch.bfloat16)[(i + Nq) % 2], (torch.float16, torch.float32)[i // 2 % 2]
+        q, kv, do, qd, kvd, dod = _case(BH, Nq, Nk, D, dtype, sdtype, ("heads", "tokens")[i // 3 % 2])
+        assert skv_pass_takes(BH, Nq, Nk, D)
+        qd.requires_grad_(True)
+        kvd.requires_grad_(True)
+        codes, scale, zp = qfa.asymmetric_quant_per_token(kvd.detach(), scale_dtype=sdtype)
+        o = qfa.quant_flash_attn(qd, kvd, (codes, scale, zp), sm)
+        grads = torch.autograd.grad(o, [qd, kvd], dod, retain_graph=True)
+        again = torch.autograd.grad(o, [qd, kvd], dod)
+        assert all(torch.equal(x, y) for x, y in zip(grads, again)), Nk
+        pick = [0, BH // 2 + 1, BH - 1]
+        q, do, codes, scale, zp, o, dq, dkv = (t.detach()[:, pick].cpu() for t in (q, do, codes, scale, zp, o, *grads))
+        (dq_ref, dkv_ref), (nq, nkv) = oracle.legacy_bwd(q, codes, scale, zp, do, sm, o=o, spread=True)
+        assert_close(f"dQ {Nk}", dq, dq_ref, scaled=True, spread=nq, cos_tol=COS_TOL if Nk > 1 else -1.0)   # one key: dQ is zero
+        assert_close(f"dKV {Nk}", dkv, dkv_ref, scaled=True, spread=nkv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq", [50, 100])
+def test_scaled_beforehand_and_rows_that_are_not_finite(qfa, Nq, D):
+    """dO in binary16 with a factor of its own beside it (the public call); an infinite query or dO row reaches dQ of its own
+    query only, and other heads not at all."""
+    BH, Nk, sm = HEADS[D], 150, 1.0 / math.sqrt(D)
+    g = torch.Generator().manual_seed(D)
+    kv, q, do = (torch.randn(s, generator=g).to(torch.float16).to(DEV) for s in ((1, BH, Nk, D), (1, BH, Nq, D), (1, BH, Nq, D)))
+    codes, scale, zp = qfa.asymmetric_quant_per_token(kv)
+    o, lse = qfa.attn_fwd_shared_kv(q, codes, scale, zp, sm)
+    want = qfa.attn_bwd_shared_kv(q, codes, scale, zp, o, do, lse, sm)
+    pick = [0, BH - 1]
+    ref, spread = oracle.legacy_bwd(*(t[:, pick].cpu() for t in (q, codes, scale, zp, do)), sm, o=o[:, pick].cpu(), spread=True)
+    for name, a, b, n in zip(("dQ", "dKV"), want, ref, spread):
+        assert_close(name, a[:, pick].cpu(), b, scaled=True, spread=n)
+    q2, do2 = q.clone(), do.clone()
+    q2[:, 3, 40, 3] = float("inf")
+    do2[:, 3, 7] = float("inf")
+    o2, lse2 = qfa.attn_fwd_shared_kv(q2, codes, scale, zp, sm)
+    got = qfa.attn_bwd_shared_kv(q2, codes, scale, zp, o2, do2, lse2, sm)
+    keep = [i for i in range(Nq) if i not in (7, 40)]
+    others = [h for h in range(BH) if h != 3]
+    assert torch.isfinite(got[0][:, 3, keep]).all() and not torch.isfinite(got[1][:, 3]).all()
+    for a, b in zip(got, want):
+        assert torch.equal(a[:, others], b[:, others])
