@@ -65,19 +65,25 @@ def test_parts_of_dq_in_the_place_of_the_others(qfa, B, H, Nq, Nk, D, causal, dt
 
 
 def _limited(f, parts):
-    """f() with all memory, and with half of `parts` bytes less than that took"""
-    res = []
-    for _ in range(2):
+    """f() with all memory, and with half of `parts` bytes less than it took beyond what was held at its start.  Both times holes in
+    the held memory that the parts could lie in are filled first: what earlier tests left there decides neither."""
+    res, total = [], torch.cuda.get_device_properties(0).total_memory
+    for limited in (False, True):
         gc.collect()
         torch.cuda.synchronize()
         torch.cuda.empty_cache()
+        held, plugs = torch.cuda.memory_reserved(), []
         try:
-            if res:
-                total = torch.cuda.get_device_properties(0).total_memory
-                torch.cuda.set_per_process_memory_fraction((peak - parts // 2) / total)
+            torch.cuda.set_per_process_memory_fraction(held / total)
+            try:
+                while True:
+                    plugs.append(torch.empty(parts // 2, dtype=torch.uint8, device=DEV))
+            except torch.OutOfMemoryError:
+                pass
+            torch.cuda.set_per_process_memory_fraction((held + taken - parts // 2) / total if limited else 1.0)
             torch.cuda.reset_peak_memory_stats()
             res.append([t.cpu() for t in f()])
-            peak = torch.cuda.max_memory_reserved()
+            taken = torch.cuda.max_memory_reserved() - held
         finally:
             torch.cuda.set_per_process_memory_fraction(1.0)
     return res
