@@ -94,6 +94,8 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
   const CopyQ cp_q(lane, (unsigned)a.sqn);
   const CopyDo cp_do(lane, (unsigned)a.sdon * 2u);
   constexpr int PIECES = CopyQ::N + CopyDo::N + CopyB::N;
+  // (head_dim 256 without a mask; see the turn of the tile)
+  constexpr bool EARLY = NSTEP == 1 && !CAUSAL;
   struct TileDesc { rsrc_t q, g, b; unsigned char *dst; };
   auto tile_desc = [&](int t) __attribute__((always_inline)) -> TileDesc {
     const int rows = min(TILE, Nq - TILE * t);
@@ -101,6 +103,13 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
             make_rsrc(wsq_bh + (int64_t)t * WS::Q_BLOB, rows > 0 ? (unsigned)WS::Q_BLOB : 0u), smem + (t - it0) % 3 * SM::BUF};
   };
   auto copy_piece = [&](const TileDesc &d, int i) __attribute__((always_inline)) {   // i: a compile-time constant everywhere
+    if constexpr (EARLY) {   // what the turn waits for comes first: the codes and the constants
+      if (i < CopyQ::N) cp_q.piece(i, d.q, d.dst + SM::OFF_Q, wave);
+      else if (i == CopyQ::N) CopyB::piece(CopyB::N - 1, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
+      else if (i <= CopyQ::N + CopyDo::N) cp_do.piece(i - CopyQ::N - 1, d.g, d.dst + SM::OFF_DO, wave);
+      else CopyB::piece(i - CopyQ::N - 1 - CopyDo::N, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
+      return;
+    }
     if (i < CopyDo::N) cp_do.piece(i, d.g, d.dst + SM::OFF_DO, wave);
     else if (i < CopyDo::N + CopyQ::N) cp_q.piece(i - CopyDo::N, d.q, d.dst + SM::OFF_Q, wave);
     else CopyB::piece(i - CopyDo::N - CopyQ::N, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
@@ -229,12 +238,25 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
       }
     };
 
+    // Turn of the tile: the next one has landed, the one after it goes into the buffer of the previous one, whose last fragments
+    // have been requested.  With one step per tile (head_dim 256) the last pieces of a copy have little time until the next turn.
+    // Without a mask the turn comes before the first request of dO there, and only the codes and constants of the next tile have to be
+    // there, dO and Qz^T one turn later (the whole backward, 64 heads of 4096: 3069 -> 3027 us; with a mask, where waves begin at
+    // different tiles: 1726 -> 1734)
+    TileDesc td;
+    auto turn = [&]() __attribute__((always_inline)) {
+      vm_wait<EARLY ? CopyDo::N + CopyB::N - 1 : 0>();
+      lds_barrier();
+      td = tile_desc(t + 2);
+    };
+    constexpr int TURN = EARLY ? NX - RING + 1 : NX;   // in front of this fragment's products
     // ---------------- dK of the previous step (Qz^T . dS) under the first part of P
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) f[kb] = mfma_16b_k8<T>(corr_q, corr_k[kb], f[kb]);
     f32x4 nd4[4];
     static_for<NX>([&](auto n_tag) __attribute__((always_inline)) {     // hh = n / DB, db = n % DB
       constexpr int n = decltype(n_tag)::value;
+      if constexpr (LAST && n == TURN) turn();
       static_for<KB>([&](auto kb_tag) __attribute__((always_inline)) {
         constexpr int kb = decltype(kb_tag)::value;
         QFA_FENCE();
@@ -249,14 +271,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
         if constexpr (kb == KB - 1 && n >= NX - 4) nd4[n - (NX - 4)] = ldf(cb + 2 * TILE * 4 + (n - (NX - 4)) * 32);
       });
     });
-    // ---------------- turn of the tile: the next one has landed, the one after it goes into the buffer of the previous one
-    // (last read by the products just issued)
-    TileDesc td;
-    if constexpr (LAST) {
-      dma_wait();
-      lds_barrier();
-      td = tile_desc(t + 2);
-    }
+    if constexpr (LAST && TURN == NX) turn();
     constexpr int CSLOTS = KB * (NP + 2 * DB);   // the copy's pieces are spread over the slots that are left
     auto copy_slot = [&](auto s_tag) __attribute__((always_inline)) {
       constexpr int s = decltype(s_tag)::value, p0 = s * PIECES / CSLOTS, p1 = (s + 1) * PIECES / CSLOTS;
