@@ -244,16 +244,17 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) f[qb] = mfma_16b_k8<T>(corr_k, corr_q[qb], __builtin_bit_cast(f32x16, si[qb]));
     // The turn of the tile: the next one has landed, the one after it goes into the buffer of the previous one, whose last
-    // fragments have been requested.  With one step per tile (head_dim 256) the last pieces of a copy have 15 products' time until
-    // the next turn, and the wave waited for them (42 % of its time): there the turn comes before the first request of V, and only the
-    // codes and constants of the next tile have to be there, V and Kz^T one turn later.  This kernel, 64 heads of 4096 causal:
-    // 818 -> 704 us; the whole backward without a mask 3386 -> 3045 us
+    // fragments have been requested.  It comes before the first request of V: three fragments' products follow whose operands are
+    // there (dQ of 16384 x 16384, 16 heads of 128: 2273 -> 2246 us against a turn behind them, 4096 causal 671 -> 666).  With one
+    // step per tile (head_dim 256) the last pieces of a copy have 15 products' time until the next turn, and the wave waited for
+    // them (42 % of its time): there only the codes and constants of the next tile have to be there, V and Kz^T one turn later.
+    // 64 heads of 4096 causal: 818 -> 704 us; the whole backward without a mask 3386 -> 3045 us
     auto turn = [&]() __attribute__((always_inline)) {
       vm_wait<NSTEP == 1 ? CopyV::N + CopyB::N - 1 : 0>();
       lds_barrier();
       td = tile_desc(t + 2);
     };
-    constexpr int TURN = NSTEP == 1 ? XA - RING + 1 : XA;   // in front of this fragment's products
+    constexpr int TURN = XA - RING + 1;   // in front of this fragment's products
     static_for<XA>([&](auto n_tag) __attribute__((always_inline)) {     // hh = n / DB, db = n % DB
       constexpr int n = decltype(n_tag)::value;
       if constexpr (LAST && n == TURN) turn();
@@ -272,7 +273,6 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
         }
       });
     });
-    if constexpr (LAST && TURN == XA) turn();
     static_for<NP>([&](auto m_tag) __attribute__((always_inline)) {
       constexpr int m = decltype(m_tag)::value, n = P0 + m;
       static_for<QB>([&](auto qb_tag) __attribute__((always_inline)) {
