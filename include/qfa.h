@@ -107,6 +107,15 @@ int qfa_dequant_per_token(const int8_t *codes, const void *scale, int scale_dtyp
 int qfa_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
                     int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb,
                     int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, void *stream);
+/*
+ * The same with the queries [B,H,Nq,D] quantized by that launch, as qfa_quant_per_token does (no 16-bit copy of the scale; q_rowsum
+ * nullable).  q_dtype: v_dtype, or QFA_F32 where that is QFA_BF16.  Strides of q, then of its codes.
+ */
+int qfa_cache_stage_q(const void *q, int q_dtype, int8_t *q_codes, float *q_scale, int8_t *q_zp, int32_t *q_rowsum, int64_t Nq,
+                      int64_t sqb, int64_t sqh, int64_t sqn, int64_t sqcb, int64_t sqch, int64_t sqcn, const int8_t *kc, const void *ks,
+                      int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs, int vs_dtype, const int8_t *vz,
+                      void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb, int64_t skh, int64_t skn, int64_t svb,
+                      int64_t svh, int64_t svn, void *stream);
 
 /*
  * rowsum[b,h,n] = sum_d codes[b,h,n,d] (int32, dense [B*H*N]): the side output of qfa_quant_per_token, for

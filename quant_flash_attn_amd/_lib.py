@@ -31,6 +31,8 @@ _SIGNATURES = {
     "qfa_quant_qkv_f32": (c_int, [_P] * 12 + [_L, _L, _L, _L, _I] + [_L] * 15 + [_P]),
     "qfa_dequant_per_token": (c_int, [_P, _P, _I, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
     "qfa_cache_stage": (c_int, [_P, _P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _L, _L, _L, _I] + [_L] * 6 + [_P]),
+    "qfa_cache_stage_q": (c_int, [_P, _I, _P, _P, _P, _P] + [_L] * 7 + [_P, _P, _I, _P, _P, _P, _P, _I, _P, _P, _I, _L, _L, _L, _I]
+                          + [_L] * 6 + [_P]),
     "qfa_code_rowsum": (c_int, [_P, _P, _L, _L, _L, _I, _L, _L, _L, _P]),
     "qfa_attn_fwd": (c_int, [_P] * 11 + [_I, _L, _L, _L, _L, _I] + [_L] * 12 + [_F, _I, _P]),
     "qfa_attn_fwd_split_workspace_bytes": (c_int64, [_L, _L, _L, _L, _I, _I]),

@@ -140,9 +140,9 @@ int qfa_dequant_per_token(const int8_t *codes, const void *scale, int scale_dtyp
                         (hipStream_t)stream);
 }
 
-int qfa_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
-                    int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb,
-                    int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, void *stream) {
+static int cache_stage(const QuantizeQ *q, const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc,
+                       const void *vs, int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb,
+                       int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, void *stream) {
   const char *who = "cache_stage";
   if (!kc || !rowsum || !vc || !vs || !vz || !v || (ks32 && !ks)) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
   if (B <= 0 || H <= 0 || N <= 0) return set_error(QFA_EINVAL, "%s: B, H, N must be positive", who);
@@ -154,7 +154,35 @@ int qfa_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32,
   if (!strides_ok(skb, skh, skn, D, 1) || !strides_ok(svb, svh, svn, D, 1))
     return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
   const int64_t sk[3] = {skb, skh, skn}, sv[3] = {svb, svh, svn};
-  return launch_cache_stage(kc, ks, ks_dtype, ks32, rowsum, vc, vs, vs_dtype, vz, v, v_dtype, B, H, N, D, sk, sv, (hipStream_t)stream);
+  if (q) {
+    if (!q->x || !q->codes || !q->scale || !q->zp) return set_error(QFA_EINVAL, "%s: null pointer argument", who);
+    if (q->N <= 0) return set_error(QFA_EINVAL, "%s: Nq must be positive", who);
+    if (q->dtype != (v_dtype == QFA_BF16 && q->dtype == QFA_F32 ? QFA_F32 : v_dtype))
+      return set_error(QFA_EINVAL, "%s: q_dtype must be v_dtype, or QFA_F32 with a v_dtype of QFA_BF16", who);
+    if (!aligned16(q->x) || !aligned8(q->codes)) return set_error(QFA_EINVAL, "%s: q must be 16-byte, its codes 8-byte aligned", who);
+    if (!strides_ok(q->sx[0], q->sx[1], q->sx[2], D, elem_size(q->dtype)))
+      return set_error(QFA_EINVAL, "%s: q strides must be positive multiples of 16 bytes, token stride >= D", who);
+    if (q->sc[0] <= 0 || q->sc[1] <= 0 || q->sc[2] < D || q->sc[0] % 8 != 0 || q->sc[1] % 8 != 0 || q->sc[2] % 8 != 0)
+      return set_error(QFA_EINVAL, "%s: codes strides must be positive multiples of 8 bytes, token stride >= D", who);
+  }
+  return launch_cache_stage(q, kc, ks, ks_dtype, ks32, rowsum, vc, vs, vs_dtype, vz, v, v_dtype, B, H, N, D, sk, sv, (hipStream_t)stream);
+}
+
+int qfa_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
+                    int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb,
+                    int64_t skh, int64_t skn, int64_t svb, int64_t svh, int64_t svn, void *stream) {
+  return cache_stage(nullptr, kc, ks, ks_dtype, ks32, rowsum, vc, vs, vs_dtype, vz, v, v_dtype, B, H, N, D, skb, skh, skn, svb, svh, svn,
+                     stream);
+}
+
+int qfa_cache_stage_q(const void *q, int q_dtype, int8_t *q_codes, float *q_scale, int8_t *q_zp, int32_t *q_rowsum, int64_t Nq,
+                      int64_t sqb, int64_t sqh, int64_t sqn, int64_t sqcb, int64_t sqch, int64_t sqcn, const int8_t *kc, const void *ks,
+                      int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs, int vs_dtype, const int8_t *vz,
+                      void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t skb, int64_t skh, int64_t skn, int64_t svb,
+                      int64_t svh, int64_t svn, void *stream) {
+  const QuantizeQ x = {q, q_dtype, q_codes, q_scale, q_zp, q_rowsum, Nq, {sqb, sqh, sqn}, {sqcb, sqch, sqcn}};
+  return cache_stage(&x, kc, ks, ks_dtype, ks32, rowsum, vc, vs, vs_dtype, vz, v, v_dtype, B, H, N, D, skb, skh, skn, svb, svh, svn,
+                     stream);
 }
 
 int qfa_code_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, int64_t N, int D, int64_t scb,

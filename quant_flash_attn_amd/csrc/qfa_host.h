@@ -24,9 +24,19 @@ int launch_quant_pair(const void *const x[2], int x_dtype, int8_t *const codes[2
 int launch_quant_qkv(const float *const x[2], int8_t *const codes[2], float *const scale[2], int8_t *const zp[2],
                      int32_t *const rowsum[2], const float *v, void *v16, int64_t B, int64_t H, const int64_t N[2], int D,
                      const int64_t sx[2][3], const int64_t sc[2][3], const int64_t sv[3], hipStream_t st);
-int launch_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
-                       int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D,
-                       const int64_t sk[3], const int64_t sv[3], hipStream_t st);   // the two strides: batch, head, token
+// queries that are quantized on the way (their strides and their codes': batch, head, token)
+struct QuantizeQ {
+  const void *x;
+  int dtype;
+  int8_t *codes;
+  float *scale;
+  int8_t *zp;
+  int32_t *rowsum;
+  int64_t N, sx[3], sc[3];
+};
+int launch_cache_stage(const QuantizeQ *q, const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc,
+                       const void *vs, int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D,
+                       const int64_t sk[3], const int64_t sv[3], hipStream_t st);   // q: nullable
 int launch_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, int64_t N, int D, int64_t scb,
                   int64_t sch, int64_t scn, hipStream_t st);
 int launch_dequant(const int8_t *codes, const void *scale, int scale_dtype, const int8_t *zp, void *out,

@@ -422,9 +422,12 @@ int launch_rowsum(const int8_t *codes, int32_t *rowsum, int64_t B, int64_t H, in
 
 // ---------------------------------------------------------------------------------------------
 // What the INT8-score forward needs of an INT8 K / V cache, in one launch: the row sums of K and its scales in fp32, V
-// dequantized.  Bound by memory (5 bytes per element of both; 64 heads of 7001 x 128: 229 MB).  Four tokens per lane group, all
-// loads before any result, as in rowsum_kernel.
+// dequantized, and (where the caller has them) the queries quantized.  Bound by memory (5 bytes per element of K and V; 64 heads of
+// 7001 x 128: 229 MB in 40 us).  Four tokens per lane group, all loads before any result, as in rowsum_kernel.  The queries' workgroups
+// come first and go under in the rest: as a launch of their own 333 of these heads' queries were 5 us (the whole call 147 -> 142 us).
 struct CacheStageArgs {
+  QuantArgs q;
+  int blocks_q;        // workgroups of the queries (none: 0)
   const int8_t *kc, *vc;
   const void *ks, *vs;
   const int8_t *vz;
@@ -435,11 +438,17 @@ struct CacheStageArgs {
   int64_t skb, skh, skn, svb, svh, svn;
   int chunks_per_bh, blocks_k, ks_dtype, vs_dtype;
 };
-template <typename TO, int D> __global__ __launch_bounds__(256) void cache_stage_kernel(CacheStageArgs a) {
+// T: type of the queries
+template <typename T, typename TO, int D> __global__ __launch_bounds__(256) void cache_stage_kernel(CacheStageArgs a) {
+  if ((int)blockIdx.x < a.blocks_q) {
+    quant_block<T, D, false>(a.q, blockIdx.x);
+    return;
+  }
   constexpr int LPT = D / 8, TPP = 256 / LPT, U = 4;
   const int tid = threadIdx.x, sub = tid % LPT;
-  const bool is_k = (int)blockIdx.x < a.blocks_k;
-  const unsigned blk = is_k ? blockIdx.x : blockIdx.x - a.blocks_k;
+  const unsigned block = blockIdx.x - a.blocks_q;
+  const bool is_k = (int)block < a.blocks_k;
+  const unsigned blk = is_k ? block : block - a.blocks_k;
   const unsigned bh = blk / (unsigned)a.chunks_per_bh, chunk = blk - bh * a.chunks_per_bh;
   const int64_t b = index_div(bh, a.H), h = bh - b * a.H;
   const int64_t n0 = (int64_t)chunk * (TPP * U) + tid / LPT, t0 = (int64_t)bh * a.N;
@@ -491,28 +500,34 @@ template <typename TO, int D> __global__ __launch_bounds__(256) void cache_stage
     *reinterpret_cast<u32x4 *>(static_cast<TO *>(a.v) + (t0 + n[u]) * D + sub * 8) = p;
   }
 }
-template <typename TO, int D> static int launch_cache_stage_td(CacheStageArgs a, int64_t BH, hipStream_t st) {
+template <typename T, typename TO, int D> static int launch_cache_stage_td(CacheStageArgs a, int64_t BH, hipStream_t st) {
   constexpr int TOK = 8192 / D;   // tokens per workgroup
-  const int64_t chunks = (a.N + TOK - 1) / TOK;
-  if (2 * chunks * BH > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "cache_stage: too many tokens for one launch");
+  const int64_t chunks = (a.N + TOK - 1) / TOK, chunks_q = (a.q.N + TOK - 1) / TOK, total = (2 * chunks + chunks_q) * BH;
+  if (total > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "cache_stage: too many tokens for one launch");
   a.chunks_per_bh = (int)chunks;
   a.blocks_k = (int)(chunks * BH);
-  cache_stage_kernel<TO, D><<<dim3((unsigned)(2 * chunks * BH)), dim3(256), 0, st>>>(a);
+  a.q.chunks_per_bh = (int)chunks_q;
+  a.blocks_q = (int)(chunks_q * BH);
+  cache_stage_kernel<T, TO, D><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   return check_launch("qfa_cache_stage");
 }
-int launch_cache_stage(const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc, const void *vs,
-                       int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D,
+template <typename T, typename TO> static int launch_cache_stage_t(const CacheStageArgs &a, int D, int64_t BH, hipStream_t st) {
+  if (D == 64) return launch_cache_stage_td<T, TO, 64>(a, BH, st);
+  if (D == 128) return launch_cache_stage_td<T, TO, 128>(a, BH, st);
+  return launch_cache_stage_td<T, TO, 256>(a, BH, st);
+}
+int launch_cache_stage(const QuantizeQ *q, const int8_t *kc, const void *ks, int ks_dtype, float *ks32, int32_t *rowsum, const int8_t *vc,
+                       const void *vs, int vs_dtype, const int8_t *vz, void *v, int v_dtype, int64_t B, int64_t H, int64_t N, int D,
                        const int64_t sk[3], const int64_t sv[3], hipStream_t st) {
-  CacheStageArgs a = {kc, vc, ks, vs, vz, ks32, rowsum, v, N, H, sk[0], sk[1], sk[2], sv[0], sv[1], sv[2], 0, 0, ks_dtype, vs_dtype};
-  const int64_t BH = B * H;
-  if (v_dtype == QFA_BF16) {
-    if (D == 64) return launch_cache_stage_td<__bf16, 64>(a, BH, st);
-    if (D == 128) return launch_cache_stage_td<__bf16, 128>(a, BH, st);
-    return launch_cache_stage_td<__bf16, 256>(a, BH, st);
+  QuantArgs x = {};   // no queries
+  if (q) {
+    x.x = q->x; x.codes = q->codes; x.scale = q->scale; x.zp = q->zp; x.rowsum = q->rowsum; x.N = q->N; x.H = H; x.D = D;
+    x.sxb = q->sx[0]; x.sxh = q->sx[1]; x.sxn = q->sx[2]; x.scb = q->sc[0]; x.sch = q->sc[1]; x.scn = q->sc[2];
   }
-  if (D == 64) return launch_cache_stage_td<_Float16, 64>(a, BH, st);
-  if (D == 128) return launch_cache_stage_td<_Float16, 128>(a, BH, st);
-  return launch_cache_stage_td<_Float16, 256>(a, BH, st);
+  const CacheStageArgs a = {x, 0, kc, vc, ks, vs, vz, ks32, rowsum, v, N, H, sk[0], sk[1], sk[2], sv[0], sv[1], sv[2], 0, 0, ks_dtype, vs_dtype};
+  if (q && q->dtype == QFA_F32) return launch_cache_stage_t<float, __bf16>(a, D, B * H, st);
+  if (v_dtype == QFA_BF16) return launch_cache_stage_t<__bf16, __bf16>(a, D, B * H, st);
+  return launch_cache_stage_t<_Float16, _Float16>(a, D, B * H, st);
 }
 
 }  // namespace qfa

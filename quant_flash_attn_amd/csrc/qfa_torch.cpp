@@ -35,7 +35,7 @@ struct Api {
   QFA_ENTRY(qfa_quant_qkv_f32);
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
-  QFA_ENTRY(qfa_cache_stage);
+  QFA_ENTRY(qfa_cache_stage_q);
   QFA_ENTRY(qfa_attn_fwd);
   QFA_ENTRY(qfa_attn_fwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_split);
@@ -71,7 +71,7 @@ void init(const py::dict &address) {
   QFA_ENTRY(qfa_quant_qkv_f32);
   QFA_ENTRY(qfa_dequant_per_token);
   QFA_ENTRY(qfa_code_rowsum);
-  QFA_ENTRY(qfa_cache_stage);
+  QFA_ENTRY(qfa_cache_stage_q);
   QFA_ENTRY(qfa_attn_fwd);
   QFA_ENTRY(qfa_attn_fwd_split_workspace_bytes);
   QFA_ENTRY(qfa_attn_fwd_split);
@@ -532,12 +532,11 @@ CacheKept cache_stage(const Tensor &q_in, const Tensor &kc, const Tensor &ks, co
   const PairBuffer pb(q.size(0), q.size(1), q.size(2), 0, q.size(3));   // (no room for keys: they are the caller's)
   CacheKept r;
   r.buf = empty({pb.bytes}, at::kByte, q);
-  quantize_into(q, pb.view(r.buf, 0));
   r.kc = rows16(kc);
   r.kz = flat(kz, at::kChar, nk, "k.zero_point");
   require_gpu(q, kc, ks, kz, vc, vs, vz);
   check_codes(vc, "v.codes");
-  // K's row sums and fp32 scales and V dequantized, in one launch
+  // q quantized, K's row sums and fp32 scales and V dequantized, in one launch
   const Tensor v = rows16(vc), vzf = flat(vz, at::kChar, nk, "v.zero_point");
   TORCH_CHECK_TYPE(dtype_code(vs.scalar_type()) >= 0, "dtype and scale.dtype must be float16, bfloat16 or float32");
   const Tensor vsf = flat(vs, vs.scalar_type(), nk, "v.scale");
@@ -546,11 +545,14 @@ CacheKept cache_stage(const Tensor &q_in, const Tensor &kc, const Tensor &ks, co
   r.ks = widen ? empty({nk}, at::kFloat, q) : ksf;
   r.kr = empty({nk}, at::kInt, q);
   r.v16 = empty({kc.size(0), kc.size(1), kc.size(2), kc.size(3)}, io_dtype(q), q);
-  check(api.qfa_cache_stage(r.kc.data_ptr<int8_t>(), ksf.data_ptr(), dtype_code(ksf.scalar_type()),
-                            widen ? r.ks.data_ptr<float>() : nullptr, r.kr.data_ptr<int32_t>(), v.data_ptr<int8_t>(), vsf.data_ptr(),
-                            dtype_code(vsf.scalar_type()), vzf.data_ptr<int8_t>(), r.v16.data_ptr(), dtype_code(r.v16.scalar_type()),
-                            pb.B, pb.H, kc.size(2), (int)pb.D, QFA_STRIDES(r.kc), QFA_STRIDES(v), stream_of(q)),
-        "qfa_cache_stage");
+  const Quantized qq = pb.view(r.buf, 0);
+  check(api.qfa_cache_stage_q(q.data_ptr(), dtype_code(q.scalar_type()), const_cast<int8_t *>(qq.codes), const_cast<float *>(qq.scale),
+                              const_cast<int8_t *>(qq.zp), const_cast<int32_t *>(qq.rowsum), qq.N, QFA_STRIDES(q), qq.sb, qq.sh, qq.sn,
+                              r.kc.data_ptr<int8_t>(), ksf.data_ptr(), dtype_code(ksf.scalar_type()), widen ? r.ks.data_ptr<float>() : nullptr,
+                              r.kr.data_ptr<int32_t>(), v.data_ptr<int8_t>(), vsf.data_ptr(), dtype_code(vsf.scalar_type()),
+                              vzf.data_ptr<int8_t>(), r.v16.data_ptr(), dtype_code(r.v16.scalar_type()), pb.B, pb.H, kc.size(2), (int)pb.D,
+                              QFA_STRIDES(r.kc), QFA_STRIDES(v), stream_of(q)),
+        "qfa_cache_stage_q");
   return r;
 }
 CacheKept cache_forward(const Tensor &q, const Tensor &kc, const Tensor &ks, const Tensor &kz, const Tensor &vc, const Tensor &vs,
