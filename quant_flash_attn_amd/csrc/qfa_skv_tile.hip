@@ -61,6 +61,11 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   typedef SkvTileGeom<D, QW> GM;
   constexpr int TK = GM::TK, NB = GM::NB, KW = GM::KW, DB = D / 32, KD = D / 16;
   constexpr bool AHEAD = NB == 2;   // row fragments requested a body ahead (the next tile's second block is in LDS by then)
+  // A tile's codes are on their way for one tile of products, or (EARLY) go to LDS in the middle of a tile and are requested a tile
+  // earlier.  At head_dim 256 one wave per SIMD has nobody to fill that wait (256 heads, 512 x 4096: 752 -> 601 us; 1584 heads, 97 x 689:
+  // 275 -> 224); with four waves side by side at 128 and 64, two and three per SIMD, it costs 2 and 14 %, with two side by side it gains 1
+  // to 5 % together with the second tile's codes requested beside the first's (5247 heads, 40 x 300 of 128: 121 -> 114)
+  constexpr bool EARLY = D == 256 || NB == 1;
   constexpr int VA = D == 256 ? 4 : D == 128 ? 3 : 2;   // blocks of 32 columns of the transposed fragments requested ahead
   __shared__ __attribute__((aligned(256))) unsigned char smem[3 * GM::BUF];
 
@@ -79,13 +84,16 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   const int64_t tk0 = (int64_t)id.bh * a.Nk, tq0 = (int64_t)id.bh * a.Nq;
   const int t0 = split * a.tiles_per_split, nt = min(a.tiles_per_split, (a.Nk + TK - 1) / TK - t0);
 
-  SkvTileStage<D, TK, GM::SLAB> st;
+  typedef SkvTileStage<D, TK, GM::SLAB> Stage;
+  Stage st, st1;
   st.init((unsigned)a.scn, tid);
-  auto issue = [&](int t) __attribute__((always_inline)) {
+  auto issue = [&](Stage &x, int t) __attribute__((always_inline)) {
     const int64_t k0 = (int64_t)(t0 + t) * TK;
-    st.issue(codes_bh + k0 * a.scn, a.scale, a.scale_dtype == QFA_F32, a.zp, tk0 + k0, a.scn, a.Nk - (int)k0);
+    x.issue(codes_bh + k0 * a.scn, a.scale, a.scale_dtype == QFA_F32, a.zp, tk0 + k0, a.scn, a.Nk - (int)k0);
   };
-  issue(0);
+  st1 = st;
+  issue(st, 0);
+  if (nt > 1) issue(st1, 1);
 
   const int qi = 32 * qb + lr;
   u32x4 qf[KD];
@@ -190,10 +198,8 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   };
 
   st.commit(smem, a.scale_dtype, a_s);
-  if (nt > 1) {
-    issue(1);
-    st.commit(smem + GM::BUF, a.scale_dtype, a_s);
-  }
+  if (nt > 1) st1.commit(smem + GM::BUF, a.scale_dtype, a_s);
+  if (EARLY && nt > 2) issue(st, 2);
   __syncthreads();
   const int kr0 = 32 * NB * kw;
   int left = a.Nk - t0 * TK - kr0;   // keys that exist from the wave's first row of the tile on
@@ -208,13 +214,15 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   for (int t = 0; t < nt; ++t) {
     const int nxt = cur + 1 == 3 ? 0 : cur + 1, wr = nxt + 1 == 3 ? 0 : nxt + 1;
     const unsigned char *buf = smem + cur * GM::BUF, *nbuf = smem + nxt * GM::BUF;
-    if (t + 2 < nt) issue(t + 2);
-    if (active) {
-      if (NB == 2) body(buf, kr0, buf, kr0 + 32, left - 32, nbuf + kr0 * 32);
-      body(buf, kr0 + 32 * (NB - 1), nbuf, kr0, left - TK, nbuf + (kr0 + 32) * 32);
+    if (!EARLY && t + 2 < nt) issue(st, t + 2);
+    if (active && NB == 2) body(buf, kr0, buf, kr0 + 32, left - 32, nbuf + kr0 * 32);
+    if (EARLY && t + 2 < nt) {
+      st.commit(smem + wr * GM::BUF, a.scale_dtype, a_s);
+      if (t + 3 < nt) issue(st, t + 3);
     }
+    if (active) body(buf, kr0 + 32 * (NB - 1), nbuf, kr0, left - TK, nbuf + (kr0 + 32) * 32);
     left -= TK;
-    if (t + 2 < nt) st.commit(smem + wr * GM::BUF, a.scale_dtype, a_s);
+    if (!EARLY && t + 2 < nt) st.commit(smem + wr * GM::BUF, a.scale_dtype, a_s);
     __syncthreads();
     cur = nxt;
   }
