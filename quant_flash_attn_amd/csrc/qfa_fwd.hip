@@ -146,14 +146,91 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   for (int ks = 0; ks < KS; ++ks)
     qf[ks] = *reinterpret_cast<const i32x4 *>(qc_bh + (int64_t)qi_c * a.sqn + ks * 32 + g * 16);
   const int zq_i = (int)a.zq[tq0 + qi_c];
-  const float a_i = a.sq[tq0 + qi_c] * a.sm_scale_log2;        // > 0
+  const float sq_i = a.sq[tq0 + qi_c];
+  const int rq_i = a.rq[tq0 + qi_c];
+  const int q_first = m0 + wave * 32, q_last = q_first + 31;
+
+  // ---- tile range
+  int kv_end = Nk;
+  // causal: query i keeps keys j <= i + coff, the mask aligned to the last key (coff = Nk - Nq >= 0; the rule
+  // row >= col when Nq == Nk)
+  const int coff = CAUSAL ? a.Nk - a.Nq - key0 : 0;
+  if (CAUSAL) kv_end = min(Nk, m0 + FWD_BM + coff);
+  const int ntiles = SPLIT && kv_end <= 0 ? 0 : (kv_end + FWD_BN - 1) / FWD_BN;
+
+  // ---- tile copies: K and V by direct loads, the per-key constants through registers
+  typedef Swz<D> KSW;
+  typedef SwzQuad<2 * D> VSW;
+  struct KeyConst { float sk; int rk, zk; } kc, kc1;   // kc1: of the second tile, at the start
+
+  // Full tiles: one per-thread offset for all chunks (TileCopyU); ragged tiles (rows clamped to the
+  // last key) take the generic path.
+  TileCopyU<D, FWD_BN, NT, KSW> cp_k;
+  TileCopyU<2 * D, FWD_BN, NT, VSW> cp_v;
+  cp_k.init((unsigned)a.skn, tid);
+  cp_v.init((unsigned)(a.svn * sizeof(T)), tid);
+
+  // Full tiles are copied through buffer descriptors rebased to the tile's first row (scalar
+  // arithmetic), so a copy costs one instruction per 16-byte chunk and thread; the per-key constant
+  // vectors are read the same way, with exact bounds (keys past the end read as zero and are masked).
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const rsrc_t rs_sk = make_rsrc(a.sk + tk0, (unsigned)Nk * 4u);
+  const rsrc_t rs_rk = make_rsrc(a.rk + tk0, (unsigned)Nk * 4u);
+  const rsrc_t rs_zk = make_rsrc(a.zk + tk0, (unsigned)Nk);
+  auto load_kc = [&](int t, KeyConst &kc) {   // per-key constants of tile t -> registers
+    if (tid < FWD_BN) {
+      kc.sk = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_sk, tid * 4, t * FWD_BN * 4, 0));
+      kc.rk = __builtin_amdgcn_raw_buffer_load_b32(rs_rk, tid * 4, t * FWD_BN * 4, 0);
+      kc.zk = (int)(signed char)__builtin_amdgcn_raw_buffer_load_b8(rs_zk, tid, t * FWD_BN, 0);
+    }
+  };
+  auto load_k = [&](int t, int buf, KeyConst &kc) {
+    const int j0 = t * FWD_BN;
+    unsigned char *dst = smem + SM::OFF_K + buf * SM::K_BYTES;
+    if (j0 + FWD_BN <= Nk)
+      cp_k.issue(reinterpret_cast<const unsigned char *>(kc_bh) + (int64_t)j0 * a.skn, dst, wave_u);
+    else
+      dma_rows<D, FWD_BN, NT, KSW>(reinterpret_cast<const unsigned char *>(kc_bh), a.skn, j0, Nk - 1, dst, tid);
+    load_kc(t, kc);
+  };
+  auto store_k = [&](int buf, const KeyConst &kc) {
+    if (tid < FWD_BN) {
+      unsigned char *cb = smem + SM::OFF_C + buf * SM::C_BYTES;
+      reinterpret_cast<float *>(cb)[tid] = kc.sk;
+      // the A operand of the correction product as it is read: per k-group two dwords
+      u32x4 dg = {0u, 0u, 0u, 0u};
+      dg[0] = base128_pair<T>(kc.rk);                      // k-group 0: digits of rk,
+      dg[1] = pack2<T>(2048.0f, 0.0f);                    //            and the constant that meets 3*2^11 (the bias c0)
+      dg[2] = pack2<T>((float)kc.zk, (float)kc.zk);         // k-group 1: zk, zk
+      reinterpret_cast<u32x4 *>(cb + FWD_BN * 4)[tid] = dg;
+    }
+  };
+  auto load_v = [&](int t, int buf) {
+    if (QK_ONLY) return;   // the QK^T-stage variant multiplies nothing by V
+    const int j0 = t * FWD_BN;
+    unsigned char *dst = smem + SM::OFF_V + buf * SM::V_BYTES;
+    const int64_t vstride = a.svn * (int64_t)sizeof(T);
+    if (j0 + FWD_BN <= Nk)
+      cp_v.issue(reinterpret_cast<const unsigned char *>(v_bh) + (int64_t)j0 * vstride, dst, wave_u);
+    else
+      dma_rows<2 * D, FWD_BN, NT, VSW>(reinterpret_cast<const unsigned char *>(v_bh), vstride, j0, Nk - 1, dst, tid);
+  };
+  // ---- everything that the first tile needs is on its way before anything is waited for (one after the other, the queries, K(0) with
+  // V(0) and K(1) took a workgroup a memory latency each)
+  if (!SPLIT || ntiles > 0) {
+    load_k(0, 0, kc);
+    load_v(0, 0);
+  }
+  if (ntiles > 1) load_k(1, 1, kc1);
+
+  const float a_i = sq_i * a.sm_scale_log2;        // > 0
   // Query side (B operand) of the correction product, 4 k-slots per k-group: k-group 0 multiplies the two digits of
   // rk by -zq and the constant 2^11 by 3*2^11 (= c0, the bias of the pipelined loop); k-group 1 multiplies zk
   // (stored twice) by minus the two digits of c = rq - D*zq.
   // Two digits of 7 bits each (|c| <= 32640) up to head_dim 128, of 8 bits at head_dim 256 (|c| <= 65280): either
   // way each digit, shifted into place, has at most 8 significant bits and is exact in the 16-bit type.
   constexpr int SH = D > 128 ? 8 : 7;
-  const int c_i = a.rq[tq0 + qi_c] - D * zq_i;
+  const int c_i = rq_i - D * zq_i;
   u32x2 corr_q;
   {
     const int hi = c_i >> SH, lo = c_i & ((1 << SH) - 1);
@@ -162,8 +239,6 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   }
   // A operand that takes the bias out again: -2^11 in the slot that meets 3*2^11
   const u32x2 unbias_a = {0u, g == 0 ? pack2<T>(-2048.0f, 0.0f) : 0u};
-  const int q_first = m0 + wave * 32, q_last = q_first + 31;
-
   // ---- may this wave's queries use biased accumulators (see the head of the file)?  For every key:
   //   |terms of the first MFMA| <= |zq| (128 D + 127) + 128 (|c| + 2 * 2^SH) =: tq   (|rk digit sum| <= 128 D + 127, |zk| <= 128)
   //   |S| <= 255 * sum_d |qc_d - zq| =: 255 mq
@@ -184,72 +259,6 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     bias_ok = __builtin_amdgcn_ballot_w64(!ok) == 0;
   }
 
-  // ---- tile range
-  int kv_end = Nk;
-  // causal: query i keeps keys j <= i + coff, the mask aligned to the last key (coff = Nk - Nq >= 0; the rule
-  // row >= col when Nq == Nk)
-  const int coff = CAUSAL ? a.Nk - a.Nq - key0 : 0;
-  if (CAUSAL) kv_end = min(Nk, m0 + FWD_BM + coff);
-  const int ntiles = SPLIT && kv_end <= 0 ? 0 : (kv_end + FWD_BN - 1) / FWD_BN;
-
-  // ---- tile copies: K and V by direct loads, the per-key constants through registers
-  typedef Swz<D> KSW;
-  typedef SwzQuad<2 * D> VSW;
-  float c_sk;
-  int c_rk, c_zk;
-
-  // Full tiles: one per-thread offset for all chunks (TileCopyU); ragged tiles (rows clamped to the
-  // last key) take the generic path.
-  TileCopyU<D, FWD_BN, NT, KSW> cp_k;
-  TileCopyU<2 * D, FWD_BN, NT, VSW> cp_v;
-  cp_k.init((unsigned)a.skn, tid);
-  cp_v.init((unsigned)(a.svn * sizeof(T)), tid);
-
-  // Full tiles are copied through buffer descriptors rebased to the tile's first row (scalar
-  // arithmetic), so a copy costs one instruction per 16-byte chunk and thread; the per-key constant
-  // vectors are read the same way, with exact bounds (keys past the end read as zero and are masked).
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const rsrc_t rs_sk = make_rsrc(a.sk + tk0, (unsigned)Nk * 4u);
-  const rsrc_t rs_rk = make_rsrc(a.rk + tk0, (unsigned)Nk * 4u);
-  const rsrc_t rs_zk = make_rsrc(a.zk + tk0, (unsigned)Nk);
-  auto load_kc = [&](int t) {   // per-key constants of tile t -> registers
-    if (tid < FWD_BN) {
-      c_sk = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_sk, tid * 4, t * FWD_BN * 4, 0));
-      c_rk = __builtin_amdgcn_raw_buffer_load_b32(rs_rk, tid * 4, t * FWD_BN * 4, 0);
-      c_zk = (int)(signed char)__builtin_amdgcn_raw_buffer_load_b8(rs_zk, tid, t * FWD_BN, 0);
-    }
-  };
-  auto load_k = [&](int t, int buf) {
-    const int j0 = t * FWD_BN;
-    unsigned char *dst = smem + SM::OFF_K + buf * SM::K_BYTES;
-    if (j0 + FWD_BN <= Nk)
-      cp_k.issue(reinterpret_cast<const unsigned char *>(kc_bh) + (int64_t)j0 * a.skn, dst, wave_u);
-    else
-      dma_rows<D, FWD_BN, NT, KSW>(reinterpret_cast<const unsigned char *>(kc_bh), a.skn, j0, Nk - 1, dst, tid);
-    load_kc(t);
-  };
-  auto store_k = [&](int buf) {
-    if (tid < FWD_BN) {
-      unsigned char *cb = smem + SM::OFF_C + buf * SM::C_BYTES;
-      reinterpret_cast<float *>(cb)[tid] = c_sk;
-      // the A operand of the correction product as it is read: per k-group two dwords
-      u32x4 dg = {0u, 0u, 0u, 0u};
-      dg[0] = base128_pair<T>(c_rk);                      // k-group 0: digits of rk,
-      dg[1] = pack2<T>(2048.0f, 0.0f);                    //            and the constant that meets 3*2^11 (the bias c0)
-      dg[2] = pack2<T>((float)c_zk, (float)c_zk);         // k-group 1: zk, zk
-      reinterpret_cast<u32x4 *>(cb + FWD_BN * 4)[tid] = dg;
-    }
-  };
-  auto load_v = [&](int t, int buf) {
-    if (QK_ONLY) return;   // the QK^T-stage variant multiplies nothing by V
-    const int j0 = t * FWD_BN;
-    unsigned char *dst = smem + SM::OFF_V + buf * SM::V_BYTES;
-    const int64_t vstride = a.svn * (int64_t)sizeof(T);
-    if (j0 + FWD_BN <= Nk)
-      cp_v.issue(reinterpret_cast<const unsigned char *>(v_bh) + (int64_t)j0 * vstride, dst, wave_u);
-    else
-      dma_rows<2 * D, FWD_BN, NT, VSW>(reinterpret_cast<const unsigned char *>(v_bh), vstride, j0, Nk - 1, dst, tid);
-  };
   // this lane's read offsets inside a tile (the swizzle terms only depend on the lane)
   const int k_swz = KSW::swz(lr);                                        // rows 32*nb + lr
   int kq[KS];                                                            // K fragment ks of the lane's row
@@ -378,15 +387,8 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   };
 
   // ---- prologue: K(0), K(1) (with their constants) and V(0) resident
-  if (!SPLIT || ntiles > 0) {
-    load_k(0, 0);
-    load_v(0, 0);
-    store_k(0);
-  }
-  if (ntiles > 1) {
-    load_k(1, 1);
-    store_k(1);
-  }
+  if (!SPLIT || ntiles > 0) store_k(0, kc);
+  if (ntiles > 1) store_k(1, kc1);
   dma_wait();
   __syncthreads();
 
@@ -589,7 +591,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     // of them has the whole second body to land before the wait at the end of the tile (2 % at the causal headline
     // size against one chunk per phase over both bodies; all six at once, or three and three, are slower again)
     auto steady_tile = [&](auto b0, auto b1, auto b2, int tt) __attribute__((always_inline)) {
-      load_kc(tt + 2);
+      load_kc(tt + 2, kc);
       const rsrc_t rs_k =
           make_rsrc(reinterpret_cast<const unsigned char *>(kc_bh) + (int64_t)(tt + 2) * FWD_BN * a.skn, 0x7fffffffu);
       const rsrc_t rs_v = make_rsrc(
@@ -606,7 +608,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
         for (int c = 0; c < PER; ++c) chunk(PER * decltype(i)::value + c);
       });
       body(b0, ic<1>{}, b1, ic<0>{}, b1, ic<1>{}, no_copy);
-      store_k((int)b2);
+      store_k((int)b2, kc);
       dma_wait();
       __syncthreads();
     };
@@ -632,11 +634,11 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     // the rest of the unmasked tiles (at most two of the steady kind, then the ones whose copies are ragged or
     // missing), with run-time buffer indices (kb_cur == t % 3 here)
     for (; t < t_hot; ++t) {
-      if (t + 2 < ntiles) load_k(t + 2, kb_free);
+      if (t + 2 < ntiles) load_k(t + 2, kb_free, kc);
       if (t + 1 < ntiles) load_v(t + 1, kb_nxt);
       body(kb_cur, ic<0>{}, kb_cur, ic<1>{}, kb_nxt, ic<0>{}, no_copy);
       body(kb_cur, ic<1>{}, kb_nxt, ic<0>{}, kb_nxt, ic<1>{}, no_copy);
-      if (t + 2 < ntiles) store_k(kb_free);
+      if (t + 2 < ntiles) store_k(kb_free, kc);
       const int tmp = kb_cur; kb_cur = kb_nxt; kb_nxt = kb_free; kb_free = tmp;
       dma_wait();
       __syncthreads();
@@ -649,7 +651,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
     // block keeps the pipelined pace (the generic loop below took 2 900 cycles per block where this takes 1 600).
     if (!QK_ONLY && CAUSAL && D <= 128 && t < ntiles && coff % 32 == 0 && t == (q_first + coff + 1) / FWD_BN &&
         (t + 1) * FWD_BN <= Nk) {
-      if (t + 2 < ntiles) load_k(t + 2, kb_free);
+      if (t + 2 < ntiles) load_k(t + 2, kb_free, kc);
       if (t + 1 < ntiles) load_v(t + 1, kb_nxt);
       const int j0 = t * FWD_BN;
       const int nb_d = (q_first + coff - j0) / 32;   // 0 or 1, wave-uniform: the block that holds the diagonal
@@ -665,7 +667,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
         }
       rescale_if_needed(max_across_halves(mt));
       exp_pv(kb_cur, nb_d, u);
-      if (t + 2 < ntiles) store_k(kb_free);
+      if (t + 2 < ntiles) store_k(kb_free, kc);
       const int tmp = kb_cur; kb_cur = kb_nxt; kb_nxt = kb_free; kb_free = tmp;
       dma_wait();
       __syncthreads();
@@ -697,7 +699,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   asm volatile("" : "+s"(o_at), "+s"(son), "+s"(out), "+s"(out32), "+s"(lse));
   // ---- masked tiles (diagonal, ragged end): one block at a time, nothing carried between blocks
   for (; t < ntiles; ++t) {
-    if (t + 2 < ntiles) load_k(t + 2, kb_free);
+    if (t + 2 < ntiles) load_k(t + 2, kb_free, kc);
     if (t + 1 < ntiles) load_v(t + 1, kb_nxt);
     const int j0 = t * FWD_BN;
 #pragma unroll
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
       rescale_if_needed(prep(kb_cur, nb, s, u, j0, std::true_type{}));
       exp_pv(kb_cur, nb, u);
     }
-    if (t + 2 < ntiles) store_k(kb_free);
+    if (t + 2 < ntiles) store_k(kb_free, kc);
     const int tmp = kb_cur; kb_cur = kb_nxt; kb_nxt = kb_free; kb_free = tmp;
     dma_wait();
     __syncthreads();
