@@ -288,6 +288,7 @@ struct SkvDkvSmem {
   static constexpr int STAGE = 32 * 128;                         // per wave: 64 columns of its tile's dKV rows on their way out
   static constexpr int TOTAL = OFF_STAT + 4 * 32 * 4;            // statistics: lse (log2), delta, rowsum(Q), rowsum(dO)
   static_assert(4 * STAGE <= BUF && STAGE <= SLOT, "the output stage overlays the rows or the slot");
+  static_assert(2 * BUF <= OFF_STAT, "the tile copies leave room for a second block of rows");
   static_assert(ROWS % 256 == 0, "row offsets are XOR-ed with block offsets");
   static_assert(2 * TOTAL <= 160 * 1024, "two workgroups per CU");
 };
@@ -300,7 +301,21 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   constexpr int D = SM::D, DS = SM::DS;
   typedef Swz<D> KSW;
   typedef TileCopy<D, SKV_TILE, 64, KSW> Copy;
-  typedef TileCopy<D * 2, 32, 256, RowSwz<D>> RowCopy;
+  // 32 rows by 256 threads: a thread's chunks lie 8 rows apart and their swizzle repeats after 16, so two offsets serve all four
+  struct RowCopy {
+    unsigned off[2], step;
+    __device__ __forceinline__ void init(unsigned stride, int tid) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = tid / 32 + 8 * i;
+        off[i] = (unsigned)row * stride + (unsigned)((tid % 32 ^ RowSwz<D>::swz(row)) << 4);
+      }
+      step = 16 * stride;
+    }
+    __device__ __forceinline__ void issue_one(rsrc_t rs, unsigned char *lds, int wave, int i) const {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)(lds + (wave * 64 + 256 * i) * 16), 16, (int)off[i % 2], (int)(step * (unsigned)(i / 2)), 0, 0);
+    }
+  };
   constexpr int DB = D / 32, DBW = DB / DS, CPR = D / 8, KD = D / 16;
   __shared__ __attribute__((aligned(256))) unsigned char smem[SM::TOTAL];
 
@@ -327,22 +342,20 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   cq.init((unsigned)(a.sqn * 2), tid);
   cd.init((unsigned)(a.sdon * 2), tid);
   const _Float16 *q_bh = a.q + b * a.sqb + h * a.sqh, *d_bh = a.dout + b * a.sdob + h * a.sdoh, *o_bh = a.o + b * a.sob + h * a.soh;
-  auto issue_rows = [&](int qb) {
-    unsigned char *buf = smem;
+  auto issue_rows = [&](int qb, unsigned char *buf) {
     const int rows = min(32, a.Nq - 32 * qb);
     // rows past Nq read as zeros (exact bounds)
     const rsrc_t rq = make_rsrc(q_bh + (int64_t)32 * qb * a.sqn, (unsigned)(((rows - 1) * (int)a.sqn + D) * 2));
     const rsrc_t rd = make_rsrc(d_bh + (int64_t)32 * qb * a.sdon, (unsigned)(((rows - 1) * (int)a.sdon + D) * 2));
 #pragma unroll
-    for (int c = 0; c < RowCopy::N; ++c) {
-      cq.issue_one(rq, buf, wave, tid, c);
-      cd.issue_one(rd, buf + SM::ROWS, wave, tid, c);
+    for (int c = 0; c < 4; ++c) {
+      cq.issue_one(rq, buf, wave, c);
+      cd.issue_one(rd, buf + SM::ROWS, wave, c);
     }
   };
   // delta, row sums, LSE of block qb from its rows (thread = row tid/8, chunks tid%8 + 8k); `og` holds this thread's chunks
   // of O, which does not pass through LDS
-  auto block_stats = [&](int qb, const u32x4 *og) {
-    const unsigned char *buf = smem;
+  auto block_stats = [&](int qb, const u32x4 *og, float lse, const unsigned char *buf) {
     float *stat = reinterpret_cast<float *>(smem + SM::OFF_STAT);
     const int pi = tid / 8, part = tid % 8;
     float dsum = 0.f, rq = 0.f, rd = 0.f;
@@ -369,13 +382,14 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
     }
     if (part == 0) {
       const int qi = 32 * qb + pi;
-      stat[pi] = qi < a.Nq ? a.lse[tq0 + qi] * kLog2e : INFINITY;
+      stat[pi] = qi < a.Nq ? lse * kLog2e : INFINITY;
       stat[32 + pi] = dsum;
       stat[64 + pi] = rq;
       stat[96 + pi] = rd;
     }
   };
-  auto load_o = [&](int qb, u32x4 *og) {
+  auto load_o = [&](int qb, u32x4 *og, float &lse) {
+    lse = a.lse[tq0 + min(32 * qb + tid / 8, a.Nq - 1)];
     const int pi = tid / 8, part = tid % 8;
     const bool live = 32 * qb + pi < a.Nq;
 #pragma unroll
@@ -391,7 +405,6 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   };
 
   // ---- per-lane LDS offsets inside a row block (as in the fused kernel)
-  const unsigned lds0 = lds_addr(smem);
   const int row_off = lr * (D * 2), row_swz = RowSwz<D>::swz(lr);
   const int s16 = lane % 16, G = lane / 16;
   unsigned qt_off[2][2];
@@ -424,8 +437,7 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
 
   f32x16 dkv[DBW];
   // dKV^T of this wave's tile += contributions of query block qb (its rows and statistics are in LDS)
-  auto add_block = [&](int qb, bool key_ok) {
-    const unsigned char *buf = smem;
+  auto add_block = [&](bool key_ok, const unsigned char *buf) {
     const float *stat = reinterpret_cast<const float *>(smem + SM::OFF_STAT);
     const float a_sk = key_ok ? a.sm_scale_log2 * sk : 0.f;
     const float sm_k = key_ok ? a.sm_scale : 0.f;
@@ -463,7 +475,7 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
       for (int hh = 0; hh < 2; ++hh)
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-          const unsigned ad = lds0 + (qt_off[hh][r] ^ ((4 * (db0 + db)) << 4));
+          const unsigned ad = lds_addr(buf) + (qt_off[hh][r] ^ ((4 * (db0 + db)) << 4));
           fr[0][hh][r] = lds_read_tr16_async<SM::ROWS>(ad);
           fr[1][hh][r] = lds_read_tr16_async<0>(ad);
         }
@@ -535,14 +547,15 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   };
 
   u32x4 og[(CPR + 7) / 8];
+  float lse;
   if (KEEP) {
     // ---- the rows and the first tile, copied together; statistics once
     if (tile_of(c_begin) < ntiles) issue_tile(tile_of(c_begin));
-    issue_rows(0);
-    load_o(0, og);
+    issue_rows(0, smem);
+    load_o(0, og, lse);
     dma_wait();
     __syncthreads();
-    block_stats(0, og);
+    block_stats(0, og, lse, smem);
     __syncthreads();
     // The output stage is the wave's tile slot once its operands are in registers, so the next tile's copy goes out after the
     // stores, and the wait at the top of the next round covers both.
@@ -554,7 +567,7 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
       const int tn = tile_of(c + 1);
       clear_dkv();
       const int j0 = t * SKV_TILE;
-      add_block(0, j0 + lr < a.Nk);
+      add_block(j0 + lr < a.Nk, smem);
       write_out(slot, j0);
       if (c + 1 < c_end && tn < ntiles) {
         lds_wait_all();
@@ -569,21 +582,24 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   const bool t_ok = t < ntiles;                   // (a wave without a tile still takes part in copies and barriers)
   const int j0 = t * SKV_TILE;
   if (t_ok) issue_tile(t);
-  issue_rows(0);   // together with the tile: one memory latency for both
+  issue_rows(0, smem);   // together with the tile: one memory latency for both
+  load_o(0, og, lse);
   dma_wait();
   if (t_ok) expand_tile();
   clear_dkv();
+  // Every tile is in registers: the next block's rows land where the copies were, and its O and LSE are on their way, while this one
+  // is worked on (one block after the other waited for memory: whole backward, 1584 heads, 97 x 689: 1148 -> 1090 us; 256 heads, 512 x
+  // 4096: 3246 -> 3134)
+  __syncthreads();
   for (int qb = 0; qb < nqb; ++qb) {
-    if (qb > 0) {
-      __syncthreads();   // everybody is done with block qb-1
-      issue_rows(qb);
-    }
-    load_o(qb, og);
-    dma_wait();          // this thread's share of block qb has landed ...
-    __syncthreads();     // ... and everybody's
-    block_stats(qb, og);
-    __syncthreads();
-    if (t_ok) add_block(qb, j0 + lr < a.Nk);
+    unsigned char *buf = smem + qb % 2 * SM::BUF;
+    if (qb + 1 < nqb) issue_rows(qb + 1, smem + (qb + 1) % 2 * SM::BUF);
+    block_stats(qb, og, lse, buf);
+    if (qb + 1 < nqb) load_o(qb + 1, og, lse);
+    lds_barrier();
+    if (t_ok) add_block(j0 + lr < a.Nk, buf);
+    dma_wait();          // this thread's share of the next block has landed ...
+    lds_barrier();       // ... and everybody's, and everybody is done with this one
   }
   __syncthreads();   // the rows are done with: the stages overlay them
   if (t_ok) write_out(smem + wave * SM::STAGE, j0);
