@@ -62,10 +62,11 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   constexpr int TK = GM::TK, NB = GM::NB, KW = GM::KW, DB = D / 32, KD = D / 16;
   constexpr bool AHEAD = NB == 2;   // row fragments requested a body ahead (the next tile's second block is in LDS by then)
   // A tile's codes are on their way for one tile of products, or (EARLY) go to LDS in the middle of a tile and are requested a tile
-  // earlier.  At head_dim 256 one wave per SIMD has nobody to fill that wait (256 heads, 512 x 4096: 752 -> 601 us; 1584 heads, 97 x 689:
-  // 275 -> 224); with four waves side by side at 128 and 64, two and three per SIMD, it costs 2 and 14 %, with two side by side it gains 1
-  // to 5 % together with the second tile's codes requested beside the first's (5247 heads, 40 x 300 of 128: 121 -> 114)
-  constexpr bool EARLY = D == 256 || NB == 1;
+  // earlier; the second tile's are requested beside the first's (BOTH) or behind them.  At head_dim 256 with four waves side by side,
+  // one wave per SIMD, nobody fills that wait (256 heads, 512 x 4096: 752 -> 601 us; 1584 heads, 97 x 689: 275 -> 224).  With four
+  // waves at 128 and 64, two and three per SIMD, EARLY costs 2 and 14 %; with two waves it gains up to 4 % there (5247 heads, 40 x 300 of
+  // 128: 121 -> 116) and nothing at 256, where BOTH costs 5 % of short calls (256 heads, 64 x 512: 25.0 -> 26.2)
+  constexpr bool EARLY = D == 256 ? NB == 2 : NB == 1, BOTH = D < 256 || NB == 2;
   constexpr int VA = D == 256 ? 4 : D == 128 ? 3 : 2;   // blocks of 32 columns of the transposed fragments requested ahead
   __shared__ __attribute__((aligned(256))) unsigned char smem[3 * GM::BUF];
 
@@ -93,7 +94,7 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   };
   st1 = st;
   issue(st, 0);
-  if (nt > 1) issue(st1, 1);
+  if (BOTH && nt > 1) issue(st1, 1);
 
   const int qi = 32 * qb + lr;
   u32x4 qf[KD];
@@ -198,7 +199,11 @@ template <int D, int QW> __global__ __launch_bounds__(256, D == 256 ? 1 : D == 1
   };
 
   st.commit(smem, a.scale_dtype, a_s);
-  if (nt > 1) st1.commit(smem + GM::BUF, a.scale_dtype, a_s);
+  if (nt > 1) {
+    Stage &second = BOTH ? st1 : st;
+    if (!BOTH) issue(second, 1);
+    second.commit(smem + GM::BUF, a.scale_dtype, a_s);
+  }
   if (EARLY && nt > 2) issue(st, 2);
   __syncthreads();
   const int kr0 = 32 * NB * kw;
