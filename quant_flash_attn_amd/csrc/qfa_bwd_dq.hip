@@ -17,7 +17,7 @@
 // take longer than its products.  Bound by the instructions a wave can issue (74 vector instructions beside 21 MFMAs of 32
 // cycles per 32 x 32 block; matrix pipe busy 72 % at 1.85 GHz on the long sequence below, 54 % on the causal one), then by power.
 // Measured, this kernel alone against the one before it (32 queries per wave, scheduled by the compiler, no bias trick):
-// 16384 x 16384, 16 heads of 128: 2890 -> 2200 us; 4096 causal, 128 heads of 128: 789 -> 650; 64 heads of 256: 1276 -> 789;
+// 16384 x 16384, 16 heads of 128: 2890 -> 2200 us; 4096 causal, 128 heads of 128: 789 -> 650; 64 heads of 256: 1276 -> 671;
 // 2048 causal, 256 heads of 64: 251 -> 226.
 #include <type_traits>
 

@@ -22,7 +22,7 @@
 // waits 27 and 36 %: eleven tiles between a workgroup's start and end, and the fourth block of 32 queries holds one.
 // Measured, 16-query kernels -> these (us, one GPU): 5247 heads, 97 x 689: forward 538 -> 298, dQ with the scaling of dO 679 -> 439
 // at head_dim 128, 333 -> 186 and 420 -> 248 at 64; 512 heads, 512 x 4096: 1069 -> 566 and 1141 -> 831 (128), 670 -> 349 and 732 ->
-// 476 (64); 256 heads of 256: forward 997 -> 771 (dQ stays with the 16-query kernel).
+// 476 (64); 256 heads of 256: forward 997 -> 601 (dQ stays with the 16-query kernel).
 #include <type_traits>
 
 #include "qfa_host.h"
