@@ -38,12 +38,10 @@ int by_dim(int D) { return D == 256 ? 2 : D == 128 ? 1 : 0; }
 //                               head_dim 64                              128                                      256
 // 16 queries per workgroup, tiles of 32 keys dealt to four waves
 const Cost kFwd16[3] = {{3.6f, .639f, .361f, .34f, .56f, 2.9f, 2.3f, 3}, {3.9f, .890f, .556f, .84f, 1.05f, 2.8f, 1.9f, 3}, {4.0f, 1.387f, .957f, 2.49f, 2.51f, 3.1f, 1.3f, 2}};
-// 32 queries per wave, tiles of 64 keys; two and four waves side by side (four at 256: fitted again to 256 workgroups of 8 to 128 tiles
-// since their codes are requested a tile earlier; of 45 shapes of 11 to 1428 heads that they take over by it 43 are faster, 0.89 times in
-// the geometric mean, 1.017 at most)
+// 32 queries per wave, tiles of 64 keys; two and four waves side by side
 const Cost kFwdTile[2][3] = {
     {{4.6f, .673f, .377f, .52f, 1.12f, 2.5f, 1.7f, 3}, {2.9f, .870f, .600f, 3.88f, 2.61f, 1.9f, 2.3f, 2}, {1.6f, 1.507f, 0.f, 8.67f, 0.f, 1.1f, 2.5f, 1}},
-    {{4.5f, .934f, .607f, .50f, 1.15f, 2.7f, 1.9f, 3}, {3.4f, 1.183f, .908f, 2.64f, 2.50f, 2.5f, 2.4f, 2}, {0.2f, 2.07f, 0.f, 8.9f, 0.f, 2.1f, 2.6f, 1}}};
+    {{4.5f, .934f, .607f, .50f, 1.15f, 2.7f, 1.9f, 3}, {3.4f, 1.183f, .908f, 2.64f, 2.50f, 2.5f, 2.4f, 2}, {0.2f, 2.467f, 0.f, 8.17f, 0.f, 2.1f, 2.6f, 1}}};
 // one-pass backward: up to 16 queries, up to 32 (650 launches each of 1 to 1500 heads, 300 to 24000 keys, 5 to 8 % rms)
 const Cost kPass[2][3] = {
     {{6.1f, 1.638f, 1.159f, .74f, .52f, 2.7f, 2.4f, 2}, {6.0f, 2.717f, 2.163f, 3.18f, 2.53f, 1.8f, 1.5f, 2}, {2.2f, 5.371f, 4.535f, 13.27f, 11.20f, 0.6f, 1.7f, 1}},
