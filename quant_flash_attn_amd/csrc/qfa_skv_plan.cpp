@@ -38,7 +38,10 @@ int by_dim(int D) { return D == 256 ? 2 : D == 128 ? 1 : 0; }
 //                               head_dim 64                              128                                      256
 // 16 queries per workgroup, tiles of 32 keys dealt to four waves
 const Cost kFwd16[3] = {{3.6f, .639f, .361f, .34f, .56f, 2.9f, 2.3f, 3}, {3.9f, .890f, .556f, .84f, 1.05f, 2.8f, 1.9f, 3}, {4.0f, 1.387f, .957f, 2.49f, 2.51f, 3.1f, 1.3f, 2}};
-// 32 queries per wave, tiles of 64 keys; two and four waves side by side
+// 32 queries per wave, tiles of 64 keys; two and four waves side by side.  (Four at 256 are faster since their codes are requested a
+// tile earlier: fitted again, 2.07 and 8.9, they would take calls at 0.89 of the time in the mean.  Not done: those calls would have
+// one reference maximum per query instead of two or four, and an fp16 error against 64 bits 1.0004 to 1.08 times as large, most at
+// few keys.)
 const Cost kFwdTile[2][3] = {
     {{4.6f, .673f, .377f, .52f, 1.12f, 2.5f, 1.7f, 3}, {2.9f, .870f, .600f, 3.88f, 2.61f, 1.9f, 2.3f, 2}, {1.6f, 1.507f, 0.f, 8.67f, 0.f, 1.1f, 2.5f, 1}},
     {{4.5f, .934f, .607f, .50f, 1.15f, 2.7f, 1.9f, 3}, {3.4f, 1.183f, .908f, 2.64f, 2.50f, 2.5f, 2.4f, 2}, {0.2f, 2.467f, 0.f, 8.17f, 0.f, 2.1f, 2.6f, 1}}};
