@@ -4,7 +4,7 @@
 // At this width a wave's operands -- Q and dO rows, 32 columns of dO^T and Q^T for all queries -- and its accumulators fit 256
 // registers and a workgroup 52 KB of LDS, so two workgroups run on a CU and fill each other's waits: scheduled by the compiler, one
 // buffer of P and dS, two barriers a tile.  (Written out with one wave per SIMD, as at 128, it took 590 us for 5247 heads, 97 x 689,
-// this one 440, the two kernels it stands for 580; from 320 heads on 0.75 to 0.86 times their time in the mean over 250 calls.
+// this one 440, the two kernels it stands for 580; where it is taken: skv_pass_takes.
 // Exponentials and vector work take longer than the products here, and one wave issues an instruction every 4 cycles.)
 #include "qfa_host.h"
 #include "qfa_skv_tile.h"

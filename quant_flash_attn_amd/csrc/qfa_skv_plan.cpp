@@ -146,15 +146,26 @@ SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {
 }
 
 // One workgroup per (batch, head) does the whole backward, one on a CU at head_dim 128 and two at 64.  Timed beside the two kernels
-// with their splits in 2200 calls of 8 to 3000 heads, 33 to 128 queries and 64 to 16000 keys, time over theirs: head_dim 128 from 128
-// heads on 0.71 to 0.89 in the mean, at most 1.00, but 1.02 to 1.05 where a few heads more than the CUs leave a second round nearly
-// empty (257 to 280 heads) and where thousands of heads have one or two tiles each (its start weighs more than theirs); 64 to
-// 128 heads 0.98 to 1.01, up to 1.6 for long sequences, whose keys the others split.  head_dim 64 from 320 heads on 0.75 to 0.86, below
-// 0.97 to 1.3.
+// with their splits in 15000 calls of 128 to 3000 heads, 33 to 128 queries and 16 to 65000 keys: 0.77 of their time in the mean at
+// head_dim 64, 0.73 at 128, at most 1.04 (20 more heads than an edge below, 6000 keys and more).  Left out:
+//   few heads: 64 to 128 heads of 128 take 0.98 to 1.01, up to 1.6 for long sequences, whose keys the others split, and 128 to 139 of
+//     them up to 1.17 beyond 4000 keys; 64 to 319 heads of 64 0.97 to 1.3, 320 to 339 up to 1.21 beyond 2750 keys and 340 to 383 up
+//     to 1.07 beyond 6000;
+//   a few heads more than fill the chip, whose last round is nearly empty while the others split evenly: 257 to 287 of 128 1.02 to
+//     1.06, 288 to 299 up to 1.10 beyond 2000 keys; 513 to 589 of 64 up to 1.18 beyond 2250, 590 to 689 up to 1.07 from there to 3250
+//     (behind a second full round the worst is 0.99);
+//   thousands of heads of 128 with one or two tiles each: its start weighs more than theirs (1.02).
 bool skv_pass_takes(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   if (Nq <= 32 || Nq > 128 || BH > 0x7fffffffLL) return false;
-  if (D == 64) return BH >= 320;
-  return D == 128 && BH >= 128 && (BH <= 256 || BH >= 288) && (Nk > 128 || BH <= 1024);
+  if (D == 64) {
+    if (BH < 384) return BH >= 320 && Nk <= (BH < 340 ? 2750 : 6000);
+    if (BH > 512 && BH < 690) return Nk <= 2250 || (BH >= 590 && Nk > 3250);
+    return true;
+  }
+  if (D != 128) return false;
+  if (BH < 140) return BH >= 128 && Nk <= 4000;
+  if (BH > 256 && BH < 300) return BH >= 288 && Nk <= 2000;
+  return Nk > 128 || BH <= 1024;
 }
 
 int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D) {

@@ -31,6 +31,20 @@ def test_line(qfa):
     assert not skv_pass_takes(270, 64, 500, 128) and not skv_pass_takes(5000, 64, 128, 128)
 
 
+@pytest.mark.parametrize("BH,Nq,Nk,D,us", [   # us of the one pass and of the two kernels with their splits, on an MI355X
+    (320, 72, 16000, 64, (746, 616)), (327, 86, 4558, 64, (216, 204)), (340, 72, 16000, 64, (743, 693)), (320, 40, 2500, 64, (84, 90)),
+    (360, 72, 6000, 64, (281, 288)), (384, 96, 16000, 64, (766, 760)), (512, 65, 4000, 64, (194, 253)),
+    (513, 40, 16000, 64, (916, 776)), (525, 34, 6365, 64, (377, 325)), (576, 33, 4000, 64, (236, 226)), (513, 65, 1500, 64, (120, 122)),
+    (660, 40, 2500, 64, (172, 161)), (660, 72, 4000, 64, (323, 334)), (700, 40, 2500, 64, (171, 174)),
+    (128, 65, 16000, 128, (539, 462)), (136, 74, 14424, 128, (486, 479)), (128, 97, 1000, 128, (44, 64)), (160, 65, 16000, 128, (550, 577)),
+    (274, 111, 3997, 128, (366, 345)), (288, 65, 8000, 128, (569, 554)), (288, 97, 1000, 128, (88, 113)), (320, 65, 16000, 128, (1100, 1161)),
+    (513, 97, 4000, 128, (454, 634))])
+def test_choice_is_not_slower(qfa, BH, Nq, Nk, D, us):
+    """Few heads, and a few more than fill the chip: whichever way a call goes is not a fiftieth slower than the other."""
+    takes = skv_pass_takes(BH, Nq, Nk, D)
+    assert us[0 if takes else 1] <= 1.02 * us[1 if takes else 0]
+
+
 def _case(BH, Nq, Nk, D, dtype, sdtype, layout):
     g = torch.Generator().manual_seed(1000 * Nq + Nk + D)
     r = lambda n: torch.randn((1, BH, n, D), generator=g)
