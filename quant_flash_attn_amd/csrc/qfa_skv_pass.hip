@@ -436,6 +436,9 @@ template <typename S, typename G, int QW> __global__ __launch_bounds__(256, 1) v
   });
   acc_settle();
   const int pin = 2 * GM::OFF_P + GM::PBUF - pout;
+  // (zero wins over dS where a key's scale is zero, also where the key exists: what is not finite in a query's dS, because its dO or LSE
+  // is not, reaches its dQ here)
+  const float osc_q = __builtin_isfinite(nd) && nlse2 == nlse2 ? osc : __builtin_nanf("");
   unsigned char *stage = smem + (wave < 2 ? kbuf : next_of(kbuf)) + wave % 2 * 64 * D;
   static_assert(2 * 64 * D <= GM::BUF && GM::ROWS * 2 * D + 128 <= 2 * GM::BUF, "two stages in a buffer");
   const rsrc_t before = nt > 1 ? ro : make_rsrc(a.dkv, 0u);
@@ -455,7 +458,7 @@ template <typename S, typename G, int QW> __global__ __launch_bounds__(256, 1) v
       }
       if constexpr (KW == 1 && s >= 8 && s < 8 + 4 * DB) {   // quad aa of columns 32db: as store_tile_rows lays them down
         constexpr int q = s - 8, R = 4 * q;
-        const float x0 = acc_read_reg<R>() * osc, x1 = acc_read_reg<R + 1>() * osc, x2 = acc_read_reg<R + 2>() * osc, x3 = acc_read_reg<R + 3>() * osc;
+        const float x0 = acc_read_reg<R>() * osc_q, x1 = acc_read_reg<R + 1>() * osc_q, x2 = acc_read_reg<R + 2>() * osc_q, x3 = acc_read_reg<R + 3>() * osc_q;
         *reinterpret_cast<u32x2 *>(stage + lr * 2 * D + ((q ^ lr % 16) * 16) + 8 * g) = u32x2{pack2<G>(x0, x1), pack2<G>(x2, x3)};
       }
     });
@@ -489,7 +492,7 @@ template <typename S, typename G, int QW> __global__ __launch_bounds__(256, 1) v
     if (kw > 0 || 32 * qb >= a.Nq) return;
 #pragma unroll
     for (int i = 0; i < 16 * DB; ++i) x[i / 16][i % 16] += mine[i * 64];
-    store_tile_rows<G, D>(x, osc, smem + qb * GM::MERGE, dq, a.sdqn, 32 * qb, a.Nq, lane);
+    store_tile_rows<G, D>(x, osc_q, smem + qb * GM::MERGE, dq, a.sdqn, 32 * qb, a.Nq, lane);
   }
 #endif
 }

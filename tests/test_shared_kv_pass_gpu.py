@@ -104,3 +104,29 @@ def test_scaled_beforehand_and_rows_that_are_not_finite(qfa, Nq, D):
     assert torch.isfinite(got[0][:, 3, keep]).all() and not torch.isfinite(got[1][:, 3]).all()
     for a, b in zip(got, want):
         assert torch.equal(a[:, others], b[:, others])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq", [50, 100])
+def test_scales_of_zero_hide_nothing(qfa, Nq, D):
+    """Keys whose scales are zero (a scale below binary16's range is stored as one) are keys: what is not finite in dO reaches dQ of its
+    query through them, and a finite row's dQ is zero."""
+    BH, Nk, sm = HEADS[D], 150, 1.0 / math.sqrt(D)
+    g = torch.Generator().manual_seed(D)
+    kv, q, do = (torch.randn(s, generator=g).to(torch.float16).to(DEV) for s in ((1, BH, Nk, D), (1, BH, Nq, D), (1, BH, Nq, D)))
+    codes, scale, zp = qfa.asymmetric_quant_per_token(kv)
+    scale[:, 3] = 0
+    scale[:, 4, ::2] = 0
+    do[:, 3:5, 7, 2] = float("inf")
+    o, lse = qfa.attn_fwd_shared_kv(q, codes, scale, zp, sm)
+    dq, dkv = qfa.attn_bwd_shared_kv(q, codes, scale, zp, o, do, lse, sm)
+    rows = torch.isfinite(dq).all(-1)[0]
+    want = torch.ones_like(rows)
+    want[3:5, 7] = False
+    assert torch.equal(rows, want)
+    assert (dq[0, 3, :7] == 0).all() and (dq[0, 3, 8:] == 0).all()
+    pick = [0, 5, BH - 1]
+    ref, spread = oracle.legacy_bwd(*(t[:, pick].cpu() for t in (q, codes, scale, zp, do)), sm, o=o[:, pick].cpu(), spread=True)
+    for name, a, b, n in zip(("dQ", "dKV"), (dq, dkv), ref, spread):
+        assert_close(name, a[:, pick].cpu(), b, scaled=True, spread=n)
