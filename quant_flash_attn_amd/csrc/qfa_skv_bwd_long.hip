@@ -653,9 +653,7 @@ template <typename S, int D> static int launch_skv_bwd_long_sd(const SkvAttnArgs
 }
 
 int launch_skv_bwd_long(const SkvAttnArgs &x, hipStream_t st) {
-  // (that pass forms the offsets of a head's rows in 31 bits)
-  const int64_t rows = x.Nk + 512, most = 1 << 23;
-  if (skv_pass_takes(x.B * x.H, x.Nq, x.Nk, x.D) && rows * x.scn < (1LL << 31) && rows * x.sdkn < (1LL << 30) && x.sdqn < most && x.sdkn < most)
+  if (skv_pass_takes(x.B * x.H, x.Nq, x.Nk, x.D) && skv_pass_fits(x.Nk, x.scn, x.sdqn, x.sdkn))
     return launch_skv_pass(x, st);
   const bool s32 = x.scale_dtype == QFA_F32;
   if (x.D == 256) return s32 ? launch_skv_bwd_long_sd<float, 256>(x, st) : launch_skv_bwd_long_sd<_Float16, 256>(x, st);

@@ -177,7 +177,9 @@ int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D) {
 }
 
 int64_t skv_bwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D) {
-  if (skv_pass_takes(B * H, Nq, Nk, D)) return 0;
+  // The one pass needs none.  Where a layout with the heads inside the tokens would not fit it (skv_pass_fits; the strides are not known
+  // here) the answer is what the two kernels want; still wider strides run without.
+  if (skv_pass_takes(B * H, Nq, Nk, D) && skv_pass_fits(Nk, H * D, H * D, H * D)) return 0;
   const int s = skv_bwd_one_pass(Nq, D) ? skv_bwd_splits(B * H, Nq, Nk, D) : skv_tile_dq_plan(B * H, Nq, Nk, D).splits;
   return s > 1 ? B * H * Nq * s * (int64_t)D * 4 : 0;
 }

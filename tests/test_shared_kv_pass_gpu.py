@@ -9,7 +9,7 @@ import torch
 
 from helpers import COS_TOL, assert_close
 from oracle import oracle
-from plans import skv_pass_takes
+from plans import skv_pass_takes, skv_tile_dq_plan
 from quant_flash_attn_amd import _lib
 
 DEV = "cuda:0"
@@ -29,6 +29,15 @@ def test_line(qfa):
                     assert _lib.lib().qfa_attn_bwd_shared_kv_workspace_bytes(1, BH, Nq, 500, D) == 0
     assert not skv_pass_takes(5000, 64, 500, 256)
     assert not skv_pass_takes(270, 64, 500, 128) and not skv_pass_takes(5000, 64, 128, 128)
+
+
+def test_scratch_where_strides_may_not_fit(qfa):
+    """Rows of a head further apart than 31-bit offsets reach go to the two kernels, which want scratch to split few heads' keys."""
+    for B, H, Nq, Nk, D in [(1, 160, 128, 70000, 128), (2, 128, 100, 70000, 128), (1, 448, 128, 70000, 64)]:
+        assert skv_pass_takes(B * H, Nq, Nk, D)
+        plan = skv_tile_dq_plan(B * H, Nq, Nk, D)
+        want = B * H * Nq * plan.splits * D * 4
+        assert plan.splits > 1 and _lib.lib().qfa_attn_bwd_shared_kv_workspace_bytes(B, H, Nq, Nk, D) == want
 
 
 @pytest.mark.parametrize("BH,Nq,Nk,D,us", [   # us of the one pass and of the two kernels with their splits, on an MI355X
@@ -130,3 +139,42 @@ def test_scales_of_zero_hide_nothing(qfa, Nq, D):
     ref, spread = oracle.legacy_bwd(*(t[:, pick].cpu() for t in (q, codes, scale, zp, do)), sm, o=o[:, pick].cpu(), spread=True)
     for name, a, b, n in zip(("dQ", "dKV"), (dq, dkv), ref, spread):
         assert_close(name, a[:, pick].cpu(), b, scaled=True, spread=n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("which", ["codes", "dkv", "dq"])
+def test_rows_far_apart(qfa, which, D):
+    """Rows as far apart as the 31-bit offsets of the pass reach give the bits of dense ones; a step further the two kernels take the
+    call, without scratch.  Their sums run in another order and the power of two that dO is scaled by is another one: the same
+    products but for what binary16 loses (2^-10 of a value)."""
+    BH, Nq, Nk = HEADS[D], 40, 1500
+    L, g, sm = _lib.lib(), torch.Generator(device=DEV).manual_seed(D), 1.0 / math.sqrt(D)
+    q, do = (torch.randn((1, BH, Nq, D), generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    kv = torch.randn((1, BH, Nk, D), generator=g, device=DEV, dtype=torch.float16)
+    codes, scale, zp = qfa.asymmetric_quant_per_token(kv)
+    o, lse = qfa.attn_fwd_shared_kv(q, codes, scale, zp, sm)
+
+    def apart(t, stride):   # the same tensor (or room for it) with tokens `stride` elements apart, the heads of a token side by side
+        x = torch.empty((t.size(2) - 1) * stride + BH * D, dtype=t.dtype, device=DEV).as_strided(t.shape, (BH * D, D, stride, 1))
+        return x.copy_(t)
+
+    def run(codes, dq, dkv):
+        st = lambda t: t.stride()[:3]
+        rc = L.qfa_attn_bwd_shared_kv_direct(q.data_ptr(), codes.data_ptr(), scale.data_ptr(), 1, zp.data_ptr(), o.data_ptr(), do.data_ptr(),
+                                             lse.data_ptr(), dq.data_ptr(), dkv.data_ptr(), 1, 1, 1, 1, BH, Nq, Nk, D, *st(q), *st(codes),
+                                             *st(o), *st(do), *st(dq), *st(dkv), sm, None, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, L.qfa_last_error()
+        return dq, dkv
+    want = run(codes, torch.zeros_like(q), torch.zeros_like(kv))
+    rows = Nk + 512
+    past = {"codes": -(-(1 << 31) // rows), "dkv": -(-(1 << 30) // rows), "dq": 1 << 23}[which]   # the first stride that does not fit
+    past = -(-past // 16) * 16
+    for stride in (past - 16, past):
+        args = [codes, torch.zeros_like(q), torch.zeros_like(kv)]
+        i = ["codes", "dq", "dkv"].index(which)
+        args[i] = apart(args[i], stride)
+        got = run(*args)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)) == (stride < past)
+        for a, b in zip(got, want):
+            assert (a.double() - b.double()).norm() <= 2.0 ** -9 * b.double().norm()
