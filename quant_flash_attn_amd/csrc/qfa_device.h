@@ -159,7 +159,9 @@ template <int ROW_BYTES> struct Swz {
 };
 
 // Raw buffer descriptor over [p, p + bytes): loads through it take a per-lane 32-bit offset plus a
-// scalar offset (no 64-bit address arithmetic on the vector pipe) and return zero out of range.
+// scalar offset (no 64-bit address arithmetic on the vector pipe) and return zero where the two together reach past
+// the end -- also where the scalar offset alone does, and with no bytes at all.  (The compiler's documentation does not
+// promise that of the scalar offset; the hardware does it: tests/test_buffer_bounds_gpu.py.)
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);

@@ -344,7 +344,7 @@ template <typename S, bool KEEP> __global__ __launch_bounds__(256, 2) void skv_d
   const _Float16 *q_bh = a.q + b * a.sqb + h * a.sqh, *d_bh = a.dout + b * a.sdob + h * a.sdoh, *o_bh = a.o + b * a.sob + h * a.soh;
   auto issue_rows = [&](int qb, unsigned char *buf) {
     const int rows = min(32, a.Nq - 32 * qb);
-    // rows past Nq read as zeros (exact bounds)
+    // rows past Nq read as zeros (exact bounds; rows 16 on are in the scalar offset: see make_rsrc)
     const rsrc_t rq = make_rsrc(q_bh + (int64_t)32 * qb * a.sqn, (unsigned)(((rows - 1) * (int)a.sqn + D) * 2));
     const rsrc_t rd = make_rsrc(d_bh + (int64_t)32 * qb * a.sdon, (unsigned)(((rows - 1) * (int)a.sdon + D) * 2));
 #pragma unroll
