@@ -93,9 +93,9 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
   typedef BlobCopy<WS::T_BYTES, SM::C_COPY> CopyB;
   const CopyQ cp_q(lane, (unsigned)a.sqn);
   const CopyDo cp_do(lane, (unsigned)a.sdon * 2u);
-  constexpr int PIECES = CopyQ::N + CopyDo::N + CopyB::N;
-  // (head_dim 256 without a mask; see the turn of the tile)
+  // pieces of a tile; at head_dim 256 without a mask the FIRST of them, the codes and the constants, are what the turn of the tile waits for
   constexpr bool EARLY = NSTEP == 1 && !CAUSAL;
+  constexpr int PIECES = CopyQ::N + CopyDo::N + CopyB::N, FIRST = EARLY ? CopyQ::N + 1 : PIECES;
   struct TileDesc { rsrc_t q, g, b; unsigned char *dst; };
   auto tile_desc = [&](int t) __attribute__((always_inline)) -> TileDesc {
     const int rows = min(TILE, Nq - TILE * t);
@@ -103,11 +103,11 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
             make_rsrc(wsq_bh + (int64_t)t * WS::Q_BLOB, rows > 0 ? (unsigned)WS::Q_BLOB : 0u), smem + (t - it0) % 3 * SM::BUF};
   };
   auto copy_piece = [&](const TileDesc &d, int i) __attribute__((always_inline)) {   // i: a compile-time constant everywhere
-    if constexpr (EARLY) {   // what the turn waits for comes first: the codes and the constants
-      if (i < CopyQ::N) cp_q.piece(i, d.q, d.dst + SM::OFF_Q, wave);
-      else if (i == CopyQ::N) CopyB::piece(CopyB::N - 1, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
-      else if (i <= CopyQ::N + CopyDo::N) cp_do.piece(i - CopyQ::N - 1, d.g, d.dst + SM::OFF_DO, wave);
-      else CopyB::piece(i - CopyQ::N - 1 - CopyDo::N, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
+    if constexpr (EARLY) {
+      if (i < FIRST - 1) cp_q.piece(i, d.q, d.dst + SM::OFF_Q, wave);
+      else if (i == FIRST - 1) CopyB::piece(CopyB::N - 1, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
+      else if (i < FIRST + CopyDo::N) cp_do.piece(i - FIRST, d.g, d.dst + SM::OFF_DO, wave);
+      else CopyB::piece(i - FIRST - CopyDo::N, d.b, d.dst + SM::OFF_QT, d.dst + SM::OFF_C, wave, lane);
       return;
     }
     if (i < CopyDo::N) cp_do.piece(i, d.g, d.dst + SM::OFF_DO, wave);
@@ -245,7 +245,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     // different tiles: 1726 -> 1734)
     TileDesc td;
     auto turn = [&]() __attribute__((always_inline)) {
-      vm_wait<EARLY ? CopyDo::N + CopyB::N - 1 : 0>();
+      vm_wait<PIECES - FIRST>();
       lds_barrier();
       td = tile_desc(t + 2);
     };

@@ -86,7 +86,8 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
   typedef BlobCopy<WS::T_BYTES, SM::C_COPY> CopyB;
   const CopyK cp_k(lane, (unsigned)a.skn);
   const CopyV cp_v(lane, (unsigned)a.svn * 2u);
-  constexpr int PIECES = CopyK::N + CopyV::N + CopyB::N;
+  // pieces of a tile; with one step per tile the FIRST of them, the codes and the constants, are what the turn of the tile waits for
+  constexpr int PIECES = CopyK::N + CopyV::N + CopyB::N, FIRST = NSTEP == 1 ? CopyK::N + 1 : PIECES;
   struct TileDesc { rsrc_t k, v, b; unsigned char *dst; };
   auto tile_desc = [&](int t) __attribute__((always_inline)) -> TileDesc {
     const int rows = t < ntiles ? min(TILE, Nk - TILE * t) : 0;
@@ -94,11 +95,11 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
             make_rsrc(wsk_bh + (int64_t)t * WS::K_BLOB, rows > 0 ? (unsigned)WS::K_BLOB : 0u), smem + t % 3 * SM::BUF};
   };
   auto copy_piece = [&](const TileDesc &d, int i) __attribute__((always_inline)) {   // i: a compile-time constant everywhere
-    if constexpr (NSTEP == 1) {   // what the turn waits for comes first: the codes and the constants
-      if (i < CopyK::N) cp_k.piece(i, d.k, d.dst + SM::OFF_K, wave);
-      else if (i == CopyK::N) CopyB::piece(CopyB::N - 1, d.b, d.dst + SM::OFF_KT, d.dst + SM::OFF_C, wave, lane);
-      else if (i <= CopyK::N + CopyV::N) cp_v.piece(i - CopyK::N - 1, d.v, d.dst + SM::OFF_V, wave);
-      else CopyB::piece(i - CopyK::N - 1 - CopyV::N, d.b, d.dst + SM::OFF_KT, d.dst + SM::OFF_C, wave, lane);
+    if constexpr (FIRST < PIECES) {
+      if (i < FIRST - 1) cp_k.piece(i, d.k, d.dst + SM::OFF_K, wave);
+      else if (i == FIRST - 1) CopyB::piece(CopyB::N - 1, d.b, d.dst + SM::OFF_KT, d.dst + SM::OFF_C, wave, lane);
+      else if (i < FIRST + CopyV::N) cp_v.piece(i - FIRST, d.v, d.dst + SM::OFF_V, wave);
+      else CopyB::piece(i - FIRST - CopyV::N, d.b, d.dst + SM::OFF_KT, d.dst + SM::OFF_C, wave, lane);
       return;
     }
     if (i < CopyV::N) cp_v.piece(i, d.v, d.dst + SM::OFF_V, wave);
@@ -250,7 +251,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
     // them (42 % of its time): there only the codes and constants of the next tile have to be there, V and Kz^T one turn later.
     // 64 heads of 4096 causal: 818 -> 704 us; the whole backward without a mask 3386 -> 3045 us
     auto turn = [&]() __attribute__((always_inline)) {
-      vm_wait<NSTEP == 1 ? CopyV::N + CopyB::N - 1 : 0>();
+      vm_wait<PIECES - FIRST>();
       lds_barrier();
       td = tile_desc(t + 2);
     };

@@ -255,7 +255,10 @@ template <int ROW_BYTES, int ROWS, int NT, typename S = Swz<ROW_BYTES>> struct T
 // all direct loads of this wave have landed (vmcnt(0)); follow with a barrier before other waves read
 __device__ __forceinline__ void dma_wait() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 // ... all but the last N (at most 15) of them
-template <int N> __device__ __forceinline__ void vm_wait() { __builtin_amdgcn_s_waitcnt(0x0f70 | N); }
+template <int N> __device__ __forceinline__ void vm_wait() {
+  static_assert(N >= 0 && N <= 15, "the low four bits of the count");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | N);
+}
 // ds_read_b64_tr_b16: inside each group of 16 lanes, lane i receives element i%4 of the four 8-byte
 // rows addressed by lanes (i%16)/4, +4, +8, +12 of its group -- a 16-bit transpose on the way out of LDS.
 // It is issued behind the compiler's back, with an explicit wait: the compiler makes every such read
