@@ -13,8 +13,8 @@ template <int SLAB> __device__ __forceinline__ int skv_tile_off(int r, int c, in
 }
 
 // A thread's share of a tile on its way from memory to LDS: N chunks of 16 codes with their rows' zero points, one key scale
-template <int D, int TK, int SLAB, int THREADS = 256> struct SkvTileStage {
-  static constexpr int CPR = D / 16, RPW = 64 / CPR, N = TK * CPR / THREADS, STEP = THREADS / 64 * RPW;   // STEP: rows between a thread's chunks
+template <int D, int TK, int SLAB> struct SkvTileStage {
+  static constexpr int CPR = D / 16, RPW = 64 / CPR, N = TK * CPR / 256, STEP = 4 * RPW;   // STEP: rows between a thread's chunks
   unsigned off, row_step;   // of chunk 0; bytes between a thread's chunks
   int row, lds;
   int tid;
