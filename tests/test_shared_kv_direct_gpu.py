@@ -50,9 +50,11 @@ def _scaled_first(q, o, do, codes, scale, zp, lse, sm):
 @pytest.mark.parametrize("dtype,sdtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float16), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("B,H,Nq,Nk,D", [(1, 1, 1, 33, 64), (1, 3, 16, 700, 128), (2, 3, 17, 257, 64), (1, 2, 32, 4000, 128),
                                          (1, 2, 5, 100, 256), (1, 4, 16, 3001, 256), (300, 2, 3, 31, 64),
-                                         # two kernels: 16 or 32 queries per wave in dQ, keys split or not
+                                         # two kernels: 16 or 32 queries per wave in dQ, keys split or not (1060 heads over 300 keys: one pass)
                                          (1, 4, 33, 700, 128), (20, 53, 97, 300, 128), (1, 2, 128, 4097, 64), (3, 64, 65, 1000, 64),
-                                         (1, 1, 128, 31, 128)])
+                                         (1, 1, 128, 31, 128), (20, 53, 97, 100, 128), (5, 56, 97, 300, 64),
+                                         # one pass, a workgroup per head: ends of the scan for the largest key scale
+                                         (2, 64, 40, 1024, 128), (4, 32, 97, 1025, 128), (1, 320, 40, 2049, 64), (5, 64, 97, 2048, 64)])
 def test_direct_against_scaled_first(qfa, B, H, Nq, Nk, D, dtype, sdtype):
     t = _tensors(B, H, Nq, Nk, D, dtype, sdtype)
     t[2].mul_(1e-4)

@@ -117,6 +117,33 @@ def test_scaled_beforehand_and_rows_that_are_not_finite(qfa, Nq, D):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq,Nk", [(40, 1025), (97, 1025), (40, 2049), (97, 2049)])
+@pytest.mark.parametrize("dtype,sdtype", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32)])
+def test_a_large_scale_at_the_last_key(qfa, Nq, Nk, D, dtype, sdtype):
+    """dO is scaled by what the largest key scale of the head leaves room for: the one that matters comes last, 2^14 times the others,
+    where the scan for it starts another round of 1024 keys.  (Without it dP of that key is 5e8 and dS * scale 3e5: beyond binary16.)"""
+    BH, sm = HEADS[D], 1.0 / math.sqrt(D)
+    assert skv_pass_takes(BH, Nq, Nk, D)
+    g = torch.Generator().manual_seed(Nq + Nk)
+    kv = torch.randn((1, BH, Nk, D), generator=g) * 2.0 ** -6
+    kv[:, :, -1] = 256.0 * (1.0 + 64.0 * kv[:, :, -1])
+    q = (torch.randn((1, BH, Nq, D), generator=g) / 256.0).to(dtype)
+    kv, do = kv.to(dtype), torch.full((1, BH, Nq, D), 2.0 ** -6, dtype=dtype)
+    qd, kvd = q.to(DEV).requires_grad_(True), kv.to(DEV).requires_grad_(True)
+    quant = qfa.asymmetric_quant_per_token(kvd.detach(), scale_dtype=sdtype)
+    o = qfa.quant_flash_attn(qd, kvd, quant, sm)
+    dq, dkv = torch.autograd.grad(o, [qd, kvd], do.to(DEV))
+    assert torch.isfinite(dq).all() and torch.isfinite(dkv).all()
+    pick = [0, BH - 1]
+    q, do, codes, scale, zp, o, dq, dkv = (t.detach()[:, pick].cpu() for t in (q, do, *quant, o, dq, dkv))
+    assert (scale[:, :, -1] > 1000 * scale[:, :, :-1].amax(2)).all()
+    (dq_ref, dkv_ref), (nq, nkv) = oracle.legacy_bwd(q, codes, scale, zp, do, sm, o=o, spread=True)
+    assert_close("dQ", dq, dq_ref, scaled=True, spread=nq)
+    assert_close("dKV", dkv, dkv_ref, scaled=True, spread=nkv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("Nq", [50, 100])
 def test_scales_of_zero_hide_nothing(qfa, Nq, D):
     """Keys whose scales are zero (a scale below binary16's range is stored as one) are keys: what is not finite in dO reaches dQ of its

@@ -1,5 +1,6 @@
 """The shared-KV kernels that expand a tile of keys once per workgroup (forward, dQ), the dKV kernel with resident rows, and
-the backward with its keys split over workgroups, at the sizes where they can go wrong: one key, tiles and blocks of 32, 64
+the backward with its keys split over workgroups, at the sizes where they can go wrong (the backward of 33 to 128 queries in one
+pass has tests of its own; cases here are on both sides of its line): one key, tiles and blocks of 32, 64
 and 128 with one more or one less, two and four waves side by side, one wave without queries, and few heads (splits).
 Many heads make the dispatch take these kernels at small sizes; the first, a middle and the last head are compared with the
 oracle, with the tolerances of helpers.py."""
@@ -11,24 +12,35 @@ import torch
 
 from helpers import COS_TOL, assert_close, max_abs
 from oracle import oracle
-from plans import skv_tile_dq_plan, skv_tile_fwd_plan
+from plans import skv_pass_takes, skv_tile_dq_plan, skv_tile_fwd_plan
 from quant_flash_attn_amd import _lib
 
 DEV = "cuda:0"
 
 # the kernels that forward and backward (dQ) of a case are to reach, at head_dim 64, 128 and 256
 TILES = ["tiles, tiles"] * 3
+PASS = ["tiles, pass per head"] * 2 + TILES[:1]
 CASES = [
     # heads, Nq, Nk, dtype, scale dtype, kernels
-    (512, 33, 1, torch.float16, torch.float16, ["16 queries, tiles", "tiles, 16 queries", "16 queries, 16 queries"]),   # one key
-    (512, 65, 1, torch.float16, torch.float16, TILES),
-    (512, 65, 31, torch.float16, torch.float32, TILES),     # three blocks on four waves, one key less than a block
+    (512, 33, 1, torch.float16, torch.float16, ["16 queries, pass per head", "tiles, pass per head", "16 queries, 16 queries"]),   # one key
+    (512, 65, 1, torch.float16, torch.float16, PASS),
+    (512, 65, 31, torch.float16, torch.float32, PASS),     # three blocks on four waves, one key less than a block
     (300, 200, 33, torch.bfloat16, torch.float16, TILES),   # two workgroups per head, four and three blocks
-    (256, 97, 65, torch.float16, torch.float16, TILES),     # one key more than a tile; resident rows, the last block one query
-    (256, 128, 129, torch.float16, torch.float16, TILES),   # all resident rows, one key more than four waves' tiles
+    (256, 97, 65, torch.float16, torch.float16, TILES[:1] + PASS[1:]),     # one key more than a tile; resident rows, the last block one query
+    (256, 128, 129, torch.float16, torch.float16, TILES[:1] + PASS[1:]),   # all resident rows, one key more than four waves' tiles
     (256, 129, 128, torch.bfloat16, torch.float32, TILES),  # one query more than the resident rows
     (64, 512, 97, torch.float16, torch.float16, TILES),
-    (600, 64, 70, torch.float16, torch.bfloat16, TILES[:2] + ["16 queries, 16 queries"]),
+    (600, 64, 70, torch.float16, torch.bfloat16, PASS[:2] + ["16 queries, 16 queries"]),
+    # the two kernels beside the line of the pass: 257 to 319 heads of 64, more than 1024 heads of 128 with two tiles of keys at most
+    (270, 64, 1, torch.bfloat16, torch.float32, ["16 queries, tiles"] + ["16 queries, 16 queries"] * 2),
+    (270, 65, 31, torch.float16, torch.float16, ["16 queries, tiles", "tiles, 16 queries", "16 queries, 16 queries"]),
+    (300, 64, 70, torch.bfloat16, torch.float16, ["16 queries, tiles", "16 queries, pass per head", "16 queries, 16 queries"]),
+    (270, 97, 65, torch.float16, torch.float16, TILES),
+    (280, 128, 129, torch.float16, torch.float32, TILES),
+    (1100, 64, 1, torch.float16, torch.float16, PASS[:1] + ["tiles, tiles", "16 queries, tiles"]),
+    (1100, 97, 31, torch.bfloat16, torch.float32, PASS[:1] + TILES[1:]),
+    (1100, 128, 65, torch.float16, torch.float16, PASS[:1] + TILES[1:]),
+    (1100, 65, 128, torch.bfloat16, torch.float16, PASS[:1] + TILES[1:]),
     (40, 100, 2001, torch.float16, torch.float16, ["tiles split, 16 queries"] * 3),
     (40, 65, 5001, torch.bfloat16, torch.float16, ["tiles split, tiles split"] * 2 + ["tiles split, 16 queries"]),
     (600, 32, 70, torch.float16, torch.float16, ["16 queries, one pass"] * 2 + ["16 queries, 16 queries"]),
@@ -42,7 +54,8 @@ def _kernels(BH, Nq, Nk, D):
     L, fwd, dq = _lib.lib(), skv_tile_fwd_plan(BH, Nq, Nk, D), skv_tile_dq_plan(BH, Nq, Nk, D)
     parts = [f(1, BH, Nq, Nk, D) for f in (L.qfa_attn_fwd_shared_kv_workspace_bytes, L.qfa_attn_bwd_shared_kv_workspace_bytes)]
     names = ["tiles" if fwd.waves else "16 queries",
-             "one pass" if Nq <= (16 if D == 256 else 32) else "tiles" if dq.waves else "16 queries"]
+             "one pass" if Nq <= (16 if D == 256 else 32) else "pass per head" if skv_pass_takes(BH, Nq, Nk, D) else
+             "tiles" if dq.waves else "16 queries"]
     return ", ".join(n + (" split" if p else "") for n, p in zip(names, parts))
 
 
@@ -77,12 +90,13 @@ def test_tiles_vs_oracle(qfa, BH, Nq, Nk, dtype, sdtype, D):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("D", [64, 128, 256])
-def test_infinite_rows_stay_with_their_queries(qfa, D):
+@pytest.mark.parametrize("D,BH,whole", [(64, 512, True), (64, 300, False), (128, 512, True), (128, 1100, False), (256, 512, False)])
+def test_infinite_rows_stay_with_their_queries(qfa, D, BH, whole):
     """An infinite query or dO row reaches O and dQ of its own query only.  The others may be taken against another reference
     maximum (a wave moves its queries' references together), which rounds their probabilities differently: 2^-11 each, so
     2^-9 of the largest value bounds what two roundings of a weighted sum and of the result can move."""
-    BH, Nq, Nk = 512, 65, 70
+    Nq, Nk = 65, 70
+    assert _kernels(BH, Nq, Nk, D).split(", ")[1] == ("pass per head" if whole else "tiles")
     g = torch.Generator().manual_seed(D)
     kv, q, do = (torch.randn(s, generator=g).to(torch.float16).to(DEV) for s in ((1, BH, Nk, D), (1, BH, Nq, D), (1, BH, Nq, D)))
     codes, scale, zp = qfa.asymmetric_quant_per_token(kv)
