@@ -145,27 +145,43 @@ SkvTilePlan skv_tile_dq_plan(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   return t < limit ? p : SkvTilePlan{0, 1, 0};
 }
 
-// One workgroup per (batch, head) does the whole backward, one on a CU at head_dim 128 and two at 64.  Timed beside the two kernels
-// with their splits in 15000 calls of 128 to 3000 heads, 33 to 128 queries and 16 to 65000 keys: 0.77 of their time in the mean at
-// head_dim 64, 0.73 at 128, at most 1.04 (20 more heads than an edge below, 6000 keys and more).  Left out:
-//   few heads: 64 to 128 heads of 128 take 0.98 to 1.01, up to 1.6 for long sequences, whose keys the others split, and 128 to 139 of
-//     them up to 1.17 beyond 4000 keys; 64 to 319 heads of 64 0.97 to 1.3, 320 to 339 up to 1.21 beyond 2750 keys and 340 to 383 up
-//     to 1.07 beyond 6000;
-//   a few heads more than fill the chip, whose last round is nearly empty while the others split evenly: 257 to 287 of 128 1.02 to
-//     1.06, 288 to 299 up to 1.10 beyond 2000 keys; 513 to 589 of 64 up to 1.18 beyond 2250, 590 to 689 up to 1.07 from there to 3250
-//     (behind a second full round the worst is 0.99);
+// One workgroup per (batch, head) does the whole backward, one on a CU at head_dim 128 and two at 64, and leaves the head's keys
+// unsplit.  Timed beside the two kernels with their splits in 29000 calls of 48 to 6000 heads, 33 to 128 queries and 16 to 65000 keys,
+// it takes 0.79 (head_dim 64) and 0.73 (128) of their time in the mean of what it is given.  Left out:
+//   few heads over long keys, which the others split (95 heads, 117 x 8400 of 64: 308 against 146 us), and with them all calls of
+//     fewer than 320 heads of 64 and 128 of 128, where it would be faster up to about 1500 keys (151 heads, 128 x 24: 7 against 18);
+//   257 to 287 heads of 128, a second round of a few heads: 1.02 to 1.06 over long keys;
 //   thousands of heads of 128 with one or two tiles each: its start weighs more than theirs (1.02).
+// Over long keys 320 to 699 heads of 64 and 128 to 329 of 128 leave a round nearly empty or the first one half full, and which is faster
+// depends on the queries too: there both are estimated.
+namespace {
+// us of the pass: start, a tile, a tile of 1000 heads (the clock falls with the CUs at work; with more than 96 queries `wave4` more), and
+// the second round, its tiles and its start, where there are more heads than workgroups at once
+struct PassCost { float start, tile, heads, wave4, tile2, start2; };
+// of the two kernels, in proportion to 1000 heads but for the start: a tile, that for every 16 queries, every 32, a head, and what a tile
+// takes less with at most 48 queries (the 16-query kernel forms dQ)
+struct TwoCost { float start, tile, q16, q32, head, few; };
+// Fitted to 3900 calls of 64 and 4000 of 128, 1500 to 65000 keys (3 % rms, the two kernels 5).  What it chooses takes 1.003 (64) and 1.000
+// (128) times the better one in the mean of 9000 such calls, more than 1.04 times in 136 and 12, 1.11 at most; the pass always 1.008 and
+// 1.001, 360 and 54, 1.21; edges in heads and keys alone 1.014 and 1.012, 654 and 396, 1.38 (297 heads, 116 x 2560 of 128: 290, 210 us)
+const PassCost kPassHead[2][2] = {{{3.7f, 1.693f, 1.133f, 0.f, 1.467f, -4.2f}, {4.1f, 2.461f, 1.544f, .484f, 1.635f, 3.1f}},
+                                  {{0.9f, 1.283f, 2.816f, 0.f, 1.222f, 5.5f}, {7.3f, 1.705f, 3.374f, .463f, 1.772f, 8.5f}}};
+const TwoCost kTwo[2] = {{21.6f, 3.032f, .085f, 1.487f, -0.7f, .433f}, {35.5f, 5.198f, .478f, 2.281f, -5.1f, .834f}};
+bool pass_pays(int64_t BH, int64_t Nq, int64_t Nk, int D) {
+  const PassCost &p = kPassHead[by_dim(D)][Nq > 64];
+  const TwoCost &w = kTwo[by_dim(D)];
+  const float tiles = (float)((Nk + 63) / 64), heads = 1e-3f * (float)BH;
+  const float pass = p.start + tiles * (p.tile + heads * (p.heads + (Nq > 96 ? p.wave4 : 0.f))) + (BH > (D == 64 ? 512 : 256) ? p.start2 + p.tile2 * tiles : 0.f);
+  const float two = w.start + heads * (w.head + tiles * (w.tile - (Nq <= 48 ? w.few : 0.f) + w.q16 * (float)((Nq + 15) / 16) + w.q32 * (float)((Nq + 31) / 32)));
+  return pass <= 1.01f * two;
+}
+}  // namespace
+
 bool skv_pass_takes(int64_t BH, int64_t Nq, int64_t Nk, int D) {
   if (Nq <= 32 || Nq > 128 || BH > 0x7fffffffLL) return false;
-  if (D == 64) {
-    if (BH < 384) return BH >= 320 && Nk <= (BH < 340 ? 2750 : 6000);
-    if (BH > 512 && BH < 690) return Nk <= 2250 || (BH >= 590 && Nk > 3250);
-    return true;
-  }
-  if (D != 128) return false;
-  if (BH < 140) return BH >= 128 && Nk <= 4000;
-  if (BH > 256 && BH < 300) return BH >= 288 && Nk <= 2000;
-  return Nk > 128 || BH <= 1024;
+  if (D == 64) return BH >= 320 && (BH >= 700 || Nk < 1500 || pass_pays(BH, Nq, Nk, D));
+  if (D != 128 || BH < 128 || (BH > 256 && BH < 288)) return false;
+  return BH < 330 ? Nk < 1500 || pass_pays(BH, Nq, Nk, D) : Nk > 128 || BH <= 1024;
 }
 
 int skv_bwd_splits(int64_t BH, int64_t Nq, int64_t Nk, int D) {
