@@ -30,7 +30,7 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-
 PER_FILE = {f: ["-ffp-contract=off", "-fno-fast-math"] for f in ("qfa_quant.hip", "qfa_cache.hip")}
 # accumulators in AccVGPRs by hand (see qfa_acc.h): other MFMA results in vector registers, and the assembly is checked
 BY_HAND = ("qfa_fwd_wide.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv_pass.hip")
-# MFMA results in vector registers: head_dim 256 with four waves side by side then spills none instead of 5 (dQ) and 6 (forward);
+# MFMA results in vector registers: head_dim 256 with four waves side by side then spills none instead of 5 (dQ) and 1 instead of 4 (forward);
 # elsewhere only the forward of 64 with four waves does, 4 registers, with and without (dKV: no difference in registers)
 PER_FILE["qfa_skv_tile.hip"] = PER_FILE["qfa_skv_dkv.hip"] = PER_FILE["qfa_skv_pass64.hip"] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 for _f in BY_HAND:

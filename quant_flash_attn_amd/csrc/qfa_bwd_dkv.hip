@@ -241,7 +241,7 @@ template <typename T, int D, int KB, bool CAUSAL> __global__ __launch_bounds__(2
     // Turn of the tile: the next one has landed, the one after it goes into the buffer of the previous one, whose last fragments
     // have been requested.  With one step per tile (head_dim 256) the last pieces of a copy have little time until the next turn.
     // Without a mask the turn comes before the first request of dO there, and only the codes and constants of the next tile have to be
-    // there, dO and Qz^T one turn later (the whole backward, 64 heads of 4096: 3069 -> 3027 us; with a mask, where waves begin at
+    // there, dO and Qz^T one turn later (the whole backward, 64 heads of 4096: 2976 -> 2949 us; with a mask, where waves begin at
     // different tiles: 1726 -> 1734)
     TileDesc td;
     auto turn = [&]() __attribute__((always_inline)) {

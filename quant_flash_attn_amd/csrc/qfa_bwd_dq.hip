@@ -17,8 +17,8 @@
 // take longer than its products.  Bound by the instructions a wave can issue (74 vector instructions beside 21 MFMAs of 32
 // cycles per 32 x 32 block; matrix pipe busy 72 % at 1.85 GHz on the long sequence below, 54 % on the causal one), then by power.
 // Measured, this kernel alone against the one before it (32 queries per wave, scheduled by the compiler, no bias trick):
-// 16384 x 16384, 16 heads of 128: 2890 -> 2200 us; 4096 causal, 128 heads of 128: 789 -> 650; 64 heads of 256: 1276 -> 671;
-// 2048 causal, 256 heads of 64: 251 -> 226.
+// 16384 x 16384, 16 heads of 128: 2890 -> 2200 us; 4096 causal, 128 heads of 128: 789 -> 650; 64 heads of 256: 1276 -> 789
+// (less since: see the turn of the tile); 2048 causal, 256 heads of 64: 251 -> 226.
 #include <type_traits>
 
 #include "qfa_acc.h"
@@ -249,7 +249,7 @@ template <typename T, int D, int QB, bool CAUSAL> __global__ __launch_bounds__(2
     // there (dQ of 16384 x 16384, 16 heads of 128: 2273 -> 2246 us against a turn behind them, 4096 causal 671 -> 666).  With one
     // step per tile (head_dim 256) the last pieces of a copy have 15 products' time until the next turn, and the wave waited for
     // them (42 % of its time): there only the codes and constants of the next tile have to be there, V and Kz^T one turn later.
-    // 64 heads of 4096 causal: 818 -> 704 us; the whole backward without a mask 3386 -> 3045 us
+    // 64 heads of 4096 causal: 818 -> 704 us; the whole backward without a mask 3394 -> 2976 us
     auto turn = [&]() __attribute__((always_inline)) {
       vm_wait<PIECES - FIRST>();
       lds_barrier();

@@ -12,7 +12,7 @@
 // The kernel before it copied and summed the rows once per 128 keys, met at two barriers per 32 queries (52 % of its time was
 // waiting) and removed the codes' offset by two more MFMAs per block.  Measured, that one -> this (us, one GPU): 5247 heads, 97 x 689
 // 941 -> 668 at head_dim 128, 497 -> 327 at 64; 512 heads, 512 x 4096 1565 -> 1180 and 842 -> 599.  Up to 64 queries it had its rows
-// resident too and was 7 to 9 % faster at 128 (1470 heads, 47 x 2737: 532 against 572).
+// resident too and was 7 to 9 % faster at 128 (1470 heads, 47 x 2737: 532 against 572; so many heads go to qfa_skv_pass.hip now).
 // What bounds it: at 512 queries the matrix pipe is busy 45 % at 1.89 GHz, issue stalls 37 %; the S and dP of the next block
 // beside the vector work of this one (32 registers more) changed nothing.  At 97 x 689 it is busy 33 % with 41 % waits: 16 KB
 // of rows and 16 KB transposed out of LDS for 32 products, and the last block of 32 queries holds one.
