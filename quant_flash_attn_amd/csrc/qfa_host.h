@@ -131,6 +131,7 @@ int launch_skv_tile_dq(const SkvAttnArgs &a, const SkvTilePlan &p, hipStream_t s
 int launch_skv_dkv(const SkvAttnArgs &a, hipStream_t st);
 // dQ and dKV of 33 to 128 queries in one pass (head_dim 64 and 128): a workgroup per head, where there are enough of them
 bool skv_pass_takes(int64_t BH, int64_t Nq, int64_t Nk, int D);
+bool skv_pass_takes_unsplit(int64_t BH, int64_t Nq, int64_t Nk, int D);   // ... of a call without scratch
 // ... if the offsets of a head's rows, those of a few tiles past its end included, fit 31 bits
 inline bool skv_pass_fits(int64_t Nk, int64_t scn, int64_t sdqn, int64_t sdkn) {
   const int64_t rows = Nk + 512, most = 1 << 23;

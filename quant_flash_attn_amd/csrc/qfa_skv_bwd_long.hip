@@ -653,8 +653,8 @@ template <typename S, int D> static int launch_skv_bwd_long_sd(const SkvAttnArgs
 }
 
 int launch_skv_bwd_long(const SkvAttnArgs &x, hipStream_t st) {
-  if (skv_pass_takes(x.B * x.H, x.Nq, x.Nk, x.D) && skv_pass_fits(x.Nk, x.scn, x.sdqn, x.sdkn))
-    return launch_skv_pass(x, st);
+  const bool pass = x.workspace ? skv_pass_takes(x.B * x.H, x.Nq, x.Nk, x.D) : skv_pass_takes_unsplit(x.B * x.H, x.Nq, x.Nk, x.D);
+  if (pass && skv_pass_fits(x.Nk, x.scn, x.sdqn, x.sdkn)) return launch_skv_pass(x, st);
   const bool s32 = x.scale_dtype == QFA_F32;
   if (x.D == 256) return s32 ? launch_skv_bwd_long_sd<float, 256>(x, st) : launch_skv_bwd_long_sd<_Float16, 256>(x, st);
   if (x.D == 128) return s32 ? launch_skv_bwd_long_sd<float, 128>(x, st) : launch_skv_bwd_long_sd<_Float16, 128>(x, st);

@@ -40,3 +40,7 @@ def skv_tile_dq_plan(BH, Nq, Nk, D):
 
 def skv_pass_takes(BH, Nq, Nk, D):
     return _plan("_ZN3qfa14skv_pass_takesEllli", ctypes.c_bool, [_L, _L, _L, _I])(BH, Nq, Nk, D)
+
+
+def skv_pass_takes_unsplit(BH, Nq, Nk, D):
+    return _plan("_ZN3qfa22skv_pass_takes_unsplitEllli", ctypes.c_bool, [_L, _L, _L, _I])(BH, Nq, Nk, D)

@@ -9,7 +9,7 @@ import torch
 
 from helpers import COS_TOL, assert_close
 from oracle import oracle
-from plans import skv_pass_takes, skv_tile_dq_plan
+from plans import skv_pass_takes, skv_pass_takes_unsplit, skv_tile_dq_plan
 from quant_flash_attn_amd import _lib
 
 DEV = "cuda:0"
@@ -56,6 +56,34 @@ def test_choice_is_not_slower(qfa, BH, Nq, Nk, D, us):
     of the two are off together: 3 and 5 % rms, 8 %."""
     takes = skv_pass_takes(BH, Nq, Nk, D)
     assert us[0 if takes else 1] <= 1.08 * us[1 if takes else 0]
+
+
+@pytest.mark.parametrize("BH,Nq,Nk,D,split", [(355, 85, 13075, 64, True), (130, 60, 23096, 128, True), (521, 40, 5877, 64, False),
+                                              (270, 100, 8000, 128, False), (300, 100, 8000, 64, False), (512, 129, 8000, 64, False)])
+def test_without_scratch(qfa, BH, Nq, Nk, D, split):
+    """A call that would go to the two kernels for their split goes to the one pass if it brings no scratch; others do not."""
+    assert not skv_pass_takes(BH, Nq, Nk, D) and (Nq > 128 or not split or skv_tile_dq_plan(BH, Nq, Nk, D).splits > 1)
+    assert skv_pass_takes_unsplit(BH, Nq, Nk, D) == split
+    assert skv_pass_takes_unsplit(BH, 64, 500, D) == skv_pass_takes(BH, 64, 500, D)
+
+
+@pytest.mark.gpu
+def test_with_and_without_scratch(qfa):
+    """The autograd entry, which brings scratch, and the public call, which does not, take different kernels: both against the oracle."""
+    BH, Nq, Nk, D, sm = 330, 72, 8500, 64, 0.125
+    assert not skv_pass_takes(BH, Nq, Nk, D) and skv_pass_takes_unsplit(BH, Nq, Nk, D)
+    q, kv, do, qd, kvd, dod = _case(BH, Nq, Nk, D, torch.float16, torch.float16, "heads")
+    quant = qfa.asymmetric_quant_per_token(kvd)
+    o, lse = qfa.attn_fwd_shared_kv(qd, *quant, sm)
+    got = {"public": qfa.attn_bwd_shared_kv(qd, *quant, o, dod, lse, sm)}
+    leaves = qd.requires_grad_(True), kvd.requires_grad_(True)
+    got["autograd"] = torch.autograd.grad(qfa.quant_flash_attn(*leaves, quant, sm), leaves, dod)
+    assert not torch.equal(got["public"][0], got["autograd"][0])
+    pick = [0, BH // 2, BH - 1]
+    refs, spreads = oracle.legacy_bwd(*(t[:, pick].detach().cpu() for t in (q, *quant, do)), sm, o=o[:, pick].cpu(), spread=True)
+    for name, grads in got.items():
+        for a, b, n in zip(grads, refs, spreads):
+            assert_close(name, a[:, pick].cpu(), b, scaled=True, spread=n)
 
 
 def _case(BH, Nq, Nk, D, dtype, sdtype, layout):
