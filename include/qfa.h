@@ -228,8 +228,9 @@ int qfa_attn_fwd_shared_kv_static(const void *q, const int8_t *codes, const void
  * _bwd_preprocess_kernel (:87-101; delta is computed inside) and _attn_bwd_kernel_quantized
  * (:104-166), which also stores the single gradient dKV = dV + dK (:161).  Up to 32 queries per
  * (batch, head) run in one fused pass (one workgroup per (batch, head) streams the codes once and
- * writes each dKV row once); longer query blocks run a dQ kernel (one workgroup per 16 queries) and
- * a dKV kernel (one workgroup per 128 keys walking over the queries).
+ * writes each dKV row once), and so do 33 to 128 of many heads of 64 or 128; longer query blocks run a
+ * dQ kernel (a workgroup per 16, 64 or 128 queries) and a dKV kernel (a workgroup per 128 keys or more,
+ * walking over the queries).
  *   q, o, dout [B,H,Nq,D] fp16 (io_dtype must be QFA_F16: the kernels compute in binary16), strides as given;
  *   dq [B,H,Nq,D], dkv [B,H,Nk,D] of grad_dtype (QFA_F16 or QFA_BF16);
  *   grad_scale  nullable DEVICE pointer to one float that multiplies dq and dkv before they are rounded.

@@ -73,8 +73,8 @@ def attn_bwd_shared_kv(q: torch.Tensor, codes: torch.Tensor, scale: torch.Tensor
     [B,H,Nq,D] (the kernels compute in binary16); lse as returned by the forward.  dQ and dKV come back
     in `grad_dtype` (fp16 by default, or bf16), multiplied by the one-element device tensor `grad_scale`
     if given.  Up to 32 queries (16 at head_dim 256), and 33 to 128 of many heads of 64 or 128, run in one
-    fused pass over the codes, longer blocks in a dQ kernel plus a dKV kernel.  The keys are not split over workgroups here (`quant_flash_attn`'s backward does where
-    there are few heads)."""
+    fused pass over the codes, longer blocks in a dQ kernel plus a dKV kernel.  The keys are not split over
+    workgroups here (`quant_flash_attn`'s backward does where there are few heads)."""
     return _lib.host().skv_bwd(q, codes, scale, zero_point, o, do, lse, float(sm_scale), grad_dtype or torch.float16,
                                grad_scale)
 
