@@ -3,8 +3,9 @@
 Their inline MFMAs name AccVGPRs that the compiler does not know to hold anything between two statements, and it does not
 see these MFMAs' hazards.  So the build looks at what it made of them:
 
-  1. no instruction of the compiler's touches a register that inline assembly uses as an AccVGPR, between the statements
-     or anywhere else in the kernel (it may use the others);
+  1. no instruction of the compiler's touches a register that holds an accumulator of inline assembly, between the statements or
+     anywhere else, and none reads one that inline assembly has overwritten (it may use the others, and in a part of the kernel that
+     shares no path with these statements all);
   2. a vector instruction that writes A or B of an inline MFMA is followed by at least two wait states before it, and one that
      writes an accumulator likewise;
   3. an accumulator is read, or written by a vector instruction, no earlier than 20 wait states behind an MFMA that writes it;
@@ -21,7 +22,7 @@ from typing import Dict, List, NamedTuple, Set, Tuple
 VALU_TO_MFMA = 2     # wait states between a vector instruction and an MFMA that reads what it wrote
 MFMA_TO_VALU = 20    # ... between a 32x32 MFMA (16 passes) and a vector instruction on its result
 
-_REG = re.compile(r"\b([va])(?:(\d+)\b|\[(\w+):(\w+)\])")
+_REG = re.compile(r"\b([va])(?:(\d+)\b|\[(\w+)(?::(\w+))?\])")
 
 
 class Instr(NamedTuple):
@@ -40,7 +41,7 @@ def _regs(text: str) -> Set[Tuple[str, int]]:
         if m.group(2) is not None:
             out.add((m.group(1), int(m.group(2))))
         else:
-            out |= {(m.group(1), r) for r in range(int(m.group(3), 0), int(m.group(4), 0) + 1)}
+            out |= {(m.group(1), r) for r in range(int(m.group(3), 0), int(m.group(4) or m.group(3), 0) + 1)}
     return out
 
 
@@ -101,6 +102,32 @@ def check(path: str) -> List[str]:
             if i.target in labels:
                 before.setdefault(labels[i.target], []).append(k)
 
+        # For each instruction, as bits: the accumulators that inline assembly may read from there on before it writes them anew, and those
+        # that it has written since the compiler last did, on any path.  (A kernel may hold two loops of which a workgroup runs one:
+        # registers of one are the compiler's in the other.)
+        after: Dict[int, List[int]] = {}
+        for k, ps in before.items():
+            for p in ps:
+                after.setdefault(p, []).append(k)
+        bits = lambda regs: sum(1 << n for kind, n in regs if kind == "a")  # noqa: E731
+        reads, writes = [bits(i.reads & acc) for i in ins], [bits(i.writes & acc) for i in ins]
+
+        def flow(gen: List[int], kill: List[int], to: Dict[int, List[int]], order) -> List[int]:
+            """What arrives at each instruction: gen and whatever arrived without kill goes on along the edges."""
+            arrived, todo = [0] * len(ins), list(order)
+            while todo:
+                k = todo.pop()
+                out = gen[k] | arrived[k] & ~kill[k]
+                for n in to.get(k, []):
+                    if out & ~arrived[n]:
+                        arrived[n] |= out
+                        todo.append(n)
+            return arrived
+
+        by_asm = lambda x: [b if i.inline else 0 for b, i in zip(x, ins)]   # noqa: E731
+        wanted = flow(by_asm(reads), by_asm(writes), before, range(len(ins)))
+        dirty = flow(by_asm(writes), [0 if i.inline else w for w, i in zip(writes, ins)], after, reversed(range(len(ins))))
+
         def written_within(k: int, regs, states: int, writer) -> bool:
             """Is there a path on which an instruction `writer` accepts writes one of `regs` fewer than `states` before k?"""
             todo, seen = [(p, states) for p in before.get(k, [])], {}
@@ -118,7 +145,7 @@ def check(path: str) -> List[str]:
         valu = lambda i: i.op.startswith("v_") and not mfma(i)              # noqa: E731
         for k, i in enumerate(ins):
             used = i.reads | i.writes
-            if not i.inline and used & acc:
+            if not i.inline and ((reads[k] | writes[k]) & wanted[k] or reads[k] & dirty[k]):
                 tell(i, "the compiler uses an accumulator's register")
             if i.inline and mfma(i):
                 if written_within(k, i.reads | i.writes, VALU_TO_MFMA, valu):

@@ -70,3 +70,18 @@ def test_the_library_as_built(src):
     assert acc_check.check(asm) == []
     text = open(asm).read()
     assert text.count("_kernel") > 0 and "ASMSTART" in text
+
+
+def test_a_register_named_in_brackets(tmp_path):
+    assert _kernel(tmp_path, "!" + MFMA, "!v_accvgpr_read_b32 v9, a[3]")
+    assert not _kernel(tmp_path, "!" + MFMA, "!v_accvgpr_read_b32 v9, a[16]")
+
+
+def test_two_loops_of_which_a_workgroup_runs_one(tmp_path):
+    """The second one's accumulators are the compiler's in the first, also where a path leads on from it, as long as they begin anew."""
+    other = "v_mfma_f32_32x32x16_bf16 a[16:31], v[0:3], v[4:7], a[16:31]"
+    zero = [f"!v_accvgpr_write_b32 a[{r}], 0" for r in range(16, 32)]
+    first = ["s_cbranch_scc1 .LBB0_2", "v_accvgpr_write_b32 a16, v9", "s_nop 1", "!" + MFMA, "v_accvgpr_read_b32 v9, a16"]
+    assert not _kernel(tmp_path, *first, ".LBB0_2:", *zero, "s_nop 1", "!" + other)
+    assert _kernel(tmp_path, *first, ".LBB0_2:", *zero[1:], "s_nop 1", "!" + other)
+    assert _kernel(tmp_path, *first[:-1], "!" + zero[0][1:], first[-1])   # the compiler's value is gone
