@@ -29,13 +29,14 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-
 # whatever quantizes must evaluate its expressions as single IEEE operations (bit-exact codes)
 PER_FILE = {f: ["-ffp-contract=off", "-fno-fast-math"] for f in ("qfa_quant.hip", "qfa_cache.hip")}
 # accumulators in AccVGPRs by hand (see qfa_acc.h): other MFMA results in vector registers, and the assembly is checked
-BY_HAND = ("qfa_fwd_wide.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv_pass.hip")
+_BWD_PAIR = tuple(f"qfa_bwd_pair_{x}.hip" for x in ("128_bf16", "128_f16", "256_bf16", "256_f16", "64_bf16", "64_f16"))
+BY_HAND = ("qfa_fwd_wide.hip", *_BWD_PAIR, "qfa_skv_pass.hip")
 # MFMA results in vector registers: head_dim 256 with four waves side by side then spills none instead of 5 (dQ) and 1 instead of 4 (forward);
 # elsewhere only the forward of 64 with four waves does, 4 registers, with and without (dKV: no difference in registers)
 PER_FILE["qfa_skv_tile.hip"] = PER_FILE["qfa_skv_dkv.hip"] = PER_FILE["qfa_skv_pass64.hip"] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 for _f in BY_HAND:
     PER_FILE[_f] = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_fwd_wide.hip", "qfa_split_plan.cpp", "qfa_bwd.hip", "qfa_bwd_dkv.hip", "qfa_bwd_dq.hip", "qfa_skv_plan.cpp", "qfa_skv.hip", "qfa_skv_tile.hip", "qfa_skv_dkv.hip", "qfa_skv_pass.hip", "qfa_skv_pass64.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
+SOURCES = ["qfa_api.cpp", "qfa_quant.hip", "qfa_fwd.hip", "qfa_fwd_wide.hip", "qfa_split_plan.cpp", "qfa_bwd.hip", *_BWD_PAIR, "qfa_skv_plan.cpp", "qfa_skv.hip", "qfa_skv_tile.hip", "qfa_skv_dkv.hip", "qfa_skv_pass.hip", "qfa_skv_pass64.hip", "qfa_skv_bwd.hip", "qfa_skv_bwd_long.hip",
            "qfa_cache.hip"]
 
 

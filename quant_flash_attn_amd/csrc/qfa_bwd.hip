@@ -1,18 +1,18 @@
-// Backward for gfx950: the staging passes here, then two MFMA kernels that recompute P = exp(S - LSE) from the INT8 codes
-// exactly as the forward does.
+// Backward for gfx950: the staging passes here, then one launch of two kinds of workgroups (qfa_bwd_pair.h) that recompute
+// P = exp(S - LSE) from the INT8 codes exactly as the forward does.
 //
 //   prep_q       per 64-query tile: delta = rowsum(O o dO) in fp32; Qz^T = ((Qc - zq) * sq)^T as a
 //                16-bit tile [d][query] in the key order the MFMA layouts want; per-query constants
 //   prep_k       per 64-key tile: Kz^T = ((Kc - zk) * sk)^T likewise; per-key constants
 //                (both write into the caller's workspace; every tile is converted and transposed
 //                once instead of once per consuming workgroup)
-//   dK / dV      qfa_bwd_dkv.hip: a workgroup owns keys and streams query tiles
-//   dQ           qfa_bwd_dq.hip: a workgroup owns queries and streams key tiles
+//   dK / dV      qfa_bwd_dkv.inc: a workgroup owns keys and streams query tiles
+//   dQ           qfa_bwd_dq.inc: a workgroup owns queries and streams key tiles
 // In both, the wave's own operand (queries resp. keys) stays in registers as the MFMA B operand
 // for the whole loop and the streamed operand comes from LDS as the A operand.  The 32x32
 // accumulator layout then leaves P / dS in registers exactly in the B-operand layout of the next
 // product; the transposed tiles (Kz^T, Qz^T) are written in the matching permuted order.
-// dQ is produced by its own kernel instead of atomics, so results are deterministic.
+// dQ is produced by workgroups of its own instead of atomics, so results are deterministic.
 // The scales of the streamed operand are folded into its transposed 16-bit tile (Kz^T, Qz^T) by the staging
 // pass, so dS is used as it comes: the tiles then hold the dequantized K and Q rounded to the 16-bit type, the
 // operands an unquantized backward would use.
@@ -350,13 +350,13 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
     k.split_stride = x.Nk * D;
     k.grad_f32 = 1;
   }
-  if (int e = launch_dkv<T, D>(k, BH, x.causal, plan.blocks_dkv, plan.splits_dkv, st)) return e;
   auto add_parts = [&]() -> int {
     if (sum.count == 0) return 0;
     bwd_sum_kernel<T, D><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(sum);
     return check_launch("qfa_attn_bwd (sum)");
   };
   if (plan.sum_between) {   // dQ's parts take the place of these
+    if (int e = launch_bwd_pair<T, D>(k, plan.blocks_dkv, plan.splits_dkv, a, plan.blocks_dq, 0, BH, x.causal, st)) return e;
     if (int e = add_parts()) return e;
     part = parts;
     sum.count = 0;
@@ -371,7 +371,7 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
     q.split_stride = x.Nq * D;
     q.grad_f32 = 1;
   }
-  if (int e = launch_dq<T, D>(q, BH, x.causal, plan.blocks_dq, plan.splits_dq, st)) return e;
+  if (int e = launch_bwd_pair<T, D>(k, plan.blocks_dkv, plan.sum_between ? 0 : plan.splits_dkv, q, plan.blocks_dq, plan.splits_dq, BH, x.causal, st)) return e;
   return add_parts();
 }
 

@@ -1,5 +1,5 @@
 // Workspace layout, arguments and small helpers shared by the backward kernels (qfa_bwd.hip: staging passes;
-// qfa_bwd_dkv.hip: dK / dV; qfa_bwd_dq.hip: dQ).
+// qfa_bwd_pair.h: dK, dV and dQ).
 #pragma once
 #include "qfa_device.h"
 #include "qfa_host.h"
@@ -56,7 +56,7 @@ template <int D> __device__ __forceinline__ int qt_offset(int d, int pos) {
   return (pos / 16 * (D / 32) + d / 32) * 1024 + d % 32 * 32 + (((pos / 8) % 2 ^ (d / 8) % 2) << 4) + pos % 8 * 2;
 }
 
-// ---- slab layout of row tiles in LDS (see the head of qfa_bwd_dkv.hip)
+// ---- slab layout of row tiles in LDS (see the head of qfa_bwd_dkv.inc)
 template <int D> struct BwdSlab {
   static constexpr int SLAB = BwdWs<D>::TILE * 32 + 128;   // bytes between slabs
 };
@@ -100,8 +100,9 @@ template <int T_BYTES, int C_COPY> struct BlobCopy {
   }
 };
 
-// blocks: 32-row blocks per wave (2 only at head_dim 128); splits: parts of the streamed rows (grid.y)
-template <typename T, int D> int launch_dkv(BwdArgs a, int64_t BH, bool causal, int blocks, int splits, hipStream_t st);
-template <typename T, int D> int launch_dq(BwdArgs a, int64_t BH, bool causal, int blocks, int splits, hipStream_t st);
+// dK and dV by `dkv`, dQ by `dq`, either of them or both in one launch (qfa_bwd_pair.h).  blocks: 32-row blocks per wave (2 only at
+// head_dim 128), splits: parts of the streamed rows; 0: that part is not wanted
+template <typename T, int D>
+int launch_bwd_pair(const BwdArgs &dkv, int blocks_dkv, int splits_dkv, const BwdArgs &dq, int blocks_dq, int splits_dq, int64_t BH, bool causal, hipStream_t st);
 
 }  // namespace qfa

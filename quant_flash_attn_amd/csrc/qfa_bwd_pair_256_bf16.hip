@@ -1,0 +1,6 @@
+// The backward's kernel at head_dim 256, bf16 (one instance per file: each takes minutes to compile)
+#include "qfa_bwd_pair.h"
+
+namespace qfa {
+template int launch_bwd_pair<__bf16, 256>(const BwdArgs &, int, int, const BwdArgs &, int, int, int64_t, bool, hipStream_t);
+}  // namespace qfa

@@ -3,7 +3,7 @@
 //
 // A workgroup is 4 waves; a wave owns QB blocks of 32 queries, whose O^T accumulators live in AccVGPRs by hand (qfa_acc.h).
 // Keys stream through LDS in tiles of 64, three buffers, one barrier per tile; the LDS layout is the slab layout of the
-// backward kernels (qfa_bwd_dkv.hip).  A step (32 keys) is one straight line whose MFMAs come in the order
+// backward kernels (qfa_bwd_dkv.inc).  A step (32 keys) is one straight line whose MFMAs come in the order
 //     P.V of the previous step, all but its last fragment  |  S of the next step  |  last fragment of P.V
 // with the vector work of this step's P dealt to them at an even pace.  Every LDS request is issued three fragments before
 // its use, behind the compiler's back, and waited for by count (LDS returns in order).
@@ -139,7 +139,7 @@ template <typename T, int D, int QB, bool CAUSAL, bool SPLIT> __global__ __launc
   store_kc(0);
   load_kc(1);
 
-  // ---- per-lane read offsets (see qfa_bwd_dkv.hip): rows, transposing reads
+  // ---- per-lane read offsets (see qfa_bwd_dkv.inc): rows, transposing reads
   const int row_l = slab_row(lr, g);
   const int s16 = lane % 16, u16 = (lane / 16) % 2;
   const int tr_l = u16 * SLAB + (4 * g + s16 / 4) * 32 + ((s16 % 4) / 2) * 16 + (s16 % 2) * 8;

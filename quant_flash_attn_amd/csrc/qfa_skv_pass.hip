@@ -10,7 +10,7 @@
 // AccVGPRs for the whole kernel.  So a code is expanded once, and S, dP and the exponentials are formed once, where the two kernels
 // (skv_tile_dq_kernel, skv_dkv_kernel) do all of it twice: 5 products per pair of query and key instead of 7.
 //
-// One wave per SIMD, written out as in qfa_bwd_dq.hip.  A step (32 keys per wave) is one straight line of MFMAs in the order
+// One wave per SIMD, written out as in qfa_bwd_dq.inc.  A step (32 keys per wave) is one straight line of MFMAs in the order
 //     dQ of the previous step and, in turn, S and dP of the next one  |  dKV of the previous tile
 // and the vector work of this step's P and dS, the expansion of the tile after the next and the way of the finished dKV rows to
 // memory are dealt to them, so that no product waits for the vector work it depends on.  One barrier per tile: four or five buffers

@@ -1,5 +1,5 @@
 // Into how many parts the streamed rows of the INT8-score kernels are dealt: the keys of the forward (qfa_fwd.hip,
-// qfa_fwd_wide.hip) and of dQ (qfa_bwd_dq.hip), the queries of dK and dV (qfa_bwd_dkv.hip).
+// qfa_fwd_wide.hip) and of dQ (qfa_bwd_dq.inc), the queries of dK and dV (qfa_bwd_dkv.inc).
 //
 // A workgroup is a chain of tiles whose pace hardly depends on what the rest of the chip does, so few rows against many take the
 // time of one chain while the other CUs idle (forward, 4 heads, 333 queries, 30000 keys of 128: 12 workgroups, 458 us; their
