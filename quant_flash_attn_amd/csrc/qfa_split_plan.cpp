@@ -190,6 +190,101 @@ static void bwd_part(int64_t BH, int64_t rows, int64_t streamed, int D, bool cau
   *per_split = (int)each;
 }
 
+// ---- both kinds of workgroups in one launch (qfa_bwd_pair.h)
+// Each kind by itself is planned above; together they leave less idle, so parts that fill the chip for one alone can be too many, and
+// wide blocks too few no longer.  The estimate: where all workgroups run at once, the longest and a share of the mean load (they
+// slow each other down); otherwise the mean load and what is left of the last dQ workgroup, or again the longest.  Fitted to 7100 shapes
+// of 1 to 400 heads, 64 to 8192 keys, causal or not, with up to 29 divisions of both kinds each.  Only a division that it promises
+// to be a tenth faster than the plan is taken: of 8300 more shapes 900 move, to 0.90, 0.89 and 0.87 of the time in the mean (head_dim 64,
+// 128, 256), eight of them to more than 1.04 times (1.14 at most: 7 heads of 4116 x 128, 218 -> 249 us); taken whenever it is the
+// fastest, 5 in a hundred of all calls at 128 would take more than 1.04 times.  8 heads of 1702 x 128 causal 73 -> 57 us,
+// 2 x 1936 x 256 78 -> 56.
+struct PairCost {
+  double base, prep, sum, mb;   // us: launches; staging per MB (10^6 elements); the sum of parts and what it takes per MB
+  double start[2], tail;        // of a workgroup of dK / dV and of dQ, in tiles; share of the last one that runs alone
+  double tile[2][2];            // us per tile: [dK / dV, dQ][32, 64 rows per wave; at head_dim 64 one, two workgroups per CU]
+  double crowd, over;           // share of the mean load beside the longest workgroup, within one round and beyond
+};
+constexpr int64_t SUM_BETWEEN = 128 << 20;   // of parts: more of both, and they are added between two launches
+struct Share { int blocks, splits, each; double n, tiles, last, mbytes; };   // workgroups, tiles of all, of the longest
+
+static double pair_time(const PairCost &c, int D, const Share &kv, const Share &q) {
+  const double slots = D == 64 ? 512.0 : 256.0, n = kv.n + q.n;
+  const double tk = c.tile[0][D == 64 ? n > 256.0 : kv.blocks - 1], tq = c.tile[1][D == 64 ? n > 256.0 : q.blocks - 1];
+  const double ek = (kv.last + c.start[0]) * tk, eq = (q.last + c.start[1]) * tq, longest = std::max(ek, eq);
+  const double mean = ((kv.tiles + kv.n * c.start[0]) * tk + (q.tiles + q.n * c.start[1]) * tq) / slots, mb = kv.mbytes + q.mbytes;
+  const double body = n <= slots ? longest + c.crowd * mean : std::max(mean + c.tail * eq, longest + c.over * mean);
+  return body + (mb > 0.0 ? c.sum + c.mb * mb : 0.0);
+}
+
+// divisions of one kind that are worth an estimate, the plan's own first; returns how many
+constexpr int MAX_SHARES = 23;
+static int shares(int64_t BH, int64_t rows, int64_t streamed, int D, bool causal, bool ends, int64_t coff, int tensors, int blocks, int splits,
+                  int each, Share *out) {
+  static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24};
+  const int64_t tiles = (streamed + 63) / 64;
+  int found = 0;
+  SplitWork w;
+  auto work = [&](int r) {
+    w = {BH, (rows + 128 * r - 1) / (128 * r), 128 * r, streamed, 32, coff, causal, ends, bwd_group_log2(streamed, D, ends)};
+    w.count();
+  };
+  auto add = [&](int r, int64_t s, int64_t e) {
+    Share &x = out[found++];
+    x.blocks = r; x.splits = (int)s; x.each = (int)e;
+    w.first_xcd(s, e, &x.n, &x.tiles);
+    x.n *= 8.0;
+    x.tiles *= 8.0;
+    x.last = std::min(w.longest, (double)(e / 32));
+    x.mbytes = s > 1 ? 8e-6 * (double)(BH * rows * s) * D * tensors : 0.0;
+  };
+  work(blocks);
+  add(blocks, splits, each);
+  for (int r = 1; r <= (D == 128 ? 2 : 1); ++r) {
+    work(r);
+    int64_t last = 0;
+    for (const int64_t s : counts) {
+      const int64_t e = (tiles + s - 1) / s, real = (tiles + e - 1) / e;
+      if (real == last || (real > 1 && (BH * w.blocks * real > 600 || BH * rows * D * tensors * real > MAX_PART_FLOATS))) continue;
+      last = real;
+      add(r, real, e * 64);
+    }
+  }
+  return found;
+}
+
+static void plan_pair(int64_t BH, int64_t Nq, int64_t Nk, int D, bool causal, BwdPlan *p) {
+  static const PairCost cost[3][2] = {   // [head_dim 64, 128, 256][causal]
+      {{8.73, 0.496, 3.04, 0.196, {2.45, 5.76}, 0.739, {{0.647, 0.649}, {0.324, 0.409}}, 0.333, 0.167},
+       {7.42, 0.435, 3.08, 0.162, {7.66, 8.85}, 0.797, {{0.506, 0.491}, {0.324, 0.368}}, 0.508, 0.232}},
+      {{8.99, 0.352, 3.34, 0.145, {5.54, 7.33}, 0.646, {{0.814, 1.36}, {0.474, 0.745}}, 0.172, 0.0225},
+       {9.07, 0.353, 3.17, 0.145, {8.54, 7.68}, 0.551, {{0.661, 1.09}, {0.451, 0.738}}, 0.184, -0.0585}},
+      {{4.44, 0.268, 5.36, 0.139, {9.65, 6.67}, 0.545, {{1.25, 0}, {0.949, 0}}, 0.038, -0.047},
+       {4.04, 0.24, 4.86, 0.137, {13.2, 8}, 0.522, {{1.06, 0}, {0.872, 0}}, 0.0869, -0.0534}}};
+  const auto two_launches = [](const Share &a, const Share &b) { return a.splits > 1 && b.splits > 1 && 5e5 * (a.mbytes + b.mbytes) > SUM_BETWEEN; };
+  if (BH > MAX_WGS_BWD || BH * ((Nq + 127) / 128 + (Nk + 127) / 128) > MAX_WGS_BWD) return;
+  const PairCost &c = cost[D == 64 ? 0 : D == 128 ? 1 : 2][causal];
+  Share kv[MAX_SHARES], q[MAX_SHARES];
+  const int nkv = shares(BH, Nk, Nq, D, causal, false, Nk - Nq, 2, p->blocks_dkv, p->splits_dkv, p->queries_per_split, kv);
+  const int nq = shares(BH, Nq, Nk, D, causal, true, Nk - Nq, 1, p->blocks_dq, p->splits_dq, p->keys_per_split, q);
+  // (of parts this large each kind fills the chip by itself: 2 heads, 7500 to 8000 of 256, causal, lost 3 to 5 % by the estimate)
+  if (kv[0].splits > 1 && q[0].splits > 1 && 5e5 * (kv[0].mbytes + q[0].mbytes) > SUM_BETWEEN * 5 / 8) return;
+  const double fixed = c.base + c.prep * 1e-6 * (double)BH * D * (double)(7 * Nq + 3 * Nk);
+  double best = 0.9 * (fixed + pair_time(c, D, kv[0], q[0])) - fixed;
+  const Share *bk = &kv[0], *bq = &q[0];
+  for (int i = 0; i < nkv; ++i)
+    for (int j = 0; j < nq; ++j) {
+      const double t = pair_time(c, D, kv[i], q[j]);
+      if (t < best && !two_launches(kv[i], q[j])) {
+        best = t;
+        bk = &kv[i];
+        bq = &q[j];
+      }
+    }
+  p->blocks_dkv = bk->blocks; p->splits_dkv = bk->splits; p->queries_per_split = bk->each;
+  p->blocks_dq = bq->blocks; p->splits_dq = bq->splits; p->keys_per_split = bq->each;
+}
+
 BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_split) {
   // [head_dim][32-row blocks per wave], in tiles of 32 rows
   static const SplitCost dkv64[2] = {{{0.522, 0.590, 0}, 2, 0.462, 0.662, 2.96, 0.186, 0}, {}},
@@ -204,11 +299,12 @@ BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_
            &p.splits_dkv, &p.queries_per_split);
   bwd_part(BH, Nq, Nk, D, causal, true, Nk - Nq, f, may_split, D == 64 ? dq64 : D == 128 ? dq128 : dq256, 1, &p.blocks_dq, &p.splits_dq,
            &p.keys_per_split);
+  if (may_split) plan_pair(BH, Nq, Nk, D, causal != 0, &p);
   const int64_t kv = p.splits_dkv > 1 ? BH * D * 8 * Nk * p.splits_dkv : 0, q = p.splits_dq > 1 ? BH * D * 4 * Nq * p.splits_dq : 0;
   // large parts of both: dK and dV are added before dQ starts, whose parts take their place.  One launch more, of a call of
   // milliseconds (2 heads, 16384 x 16384 of 256, causal, forward and backward: 1939 -> 1908 us); smaller ones lose by it (4 heads of
   // 2300: 188 -> 191)
-  p.sum_between = kv > 0 && q > 0 && kv + q > (128 << 20);
+  p.sum_between = kv > 0 && q > 0 && kv + q > SUM_BETWEEN;
   p.part_bytes = p.sum_between ? std::max(kv, q) : kv + q;
   return p;
 }
