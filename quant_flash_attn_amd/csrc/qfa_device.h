@@ -213,9 +213,9 @@ template <int ROW_BYTES, int ROWS, int NT, typename S = Swz<ROW_BYTES>> struct T
     }
   }
   // one chunk (index i < N) of a copy whose descriptor the caller made with make_rsrc(tile_base, ...)
-  __device__ __forceinline__ void issue_one(rsrc_t rs, unsigned char *lds, int wave_u, int tid, int i) const {
+  template <int HINT = 0> __device__ __forceinline__ void issue_one(rsrc_t rs, unsigned char *lds, int wave_u, int tid, int i) const {
     if (TOTAL % NT == 0 || tid + NT * i < TOTAL)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)(lds + (wave_u * 64 + NT * i) * 16), 16, (int)off[i], 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)(lds + (wave_u * 64 + NT * i) * 16), 16, (int)off[i], 0, 0, HINT);
   }
   // tile_base and lds must be wave-uniform; wave_u = wave index held in a scalar register
   __device__ __forceinline__ void issue(const void *tile_base, unsigned char *lds, int wave_u, int tid) const {

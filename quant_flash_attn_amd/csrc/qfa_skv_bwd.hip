@@ -77,8 +77,9 @@ template <int CPR> __device__ __forceinline__ int row_swizzle(int i) {
 template <int OFF> __device__ __forceinline__ u32x2 lds_tr16(unsigned addr) { return lds_read_tr16_async<OFF>(addr); }
 
 // S: element type of the scale vector (float or _Float16).  HALF: at most 16 queries -- rows 16..31 of the
-// query block are padding, so their share of steps 2 and 4 is skipped (P and dS are zero there).
-template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void skv_bwd_kernel(SkvBwdArgs a) {
+// query block are padding, so their share of steps 2 and 4 is skipped (P and dS are zero there).  STREAM: the codes' loads and
+// dKV's stores are non-temporal (LOAD_ONCE).
+template <typename S, int D, bool HALF, bool STREAM> __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void skv_bwd_kernel(SkvBwdArgs a) {
   constexpr int QH = HALF ? 1 : 2;   // 16-query halves of the block that hold queries
   typedef SkvBwdSmem<D> SM;
   typedef Swz<D> KSW;
@@ -115,7 +116,7 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
     const int rows = min(SKV_TILE, a.Nk - t * SKV_TILE);
     const rsrc_t rs_k = make_rsrc(codes_bh + (int64_t)t * SKV_TILE * a.scn, (unsigned)((rows - 1) * (int)a.scn + D));
 #pragma unroll
-    for (int c = 0; c < Copy::N; ++c) cp.issue_one(rs_k, slot, 0, lane, c);
+    for (int c = 0; c < Copy::N; ++c) cp.template issue_one<STREAM ? LOAD_ONCE : 0>(rs_k, slot, 0, lane, c);
     const rsrc_t rs_s = make_rsrc(reinterpret_cast<const S *>(a.scale) + tk0 + (int64_t)t * SKV_TILE,
                                   (unsigned)rows * (unsigned)sizeof(S));
     const rsrc_t rs_z = make_rsrc(a.zp + tk0 + (int64_t)t * SKV_TILE, (unsigned)rows);
@@ -399,7 +400,11 @@ template <typename S, int D, bool HALF> __global__ __launch_bounds__(256, D == 2
         for (int it = 0; it < 4; ++it) {
           const u32x4 row16 = *reinterpret_cast<const u32x4 *>(stage + st_r + it * 1024);
           const int j = j0 + 8 * it + lane / 8;
-          if (j < a.Nk) *reinterpret_cast<u32x4 *>(dkv_bh + (int64_t)j * a.sdkn + 32 * (db - 1) + 8 * (lane % 8)) = row16;
+          u32x4 *out = reinterpret_cast<u32x4 *>(dkv_bh + (int64_t)j * a.sdkn + 32 * (db - 1) + 8 * (lane % 8));
+          if (j < a.Nk) {
+            if constexpr (STREAM) __builtin_nontemporal_store(row16, out);
+            else *out = row16;
+          }
         }
       }
     }
@@ -491,8 +496,14 @@ template <typename S, int D> static int launch_skv_bwd_sd(const SkvAttnArgs &x, 
   }
   const int64_t total = xcd_grid(x.B * x.H, a.splits);
   if (total > 0x7fffffffLL) return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: too many (batch, head) pairs for one launch");
-  if (x.Nq <= 16) skv_bwd_kernel<S, D, true><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
-  else if constexpr (D <= 128) skv_bwd_kernel<S, D, false><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
+  // Codes and dKV (three bytes an element) beyond the last-level cache: loads and stores non-temporal, both or neither (8192 heads,
+  // 16 x 3000 of 128: 1958 us; the loads alone 2058, the stores alone 1954, both 1894).  300 random calls: 0.97 of the time at head_dim 128,
+  // 0.966 at 256, 0.96 at 64 up to 256 MiB of codes, beyond which 64 gains nothing (1.01)
+  const int64_t codes = x.B * x.H * x.Nk * D;
+  const bool once = 3 * codes > LAST_LEVEL_BYTES && (D > 64 || codes < LAST_LEVEL_BYTES);
+  const dim3 grid((unsigned)total);
+  if (x.Nq <= 16) once ? skv_bwd_kernel<S, D, true, true><<<grid, dim3(256), 0, st>>>(a) : skv_bwd_kernel<S, D, true, false><<<grid, dim3(256), 0, st>>>(a);
+  else if constexpr (D <= 128) once ? skv_bwd_kernel<S, D, false, true><<<grid, dim3(256), 0, st>>>(a) : skv_bwd_kernel<S, D, false, false><<<grid, dim3(256), 0, st>>>(a);
   else return set_error(QFA_EUNSUPPORTED, "attn_bwd_shared_kv: the one-pass kernel takes at most 16 queries at head_dim 256");
   if (int e = check_launch("qfa_attn_bwd_shared_kv")) return e;
   return a.splits > 1 ? launch_split_sum(x, a.splits, st) : 0;

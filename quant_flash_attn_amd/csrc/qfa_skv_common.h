@@ -129,6 +129,13 @@ struct XcdBlock {
   }
 };
 
+// Codes that one workgroup reads, and nobody again before as much as the last-level cache holds has passed: their loads are
+// non-temporal then (the cache hint of a buffer load) and leave the caches to others.  Whoever shares codes between workgroups
+// (several blocks of queries), or finds them in that cache when it is called again, loses by it: up to 30 % for a decoding loop over
+// one cache of 200 MB.
+constexpr int LOAD_ONCE = 2;
+constexpr int64_t LAST_LEVEL_BYTES = 256 << 20;
+
 // wait for every LDS operation of this wave; `tie` keeps the users of an asynchronously loaded
 // register pair behind the wait that precedes it in program order
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }

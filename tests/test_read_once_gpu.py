@@ -1,0 +1,56 @@
+"""Codes beyond the last-level cache, which the short-query kernels read (and dKV, which the backward writes) with non-temporal accesses:
+sampled heads against fp64 attention on the dequantized tensors, ragged ends included."""
+import math
+
+import pytest
+import torch
+
+from helpers import assert_close
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _dequant(t, h):
+    return oracle.dequantize_per_token(*(x[:, h:h + 1].cpu() for x in t[:3]), torch.float64)
+
+
+@pytest.mark.parametrize("H,Nq,Nk,D,dtype", [(2700, 1, 1029, 64, torch.bfloat16), (1340, 16, 1025, 128, torch.float16), (650, 5, 1100, 256, torch.float32),
+                                             (40, 1, 33001, 128, torch.bfloat16)])
+def test_cache(qfa, H, Nq, Nk, D, dtype):
+    assert 2 * H * Nk * D > 320 << 20
+    g, sm = torch.Generator(device=DEV).manual_seed(D + Nk), 1.0 / math.sqrt(D)
+    mk = lambda n: torch.randn((1, H, n, D), generator=g, device=DEV, dtype=torch.float16)
+    q = mk(Nq).to(dtype)
+    kq, vq = (qfa.asymmetric_quant_per_token(mk(Nk)) for _ in range(2))
+    none = torch.empty(0, dtype=dtype, device=DEV)
+    with torch.no_grad():
+        o = qfa.quant_flash_attn_quantized_kv(q, none, none, kq, vq, True, sm)
+    qq = qfa.quantize_for_attention(q)
+    for h in (0, H // 2, H - 1):
+        for i in (0, Nq - 1):
+            n = Nk - Nq + i + 1
+            want, _ = oracle.attn_fwd(_dequant(qq, h)[:, :, i:i + 1], _dequant(kq, h)[:, :, :n], _dequant(vq, h)[:, :, :n], False, sm)
+            assert_close(f"O, head {h}, row {i}", o[:, h:h + 1, i:i + 1].double().cpu(), want, scaled=True, rel=2.0 ** -7)
+
+
+@pytest.mark.parametrize("H,Nq,Nk,D,dtype", [(1500, 32, 1029, 64, torch.float16), (1500, 7, 1029, 64, torch.bfloat16), (2080, 16, 1025, 128, torch.float16),
+                                             (900, 31, 1029, 128, torch.bfloat16), (1040, 3, 1027, 256, torch.float16)])
+def test_shared_kv(qfa, H, Nq, Nk, D, dtype):
+    codes = H * Nk * D
+    assert 3 * codes > 256 << 20 and (D > 64 or codes < 256 << 20)
+    g, sm = torch.Generator(device=DEV).manual_seed(D + Nq), 1.0 / math.sqrt(D)
+    mk = lambda n: torch.randn((1, H, n, D), generator=g, device=DEV, dtype=dtype)
+    q, kv, do = mk(Nq).requires_grad_(True), mk(Nk).requires_grad_(True), mk(Nq)
+    kvq = qfa.asymmetric_quant_per_token(kv.detach())
+    o = qfa.quant_flash_attn(q, kv, kvq, sm)
+    dq, dkv = torch.autograd.grad(o, (q, kv), do)
+    assert torch.isfinite(dkv).all()
+    for h in (0, H // 2, H - 1):
+        qh, kvh, doh = q.detach()[:, h:h + 1].double().cpu(), _dequant(kvq, h), do[:, h:h + 1].double().cpu()
+        qh, kvh = (t.requires_grad_(True) for t in (qh, kvh))
+        want = torch.softmax(qh @ kvh.transpose(-1, -2) * sm, -1) @ kvh
+        grads = torch.autograd.grad(want, (qh, kvh), doh)
+        for name, got, ref in (("O", o, want), ("dQ", dq, grads[0]), ("dKV", dkv, grads[1])):
+            assert_close(f"{name}, head {h}", got[:, h:h + 1].detach().double().cpu(), ref.detach(), scaled=True, rel=2.0 ** -7)
