@@ -155,9 +155,9 @@ __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 1
 // 32 rows of a row-major tensor from tiles T0 .. T0 + D/32 - 1, scaled and rounded (store_tile_rows)
 template <typename T, int D, int T0, int... DB>
 __device__ __forceinline__ void acc_store_rows_seq(std::integer_sequence<int, DB...>, float scale, unsigned char *stage, T *rows,
-                                                   int64_t stride, int row0, int nrows, int lane) {
+                                                   int64_t stride, int row0, int nrows, int lane, bool once) {
   const f32x16 acc[sizeof...(DB)] = {acc_read<T0 + DB>()...};
-  store_tile_rows<T, D>(acc, scale, stage, rows, stride, row0, nrows, lane);
+  store_tile_rows<T, D>(acc, scale, stage, rows, stride, row0, nrows, lane, once);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the stage may be written again
 }
 template <int D, int T0, int... DB>
@@ -172,8 +172,8 @@ __device__ __forceinline__ void acc_store_rows_f32(float scale, float *rows, int
 }
 template <typename T, int D, int T0>
 __device__ __forceinline__ void acc_store_rows(float scale, unsigned char *stage, T *rows, int64_t stride, int row0, int nrows,
-                                               int lane) {
-  acc_store_rows_seq<T, D, T0>(std::make_integer_sequence<int, D / 32>{}, scale, stage, rows, stride, row0, nrows, lane);
+                                               int lane, bool once = false) {
+  acc_store_rows_seq<T, D, T0>(std::make_integer_sequence<int, D / 32>{}, scale, stage, rows, stride, row0, nrows, lane, once);
 }
 
 // ---- INT8 scores that need no conversion: with 0x4B400000, the bits of 1.5 * 2^23, as their initial value the int32 results

@@ -316,10 +316,10 @@ template <int N> __device__ __forceinline__ void lds_wait_async(u32x2 (&r)[4]) {
 // row0 .. row0+31 (those below nrows) of a row-major tensor.  Stored directly, one instruction would write 16 bytes
 // to each of 32 rows; the tile goes through `stage` (32 * 2D bytes of LDS owned by this wave, not in use by anybody
 // else) and leaves as whole rows, 16 bytes per lane.  Chunks are XORed with the row so that the 32 rows of one LDS
-// write spread over the banks.
+// write spread over the banks.  once: non-temporal stores (uniform; see LAST_LEVEL_BYTES).
 template <typename T, int D>
 __device__ __forceinline__ void store_tile_rows(const f32x16 (&acc)[D / 32], float scale, unsigned char *stage,
-                                                T *base, int64_t row_stride, int row0, int nrows, int lane) {
+                                                T *base, int64_t row_stride, int row0, int nrows, int lane, bool once = false) {
   constexpr int ROWB = 2 * D, CPR = ROWB / 16;
   asm volatile("" : "+v"(lane));   // addresses are formed here, not hoisted above the caller's main loop
   const int lr = lane % 32, g = lane / 32;
@@ -337,7 +337,16 @@ __device__ __forceinline__ void store_tile_rows(const f32x16 (&acc)[D / 32], flo
   for (int i = 0; i < 32 * CPR / 64; ++i) {
     const int p = lane + 64 * i, row = p / CPR, c = p % CPR;
     const u32x4 w = *reinterpret_cast<const u32x4 *>(stage + row * ROWB + ((c ^ (row % CPR)) * 16));
-    if (row0 + row < nrows) *reinterpret_cast<u32x4 *>(base + (int64_t)(row0 + row) * row_stride + c * 8) = w;
+    if (row0 + row < nrows) {
+      u32x4 *out = reinterpret_cast<u32x4 *>(base + (int64_t)(row0 + row) * row_stride + c * 8);
+      if (once) {
+        asm volatile("");   // (else the compiler makes one store of the two, without the hint)
+        __builtin_nontemporal_store(w, out);
+        asm volatile("");
+      } else {
+        *out = w;
+      }
+    }
   }
 }
 

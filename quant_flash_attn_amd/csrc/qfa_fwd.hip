@@ -696,6 +696,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   int64_t o_at = eb * ep->sob + eh * ep->soh, son = ep->son;
   void *out = SPLIT ? (void *)ep->po : ep->o;
   float *out32 = SPLIT ? ep->pml : ep->o32, *lse = ep->lse;
+  const int o_once = ep->o_once;
   asm volatile("" : "+s"(o_at), "+s"(son), "+s"(out), "+s"(out32), "+s"(lse));
   // ---- masked tiles (diagonal, ragged end): one block at a time, nothing carried between blocks
   for (; t < ntiles; ++t) {
@@ -744,7 +745,7 @@ __global__ __launch_bounds__(64 * NW, FwdSmem<D>::WG_PER_CU) void fwd_kernel(Fwd
   if (out32) store_tile_rows_f32<D>(oacc, inv, out32 + tq0 * D, D, m0 + wave * 32, a.Nq, lane);
   if (out)
     store_tile_rows<T, D>(oacc, inv, smem + SM::OFF_K + wave * (32 * 2 * D), static_cast<T *>(out) + o_at, son, m0 + wave * 32, a.Nq,
-                          lane);
+                          lane, o_once);
   if (qi < a.Nq && g == 0) lse[tq0 + qi] = (a_i * m_ref + __log2f(l_tot)) * kLn2;
 }
 
@@ -759,6 +760,11 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
   a.sm_scale_log2 = x.sm_scale * kLog2e;
   constexpr int FWD_BM = 32 * FWD_WAVES;
   a.mblocks = (int)((x.Nq + FWD_BM - 1) / FWD_BM);
+  // O past the caches where codes, V and O exceed the last-level cache: else it pushes out the K and V that other workgroups read next.
+  // The forward, and with a product that reads O behind it, us: 64 heads of 4096 x 256 causal 618 -> 582, 682 -> 669; 1000 of 200 x 256
+  // 176 -> 160, 232 -> 224; 128 of 4096 x 128 causal 561 -> 550, 618 -> 613.  Below it nothing is gained and the product loses (1024 of
+  // 300 x 128: 123 -> 123, 159 -> 163), and at head_dim 64 nothing was seen
+  a.o_once = D >= 128 && x.B * x.H * (x.Nq + x.Nk) * D * 3 > LAST_LEVEL_BYTES;
   a.splits = 1;
   a.keys_per_split = 0;
   a.po = a.pml = nullptr;

@@ -19,6 +19,7 @@ struct FwdArgs {
   int blocks_per_xcd;    // ceil(total_blocks / 8)
   int splits, keys_per_split;   // workgroups that share the keys of a query block (a multiple of 64 each)
   float *po, *pml;       // splits > 1: partial results per query and split (qfa_merge.h)
+  int o_once;            // O is written with non-temporal stores
   int group_log2;        // causal: log2 of the number of heads whose query blocks are dispatched together
 };
 

@@ -414,7 +414,7 @@ template <typename T, int D, int QB, bool CAUSAL, bool SPLIT> __global__ __launc
       return;
     }
     if (a.o32) acc_store_rows_f32<D, qb * DB>(1.0f / l_tot, a.o32 + tq0 * D, D, q_first + 32 * qb, a.Nq, lane);
-    if (a.o) acc_store_rows<T, D, qb * DB>(1.0f / l_tot, stage, o_bh, a.son, q_first + 32 * qb, a.Nq, lane);
+    if (a.o) acc_store_rows<T, D, qb * DB>(1.0f / l_tot, stage, o_bh, a.son, q_first + 32 * qb, a.Nq, lane, a.o_once);
     if (qi < a.Nq && g == 0) a.lse[tq0 + qi] = (a_i[qb] * m_ref[qb] + __log2f(l_tot)) * kLn2;
   });
 #endif

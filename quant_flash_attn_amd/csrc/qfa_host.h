@@ -94,6 +94,10 @@ inline int64_t xcd_grid(int64_t BH, int64_t per_bh) {
   return xcd_whole_heads(BH) ? (BH + 7) / 8 * 8 * per_bh : (BH * per_bh + 7) / 8 * 8;
 }
 
+// What a launch reads and writes beyond this, nobody finds in the last-level cache afterwards: what is touched once is better kept out of
+// the caches then, which others still need
+constexpr int64_t LAST_LEVEL_BYTES = 256 << 20;
+
 // Shared-KV attention (K = V = one quantized tensor, Q in 16-bit float), after validation.
 struct SkvAttnArgs {
   const void *q; const int8_t *codes; const void *scale; const int8_t *zp;

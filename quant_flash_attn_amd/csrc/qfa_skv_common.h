@@ -134,7 +134,6 @@ struct XcdBlock {
 // (several blocks of queries), or finds them in that cache when it is called again, loses by it: up to 30 % for a decoding loop over
 // one cache of 200 MB.
 constexpr int LOAD_ONCE = 2;
-constexpr int64_t LAST_LEVEL_BYTES = 256 << 20;
 
 // wait for every LDS operation of this wave; `tie` keeps the users of an asynchronously loaded
 // register pair behind the wait that precedes it in program order

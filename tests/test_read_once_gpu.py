@@ -54,3 +54,15 @@ def test_shared_kv(qfa, H, Nq, Nk, D, dtype):
         grads = torch.autograd.grad(want, (qh, kvh), doh)
         for name, got, ref in (("O", o, want), ("dQ", dq, grads[0]), ("dKV", dkv, grads[1])):
             assert_close(f"{name}, head {h}", got[:, h:h + 1].detach().double().cpu(), ref.detach(), scaled=True, rel=2.0 ** -7)
+
+
+@pytest.mark.parametrize("H,N,D,causal", [(1200, 300, 128, True), (1200, 300, 128, False), (600, 301, 256, True), (600, 301, 256, False)])
+def test_output_past_the_caches(qfa, H, N, D, causal):
+    """O of a forward beyond the last-level cache, written with non-temporal stores: the bits of its halves, which are not."""
+    assert 3 * H * 2 * N * D > 256 << 20 > 3 * H * N * D
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v = (torch.randn((1, H, N, D), generator=g, device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    with torch.no_grad():
+        o = qfa.quant_flash_attn_qkv(q, k, v, causal, 0.07)
+        halves = [qfa.quant_flash_attn_qkv(*(t[:, x] for t in (q, k, v)), causal, 0.07) for x in (slice(0, H // 2), slice(H // 2, H))]
+    assert torch.equal(o, torch.cat(halves, 1))
