@@ -6,8 +6,8 @@
 // Bound by reading the cache once (2 D + 6 bytes per key).  Through the kernels for long query blocks the same call
 // dequantizes V to 16 bits first (2 D more bytes written and read), sums K's codes in a pass of its own and then walks
 // each (batch, head) with one workgroup of 128 query rows, nearly all of them padding: B8 H32 Nq1 Nk8192 D128 took 459 us
-// that way (dequantize 175, row sums 100, attention 200 with the casts); this kernel and its merge take 96 us (5.7 TB/s of
-// cache; 35 -> 17.5 for B1).
+// that way (dequantize 175, row sums 100, attention 200 with the casts); this kernel and its merge take 83 us (6.6 TB/s of
+// cache; 96 before its loads were non-temporal; 35 -> 17.5 for B1).
 //
 // Work split.  A workgroup = 4 waves = 16 queries of one (batch, head) and a share of its keys (split_plan, qfa_merge.h);
 // its 32-key tiles are dealt to the waves, each with its own online softmax.  The tile lives in registers, double-buffered:
