@@ -217,10 +217,10 @@ static double pair_time(const PairCost &c, int D, const Share &kv, const Share &
   return body + (mb > 0.0 ? c.sum + c.mb * mb : 0.0);
 }
 
-// divisions of one kind that are worth an estimate, the plan's own first; returns how many
+// divisions of one kind that are worth an estimate (`parts`: also those into more than one), the plan's own first; returns how many
 constexpr int MAX_SHARES = 23;
-static int shares(int64_t BH, int64_t rows, int64_t streamed, int D, bool causal, bool ends, int64_t coff, int tensors, int blocks, int splits,
-                  int each, Share *out) {
+static int shares(int64_t BH, int64_t rows, int64_t streamed, int D, bool causal, bool ends, int64_t coff, int tensors, bool parts, int blocks,
+                  int splits, int each, Share *out) {
   static const int counts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24};
   const int64_t tiles = (streamed + 63) / 64;
   int found = 0;
@@ -244,6 +244,7 @@ static int shares(int64_t BH, int64_t rows, int64_t streamed, int D, bool causal
     work(r);
     int64_t last = 0;
     for (const int64_t s : counts) {
+      if (s > 1 && !parts) break;
       const int64_t e = (tiles + s - 1) / s, real = (tiles + e - 1) / e;
       if (real == last || (real > 1 && (BH * w.blocks * real > 600 || BH * rows * D * tensors * real > MAX_PART_FLOATS))) continue;
       last = real;
@@ -262,9 +263,10 @@ static void plan_pair(int64_t BH, int64_t Nq, int64_t Nk, int D, bool causal, Bw
       {{4.44, 0.268, 5.36, 0.139, {9.65, 6.67}, 0.545, {{1.25, 0}, {0.949, 0}}, 0.038, -0.047},
        {4.04, 0.24, 4.86, 0.137, {13.2, 8}, 0.522, {{1.06, 0}, {0.872, 0}}, 0.0869, -0.0534}}};
   const auto two_launches = [](const Share &a, const Share &b) { return a.splits > 1 && b.splits > 1 && 5e5 * (a.mbytes + b.mbytes) > SUM_BETWEEN; };
-  // More workgroups are not divided, but at head_dim 128 their rows per wave are chosen together too, by constants fitted to 650 such
-  // shapes (218 more: 20 move, to 0.93 of the time in the mean, 1.02 at most; 170 heads of 1056, 428 -> 364 us).  Up to where it was
-  // measured; it takes longer the more workgroups there are
+  // More workgroups are not divided here (96 heads of 691, causal, 94.9 us, took 117.7 with dQ's keys in two parts), but at head_dim 128
+  // their rows per wave are chosen together too, by constants fitted to 650 such shapes (218 more: 20 move, to 0.93 of the time in the
+  // mean, 1.02 at most; 170 heads of 1056, 428 -> 364 us), none of them divided: they know no cost of parts.  Up to where it was measured;
+  // it takes longer the more workgroups there are
   static const PairCost full128[2] = {{8.37, 0.4, 0, 0, {12.2, 3.76}, 0.306, {{0.532, 0.865}, {0.764, 1.12}}, 0, 0.0225},
                                       {7.78, 0.325, 0, 0, {9.93, 7.46}, 0.663, {{0.792, 1.29}, {0.429, 0.613}}, 0, -0.0585}};
   const int64_t wgs = BH * ((Nq + 127) / 128 + (Nk + 127) / 128);
@@ -272,8 +274,8 @@ static void plan_pair(int64_t BH, int64_t Nq, int64_t Nk, int D, bool causal, Bw
   if (full && (D != 128 || wgs > 6000 || p->splits_dkv > 1 || p->splits_dq > 1)) return;
   const PairCost &c = full ? full128[causal] : cost[D == 64 ? 0 : D == 128 ? 1 : 2][causal];
   Share kv[MAX_SHARES], q[MAX_SHARES];
-  const int nkv = shares(BH, Nk, Nq, D, causal, false, Nk - Nq, 2, p->blocks_dkv, p->splits_dkv, p->queries_per_split, kv);
-  const int nq = shares(BH, Nq, Nk, D, causal, true, Nk - Nq, 1, p->blocks_dq, p->splits_dq, p->keys_per_split, q);
+  const int nkv = shares(BH, Nk, Nq, D, causal, false, Nk - Nq, 2, !full, p->blocks_dkv, p->splits_dkv, p->queries_per_split, kv);
+  const int nq = shares(BH, Nq, Nk, D, causal, true, Nk - Nq, 1, !full, p->blocks_dq, p->splits_dq, p->keys_per_split, q);
   // (of parts this large each kind fills the chip by itself: 2 heads, 7500 to 8000 of 256, causal, lost 3 to 5 % by the estimate)
   if (kv[0].splits > 1 && q[0].splits > 1 && 5e5 * (kv[0].mbytes + q[0].mbytes) > SUM_BETWEEN * 5 / 8) return;
   const double fixed = c.base + c.prep * 1e-6 * (double)BH * D * (double)(7 * Nq + 3 * Nk);

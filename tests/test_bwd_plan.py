@@ -1,11 +1,12 @@
-"""Divisions of the backward that were chosen while a launch's workgroups were counted as if they were dealt evenly to the XCDs, and
-that took longer than the undivided kernels (us on an MI355X, whole backward): the plan may not choose them."""
+"""Divisions of the backward that took longer than the undivided kernels (us on an MI355X, whole backward): the plan may not choose
+them."""
 import pytest
 
 from plans import bwd_plan
 
 SLOWER = [
     # heads, Nq, Nk, D, causal, (rows per wave / 32, parts) of dK / dV and of dQ, us undivided, us so divided
+    # chosen while a launch's workgroups were counted as if they were dealt evenly to the XCDs
     (5, 4270, 4270, 128, False, (2, 3), (2, 3), 219.3, 259.7),      # 33 workgroups on one XCD of 32 CUs
     (7, 4502, 4502, 128, True, (2, 3), (1, 1), 207.5, 242.6),
     (5, 4555, 4555, 128, True, (2, 4), (2, 4), 200.5, 230.5),
@@ -16,10 +17,31 @@ SLOWER = [
     (2, 15938, 15938, 256, True, (1, 4), (1, 4), 1185.5, 1433.7),
     (10, 3567, 3567, 256, True, (1, 1), (1, 3), 296.9, 337.1),
     (9, 3345, 3345, 64, True, (1, 3), (1, 3), 115.4, 122.8),
+    # chosen by an estimate that was fitted to undivided launches of more than 1100 workgroups, and in which parts cost nothing
+    (96, 691, 691, 128, True, (2, 1), (2, 2), 94.9, 117.7),
+    (107, 227, 1168, 128, True, (2, 1), (2, 3), 97.0, 118.5),
+    (74, 942, 942, 128, True, (2, 1), (2, 2), 116.2, 137.6),
+    (159, 216, 1186, 128, False, (2, 1), (2, 2), 140.0, 162.0),
+    (71, 1014, 1014, 128, False, (2, 1), (2, 2), 160.5, 183.7),
+    (75, 975, 975, 128, False, (2, 1), (2, 2), 165.0, 187.3),
+    (106, 199, 1034, 128, True, (2, 1), (2, 3), 94.8, 106.9),
+    (58, 508, 2568, 128, False, (2, 1), (2, 4), 171.4, 190.9),
+    (78, 158, 2145, 128, False, (2, 1), (2, 5), 117.9, 126.2),
+    (27, 1513, 5602, 128, False, (2, 1), (2, 3), 365.1, 385.7),
 ]
+
+FULL = [s[:5] for s in SLOWER[10:]] + [(188, 127, 1876, 128, False), (103, 231, 3686, 128, True), (170, 1056, 1056, 128, False)]
 
 
 @pytest.mark.parametrize("BH,Nq,Nk,D,causal,dkv,dq,undivided,divided", SLOWER)
 def test_slower_division_is_not_chosen(qfa, BH, Nq, Nk, D, causal, dkv, dq, undivided, divided):
     p = bwd_plan(BH, Nq, Nk, D, causal)
     assert ((p.blocks_dkv, p.splits_dkv), (p.blocks_dq, p.splits_dq)) != (dkv, dq), divided / undivided
+
+
+@pytest.mark.parametrize("BH,Nq,Nk,D,causal", FULL)
+def test_a_full_chip_is_not_divided(qfa, BH, Nq, Nk, D, causal):
+    """More than 1100 workgroups, of which neither kind by itself is worth dividing."""
+    assert BH * ((Nq + 127) // 128 + (Nk + 127) // 128) > 1100
+    p = bwd_plan(BH, Nq, Nk, D, causal)
+    assert (p.splits_dkv, p.splits_dq, p.part_bytes) == (1, 1, 0)
