@@ -264,14 +264,17 @@ static void plan_pair(int64_t BH, int64_t Nq, int64_t Nk, int D, bool causal, Bw
        {4.04, 0.24, 4.86, 0.137, {13.2, 8}, 0.522, {{1.06, 0}, {0.872, 0}}, 0.0869, -0.0534}}};
   const auto two_launches = [](const Share &a, const Share &b) { return a.splits > 1 && b.splits > 1 && 5e5 * (a.mbytes + b.mbytes) > SUM_BETWEEN; };
   // More workgroups are not divided here (96 heads of 691, causal, 94.9 us, took 117.7 with dQ's keys in two parts), but at head_dim 128
-  // their rows per wave are chosen together too, by constants fitted to 650 such shapes (218 more: 20 move, to 0.93 of the time in the
-  // mean, 1.02 at most; 170 heads of 1056, 428 -> 364 us), none of them divided: they know no cost of parts.  Up to where it was measured;
-  // it takes longer the more workgroups there are
+  // their rows per wave are chosen together too, by constants fitted to 650 such shapes, none of them divided: they know no cost of
+  // parts.  Where queries and keys are within a factor of two and a sixteenth is promised, and up to where it was measured; it takes
+  // longer the more workgroups there are.  Against each kind's own choice, in one launch too, over 1128 of the shapes that move: 0.918 of the
+  // time without a mask and as many queries as keys, 0.951 with other numbers, causal 0.958, six of them more than 1.04 times (1.065
+  // at most); 170 heads of 1056 454 -> 412 us.  Beyond a factor of four 0.965, but one in six more than 1.04 times (53 heads, 415 x 2158:
+  // 125 -> 147 us)
   static const PairCost full128[2] = {{8.37, 0.4, 0, 0, {12.2, 3.76}, 0.306, {{0.532, 0.865}, {0.764, 1.12}}, 0, 0.0225},
                                       {7.78, 0.325, 0, 0, {9.93, 7.46}, 0.663, {{0.792, 1.29}, {0.429, 0.613}}, 0, -0.0585}};
   const int64_t wgs = BH * ((Nq + 127) / 128 + (Nk + 127) / 128);
   const bool full = BH > MAX_WGS_BWD || wgs > MAX_WGS_BWD;
-  if (full && (D != 128 || wgs > 6000 || p->splits_dkv > 1 || p->splits_dq > 1)) return;
+  if (full && (D != 128 || wgs > 6000 || 2 * std::min(Nq, Nk) < std::max(Nq, Nk) || p->splits_dkv > 1 || p->splits_dq > 1)) return;
   const PairCost &c = full ? full128[causal] : cost[D == 64 ? 0 : D == 128 ? 1 : 2][causal];
   Share kv[MAX_SHARES], q[MAX_SHARES];
   const int nkv = shares(BH, Nk, Nq, D, causal, false, Nk - Nq, 2, !full, p->blocks_dkv, p->splits_dkv, p->queries_per_split, kv);
@@ -279,7 +282,7 @@ static void plan_pair(int64_t BH, int64_t Nq, int64_t Nk, int D, bool causal, Bw
   // (of parts this large each kind fills the chip by itself: 2 heads, 7500 to 8000 of 256, causal, lost 3 to 5 % by the estimate)
   if (kv[0].splits > 1 && q[0].splits > 1 && 5e5 * (kv[0].mbytes + q[0].mbytes) > SUM_BETWEEN * 5 / 8) return;
   const double fixed = c.base + c.prep * 1e-6 * (double)BH * D * (double)(7 * Nq + 3 * Nk);
-  double best = (full ? 0.98 : 0.9) * (fixed + pair_time(c, D, kv[0], q[0])) - fixed;
+  double best = (full ? 0.94 : 0.9) * (fixed + pair_time(c, D, kv[0], q[0])) - fixed;
   const Share *bk = &kv[0], *bq = &q[0];
   for (int i = 0; i < nkv; ++i)
     for (int j = 0; j < nq; ++j) {

@@ -45,3 +45,23 @@ def test_a_full_chip_is_not_divided(qfa, BH, Nq, Nk, D, causal):
     assert BH * ((Nq + 127) // 128 + (Nk + 127) // 128) > 1100
     p = bwd_plan(BH, Nq, Nk, D, causal)
     assert (p.splits_dkv, p.splits_dq, p.part_bytes) == (1, 1, 0)
+
+
+OTHER_ROWS = [
+    # heads, Nq, Nk, causal, rows per wave / 32 of dK / dV and of dQ, us with each kind's own choice, us with this one (in one launch both)
+    (53, 415, 2158, False, (2, 2), 125.4, 146.7),
+    (118, 355, 3301, True, (2, 1), 343.1, 393.8),
+    (119, 378, 4799, True, (2, 1), 486.6, 553.8),
+    (87, 380, 5964, False, (2, 1), 474.2, 539.5),
+    (94, 345, 3632, False, (2, 1), 328.2, 372.5),
+    (102, 145, 1237, False, (2, 2), 88.6, 100.2),
+    (126, 364, 5066, False, (2, 1), 541.2, 610.3),
+    (22, 1173, 5651, False, (2, 2), 275.0, 307.1),
+]
+
+
+@pytest.mark.parametrize("BH,Nq,Nk,causal,rows,own,joint", OTHER_ROWS)
+def test_slower_rows_per_wave_are_not_chosen(qfa, BH, Nq, Nk, causal, rows, own, joint):
+    """Many workgroups whose estimate was fitted to sequences of about the same length."""
+    p = bwd_plan(BH, Nq, Nk, 128, causal)
+    assert (p.blocks_dkv, p.blocks_dq) != rows, joint / own
