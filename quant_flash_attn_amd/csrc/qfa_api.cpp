@@ -583,8 +583,7 @@ static int attn_bwd(const char *who, int f32, const int8_t *qc, const float *sq,
   if (!strides_ok(sdob, sdoh, sdon, D, es) || !strides_ok(sdqb, sdqh, sdqn, D, es) ||
       !strides_ok(sdkb, sdkh, sdkn, D, es) || !strides_ok(sdvb, sdvh, sdvn, D, es))
     return set_error(QFA_EINVAL, "%s: strides must be positive multiples of 16 bytes, token stride >= D", who);
-  const int64_t parts = bwd_split_bytes(B, H, Nq, Nk, D, causal);
-  a.may_split = parts > 0 && workspace_bytes - need >= parts;
+  a.bwd = bwd_plan_within(B * H, Nq, Nk, D, causal, workspace_bytes - need);
   return launch_bwd(a, (hipStream_t)stream);
 }
 

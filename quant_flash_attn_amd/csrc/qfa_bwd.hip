@@ -325,7 +325,7 @@ template <typename T, int D> static int launch_bwd_td(const AttnArgs &x, hipStre
     return set_error(QFA_EUNSUPPORTED, "attn_bwd: too many tiles for one launch");
   bwd_prep_kernel<T, D><<<dim3((unsigned)(BH * (a.tiles_q + a.tiles_k))), dim3(256), 0, st>>>(a, (int)(BH * a.tiles_q));
   if (int e = check_launch("qfa_attn_bwd (staging)")) return e;
-  const BwdPlan plan = bwd_plan(BH, x.Nq, x.Nk, D, x.causal, x.may_split);
+  const BwdPlan &plan = x.bwd;
   float *const parts = reinterpret_cast<float *>(a.ws_q + (x.f32 ? bwd_f32_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)
                                                          : bwd_workspace_bytes(x.B, x.H, x.Nq, x.Nk, D)));
   float *part = parts;

@@ -43,6 +43,10 @@ int launch_dequant(const int8_t *codes, const void *scale, int scale_dtype, cons
                    int out_dtype, int64_t B, int64_t H, int64_t N, int D, int64_t scb, int64_t sch, int64_t scn,
                    int64_t sob, int64_t soh, int64_t son, hipStream_t st);
 
+// How the backward's two kinds of workgroups are launched: 32-row blocks per wave, and the parts of the streamed rows; the memory of the
+// parts, and whether those of dQ take the place of the others
+struct BwdPlan { int blocks_dkv, splits_dkv, queries_per_split, blocks_dq, splits_dq, keys_per_split, sum_between; int64_t part_bytes; };
+
 // Tensors of one attention call, after validation.  Strides in elements.
 struct AttnArgs {
   const int8_t *qc; const float *sq; const int8_t *zq; const int32_t *rq;
@@ -58,7 +62,7 @@ struct AttnArgs {
   int io_dtype;
   float *o32;   // forward: nullable, O in fp32 (dense); o is nullable then
   int f32;      // backward: dO and the gradients are fp32, the workspace holds bwd_f32_workspace_bytes
-  int may_split;   // backward: and bwd_split_bytes behind them
+  BwdPlan bwd;  // backward: and bwd.part_bytes behind them
 };
 
 int launch_fwd(const AttnArgs &a, hipStream_t st, bool qk_only = false);   // workspace: nullable, the keys are split with one
@@ -74,9 +78,6 @@ inline int64_t bwd_f32_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t
   return bwd_workspace_bytes(B, H, Nq, Nk, D) + B * H * Nq * D * 2;
 }
 
-// How the backward's two MFMA kernels are launched: 32-row blocks per wave, and the parts of the streamed rows; the memory of the
-// parts, and whether those of dQ take the place of the others
-struct BwdPlan { int blocks_dkv, splits_dkv, queries_per_split, blocks_dq, splits_dq, keys_per_split, sum_between; int64_t part_bytes; };
 // causal: log2 of the heads whose blocks are dispatched together, `streamed` rows of 5 bytes per element each.  Pairs (N=4096,
 // D=128: 5.2 MB against the XCD's 4 MB L2) are 1 % better than single heads, four heads are not: within about 6 MB
 inline int bwd_group_log2(int64_t streamed, int D, bool dq) {
@@ -86,6 +87,8 @@ inline int bwd_group_log2(int64_t streamed, int D, bool dq) {
   return g;
 }
 BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_split);
+// what a call with `room` bytes for parts launches (an entry makes it once: up to 7 us, which small calls notice)
+BwdPlan bwd_plan_within(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int64_t room);
 int64_t bwd_split_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal);
 
 // grid of a kernel that maps ids with XcdBlock (qfa_skv_common.h): per_bh workgroups for each of BH heads

@@ -195,10 +195,10 @@ static void bwd_part(int64_t BH, int64_t rows, int64_t streamed, int D, bool cau
 // wide blocks too few no longer.  The estimate: where all workgroups run at once, the longest and a share of the mean load (they
 // slow each other down); otherwise the mean load and what is left of the last dQ workgroup, or again the longest.  Fitted to 7100 shapes
 // of 1 to 400 heads, 64 to 8192 keys, causal or not, with up to 29 divisions of both kinds each.  Only a division that it promises
-// to be a tenth faster than the plan is taken: of 8300 more shapes 900 move, to 0.90, 0.89 and 0.87 of the time in the mean (head_dim 64,
-// 128, 256), eight of them to more than 1.04 times (1.14 at most: 7 heads of 4116 x 128, 218 -> 249 us); taken whenever it is the
-// fastest, 5 in a hundred of all calls at 128 would take more than 1.04 times.  8 heads of 1702 x 128 causal 73 -> 57 us,
-// 2 x 1936 x 256 78 -> 56.
+// to be a tenth faster than the plan is taken: one call in nine, and of 2100 new ones (700 of a head_dim, timed as they are launched)
+// it makes 0.90, 0.89 and 0.87 of the time in the mean (head_dim 64, 128, 256), 27 of them more than 1.04 times (1.14 at most: 3 heads,
+// 31 x 357 of 256, 19.9 -> 22.6 us; 4 heads of 3917 x 128, 131 -> 147); taken whenever it is the fastest, 5 in a hundred of all calls
+// at 128 would take more than 1.04 times.  8 heads of 1702 x 128 causal 73 -> 57 us, 2 x 1936 x 256 78 -> 56.
 struct PairCost {
   double base, prep, sum, mb;   // us: launches; staging per MB (10^6 elements); the sum of parts and what it takes per MB
   double start[2], tail;        // of a workgroup of dK / dV and of dQ, in tiles; share of the last one that runs alone
@@ -319,6 +319,11 @@ BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_
   p.sum_between = kv > 0 && q > 0 && kv + q > SUM_BETWEEN;
   p.part_bytes = p.sum_between ? std::max(kv, q) : kv + q;
   return p;
+}
+
+BwdPlan bwd_plan_within(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int64_t room) {
+  const BwdPlan p = bwd_plan(BH, Nq, Nk, D, causal, 1);
+  return p.part_bytes <= room ? p : bwd_plan(BH, Nq, Nk, D, causal, 0);
 }
 
 int64_t bwd_split_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D, int causal) {

@@ -30,6 +30,11 @@ def bwd_plan(BH, Nq, Nk, D, causal, may_split=1):
     return _plan("_ZN3qfa8bwd_planEllliii", BwdPlan, [_L, _L, _L, _I, _I, _I])(BH, Nq, Nk, D, int(causal), may_split)
 
 
+def bwd_plan_within(BH, Nq, Nk, D, causal, room):
+    """what a call with `room` bytes for parts launches"""
+    return _plan("_ZN3qfa15bwd_plan_withinEllliil", BwdPlan, [_L, _L, _L, _I, _I, _L])(BH, Nq, Nk, D, int(causal), room)
+
+
 def skv_tile_fwd_plan(BH, Nq, Nk, D):
     return _plan("_ZN3qfa12skv_fwd_planEllli", SkvFwdPlan, [_L, _L, _L, _I])(BH, Nq, Nk, D).tile
 

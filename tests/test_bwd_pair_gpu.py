@@ -1,13 +1,15 @@
 """dK / dV and dQ in one launch whose two kinds of workgroups are divided differently: other rows per wave, other numbers of parts, one
 kind divided and the other not.  Against fp64 attention on the dequantized Q and K."""
+import ctypes
 import math
+import re
 
 import pytest
 import torch
 
 from helpers import assert_close
 from oracle import oracle
-from plans import bwd_plan
+from plans import bwd_plan, bwd_plan_within
 from test_bwd_split_gpu import _inputs
 
 CASES = [
@@ -43,3 +45,74 @@ def test_both_kinds_in_one_launch(qfa, B, H, Nq, Nk, D, causal, dtype, plan):
     refs, spreads = oracle.attn_bwd(qh, kh, v16, do16, causal, sm, o=o16, spread=True)
     for name, got, want, sp in zip(("dQ", "dK", "dV"), grads, refs, spreads):
         assert_close(name, got.double().cpu(), want, scaled=True, rel=2.0 ** -7, spread=sp)   # (as the split backward's)
+
+
+class _KernelNode(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def _launches(forward, backward):
+    """(name, workgroups) of the kernels that backward(forward()) launches after its forward, in order, as a graph's nodes have them"""
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        o = forward()
+        backward(o)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        backward(o)
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    handle, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(handle, None, ctypes.byref(n)) == 0
+    nodes, out = (ctypes.c_void_p * n.value)(), []
+    assert hip.hipGraphGetNodes(handle, nodes, ctypes.byref(n)) == 0
+    for node in nodes:
+        p = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        out.append((hip.hipKernelNameRefByPtr(p.func, None).decode(), p.grid[0]))
+    return out
+
+
+def _workgroups(BH, rows, blocks, splits):
+    return (BH * -(-rows // (128 * blocks)) + 7) // 8 * 8 * splits
+
+
+LAUNCHED = [
+    # heads, Nq, Nk, D, causal: undivided, with other rows per wave than either kind would take by itself; then divided; then a full chip
+    (7, 1542, 4268, 128, False), (15, 782, 2179, 128, True), (6, 3420, 3420, 128, False), (170, 1056, 1056, 128, False),
+    (12, 279, 2790, 128, True), (3, 1866, 1866, 64, True), (2, 1936, 1936, 256, False), (96, 691, 691, 128, True),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Nq,Nk,D,causal", LAUNCHED)
+def test_the_planned_division_is_launched(qfa, H, Nq, Nk, D, causal):
+    p = bwd_plan(H, Nq, Nk, D, causal)
+    *leaves, do = _inputs(1, H, Nq, Nk, D, torch.bfloat16)
+    for t in leaves:
+        t.requires_grad_(True)
+    names = _launches(lambda: qfa.quant_flash_attn_qkv(*leaves, causal, 0.1), lambda o: torch.autograd.grad(o, leaves, do, retain_graph=True))
+    pair, = (x for x in names if "bwd_pair_kernel" in x[0])
+    assert [int(x) for x in re.findall(r"Li(\d+)E", pair[0])] == [D, p.blocks_dkv, p.blocks_dq], pair
+    assert pair[1] == _workgroups(H, Nk, p.blocks_dkv, p.splits_dkv) + _workgroups(H, Nq, p.blocks_dq, p.splits_dq), pair
+    assert any("bwd_sum_kernel" in x[0] for x in names) == (p.part_bytes > 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Nq,Nk,causal", [(170, 1056, 1056, False), (15, 782, 2179, True), (6, 3420, 3420, False)])
+def test_rows_per_wave_do_not_change_the_bits(qfa, H, Nq, Nk, causal):
+    """The undivided call and its heads one by one, whose rows per wave are others."""
+    q, k, v, do = _inputs(1, H, Nq, Nk, 128, torch.bfloat16)
+    qq, kq = qfa.quantize_for_attention(q), qfa.quantize_for_attention(k)
+    o, lse = qfa.attn_fwd_quantized(qq, kq, v, causal, 0.1)
+    whole = qfa.attn_bwd_quantized(qq, kq, v, o, do, lse, causal, 0.1)
+    one, all_ = (bwd_plan_within(n, Nq, Nk, 128, causal, 0) for n in (1, H))
+    assert (one.blocks_dkv, one.blocks_dq) != (all_.blocks_dkv, all_.blocks_dq)
+    for h in (0, H // 2, H - 1):
+        cut = lambda t: t[:, h:h + 1].contiguous()   # noqa: E731
+        part = qfa.attn_bwd_quantized(type(qq)(*map(cut, qq)), type(kq)(*map(cut, kq)), cut(v), cut(o), cut(do), cut(lse), causal, 0.1)
+        for name, got, want in zip(("dQ", "dK", "dV"), part, whole):
+            assert torch.equal(got, cut(want)), (name, h)

@@ -1,8 +1,11 @@
 """Divisions of the backward that took longer than the undivided kernels (us on an MI355X, whole backward): the plan may not choose
 them."""
+import math
+import random
+
 import pytest
 
-from plans import bwd_plan
+from plans import bwd_plan, bwd_plan_within
 
 SLOWER = [
     # heads, Nq, Nk, D, causal, (rows per wave / 32, parts) of dK / dV and of dQ, us undivided, us so divided
@@ -65,3 +68,28 @@ def test_slower_rows_per_wave_are_not_chosen(qfa, BH, Nq, Nk, causal, rows, own,
     """Many workgroups whose estimate was fitted to sequences of about the same length."""
     p = bwd_plan(BH, Nq, Nk, 128, causal)
     assert (p.blocks_dkv, p.blocks_dq) != rows, joint / own
+
+
+def _fields(p):
+    return tuple(getattr(p, n) for n, _ in p._fields_)
+
+
+def test_what_is_planned_is_launched(qfa):
+    """With the memory that the size query asks for the launch gets the plan that the query made, also where that is none for parts
+    but rows per wave; with less it is undivided, with more the same."""
+    rng, undivided = random.Random(5), 0
+    log = lambda lo, hi: int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+    shapes = [(170, 1056, 1056, 128, False), (7, 1542, 4268, 128, False), (15, 782, 2179, 128, True), (6, 5995, 5995, 128, True)]
+    for _ in range(5000):
+        Nk = log(16, 8192)
+        shapes.append((log(1, 800), Nk if rng.random() < 0.6 else log(1, Nk), Nk, rng.choice((64, 128, 128, 256)), rng.random() < 0.5))
+    for s in shapes:
+        p = bwd_plan(*s)
+        assert _fields(bwd_plan_within(*s, p.part_bytes)) == _fields(bwd_plan_within(*s, p.part_bytes + 999)) == _fields(p), s
+        if p.part_bytes > 0:
+            less = bwd_plan_within(*s, p.part_bytes - 1)
+            assert (less.splits_dkv, less.splits_dq, less.part_bytes) == (1, 1, 0), s
+        else:
+            alone = bwd_plan(*s, may_split=0)   # (each kind's rows per wave as if it had the chip to itself)
+            undivided += (p.blocks_dkv, p.blocks_dq) != (alone.blocks_dkv, alone.blocks_dq)
+    assert undivided > 20
