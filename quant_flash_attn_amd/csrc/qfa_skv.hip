@@ -365,7 +365,8 @@ template <typename T, typename S, int D> static int launch_skv_fwd_tsd(const Skv
   // 256, also on the same codes again and again (0.958, 0.953), 0.99 and 1.00 at 64; 100 to 256 MiB 0.97, and 1.01 to 1.04 on the same codes.
   // 8192 heads, 16 x 3000 of 128: 584 -> 554 us (5.4 -> 5.7 TB/s)
   const dim3 grid((unsigned)total);
-  if (D >= 128 && a.qblocks == 1 && x.B * x.H * x.Nk * D > LAST_LEVEL_BYTES) skv_fwd_kernel<T, S, D, (D >= 128)><<<grid, dim3(256), 0, st>>>(a);
+  const bool once = a.qblocks == 1 && x.B * x.H * x.Nk * D > LAST_LEVEL_BYTES && rows_own_lines(x.codes, x.scb, x.sch, x.scn, D);
+  if (D >= 128 && once) skv_fwd_kernel<T, S, D, (D >= 128)><<<grid, dim3(256), 0, st>>>(a);
   else skv_fwd_kernel<T, S, D, false><<<grid, dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_shared_kv")) return e;
   if (a.splits > 1) {

@@ -500,7 +500,8 @@ template <typename S, int D> static int launch_skv_bwd_sd(const SkvAttnArgs &x, 
   // 16 x 3000 of 128: 1958 us; the loads alone 2058, the stores alone 1954, both 1894).  300 random calls: 0.97 of the time at head_dim 128,
   // 0.966 at 256, 0.96 at 64 up to 256 MiB of codes, beyond which 64 gains nothing (1.01)
   const int64_t codes = x.B * x.H * x.Nk * D;
-  const bool once = 3 * codes > LAST_LEVEL_BYTES && (D > 64 || codes < LAST_LEVEL_BYTES);
+  const bool once = 3 * codes > LAST_LEVEL_BYTES && (D > 64 || codes < LAST_LEVEL_BYTES) && rows_own_lines(x.codes, x.scb, x.sch, x.scn, D) &&
+                    rows_own_lines(x.dkv, x.sdkb, x.sdkh, x.sdkn, 2 * D, 2);
   const dim3 grid((unsigned)total);
   if (x.Nq <= 16) once ? skv_bwd_kernel<S, D, true, true><<<grid, dim3(256), 0, st>>>(a) : skv_bwd_kernel<S, D, true, false><<<grid, dim3(256), 0, st>>>(a);
   else if constexpr (D <= 128) once ? skv_bwd_kernel<S, D, false, true><<<grid, dim3(256), 0, st>>>(a) : skv_bwd_kernel<S, D, false, false><<<grid, dim3(256), 0, st>>>(a);

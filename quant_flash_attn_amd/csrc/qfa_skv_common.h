@@ -131,8 +131,8 @@ struct XcdBlock {
 
 // Codes that one workgroup reads, and nobody again before as much as the last-level cache holds has passed: their loads are
 // non-temporal then (the cache hint of a buffer load) and leave the caches to others.  Whoever shares codes between workgroups
-// (several blocks of queries), or finds them in that cache when it is called again, loses by it: up to 30 % for a decoding loop over
-// one cache of 200 MB.
+// (several blocks of queries, or lines that hold rows of two heads: rows_own_lines), or finds them in that cache when it is called
+// again, loses by it: up to 30 % for a decoding loop over one cache of 200 MB.
 constexpr int LOAD_ONCE = 2;
 
 // wait for every LDS operation of this wave; `tie` keeps the users of an asynchronously loaded

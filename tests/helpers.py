@@ -1,4 +1,6 @@
 """Shared helpers for the parity tests (not collected by pytest)."""
+import ctypes
+
 import torch
 
 
@@ -88,3 +90,32 @@ def rounded_output_floor(qh, kh, v, do, o_ref, lse_ref, out_dtype, causal, sm):
     delta = (o_ref.to(out_dtype).double() * do.double()).sum(-1, keepdim=True)
     ds = p * (do.double() @ v.double().transpose(-1, -2) - delta)
     return (ds @ kh) * sm, (ds.transpose(-1, -2) @ qh) * sm
+
+
+class _KernelNode(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def launches(forward, backward):
+    """(name, workgroups) of the kernels that backward(forward()) launches after its forward, in order, as a graph's nodes have them"""
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        o = forward()
+        backward(o)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        backward(o)
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    handle, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(handle, None, ctypes.byref(n)) == 0
+    nodes, out = (ctypes.c_void_p * n.value)(), []
+    assert hip.hipGraphGetNodes(handle, nodes, ctypes.byref(n)) == 0
+    for node in nodes:
+        p = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        out.append((hip.hipKernelNameRefByPtr(p.func, None).decode(), p.grid[0]))
+    return out

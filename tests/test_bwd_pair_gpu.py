@@ -1,13 +1,12 @@
 """dK / dV and dQ in one launch whose two kinds of workgroups are divided differently: other rows per wave, other numbers of parts, one
 kind divided and the other not.  Against fp64 attention on the dequantized Q and K."""
-import ctypes
 import math
 import re
 
 import pytest
 import torch
 
-from helpers import assert_close
+from helpers import assert_close, launches
 from oracle import oracle
 from plans import bwd_plan, bwd_plan_within
 from test_bwd_split_gpu import _inputs
@@ -47,35 +46,6 @@ def test_both_kinds_in_one_launch(qfa, B, H, Nq, Nk, D, causal, dtype, plan):
         assert_close(name, got.double().cpu(), want, scaled=True, rel=2.0 ** -7, spread=sp)   # (as the split backward's)
 
 
-class _KernelNode(ctypes.Structure):   # hipKernelNodeParams
-    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
-                ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
-
-
-def _launches(forward, backward):
-    """(name, workgroups) of the kernels that backward(forward()) launches after its forward, in order, as a graph's nodes have them"""
-    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
-    stream.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(stream):
-        o = forward()
-        backward(o)
-    torch.cuda.synchronize()
-    with torch.cuda.graph(graph, stream=stream):
-        backward(o)
-    hip = ctypes.CDLL("libamdhip64.so")
-    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
-    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
-    handle, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
-    assert hip.hipGraphGetNodes(handle, None, ctypes.byref(n)) == 0
-    nodes, out = (ctypes.c_void_p * n.value)(), []
-    assert hip.hipGraphGetNodes(handle, nodes, ctypes.byref(n)) == 0
-    for node in nodes:
-        p = _KernelNode()
-        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
-        out.append((hip.hipKernelNameRefByPtr(p.func, None).decode(), p.grid[0]))
-    return out
-
-
 def _workgroups(BH, rows, blocks, splits):
     return (BH * -(-rows // (128 * blocks)) + 7) // 8 * 8 * splits
 
@@ -94,7 +64,7 @@ def test_the_planned_division_is_launched(qfa, H, Nq, Nk, D, causal):
     *leaves, do = _inputs(1, H, Nq, Nk, D, torch.bfloat16)
     for t in leaves:
         t.requires_grad_(True)
-    names = _launches(lambda: qfa.quant_flash_attn_qkv(*leaves, causal, 0.1), lambda o: torch.autograd.grad(o, leaves, do, retain_graph=True))
+    names = launches(lambda: qfa.quant_flash_attn_qkv(*leaves, causal, 0.1), lambda o: torch.autograd.grad(o, leaves, do, retain_graph=True))
     pair, = (x for x in names if "bwd_pair_kernel" in x[0])
     assert [int(x) for x in re.findall(r"Li(\d+)E", pair[0])] == [D, p.blocks_dkv, p.blocks_dq], pair
     assert pair[1] == _workgroups(H, Nk, p.blocks_dkv, p.splits_dkv) + _workgroups(H, Nq, p.blocks_dq, p.splits_dq), pair

@@ -1,11 +1,12 @@
 """Codes beyond the last-level cache, which the short-query kernels read (and dKV, which the backward writes) with non-temporal accesses:
 sampled heads against fp64 attention on the dequantized tensors, ragged ends included."""
 import math
+import re
 
 import pytest
 import torch
 
-from helpers import assert_close
+from helpers import assert_close, launches
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,52 @@ def test_output_past_the_caches(qfa, H, N, D, causal):
         o = qfa.quant_flash_attn_qkv(q, k, v, causal, 0.07)
         halves = [qfa.quant_flash_attn_qkv(*(t[:, x] for t in (q, k, v)), causal, 0.07) for x in (slice(0, H // 2), slice(H // 2, H))]
     assert torch.equal(o, torch.cat(halves, 1))
+
+
+def _between(t):
+    """the same codes, [B, N, H, D] in memory: a head's rows have those of the others between them"""
+    return (t[0].transpose(1, 2).contiguous().transpose(1, 2), *t[1:])
+
+
+def _hint(names, kernel):
+    """whether `kernel` was launched with the hint, by its last template argument"""
+    name, = (n for n, _ in names if kernel in n)
+    return re.findall(r"Lb([01])E", name)[-1] == "1"
+
+
+@pytest.mark.parametrize("H,Nk,D,offset,hint", [(2700, 1029, 64, 0, False), (1340, 1025, 128, 0, True), (1340, 1025, 128, 64, False)])
+def test_lines_of_two_heads_are_read_without_the_hint(qfa, H, Nk, D, offset, hint):
+    """Rows of 64 bytes, or rows that begin in the middle of a line, between rows of other heads: two workgroups read each line.  The
+    result is that of rows in one piece, for which the hint stays."""
+    g, sm = torch.Generator(device=DEV).manual_seed(D), 1.0 / math.sqrt(D)
+    mk = lambda n: torch.randn((1, H, n, D), generator=g, device=DEV, dtype=torch.float16)   # noqa: E731
+    q, kq, vq = mk(1), qfa.asymmetric_quant_per_token(mk(Nk)), qfa.asymmetric_quant_per_token(mk(Nk))
+    none = torch.empty(0, dtype=q.dtype, device=DEV)
+
+    def moved(t):
+        out = torch.empty(t[0].numel() + offset, dtype=torch.int8, device=DEV)[offset:].view(1, Nk, H, D).transpose(1, 2)
+        return (out.copy_(t[0]), *t[1:])
+
+    def step(k, v):
+        with torch.no_grad():
+            return qfa.quant_flash_attn_quantized_kv(q, none, none, k, v, True, sm)
+    other = moved(kq), moved(vq)
+    for pair, want in (((kq, vq), True), (other, hint), ((kq, other[1]), hint)):
+        assert _hint(launches(lambda: None, lambda _: step(*pair)), "cache_fwd_kernel") == want
+        assert torch.equal(step(*pair), step(kq, vq))
+
+
+@pytest.mark.parametrize("H,Nq,Nk,D", [(1500, 32, 1029, 64), (1500, 16, 1029, 64), (2080, 16, 1025, 128)])
+def test_shared_lines_of_two_heads(qfa, H, Nq, Nk, D):
+    g, sm = torch.Generator(device=DEV).manual_seed(D + Nq), 1.0 / math.sqrt(D)
+    mk = lambda n: torch.randn((1, H, n, D), generator=g, device=DEV, dtype=torch.float16)   # noqa: E731
+    q, do, kvq, results = mk(Nq), mk(Nq), qfa.asymmetric_quant_per_token(mk(Nk)), []
+    for codes, hint in ((kvq, True), (_between(kvq), D == 128)):
+        fwd = lambda: qfa.attn_fwd_shared_kv(q, *codes, sm)   # noqa: E731
+        o, lse = fwd()
+        bwd = lambda: qfa.attn_bwd_shared_kv(q, *codes, o, do, lse, sm)   # noqa: E731
+        assert _hint(launches(lambda: None, lambda _: bwd()), "skv_bwd_kernel") == hint
+        if D == 128:
+            assert _hint(launches(lambda: None, lambda _: fwd()), "skv_fwd_kernel") == hint
+        results.append((o, *bwd()))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
