@@ -760,11 +760,7 @@ template <typename T, int D> static int launch_fwd_td(const AttnArgs &x, hipStre
   a.sm_scale_log2 = x.sm_scale * kLog2e;
   constexpr int FWD_BM = 32 * FWD_WAVES;
   a.mblocks = (int)((x.Nq + FWD_BM - 1) / FWD_BM);
-  // O past the caches where codes, V and O exceed the last-level cache: else it pushes out the K and V that other workgroups read next.
-  // The forward, and with a product that reads O behind it, us: 64 heads of 4096 x 256 causal 618 -> 582, 682 -> 669; 1000 of 200 x 256
-  // 176 -> 160, 232 -> 224; 128 of 4096 x 128 causal 561 -> 550, 618 -> 613.  Below it nothing is gained and the product loses (1024 of
-  // 300 x 128: 123 -> 123, 159 -> 163), and at head_dim 64 nothing was seen
-  a.o_once = D >= 128 && x.B * x.H * (x.Nq + x.Nk) * D * 3 > LAST_LEVEL_BYTES;
+  a.o_once = fwd_o_once(x.B * x.H, x.Nq, x.Nk, D, x.o, x.sob, x.soh, x.son);
   a.splits = 1;
   a.keys_per_split = 0;
   a.po = a.pml = nullptr;

@@ -107,6 +107,9 @@ inline bool rows_own_lines(const void *p, int64_t sb, int64_t sh, int64_t sn, in
   return sn * es == row_bytes || (((int64_t)reinterpret_cast<uintptr_t>(p) | sb * es | sh * es | sn * es | row_bytes) & 127) == 0;
 }
 
+// Whether the forward's O, 16 bit, is written past the caches (qfa_split_plan.cpp)
+bool fwd_o_once(int64_t BH, int64_t Nq, int64_t Nk, int D, const void *o, int64_t sob, int64_t soh, int64_t son);
+
 // Shared-KV attention (K = V = one quantized tensor, Q in 16-bit float), after validation.
 struct SkvAttnArgs {
   const void *q; const int8_t *codes; const void *scale; const int8_t *zp;

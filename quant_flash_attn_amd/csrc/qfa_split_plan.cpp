@@ -134,6 +134,17 @@ int64_t fwd_workspace_bytes(int64_t B, int64_t H, int64_t Nq, int64_t Nk, int D,
   return splits > 1 ? B * H * Nq * splits * (int64_t)(D + 2) * 4 : 0;
 }
 
+// O past the caches where codes, V and O exceed the last-level one: else it pushes out what other workgroups read next, and where
+// there are few keys its lines are still the cheaper to write.  29 calls of 256 to 2500 MiB, with and without a mask, the whole call
+// (with a product that reads O behind it) against the same without the hint: head_dim 256 0.968 (0.984) of the time in the mean, 0.906 to
+// 0.999 (0.963 to 0.998); 128 0.982 (0.994), 0.928 to 0.998 (0.979 to 1.016).  64 heads of 4096 x 256 causal 616 -> 579 us, 225 of 1525 x 572
+// 327 -> 300, 256 of 4096 x 256 keys of 128 270 -> 251, 128 of 4096 x 128 causal 555 -> 544.  Below that size nothing is gained and the
+// product loses (1024 of 300 x 128: 123 -> 123, 159 -> 163), and at head_dim 64 nothing was seen.  Rows that share their lines with those
+// of other heads are written in pieces, which may take longer with the hint (1798 heads of 231 x 256, 266 -> 278 us)
+bool fwd_o_once(int64_t BH, int64_t Nq, int64_t Nk, int D, const void *o, int64_t sob, int64_t soh, int64_t son) {
+  return D >= 128 && BH * (Nq + Nk) * D * 3 > LAST_LEVEL_BYTES && rows_own_lines(o, sob, soh, son, 2 * D, 2);
+}
+
 // ---- backward
 // Blocks of 32 rows per wave.  Two at head_dim 128: a step of 64 rows per wave costs 1 / 0.62 of one of 32, which need more LDS
 // reads per row, but fill the chip with twice the workgroups and waste less of the last one (1024 x 1024, 16 heads: dQ 44 -> 22

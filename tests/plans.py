@@ -26,6 +26,11 @@ def _plan(name, result, args):
     return f
 
 
+def fwd_o_once(BH, Nq, Nk, D, o, strides):
+    """whether the forward's O at address `o` is written past the caches; strides of its [B, H, N] in elements"""
+    return _plan("_ZN3qfa10fwd_o_onceEllliPKvlll", ctypes.c_bool, [_L, _L, _L, _I, ctypes.c_void_p, _L, _L, _L])(BH, Nq, Nk, D, o, *strides)
+
+
 def bwd_plan(BH, Nq, Nk, D, causal, may_split=1):
     return _plan("_ZN3qfa8bwd_planEllliii", BwdPlan, [_L, _L, _L, _I, _I, _I])(BH, Nq, Nk, D, int(causal), may_split)
 
