@@ -3,7 +3,7 @@
 // Neither reads what the other writes, and both take a SIMD's registers and most of a CU's LDS (one workgroup per CU, two at head_dim
 // 64).  As two launches each left CUs idle: all that its blocks do not fill, the last round of a launch, and the time between the two.
 // dK and dV come first: their workgroups take longer, so those of dQ fill up what they leave.  Either goes out alone where
-// the parts of one take the memory of the other's (BwdPlan::sum_between).
+// the parts of one take the memory of the other's, or one launch does not hold both (BwdPlan::sum_between).
 // Measured, the whole backward before and after, us, bf16, one GPU: 8 heads of 1000 x 128 causal 60 -> 38; 18 x 805 x 128 57 -> 41;
 // 45 x 1500 x 256 421 -> 349; 3 x 1866 x 64 causal 55 -> 31; 100 x 1000 x 128 causal 178 -> 145; 33 x 4626 x 128 1085 -> 977; 525 x 140 x 64
 // causal 55 -> 46; 20 x 4000 x 64 355 -> 293; chips that both fill in whole rounds take as long as before (128 x 4096 x 128 causal 1689 ->

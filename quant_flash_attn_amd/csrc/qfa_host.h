@@ -44,7 +44,7 @@ int launch_dequant(const int8_t *codes, const void *scale, int scale_dtype, cons
                    int64_t sob, int64_t soh, int64_t son, hipStream_t st);
 
 // How the backward's two kinds of workgroups are launched: 32-row blocks per wave, and the parts of the streamed rows; the memory of the
-// parts, and whether those of dQ take the place of the others
+// parts, and whether dQ is a launch of its own (its parts then take the place of the others)
 struct BwdPlan { int blocks_dkv, splits_dkv, queries_per_split, blocks_dq, splits_dq, keys_per_split, sum_between; int64_t part_bytes; };
 
 // Tensors of one attention call, after validation.  Strides in elements.

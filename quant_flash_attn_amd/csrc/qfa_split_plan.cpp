@@ -327,7 +327,10 @@ BwdPlan bwd_plan(int64_t BH, int64_t Nq, int64_t Nk, int D, int causal, int may_
   // large parts of both: dK and dV are added before dQ starts, whose parts take their place.  One launch more, of a call of
   // milliseconds (2 heads, 16384 x 16384 of 256, causal, forward and backward: 1939 -> 1908 us); smaller ones lose by it (4 heads of
   // 2300: 188 -> 191)
-  p.sum_between = kv > 0 && q > 0 && kv + q > SUM_BETWEEN;
+  // (and what one launch of 2^32 - 1 threads does not hold: 8388607 heads, whose staging launch is not too large)
+  const auto wgs = [&](int64_t rows, int blocks, int splits) { return (BH * ((rows + 128 * blocks - 1) / (128 * blocks)) + 7) / 8 * 8 * splits; };
+  p.sum_between = (kv > 0 && q > 0 && kv + q > SUM_BETWEEN) ||
+                  wgs(Nk, p.blocks_dkv, p.splits_dkv) + wgs(Nq, p.blocks_dq, p.splits_dq) > 0xffffffffLL / 256;
   p.part_bytes = p.sum_between ? std::max(kv, q) : kv + q;
   return p;
 }

@@ -93,3 +93,12 @@ def test_what_is_planned_is_launched(qfa):
             alone = bwd_plan(*s, may_split=0)   # (each kind's rows per wave as if it had the chip to itself)
             undivided += (p.blocks_dkv, p.blocks_dq) != (alone.blocks_dkv, alone.blocks_dq)
     assert undivided > 20
+
+
+def test_more_than_one_launch_holds(qfa):
+    """2^32 - 1 threads: of so many heads dK / dV and dQ go out one after the other, as long as the staging launch (two tiles a head) fits."""
+    for BH, two in ((8388600, 0), (8388601, 1), (8388607, 1)):
+        assert 2 * BH * 256 < 2 ** 32
+        p = bwd_plan(BH, 1, 1, 64, False)
+        assert (p.sum_between, p.part_bytes, p.splits_dkv, p.splits_dq) == (two, 0, 1, 1)
+        assert two or 2 * ((BH + 7) // 8 * 8) * 256 < 2 ** 32
