@@ -304,6 +304,13 @@ static void plan_pair(int64_t BH, int64_t Nq, int64_t Nk, int D, bool causal, Bw
         bq = &q[j];
       }
     }
+  // Undivided dK / dV of 64 rows per wave beside workgroups of dQ that do not run at once with them: the estimate takes too little where those
+  // of 32 rows would all run at once, since half as many take twice as long each and have nothing behind which to hide what is left of
+  // dQ.  Of 139 random calls for which 64 rows were chosen ten are such, and they took 1.07 to 1.17 times as long as with 32 (7 heads of
+  // 4192: 208 -> 243 us; 0.95 without a mask and with whole tiles of queries, 4224: 205 -> 195); the others 0.898, 1.06 at most
+  if (!full && bk != kv && bk->blocks == 2 && bk->splits == 1 && bq->splits == 1 && bk->n + bq->n > 256.0)
+    for (int i = 0; i < nkv; ++i)
+      if (kv[i].blocks == 1 && kv[i].splits == 1 && kv[i].n <= 256.0) bk = &kv[i];
   p->blocks_dkv = bk->blocks; p->splits_dkv = bk->splits; p->queries_per_split = bk->each;
   p->blocks_dq = bq->blocks; p->splits_dq = bq->splits; p->keys_per_split = bq->each;
 }

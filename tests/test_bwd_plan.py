@@ -70,6 +70,25 @@ def test_slower_rows_per_wave_are_not_chosen(qfa, BH, Nq, Nk, causal, rows, own,
     assert (p.blocks_dkv, p.blocks_dq) != rows, joint / own
 
 
+LONG_CHAINS = [
+    # heads, Nq, Nk, causal, us undivided with 32 rows per wave, us with 64 of dK / dV
+    (7, 4143, 4143, False, 199.7, 232.5),
+    (7, 4192, 4192, False, 203.5, 236.1),
+    (7, 4159, 4188, False, 203.7, 233.6),
+    (7, 4324, 4324, False, 210.9, 250.5),
+    (7, 4288, 4288, True, 161.5, 175.6),
+    (7, 4546, 4546, True, 176.2, 187.9),
+    (6, 4909, 4909, True, 180.5, 198.6),
+]
+
+
+@pytest.mark.parametrize("BH,Nq,Nk,causal,short,long", LONG_CHAINS)
+def test_dkv_stays_at_32_rows_where_it_runs_all_at_once(qfa, BH, Nq, Nk, causal, short, long):
+    """Half as many workgroups of twice the length, beside as many of dQ as before."""
+    p = bwd_plan(BH, Nq, Nk, 128, causal)
+    assert ((p.blocks_dkv, p.splits_dkv), (p.blocks_dq, p.splits_dq)) != ((2, 1), (1, 1)), long / short
+
+
 def _fields(p):
     return tuple(getattr(p, n) for n, _ in p._fields_)
 
