@@ -377,7 +377,7 @@ int qfa_bwd_delta(const void *o, const void *dout, float *delta, int io_dtype, i
  *              16-byte aligned, overwritten: two staging passes fill it with delta = rowsum(O o dO),
  *              the transposed 16-bit tiles Q^^T, K^^T (the dequantized Q and K rounded to
  *              io_dtype, the operands of the dK and dQ products) and per-token constants, once
- *              per call, so that the two MFMA kernels stream ready-made tiles.  The scores S, and
+ *              per call, so that the MFMA kernel streams ready-made tiles.  The scores S, and
  *              with them P, come from the INT8 codes exactly as in the forward.
  *   dq [B,H,Nq,D], dk, dv [B,H,Nk,D] of io_dtype, strides as given.
  */

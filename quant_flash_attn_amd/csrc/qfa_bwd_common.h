@@ -38,7 +38,7 @@ struct BwdArgs {
   void *do16;
   int64_t sd32b, sd32h, sd32n;
   int grad_f32;         // dQ, dK, dV are fp32
-  int per_split;        // streamed rows per part (a multiple of 64), part blockIdx.y; all of them in one where not split
+  int per_split;        // streamed rows per part (a multiple of 64); all of them in one where not split
   int last_part;        // first row of the last part
   int64_t split_stride; // fp32 elements from one part's gradients to the next's
   int group_log2;       // causal: log2 of the number of heads whose blocks are dispatched together (set per launch)

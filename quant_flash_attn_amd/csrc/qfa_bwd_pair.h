@@ -4,10 +4,12 @@
 // 64).  As two launches each left CUs idle: all that its blocks do not fill, the last round of a launch, and the time between the two.
 // dK and dV come first: their workgroups take longer, so those of dQ fill up what they leave.  Either goes out alone where
 // the parts of one take the memory of the other's, or one launch does not hold both (BwdPlan::sum_between).
-// Measured, the whole backward before and after, us, bf16, one GPU: 8 heads of 1000 x 128 causal 60 -> 38; 18 x 805 x 128 57 -> 41;
-// 45 x 1500 x 256 421 -> 349; 3 x 1866 x 64 causal 55 -> 31; 100 x 1000 x 128 causal 178 -> 145; 33 x 4626 x 128 1085 -> 977; 525 x 140 x 64
-// causal 55 -> 46; 20 x 4000 x 64 355 -> 293; chips that both fill in whole rounds take as long as before (128 x 4096 x 128 causal 1689 ->
-// 1685; 256 x 2048 x 64 causal 605 -> 595; 16 x 16384 x 128 5194 -> 5195; the kernels sent one after the other 1678, 607, 5204).
+// Measured, the whole backward with two launches, each divided by itself, and now, us, bf16, one GPU: 8 heads of 1000 x 128 causal 64 -> 43;
+// 18 x 805 x 128 62 -> 45; 45 x 1500 x 256 432 -> 360; 3 x 1866 x 64 causal 45 -> 35; 100 x 1000 x 128 causal 181 -> 148; 33 x 4626 x 128
+// 1113 -> 1024; 525 x 140 x 64 causal 60 -> 51; 20 x 4000 x 64 364 -> 303; chips that both fill in whole rounds take as long as before
+// (128 x 4096 x 128 causal 1636 -> 1631; 256 x 2048 x 64 causal 592 -> 584; 16 x 16384 x 128 5293 -> 5276).
+// Counters of the last three and of 64 x 4096 x 256 causal: matrix pipe busy 55, 43, 70 and 51 % of the time at 2.04, 2.08, 1.79 and 1.98 GHz,
+// waits 21, 27, 15 and 25 % of the waves' time, issue stalls 24, 28, 24 and 25 %: the long sequence is bound by power, the others are not.
 #pragma once
 #include <cstddef>
 

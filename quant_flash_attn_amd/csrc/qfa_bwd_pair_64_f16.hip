@@ -1,4 +1,4 @@
-// The backward's kernel at head_dim 64, Float16 (one instance per file: each takes minutes to compile)
+// The backward's kernel at head_dim 64, Float16 (one instance per file: they are compiled side by side)
 #include "qfa_bwd_pair.h"
 
 namespace qfa {

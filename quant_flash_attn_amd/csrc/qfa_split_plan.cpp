@@ -214,7 +214,7 @@ struct PairCost {
   double base, prep, sum, mb;   // us: launches; staging per MB (10^6 elements); the sum of parts and what it takes per MB
   double start[2], tail;        // of a workgroup of dK / dV and of dQ, in tiles; share of the last one that runs alone
   double tile[2][2];            // us per tile: [dK / dV, dQ][32, 64 rows per wave; at head_dim 64 one, two workgroups per CU]
-  double crowd, over;           // share of the mean load beside the longest workgroup, within one round and beyond
+  double crowd, over;           // of the mean load, added to the longest workgroup: within one round its share, beyond a fitted correction (below zero too)
 };
 constexpr int64_t SUM_BETWEEN = 128 << 20;   // of parts: more of both, and they are added between two launches
 struct Share { int blocks, splits, each; double n, tiles, last, mbytes; };   // workgroups, tiles of all, of the longest
