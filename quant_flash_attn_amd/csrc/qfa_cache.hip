@@ -383,12 +383,13 @@ template <typename S, int D> static int launch_cache_sd(const CacheAttnArgs &x, 
   const int64_t total = xcd_grid(a.BH, (int64_t)a.qblocks * a.splits);
   if (x.B * x.H > 0x7fffffffLL || total > 0x7fffffffLL || x.B * x.H * x.Nq > 0x7fffffffLL)
     return set_error(QFA_EUNSUPPORTED, "attn_fwd_cache: too many query blocks for one launch");
-  // Non-temporal loads (LOAD_ONCE), measured over 1400 random calls: from 320 MiB and 1024 keys on, 0.96 (head_dim 64, 128) and 0.975 (256) of
-  // the time on three caches in turn, 0.97 and 0.99 on one and the same; shorter sequences of many heads 1.03 to 1.09, 100 to 256 MiB
-  // 0.97 on three caches but 1.06 to 1.1 on one.  8 x 32 heads, one query on 8192 keys of 128: 95.5 -> 83 us (5.8 -> 6.6 TB/s)
+  // Non-temporal loads (LOAD_ONCE), measured over 1400 random calls: from 320 MiB and 1024 keys on, 0.96 of the time at head_dim 64 and 128 on
+  // three caches in turn, 0.97 on one and the same; shorter sequences of many heads 1.03 to 1.09, 100 to 256 MiB 0.97 on three caches but
+  // 1.06 to 1.1 on one.  Not at 256: 46 calls 0.915 to 1.113, 1.011 in the mean (1.03 with 16 queries: 2083 heads on 1434 keys 321 -> 345 us).
+  // 8 x 32 heads, one query on 8192 keys of 128: 95.5 -> 83 us (5.8 -> 6.6 TB/s)
   const bool once = a.qblocks == 1 && x.Nk >= 1024 && 2 * x.B * x.H * x.Nk * D > LAST_LEVEL_BYTES / 4 * 5 &&
                     rows_own_lines(x.kc, x.skb, x.skh, x.skn, D) && rows_own_lines(x.vc, x.svb, x.svh, x.svn, D);
-  if (once) cache_fwd_kernel<S, D, true><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
+  if (D < 256 && once) cache_fwd_kernel<S, D, (D < 256)><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   else cache_fwd_kernel<S, D, false><<<dim3((unsigned)total), dim3(256), 0, st>>>(a);
   if (int e = check_launch("qfa_attn_fwd_cache")) return e;
   if (a.splits > 1) {

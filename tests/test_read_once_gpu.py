@@ -116,3 +116,18 @@ def test_shared_lines_of_two_heads(qfa, H, Nq, Nk, D):
             assert _hint(launches(lambda: None, lambda _: fwd()), "skv_fwd_kernel") == hint
         results.append((o, *bwd()))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("Nq", [1, 16])
+@pytest.mark.parametrize("H,D,hint", [(2700, 64, True), (1340, 128, True), (670, 256, False)])
+def test_widest_caches_are_read_without_the_hint(qfa, H, Nq, D, hint):
+    """Where it takes longer: up to 1.11 times at head_dim 256, the same calls at 64 and 128 0.96."""
+    g = torch.Generator(device=DEV).manual_seed(D)
+    mk = lambda n: torch.randn((1, H, n, D), generator=g, device=DEV, dtype=torch.float16)   # noqa: E731
+    q, k, v = mk(Nq), qfa.asymmetric_quant_per_token(mk(1029)), qfa.asymmetric_quant_per_token(mk(1029))
+    none = torch.empty(0, dtype=q.dtype, device=DEV)
+
+    def step(_):
+        with torch.no_grad():
+            return qfa.quant_flash_attn_quantized_kv(q, none, none, k, v, True, 0.1)
+    assert _hint(launches(lambda: None, step), "cache_fwd_kernel") == hint
